@@ -304,19 +304,19 @@ struct SpatialGeom {
     int steps;      // gpw rounded up to a multiple of NST
 };
 
-// Sums of U (2 or 4) values per lane over each row of 16 lanes of a wave: every lane
-// ends up with its row's total of value number (lane % U).  The first steps halve the
+// Sums of U (2 or 4) values per lane over the wave: every lane ends up with the total of
+// value number (lane % U).  The first steps halve the
 // number of values a lane carries instead of adding U full sums side by side: lane
 // pairs exchange the value the other keeps (quad permutes); then the quads of a row add
-// up by rotation.  (The four rows of a wave are left apart: bringing them together takes
-// lane-indexed reads through the LDS unit, whose counter the kernel's scalar weight
-// loads share - waiting for one drains the other's prefetch.)
+// up by rotation, and the rows of the wave by swapping rows and halves of it (gfx950's lane
+// swaps, on the vector ALU: reads through the LDS unit would share the counter of the
+// kernel's scalar weight loads - waiting for one drains the other's prefetch).
 template <int CTRL>
 __device__ __forceinline__ float from_permuted(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
 }
 template <int U>
-__device__ __forceinline__ float row_sums(const float (&v)[U], int lane) {
+__device__ __forceinline__ float wave_sums(const float (&v)[U], int lane) {
     static_assert(U == 2 || U == 4, "two or four values per lane");
     const bool b0 = lane & 1, b1 = lane & 2;
     float k = (b0 ? v[1] : v[0]) + from_permuted<0xB1 /* quad_perm [1,0,3,2] */>(b0 ? v[0] : v[1]);
@@ -328,12 +328,14 @@ __device__ __forceinline__ float row_sums(const float (&v)[U], int lane) {
     }
     k += from_permuted<0x124 /* row_ror:4 */>(k);
     k += from_permuted<0x128 /* row_ror:8 */>(k);
-    return k;
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(k), __float_as_uint(k), false, false);
+    k = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(k), __float_as_uint(k), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
 // POOL: the kernel also leaves, per sample, pixel tile and channel, the sum of the
-// feature map over the pixels of a quarter of the tile (the lanes of one row of 16) in
-// pool_part[((n * tiles + tile) * 4 + row) * C + c] (fp32) -
+// feature map over the pixels of the tile in pool_part[(n * tiles + tile) * C + c] (fp32) -
 // the global average pool in front of the channel branch, from the values this kernel
 // has in registers anyway.  Under stride 2 (even H and W) the lane also loads the
 // feature row below its own, and both columns where it otherwise takes one; those lines
@@ -426,11 +428,11 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
 #pragma unroll
         for (int k = 0; k < VP; ++k) acc[t][k] = 0.f;
     // POOL: where this lane's sums of the wave's first channel group go (one partial sum
-    // per row of 16 lanes: four per tile), and how many groups the wave keeps sums of (head
+    // per tile), and how many groups the wave keeps sums of (head
     // 0 of a sample does it for all heads).  Worked out here and pinned: formed inside the
     // walk they take a scalar load of a launch dimension, and the wait for it also waits
     // for the weights that were just requested for the next step.  The sums go out through
-    // a buffer descriptor of the tile's 4 * C values, lanes with nothing to write at an
+    // a buffer descriptor of the tile's C values, lanes with nothing to write at an
     // offset outside it: a store under a branch leaves the compiler unable to count the
     // loads in flight where the branch joins, and it then waits for all of them.
     // (Collecting the sums in LDS and writing them after the walk was no faster.)
@@ -438,10 +440,9 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     uint32_t pool_off = kOutside;
     int pool_groups = 0;
     if constexpr (POOL) {
-        pool_rsrc = plane_rsrc(pool_part + ((n * gridDim.x + blockIdx.x) * 4) * g.C,
-                               (uint32_t)(4 * g.C) * (uint32_t)sizeof(float));
-        if (head == 0 && (lane & 15) < U)
-            pool_off = (uint32_t)((lane >> 4) * g.C + j0 * U + (lane & 15)) * (uint32_t)sizeof(float);
+        pool_rsrc = plane_rsrc(pool_part + (n * gridDim.x + blockIdx.x) * g.C,
+                               (uint32_t)g.C * (uint32_t)sizeof(float));
+        if (head == 0 && lane < U) pool_off = (uint32_t)(j0 * U + lane) * (uint32_t)sizeof(float);
         pool_groups = head == 0 ? min(g.gpw, g.ngroups - j0) : 0;
         asm volatile("" : "+v"(pool_off), "+s"(pool_groups));
     }
@@ -483,7 +484,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
                     }
                     psum[u] = ps;
                 }
-                const float tot = row_sums<U>(psum, lane);
+                const float tot = wave_sums<U>(psum, lane);
                 __builtin_amdgcn_raw_buffer_store_b32(
                     __float_as_uint(tot), pool_rsrc,
                     (int)(keep ? pool_off + (uint32_t)(i * U) * (uint32_t)sizeof(float) : kOutside), 0, 0);
@@ -591,6 +592,33 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     }
 }
 
+// out[n * C + c] = sum of parts[(n * nparts + p) * C + c] over p.  Every workgroup of the
+// channel branch starts from the pooled vectors; with dozens of partial sums per value each
+// of them would spend longer adding up than on its own work (8 x 64 x 200 x 300 fp16: 472
+// sums per value then, 37 of the layer's 107 us), so planes of many tiles pay for one launch.
+constexpr int kMaxParts = 8;             // partial sums the channel branch reads in one round trip
+constexpr int kCollapseChannels = 64, kCollapseGroups = 8;
+__global__ __launch_bounds__(kCollapseChannels * kCollapseGroups) void k_collapse_parts(
+    const float *__restrict__ parts, float *__restrict__ out, int C, int nparts) {
+    __shared__ float red[kCollapseGroups][kCollapseChannels];
+    const int i = threadIdx.x % kCollapseChannels, grp = threadIdx.x / kCollapseChannels;
+    const int c = blockIdx.x * kCollapseChannels + i;
+    const int64_t n = blockIdx.y;
+    float a = 0.f;
+    if (c < C) {
+        const float *src = parts + n * nparts * C + c;
+#pragma unroll 8
+        for (int q = grp; q < nparts; q += kCollapseGroups) a += src[(int64_t)q * C];
+    }
+    red[grp][i] = a;
+    __syncthreads();
+    if (grp == 0 && c < C) {
+#pragma unroll
+        for (int k = 1; k < kCollapseGroups; ++k) a += red[k][i];
+        out[n * C + c] = a;
+    }
+}
+
 // Butterfly steps through the VALU's lane-permute path.  (Shuffles through the
 // LDS crossbar cost a round trip each and made these kernels several times slower.)
 template <int CTRL>
@@ -637,7 +665,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         const int64_t n = n0 + min(s, ns - 1);
         if (parts) {
             float a = 0.f;
-#pragma unroll 4
+#pragma unroll 8
             for (int q = 0; q < nparts; ++q) a += parts[(n * nparts + q) * C + c];
             v[i] = a * scale;
         } else {
@@ -1046,17 +1074,22 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     g.gpw = (int)cdiv(g.ngroups, waves);
     g.steps = (int)cdiv(g.gpw, NST) * NST;
     if (N > 65535 || head > 65535) return hipErrorNotSupported;
+    bool collapse = false;
     if (pool) {
-        if (N * tiles * 4 * C > pool_capacity) return hipErrorInvalidValue;
-        *pool_parts = tiles * 4;
+        // (more tiles than kMaxParts: their sums go behind the N * C totals that
+        // k_collapse_parts then makes of them)
+        collapse = tiles > kMaxParts;
+        if (N * (tiles + (collapse ? 1 : 0)) * C > pool_capacity) return hipErrorInvalidValue;
+        *pool_parts = collapse ? 1 : tiles;
     }
+    float *parts_out = collapse ? pool_part + N * C : pool_part;
     const dim3 grid((unsigned)tiles, (unsigned)head, (unsigned)N);
 #define DDF_STREAM_LAUNCH(VP_, S_, WAVES_)                                                        \
     do {                                                                                          \
         if (pool) {                                                                               \
             hipLaunchKernelGGL((k_spatial_stream<T, KK, VP_, S_, WAVES_, U, NST, true>), grid,    \
                                dim3(WAVES_ * kWave), 0, st, g, x, w, bias, sf, (float)gain,       \
-                               gain_vec, offset_vec, pool_part);                                  \
+                               gain_vec, offset_vec, parts_out);                                  \
             break;                                                                                \
         }                                                                                         \
         hipLaunchKernelGGL((k_spatial_stream<T, KK, VP_, S_, WAVES_, U, NST, false>), grid,       \
@@ -1084,6 +1117,9 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     }
 #undef DDF_STREAM_WAVES
 #undef DDF_STREAM_LAUNCH
+    if (collapse)
+        hipLaunchKernelGGL(k_collapse_parts, dim3((unsigned)cdiv(C, kCollapseChannels), (unsigned)N),
+                           dim3(kCollapseChannels * kCollapseGroups), 0, st, parts_out, pool_part, (int)C, tiles);
     return hipGetLastError();
 }
 
