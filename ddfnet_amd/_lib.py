@@ -45,6 +45,10 @@ SYMBOLS = {
                                     [_i] * 3 + [ctypes.c_double] + [_vp] * 2 + [_i, _vp]),
     'ddf_hip_channel_branch_parts': (_i, [_vp, _i, ctypes.c_double] + [_vp] * 5 + [_i64] * 3 +
                                      [_i, ctypes.c_double] + [_vp] * 2 + [_i, _vp]),
+    'ddf_hip_pack_filters': (_i, [_vp] * 14 + [_i64] * 6 + [_i] * 3 + [ctypes.c_double] * 2 + [_vp, _i, _vp]),
+    'ddf_hip_pack_backward_workspace_bytes': (_sz, [_i64] * 5 + [_i] * 4),
+    'ddf_hip_pack_backward': (_i, [_vp] * 10 + [ctypes.c_double] + [_vp] * 9 + [_sz] + [_i64] * 5 + [_i] * 4 +
+                              [_vp]),
     'ddf_hip_up_forward': (_i, [_vp] * 4 + [_i64] * 4 + [_i] * 5 + [_vp]),
     'ddf_hip_up_backward_workspace_bytes': (_sz, [_i64] * 4 + [_i] * 5 + [_u]),
     'ddf_hip_up_backward': (_i, [_vp] * 8 + [_sz] + [_i64] * 4 + [_i] * 5 + [_u, _vp]),

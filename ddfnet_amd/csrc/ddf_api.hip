@@ -275,6 +275,38 @@ int up_backward_typed(const ddf::Problem &p, int scale, const void *go, const vo
     return DDF_OK;
 }
 
+template <typename T>
+int pack_filters_typed(const void *x, const void *ws, const void *bs, const void *w1, const void *b1, const void *w2,
+                       const void *b2, void *raw, void *sf, void *cf, const ddf::ChannelSave &save, float *parts,
+                       int64_t capacity, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid, int head, int k,
+                       int stride, double sgain, double cgain, const void *cgain_vec, hipStream_t st) {
+    int n_parts = 0;
+    hipError_t err = ddf::spatial_branch<T>((const T *)x, (const T *)ws, (const T *)bs, (T *)sf, N, C, H, W, head, k,
+                                            stride, sgain, (const T *)nullptr, (const T *)nullptr, st, parts,
+                                            capacity, &n_parts, (T *)raw);
+    if (err == hipErrorNotSupported) return fail(DDF_ERR_UNSUPPORTED, "pack filters: sizes not covered");
+    if (err == hipErrorInvalidValue) return fail(DDF_ERR_WORKSPACE, "pack filters: the buffer of partial sums is too small");
+    if (err != hipSuccess) return fail_hip(err, "ddf_hip_pack_filters spatial launch");
+    err = ddf::channel_branch<T>((const T *)nullptr, (const T *)w1, (const T *)b1, (const T *)w2, (const T *)b2, (T *)cf,
+                                 N, C, mid, k, cgain, (const T *)cgain_vec, (const T *)nullptr, st, parts, n_parts,
+                                 1.0 / (double)(H * W), save);
+    if (err == hipErrorNotSupported) return fail(DDF_ERR_UNSUPPORTED, "pack filters: sizes not covered");
+    return err == hipSuccess ? DDF_OK : fail_hip(err, "ddf_hip_pack_filters channel launch");
+}
+
+template <typename T>
+int pack_backward_typed(const void *x, const void *dcf, const void *draw, const float *pooled, const float *hidden,
+                        const float *taps, const void *ws, const void *w1, const void *w2, const void *gain_vec,
+                        double gain, void *dx, void *dws, void *dbs, void *dw1, void *db1, void *dw2, void *db2,
+                        void *dgain, void *workspace, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid,
+                        int head, int stride, hipStream_t st) {
+    const ddf::PackBackward<T> b{(const T *)x, (const T *)dcf, (const T *)draw, pooled, hidden, taps,
+                                 (const T *)ws, (const T *)w1, (const T *)w2, (const T *)gain_vec, gain,
+                                 (T *)dx, (T *)dws, (T *)dbs, (T *)dw1, (T *)db1, (T *)dw2, (T *)db2, (T *)dgain};
+    const hipError_t err = ddf::pack_backward<T>(b, N, C, H, W, mid, head, stride, workspace, st);
+    return err == hipSuccess ? DDF_OK : fail_hip(err, "ddf_hip_pack_backward launch");
+}
+
 }  // namespace
 
 extern "C" {
@@ -644,6 +676,66 @@ int ddf_hip_channel_branch_parts(const float *pool_parts, int n_parts, double sc
     if (!pool_parts) return fail(DDF_ERR_BAD_ARG, "ddf_hip_channel_branch_parts: null partial sums");
     return channel_branch_impl(nullptr, pool_parts, n_parts, scale, weight1, bias1, weight2, bias2,
                                channel_filter, N, C, mid, kernel_size, gain, gain_vec, offset_vec, dtype, stream);
+}
+
+int ddf_hip_pack_filters(const void *features, const void *spatial_weight, const void *spatial_bias,
+                         const void *weight1, const void *bias1, const void *weight2, const void *bias2,
+                         void *raw_spatial_filter, void *spatial_filter, void *channel_filter, float *pooled,
+                         float *hidden, float *channel_taps, float *pool_parts, int64_t pool_capacity, int64_t N,
+                         int64_t C, int64_t H, int64_t W, int64_t mid, int head, int kernel_size, int stride,
+                         double spatial_gain, double channel_gain, const void *channel_gain_vec, int dtype,
+                         void *stream) {
+    if (ddf_hip_pack_backward_workspace_bytes(N, C, H, W, mid, head, kernel_size, stride, dtype) == 0)
+        return fail(DDF_ERR_UNSUPPORTED, "pack filters: layer not covered");
+    if (!features || !spatial_weight || !weight1 || !weight2 || !raw_spatial_filter || !spatial_filter ||
+        !channel_filter || !pooled || !hidden || !channel_taps || !pool_parts)
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    const ddf::ChannelSave save{pooled, hidden, channel_taps};
+    hipStream_t st = (hipStream_t)stream;
+#define DDF_PACK_CASE(T_)                                                                                      \
+    return pack_filters_typed<T_>(features, spatial_weight, spatial_bias, weight1, bias1, weight2, bias2,      \
+                                  raw_spatial_filter, spatial_filter, channel_filter, save, pool_parts,        \
+                                  pool_capacity, N, C, H, W, mid, head, kernel_size, stride, spatial_gain,     \
+                                  channel_gain, channel_gain_vec, st)
+    if (dtype == DDF_F16) DDF_PACK_CASE(__half);
+    DDF_PACK_CASE(float);
+#undef DDF_PACK_CASE
+}
+
+size_t ddf_hip_pack_backward_workspace_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid, int head,
+                                             int kernel_size, int stride, int dtype) {
+    if ((dtype != DDF_F16 && dtype != DDF_F32) || stride < 1 ||
+        !ddf::pack_backward_supported(N, C, mid, H, W, head, kernel_size, stride, dtype))
+        return 0;
+    return ddf::pack_backward_workspace(N, C, mid, H, W, head, stride, dtype);
+}
+
+int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter, const void *grad_raw_spatial_filter,
+                          const float *pooled, const float *hidden, const float *channel_taps,
+                          const void *spatial_weight, const void *weight1, const void *weight2,
+                          const void *channel_gain_vec, double channel_gain, void *grad_features,
+                          void *grad_spatial_weight, void *grad_spatial_bias, void *grad_weight1, void *grad_bias1,
+                          void *grad_weight2, void *grad_bias2, void *grad_channel_gain, void *workspace,
+                          size_t workspace_bytes, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid, int head,
+                          int kernel_size, int stride, int dtype, void *stream) {
+    const size_t want = ddf_hip_pack_backward_workspace_bytes(N, C, H, W, mid, head, kernel_size, stride, dtype);
+    if (want == 0) return fail(DDF_ERR_UNSUPPORTED, "pack backward: layer not covered");
+    if (!features || !grad_channel_filter || !grad_raw_spatial_filter || !pooled || !hidden || !channel_taps ||
+        !spatial_weight || !weight1 || !weight2 || !grad_spatial_weight || !grad_weight1 || !grad_weight2)
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    if (!workspace || workspace_bytes < want || ((uintptr_t)workspace & 255u) != 0)
+        return fail(DDF_ERR_WORKSPACE, "workspace of %zu bytes (256-byte aligned) needed, %zu given", want,
+                    workspace ? workspace_bytes : (size_t)0);
+    hipStream_t st = (hipStream_t)stream;
+#define DDF_PACK_CASE(T_)                                                                                       \
+    return pack_backward_typed<T_>(features, grad_channel_filter, grad_raw_spatial_filter, pooled, hidden,      \
+                                   channel_taps, spatial_weight, weight1, weight2, channel_gain_vec,            \
+                                   channel_gain, grad_features, grad_spatial_weight, grad_spatial_bias,         \
+                                   grad_weight1, grad_bias1, grad_weight2, grad_bias2, grad_channel_gain,       \
+                                   workspace, N, C, H, W, mid, head, stride, st)
+    if (dtype == DDF_F16) DDF_PACK_CASE(__half);
+    DDF_PACK_CASE(float);
+#undef DDF_PACK_CASE
 }
 
 int ddf_hip_up_forward(const void *features, const void *const *channel_filters,

@@ -344,7 +344,7 @@ template <typename T, int KK, int VP, int S, int WAVES, int U, int NST, bool POO
 __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     SpatialGeom g, const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
     T *__restrict__ sf, float gain, const T *__restrict__ gain_vec, const T *__restrict__ offset_vec,
-    float *__restrict__ pool_part) {
+    float *__restrict__ pool_part, T *__restrict__ raw) {
     // feature elements a lane loads per channel (pooling under stride 2: both columns)
     constexpr int XE = S == 1 ? VP : (VP == 1 && !POOL ? 1 : 2 * VP);
     constexpr int kXB = XE * sizeof(T), NWX = vec_words(kXB);
@@ -572,6 +572,20 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     }
     TapParams<T, KK> params;
     params.load(head, gain, gain_vec, offset_vec, bias);
+    const int64_t taps_at = ((n * heads + head) * KK) * (int64_t)g.npix;
+    const uint32_t ob = live ? (uint32_t)p * (uint32_t)sizeof(T) : kOutside;
+    if (raw) {   // (training: the gradient of the normalisation wants the taps as they go into it)
+        const __amdgpu_buffer_rsrc_t rr = plane_rsrc(raw + taps_at, (uint32_t)KK * (uint32_t)g.npix * (uint32_t)sizeof(T));
+#pragma unroll
+        for (int t = 0; t < KK; ++t) {
+            float r[VP];
+#pragma unroll
+            for (int k = 0; k < VP; ++k) r[k] = acc[t][k] + params.bias[t];
+            uint32_t ow[NWO];
+            rows::pack<T, VP, float>(r, ow);
+            store_vec_nt<kOB>(rr, ob + (uint32_t)t * (uint32_t)g.npix * (uint32_t)sizeof(T), ow);
+        }
+    }
 #pragma unroll
     for (int k = 0; k < VP; ++k) {
         float r[KK];
@@ -581,9 +595,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
 #pragma unroll
         for (int t = 0; t < KK; ++t) acc[t][k] = r[t];
     }
-    T *on = sf + ((n * heads + head) * KK) * (int64_t)g.npix;
-    const __amdgpu_buffer_rsrc_t orr = plane_rsrc(on, (uint32_t)KK * (uint32_t)g.npix * (uint32_t)sizeof(T));
-    const uint32_t ob = live ? (uint32_t)p * (uint32_t)sizeof(T) : kOutside;
+    const __amdgpu_buffer_rsrc_t orr = plane_rsrc(sf + taps_at, (uint32_t)KK * (uint32_t)g.npix * (uint32_t)sizeof(T));
 #pragma unroll
     for (int t = 0; t < KK; ++t) {
         uint32_t ow[NWO];
@@ -649,7 +661,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const T *__restrict__ pooled, const T *__restrict__ w1, const T *__restrict__ b1,
     const T *__restrict__ w2, const T *__restrict__ b2, T *__restrict__ cf, int N, int C, int mid,
     float gain, const T *__restrict__ gain_vec, const T *__restrict__ offset_vec,
-    const float *__restrict__ parts, int nparts, float scale) {
+    const float *__restrict__ parts, int nparts, float scale, ChannelSave save) {
     extern __shared__ float branch_smem[];
     float *v = branch_smem;            // [NS][C]
     float *h = v + NS * C;             // [NS][mid]
@@ -671,6 +683,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         } else {
             v[i] = ld(pooled + n * C + c);
         }
+        if (save.pooled && blockIdx.x == 0 && s < ns) save.pooled[n * C + c] = v[i];
     }
     __syncthreads();
     // Dot products with sixteen lanes along a weight row and four rows per wave at a
@@ -694,7 +707,11 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const float tot = row_sum(p[s]);
-            if (sl == 0 && m0 + seg < mid) h[s * mid + m0 + seg] = fmaxf(tot + bias, 0.f);
+            if (sl == 0 && m0 + seg < mid) {
+                const float hm = fmaxf(tot + bias, 0.f);
+                h[s * mid + m0 + seg] = hm;
+                if (save.hidden && blockIdx.x == 0 && s < ns) save.hidden[(n0 + s) * mid + m0 + seg] = hm;
+            }
         }
     }
     __syncthreads();
@@ -729,7 +746,10 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 const float tot = row_sum(p[u][s]);
-                if (sl == 0 && r < rows) f[s * BLOCK * KK + r] = tot + bias;
+                if (sl == 0 && r < rows) {
+                    f[s * BLOCK * KK + r] = tot + bias;
+                    if (save.taps && s < ns) save.taps[((n0 + s) * C + cb) * KK + r] = tot + bias;
+                }
             }
         }
     }
@@ -799,7 +819,8 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
     const __half *__restrict__ pooled, const __half *__restrict__ w1, const __half *__restrict__ b1,
     const __half *__restrict__ w2, const __half *__restrict__ b2, __half *__restrict__ cf, int N, int C,
     int mid, int block, float gain, const __half *__restrict__ gain_vec,
-    const __half *__restrict__ offset_vec, const float *__restrict__ parts, int nparts, float scale) {
+    const __half *__restrict__ offset_vec, const float *__restrict__ parts, int nparts, float scale,
+    ChannelSave save) {
     extern __shared__ __align__(16) _Float16 mma_smem[];
     _Float16 *pv = mma_smem;                        // [C / 32][16 samples][32]: pooled vectors
     _Float16 *hv = pv + (C / kMmaStep) * kMmaTile;  // [tiles of mid][16 samples][32]: hidden vectors
@@ -841,6 +862,10 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
                 v = load_half4(pooled + n * C + c4 * 4);
             }
             *reinterpret_cast<half4_t *>(pv + ((c4 >> 3) * kMmaSamples + s) * kMmaStep + (c4 & 7) * 4) = v;
+            if (save.pooled && blockIdx.x == 0 && n0 + s < N) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) save.pooled[n * C + c4 * 4 + e] = (float)v[e];
+            }
         }
         for (int i = threadIdx.x; i < kMmaTile / 2; i += WAVES * kWave)
             reinterpret_cast<uint32_t *>(hv + (ktiles - 1) * kMmaTile)[i] = 0u;
@@ -903,8 +928,9 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
                 if (m < t * 16) continue;    // (the last tile's overlap: those rows belong to the tile before)
                 const float bias = b1 ? ld(b1 + m) : 0.f;
                 const int kt = min(m / kMmaStep, ktiles - 1);
-                hv[(kt * kMmaSamples + col) * kMmaStep + m - min(kt * kMmaStep, klast)] =
-                    (_Float16)fmaxf(acc[e] + bias, 0.f);
+                const _Float16 hm = (_Float16)fmaxf(acc[e] + bias, 0.f);
+                hv[(kt * kMmaSamples + col) * kMmaStep + m - min(kt * kMmaStep, klast)] = hm;
+                if (save.hidden && blockIdx.x == 0 && n0 + col < N) save.hidden[(int64_t)(n0 + col) * mid + m] = (float)hm;
             }
         }
         __syncthreads();
@@ -998,6 +1024,11 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
                 params.offset[j] = offset_vec ? (float)po[at >> 2][at & 3] : 0.f;
                 params.bias[j] = b2 ? (float)pb[at >> 2][at & 3] : 0.f;
             }
+            if (save.taps) {
+                float *zp = save.taps + ((int64_t)n * C + c0 + quad * 4 + e) * KK;
+#pragma unroll
+                for (int j = 0; j < KK; ++j) zp[j] = u[j] + params.bias[j];
+            }
             normalise<__half, KK>(u, params);
 #pragma unroll
             for (int j = 0; j < KK; ++j) {
@@ -1021,7 +1052,7 @@ template <typename T>
 hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t N, int64_t C, int64_t H,
                           int64_t W, int head, int stride, double gain, const T *gain_vec,
                           const T *offset_vec, hipStream_t st, float *pool_part = nullptr,
-                          int64_t pool_capacity = 0, int *pool_parts = nullptr) {
+                          int64_t pool_capacity = 0, int *pool_parts = nullptr, T *raw = nullptr) {
     constexpr int KK = 9, NST = 3;
     constexpr int U = sizeof(T) == 2 ? 4 : 2;
     constexpr int esz = (int)sizeof(T);
@@ -1089,12 +1120,12 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
         if (pool) {                                                                               \
             hipLaunchKernelGGL((k_spatial_stream<T, KK, VP_, S_, WAVES_, U, NST, true>), grid,    \
                                dim3(WAVES_ * kWave), 0, st, g, x, w, bias, sf, (float)gain,       \
-                               gain_vec, offset_vec, parts_out);                                  \
+                               gain_vec, offset_vec, parts_out, raw);                             \
             break;                                                                                \
         }                                                                                         \
         hipLaunchKernelGGL((k_spatial_stream<T, KK, VP_, S_, WAVES_, U, NST, false>), grid,       \
                            dim3(WAVES_ * kWave), 0, st, g, x, w, bias, sf, (float)gain, gain_vec, \
-                           offset_vec, (float *)nullptr);                                         \
+                           offset_vec, (float *)nullptr, (T *)nullptr);                           \
     } while (0)
 #define DDF_STREAM_WAVES(VP_, S_)                                                                 \
     do {                                                                                          \
@@ -1127,13 +1158,13 @@ template <typename T>
 hipError_t spatial_branch(const T *x, const T *w, const T *bias, T *sf, int64_t N, int64_t C,
                           int64_t H, int64_t W, int head, int k, int stride, double gain,
                           const T *gain_vec, const T *offset_vec, hipStream_t st, float *pool_part,
-                          int64_t pool_capacity, int *pool_parts) {
+                          int64_t pool_capacity, int *pool_parts, T *raw) {
     const int64_t Ho = H / stride, Wo = W / stride;
     if (N == 0 || C == 0 || Ho * Wo == 0 || head == 0) return hipSuccess;
     if (N > 65535 || head > 65535 || C > (1 << 24) || H * W >= (1ll << 31)) return hipErrorNotSupported;
     if (k == 3) {
         const hipError_t err = spatial_stream<T>(x, w, bias, sf, N, C, H, W, head, stride, gain, gain_vec,
-                                                 offset_vec, st, pool_part, pool_capacity, pool_parts);
+                                                 offset_vec, st, pool_part, pool_capacity, pool_parts, raw);
         if (err != hipErrorNotSupported) return err;
     }
     if (pool_part) return hipErrorNotSupported;   // (only the streaming kernel pools)
@@ -1205,7 +1236,7 @@ hipError_t spatial_branch(const T *x, const T *w, const T *bias, T *sf, int64_t 
 template <typename T>
 hipError_t channel_branch_mma(const T *, const T *, const T *, const T *, const T *, T *, int64_t, int64_t,
                               int64_t, int, double, const T *, const T *, hipStream_t, const float *, int,
-                              double) {
+                              double, const ChannelSave &) {
     return hipErrorNotSupported;
 }
 template <>
@@ -1213,7 +1244,7 @@ hipError_t channel_branch_mma<__half>(const __half *pooled, const __half *w1, co
                                       const __half *w2, const __half *b2, __half *cf, int64_t N, int64_t C,
                                       int64_t mid, int k, double gain, const __half *gain_vec,
                                       const __half *offset_vec, hipStream_t st, const float *parts,
-                                      int nparts, double scale) {
+                                      int nparts, double scale, const ChannelSave &save) {
     if (tune_int("DDF_TUNE_CHANNEL_MMA", 1) == 0) return hipErrorNotSupported;
     auto aligned = [](const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
     const size_t lds = (size_t)(C / kMmaStep + cdiv(mid, kMmaStep)) * kMmaTile * sizeof(__half);
@@ -1231,7 +1262,7 @@ hipError_t channel_branch_mma<__half>(const __half *pooled, const __half *w1, co
 #define DDF_MMA_LAUNCH(KK_, WAVES_)                                                                  \
     hipLaunchKernelGGL((k_channel_branch_mma<KK_, WAVES_>), grid, dim3(WAVES_ * kWave), lds, st, pooled, \
                        w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, block, (float)gain, gain_vec,      \
-                       offset_vec, parts, nparts, (float)scale)
+                       offset_vec, parts, nparts, (float)scale, save)
     if (k == 3 && waves == 8) DDF_MMA_LAUNCH(9, 8);
     else if (k == 3) DDF_MMA_LAUNCH(9, 4);
     else DDF_MMA_LAUNCH(25, 4);
@@ -1243,11 +1274,11 @@ template <typename T>
 hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2, const T *b2,
                           T *cf, int64_t N, int64_t C, int64_t mid, int k, double gain,
                           const T *gain_vec, const T *offset_vec, hipStream_t st, const float *parts,
-                          int nparts, double scale) {
+                          int nparts, double scale, ChannelSave save) {
     if (N == 0 || C == 0) return hipSuccess;
     const int kk = k * k;
     if (hipError_t e = channel_branch_mma(pooled, w1, b1, w2, b2, cf, N, C, mid, k, gain, gain_vec,
-                                          offset_vec, st, parts, nparts, scale);
+                                          offset_vec, st, parts, nparts, scale, save);
         e != hipErrorNotSupported)
         return e;
     // (wide layers: fewer, larger blocks, as every block of a sample recomputes the hidden vector)
@@ -1264,7 +1295,7 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
 #define DDF_CHANNEL_LAUNCH(KK_, BLOCK_, NS_)                                                     \
     hipLaunchKernelGGL((k_channel_branch<T, KK_, BLOCK_, NS_>), grid, dim3(kChannelThreads), lds, \
                        st, pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain,    \
-                       gain_vec, offset_vec, parts, nparts, (float)scale)
+                       gain_vec, offset_vec, parts, nparts, (float)scale, save)
 #define DDF_CHANNEL_CASE(KK_, BLOCK_)                                                            \
     do {                                                                                         \
         if (ns == 4) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 4);                                         \
@@ -1284,10 +1315,10 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
 #define DDF_INSTANTIATE_BRANCHES(T)                                                              \
     template hipError_t spatial_branch<T>(const T *, const T *, const T *, T *, int64_t, int64_t, \
                                           int64_t, int64_t, int, int, int, double, const T *,    \
-                                          const T *, hipStream_t, float *, int64_t, int *);      \
+                                          const T *, hipStream_t, float *, int64_t, int *, T *); \
     template hipError_t channel_branch<T>(const T *, const T *, const T *, const T *, const T *, \
                                           T *, int64_t, int64_t, int64_t, int, double, const T *, \
-                                          const T *, hipStream_t, const float *, int, double);
+                                          const T *, hipStream_t, const float *, int, double, ChannelSave);
 DDF_INSTANTIATE_BRANCHES(__half)
 DDF_INSTANTIATE_BRANCHES(float)
 #undef DDF_INSTANTIATE_BRANCHES

@@ -93,6 +93,11 @@ hipError_t filter_norm_backward(const T *dy, const T *x, T *dx, T *terms, int64_
 // bottleneck MLP on the pooled features + channel filter normalisation.
 // hipErrorNotSupported: kernel size or sizes not covered, nothing launched.
 bool branch_kernel_size_built(int k);
+// What the channel branch leaves for its gradient (each may be null), fp32: the pooled
+// vectors (N, C), the hidden vectors behind the ReLU (N, mid) and the taps in front of the
+// normalisation (N, C * k*k), as the forward pass used them.
+struct ChannelSave { float *pooled = nullptr, *hidden = nullptr, *taps = nullptr; };
+// raw (may be null; with pool_part only): the taps in front of the normalisation.
 template <typename T>
 // pool_part (may be null): the launch also leaves the sums of the feature map over
 // the pixels of each of *pool_parts parts of a plane, fp32, [(n * parts + p) * C + c]; at most
@@ -101,14 +106,36 @@ hipError_t spatial_branch(const T *x, const T *w, const T *bias, T *sf, int64_t 
                           int64_t H, int64_t W, int head, int k, int stride, double gain,
                           const T *gain_vec, const T *offset_vec, hipStream_t st,
                           float *pool_part = nullptr, int64_t pool_capacity = 0,
-                          int *pool_parts = nullptr);
+                          int *pool_parts = nullptr, T *raw = nullptr);
 // parts (may be null): the pooled vectors are scale * the sums of nparts such partial
 // sums instead of `pooled`.
 template <typename T>
 hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2, const T *b2,
                           T *cf, int64_t N, int64_t C, int64_t mid, int k, double gain,
                           const T *gain_vec, const T *offset_vec, hipStream_t st,
-                          const float *parts = nullptr, int nparts = 0, double scale = 1.0);
+                          const float *parts = nullptr, int nparts = 0, double scale = 1.0,
+                          ChannelSave save = ChannelSave());
+
+// Gradients of both branches (ddf_pack_backward.hip; 3 x 3 taps): from dcf and draw (the
+// gradients of the channel filter and of the un-normalised spatial taps) and what the
+// forward pass saved, to every parameter's gradient (dbs, db1, db2 and dgain may be null)
+// and, unless dx is null, added to the operator's own feature gradient in dx.
+template <typename T>
+struct PackBackward {
+    const T *x, *dcf, *draw;
+    const float *pooled, *hidden, *taps;   // ChannelSave
+    const T *ws, *w1, *w2, *gain_vec;      // gain_vec null: the scalar gain
+    double gain;
+    T *dx, *dws, *dbs, *dw1, *db1, *dw2, *db2, *dgain;
+};
+// (sizes both halves cover: the forward launches that save for it, and pack_backward)
+bool pack_backward_supported(int64_t N, int64_t C, int64_t mid, int64_t H, int64_t W, int head, int k,
+                             int stride, int dtype);
+size_t pack_backward_workspace(int64_t N, int64_t C, int64_t mid, int64_t H, int64_t W, int head, int stride,
+                               int dtype);
+template <typename T>
+hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid,
+                         int head, int stride, void *ws, hipStream_t st);
 
 // All scale*scale sub-pixel branches of an up-sampling DDF in one launch,
 // written into the pixel-shuffled (N, C, H*scale, W*scale) result; cf / sf are

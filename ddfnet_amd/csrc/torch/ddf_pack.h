@@ -1,0 +1,250 @@
+// DDFPack (ddf/ddf.py:195-222 of the reference) as one native call: inference, and a
+// training step's forward as one autograd node whose backward runs the operator's gradient
+// kernels, the normalisation's and both branches'.  A layer made of torch modules issues
+// some thirty launches per training step, each through the interpreter, the dispatcher and
+// the convolution library: at ResNet-50's sizes a step was 0.7-0.8 ms of host time around
+// 0.2 ms of kernels.
+#pragma once
+
+#include "module_guard.h"
+
+#include <torch/csrc/autograd/functions/basic_ops.h>
+
+namespace ddf_torch {
+
+constexpr size_t kAlign = 256;
+inline size_t aligned_bytes(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
+
+// What a DDFPack is made of, collected once by DDFPack._native_plan in modules.py (which
+// has checked that both branches are the stock ones).
+struct PackPlan {
+    ModuleGuard guard;
+    // 1x1 convolutions (weight, bias): spatial branch, first and second of the channel branch
+    at::Tensor ws, bs, w1, b1, w2, b2;
+    // FilterNorm: learned gains and offsets, or the constant gain
+    c10::optional<at::Tensor> sgain_vec, soffset_vec, cgain_vec, coffset_vec;
+    double sgain, cgain;
+    int k, d, s, head, combine;
+    bool fuse_pool, fuse_norm;
+
+    PackPlan(py::list same, py::list empty, std::vector<at::Tensor> convs,
+             c10::optional<at::Tensor> sgain_vec_, c10::optional<at::Tensor> soffset_vec_,
+             c10::optional<at::Tensor> cgain_vec_, c10::optional<at::Tensor> coffset_vec_, double sgain_,
+             double cgain_, int k_, int d_, int s_, int head_, const std::string &combine_, bool fuse_pool_,
+             bool fuse_norm_)
+        : guard(std::move(same), std::move(empty)), sgain_vec(std::move(sgain_vec_)),
+          soffset_vec(std::move(soffset_vec_)), cgain_vec(std::move(cgain_vec_)),
+          coffset_vec(std::move(coffset_vec_)), sgain(sgain_), cgain(cgain_), k(k_), d(d_), s(s_), head(head_),
+          combine(combine_ == "add" ? DDF_ADD : DDF_MUL), fuse_pool(fuse_pool_), fuse_norm(fuse_norm_) {
+        TORCH_CHECK(convs.size() == 6, "six convolution tensors expected");
+        ws = convs[0]; bs = convs[1]; w1 = convs[2]; b1 = convs[3]; w2 = convs[4]; b2 = convs[5];
+    }
+    // Every tensor lives with the features, in their dtype, laid out densely.
+    bool fits(const at::Tensor &x) const {
+        const auto type = x.scalar_type();
+        const auto dev = x.device();
+        for (const at::Tensor *t : {&ws, &bs, &w1, &b1, &w2, &b2})
+            if (t->defined() && (t->scalar_type() != type || t->device() != dev || !t->is_contiguous())) return false;
+        for (const auto *t : {&sgain_vec, &soffset_vec, &cgain_vec, &coffset_vec})
+            if (t->has_value() && ((*t)->scalar_type() != type || (*t)->device() != dev || !(*t)->is_contiguous()))
+                return false;
+        const int64_t c = x.size(1), kk = (int64_t)k * k;
+        return ws.size(0) == head * kk && ws.size(1) == c && w1.size(1) == c && w2.size(0) == c * kk &&
+               w2.size(1) == w1.size(0) && c % head == 0;
+    }
+    bool wants_gradients(const at::Tensor &x) const {
+        if (x.requires_grad()) return true;
+        for (const at::Tensor *t : {&ws, &bs, &w1, &b1, &w2, &b2})
+            if (t->defined() && t->requires_grad()) return true;
+        for (const auto *t : {&sgain_vec, &soffset_vec, &cgain_vec, &coffset_vec})
+            if (t->has_value() && (*t)->requires_grad()) return true;
+        return false;
+    }
+};
+
+inline const void *ptr_or_null(const c10::optional<at::Tensor> &t) {
+    return t.has_value() && t->defined() ? t->data_ptr() : nullptr;
+}
+inline const void *ptr_or_null(const at::Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+// Without gradients: spatial branch (leaving the planes' partial sums where its kernel
+// can), channel branch, operator.
+inline at::Tensor pack_infer(const PackPlan &p, const at::Tensor &features) {
+    const int dt = dtype_code(features.scalar_type());
+    const at::Tensor x = features.contiguous();
+    const int64_t b = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3), mid = p.w1.size(0);
+    const int64_t ho = h / p.s, wo = w / p.s, kk = (int64_t)p.k * p.k;
+    c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+    hipStream_t st = current_stream(x);
+    at::Tensor out = at::empty({b, c, ho, wo}, x.options());
+    // both filters and the partial sums in one piece of scratch
+    const size_t esz = x.element_size();
+    const size_t cf_bytes = aligned_bytes(b * c * kk * esz), sf_bytes = aligned_bytes(b * p.head * kk * ho * wo * esz);
+    const int64_t cap = p.fuse_pool ? b * c * ((ho * wo + 63) / 64 + 1) : 0;
+    at::Tensor scratch = at::empty({(int64_t)(cf_bytes + sf_bytes + cap * sizeof(float))}, x.options().dtype(at::kByte));
+    char *base = static_cast<char *>(scratch.data_ptr());
+    void *cf = base, *sf = base + cf_bytes;
+    // The spatial branch reads every feature plane anyway: where its kernel can, it leaves
+    // the planes' partial sums and the channel branch pools from those (one launch and
+    // one read of the feature map fewer); else pool first.
+    bool pooled_on_the_way = false;
+    if (p.fuse_pool && b * c * ho * wo > 0) {
+        float *parts = reinterpret_cast<float *>(base + cf_bytes + sf_bytes);
+        int n_parts = 0;
+        const int rc = ddf_hip_spatial_branch_pool(
+            x.data_ptr(), p.ws.data_ptr(), ptr_or_null(p.bs), sf, parts, cap, &n_parts, b, c, h, w, p.head, p.k, p.s,
+            p.sgain, ptr_or_null(p.sgain_vec), ptr_or_null(p.soffset_vec), dt, st);
+        if (rc != DDF_ERR_UNSUPPORTED) {
+            check_status(rc);
+            check_status(ddf_hip_channel_branch_parts(
+                parts, n_parts, 1.0 / (double)(h * w), p.w1.data_ptr(), ptr_or_null(p.b1), p.w2.data_ptr(),
+                ptr_or_null(p.b2), cf, b, c, mid, p.k, p.cgain, ptr_or_null(p.cgain_vec),
+                ptr_or_null(p.coffset_vec), dt, st));
+            pooled_on_the_way = true;
+        }
+    }
+    if (!pooled_on_the_way) {
+        const at::Tensor pooled = at::mean(x, {2, 3});
+        check_status(ddf_hip_channel_branch(
+            pooled.data_ptr(), p.w1.data_ptr(), ptr_or_null(p.b1), p.w2.data_ptr(), ptr_or_null(p.b2), cf, b, c, mid,
+            p.k, p.cgain, ptr_or_null(p.cgain_vec), ptr_or_null(p.coffset_vec), dt, st));
+        check_status(ddf_hip_spatial_branch(
+            x.data_ptr(), p.ws.data_ptr(), ptr_or_null(p.bs), sf, b, c, h, w, p.head, p.k, p.s, p.sgain,
+            ptr_or_null(p.sgain_vec), ptr_or_null(p.soffset_vec), dt, st));
+    }
+    // heads are folded into the batch: (b * head, c / head, h, w)
+    check_status(ddf_hip_forward(x.data_ptr(), cf, sf, out.data_ptr(), b * p.head, c / p.head, h, w, p.k, p.d, p.s,
+                                 p.combine, dt, DDF_VARIANT_AUTO, st));
+    return out;
+}
+
+// A training step's layer.  What the backward pass wants of the forward (the filters, the
+// un-normalised taps, the pooled and hidden vectors) sits in one buffer:
+//   cf | sf | raw sf (features' dtype) | pooled | hidden | channel taps (fp32)
+struct PackSizes {
+    int64_t b, c, h, w, ho, wo, mid, kk;
+    size_t cf, sf, pooled, hidden, taps, saved;
+    PackSizes(const at::Tensor &x, int64_t mid_, int k, int s, int head) {
+        b = x.size(0); c = x.size(1); h = x.size(2); w = x.size(3);
+        ho = h / s; wo = w / s; mid = mid_; kk = (int64_t)k * k;
+        const size_t esz = x.element_size();
+        cf = aligned_bytes(b * c * kk * esz);
+        sf = aligned_bytes(b * head * kk * ho * wo * esz);
+        pooled = aligned_bytes(b * c * sizeof(float));
+        hidden = aligned_bytes(b * mid * sizeof(float));
+        taps = aligned_bytes(b * c * kk * sizeof(float));
+        saved = cf + 2 * sf + pooled + hidden + taps;
+    }
+};
+
+class PackAutograd : public torch::autograd::Function<PackAutograd> {
+public:
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x, const at::Tensor &ws, const at::Tensor &bs,
+                              const at::Tensor &w1, const at::Tensor &b1, const at::Tensor &w2, const at::Tensor &b2,
+                              const at::Tensor &gain_vec, double sgain, int64_t k, int64_t d, int64_t s,
+                              int64_t head, int64_t combine) {
+        const PackSizes z(x, w1.size(0), k, s, head);
+        const int dt = dtype_code(x.scalar_type());
+        c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+        hipStream_t st = current_stream(x);
+        at::Tensor out = at::empty({z.b, z.c, z.ho, z.wo}, x.options());
+        at::Tensor saved = at::empty({(int64_t)z.saved}, x.options().dtype(at::kByte));
+        const int64_t cap = z.b * z.c * ((z.ho * z.wo + 63) / 64 + 1);
+        at::Tensor parts = at::empty({cap}, x.options().dtype(at::kFloat));
+        char *q = static_cast<char *>(saved.data_ptr());
+        void *cf = q, *sf = q + z.cf, *raw = q + z.cf + z.sf;
+        float *pooled = reinterpret_cast<float *>(q + z.cf + 2 * z.sf);
+        float *hidden = pooled + z.pooled / sizeof(float), *taps = hidden + z.hidden / sizeof(float);
+        check_status(ddf_hip_pack_filters(x.data_ptr(), ws.data_ptr(), bs.data_ptr(), w1.data_ptr(), b1.data_ptr(),
+                                          w2.data_ptr(), b2.data_ptr(), raw, sf, cf, pooled, hidden, taps,
+                                          parts.data_ptr<float>(), cap, z.b, z.c, z.h, z.w, z.mid, (int)head, (int)k,
+                                          (int)s, sgain, 1.0, gain_vec.data_ptr(), dt, st));
+        check_status(ddf_hip_forward(x.data_ptr(), cf, sf, out.data_ptr(), z.b * head, z.c / head, z.h, z.w, (int)k,
+                                     (int)d, (int)s, (int)combine, dt, DDF_VARIANT_AUTO, st));
+        ctx->save_for_backward({x, ws, w1, w2, gain_vec, bs, b1, b2, saved});
+        ctx->saved_data["conf"] = std::vector<int64_t>{k, d, s, head, combine};
+        ctx->saved_data["sgain"] = sgain;
+        return out;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto sv = ctx->get_saved_variables();
+        const at::Tensor &x = sv[0], &ws = sv[1], &w1 = sv[2], &w2 = sv[3], &gain_vec = sv[4], &saved = sv[8];
+        const auto conf = ctx->saved_data["conf"].toIntVector();
+        const int k = (int)conf[0], d = (int)conf[1], s = (int)conf[2], head = (int)conf[3], combine = (int)conf[4];
+        const double sgain = ctx->saved_data["sgain"].toDouble();
+        const PackSizes z(x, w1.size(0), k, s, head);
+        const int dt = dtype_code(x.scalar_type());
+        const at::Tensor go = grads[0].to(x.scalar_type()).contiguous();
+        c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+        hipStream_t st = current_stream(x);
+        const bool want_dx = ctx->needs_input_grad(0);
+        const unsigned need = (want_dx ? DDF_NEED_DX : 0u) | DDF_NEED_DCF | DDF_NEED_DSF;
+        const int64_t n = z.b * head, cg = z.c / head;
+        const size_t op_bytes = aligned_bytes(ddf_hip_backward_spatial_norm_workspace_bytes(
+            n, cg, z.h, z.w, k, d, s, combine, dt, need, DDF_VARIANT_AUTO));
+        const size_t br_bytes = ddf_hip_pack_backward_workspace_bytes(z.b, z.c, z.h, z.w, z.mid, head, k, s, dt);
+        at::Tensor work = at::empty({(int64_t)(z.cf + z.sf + op_bytes + br_bytes)}, x.options().dtype(at::kByte));
+        char *wq = static_cast<char *>(work.data_ptr());
+        void *dcf = wq, *draw = wq + z.cf, *op_ws = wq + z.cf + z.sf, *br_ws = wq + z.cf + z.sf + op_bytes;
+        char *q = static_cast<char *>(saved.data_ptr());
+        void *cf = q, *sf = q + z.cf, *raw = q + z.cf + z.sf;
+        float *pooled = reinterpret_cast<float *>(q + z.cf + 2 * z.sf);
+        float *hidden = pooled + z.pooled / sizeof(float), *taps = hidden + z.hidden / sizeof(float);
+        at::Tensor dx;
+        if (want_dx) dx = at::empty_like(x);
+        at::Tensor dws = at::empty_like(ws), dw1 = at::empty_like(w1), dw2 = at::empty_like(w2),
+                   dgain = at::empty_like(gain_vec), dbs = at::empty_like(sv[5]), db1 = at::empty_like(sv[6]),
+                   db2 = at::empty_like(sv[7]);
+        void *dxp = want_dx ? dx.data_ptr() : nullptr;
+        check_status(ddf_hip_backward_spatial_norm(
+            go.data_ptr(), x.data_ptr(), cf, sf, raw, dxp, dcf, draw, nullptr, op_ws, op_bytes, n, cg, z.h, z.w, k, d,
+            s, combine, dt, need, head, sgain, nullptr, DDF_VARIANT_AUTO, st));
+        check_status(ddf_hip_pack_backward(
+            x.data_ptr(), dcf, draw, pooled, hidden, taps, ws.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+            gain_vec.data_ptr(), 1.0, dxp, dws.data_ptr(), dbs.data_ptr(), dw1.data_ptr(), db1.data_ptr(),
+            dw2.data_ptr(), db2.data_ptr(), dgain.data_ptr(), br_ws, br_bytes, z.b, z.c, z.h, z.w, z.mid, head, k, s,
+            dt, st));
+        variable_list out = {dx, dws, dbs, dw1, db1, dw2, db2, dgain};
+        if (at::GradMode::is_enabled()) {
+            // (create_graph: there is no second derivative; asking for one raises)
+            for (auto &t : out)
+                if (t.defined()) t.set_requires_grad(true);
+            auto node = std::make_shared<torch::autograd::DelayedError>(
+                "trying to differentiate twice a function that was marked with @once_differentiable",
+                (int64_t)out.size());
+            out = (*node)(std::move(out));
+        }
+        out.resize(14);
+        return out;
+    }
+};
+
+// DDFPack.forward through a plan: the result, or None where the plan does not (any longer)
+// describe the layer or the native path does not cover the call.
+inline py::object pack_forward(const PackPlan &p, const at::Tensor &x) {
+    if (!p.guard.holds() || !x.is_cuda() || x.dim() != 4) return py::none();
+    const int dt = dtype_code(x.scalar_type());
+    // (a size the stride does not divide fails in the layer's own code, as in the reference
+    // at ddf/ddf.py:215-218)
+    if ((dt != DDF_F16 && dt != DDF_F32) || x.size(2) % p.s || x.size(3) % p.s || !p.fits(x)) return py::none();
+    if (!(at::GradMode::is_enabled() && p.wants_gradients(x))) return py::cast(pack_infer(p, x));
+    // Training: the stock configuration only (constant spatial gain, learned channel gain, no
+    // offsets, biases present), everything trained.
+    if (!p.fuse_norm || p.sgain_vec || p.soffset_vec || p.coffset_vec || !p.cgain_vec) return py::none();
+    for (const at::Tensor *t : {&p.ws, &p.bs, &p.w1, &p.b1, &p.w2, &p.b2})
+        if (!t->defined() || !t->requires_grad()) return py::none();
+    if (!p.cgain_vec->requires_grad() || at::autocast::is_autocast_enabled(at::kCUDA)) return py::none();
+    if (x.numel() == 0) return py::none();
+    // (the streaming kernel's addresses: weights in whole words, features in whole vectors)
+    const bool covered =
+        reinterpret_cast<uintptr_t>(p.ws.data_ptr()) % 4 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+        ddf_hip_pack_backward_workspace_bytes(x.size(0), x.size(1), x.size(2), x.size(3), p.w1.size(0), p.head, p.k,
+                                              p.s, dt) > 0;
+    if (!covered) return py::none();
+    return py::cast(PackAutograd::apply(x.contiguous(), p.ws, p.bs, p.w1, p.b1, p.w2, p.b2, *p.cgain_vec, p.sgain,
+                                        (int64_t)p.k, (int64_t)p.d, (int64_t)p.s, (int64_t)p.head,
+                                        (int64_t)p.combine));
+}
+
+}  // namespace ddf_torch

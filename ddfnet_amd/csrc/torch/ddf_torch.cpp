@@ -18,7 +18,7 @@
 
 #include "ddf_hip.h"
 
-namespace {
+namespace ddf_torch {
 
 namespace py = pybind11;
 using torch::autograd::AutogradContext;
@@ -26,14 +26,14 @@ using torch::autograd::variable_list;
 
 // `assert cond, msg` of the Python front end.
 // (Also reached from the autograd engine's threads, which do not hold the GIL.)
-[[noreturn]] void assertion_error(const std::string &msg) {
+[[noreturn]] inline void assertion_error(const std::string &msg) {
     py::gil_scoped_acquire gil;
     PyErr_SetString(PyExc_AssertionError, msg.c_str());
     throw py::error_already_set();
 }
 
 // A failed library call, raised as ddfnet_amd._lib.DDFHipError.
-void check_status(int status) {
+inline void check_status(int status) {
     if (status == DDF_OK) return;
     const std::string msg = std::string(ddf_hip_status_string(status)) + ": " + ddf_hip_last_error();
     py::gil_scoped_acquire gil;
@@ -42,7 +42,7 @@ void check_status(int status) {
     throw py::error_already_set();
 }
 
-int dtype_code(at::ScalarType t) {
+inline int dtype_code(at::ScalarType t) {
     switch (t) {
         case at::kHalf: return DDF_F16;
         case at::kFloat: return DDF_F32;
@@ -60,7 +60,7 @@ std::string size_string(const at::Tensor &t) {
     return os.str();
 }
 
-hipStream_t current_stream(const at::Tensor &t) {
+inline hipStream_t current_stream(const at::Tensor &t) {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
@@ -339,91 +339,12 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
                                 (int64_t)combine);
 }
 
-const void *ptr_or_null(const c10::optional<at::Tensor> &t) {
-    return t.has_value() && t->defined() ? t->data_ptr() : nullptr;
-}
+}  // namespace ddf_torch
 
-// DDFPack.forward without gradients (ddf/ddf.py:195-222 of the reference), four
-// launches: global average pool (torch), channel branch, spatial branch, operator.
-// The caller (DDFPack._inference_forward in modules.py) has checked that the
-// branches are the stock ones and that every tensor is a device tensor of the
-// features' dtype; weights are the 1x1 convolutions' (out, in, 1, 1) tensors.
-at::Tensor ddf_pack_forward(const at::Tensor &features, const at::Tensor &conv_weight,
-                            const c10::optional<at::Tensor> &conv_bias, double spatial_gain,
-                            const c10::optional<at::Tensor> &spatial_gain_vec,
-                            const c10::optional<at::Tensor> &spatial_offset_vec,
-                            const at::Tensor &fc1_weight, const c10::optional<at::Tensor> &fc1_bias,
-                            const at::Tensor &fc2_weight, const c10::optional<at::Tensor> &fc2_bias,
-                            double channel_gain, const c10::optional<at::Tensor> &channel_gain_vec,
-                            const c10::optional<at::Tensor> &channel_offset_vec,
-                            int64_t kernel_size, int64_t dilation, int64_t stride, int64_t head,
-                            const std::string &kernel_combine, bool fuse_pool) {
-    TORCH_CHECK(features.is_cuda() && features.dim() == 4, "features must be a 4-d device tensor");
-    const int dt = dtype_code(features.scalar_type());
-    TORCH_CHECK(dt == DDF_F16 || dt == DDF_F32, "ddf_pack_forward covers fp16 and fp32");
-    int combine;
-    if (kernel_combine == "mul") combine = DDF_MUL;
-    else if (kernel_combine == "add") combine = DDF_ADD;
-    else assertion_error("only support mul or add combination, instead of " + kernel_combine);
-    const at::Tensor x = features.contiguous();
-    const int64_t b = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3);
-    const int64_t ho = h / stride, wo = w / stride, kk = kernel_size * kernel_size;
-    TORCH_CHECK(head >= 1 && c % head == 0, "channels must divide into heads");
-    TORCH_CHECK(conv_weight.is_contiguous() && fc1_weight.is_contiguous() && fc2_weight.is_contiguous(),
-                "weights must be contiguous");
-    TORCH_CHECK(conv_weight.size(0) == head * kk && conv_weight.size(1) == c &&
-                fc1_weight.size(1) == c && fc2_weight.size(0) == c * kk &&
-                fc2_weight.size(1) == fc1_weight.size(0), "branch weights do not fit the features");
-    const int64_t mid = fc1_weight.size(0);
-
-    c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
-    hipStream_t st = current_stream(x);
-    at::Tensor cf = at::empty({b, c, kernel_size, kernel_size}, x.options());
-    at::Tensor sf = at::empty({b, head * kk, ho, wo}, x.options());
-    // The spatial branch reads every feature plane anyway: where its kernel can, it leaves
-    // the planes' partial sums and the channel branch pools from those (one launch and
-    // one read of the feature map fewer); else pool first.
-    bool pooled_on_the_way = false;
-    if (fuse_pool && b * c * ho * wo > 0) {
-        const int64_t cap = b * c * ((ho * wo + 63) / 64) * 4;
-        at::Tensor parts = at::empty({cap}, x.options().dtype(at::kFloat));
-        int n_parts = 0;
-        const int rc = ddf_hip_spatial_branch_pool(
-            x.data_ptr(), conv_weight.data_ptr(), ptr_or_null(conv_bias), sf.data_ptr(),
-            parts.data_ptr<float>(), cap, &n_parts, b, c, h, w, (int)head, (int)kernel_size, (int)stride,
-            spatial_gain, ptr_or_null(spatial_gain_vec), ptr_or_null(spatial_offset_vec), dt, st);
-        if (rc != DDF_ERR_UNSUPPORTED) {
-            check_status(rc);
-            check_status(ddf_hip_channel_branch_parts(
-                parts.data_ptr<float>(), n_parts, 1.0 / (double)(h * w), fc1_weight.data_ptr(),
-                ptr_or_null(fc1_bias), fc2_weight.data_ptr(), ptr_or_null(fc2_bias), cf.data_ptr(), b, c, mid,
-                (int)kernel_size, channel_gain, ptr_or_null(channel_gain_vec),
-                ptr_or_null(channel_offset_vec), dt, st));
-            pooled_on_the_way = true;
-        }
-    }
-    if (!pooled_on_the_way) {
-        const at::Tensor pooled = at::mean(x, {2, 3});
-        check_status(ddf_hip_channel_branch(
-            pooled.data_ptr(), fc1_weight.data_ptr(), ptr_or_null(fc1_bias), fc2_weight.data_ptr(),
-            ptr_or_null(fc2_bias), cf.data_ptr(), b, c, mid, (int)kernel_size, channel_gain,
-            ptr_or_null(channel_gain_vec), ptr_or_null(channel_offset_vec), dt, st));
-        check_status(ddf_hip_spatial_branch(
-            x.data_ptr(), conv_weight.data_ptr(), ptr_or_null(conv_bias), sf.data_ptr(), b, c, h, w,
-            (int)head, (int)kernel_size, (int)stride, spatial_gain, ptr_or_null(spatial_gain_vec),
-            ptr_or_null(spatial_offset_vec), dt, st));
-    }
-    at::Tensor out = at::empty({b, c, ho, wo}, x.options());
-    // heads are folded into the batch: (b * head, c / head, h, w)
-    check_status(ddf_hip_forward(x.data_ptr(), cf.data_ptr(), sf.data_ptr(), out.data_ptr(), b * head,
-                                 c / head, h, w, (int)kernel_size, (int)dilation, (int)stride, combine,
-                                 dt, DDF_VARIANT_AUTO, st));
-    return out;
-}
-
-}  // namespace
+#include "ddf_pack.h"
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    using namespace ddf_torch;
     m.doc() = "ddf operator of libddf_hip.so as a C++ autograd function";
     m.def("ddf", &ddf, py::arg("features"), py::arg("channel_filter"), py::arg("spatial_filter"),
           py::arg("kernel_size") = 3, py::arg("dilation") = 1, py::arg("stride") = 1,
@@ -431,7 +352,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("ddf_up", &ddf_up, py::arg("features"), py::arg("channel_filters"),
           py::arg("spatial_filters"), py::arg("kernel_size") = 3, py::arg("dilation") = 1,
           py::arg("scale_factor") = 2, py::arg("kernel_combine") = "mul");
-    m.def("ddf_pack_forward", &ddf_pack_forward,
+    py::class_<PackPlan>(m, "PackPlan")
+        .def(py::init<py::list, py::list, std::vector<at::Tensor>, c10::optional<at::Tensor>,
+                      c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>, double, double,
+                      int, int, int, int, const std::string &, bool, bool>())
+        .def("valid", [](const PackPlan &p) { return p.guard.holds(); });
+    m.def("pack_forward", &pack_forward, "DDFPack.forward through a plan, or None");
+    m.def("pack_infer", &pack_infer,
           "DDFPack.forward without gradients: spatial branch (pooling on the way where it can), "
           "channel branch, operator");
     m.def("library_version", []() { return ddf_hip_version(); });

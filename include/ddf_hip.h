@@ -310,6 +310,43 @@ int ddf_hip_channel_branch_parts(const float *pool_parts, int n_parts,
                                  int dtype, void *stream);
 
 /*
+ * Training of DDFPack's filter branches (3 x 3 taps).
+ * ddf_hip_pack_filters is the two branch calls above, pooling on the way, that also leave
+ * what the gradients need: `raw_spatial_filter` (the spatial taps in front of their
+ * normalisation, shaped and typed like `spatial_filter`) and, fp32, `pooled` (N, C),
+ * `hidden` (N, mid; behind the ReLU) and `channel_taps` (N, C * k*k; in front of the
+ * normalisation).  `pool_parts` is scratch of pool_capacity floats as in
+ * ddf_hip_spatial_branch_pool.
+ * ddf_hip_pack_backward is what autograd derives in the reference from
+ * build_spatial_branch and build_channel_branch (ddf/ddf.py:176-192): given
+ * `grad_channel_filter` and `grad_raw_spatial_filter` (ddf_hip_backward_spatial_norm), it
+ * writes the gradients of the branches' parameters (any of the biases' and gains' may be
+ * NULL) and adds the branches' part of the feature gradient to `grad_features`, which
+ * holds the operator's (NULL: not wanted).  `workspace`:
+ * ddf_hip_pack_backward_workspace_bytes(...) bytes, 256-byte aligned; that function
+ * returns 0 where the two calls do not cover the layer (kernel size other than 3, fp64,
+ * heads other than 1, 2 and 4, strides other than 1 and 2).
+ */
+int ddf_hip_pack_filters(const void *features, const void *spatial_weight, const void *spatial_bias,
+                         const void *weight1, const void *bias1, const void *weight2, const void *bias2,
+                         void *raw_spatial_filter, void *spatial_filter, void *channel_filter,
+                         float *pooled, float *hidden, float *channel_taps, float *pool_parts,
+                         int64_t pool_capacity, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid,
+                         int head, int kernel_size, int stride, double spatial_gain, double channel_gain,
+                         const void *channel_gain_vec, int dtype, void *stream);
+size_t ddf_hip_pack_backward_workspace_bytes(int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid, int head,
+                                             int kernel_size, int stride, int dtype);
+int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
+                          const void *grad_raw_spatial_filter, const float *pooled, const float *hidden,
+                          const float *channel_taps, const void *spatial_weight, const void *weight1,
+                          const void *weight2, const void *channel_gain_vec, double channel_gain,
+                          void *grad_features, void *grad_spatial_weight, void *grad_spatial_bias,
+                          void *grad_weight1, void *grad_bias1, void *grad_weight2, void *grad_bias2,
+                          void *grad_channel_gain, void *workspace, size_t workspace_bytes, int64_t N,
+                          int64_t C, int64_t H, int64_t W, int64_t mid, int head, int kernel_size, int stride,
+                          int dtype, void *stream);
+
+/*
  * Up-sampling DDF forward (DDFUpPack.forward, ddf/ddf.py:257-272): the
  * reference calls `ddf` once per sub-pixel branch b = 0 .. scale*scale-1 on
  * the same features with that branch's filters (ddf.py:264-269), stacks the
