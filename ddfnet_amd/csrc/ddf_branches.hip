@@ -1074,7 +1074,12 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     const int vp_max = (stride == 1 ? 16 : 8) / esz;
     // ... that still leaves enough waves to fill the machine: the waves of a workgroup
     // share its pixels and split the channels, at least two pipeline rounds each
-    const int64_t want = tune_int("DDF_TUNE_SPATIAL_WANT", 2048);
+    // (measured over batches of 1 to 128, 7 x 7 to 200 x 300, 64 to 512 channels: 1 280 waves
+    // are enough at four or eight pixels per lane, and single-pixel loads only pay where two
+    // pixels per lane leave fewer than 448 - 64 x 128 x 56 x 56 fp16 under stride 2 took
+    // 23.7 us at one pixel and takes 15.3 at two, 16 x 128 x 28 x 28 8.5 and 6.5)
+    auto enough = [](int vp) { return vp == 2 ? 448 : 1280; };
+    const int64_t want = 2048;
     int vp = 0, waves = 1;
     for (int cand = vp_max; cand >= 1; cand /= 2) {
         if (!fits(cand)) continue;
@@ -1087,7 +1092,7 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
                 wv *= 2;
         vp = cand;
         waves = wv;
-        if (tiles * wv >= want || wv == 1) break;
+        if (tiles * wv >= enough(cand) || wv == 1) break;
     }
     const int fvp = tune_int("DDF_TUNE_SPATIAL_VP", 0), fwv = tune_int("DDF_TUNE_SPATIAL_WAVES", 0);
     if (fvp > 0 && fvp <= vp_max && fits(fvp)) vp = fvp;

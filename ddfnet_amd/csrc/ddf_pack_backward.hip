@@ -39,12 +39,13 @@ struct PackDims {
 };
 
 // ---- second convolution of the channel branch --------------------------------
-// A workgroup takes kFc2Channels channels (72 rows of W2) and 64 hidden values, a lane one
-// hidden value; samples come in chunks through LDS.  dW2: every wave owns 18 of the rows and
-// reads their dZ2 as LDS broadcasts; dh: every wave owns every fourth sample, with the
-// lane's column of the 72 rows of W2 in registers.
-constexpr int kFc2Channels = 8, kFc2Rows = kFc2Channels * KK, kFc2Samples = kThreads / kFc2Channels;
-constexpr int kFc2RowsPerWave = kFc2Rows / kWaves;
+// A workgroup takes kFc2Channels channels (36 rows of W2) and 64 hidden values, a lane one
+// hidden value; samples come in chunks of 64 through LDS.  dW2: every wave owns one channel's
+// rows and reads their dZ2 as LDS broadcasts; dh: every wave owns every fourth sample, with
+// the lane's column of the 36 rows of W2 in registers.  (Eight channels and chunks of 32
+// samples: 22.8 us at 64 x 128 where this takes 13.)
+constexpr int kFc2Channels = kWaves, kFc2Rows = kFc2Channels * KK, kFc2Samples = kThreads / kFc2Channels;
+constexpr int kFc2Pitch = 12;    // a channel's nine values, 16-byte rows
 
 template <typename T>
 struct Fc2Args {
@@ -57,7 +58,7 @@ struct Fc2Args {
 };
 
 struct Fc2Smem {
-    float dz[kFc2Samples][kFc2Rows];
+    float dz[kFc2Samples][kFc2Channels][kFc2Pitch];
     float dg[kFc2Samples][kFc2Rows];
     float h[kFc2Samples][kWave];
 };
@@ -75,9 +76,9 @@ __device__ __forceinline__ void fc2_block(const PackDims &d, const Fc2Args<T> &a
     float w2[kFc2Rows];
 #pragma unroll
     for (int r = 0; r < kFc2Rows; ++r) w2[r] = ld(a.w2 + ((int64_t)cb * KK + min(r, rows - 1)) * d.mid + mc);
-    float acc[kFc2RowsPerWave];
+    float acc[KK];
 #pragma unroll
-    for (int q = 0; q < kFc2RowsPerWave; ++q) acc[q] = 0.f;
+    for (int t = 0; t < KK; ++t) acc[t] = 0.f;
     float col_sum = 0.f;
     const int item_n = threadIdx.x / kFc2Channels, item_c = threadIdx.x % kFc2Channels;
     for (int n0 = 0; n0 < d.N; n0 += kFc2Samples) {
@@ -119,7 +120,7 @@ __device__ __forceinline__ void fc2_block(const PackDims &d, const Fc2Args<T> &a
             }
 #pragma unroll
             for (int t = 0; t < KK; ++t) {
-                sm.dz[item_n][item_c * KK + t] = dz[t];
+                sm.dz[item_n][item_c][t] = dz[t];
                 sm.dg[item_n][item_c * KK + t] = dg[t];
             }
         }
@@ -128,32 +129,35 @@ __device__ __forceinline__ void fc2_block(const PackDims &d, const Fc2Args<T> &a
             sm.h[i][mm] = (i < cnt && m0 + mm < d.mid) ? a.hidden[(int64_t)(n0 + i) * d.mid + m0 + mm] : 0.f;
         }
         __syncthreads();
-#pragma unroll 2
+#pragma unroll 4
         for (int i = 0; i < cnt; ++i) {
             const float hv = sm.h[i][lane];
 #pragma unroll
-            for (int q = 0; q < kFc2RowsPerWave; ++q)
-                acc[q] = fmaf(sm.dz[i][wave * kFc2RowsPerWave + q], hv, acc[q]);
+            for (int t = 0; t < KK; ++t) acc[t] = fmaf(sm.dz[i][wave][t], hv, acc[t]);
         }
+#pragma unroll 2
         for (int i = wave; i < cnt; i += kWaves) {
-            float p[4] = {0.f, 0.f, 0.f, 0.f};
+            float p[kFc2Channels];
 #pragma unroll
-            for (int r = 0; r < kFc2Rows; ++r) p[r & 3] = fmaf(sm.dz[i][r], w2[r], p[r & 3]);
+            for (int c = 0; c < kFc2Channels; ++c) {
+                p[c] = 0.f;
+#pragma unroll
+                for (int t = 0; t < KK; ++t) p[c] = fmaf(sm.dz[i][c][t], w2[c * KK + t], p[c]);
+            }
             if (mok) a.dh_part[((int64_t)blk * d.N + n0 + i) * d.mid + m] = (p[0] + p[1]) + (p[2] + p[3]);
         }
         if (m0 == 0 && threadIdx.x < 2 * kFc2Rows) {
-            const int col = threadIdx.x < kFc2Rows ? threadIdx.x : threadIdx.x - kFc2Rows;
-            const float(*src)[kFc2Rows] = threadIdx.x < kFc2Rows ? sm.dz : sm.dg;
+            const bool gain = threadIdx.x >= kFc2Rows;
+            const int col = gain ? threadIdx.x - kFc2Rows : threadIdx.x;
+            const float *src = gain ? &sm.dg[0][col] : &sm.dz[0][col / KK][col % KK];
+            const int pitch = gain ? kFc2Rows : kFc2Channels * kFc2Pitch;
 #pragma unroll 8
-            for (int i = 0; i < cnt; ++i) col_sum += src[i][col];
+            for (int i = 0; i < cnt; ++i) col_sum += src[i * pitch];
         }
     }
-    if (mok) {
+    if (mok && cb + wave < d.C) {
 #pragma unroll
-        for (int q = 0; q < kFc2RowsPerWave; ++q) {
-            const int r = wave * kFc2RowsPerWave + q;
-            if (r < rows) st(a.dw2 + ((int64_t)cb * KK + r) * d.mid + m, acc[q]);
-        }
+        for (int t = 0; t < KK; ++t) st(a.dw2 + ((int64_t)(cb + wave) * KK + t) * d.mid + m, acc[t]);
     }
     if (m0 == 0) {
         const int r = threadIdx.x;
@@ -321,8 +325,9 @@ __global__ __launch_bounds__(kThreads) void k_pack_hidden(PackDims d, const floa
 }
 
 // ---- first convolution of the channel branch ----------------------------------
-// Lanes are channels.  dW1: a wave takes kFc1 rows of W1 and all samples; dv: kFc1 samples
-// and all rows.  The other factor, dz1, is the same for every lane.
+// Lanes are channels.  dW1: a workgroup takes kFc1 rows of W1, its waves a quarter of the
+// samples each; dv: kFc1 samples and a quarter of the rows per wave.  The other factor, dz1,
+// is the same for every lane.
 constexpr int kFc1 = 4;
 
 template <typename T>
@@ -331,49 +336,63 @@ __global__ __launch_bounds__(kThreads) void k_pack_fc1(PackDims d, const float *
                                                        const T *__restrict__ w1, T *__restrict__ dw1,
                                                        T *__restrict__ db1, float *__restrict__ dv, int cblks,
                                                        int mblks) {
+    __shared__ float red[kWaves][2 * kFc1][kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int cblk = blockIdx.x % cblks, rest = blockIdx.x / cblks;
     const int c = cblk * kWave + lane;
     const int cc = min(c, d.C - 1);
-    float acc[kFc1];
+    const bool weights = rest < mblks;
+    const int q0 = (weights ? rest : rest - mblks) * kFc1;       // first hidden value / sample
+    const int summed = weights ? d.N : d.mid;
+    const int per = (summed + kWaves - 1) / kWaves;
+    const int i0 = wave * per, i1 = min(i0 + per, summed);
+    float acc[kFc1], bsum[kFc1];
 #pragma unroll
-    for (int q = 0; q < kFc1; ++q) acc[q] = 0.f;
-    if (rest < mblks) {
-        const int m0 = (rest * kWaves + wave) * kFc1;
-        if (m0 >= d.mid) return;
-        float bsum[kFc1] = {};
+    for (int q = 0; q < kFc1; ++q) acc[q] = bsum[q] = 0.f;
+    if (weights) {
 #pragma unroll 8
-        for (int n = 0; n < d.N; ++n) {
+        for (int n = i0; n < i1; ++n) {
             const float p = pooled[(int64_t)n * d.C + cc];
 #pragma unroll
             for (int q = 0; q < kFc1; ++q) {
-                const float z = dz1[(int64_t)n * d.mid + min(m0 + q, d.mid - 1)];
+                const float z = dz1[(int64_t)n * d.mid + min(q0 + q, d.mid - 1)];
                 acc[q] = fmaf(z, p, acc[q]);
                 bsum[q] += z;
             }
         }
-#pragma unroll
-        for (int q = 0; q < kFc1; ++q) {
-            if (m0 + q >= d.mid) break;
-            if (c < d.C) st(dw1 + (int64_t)(m0 + q) * d.C + c, acc[q]);
-            if (db1 && cblk == 0 && lane == 0) st(db1 + m0 + q, bsum[q]);
-        }
     } else {
-        const int n0 = ((rest - mblks) * kWaves + wave) * kFc1;
-        if (n0 >= d.N) return;
 #pragma unroll 8
-        for (int m = 0; m < d.mid; ++m) {
+        for (int m = i0; m < i1; ++m) {
             const float wv = ld(w1 + (int64_t)m * d.C + cc);
 #pragma unroll
             for (int q = 0; q < kFc1; ++q)
-                acc[q] = fmaf(dz1[(int64_t)min(n0 + q, d.N - 1) * d.mid + m], wv, acc[q]);
+                acc[q] = fmaf(dz1[(int64_t)min(q0 + q, d.N - 1) * d.mid + m], wv, acc[q]);
         }
+    }
 #pragma unroll
-        for (int q = 0; q < kFc1; ++q)
-            if (n0 + q < d.N && c < d.C) dv[(int64_t)(n0 + q) * d.C + c] = acc[q];
+    for (int q = 0; q < kFc1; ++q) {
+        red[wave][q][lane] = acc[q];
+        red[wave][kFc1 + q][lane] = bsum[q];
+    }
+    __syncthreads();
+    // (wave q finishes output q)
+    const int q = q0 + wave;
+    float tot = 0.f, btot = 0.f;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+        tot += red[k][wave][lane];
+        btot += red[k][kFc1 + wave][lane];
+    }
+    if (weights) {
+        if (q >= d.mid) return;
+        if (c < d.C) st(dw1 + (int64_t)q * d.C + c, tot);
+        if (db1 && cblk == 0 && lane == 0) st(db1 + q, btot);
+    } else if (q < d.N && c < d.C) {
+        dv[(int64_t)q * d.C + c] = tot;
     }
 }
+static_assert(kFc1 == kWaves, "a wave finishes one output");
 
 // ---- feature gradient ----------------------------------------------------------
 // A lane owns VP neighbouring pixels of a sample and keeps the spatial branch's tap
@@ -524,8 +543,8 @@ hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t
     hipLaunchKernelGGL((k_pack_hidden<T>), dim3((unsigned)(hid_blocks + cdiv((int64_t)head * KK * (C + 1), kSumCols))),
                        dim3(kThreads), 0, st, d, dh_part, b.hidden, dz1, cblocks, hid_blocks, ws_part,
                        (int)(N * splits), b.dws, b.dbs);
-    const int cblks = (int)cdiv(C, kWave), mblks = (int)cdiv(mid, kWaves * kFc1);
-    const int nblks = b.dx ? (int)cdiv(N, kWaves * kFc1) : 0;
+    const int cblks = (int)cdiv(C, kWave), mblks = (int)cdiv(mid, kFc1);
+    const int nblks = b.dx ? (int)cdiv(N, kFc1) : 0;
     hipLaunchKernelGGL((k_pack_fc1<T>), dim3((unsigned)(cblks * (mblks + nblks))), dim3(kThreads), 0, st, d, dz1,
                        b.pooled, b.w1, b.dw1, b.db1, dv, cblks, mblks);
     if (b.dx) {
