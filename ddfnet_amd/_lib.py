@@ -49,6 +49,11 @@ SYMBOLS = {
     'ddf_hip_pack_backward_workspace_bytes': (_sz, [_i64] * 5 + [_i] * 4),
     'ddf_hip_pack_backward': (_i, [_vp] * 10 + [ctypes.c_double] + [_vp] * 9 + [_sz] + [_i64] * 5 + [_i] * 4 +
                               [_vp]),
+    'ddf_hip_net_conv': (_i, [_vp] * 5 + [_i64] * 5 + [_i] * 2 + [_vp]),
+    'ddf_hip_net_stem': (_i, [_vp] * 4 + [_i64] * 3 + [_vp]),
+    'ddf_hip_net_spatial': (_i, [_vp] * 5 + [ctypes.POINTER(ctypes.c_int)] + [_i64] * 4 + [_i, ctypes.c_double, _vp]),
+    'ddf_hip_net_filter': (_i, [_vp] * 5 + [_i64] * 4 + [_i] * 2 + [_vp]),
+    'ddf_hip_net_pool': (_i, [_vp] * 2 + [_i64] * 3 + [_vp]),
     'ddf_hip_up_forward': (_i, [_vp] * 4 + [_i64] * 4 + [_i] * 5 + [_vp]),
     'ddf_hip_up_backward_workspace_bytes': (_sz, [_i64] * 4 + [_i] * 5 + [_u]),
     'ddf_hip_up_backward': (_i, [_vp] * 8 + [_sz] + [_i64] * 4 + [_i] * 5 + [_u, _vp]),

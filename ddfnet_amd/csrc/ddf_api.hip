@@ -738,6 +738,71 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
 #undef DDF_PACK_CASE
 }
 
+namespace {
+ddf::NetNorm net_norm(const ddf_net_norm_t *n) {
+    return n ? ddf::NetNorm{n->weight, n->bias, n->running_mean, n->running_var, n->conv_bias, n->eps}
+             : ddf::NetNorm{nullptr, nullptr, nullptr, nullptr, nullptr, 0.f};
+}
+int net_result(hipError_t err, const char *what) {
+    if (err == hipErrorNotSupported) return fail(DDF_ERR_UNSUPPORTED, "%s: sizes not covered", what);
+    return err == hipSuccess ? DDF_OK : fail_hip(err, what);
+}
+bool net_norm_ok(const ddf_net_norm_t *n) {
+    return !n || !n->running_var || (n->weight && n->bias && n->running_mean);
+}
+}  // namespace
+
+int ddf_hip_net_conv(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
+                     void *output, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int stride, int relu,
+                     void *stream) {
+    if (N < 0 || H < 1 || W < 1 || C < 1 || O < 1 || stride < 1 || C > (1 << 24) || O > (1 << 24) || H * W >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_conv: bad sizes");
+    if (!features || !weight || !output || !net_norm_ok(norm)) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    const int64_t Ho = (H - 1) / stride + 1, Wo = (W - 1) / stride + 1;
+    const ddf::NetConv a{features, weight, residual, output, net_norm(norm), N * Ho * Wo, (int)O, (int)C, relu,
+                         stride, (int)H, (int)W, (int)Wo, (int)(Ho * Wo)};
+    return net_result(ddf::net_conv(a, (hipStream_t)stream), "ddf_hip_net_conv launch");
+}
+
+int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,
+                     int64_t H, int64_t W, void *stream) {
+    if (N < 0 || H < 1 || W < 1) return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_stem: bad sizes");
+    if (!image || !weight || !output || !net_norm_ok(norm)) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    return net_result(ddf::net_stem(image, weight, net_norm(norm), output, N, H, W, (hipStream_t)stream),
+                      "ddf_hip_net_stem launch");
+}
+
+int ddf_hip_net_spatial(const void *features, const void *weight, const void *bias, void *spatial_filter,
+                        float *pool_parts, int *n_parts, int64_t N, int64_t H, int64_t W, int64_t C, int stride,
+                        double gain, void *stream) {
+    if (N < 1 || H < 1 || W < 1 || C < 1 || stride < 1 || H / stride < 1 || W / stride < 1)
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_spatial: bad sizes");
+    if (!features || !weight || !spatial_filter || !pool_parts || !n_parts)
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    return net_result(ddf::net_spatial(features, weight, bias, spatial_filter, pool_parts, n_parts, N, H, W, C, stride,
+                                       gain, (hipStream_t)stream),
+                      "ddf_hip_net_spatial launch");
+}
+
+int ddf_hip_net_filter(const void *features, const void *channel_filter, const void *spatial_filter,
+                       const ddf_net_norm_t *norm, void *output, int64_t N, int64_t H, int64_t W, int64_t C,
+                       int stride, int combine, void *stream) {
+    if (N < 0 || H < 1 || W < 1 || C < 1 || stride < 1 || (combine != DDF_MUL && combine != DDF_ADD))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_filter: bad sizes");
+    if (!features || !channel_filter || !spatial_filter || !output || !net_norm_ok(norm))
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    return net_result(ddf::net_filter(features, channel_filter, spatial_filter, net_norm(norm), output, N, H, W, C,
+                                      stride, combine == DDF_MUL, (hipStream_t)stream),
+                      "ddf_hip_net_filter launch");
+}
+
+int ddf_hip_net_pool(const void *features, void *output, int64_t N, int64_t pixels, int64_t C, void *stream) {
+    if (N < 0 || pixels < 1 || C < 1 || C > (1 << 24) || pixels >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_pool: bad sizes");
+    if (!features || !output) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    return net_result(ddf::net_pool(features, output, N, pixels, C, (hipStream_t)stream), "ddf_hip_net_pool launch");
+}
+
 int ddf_hip_up_forward(const void *features, const void *const *channel_filters,
                        const void *const *spatial_filters, void *output, int64_t N, int64_t C,
                        int64_t H, int64_t W, int kernel_size, int dilation, int scale,

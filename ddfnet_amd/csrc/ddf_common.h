@@ -137,6 +137,33 @@ template <typename T>
 hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid,
                          int head, int stride, void *ws, hipStream_t st);
 
+// Channels-last fp16 kernels of the DDF-ResNets' inference (ddf_net.hip).
+// The per-channel affine map behind a convolution: its bias and the BatchNorm (eval mode)
+// that follows; null pointers: absent (var null: no BatchNorm).
+struct NetNorm {
+    const void *weight, *bias, *mean, *var, *conv_bias;
+    float eps;
+};
+// out (M, N) = act(norm(x (rows of K) . w (N, K)) + res (M, N)); stride > 1: row m of x is the
+// pixel of an (n, H, W) batch that result m = (n, y, x) of npix = Ho * Wo samples.
+struct NetConv {
+    const void *x, *w, *res;
+    void *out;
+    NetNorm norm;
+    int64_t M;
+    int N, K, relu, stride, H, W, Wo, npix;
+};
+bool net_conv_supported(const NetConv &a);
+hipError_t net_conv(const NetConv &a, hipStream_t st);
+hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,
+                    hipStream_t st);
+int net_spatial_chunks(int64_t N, int64_t npix);
+hipError_t net_spatial(const void *x, const void *w, const void *bias, void *sf, float *parts, int *n_parts, int64_t N,
+                       int64_t H, int64_t W, int64_t C, int stride, double gain, hipStream_t st);
+hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNorm &norm, void *out, int64_t N,
+                      int64_t H, int64_t W, int64_t C, int stride, bool mul, hipStream_t st);
+hipError_t net_pool(const void *x, void *out, int64_t N, int64_t plane, int64_t C, hipStream_t st);
+
 // All scale*scale sub-pixel branches of an up-sampling DDF in one launch,
 // written into the pixel-shuffled (N, C, H*scale, W*scale) result; cf / sf are
 // host arrays of scale*scale device pointers.

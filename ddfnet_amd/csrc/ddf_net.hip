@@ -1,0 +1,835 @@
+// DDF-ResNet inference in fp16 with channels-last activations (gfx950).
+//
+// Between the image and the logits a network is its own world: its activations have no
+// layout anybody else sees.  Here they are (N, H, W, C): a 1x1 convolution is then a
+// product of two row-major matrices whose summed dimension is contiguous in both, which is
+// what the matrix cores read; a lane of the dynamic filter owns eight channels of a pixel
+// and its neighbours are whole vectors, whatever the row length; and BatchNorm, ReLU and
+// the residual addition ride on the kernel that produces the values.  A bottleneck is
+// five launches, each activation is written once:
+//   k_net_conv     1x1 convolution (+ BatchNorm, residual, ReLU)
+//   k_net_spatial  spatial filter branch, planes' partial sums for the pooling on the way
+//   (k_channel_branch / _mma, ddf_branches.hip)
+//   k_net_filter   dynamic filter + BatchNorm + ReLU
+//   k_net_conv
+// and k_net_stem is the 7x7 convolution, BatchNorm, ReLU and max-pool in one.
+// At batch 128 the network took 8.85 ms as torch modules around the operator: 3.2 ms of
+// BatchNorm, 1.6 ms of ReLU and additions, 3 ms of convolutions (ddf_resnet.py:34-111 of
+// the reference is the same composition).  Sums are fp32; what is stored is rounded to
+// fp16 where the modules round it, and less often (not between convolution and BatchNorm's
+// ReLU).
+#include <algorithm>
+#include <type_traits>
+
+#include "ddf_common.h"
+#include "ddf_rows.h"
+
+namespace ddf {
+namespace {
+using rows::from_left;
+using rows::half2_t;
+using rows::kOutside;
+using rows::load_words;
+using rows::plane_rsrc;
+
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t rows_u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256;
+constexpr int kXcd = 8;
+
+// Workgroups are handed to the XCDs round-robin: consecutive logical blocks share one.
+__device__ __forceinline__ int xcd_block(int block, int blocks) {
+    const int per = (blocks + kXcd - 1) / kXcd;
+    return (block % kXcd) * per + block / kXcd;   // (may be >= blocks: nothing to do then)
+}
+inline unsigned xcd_grid(int64_t blocks) { return (unsigned)(cdiv(blocks, kXcd) * kXcd); }
+
+// (NaN stays NaN, as torch's ReLU has it)
+__device__ __forceinline__ float relu(float f) { return f < 0.f ? 0.f : f; }
+
+// y = scale * x + shift of the convolution's bias and the BatchNorm behind it.
+__device__ __forceinline__ void affine(const NetNorm &n, int c, float &scale, float &shift) {
+    scale = 1.f;
+    shift = 0.f;
+    if (n.var) {
+        scale = ld((const __half *)n.weight + c) / sqrtf(ld((const __half *)n.var + c) + n.eps);
+        shift = ld((const __half *)n.bias + c) - ld((const __half *)n.mean + c) * scale;
+    }
+    if (n.conv_bias) shift += ld((const __half *)n.conv_bias + c) * scale;
+}
+
+// ---- 1x1 convolution ----------------------------------------------------------
+// out[m, o] = act(affine(sum_k x[row(m), k] w[o, k]) (+ res[m, o])), row(m) the sampled
+// pixel under a stride.  Tiles of BM pixels x BN channels; four waves, 2 x 2 over the tile,
+// each in 32x32x16 steps.  W is the A operand, so a lane ends with runs of four channels of
+// one pixel; the tile goes through LDS once more and leaves as whole 16-byte vectors.
+// K comes in steps of 64 (128 bytes of a row per eight lanes), the next step's vectors in
+// registers while this one's are multiplied, LDS double-buffered: one barrier per step.
+// LDS rows of eight 16-byte chunks, chunk number xor row % 8: both the writes and the
+// operand reads (32 rows at one chunk) touch all banks.
+constexpr int kStep = 64, kChunks = kStep / 8;
+
+template <int BM, int BN>
+constexpr int conv_lds_halves(bool two) {
+    const int stage = (BM + BN) * kStep * (two ? 2 : 1), tile = BM * (BN + 8);
+    return stage > tile ? stage : tile;
+}
+
+template <int BM, int BN>
+__global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n, int tiles) {
+    constexpr int RX = BM * kChunks / kThreads, RW = BN * kChunks / kThreads;
+    constexpr int TM = BM / 64, TN = BN / 64;      // 32-wide tiles per wave: pixels, channels
+    constexpr int PITCH = BN + 8;
+    extern __shared__ __align__(16) _Float16 net_smem[];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int block = xcd_block(blockIdx.x, tiles);
+    if (block >= tiles) return;
+    const int tm = block / tiles_n, tn = block - tm * tiles_n;
+    const int64_t m0 = (int64_t)tm * BM;
+    const int n0 = tn * BN;
+    const _Float16 *x = static_cast<const _Float16 *>(a.x), *w = static_cast<const _Float16 *>(a.w);
+
+    const _Float16 *xp[RX], *wp[RW];
+    int xs[RX], wsl[RW];                           // LDS positions
+#pragma unroll
+    for (int i = 0; i < RX; ++i) {
+        const int q = tid + i * kThreads, r = q / kChunks, ch = q % kChunks;
+        int64_t m = m0 + r < a.M ? m0 + r : a.M - 1;
+        if (a.stride > 1) {
+            const int64_t n = m / a.npix;
+            const int p = (int)(m - n * a.npix), y = p / a.Wo, xx = p - y * a.Wo;
+            m = (n * a.H + y * a.stride) * a.W + xx * a.stride;
+        }
+        xp[i] = x + m * a.K + ch * 8;
+        xs[i] = r * kStep + (ch ^ (r & 7)) * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+        const int q = tid + i * kThreads, r = q / kChunks, ch = q % kChunks;
+        wp[i] = w + (int64_t)min(n0 + r, a.N - 1) * a.K + ch * 8;
+        wsl[i] = BM * kStep + r * kStep + (ch ^ (r & 7)) * 8;
+    }
+    half8_t xr[RX], wr[RW];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int i = 0; i < RX; ++i) xr[i] = *reinterpret_cast<const half8_t *>(xp[i] + k);
+#pragma unroll
+        for (int i = 0; i < RW; ++i) wr[i] = *reinterpret_cast<const half8_t *>(wp[i] + k);
+    };
+    auto park = [&](int buf) {
+        _Float16 *s = net_smem + buf * (BM + BN) * kStep;
+#pragma unroll
+        for (int i = 0; i < RX; ++i) *reinterpret_cast<half8_t *>(s + xs[i]) = xr[i];
+#pragma unroll
+        for (int i = 0; i < RW; ++i) *reinterpret_cast<half8_t *>(s + wsl[i]) = wr[i];
+    };
+    const int wm = wave & 1, wn = wave >> 1;
+    const int l32 = lane & 31, hi = lane >> 5;
+    float16_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    auto multiply = [&](int buf) {
+        const _Float16 *s = net_smem + buf * (BM + BN) * kStep;
+#pragma unroll
+        for (int kk = 0; kk < kStep / 16; ++kk) {
+            const int ch = kk * 2 + hi;
+            half8_t xv[TM], wv[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int r = wm * (BM / 2) + i * 32 + l32;
+                xv[i] = *reinterpret_cast<const half8_t *>(s + r * kStep + (ch ^ (r & 7)) * 8);
+            }
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int r = wn * (BN / 2) + j * 32 + l32;
+                wv[j] = *reinterpret_cast<const half8_t *>(s + BM * kStep + r * kStep + (ch ^ (r & 7)) * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[j], xv[i], acc[i][j], 0, 0, 0);
+        }
+    };
+    const int nk = a.K / kStep;
+    load(0);
+    park(0);
+    if (nk > 1) load(kStep);
+    __syncthreads();
+    for (int k = 0; k < nk; ++k) {
+        multiply(k & 1);
+        if (k + 1 < nk) park((k + 1) & 1);
+        if (k + 2 < nk) load((k + 2) * kStep);
+        __syncthreads();
+    }
+
+    // The tile, rounded to fp16, through LDS: [pixel][channel].  D of a 32x32 step: lane
+    // column = pixel l32, rows (channels) 8 * g + 4 * hi + 0..3 in registers 4g .. 4g+3.
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                half4_t v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = (_Float16)acc[i][j][4 * g + e];
+                const int px = wm * (BM / 2) + i * 32 + l32, ch = wn * (BN / 2) + j * 32 + 8 * g + 4 * hi;
+                *reinterpret_cast<half4_t *>(net_smem + px * PITCH + ch) = v;
+            }
+    __syncthreads();
+    constexpr int CPR = BN / 8;                     // vectors per pixel
+    const int cq = tid % CPR, c = n0 + cq * 8;
+    float sc[8], sh[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) affine(a.norm, min(c + e, a.N - 1), sc[e], sh[e]);
+    const _Float16 *res = static_cast<const _Float16 *>(a.res);
+    _Float16 *out = static_cast<_Float16 *>(a.out);
+#pragma unroll 4
+    for (int r = tid / CPR; r < BM; r += kThreads / CPR) {
+        const int64_t m = m0 + r;
+        if (m >= a.M || c >= a.N) continue;
+        const half8_t v = *reinterpret_cast<const half8_t *>(net_smem + r * PITCH + cq * 8);
+        half8_t rv = {0, 0, 0, 0, 0, 0, 0, 0}, o;
+        if (res) rv = *reinterpret_cast<const half8_t *>(res + m * a.N + c);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float f = fmaf((float)v[e], sc[e], sh[e]) + (float)rv[e];
+            if (a.relu) f = relu(f);
+            o[e] = (_Float16)f;
+        }
+        *reinterpret_cast<half8_t *>(out + m * a.N + c) = o;
+    }
+}
+
+// Few pixels or a small batch, where tiles of 64 leave most of the chip idle: a workgroup
+// takes 32 pixels x 32 channels, its WAVES waves a range of K each, operands straight from
+// memory (every value is used by one wave only), eight steps of them requested ahead of use;
+// the waves' sums meet in LDS.
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int tiles_n) {
+    constexpr int U = 4, P = 33;
+    __shared__ float red[WAVES][32][P];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+    const int l32 = lane & 31, hi = lane >> 5;
+    const int n0 = tn * 32;
+    int64_t m = (int64_t)tm * 32 + l32;
+    if (m >= a.M) m = a.M - 1;
+    if (a.stride > 1) {
+        const int64_t n = m / a.npix;
+        const int p = (int)(m - n * a.npix), y = p / a.Wo, xx = p - y * a.Wo;
+        m = (n * a.H + y * a.stride) * a.W + xx * a.stride;
+    }
+    const int steps = a.K / 16, per = (steps + WAVES - 1) / WAVES;
+    const int s0 = wave * per, s1 = min(s0 + per, steps);
+    const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + hi * 8;
+    const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + l32, a.N - 1) * a.K + hi * 8;
+    float16_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    half8_t xv[2][U], wv[2][U];
+    auto request = [&](auto set, int s) {
+        constexpr int B = decltype(set)::value;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(s + u, steps - 1) * 16;    // (past the wave's range: not used)
+            xv[B][u] = *reinterpret_cast<const half8_t *>(xp + k);
+            wv[B][u] = *reinterpret_cast<const half8_t *>(wp + k);
+        }
+    };
+    auto use = [&](auto set, int s) {
+        constexpr int B = decltype(set)::value;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u < s1) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[B][u], xv[B][u], acc, 0, 0, 0);
+    };
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    if (s0 < s1) {
+        request(Zero{}, s0);
+        for (int s = s0; s < s1; s += 2 * U) {
+            request(One{}, s + U);
+            __builtin_amdgcn_sched_barrier(0);
+            use(Zero{}, s);
+            request(Zero{}, s + 2 * U);
+            __builtin_amdgcn_sched_barrier(0);
+            use(One{}, s + U);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) red[wave][8 * g + 4 * hi + e][l32] = acc[4 * g + e];
+    __syncthreads();
+    const _Float16 *res = static_cast<const _Float16 *>(a.res);
+    _Float16 *out = static_cast<_Float16 *>(a.out);
+    // (lane = channel: 64-byte runs of a pixel's channels)
+    for (int i = tid; i < 32 * 32; i += WAVES * kWave) {
+        const int c = i & 31, px = i >> 5;
+        const int64_t mm = (int64_t)tm * 32 + px;
+        if (mm >= a.M || n0 + c >= a.N) continue;
+        float f = 0.f;
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) f += red[k][c][px];
+        float sc, sh;
+        affine(a.norm, n0 + c, sc, sh);
+        f = fmaf((float)(_Float16)f, sc, sh);
+        if (res) f += (float)res[mm * a.N + n0 + c];
+        if (a.relu) f = relu(f);
+        out[mm * a.N + n0 + c] = (_Float16)f;
+    }
+}
+
+// ---- stem: 7x7 convolution of stride 2, BatchNorm, ReLU, 3x3 max-pool of stride 2 ----
+// A workgroup produces 8 x 8 pooled pixels x 64 channels at a time: 17 x 17 convolution
+// results from 39 x 39 image pixels.  The image tile sits in LDS as [row][column][4
+// channels, the last one zero]: for a filter row the eight columns under a result are 32
+// contiguous values, one step of the 16x16x32 matrix instruction (the eighth column and the
+// fourth channel meet zero weights).  The weights stay in registers over the tiles a
+// workgroup walks.  Convolution results never leave LDS (205 MB at batch 128).
+constexpr int kPoolTile = 8, kConvTile = 2 * kPoolTile + 1, kImgRows = 2 * (kConvTile - 1) + 7, kImgCols = kImgRows + 1;
+constexpr int kConvPitch = 64 + 8, kStemOut = 64;
+constexpr int kStemPixels = kConvTile * kConvTile, kStemTiles = (kStemPixels + 15) / 16;
+
+__global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__restrict__ img,
+                                                          const _Float16 *__restrict__ w, NetNorm norm,
+                                                          _Float16 *__restrict__ out, int N, int H, int W, int tiles_x,
+                                                          int tiles_y) {
+    __shared__ __align__(16) _Float16 tile[kImgRows * kImgCols * 4];
+    __shared__ __align__(16) _Float16 conv[kStemTiles * 16 * kConvPitch];
+    static_assert(kStemOut * 7 * 32 <= kStemTiles * 16 * kConvPitch, "the weights pass through the results' space");
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int row = lane & 15, quad = lane >> 4;
+    const int Hc = H / 2, Wc = W / 2, Hp = Hc / 2, Wp = Wc / 2;
+    // weights to LDS as [output][filter row][column * 4 + channel], then to registers
+    for (int i = tid; i < kStemOut * 7 * 32; i += kThreads) {
+        const int o = i / 224, r = i - o * 224, ky = r / 32, kx = (r & 31) >> 2, ch = r & 3;
+        conv[i] = (kx < 7 && ch < 3) ? w[((o * 3 + ch) * 7 + ky) * 7 + kx] : (_Float16)0;
+    }
+    __syncthreads();
+    half8_t wv[4][7];
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+        for (int ky = 0; ky < 7; ++ky)
+            wv[ct][ky] = *reinterpret_cast<const half8_t *>(conv + ((ct * 16 + row) * 7 + ky) * 32 + quad * 8);
+    float sc[4][4], sh[4][4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) affine(norm, ct * 16 + quad * 4 + e, sc[ct][e], sh[ct][e]);
+
+    const int per_image = tiles_x * tiles_y, total = N * per_image;
+    for (int t = blockIdx.x; t < total; t += gridDim.x) {
+        const int n = t / per_image, r = t - n * per_image, ty = r / tiles_x, tx = r - ty * tiles_x;
+        const int cy0 = 2 * ty * kPoolTile - 1, cx0 = 2 * tx * kPoolTile - 1;   // first convolution result
+        const int iy0 = 2 * cy0 - 3, ix0 = 2 * cx0 - 3;                         // first image pixel
+        const _Float16 *in = img + (int64_t)n * 3 * H * W;
+        for (int i = tid; i < kImgRows * kImgCols; i += kThreads) {
+            const int yy = iy0 + i / kImgCols, xx = ix0 + i % kImgCols;
+            half4_t v = {0, 0, 0, 0};
+            if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
+                const int64_t at = (int64_t)yy * W + xx;
+#pragma unroll
+                for (int ch = 0; ch < 3; ++ch) v[ch] = in[at + (int64_t)ch * H * W];
+            }
+            *reinterpret_cast<half4_t *>(tile + i * 4) = v;
+        }
+        __syncthreads();   // (also: the weights, or the last tile's results, have been read)
+        for (int pt = wave; pt < kStemTiles; pt += kThreads / kWave) {
+            const int px = pt * 16 + row, pc = min(px, kStemPixels - 1);
+            const int cy = pc / kConvTile, cx = pc - cy * kConvTile;
+            const _Float16 *src = tile + (2 * cy * kImgCols + 2 * cx + quad * 2) * 4;
+            float4_t acc[4];
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct) acc[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ky = 0; ky < 7; ++ky) {
+                const half8_t b = *reinterpret_cast<const half8_t *>(src + ky * kImgCols * 4);
+#pragma unroll
+                for (int ct = 0; ct < 4; ++ct)
+                    acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[ct][ky], b, acc[ct], 0, 0, 0);
+            }
+            // (results outside the image: zero, which no maximum of ReLUs notices)
+            const int yy = cy0 + cy, xx = cx0 + cx;
+            const bool in_image = yy >= 0 && yy < Hc && xx >= 0 && xx < Wc;
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct) {
+                half4_t v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float f = relu(fmaf((float)(_Float16)acc[ct][e], sc[ct][e], sh[ct][e]));
+                    v[e] = in_image ? (_Float16)f : (_Float16)0;
+                }
+                *reinterpret_cast<half4_t *>(conv + px * kConvPitch + ct * 16 + quad * 4) = v;
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < kPoolTile * kPoolTile * 8; i += kThreads) {
+            const int cq = i & 7, p = i >> 3, py = p / kPoolTile, pxx = p % kPoolTile;
+            const int oy = ty * kPoolTile + py, ox = tx * kPoolTile + pxx;
+            half8_t m = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) {
+                    const half8_t v = *reinterpret_cast<const half8_t *>(
+                        conv + ((2 * py + dy) * kConvTile + 2 * pxx + dx) * kConvPitch + cq * 8);
+                    m = __builtin_elementwise_maximum(m, v);
+                }
+            if (oy < Hp && ox < Wp)
+                *reinterpret_cast<half8_t *>(out + (((int64_t)n * Hp + oy) * Wp + ox) * kStemOut + cq * 8) = m;
+        }
+        // (the next tile's image part does not touch `conv`, and its barrier comes before
+        // the next results do)
+    }
+}
+
+// ---- spatial filter branch ------------------------------------------------------
+// Pixels are the columns, the nine taps nine of the sixteen rows of 16x16x32 steps over the
+// channels; both operands contiguous.  A wave walks tiles of sixteen pixels of one sample;
+// the same vectors feed the plane sums (KS * 8 fp32 values per lane, brought together at the
+// end).  A pixel's taps end up on four lanes, which normalise them across the wave's
+// rows; they are stored as (pixel, 12), nine taps and padding.  Under stride 2 the three
+// unsampled pixels of a 2 x 2 block only go into the sums.
+constexpr int kTapPitch = 12;
+
+__device__ __forceinline__ float rows_total(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ float add_permuted(float x) {
+    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lanes16_total(float v) {
+    v = add_permuted<0xB1>(v);
+    v = add_permuted<0x4E>(v);
+    v = add_permuted<0x141>(v);
+    return add_permuted<0x140>(v);
+}
+
+template <int KS, int S>
+__global__ __launch_bounds__(kThreads) void k_net_spatial(const _Float16 *__restrict__ x,
+                                                          const _Float16 *__restrict__ w,
+                                                          const _Float16 *__restrict__ bias,
+                                                          _Float16 *__restrict__ sf, float *__restrict__ parts,
+                                                          int W, int Wo, int npix, int plane, int tiles_per_chunk,
+                                                          float gain) {
+    constexpr int C = KS * 32, KK = 9, NPX = S * S;
+    constexpr bool kHold = KS <= 8;               // weights in registers over the walk
+    constexpr int kWaves = kThreads / kWave;
+    __shared__ float red[kWaves][C];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int col = lane & 15, quad = lane >> 4;
+    const int n = blockIdx.y;
+    const uint32_t bytes = (uint32_t)plane * C * 2;
+    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + (int64_t)n * plane * C, bytes);
+    auto weights = [&](int ks) {
+        half8_t v = *reinterpret_cast<const half8_t *>(w + (int64_t)min(col, KK - 1) * C + ks * 32 + quad * 8);
+        if (col >= KK) v = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        return v;
+    };
+    half8_t wv[kHold ? KS : 1];
+    if constexpr (kHold) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) wv[ks] = weights(ks);
+    }
+    float b[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = (bias && quad * 4 + e < KK) ? (float)bias[quad * 4 + e] : 0.f;
+    float pool[KS * 8];
+#pragma unroll
+    for (int i = 0; i < KS * 8; ++i) pool[i] = 0.f;
+
+    const int tiles = (npix + 15) / 16;
+    const int t_end = min((int)(blockIdx.x + 1) * tiles_per_chunk, tiles);
+    for (int t = blockIdx.x * tiles_per_chunk + wave; t < t_end; t += kWaves) {
+        const int p = t * 16 + col;
+        const bool live = p < npix;
+        uint32_t off[NPX];
+        if constexpr (S == 1) {
+            off[0] = live ? (uint32_t)p * C * 2 + quad * 16 : kOutside;
+        } else {
+            const int y = p / Wo, xx = p - y * Wo;
+#pragma unroll
+            for (int q = 0; q < NPX; ++q)
+                off[q] = live ? (uint32_t)((2 * y + q / 2) * W + 2 * xx + q % 2) * C * 2 + quad * 16 : kOutside;
+        }
+        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+        constexpr int G = KS < 4 ? KS : 4;        // steps requested together
+#pragma unroll
+        for (int k0 = 0; k0 < KS; k0 += G) {
+            half8_t v[NPX][G], wl[kHold ? 1 : G];
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int q = 0; q < NPX; ++q)
+                    v[q][g] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                        xr, (int)off[q], (k0 + g) * 64, 0));
+            if constexpr (!kHold) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) wl[g] = weights(k0 + g);
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const half8_t a = kHold ? wv[kHold ? k0 + g : 0] : wl[kHold ? 0 : g];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, v[0][g], acc, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < NPX; ++q)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) pool[(k0 + g) * 8 + e] += (float)v[q][g][e];
+            }
+        }
+        // taps 4 * quad + e of pixel p
+        float v[4], s = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = acc[e] + b[e];
+            s += v[e];                             // (rows past the ninth: zero weights, zero bias)
+        }
+        const float mean = rows_total(s) / (float)KK;
+        float sq = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] -= mean;
+            if (quad * 4 + e < KK) sq += v[e] * v[e];
+        }
+        const float inv = gain / (sqrtf(rows_total(sq) / (float)(KK - 1)) + 1e-10f);
+        half4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (_Float16)(v[e] * inv);
+        if (live && quad < 3) *reinterpret_cast<half4_t *>(sf + ((int64_t)n * npix + p) * kTapPitch + quad * 4) = o;
+    }
+#pragma unroll
+    for (int i = 0; i < KS * 8; ++i) pool[i] = lanes16_total(pool[i]);
+    if (col == 0) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) red[wave][ks * 32 + quad * 8 + e] = pool[ks * 8 + e];
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < C; c += kThreads) {
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) s += red[k][c];
+        parts[((int64_t)n * gridDim.x + blockIdx.x) * C + c] = s;
+    }
+}
+
+// ---- dynamic filter + BatchNorm + ReLU ---------------------------------------------
+// C / 8 lanes own a pixel, eight channels each, and walk along a row: the window slides, so
+// a step loads one new column (three 16-byte vectors; two columns under stride 2), a step
+// ahead of use.  The channel taps of the lane's channels stay in registers, tap-major in
+// pairs of channels; a pixel's nine spatial taps come with it.  comb(CF, SF) of two channels
+// is one packed fp16 operation (rounded like the operands), the sums are fp32: 13 vector
+// instructions per pixel and channel quarter.  A row outside the image, a column past its
+// ends and a walk past the last pixel read zeros through the buffer descriptor.
+template <int LP, int S, bool MUL>
+__global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restrict__ x,
+                                                         const _Float16 *__restrict__ cf,
+                                                         const _Float16 *__restrict__ sf, NetNorm norm,
+                                                         _Float16 *__restrict__ out, int H, int W, int Ho, int Wo,
+                                                         int runs, int run, int units, int blocks, uint32_t x_bytes) {
+    constexpr int C = LP * 8, SLOTS = kWave / LP, KK = 9;
+    const int block = xcd_block(blockIdx.x, blocks);
+    if (block >= blocks) return;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int cl = lane % LP;
+    const int unit = (block * (kThreads / kWave) + wave) * SLOTS + lane / LP;
+    const bool live = unit < units;
+    const int u = live ? unit : units - 1;
+    const int row = u / runs, r = u - row * runs;
+    const int n = row / Ho, y = row - n * Ho;
+    const int x0 = r * run;
+    const int x1 = live ? min(x0 + run, Wo) : x0;
+    // (lanes of a wave may belong to different samples: one descriptor over all of them)
+    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x, x_bytes);
+    const _Float16 *sn = sf + ((int64_t)n * Ho + y) * Wo * kTapPitch;
+    _Float16 *on = out + ((int64_t)n * Ho + y) * Wo * C + cl * 8;
+
+    uint32_t cfp[KK][4];
+    {
+        const uint4 *src = reinterpret_cast<const uint4 *>(cf + ((int64_t)n * C + cl * 8) * KK);
+        uint32_t wd[36];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            const uint4 q = src[i];
+            wd[4 * i] = q.x; wd[4 * i + 1] = q.y; wd[4 * i + 2] = q.z; wd[4 * i + 3] = q.w;
+        }
+        auto half_at = [&](int i) { return (i & 1) ? wd[i / 2] >> 16 : wd[i / 2] & 0xffffu; };
+#pragma unroll
+        for (int t = 0; t < KK; ++t)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cfp[t][k] = half_at(18 * k + t) | (half_at(18 * k + 9 + t) << 16);
+    }
+    float sc[8], sh[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) affine(norm, cl * 8 + e, sc[e], sh[e]);
+
+    uint32_t rowo[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int yy = y * S - 1 + i;
+        rowo[i] = (live && yy >= 0 && yy < H) ? (uint32_t)(((n * H + yy) * W) * C + cl * 8) * 2 : kOutside;
+    }
+    struct Column { rows_u4 v[3]; };
+    auto column = [&](int xx) {
+        Column c;
+        const bool in = xx >= 0 && xx < W;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            c.v[i] = __builtin_bit_cast(rows_u4, __builtin_amdgcn_raw_buffer_load_b128(
+                xr, (int)(in && rowo[i] != kOutside ? rowo[i] + (uint32_t)xx * C * 2 : kOutside), 0, 0));
+        return c;
+    };
+    struct Taps { uint2 v[3]; };
+    auto taps = [&](int xx) {
+        Taps t;
+        const uint2 *p = reinterpret_cast<const uint2 *>(sn + (int64_t)min(xx, Wo - 1) * kTapPitch);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) t.v[i] = p[i];
+        return t;
+    };
+    auto emit = [&](const Column &a, const Column &b, const Column &c, const Taps &tp, int xx) {
+        float acc[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const int t = i * 3 + j;
+                const uint2 sw = tp.v[t / 4];
+                const half2_t sp = __builtin_bit_cast(half2_t, (t % 4) < 2 ? sw.x : sw.y);
+                const half2_t sv = {sp[t & 1], sp[t & 1]};
+                const rows_u4 q = j == 0 ? a.v[i] : j == 1 ? b.v[i] : c.v[i];
+                const uint32_t xw[4] = {q[0], q[1], q[2], q[3]};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const half2_t cv = __builtin_bit_cast(half2_t, cfp[t][k]);
+                    const half2_t cb = MUL ? cv * sv : cv + sv;
+                    const half2_t xv = __builtin_bit_cast(half2_t, xw[k]);
+                    acc[2 * k] = fmaf((float)xv[0], (float)cb[0], acc[2 * k]);
+                    acc[2 * k + 1] = fmaf((float)xv[1], (float)cb[1], acc[2 * k + 1]);
+                }
+            }
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            // (the complete sum is rounded as the operator's result is)
+            const float f = fmaf((float)(_Float16)acc[e], sc[e], sh[e]);
+            o[e] = (_Float16)relu(f);
+        }
+        if (xx < x1) *reinterpret_cast<half8_t *>(on + (int64_t)xx * C) = o;
+    };
+    if constexpr (S == 1) {
+        Column c0 = column(x0 - 1), c1 = column(x0), c2 = column(x0 + 1), c3;
+        Taps t0 = taps(x0), t1;
+        for (int j = 0; j < run; j += 4) {
+            const int xx = x0 + j;
+            c3 = column(xx + 2); t1 = taps(xx + 1);
+            emit(c0, c1, c2, t0, xx);
+            c0 = column(xx + 3); t0 = taps(xx + 2);
+            emit(c1, c2, c3, t1, xx + 1);
+            c1 = column(xx + 4); t1 = taps(xx + 3);
+            emit(c2, c3, c0, t0, xx + 2);
+            c2 = column(xx + 5); t0 = taps(xx + 4);
+            emit(c3, c0, c1, t1, xx + 3);
+            // (the window is c0 c1 c2 again: columns xx + 3, xx + 4, xx + 5)
+        }
+    } else {
+        Column l = column(2 * x0 - 1), m = column(2 * x0), rr = column(2 * x0 + 1);
+        Taps t0 = taps(x0), t1;
+        for (int j = 0; j < run; j += 2) {
+            const int xx = x0 + j;
+            Column m2 = column(2 * xx + 2), r2 = column(2 * xx + 3);
+            t1 = taps(xx + 1);
+            emit(l, m, rr, t0, xx);
+            m = column(2 * xx + 4);
+            Column r3 = column(2 * xx + 5);
+            t0 = taps(xx + 2);
+            emit(rr, m2, r2, t1, xx + 1);
+            l = r2;
+            rr = r3;
+        }
+    }
+}
+
+// ---- mean over the pixels -----------------------------------------------------------
+__global__ __launch_bounds__(kThreads) void k_net_pool(const _Float16 *__restrict__ x, _Float16 *__restrict__ out,
+                                                       int plane, int C) {
+    constexpr int LANES = 32, GROUPS = kThreads / LANES;
+    __shared__ float red[GROUPS][LANES * 8];
+    const int l = threadIdx.x % LANES, grp = threadIdx.x / LANES;
+    const int n = blockIdx.y, c = blockIdx.x * LANES * 8 + l * 8;
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    if (c < C) {
+        const _Float16 *p = x + (int64_t)n * plane * C + c;
+#pragma unroll 4
+        for (int i = grp; i < plane; i += GROUPS) {
+            const half8_t v = *reinterpret_cast<const half8_t *>(p + (int64_t)i * C);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] += (float)v[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[grp][l * 8 + e] = acc[e];
+    __syncthreads();
+    const int i = threadIdx.x, cc = blockIdx.x * LANES * 8 + i;
+    if (cc >= C) return;
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < GROUPS; ++k) s += red[k][i];
+    out[(int64_t)n * C + cc] = (_Float16)(s / (float)plane);
+}
+
+template <int BM, int BN>
+hipError_t launch_conv(const NetConv &a, hipStream_t st) {
+    const int tiles_n = (int)cdiv(a.N, BN);
+    const int64_t tiles = cdiv(a.M, BM) * tiles_n;
+    if (tiles > (1 << 30)) return hipErrorInvalidConfiguration;
+    const int lds = conv_lds_halves<BM, BN>(a.K > kStep) * (int)sizeof(_Float16);
+    hipLaunchKernelGGL((k_net_conv<BM, BN>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a, tiles_n, (int)tiles);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool net_conv_supported(const NetConv &a) { return a.K % kStep == 0 && a.K > 0 && a.N > 0; }
+
+hipError_t net_conv(const NetConv &a, hipStream_t st) {
+    if (a.M == 0) return hipSuccess;
+    if (!net_conv_supported(a)) return hipErrorNotSupported;
+    // The largest tiles that leave two workgroups per compute unit; whole vectors of
+    // channels for all but the small kernel.
+    auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
+    if (a.N % 8 == 0) {
+        if (a.N >= 128 && count(128, 128) >= 512) return launch_conv<128, 128>(a, st);
+        if (count(128, 64) >= 512) return launch_conv<128, 64>(a, st);
+        if (count(64, 64) >= 256) return launch_conv<64, 64>(a, st);
+    }
+    const int tiles_n = (int)cdiv(a.N, 32);
+    const int64_t blocks = cdiv(a.M, 32) * tiles_n;
+    if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
+    if (a.K >= 256)
+        hipLaunchKernelGGL((k_net_conv_small<8>), dim3((unsigned)blocks), dim3(8 * kWave), 0, st, a, tiles_n);
+    else
+        hipLaunchKernelGGL((k_net_conv_small<4>), dim3((unsigned)blocks), dim3(4 * kWave), 0, st, a, tiles_n);
+    return hipGetLastError();
+}
+
+hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,
+                    hipStream_t st) {
+    if (H % 4 != 0 || W % 4 != 0 || H * W >= (1 << 28)) return hipErrorNotSupported;
+    const int tx = (int)cdiv(W / 4, kPoolTile), ty = (int)cdiv(H / 4, kPoolTile);
+    const int64_t tiles = N * tx * ty;
+    if (tiles == 0) return hipSuccess;
+    if (tiles > (1 << 30)) return hipErrorInvalidConfiguration;
+    // (two workgroups per compute unit, each walking as many tiles as it takes)
+    hipLaunchKernelGGL(k_net_stem, dim3((unsigned)std::min<int64_t>(tiles, 512)), dim3(kThreads), 0, st,
+                       (const _Float16 *)img, (const _Float16 *)w, norm, (_Float16 *)out, (int)N, (int)H, (int)W, tx, ty);
+    return hipGetLastError();
+}
+
+// Chunks of a sample's tiles: enough workgroups, at most kMaxChunks partial sums.
+constexpr int kMaxChunks = 8;
+int net_spatial_chunks(int64_t N, int64_t npix) {
+    const int64_t tiles = cdiv(npix, 16);
+    const int64_t want = std::min<int64_t>(std::max<int64_t>(1, cdiv(1024, N)), kMaxChunks);
+    return (int)std::min<int64_t>(want, cdiv(tiles, 4));   // (a tile per wave at least)
+}
+
+hipError_t net_spatial(const void *x, const void *w, const void *bias, void *sf, float *parts, int *n_parts, int64_t N,
+                       int64_t H, int64_t W, int64_t C, int stride, double gain, hipStream_t st) {
+    if (N > 65535 || H * W * C * 2 >= (1ll << 31) || (stride == 2 && (H % 2 || W % 2))) return hipErrorNotSupported;
+    const int64_t npix = (H / stride) * (W / stride);
+    const int tiles = (int)cdiv(npix, 16);
+    int chunks = net_spatial_chunks(N, npix);
+    const int per = (int)cdiv(tiles, chunks);
+    chunks = (int)cdiv(tiles, per);
+    *n_parts = chunks;
+    const dim3 grid((unsigned)chunks, (unsigned)N);
+#define DDF_NET_SPATIAL(KS_, S_)                                                                         \
+    if (C == KS_ * 32 && stride == S_) {                                                                 \
+        hipLaunchKernelGGL((k_net_spatial<KS_, S_>), grid, dim3(kThreads), 0, st, (const _Float16 *)x,   \
+                           (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)sf, parts, (int)W,   \
+                           (int)(W / stride), (int)npix, (int)(H * W), per, (float)gain);                \
+        return hipGetLastError();                                                                        \
+    }
+    DDF_NET_SPATIAL(2, 1) DDF_NET_SPATIAL(4, 1) DDF_NET_SPATIAL(8, 1) DDF_NET_SPATIAL(16, 1)
+    DDF_NET_SPATIAL(2, 2) DDF_NET_SPATIAL(4, 2) DDF_NET_SPATIAL(8, 2) DDF_NET_SPATIAL(16, 2)
+#undef DDF_NET_SPATIAL
+    return hipErrorNotSupported;
+}
+
+hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNorm &norm, void *out, int64_t N,
+                      int64_t H, int64_t W, int64_t C, int stride, bool mul, hipStream_t st) {
+    const int64_t Ho = H / stride, Wo = W / stride;
+    if (N * Ho * Wo == 0) return hipSuccess;
+    const int step = stride == 1 ? 4 : 2;
+    if (C < 8 || C > kWave * 8) return hipErrorNotSupported;
+    const int slots = (int)(kWave * 8 / C);
+    // (32-bit offsets: as many samples at a time as stay below 2 GiB)
+    const int64_t sample = H * W * C * 2, most = ((1ll << 31) - 1) / sample;
+    if (most < 1) return hipErrorNotSupported;
+    for (int64_t n0 = 0; n0 < N; n0 += most) {
+        const int64_t cnt = std::min(most, N - n0);
+        // Walks as long as leave 4096 waves, in whole rounds of the kernel's unrolled steps
+        // (every walk loads its channel taps and two columns it does not produce).
+        int64_t runs = cdiv((int64_t)4096 * slots, cnt * Ho);
+        runs = std::max<int64_t>(1, std::min<int64_t>(runs, cdiv(Wo, step)));
+        const int run = (int)(cdiv(cdiv(Wo, runs), step) * step);
+        runs = cdiv(Wo, run);
+        const int64_t units = cnt * Ho * runs, blocks = cdiv(units, slots * (kThreads / kWave));
+        if (units > (1 << 30)) return hipErrorInvalidConfiguration;
+        const _Float16 *xn = (const _Float16 *)x + n0 * H * W * C, *cn = (const _Float16 *)cf + n0 * C * 9,
+                       *sn = (const _Float16 *)sf + n0 * Ho * Wo * kTapPitch;
+        _Float16 *on = (_Float16 *)out + n0 * Ho * Wo * C;
+        bool done = false;
+#define DDF_NET_FILTER_LAUNCH(LP_, S_, MUL_)                                                                     \
+    hipLaunchKernelGGL((k_net_filter<LP_, S_, MUL_>), dim3(xcd_grid(blocks)), dim3(kThreads), 0, st, xn, cn, sn, \
+                       norm, on, (int)H, (int)W, (int)Ho, (int)Wo, (int)runs, run, (int)units, (int)blocks,      \
+                       (uint32_t)(cnt * sample))
+#define DDF_NET_FILTER(LP_, S_)                            \
+    if (C == LP_ * 8 && stride == S_) {                    \
+        if (mul) DDF_NET_FILTER_LAUNCH(LP_, S_, true);     \
+        else DDF_NET_FILTER_LAUNCH(LP_, S_, false);        \
+        done = true;                                       \
+    }
+        DDF_NET_FILTER(8, 1) DDF_NET_FILTER(16, 1) DDF_NET_FILTER(32, 1) DDF_NET_FILTER(64, 1)
+        DDF_NET_FILTER(8, 2) DDF_NET_FILTER(16, 2) DDF_NET_FILTER(32, 2) DDF_NET_FILTER(64, 2)
+#undef DDF_NET_FILTER
+#undef DDF_NET_FILTER_LAUNCH
+        if (!done) return hipErrorNotSupported;
+    }
+    return hipGetLastError();
+}
+
+hipError_t net_pool(const void *x, void *out, int64_t N, int64_t plane, int64_t C, hipStream_t st) {
+    if (N * plane * C == 0) return hipSuccess;
+    if (N > 65535 || C % 8 != 0) return hipErrorNotSupported;
+    hipLaunchKernelGGL(k_net_pool, dim3((unsigned)cdiv(C, 256), (unsigned)N), dim3(kThreads), 0, st, (const _Float16 *)x,
+                       (_Float16 *)out, (int)plane, (int)C);
+    return hipGetLastError();
+}
+
+}  // namespace ddf

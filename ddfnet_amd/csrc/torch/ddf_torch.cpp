@@ -343,6 +343,8 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
 
 #include "ddf_pack.h"
 
+#include "ddf_net.h"
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     using namespace ddf_torch;
     m.doc() = "ddf operator of libddf_hip.so as a C++ autograd function";
@@ -361,5 +363,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("pack_infer", &pack_infer,
           "DDFPack.forward without gradients: spatial branch (pooling on the way where it can), "
           "channel branch, operator");
+    py::class_<NetPlan>(m, "NetPlan")
+        .def(py::init<py::list, py::list>())
+        .def("set_ends", &NetPlan::set_ends)
+        .def("add_block", &NetPlan::add_block)
+        .def("valid", [](const NetPlan &p) { return p.guard.holds(); });
+    m.def("net_forward", &net_forward, "DDFResNet.forward through a plan, or None");
     m.def("library_version", []() { return ddf_hip_version(); });
 }

@@ -21,8 +21,10 @@ import ctypes
 import torch
 import torch.nn as nn
 
+from . import functional
 from .functional import ddf  # noqa: F401  (re-exported: callers time the operator through this module)
-from .modules import DDFPack
+from .modules import (DDFPack, FilterNorm, _CONV_CONSTANTS, _PlanSlot, _guard_of, _plain_pointwise_conv,
+                      _unhooked)
 
 __all__ = ['DDFBottleneck', 'DDFResNet', 'ddf_mul_resnet50', 'ddf_mul_resnet101',
            'ddf_mul_resnet152', 'ddf_add_resnet50', 'ddf_add_resnet101', 'ddf_add_resnet152',
@@ -55,6 +57,19 @@ class DDFBottleneck(nn.Module):
         x = self.act2(self.bn2(self.conv2(x)))
         x = self.bn3(self.conv3(x))
         return self.act3(x + shortcut)
+
+
+def _is_plain_norm(m):
+    return type(m) is nn.Identity or (
+        type(m) is nn.BatchNorm2d and m.affine and m.track_running_stats and not m.training and
+        m.running_mean is not None and m.running_var is not None)
+
+
+def _layer_args(conv, norm):
+    """(tensors, eps) of a convolution (or None) and the BatchNorm / Identity behind it."""
+    bn = [norm.weight, norm.bias, norm.running_mean, norm.running_var] if type(norm) is nn.BatchNorm2d else [None] * 4
+    head = [None, None] if conv is None else [conv.weight, conv.bias]
+    return head + bn, (norm.eps if type(norm) is nn.BatchNorm2d else 0.0)
 
 
 class DDFResNet(nn.Module):
@@ -104,7 +119,105 @@ class DDFResNet(nn.Module):
         x = self.maxpool(self.act1(self.bn1(self.conv1(x))))
         return self.layer4(self.layer3(self.layer2(self.layer1(x))))
 
+    def _is_stock(self):
+        """The network is what the constructor builds (BatchNorms may have been folded) in
+        eval mode, of the kinds and sizes the native inference covers, and nothing listens
+        on its modules."""
+        if type(self) is not DDFResNet or not all(_unhooked(m) for m in self.modules() if m is not self):
+            return False
+        conv, pool = self.conv1, self.maxpool
+        pair = lambda v: v if isinstance(v, tuple) else (v, v)
+        if not (type(conv) is nn.Conv2d and conv.kernel_size == (7, 7) and conv.stride == (2, 2) and
+                conv.padding == (3, 3) and conv.dilation == (1, 1) and conv.groups == 1 and
+                conv.padding_mode == 'zeros' and conv.in_channels == 3 and conv.out_channels == 64 and
+                _is_plain_norm(self.bn1) and type(self.act1) is nn.ReLU and type(pool) is nn.MaxPool2d and
+                pair(pool.kernel_size) == (3, 3) and pair(pool.stride) == (2, 2) and pair(pool.padding) == (1, 1) and
+                pair(pool.dilation) == (1, 1) and not pool.ceil_mode and not pool.return_indices and
+                type(self.global_pool) is nn.AdaptiveAvgPool2d and self.global_pool.output_size in (1, (1, 1)) and
+                type(self.fc) is nn.Linear):
+            return False
+        channels = 64
+        for block in self._blocks():
+            if type(block) is not DDFBottleneck:
+                return False
+            pack, down = block.conv2, block.downsample
+            if not (_plain_pointwise_conv(block.conv1, 1) and _plain_pointwise_conv(block.conv3, 1) and
+                    all(_is_plain_norm(m) for m in (block.bn1, block.bn2, block.bn3)) and
+                    all(type(m) is nn.ReLU for m in (block.act1, block.act2, block.act3)) and
+                    type(pack) is DDFPack and pack.kernel_size == 3 and pack.dilation == 1 and pack.head == 1 and
+                    pack.stride in (1, 2) and pack._stock_spatial_branch() and pack._stock_channel_branch()):
+                return False
+            width, norm = block.conv1.out_channels, pack.spatial_branch[1]
+            if (norm.runing_std or norm.runing_mean or width not in (64, 128, 256, 512) or
+                    block.conv1.in_channels != channels or block.conv3.in_channels != width or
+                    pack.spatial_branch[0].in_channels != width or pack.channel_branch[1].in_channels != width or
+                    pack.channel_branch[4].in_channels != width):
+                return False
+            out = block.conv3.out_channels
+            if down is None:
+                if pack.stride != 1 or out != channels:
+                    return False
+            elif not (type(down) is nn.Sequential and len(down) in (1, 2) and
+                      _plain_pointwise_conv(down[0], pack.stride) and down[0].in_channels == channels and
+                      down[0].out_channels == out and (len(down) == 1 or _is_plain_norm(down[1]))):
+                return False
+            channels = out
+        return channels % 64 == 0 and self.fc.in_features == channels
+
+    def _blocks(self):
+        return [b for stage in (self.layer1, self.layer2, self.layer3, self.layer4) for b in stage]
+
+    def _native_plan(self, ext):
+        """The network's tensors for the extension's native inference, collected once and
+        again whenever the network has changed; None where that does not cover it."""
+        slot = self.__dict__.get('_plan')
+        if slot is None:
+            slot = self.__dict__['_plan'] = _PlanSlot()
+        if slot.plan is not None and slot.plan.valid():
+            return slot.plan
+        slot.plan = None
+        if not self._is_stock():
+            return None
+        own = [self.__dict__[h] for h in ('_forward_hooks', '_forward_pre_hooks', '_backward_hooks',
+                                          '_backward_pre_hooks') if h in self.__dict__]
+        same, empty = _guard_of(list(self.modules()), {
+            nn.Conv2d: _CONV_CONSTANTS, nn.BatchNorm2d: ('training', 'eps', 'affine', 'track_running_stats'),
+            nn.AdaptiveAvgPool2d: ('output_size',),
+            nn.MaxPool2d: ('kernel_size', 'stride', 'padding', 'dilation', 'ceil_mode', 'return_indices'),
+            FilterNorm: ('in_channels', 'filter_type', 'runing_std', 'runing_mean', 'std'),
+            DDFPack: ('kernel_size', 'stride', 'dilation', 'head', 'kernel_combine')})
+        plan = ext.NetPlan(same, [d for d in empty if not any(d is o for o in own)])
+        identity = nn.Identity()
+        plan.set_ends(_layer_args(self.conv1, self.bn1), _layer_args(self.fc, identity))
+        for block in self._blocks():
+            pack, down = block.conv2, block.downsample
+            conv, sp_norm = pack.spatial_branch
+            fc1, fc2, ch_norm = pack.channel_branch[1], pack.channel_branch[3], pack.channel_branch[4]
+            plan.add_block(
+                _layer_args(block.conv1, block.bn1), _layer_args(None, block.bn2),
+                _layer_args(block.conv3, block.bn3),
+                ([None] * 6, 0.0) if down is None else
+                _layer_args(down[0], down[1] if len(down) > 1 else identity),
+                [conv.weight, conv.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias,
+                 ch_norm.std if ch_norm.runing_std else None, ch_norm.mean if ch_norm.runing_mean else None],
+                sp_norm.std, 1.0 if ch_norm.runing_std else ch_norm.std, pack.stride, pack.kernel_combine)
+        slot.plan = plan
+        return plan
+
     def forward(self, x):
+        # fp16 inference natively where the extension covers it (a plan that no longer
+        # holds, or does not cover the call, answers None)
+        ext = functional.extension() if x.is_cuda and x.dtype == torch.float16 and not self.training else None
+        if ext is not None:
+            slot = self.__dict__.get('_plan')
+            plan = None if slot is None else slot.plan
+            out = None if plan is None else ext.net_forward(plan, x)
+            if out is None:
+                fresh = self._native_plan(ext)
+                if fresh is not None and fresh is not plan:
+                    out = ext.net_forward(fresh, x)
+            if out is not None:
+                return out
         x = self.global_pool(self.forward_features(x)).flatten(1)
         return self.fc(x)
 

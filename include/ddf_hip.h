@@ -347,6 +347,41 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
                           int dtype, void *stream);
 
 /*
+ * Building blocks of a DDF-ResNet's inference (ddf_resnet.py:34-111 of the reference:
+ * bottlenecks of 1x1 convolution, DDFPack, 1x1 convolution, each with its BatchNorm), fp16,
+ * activations channels-last: dense (N, H, W, C).  A ddf_net_norm_t is the per-channel
+ * affine map behind a convolution: its bias and the eval-mode BatchNorm that follows; NULL
+ * pointers: absent (running_var NULL: no BatchNorm).  Pointers are 16-byte aligned (per-channel
+ * vectors: 2).  DDF_ERR_UNSUPPORTED: sizes a kernel does not cover.
+ *   conv    out (N, Ho, Wo, O) = act(norm(1x1 convolution of stride `stride`, weight (O, C)) +
+ *           residual), residual NULL or shaped like out (which may be the same memory);
+ *           C a multiple of 64
+ *   stem    max_pool(relu(norm(7x7 convolution, stride 2, padding 3, weight (64, 3, 7, 7))), 3x3,
+ *           stride 2, padding 1) of a planar (N, 3, H, W) image; H and W multiples of 4
+ *   spatial the spatial filter branch (3x3 taps, one head): spatial_filter (N, Ho*Wo, 12), nine
+ *           taps and three of padding, and partial sums of the channels over the pixels as
+ *           ddf_hip_spatial_branch_pool's; at most 8 parts; C 64, 128, 256 or 512
+ *   filter  relu(norm(the operator)) with the filters of `spatial` and ddf_hip_channel_branch_parts
+ *   pool    mean over the pixels, (N, C)
+ */
+typedef struct {
+    const void *weight, *bias, *running_mean, *running_var, *conv_bias;
+    float eps;
+} ddf_net_norm_t;
+int ddf_hip_net_conv(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
+                     void *output, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int stride, int relu,
+                     void *stream);
+int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,
+                     int64_t H, int64_t W, void *stream);
+int ddf_hip_net_spatial(const void *features, const void *weight, const void *bias, void *spatial_filter,
+                        float *pool_parts, int *n_parts, int64_t N, int64_t H, int64_t W, int64_t C, int stride,
+                        double gain, void *stream);
+int ddf_hip_net_filter(const void *features, const void *channel_filter, const void *spatial_filter,
+                       const ddf_net_norm_t *norm, void *output, int64_t N, int64_t H, int64_t W, int64_t C,
+                       int stride, int combine, void *stream);
+int ddf_hip_net_pool(const void *features, void *output, int64_t N, int64_t pixels, int64_t C, void *stream);
+
+/*
  * Up-sampling DDF forward (DDFUpPack.forward, ddf/ddf.py:257-272): the
  * reference calls `ddf` once per sub-pixel branch b = 0 .. scale*scale-1 on
  * the same features with that branch's filters (ddf.py:264-269), stacks the

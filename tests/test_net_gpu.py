@@ -1,0 +1,154 @@
+"""The channels-last fp16 kernels of the DDF-ResNets' inference, each against plain PyTorch in
+fp32 on the same fp16 values, and the whole network against its modules."""
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import ddfnet_amd
+from ddfnet_amd import _lib, ddf_resnet
+
+pytestmark = pytest.mark.gpu
+
+
+class Norm(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ('weight', 'bias', 'mean', 'var', 'conv_bias')] + [('eps', ctypes.c_float)]
+
+
+def make_norm(c, bn, bias):
+    t = {}
+    if bn:
+        t = {'weight': torch.rand(c) + 0.5, 'bias': torch.randn(c) * 0.2, 'mean': torch.randn(c) * 0.2,
+             'var': torch.rand(c) + 0.5}
+    if bias:
+        t['conv_bias'] = torch.randn(c)
+    t = {k: v.half().cuda() for k, v in t.items()}
+    norm = Norm(**{k: v.data_ptr() for k, v in t.items()}, eps=1e-5)
+
+    def apply(y):   # y (..., c) fp32
+        if bias:
+            y = y + t['conv_bias'].float()
+        if bn:
+            y = (y - t['mean'].float()) / torch.sqrt(t['var'].float() + 1e-5) * t['weight'].float() + t['bias'].float()
+        return y
+    return norm, apply, t
+
+
+def call(name, *args):
+    conv = [ctypes.c_void_p(a.data_ptr()) if torch.is_tensor(a) else ctypes.byref(a) if isinstance(a, Norm) else a
+            for a in args]
+    _lib.check(getattr(_lib.lib(), name)(*conv, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+
+
+def close(got, want, tol):
+    err = (got.float() - want.float()).abs().max().item() / want.float().abs().max().item()
+    assert torch.isfinite(got).all() and err <= tol, err
+
+
+@pytest.mark.parametrize('n,h,w,c,o,stride,bn,bias,res,relu', [
+    (1, 1, 1, 64, 10, 1, 0, 1, 0, 0),          # the classifier: one row, channels no multiple of 8
+    (3, 5, 7, 64, 64, 1, 1, 0, 0, 1),          # one step of K, rows past the end of a tile
+    (2, 7, 7, 2048, 512, 1, 1, 0, 0, 1),       # few pixels, long rows: waves split K
+    (1, 14, 14, 256, 1024, 1, 1, 1, 1, 1),
+    (9, 56, 56, 64, 256, 1, 1, 0, 1, 1),       # tiles of 128 x 128
+    (33, 28, 28, 256, 64, 1, 1, 0, 0, 1),      # 64 channels
+    (21, 28, 28, 128, 72, 1, 1, 0, 1, 0),      # channels past a tile
+    (8, 28, 28, 192, 136, 1, 0, 1, 0, 1),      # three steps of K
+    (5, 28, 30, 256, 512, 2, 1, 0, 0, 0),      # projection under stride 2
+    (40, 56, 56, 256, 512, 2, 1, 0, 0, 0),
+])
+def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
+    torch.manual_seed(c + o)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    wt = (torch.randn(o, c, device='cuda') * c ** -0.5).half()
+    norm, apply, keep = make_norm(o, bn, bias)
+    ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
+    r = torch.randn(n, ho, wo, o, device='cuda').half() if res else None
+    want = apply(x[:, ::stride, ::stride].reshape(-1, c).float() @ wt.float().t()).reshape(n, ho, wo, o)
+    want = want + r.float() if res else want
+    want = want.clamp_min(0) if relu else want
+    out = r if res else torch.empty(n, ho, wo, o, device='cuda', dtype=torch.float16)   # (in place where it may be)
+    call('ddf_hip_net_conv', x, wt, norm, r, out, n, h, w, c, o, stride, relu)
+    close(out, want, 3e-3)
+
+
+@pytest.mark.parametrize('n,h,w', [(1, 32, 32), (2, 64, 96), (3, 40, 36), (70, 64, 64)])
+def test_stem(n, h, w):
+    torch.manual_seed(h)
+    x = torch.randn(n, 3, h, w, device='cuda').half()
+    wt = (torch.randn(64, 3, 7, 7, device='cuda') * 0.1).half()
+    norm, apply, keep = make_norm(64, 1, 1)
+    y = apply(F.conv2d(x.float(), wt.float(), stride=2, padding=3).permute(0, 2, 3, 1)).clamp_min(0)
+    want = F.max_pool2d(y.permute(0, 3, 1, 2), 3, 2, 1).permute(0, 2, 3, 1)
+    out = torch.empty(want.shape, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_stem', x, wt, norm, out, n, h, w)
+    close(out, want, 3e-3)
+
+
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('n,h,w,c,s', [(2, 56, 56, 64, 1), (1, 2, 2, 512, 1), (3, 7, 7, 512, 1), (5, 9, 13, 128, 1),
+                                       (2, 14, 14, 256, 1), (2, 4, 6, 256, 2), (1, 28, 28, 128, 2), (3, 14, 14, 512, 2),
+                                       (2, 12, 10, 64, 2), (70, 14, 14, 256, 1)])
+def test_filter_and_spatial_branch(n, h, w, c, s, combine):
+    torch.manual_seed(h * w + c)
+    x = torch.randn(n, c, h, w, device='cuda').half()
+    ws = (torch.randn(9, c, device='cuda') * c ** -0.5).half()
+    bs = torch.randn(9, device='cuda').half()
+    ho, wo = h // s, w // s
+    xl = x.permute(0, 2, 3, 1).contiguous()
+    sf = torch.empty(n, ho * wo, 12, device='cuda', dtype=torch.float16)
+    parts = torch.empty(n * c * 8, device='cuda')
+    count = ctypes.c_int(0)
+    call('ddf_hip_net_spatial', xl, ws, bs, sf, parts, ctypes.byref(count), n, h, w, c, s, 0.6)
+    raw = F.conv2d(x.float(), ws.float().view(9, c, 1, 1), bs.float(), stride=s)
+    want = (raw - raw.mean(1, keepdim=True)) / (raw.std(1, keepdim=True) + 1e-10) * 0.6
+    taps = sf[:, :, :9].permute(0, 2, 1).reshape(n, 9, ho, wo)
+    close(taps, want, 4e-3)
+    total = parts[:n * count.value * c].view(n, count.value, c).double().sum(1)
+    assert (total - x.double().sum((2, 3))).abs().max() <= 1e-5 * x.double().abs().sum((2, 3)).max()
+    cf = torch.randn(n, c, 3, 3, device='cuda').half()
+    norm, apply, keep = make_norm(c, 1, 0)
+    out = torch.empty(n, ho, wo, c, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_filter', xl, cf, sf, norm, out, n, h, w, c, s, _lib.COMBINE[combine])
+    y = ddfnet_amd.ddf(x.double(), cf.double(), taps.double().contiguous(), 3, 1, s, combine)
+    close(out, apply(y.permute(0, 2, 3, 1).float()).clamp_min(0), 4e-3)
+
+
+@pytest.mark.parametrize('build,n,size,classes', [('ddf_mul_resnet50', 2, 64, 10), ('ddf_add_resnet50', 3, 96, 1000),
+                                                  ('ddf_mul_resnet101', 1, 128, 1000), ('ddf_mul_resnet50', 40, 224, 1000)])
+def test_network_matches_its_modules(build, n, size, classes):
+    torch.manual_seed(n)
+    model = getattr(ddf_resnet, build)(num_classes=classes, zero_init_last_bn=False).cuda()
+    for m in model.modules():
+        if isinstance(m, torch.nn.BatchNorm2d):
+            torch.nn.init.uniform_(m.weight, 0.5, 1.5)
+            torch.nn.init.uniform_(m.bias, -0.2, 0.2)
+            m.running_mean.uniform_(-0.1, 0.1)
+            m.running_var.uniform_(0.5, 1.5)
+    model = model.half().eval()
+    x = torch.randn(n, 3, size, size, device='cuda').half()
+    with torch.no_grad():
+        assert ddfnet_amd.functional.extension().net_forward(
+            model._native_plan(ddfnet_amd.functional.extension()), x) is not None
+        out = model(x)
+        modules = lambda net, y: net.fc(net.global_pool(net.forward_features(y)).flatten(1))
+        by_modules = modules(model, x).float()
+        want = modules(model.float(), x.float())
+        assert out.shape == (n, classes)
+        off = lambda y: ((y.float() - want).norm() / want.norm()).item()
+        # (fp16 over so many layers is as far off as it is: not farther than the modules are)
+        most = max(4e-3, 1.3 * off(by_modules))
+        assert off(out) <= most
+        folded = ddf_resnet.fold_batchnorm(model).half()
+        assert folded._native_plan(ddfnet_amd.functional.extension()) is not None
+        assert off(folded(x)) <= 1.5 * most
+        # a change of any kind is seen: a parameter's values, a hook, train mode
+        model = model.half()
+        model.fc.weight.zero_()
+        assert torch.equal(model(x), model.fc.bias.expand(n, -1))
+        calls = []
+        handle = model.layer2[0].act1.register_forward_hook(lambda *a: calls.append(1))
+        model(x)
+        handle.remove()
+        assert calls == [1]
