@@ -51,16 +51,37 @@ inline unsigned xcd_grid(int64_t blocks) { return (unsigned)(cdiv(blocks, kXcd) 
 // (NaN stays NaN, as torch's ReLU has it)
 __device__ __forceinline__ float relu(float f) { return f < 0.f ? 0.f : f; }
 
-// y = scale * x + shift of the convolution's bias and the BatchNorm behind it.
-__device__ __forceinline__ void affine(const NetNorm &n, int c, float &scale, float &shift) {
-    scale = 1.f;
-    shift = 0.f;
-    if (n.var) {
-        scale = ld((const __half *)n.weight + c) / sqrtf(ld((const __half *)n.var + c) + n.eps);
-        shift = ld((const __half *)n.bias + c) - ld((const __half *)n.mean + c) * scale;
+// y = scale * x + shift of the convolution's bias and the BatchNorm behind it, for V
+// consecutive channels: requested as vectors early, worked out where they are needed.  (Read
+// channel by channel at the end of a kernel they cost more than small kernels do.)
+template <int V>
+struct Affine {
+    typedef _Float16 vec __attribute__((ext_vector_type(V)));
+    vec w, b, m, v, cb;
+    __device__ __forceinline__ void request(const NetNorm &n, int c) {
+        auto get = [&](const void *p, _Float16 other) {
+            vec r;
+            if (p) __builtin_memcpy(&r, static_cast<const _Float16 *>(p) + c, sizeof(vec));
+            else
+#pragma unroll
+                for (int e = 0; e < V; ++e) r[e] = other;
+            return r;
+        };
+        w = get(n.var ? n.weight : nullptr, (_Float16)1);
+        b = get(n.var ? n.bias : nullptr, (_Float16)0);
+        m = get(n.var ? n.mean : nullptr, (_Float16)0);
+        v = get(n.var, (_Float16)1);
+        cb = get(n.conv_bias, (_Float16)0);
     }
-    if (n.conv_bias) shift += ld((const __half *)n.conv_bias + c) * scale;
-}
+    __device__ __forceinline__ void finish(const NetNorm &n, float (&scale)[V], float (&shift)[V]) const {
+        const float eps = n.var ? n.eps : 0.f;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            scale[e] = (float)w[e] * rsqrtf((float)v[e] + eps);
+            shift[e] = (float)b[e] + ((float)cb[e] - (float)m[e]) * scale[e];
+        }
+    }
+};
 
 // ---- 1x1 convolution ----------------------------------------------------------
 // out[m, o] = act(affine(sum_k x[row(m), k] w[o, k]) (+ res[m, o])), row(m) the sampled
@@ -161,11 +182,32 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
         }
     };
     const int nk = a.K / kStep;
+    // what the tile's results meet on their way out: this thread's eight channels, and the
+    // residual of its pixels (requested before the last step, so with everything else where
+    // K is a single step)
+    constexpr int CPR = BN / 8;                     // vectors per pixel
+    constexpr int RO = BM * CPR / kThreads;
+    const int cq = tid % CPR, c = n0 + cq * 8;
+    const bool cok = c < a.N;
+    const _Float16 *res = static_cast<const _Float16 *>(a.res);
+    Affine<8> aff;
+    half8_t rv[RO];
+    auto residual = [&]() {
+        aff.request(a.norm, cok ? c : 0);
+#pragma unroll
+        for (int i = 0; i < RO; ++i) {
+            const int64_t m = m0 + tid / CPR + i * (kThreads / CPR);
+            rv[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+            if (res) rv[i] = *reinterpret_cast<const half8_t *>(res + (m < a.M ? m : a.M - 1) * a.N + (cok ? c : 0));
+        }
+    };
     load(0);
+    if (nk == 1) residual();
     park(0);
     if (nk > 1) load(kStep);
     __syncthreads();
     for (int k = 0; k < nk; ++k) {
+        if (nk > 1 && k == nk - 1) residual();
         multiply(k & 1);
         if (k + 1 < nk) park((k + 1) & 1);
         if (k + 2 < nk) load((k + 2) * kStep);
@@ -187,23 +229,20 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
                 *reinterpret_cast<half4_t *>(net_smem + px * PITCH + ch) = v;
             }
     __syncthreads();
-    constexpr int CPR = BN / 8;                     // vectors per pixel
-    const int cq = tid % CPR, c = n0 + cq * 8;
     float sc[8], sh[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) affine(a.norm, min(c + e, a.N - 1), sc[e], sh[e]);
-    const _Float16 *res = static_cast<const _Float16 *>(a.res);
+    aff.finish(a.norm, sc, sh);
     _Float16 *out = static_cast<_Float16 *>(a.out);
-#pragma unroll 4
-    for (int r = tid / CPR; r < BM; r += kThreads / CPR) {
+    if (!cok) return;
+#pragma unroll
+    for (int i = 0; i < RO; ++i) {
+        const int r = tid / CPR + i * (kThreads / CPR);
         const int64_t m = m0 + r;
-        if (m >= a.M || c >= a.N) continue;
+        if (m >= a.M) break;
         const half8_t v = *reinterpret_cast<const half8_t *>(net_smem + r * PITCH + cq * 8);
-        half8_t rv = {0, 0, 0, 0, 0, 0, 0, 0}, o;
-        if (res) rv = *reinterpret_cast<const half8_t *>(res + m * a.N + c);
+        half8_t o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            float f = fmaf((float)v[e], sc[e], sh[e]) + (float)rv[e];
+            float f = fmaf((float)v[e], sc[e], sh[e]) + (float)rv[i][e];
             if (a.relu) f = relu(f);
             o[e] = (_Float16)f;
         }
@@ -235,6 +274,13 @@ __global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int
     const int s0 = wave * per, s1 = min(s0 + per, steps);
     const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + hi * 8;
     const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + l32, a.N - 1) * a.K + hi * 8;
+    // (a thread finishes one channel of 32 / (2 * WAVES) pixels: 64-byte runs of a pixel's channels)
+    constexpr int PX = 2 * WAVES, RO = 32 / PX;
+    const int oc = n0 + (tid & 31);
+    const bool cok = oc < a.N;
+    const _Float16 *res = static_cast<const _Float16 *>(a.res);
+    Affine<1> aff;
+    _Float16 rv[RO];
     float16_t acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.f;
@@ -256,8 +302,14 @@ __global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int
     };
     using Zero = std::integral_constant<int, 0>;
     using One = std::integral_constant<int, 1>;
+    if (s0 < s1) request(Zero{}, s0);
+    aff.request(a.norm, cok ? oc : 0);
+#pragma unroll
+    for (int i = 0; i < RO; ++i) {
+        const int64_t mm = (int64_t)tm * 32 + (tid >> 5) + i * PX;
+        rv[i] = res ? res[(mm < a.M ? mm : a.M - 1) * a.N + (cok ? oc : 0)] : (_Float16)0;
+    }
     if (s0 < s1) {
-        request(Zero{}, s0);
         for (int s = s0; s < s1; s += 2 * U) {
             request(One{}, s + U);
             __builtin_amdgcn_sched_barrier(0);
@@ -272,22 +324,21 @@ __global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int
 #pragma unroll
         for (int e = 0; e < 4; ++e) red[wave][8 * g + 4 * hi + e][l32] = acc[4 * g + e];
     __syncthreads();
-    const _Float16 *res = static_cast<const _Float16 *>(a.res);
     _Float16 *out = static_cast<_Float16 *>(a.out);
-    // (lane = channel: 64-byte runs of a pixel's channels)
-    for (int i = tid; i < 32 * 32; i += WAVES * kWave) {
-        const int c = i & 31, px = i >> 5;
+    float sc[1], sh[1];
+    aff.finish(a.norm, sc, sh);
+    if (!cok) return;
+#pragma unroll
+    for (int i = 0; i < RO; ++i) {
+        const int px = (tid >> 5) + i * PX;
         const int64_t mm = (int64_t)tm * 32 + px;
-        if (mm >= a.M || n0 + c >= a.N) continue;
+        if (mm >= a.M) break;
         float f = 0.f;
 #pragma unroll
-        for (int k = 0; k < WAVES; ++k) f += red[k][c][px];
-        float sc, sh;
-        affine(a.norm, n0 + c, sc, sh);
-        f = fmaf((float)(_Float16)f, sc, sh);
-        if (res) f += (float)res[mm * a.N + n0 + c];
+        for (int k = 0; k < WAVES; ++k) f += red[k][tid & 31][px];
+        f = fmaf((float)(_Float16)f, sc[0], sh[0]) + (float)rv[i];
         if (a.relu) f = relu(f);
-        out[mm * a.N + n0 + c] = (_Float16)f;
+        out[mm * a.N + oc] = (_Float16)f;
     }
 }
 
@@ -314,9 +365,20 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
     const int row = lane & 15, quad = lane >> 4;
     const int Hc = H / 2, Wc = W / 2, Hp = Hc / 2, Wp = Wc / 2;
     // weights to LDS as [output][filter row][column * 4 + channel], then to registers
-    for (int i = tid; i < kStemOut * 7 * 32; i += kThreads) {
-        const int o = i / 224, r = i - o * 224, ky = r / 32, kx = (r & 31) >> 2, ch = r & 3;
-        conv[i] = (kx < 7 && ch < 3) ? w[((o * 3 + ch) * 7 + ky) * 7 + kx] : (_Float16)0;
+    {
+        constexpr int COUNT = kStemOut * 147, R = (COUNT + kThreads - 1) / kThreads;
+        _Float16 wr[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) wr[i] = w[min(tid + i * kThreads, COUNT - 1)];
+        for (int i = tid; i < kStemOut * 7 * 32 / 8; i += kThreads)
+            *reinterpret_cast<half8_t *>(conv + i * 8) = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int e = tid + i * kThreads;
+            const int o = e / 147, r = e - o * 147, ch = r / 49, q = r - ch * 49, ky = q / 7, kx = q - ky * 7;
+            if (e < COUNT) conv[(o * 7 + ky) * 32 + kx * 4 + ch] = wr[i];
+        }
     }
     __syncthreads();
     half8_t wv[4][7];
@@ -327,26 +389,45 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
             wv[ct][ky] = *reinterpret_cast<const half8_t *>(conv + ((ct * 16 + row) * 7 + ky) * 32 + quad * 8);
     float sc[4][4], sh[4][4];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) affine(norm, ct * 16 + quad * 4 + e, sc[ct][e], sh[ct][e]);
+    for (int ct = 0; ct < 4; ++ct) {
+        Affine<4> aff;
+        aff.request(norm, ct * 16 + quad * 4);
+        aff.finish(norm, sc[ct], sh[ct]);
+    }
 
     const int per_image = tiles_x * tiles_y, total = N * per_image;
+    // The image part of a tile, one pixel of three channels per item: requested a tile
+    // ahead, while the matrix cores work on the one before.
+    constexpr int RI = (kImgRows * kImgCols + kThreads - 1) / kThreads;
+    short pix[RI][3];
+    auto request = [&](int t) {
+        const int n = t / per_image, r = t - n * per_image, ty = r / tiles_x, tx = r - ty * tiles_x;
+        const int iy0 = 4 * ty * kPoolTile - 5, ix0 = 4 * tx * kPoolTile - 5;   // first image pixel
+        const uint32_t plane_b = (uint32_t)(H * W) * 2;
+        const __amdgpu_buffer_rsrc_t in = plane_rsrc(img + (int64_t)n * 3 * H * W, 3 * plane_b);
+#pragma unroll
+        for (int k = 0; k < RI; ++k) {
+            const int i = tid + k * kThreads;
+            const int yy = iy0 + i / kImgCols, xx = ix0 + i % kImgCols;
+            const uint32_t off = (yy >= 0 && yy < H && xx >= 0 && xx < W) ? (uint32_t)(yy * W + xx) * 2 : kOutside;
+#pragma unroll
+            for (int ch = 0; ch < 3; ++ch)
+                pix[k][ch] = __builtin_amdgcn_raw_buffer_load_b16(in, (int)off, (int)(ch * plane_b), 0);
+        }
+    };
+    if ((int)blockIdx.x < total) request(blockIdx.x);
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         const int n = t / per_image, r = t - n * per_image, ty = r / tiles_x, tx = r - ty * tiles_x;
         const int cy0 = 2 * ty * kPoolTile - 1, cx0 = 2 * tx * kPoolTile - 1;   // first convolution result
-        const int iy0 = 2 * cy0 - 3, ix0 = 2 * cx0 - 3;                         // first image pixel
-        const _Float16 *in = img + (int64_t)n * 3 * H * W;
-        for (int i = tid; i < kImgRows * kImgCols; i += kThreads) {
-            const int yy = iy0 + i / kImgCols, xx = ix0 + i % kImgCols;
-            half4_t v = {0, 0, 0, 0};
-            if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
-                const int64_t at = (int64_t)yy * W + xx;
 #pragma unroll
-                for (int ch = 0; ch < 3; ++ch) v[ch] = in[at + (int64_t)ch * H * W];
-            }
-            *reinterpret_cast<half4_t *>(tile + i * 4) = v;
+        for (int k = 0; k < RI; ++k) {
+            const int i = tid + k * kThreads;
+            half4_t v = {0, 0, 0, 0};
+#pragma unroll
+            for (int ch = 0; ch < 3; ++ch) v[ch] = __builtin_bit_cast(_Float16, pix[k][ch]);
+            if (i < kImgRows * kImgCols) *reinterpret_cast<half4_t *>(tile + i * 4) = v;
         }
+        if (t + (int)gridDim.x < total) request(t + gridDim.x);
         __syncthreads();   // (also: the weights, or the last tile's results, have been read)
         for (int pt = wave; pt < kStemTiles; pt += kThreads / kWave) {
             const int px = pt * 16 + row, pc = min(px, kStemPixels - 1);
@@ -564,6 +645,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     const _Float16 *sn = sf + ((int64_t)n * Ho + y) * Wo * kTapPitch;
     _Float16 *on = out + ((int64_t)n * Ho + y) * Wo * C + cl * 8;
 
+    Affine<8> aff;
+    aff.request(norm, cl * 8);
     uint32_t cfp[KK][4];
     {
         const uint4 *src = reinterpret_cast<const uint4 *>(cf + ((int64_t)n * C + cl * 8) * KK);
@@ -579,10 +662,6 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 #pragma unroll
             for (int k = 0; k < 4; ++k) cfp[t][k] = half_at(18 * k + t) | (half_at(18 * k + 9 + t) << 16);
     }
-    float sc[8], sh[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) affine(norm, cl * 8 + e, sc[e], sh[e]);
-
     uint32_t rowo[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -599,6 +678,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                 xr, (int)(in && rowo[i] != kOutside ? rowo[i] + (uint32_t)xx * C * 2 : kOutside), 0, 0));
         return c;
     };
+    float sc[8], sh[8];
     struct Taps { uint2 v[3]; };
     auto taps = [&](int xx) {
         Taps t;
@@ -642,6 +722,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     if constexpr (S == 1) {
         Column c0 = column(x0 - 1), c1 = column(x0), c2 = column(x0 + 1), c3;
         Taps t0 = taps(x0), t1;
+        aff.finish(norm, sc, sh);
         for (int j = 0; j < run; j += 4) {
             const int xx = x0 + j;
             c3 = column(xx + 2); t1 = taps(xx + 1);
@@ -657,6 +738,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     } else {
         Column l = column(2 * x0 - 1), m = column(2 * x0), rr = column(2 * x0 + 1);
         Taps t0 = taps(x0), t1;
+        aff.finish(norm, sc, sh);
         for (int j = 0; j < run; j += 2) {
             const int xx = x0 + j;
             Column m2 = column(2 * xx + 2), r2 = column(2 * xx + 3);
@@ -739,7 +821,7 @@ hipError_t net_conv(const NetConv &a, hipStream_t st) {
 
 hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,
                     hipStream_t st) {
-    if (H % 4 != 0 || W % 4 != 0 || H * W >= (1 << 28)) return hipErrorNotSupported;
+    if (H % 4 != 0 || W % 4 != 0 || H * W >= (1 << 27)) return hipErrorNotSupported;
     const int tx = (int)cdiv(W / 4, kPoolTile), ty = (int)cdiv(H / 4, kPoolTile);
     const int64_t tiles = N * tx * ty;
     if (tiles == 0) return hipSuccess;
@@ -793,12 +875,19 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
     if (most < 1) return hipErrorNotSupported;
     for (int64_t n0 = 0; n0 < N; n0 += most) {
         const int64_t cnt = std::min(most, N - n0);
-        // Walks as long as leave 4096 waves, in whole rounds of the kernel's unrolled steps
-        // (every walk loads its channel taps and two columns it does not produce).
-        int64_t runs = cdiv((int64_t)4096 * slots, cnt * Ho);
-        runs = std::max<int64_t>(1, std::min<int64_t>(runs, cdiv(Wo, step)));
-        const int run = (int)(cdiv(cdiv(Wo, runs), step) * step);
-        runs = cdiv(Wo, run);
+        // The walk: whole rounds of the kernel's unrolled steps; the length that takes the
+        // fewest steps over the rounds of resident waves it makes (three per SIMD), each walk
+        // paying for its channel taps, its BatchNorm and two columns it does not produce.
+        constexpr int kResident = 3072, kEntry = 6;
+        int run = step;
+        int64_t best = 0;
+        for (int cand = step; ; cand += step) {
+            const int64_t waves = cdiv(cnt * Ho * cdiv(Wo, cand), slots);
+            const int64_t cost = cdiv(waves, kResident) * (cand + kEntry);
+            if (best == 0 || cost < best) { best = cost; run = cand; }
+            if (cand >= Wo) break;
+        }
+        const int64_t runs = cdiv(Wo, run);
         const int64_t units = cnt * Ho * runs, blocks = cdiv(units, slots * (kThreads / kWave));
         if (units > (1 << 30)) return hipErrorInvalidConfiguration;
         const _Float16 *xn = (const _Float16 *)x + n0 * H * W * C, *cn = (const _Float16 *)cf + n0 * C * 9,
