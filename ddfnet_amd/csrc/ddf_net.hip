@@ -250,13 +250,14 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
     }
 }
 
-// Few pixels or a small batch, where tiles of 64 leave most of the chip idle: a workgroup
-// takes 32 pixels x 32 channels, its WAVES waves a range of K each, operands straight from
-// memory (every value is used by one wave only), eight steps of them requested ahead of use;
-// the waves' sums meet in LDS.
-template <int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int tiles_n) {
-    constexpr int U = 4, P = 33;
+// Few pixels, where tiles of 64 leave most of the chip idle: a workgroup takes 32 pixels x 32
+// channels, its four waves a quarter of K each, operands straight from memory (every value
+// is used by one wave only); the waves' sums meet in LDS.  K goes by in blocks of 64 of which
+// a lane takes one half, 64 contiguous bytes in four loads (the order of the summed
+// dimension is free as long as both operands agree): the 32 rows a load touches are 128-byte
+// lines that are used up at once instead of being fetched again by later steps.
+__global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tiles_n) {
+    constexpr int WAVES = kThreads / kWave, U = 4, P = 33;
     __shared__ float red[WAVES][32][P];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -270,11 +271,11 @@ __global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int
         const int p = (int)(m - n * a.npix), y = p / a.Wo, xx = p - y * a.Wo;
         m = (n * a.H + y * a.stride) * a.W + xx * a.stride;
     }
-    const int steps = a.K / 16, per = (steps + WAVES - 1) / WAVES;
-    const int s0 = wave * per, s1 = min(s0 + per, steps);
-    const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + hi * 8;
-    const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + l32, a.N - 1) * a.K + hi * 8;
-    // (a thread finishes one channel of 32 / (2 * WAVES) pixels: 64-byte runs of a pixel's channels)
+    const int blocks = a.K / 64, per = (blocks + WAVES - 1) / WAVES;
+    const int b0 = wave * per, b1 = min(b0 + per, blocks);
+    const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + hi * 32;
+    const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + l32, a.N - 1) * a.K + hi * 32;
+    // (a thread finishes one channel of four pixels: 64-byte runs of a pixel's channels)
     constexpr int PX = 2 * WAVES, RO = 32 / PX;
     const int oc = n0 + (tid & 31);
     const bool cok = oc < a.N;
@@ -285,39 +286,39 @@ __global__ __launch_bounds__(WAVES * kWave) void k_net_conv_small(NetConv a, int
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.f;
     half8_t xv[2][U], wv[2][U];
-    auto request = [&](auto set, int s) {
+    auto request = [&](auto set, int b) __attribute__((always_inline)) {
         constexpr int B = decltype(set)::value;
+        const int k = min(b, blocks - 1) * 64;    // (past the wave's range: not used)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = min(s + u, steps - 1) * 16;    // (past the wave's range: not used)
-            xv[B][u] = *reinterpret_cast<const half8_t *>(xp + k);
-            wv[B][u] = *reinterpret_cast<const half8_t *>(wp + k);
+            xv[B][u] = *reinterpret_cast<const half8_t *>(xp + k + u * 8);
+            wv[B][u] = *reinterpret_cast<const half8_t *>(wp + k + u * 8);
         }
     };
-    auto use = [&](auto set, int s) {
+    auto use = [&](auto set, int b) __attribute__((always_inline)) {
         constexpr int B = decltype(set)::value;
+        if (b < b1) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (s + u < s1) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[B][u], xv[B][u], acc, 0, 0, 0);
+            for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[B][u], xv[B][u], acc, 0, 0, 0);
+        }
     };
     using Zero = std::integral_constant<int, 0>;
     using One = std::integral_constant<int, 1>;
-    if (s0 < s1) request(Zero{}, s0);
+    if (b0 < b1) {
+        request(Zero{}, b0);
+        request(One{}, b0 + 1);
+    }
     aff.request(a.norm, cok ? oc : 0);
 #pragma unroll
     for (int i = 0; i < RO; ++i) {
         const int64_t mm = (int64_t)tm * 32 + (tid >> 5) + i * PX;
         rv[i] = res ? res[(mm < a.M ? mm : a.M - 1) * a.N + (cok ? oc : 0)] : (_Float16)0;
     }
-    if (s0 < s1) {
-        for (int s = s0; s < s1; s += 2 * U) {
-            request(One{}, s + U);
-            __builtin_amdgcn_sched_barrier(0);
-            use(Zero{}, s);
-            request(Zero{}, s + 2 * U);
-            __builtin_amdgcn_sched_barrier(0);
-            use(One{}, s + U);
-        }
+    for (int b = b0; b < b1; b += 2) {
+        use(Zero{}, b);
+        if (b + 2 < b1) request(Zero{}, b + 2);
+        use(One{}, b + 1);
+        if (b + 3 < b1) request(One{}, b + 3);
     }
 #pragma unroll
     for (int g = 0; g < 4; ++g)
@@ -627,7 +628,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                                                          const _Float16 *__restrict__ cf,
                                                          const _Float16 *__restrict__ sf, NetNorm norm,
                                                          _Float16 *__restrict__ out, int H, int W, int Ho, int Wo,
-                                                         int runs, int run, int units, int blocks, uint32_t x_bytes) {
+                                                         int runs, int run, int units, int blocks, uint32_t x_bytes,
+                                                         uint32_t out_bytes) {
     constexpr int C = LP * 8, SLOTS = kWave / LP, KK = 9;
     const int block = xcd_block(blockIdx.x, blocks);
     if (block >= blocks) return;
@@ -643,7 +645,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     // (lanes of a wave may belong to different samples: one descriptor over all of them)
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x, x_bytes);
     const _Float16 *sn = sf + ((int64_t)n * Ho + y) * Wo * kTapPitch;
-    _Float16 *on = out + ((int64_t)n * Ho + y) * Wo * C + cl * 8;
+    const __amdgpu_buffer_rsrc_t orr = plane_rsrc(out, out_bytes);
+    const uint32_t oo = (uint32_t)(((n * Ho + y) * Wo) * C + cl * 8) * 2;
 
     Affine<8> aff;
     aff.request(norm, cl * 8);
@@ -668,26 +671,32 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
         const int yy = y * S - 1 + i;
         rowo[i] = (live && yy >= 0 && yy < H) ? (uint32_t)(((n * H + yy) * W) * C + cl * 8) * 2 : kOutside;
     }
-    struct Column { rows_u4 v[3]; };
-    auto column = [&](int xx) {
-        Column c;
+    float sc[8], sh[8];
+    // Columns in rings of registers, all indices constants (as structures handed around they
+    // were parked in LDS, and every step waited for its own loads: 60 us where this takes 25
+    // at 128 x 56 x 56 x 64).
+    constexpr int RING = S == 1 ? 4 : 6;
+    uint32_t col[RING][3][4], tap[2][6];
+    auto column = [&](auto slot, int xx) __attribute__((always_inline)) {
+        constexpr int J = decltype(slot)::value % RING;
         const bool in = xx >= 0 && xx < W;
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-            c.v[i] = __builtin_bit_cast(rows_u4, __builtin_amdgcn_raw_buffer_load_b128(
-                xr, (int)(in && rowo[i] != kOutside ? rowo[i] + (uint32_t)xx * C * 2 : kOutside), 0, 0));
-        return c;
+            load_words<4>(xr, in && rowo[i] != kOutside ? rowo[i] + (uint32_t)xx * C * 2 : kOutside, col[J][i]);
     };
-    float sc[8], sh[8];
-    struct Taps { uint2 v[3]; };
-    auto taps = [&](int xx) {
-        Taps t;
+    auto taps = [&](auto slot, int xx) __attribute__((always_inline)) {
+        constexpr int J = decltype(slot)::value % 2;
         const uint2 *p = reinterpret_cast<const uint2 *>(sn + (int64_t)min(xx, Wo - 1) * kTapPitch);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) t.v[i] = p[i];
-        return t;
+        for (int i = 0; i < 3; ++i) {
+            const uint2 q = p[i];
+            tap[J][2 * i] = q.x;
+            tap[J][2 * i + 1] = q.y;
+        }
     };
-    auto emit = [&](const Column &a, const Column &b, const Column &c, const Taps &tp, int xx) {
+    // result xx from the columns in slots A, A + 1 and A + 2 and the taps in slot J
+    auto emit = [&](auto first, auto slot, int xx) __attribute__((always_inline)) {
+        constexpr int A = decltype(first)::value, J = decltype(slot)::value % 2;
         float acc[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = 0.f;
@@ -696,16 +705,13 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const int t = i * 3 + j;
-                const uint2 sw = tp.v[t / 4];
-                const half2_t sp = __builtin_bit_cast(half2_t, (t % 4) < 2 ? sw.x : sw.y);
+                const half2_t sp = __builtin_bit_cast(half2_t, tap[J][t / 2]);
                 const half2_t sv = {sp[t & 1], sp[t & 1]};
-                const rows_u4 q = j == 0 ? a.v[i] : j == 1 ? b.v[i] : c.v[i];
-                const uint32_t xw[4] = {q[0], q[1], q[2], q[3]};
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const half2_t cv = __builtin_bit_cast(half2_t, cfp[t][k]);
                     const half2_t cb = MUL ? cv * sv : cv + sv;
-                    const half2_t xv = __builtin_bit_cast(half2_t, xw[k]);
+                    const half2_t xv = __builtin_bit_cast(half2_t, col[(A + j) % RING][i][k]);
                     acc[2 * k] = fmaf((float)xv[0], (float)cb[0], acc[2 * k]);
                     acc[2 * k + 1] = fmaf((float)xv[1], (float)cb[1], acc[2 * k + 1]);
                 }
@@ -717,41 +723,48 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
             const float f = fmaf((float)(_Float16)acc[e], sc[e], sh[e]);
             o[e] = (_Float16)relu(f);
         }
-        if (xx < x1) *reinterpret_cast<half8_t *>(on + (int64_t)xx * C) = o;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, o), orr,
+                                               (int)(xx < x1 ? oo + (uint32_t)xx * C * 2 : kOutside), 0, 0);
     };
+#define DDF_I(v) std::integral_constant<int, (v)>{}
     if constexpr (S == 1) {
-        Column c0 = column(x0 - 1), c1 = column(x0), c2 = column(x0 + 1), c3;
-        Taps t0 = taps(x0), t1;
+        column(DDF_I(0), x0 - 1);
+        column(DDF_I(1), x0);
+        column(DDF_I(2), x0 + 1);
+        taps(DDF_I(0), x0);
         aff.finish(norm, sc, sh);
         for (int j = 0; j < run; j += 4) {
-            const int xx = x0 + j;
-            c3 = column(xx + 2); t1 = taps(xx + 1);
-            emit(c0, c1, c2, t0, xx);
-            c0 = column(xx + 3); t0 = taps(xx + 2);
-            emit(c1, c2, c3, t1, xx + 1);
-            c1 = column(xx + 4); t1 = taps(xx + 3);
-            emit(c2, c3, c0, t0, xx + 2);
-            c2 = column(xx + 5); t0 = taps(xx + 4);
-            emit(c3, c0, c1, t1, xx + 3);
-            // (the window is c0 c1 c2 again: columns xx + 3, xx + 4, xx + 5)
+            rows::static_for<0, 4>([&](auto q) __attribute__((always_inline)) {
+                constexpr int Q = decltype(q)::value;
+                const int xx = x0 + j + Q;
+                column(DDF_I(Q + 3), xx + 2);
+                taps(DDF_I(Q + 1), xx + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                emit(DDF_I(Q), q, xx);
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
     } else {
-        Column l = column(2 * x0 - 1), m = column(2 * x0), rr = column(2 * x0 + 1);
-        Taps t0 = taps(x0), t1;
+        // (three pairs of columns: slots 2q - 1, 2q and 2q + 1 are under result q)
+        column(DDF_I(5), 2 * x0 - 1);
+        column(DDF_I(0), 2 * x0);
+        column(DDF_I(1), 2 * x0 + 1);
+        taps(DDF_I(0), x0);
         aff.finish(norm, sc, sh);
-        for (int j = 0; j < run; j += 2) {
-            const int xx = x0 + j;
-            Column m2 = column(2 * xx + 2), r2 = column(2 * xx + 3);
-            t1 = taps(xx + 1);
-            emit(l, m, rr, t0, xx);
-            m = column(2 * xx + 4);
-            Column r3 = column(2 * xx + 5);
-            t0 = taps(xx + 2);
-            emit(rr, m2, r2, t1, xx + 1);
-            l = r2;
-            rr = r3;
+        for (int j = 0; j < run; j += 6) {
+            rows::static_for<0, 6>([&](auto q) __attribute__((always_inline)) {
+                constexpr int Q = decltype(q)::value;
+                const int xx = x0 + j + Q;
+                column(DDF_I(2 * Q + 2), 2 * xx + 2);
+                column(DDF_I(2 * Q + 3), 2 * xx + 3);
+                taps(DDF_I(Q + 1), xx + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                emit(DDF_I(2 * Q + 5), q, xx);
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
     }
+#undef DDF_I
 }
 
 // ---- mean over the pixels -----------------------------------------------------------
@@ -801,21 +814,22 @@ bool net_conv_supported(const NetConv &a) { return a.K % kStep == 0 && a.K > 0 &
 hipError_t net_conv(const NetConv &a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_conv_supported(a)) return hipErrorNotSupported;
-    // The largest tiles that leave two workgroups per compute unit; whole vectors of
-    // channels for all but the small kernel.
+    // The largest tiles that leave somewhat more than a workgroup per compute unit (measured
+    // over batches of 1 to 128 of the network's twelve products: 128 x 128 from 392 tiles on,
+    // 64 x 64 below); the splitting kernel where even tiles of 64 are few and K is long enough
+    // to split (56 x 64 -> 256 at batch 1: 4.9 us in tiles of 64, 15 split; 14 x 14 x 1024 -> 256:
+    // 9.0 and 7.1), and for odd channel counts.
     auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
-    if (a.N % 8 == 0) {
-        if (a.N >= 128 && count(128, 128) >= 512) return launch_conv<128, 128>(a, st);
-        if (count(128, 64) >= 512) return launch_conv<128, 64>(a, st);
-        if (count(64, 64) >= 256) return launch_conv<64, 64>(a, st);
+    constexpr int kEnough = 320;
+    if (a.N % 8 == 0 && !(a.K >= 512 && count(64, 64) <= 64)) {
+        if (a.N >= 128 && count(128, 128) >= kEnough) return launch_conv<128, 128>(a, st);
+        if (count(128, 64) >= kEnough) return launch_conv<128, 64>(a, st);
+        return launch_conv<64, 64>(a, st);
     }
     const int tiles_n = (int)cdiv(a.N, 32);
     const int64_t blocks = cdiv(a.M, 32) * tiles_n;
     if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
-    if (a.K >= 256)
-        hipLaunchKernelGGL((k_net_conv_small<8>), dim3((unsigned)blocks), dim3(8 * kWave), 0, st, a, tiles_n);
-    else
-        hipLaunchKernelGGL((k_net_conv_small<4>), dim3((unsigned)blocks), dim3(4 * kWave), 0, st, a, tiles_n);
+    hipLaunchKernelGGL(k_net_conv_split, dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
     return hipGetLastError();
 }
 
@@ -867,7 +881,7 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
                       int64_t H, int64_t W, int64_t C, int stride, bool mul, hipStream_t st) {
     const int64_t Ho = H / stride, Wo = W / stride;
     if (N * Ho * Wo == 0) return hipSuccess;
-    const int step = stride == 1 ? 4 : 2;
+    const int step = stride == 1 ? 4 : 6;
     if (C < 8 || C > kWave * 8) return hipErrorNotSupported;
     const int slots = (int)(kWave * 8 / C);
     // (32-bit offsets: as many samples at a time as stay below 2 GiB)
@@ -897,7 +911,7 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
 #define DDF_NET_FILTER_LAUNCH(LP_, S_, MUL_)                                                                     \
     hipLaunchKernelGGL((k_net_filter<LP_, S_, MUL_>), dim3(xcd_grid(blocks)), dim3(kThreads), 0, st, xn, cn, sn, \
                        norm, on, (int)H, (int)W, (int)Ho, (int)Wo, (int)runs, run, (int)units, (int)blocks,      \
-                       (uint32_t)(cnt * sample))
+                       (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2))
 #define DDF_NET_FILTER(LP_, S_)                            \
     if (C == LP_ * 8 && stride == S_) {                    \
         if (mul) DDF_NET_FILTER_LAUNCH(LP_, S_, true);     \

@@ -106,13 +106,12 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
     }
     const size_t wide_b = aligned_bytes(wide * 2), narrow_b = aligned_bytes(narrow * 2), taps_b = aligned_bytes(taps * 2),
                  filters_b = aligned_bytes(filters * 2), parts_b = aligned_bytes(parts * 4);
-    at::Tensor work = at::empty({(int64_t)(2 * wide_b + 2 * narrow_b + taps_b + filters_b + parts_b)},
-                                x.options().dtype(at::kByte));
+    at::Tensor work = new_tensor({(int64_t)(2 * wide_b + 2 * narrow_b + taps_b + filters_b + parts_b)}, at::kByte, x.device());
     char *q = static_cast<char *>(work.data_ptr());
     void *cur = q, *other = q + wide_b, *t1 = q + 2 * wide_b, *t2 = q + 2 * wide_b + narrow_b;
     void *sf = q + 2 * wide_b + 2 * narrow_b, *cf = static_cast<char *>(sf) + taps_b;
     float *pp = reinterpret_cast<float *>(static_cast<char *>(cf) + filters_b);
-    at::Tensor logits = at::empty({n, p.fc.t[0].size(0)}, x.options());
+    at::Tensor logits = new_tensor({n, p.fc.t[0].size(0)}, at::kHalf, dev);
     {
         py::gil_scoped_release release;    // (a network's launches take a while)
         ddf_net_norm_t nm = p.stem.norm();

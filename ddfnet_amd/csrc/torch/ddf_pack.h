@@ -76,12 +76,12 @@ inline at::Tensor pack_infer(const PackPlan &p, const at::Tensor &features) {
     const int64_t ho = h / p.s, wo = w / p.s, kk = (int64_t)p.k * p.k;
     c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
     hipStream_t st = current_stream(x);
-    at::Tensor out = at::empty({b, c, ho, wo}, x.options());
+    at::Tensor out = new_tensor({b, c, ho, wo}, x.scalar_type(), x.device());
     // both filters and the partial sums in one piece of scratch
     const size_t esz = x.element_size();
     const size_t cf_bytes = aligned_bytes(b * c * kk * esz), sf_bytes = aligned_bytes(b * p.head * kk * ho * wo * esz);
     const int64_t cap = p.fuse_pool ? b * c * ((ho * wo + 63) / 64 + 1) : 0;
-    at::Tensor scratch = at::empty({(int64_t)(cf_bytes + sf_bytes + cap * sizeof(float))}, x.options().dtype(at::kByte));
+    at::Tensor scratch = new_tensor({(int64_t)(cf_bytes + sf_bytes + cap * sizeof(float))}, at::kByte, x.device());
     char *base = static_cast<char *>(scratch.data_ptr());
     void *cf = base, *sf = base + cf_bytes;
     // The spatial branch reads every feature plane anyway: where its kernel can, it leaves
@@ -147,10 +147,10 @@ public:
         const int dt = dtype_code(x.scalar_type());
         c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
         hipStream_t st = current_stream(x);
-        at::Tensor out = at::empty({z.b, z.c, z.ho, z.wo}, x.options());
-        at::Tensor saved = at::empty({(int64_t)z.saved}, x.options().dtype(at::kByte));
+        at::Tensor out = new_tensor({z.b, z.c, z.ho, z.wo}, x.scalar_type(), x.device());
+        at::Tensor saved = new_tensor({(int64_t)z.saved}, at::kByte, x.device());
         const int64_t cap = z.b * z.c * ((z.ho * z.wo + 63) / 64 + 1);
-        at::Tensor parts = at::empty({cap}, x.options().dtype(at::kFloat));
+        at::Tensor parts = new_tensor({cap}, x.options().dtype(at::kFloat));
         char *q = static_cast<char *>(saved.data_ptr());
         void *cf = q, *sf = q + z.cf, *raw = q + z.cf + z.sf;
         float *pooled = reinterpret_cast<float *>(q + z.cf + 2 * z.sf);
@@ -184,18 +184,19 @@ public:
         const size_t op_bytes = aligned_bytes(ddf_hip_backward_spatial_norm_workspace_bytes(
             n, cg, z.h, z.w, k, d, s, combine, dt, need, DDF_VARIANT_AUTO));
         const size_t br_bytes = ddf_hip_pack_backward_workspace_bytes(z.b, z.c, z.h, z.w, z.mid, head, k, s, dt);
-        at::Tensor work = at::empty({(int64_t)(z.cf + z.sf + op_bytes + br_bytes)}, x.options().dtype(at::kByte));
+        at::Tensor work = new_tensor({(int64_t)(z.cf + z.sf + op_bytes + br_bytes)}, at::kByte, x.device());
         char *wq = static_cast<char *>(work.data_ptr());
         void *dcf = wq, *draw = wq + z.cf, *op_ws = wq + z.cf + z.sf, *br_ws = wq + z.cf + z.sf + op_bytes;
         char *q = static_cast<char *>(saved.data_ptr());
         void *cf = q, *sf = q + z.cf, *raw = q + z.cf + z.sf;
         float *pooled = reinterpret_cast<float *>(q + z.cf + 2 * z.sf);
         float *hidden = pooled + z.pooled / sizeof(float), *taps = hidden + z.hidden / sizeof(float);
+        auto like = [&](const at::Tensor &t) { return new_tensor(t.sizes(), t.scalar_type(), x.device()); };
         at::Tensor dx;
-        if (want_dx) dx = at::empty_like(x);
-        at::Tensor dws = at::empty_like(ws), dw1 = at::empty_like(w1), dw2 = at::empty_like(w2),
-                   dgain = at::empty_like(gain_vec), dbs = at::empty_like(sv[5]), db1 = at::empty_like(sv[6]),
-                   db2 = at::empty_like(sv[7]);
+        if (want_dx) dx = like(x);
+        at::Tensor dws = like(ws), dw1 = like(w1), dw2 = like(w2),
+                   dgain = like(gain_vec), dbs = like(sv[5]), db1 = like(sv[6]),
+                   db2 = like(sv[7]);
         void *dxp = want_dx ? dx.data_ptr() : nullptr;
         check_status(ddf_hip_backward_spatial_norm(
             go.data_ptr(), x.data_ptr(), cf, sf, raw, dxp, dcf, draw, nullptr, op_ws, op_bytes, n, cg, z.h, z.w, k, d,

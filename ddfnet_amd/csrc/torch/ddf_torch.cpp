@@ -11,7 +11,12 @@
 
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/VariableTypeUtils.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
 #include <sstream>
 #include <string>
@@ -64,71 +69,59 @@ inline hipStream_t current_stream(const at::Tensor &t) {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
-class DDFAutograd : public torch::autograd::Function<DDFAutograd> {
-public:
-    // Operands are contiguous device tensors of one supported dtype with matching
-    // shapes (ddf() below has seen to that).
-    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &features,
-                              const at::Tensor &channel_filter, const at::Tensor &spatial_filter,
-                              int64_t k, int64_t d, int64_t s, int64_t combine, int64_t variant) {
-        const int64_t b = features.size(0), c = features.size(1), h = features.size(2),
-                      w = features.size(3);
-        // the kernels write every element, so no zero fill
-        at::Tensor out = at::empty({b, c, h / s, w / s}, features.options());
-        {
-            c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(features.device());
-            check_status(ddf_hip_forward(features.data_ptr(), channel_filter.data_ptr(),
-                                         spatial_filter.data_ptr(), out.data_ptr(), b, c, h, w,
-                                         (int)k, (int)d, (int)s, (int)combine,
-                                         dtype_code(features.scalar_type()), (int)variant,
-                                         current_stream(features)));
-        }
-        if (features.requires_grad() || channel_filter.requires_grad() || spatial_filter.requires_grad())
-            ctx->save_for_backward({features, channel_filter, spatial_filter});
-        ctx->saved_data["k"] = k;
-        ctx->saved_data["d"] = d;
-        ctx->saved_data["s"] = s;
-        ctx->saved_data["combine"] = combine;
-        ctx->saved_data["variant"] = variant;
-        return out;
-    }
+// A new device tensor, without the dispatcher (every kernel of the library writes every
+// element, so nothing has to be filled in either).
+inline at::Tensor new_tensor(c10::IntArrayRef sizes, at::ScalarType type, const at::Device &device) {
+    return at::Tensor(at::detail::empty_cuda(sizes, type, device, c10::nullopt));
+}
 
-    static variable_list backward(AutogradContext *ctx, variable_list grads) {
-        const auto saved = ctx->get_saved_variables();
-        const at::Tensor &features = saved[0], &channel_filter = saved[1], &spatial_filter = saved[2];
-        const int k = (int)ctx->saved_data["k"].toInt(), d = (int)ctx->saved_data["d"].toInt(),
-                  s = (int)ctx->saved_data["s"].toInt(),
-                  combine = (int)ctx->saved_data["combine"].toInt();
-        // 'f' forces the tiled kernels in the forward pass only (the reference's
-        // faster modules export no backward)
-        const int variant = ctx->saved_data["variant"].toInt() == DDF_VARIANT_GENERIC
-                                ? DDF_VARIANT_GENERIC : DDF_VARIANT_AUTO;
-        if (!grads[0].is_cuda()) assertion_error("");
-        const at::Tensor go = grads[0].to(features.scalar_type()).contiguous();
+inline bool has_tangent(const at::Tensor &t) { return torch::autograd::isFwGradDefined(t); }
+
+// The operator's gradient as a node of the autograd graph.  (A torch::autograd::Function
+// does the same through a generic context - argument lists, a dictionary of boxed values,
+// lists of optional results - at a few microseconds per call and direction.)
+struct DDFNode : public torch::autograd::Node {
+    torch::autograd::SavedVariable features_, channel_filter_, spatial_filter_;
+    int k, d, s, combine, variant;
+
+    std::string name() const override { return "DDFBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        features_.reset_data();
+        channel_filter_.reset_data();
+        spatial_filter_.reset_data();
+    }
+    variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list result(3);
+        if (!grads[0].defined()) return result;
+        const at::Tensor features = features_.unpack(), channel_filter = channel_filter_.unpack(),
+                         spatial_filter = spatial_filter_.unpack();
+        const at::ScalarType type = features.scalar_type();
+        const at::Device device = features.device();
+        at::Tensor go = std::move(grads[0]);
+        if (!go.is_cuda()) assertion_error("");
+        if (go.scalar_type() != type) go = go.to(type);
+        if (!go.is_contiguous()) go = go.contiguous();
 
         // only the gradients autograd asks for are computed
         unsigned need = 0;
-        at::Tensor dx, dcf, dsf;
-        if (ctx->needs_input_grad(0)) { need |= DDF_NEED_DX; dx = at::empty_like(features); }
-        if (ctx->needs_input_grad(1)) { need |= DDF_NEED_DCF; dcf = at::empty_like(channel_filter); }
-        if (ctx->needs_input_grad(2)) { need |= DDF_NEED_DSF; dsf = at::empty_like(spatial_filter); }
-        if (need) {
-            const int64_t b = features.size(0), c = features.size(1), h = features.size(2),
-                          w = features.size(3);
-            const int dt = dtype_code(features.scalar_type());
-            c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(features.device());
-            const size_t bytes = ddf_hip_backward_workspace_bytes(b, c, h, w, k, d, s, combine, dt,
-                                                                  need, variant);
-            at::Tensor ws;
-            if (bytes) ws = at::empty({(int64_t)bytes}, features.options().dtype(at::kByte));
-            check_status(ddf_hip_backward(
-                go.data_ptr(), features.data_ptr(), channel_filter.data_ptr(),
-                spatial_filter.data_ptr(), dx.defined() ? dx.data_ptr() : nullptr,
-                dcf.defined() ? dcf.data_ptr() : nullptr, dsf.defined() ? dsf.data_ptr() : nullptr,
-                bytes ? ws.data_ptr() : nullptr, bytes, b, c, h, w, k, d, s, combine, dt, need,
-                variant, current_stream(features)));
-        }
-        return {dx, dcf, dsf, at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+        if (task_should_compute_output(0)) { need |= DDF_NEED_DX; result[0] = new_tensor(features.sizes(), type, device); }
+        if (task_should_compute_output(1)) { need |= DDF_NEED_DCF; result[1] = new_tensor(channel_filter.sizes(), type, device); }
+        if (task_should_compute_output(2)) { need |= DDF_NEED_DSF; result[2] = new_tensor(spatial_filter.sizes(), type, device); }
+        if (!need) return result;
+        const int64_t b = features.size(0), c = features.size(1), h = features.size(2), w = features.size(3);
+        const int dt = dtype_code(type);
+        c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device);
+        const size_t bytes = ddf_hip_backward_workspace_bytes(b, c, h, w, k, d, s, combine, dt, need, variant);
+        at::Tensor ws;
+        if (bytes) ws = new_tensor({(int64_t)bytes}, at::kByte, device);
+        auto ptr = [](const at::Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; };
+        check_status(ddf_hip_backward(go.data_ptr(), features.data_ptr(), channel_filter.data_ptr(),
+                                      spatial_filter.data_ptr(), ptr(result[0]), ptr(result[1]), ptr(result[2]),
+                                      ptr(ws), bytes, b, c, h, w, k, d, s, combine, dt, need, variant,
+                                      current_stream(features)));
+        return result;
     }
 };
 
@@ -159,9 +152,10 @@ at::Tensor ddf(at::Tensor features, at::Tensor channel_filter, at::Tensor spatia
     if (features.dim() != 4 || channel_filter.dim() != 4 || spatial_filter.dim() != 4)
         assertion_error("features, channel_filter and spatial_filter must be 4-dimensional");
     if (stride < 1) assertion_error("");
-    features = features.to(dtype).contiguous();
-    channel_filter = channel_filter.to(dtype).contiguous();
-    spatial_filter = spatial_filter.to(dtype).contiguous();
+    for (at::Tensor *t : {&features, &channel_filter, &spatial_filter}) {
+        if (t->scalar_type() != dtype) *t = t->to(dtype);
+        if (!t->is_contiguous()) *t = t->contiguous();
+    }
 
     const int64_t b = features.size(0), c = features.size(1), h = features.size(2), w = features.size(3);
     const int64_t out_h = h / stride, out_w = w / stride;
@@ -189,9 +183,37 @@ at::Tensor ddf(at::Tensor features, at::Tensor channel_filter, at::Tensor spatia
     else if (version == "f") variant = DDF_VARIANT_TILED;
     else assertion_error("version must be '', 'o' or 'f', instead of " + version);
 
-    return DDFAutograd::apply(features, channel_filter, spatial_filter, kernel_size, dilation, stride,
-                              (int64_t)combine, (int64_t)variant);
+    at::Tensor out = new_tensor({b, c, out_h, out_w}, dtype, features.device());
+    {
+        c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(features.device());
+        check_status(ddf_hip_forward(features.data_ptr(), channel_filter.data_ptr(), spatial_filter.data_ptr(),
+                                     out.data_ptr(), b, c, h, w, (int)kernel_size, (int)dilation, (int)stride, combine,
+                                     dtype_code(dtype), variant, current_stream(features)));
+    }
+    if (at::GradMode::is_enabled() &&
+        (features.requires_grad() || channel_filter.requires_grad() || spatial_filter.requires_grad())) {
+        if (has_tangent(features) || has_tangent(channel_filter) || has_tangent(spatial_filter))
+            throw std::runtime_error("ddf has no forward-mode derivative");
+        auto node = std::shared_ptr<DDFNode>(new DDFNode(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(features, channel_filter, spatial_filter));
+        node->k = (int)kernel_size;
+        node->d = (int)dilation;
+        node->s = (int)stride;
+        node->combine = combine;
+        // 'f' forces the tiled kernels in the forward pass only (the reference's
+        // faster modules export no backward)
+        node->variant = variant == DDF_VARIANT_GENERIC ? DDF_VARIANT_GENERIC : DDF_VARIANT_AUTO;
+        node->features_ = torch::autograd::SavedVariable(features, false);
+        node->channel_filter_ = torch::autograd::SavedVariable(channel_filter, false);
+        node->spatial_filter_ = torch::autograd::SavedVariable(spatial_filter, false);
+        torch::autograd::set_history(out, node);
+    }
+    return out;
 }
+
+// Direct entry for the ordinary call - tensors, numbers and texts by position - without
+// pybind11's argument casters; anything else goes to the function above through them.
+PyObject *ddf_fast(PyObject *self, PyObject *const *args, Py_ssize_t nargs, PyObject *kwnames);
 
 // Up-sampling DDF (DDFUpPack.forward, ddf/ddf.py:264-272 of the reference: one
 // ddf call per sub-pixel branch, torch.stack, F.pixel_shuffle) as one operator:
@@ -315,12 +337,16 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
         assertion_error(os.str());
     }
     if (features.dim() != 4) assertion_error("features must be 4-dimensional");
-    features = features.to(dtype).contiguous();
+    auto as_operand = [dtype](at::Tensor &t) {
+        if (t.scalar_type() != dtype) t = t.to(dtype);
+        if (!t.is_contiguous()) t = t.contiguous();
+    };
+    as_operand(features);
     const int64_t b = features.size(0), c = features.size(1), h = features.size(2), w = features.size(3);
     variable_list filters;
     filters.reserve(2 * branches);
     for (auto &t : channel_filters) {
-        t = t.to(dtype).contiguous();
+        as_operand(t);
         if (t.dim() != 4 || t.size(0) != b || t.size(1) != c || t.size(2) != kernel_size ||
             t.size(3) != kernel_size)
             assertion_error("channel_filter size " + size_string(t) + " does not match feature size " +
@@ -328,7 +354,7 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
         filters.push_back(t);
     }
     for (auto &t : spatial_filters) {
-        t = t.to(dtype).contiguous();
+        as_operand(t);
         if (t.dim() != 4 || t.size(0) != b || t.size(1) != kernel_size * kernel_size ||
             t.size(2) != h || t.size(3) != w)
             assertion_error("spatial_filter size " + size_string(t) + " does not match feature size " +
@@ -339,6 +365,41 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
                                 (int64_t)combine);
 }
 
+namespace {
+py::object *g_ddf_casting = nullptr;    // ddf bound through pybind11 (kept for the process)
+
+bool int_argument(PyObject *o, int64_t *v) {
+    if (!PyLong_CheckExact(o)) return false;
+    *v = PyLong_AsLongLong(o);
+    if (*v == -1 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+    return true;
+}
+}  // namespace
+
+PyObject *ddf_fast(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObject *kwnames) {
+    int64_t number[3] = {3, 1, 1};
+    std::string text[2] = {"mul", ""};
+    bool plain = nargs >= 3 && nargs <= 8 && (kwnames == nullptr || PyTuple_GET_SIZE(kwnames) == 0);
+    for (Py_ssize_t i = 0; plain && i < 3; ++i) plain = THPVariable_CheckExact(args[i]);
+    for (Py_ssize_t i = 3; plain && i < nargs && i < 6; ++i) plain = int_argument(args[i], &number[i - 3]);
+    for (Py_ssize_t i = 6; plain && i < nargs; ++i) {
+        Py_ssize_t len = 0;
+        const char *c = PyUnicode_CheckExact(args[i]) ? PyUnicode_AsUTF8AndSize(args[i], &len) : nullptr;
+        if (c) text[i - 6].assign(c, (size_t)len);
+        else { PyErr_Clear(); plain = false; }
+    }
+    if (!plain) return PyObject_Vectorcall(g_ddf_casting->ptr(), args, (size_t)nargs, kwnames);
+    HANDLE_TH_ERRORS
+    return THPVariable_Wrap(ddf(THPVariable_Unpack(args[0]), THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2]),
+                                number[0], number[1], number[2], text[0], text[1]));
+    END_HANDLE_TH_ERRORS
+}
+
+namespace {
+PyMethodDef g_ddf_method = {"ddf", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&ddf_fast)),
+                            METH_FASTCALL | METH_KEYWORDS, "ddf(features, channel_filter, spatial_filter, ...)"};
+}  // namespace
+
 }  // namespace ddf_torch
 
 #include "ddf_pack.h"
@@ -348,9 +409,11 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     using namespace ddf_torch;
     m.doc() = "ddf operator of libddf_hip.so as a C++ autograd function";
-    m.def("ddf", &ddf, py::arg("features"), py::arg("channel_filter"), py::arg("spatial_filter"),
+    m.def("_ddf_casting", &ddf, py::arg("features"), py::arg("channel_filter"), py::arg("spatial_filter"),
           py::arg("kernel_size") = 3, py::arg("dilation") = 1, py::arg("stride") = 1,
           py::arg("kernel_combine") = "mul", py::arg("version") = "");
+    g_ddf_casting = new py::object(m.attr("_ddf_casting"));
+    m.attr("ddf") = py::reinterpret_steal<py::object>(PyCFunction_NewEx(&g_ddf_method, nullptr, nullptr));
     m.def("ddf_up", &ddf_up, py::arg("features"), py::arg("channel_filters"),
           py::arg("spatial_filters"), py::arg("kernel_size") = 3, py::arg("dilation") = 1,
           py::arg("scale_factor") = 2, py::arg("kernel_combine") = "mul");
