@@ -150,7 +150,7 @@ public:
         at::Tensor out = new_tensor({z.b, z.c, z.ho, z.wo}, x.scalar_type(), x.device());
         at::Tensor saved = new_tensor({(int64_t)z.saved}, at::kByte, x.device());
         const int64_t cap = z.b * z.c * ((z.ho * z.wo + 63) / 64 + 1);
-        at::Tensor parts = new_tensor({cap}, x.options().dtype(at::kFloat));
+        at::Tensor parts = new_tensor({cap}, at::kFloat, x.device());
         char *q = static_cast<char *>(saved.data_ptr());
         void *cf = q, *sf = q + z.cf, *raw = q + z.cf + z.sf;
         float *pooled = reinterpret_cast<float *>(q + z.cf + 2 * z.sf);
