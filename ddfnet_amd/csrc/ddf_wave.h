@@ -1104,24 +1104,32 @@ __global__ __launch_bounds__(kWave * kFilterWaves) void k_backward_filters(
     }
 }
 
-// out[o, i] = sum_p part[o, p, i] for o < outer, p < parts, i < inner.  A
-// thread adds up VEC neighbouring i (inner % VEC == 0) and keeps 8 loads in
-// flight; the order of the additions is fixed, so results are reproducible.
-template <typename T, int VEC>
+// out[o, i] = sum_p part[o, p, i] for o < outer, p < parts, i < inner.  A thread adds up VEC
+// neighbouring i (inner % VEC == 0) over one of 1 << split stretches of p and keeps 8 loads in
+// flight; the stretches are added up through LDS.  The order of the additions is fixed, so
+// results are reproducible.  (One thread over all p is a serial chain where a plane has many
+// strips and few channels: 69 us at 1 x 16 x 300 x 301, where the launch before it takes 14.)
+constexpr int kSumThreadsLog2 = 8, kSumThreads = 1 << kSumThreadsLog2;
+template <typename T, int VEC, bool SPLIT>
 __device__ __forceinline__ void sum_partials_block(const typename Acc<T>::type *__restrict__ part,
                                                    T *__restrict__ out, int64_t outer, int parts,
-                                                   int64_t inner, unsigned block) {
+                                                   int64_t inner, int split_log2, unsigned block) {
     using A = typename Acc<T>::type;
+    const int split = SPLIT ? split_log2 : 0;
     const int64_t iv = inner / VEC;
-    const int64_t idx = (int64_t)block * 256 + threadIdx.x;
-    if (idx >= outer * iv) return;
-    const int64_t o = idx / iv, i = (idx - o * iv) * VEC;
+    const int per = kSumThreads >> split;   // outputs of the workgroup
+    const int slice = threadIdx.x >> (kSumThreadsLog2 - split), slot = threadIdx.x & (per - 1);
+    const int64_t idx = (int64_t)block * per + slot;
+    const bool live = idx < outer * iv;
+    const int64_t o = live ? idx / iv : 0, i = live ? (idx - o * iv) * VEC : 0;
+    const int len = (parts + (1 << split) - 1) >> split;
+    int p = slice * len;
+    const int p_end = live ? min(p + len, parts) : p;
     const A *src = part + o * parts * inner + i;
     A tot[VEC];
 #pragma unroll
     for (int k = 0; k < VEC; ++k) tot[k] = 0;
-    int p = 0;
-    for (; p + 8 <= parts; p += 8) {
+    for (; p + 8 <= p_end; p += 8) {
         Vec<A, VEC> v[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q)
@@ -1131,20 +1139,31 @@ __device__ __forceinline__ void sum_partials_block(const typename Acc<T>::type *
 #pragma unroll
             for (int k = 0; k < VEC; ++k) tot[k] += v[q].e[k];
     }
-    for (; p < parts; ++p) {
+    for (; p < p_end; ++p) {
         const Vec<A, VEC> v = *reinterpret_cast<const Vec<A, VEC> *>(src + (int64_t)p * inner);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) tot[k] += v.e[k];
     }
+    if constexpr (SPLIT) {
+        __shared__ A red[VEC][kSumThreads];
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) st(out + o * inner + i + k, tot[k]);
+        for (int k = 0; k < VEC; ++k) red[k][threadIdx.x] = tot[k];
+        __syncthreads();
+        if (slice > 0) return;
+        for (int q = 1; q < (1 << split); ++q)
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) tot[k] += red[k][q * per + slot];
+    }
+    if (live)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) st(out + o * inner + i + k, tot[k]);
 }
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(256) void k_sum_partials(
+template <typename T, int VEC, bool SPLIT>
+__global__ __launch_bounds__(kSumThreads) void k_sum_partials(
     const typename Acc<T>::type *__restrict__ part, T *__restrict__ out, int64_t outer,
-    int parts, int64_t inner) {
-    sum_partials_block<T, VEC>(part, out, outer, parts, inner, blockIdx.x);
+    int parts, int64_t inner, int split) {
+    sum_partials_block<T, VEC, SPLIT>(part, out, outer, parts, inner, split, blockIdx.x);
 }
 
 // dSF of a pixel = sum of its partial sums (PT: the accumulator type, or - one
@@ -1211,27 +1230,32 @@ struct SumJob {
     int64_t outer, inner;
     int parts;
     bool wide;         // four neighbouring elements per thread
+    int split;         // log2 of the threads that share an output
     unsigned blocks;
 };
 template <typename T>
 inline SumJob<T> sum_job(const typename Acc<T>::type *part, T *out, int64_t outer, int parts,
                          int64_t inner) {
     using A = typename Acc<T>::type;
-    SumJob<T> j{part, out, outer, inner, parts, sizeof(A) == 4 && inner % 4 == 0, 0};
+    SumJob<T> j{part, out, outer, inner, parts, sizeof(A) == 4 && inner % 4 == 0, 0, 0};
     const int64_t threads = outer * (j.wide ? inner / 4 : inner);
-    j.blocks = (unsigned)((threads + 255) / 256);
+    // as many threads per output as have a round of loads of their own (by the number of
+    // parts alone: a sample's sums come out the same in any batch)
+    while (j.split < 6 && (parts >> j.split) >= 24) ++j.split;
+    const int per = kSumThreads >> j.split;
+    j.blocks = (unsigned)((threads + per - 1) / per);
     return j;
 }
 
 // Two independent sums in one launch: the first a.blocks workgroups take a,
 // the others b.
-template <typename T>
+template <typename T, bool SPLIT>
 __global__ __launch_bounds__(256) void k_sum_partials_pair(SumJob<T> a, SumJob<T> b) {
     const bool second = blockIdx.x >= a.blocks;
     const SumJob<T> &j = second ? b : a;
     const unsigned block = second ? blockIdx.x - a.blocks : blockIdx.x;
-    if (j.wide) sum_partials_block<T, 4>(j.part, j.out, j.outer, j.parts, j.inner, block);
-    else sum_partials_block<T, 1>(j.part, j.out, j.outer, j.parts, j.inner, block);
+    if (j.wide) sum_partials_block<T, 4, SPLIT>(j.part, j.out, j.outer, j.parts, j.inner, j.split, block);
+    else sum_partials_block<T, 1, SPLIT>(j.part, j.out, j.outer, j.parts, j.inner, j.split, block);
 }
 
 // Launches k_sum_partials with the widest access the sizes allow (the
@@ -1241,10 +1265,14 @@ inline hipError_t sum_partials(const typename Acc<T>::type *part, T *out, int64_
                                int parts, int64_t inner, hipStream_t st) {
     const SumJob<T> j = sum_job<T>(part, out, outer, parts, inner);
     const dim3 grid(j.blocks), block(256);
-    if (j.wide)
-        hipLaunchKernelGGL((k_sum_partials<T, 4>), grid, block, 0, st, part, out, outer, parts, inner);
-    else
-        hipLaunchKernelGGL((k_sum_partials<T, 1>), grid, block, 0, st, part, out, outer, parts, inner);
+#define DDF_SUM(VEC_, SPLIT_)                                                                   \
+    hipLaunchKernelGGL((k_sum_partials<T, VEC_, SPLIT_>), grid, block, 0, st, part, out, outer, \
+                       parts, inner, j.split)
+    if (j.wide && j.split) DDF_SUM(4, true);
+    else if (j.wide) DDF_SUM(4, false);
+    else if (j.split) DDF_SUM(1, true);
+    else DDF_SUM(1, false);
+#undef DDF_SUM
     return hipGetLastError();
 }
 
@@ -1252,7 +1280,7 @@ inline hipError_t sum_partials(const typename Acc<T>::type *part, T *out, int64_
 // in the same launch, the dCF sum b (b.blocks == 0: none).  The dSF parts are
 // `parts` partial sums in the accumulator type, or (part_t) one part in the
 // storage type.
-template <typename T, int KK>
+template <typename T, int KK, bool SPLIT>
 __global__ __launch_bounds__(256) void k_sum_norm_pair(
     const typename Acc<T>::type *__restrict__ part_a, const T *__restrict__ part_t, int parts,
     int64_t n_samples, int64_t plane, const T *__restrict__ raw, T *__restrict__ d_raw,
@@ -1260,8 +1288,8 @@ __global__ __launch_bounds__(256) void k_sum_norm_pair(
     typename Acc<T>::type gain, unsigned norm_blocks, SumJob<T> b) {
     if (blockIdx.x >= norm_blocks) {
         const unsigned block = blockIdx.x - norm_blocks;
-        if (b.wide) sum_partials_block<T, 4>(b.part, b.out, b.outer, b.parts, b.inner, block);
-        else sum_partials_block<T, 1>(b.part, b.out, b.outer, b.parts, b.inner, block);
+        if (b.wide) sum_partials_block<T, 4, SPLIT>(b.part, b.out, b.outer, b.parts, b.inner, b.split, block);
+        else sum_partials_block<T, 1, SPLIT>(b.part, b.out, b.outer, b.parts, b.inner, b.split, block);
         return;
     }
     if (part_a)
@@ -1296,12 +1324,14 @@ inline hipError_t sum_filter_partials(const typename Acc<T>::type *ws_sf, T *dsf
         if (ws_cf) b = sum_job<T>(ws_cf, dcf, nc, nstrips, kk);
         const dim3 grid(norm_blocks + b.blocks), block(256);
         const A gain = (A)norm->gain;
-#define DDF_SUM_NORM(KK_)                                                                         \
-    hipLaunchKernelGGL((k_sum_norm_pair<T, KK_>), grid, block, 0, st, ws_sf, ws_sf ? nullptr : dsf, \
+#define DDF_SUM_NORM(KK_, SPLIT_)                                                                 \
+    hipLaunchKernelGGL((k_sum_norm_pair<T, KK_, SPLIT_>), grid, block, 0, st, ws_sf, ws_sf ? nullptr : dsf, \
                        ws_sf ? csplit : 1, n, plane, norm->raw, norm->d_raw, norm->terms,         \
                        norm->gain_vec, norm->groups, gain, norm_blocks, b)
-        if (kk == 9) DDF_SUM_NORM(9);
-        else DDF_SUM_NORM(25);
+        if (kk == 9 && b.split) DDF_SUM_NORM(9, true);
+        else if (kk == 9) DDF_SUM_NORM(9, false);
+        else if (b.split) DDF_SUM_NORM(25, true);
+        else DDF_SUM_NORM(25, false);
 #undef DDF_SUM_NORM
         norm->applied = true;
         return hipGetLastError();
@@ -1309,7 +1339,10 @@ inline hipError_t sum_filter_partials(const typename Acc<T>::type *ws_sf, T *dsf
     if (ws_sf && ws_cf) {
         const SumJob<T> a = sum_job<T>(ws_sf, dsf, n, csplit, sf_inner);
         const SumJob<T> b = sum_job<T>(ws_cf, dcf, nc, nstrips, kk);
-        hipLaunchKernelGGL((k_sum_partials_pair<T>), dim3(a.blocks + b.blocks), dim3(256), 0, st, a, b);
+        if (a.split || b.split)
+            hipLaunchKernelGGL((k_sum_partials_pair<T, true>), dim3(a.blocks + b.blocks), dim3(256), 0, st, a, b);
+        else
+            hipLaunchKernelGGL((k_sum_partials_pair<T, false>), dim3(a.blocks + b.blocks), dim3(256), 0, st, a, b);
         return hipGetLastError();
     }
     if (ws_sf) return sum_partials<T>(ws_sf, dsf, n, csplit, sf_inner, st);
