@@ -22,6 +22,7 @@ const char *sums_name(unsigned fneed, int csplit, int nstrips, bool norm = false
 }
 const char *layout_name(const RowsGeom &g) {
     if (g.Hi != g.H) return g.lp > g.lpr ? "padded,stride 2" : "plain,stride 2";
+    if (g.tail > 0) return g.segs > 0 ? "ragged segments" : "ragged";
     return g.segs > 0 ? "segments" : g.lp > g.lpr ? "padded" : "plain";
 }
 }  // namespace
@@ -31,7 +32,7 @@ const char *layout_name(const RowsGeom &g) {
 int describe_forward(const Problem &p, int dtype, char *buf, int len) {
     RowsGeom rg; int vx, r;
     WaveGeom wg; int ps, nv;
-    if (dtype != DDF_F64 && tune_int("DDF_TUNE_ROWS", 1) != 0 && rows_geometry(p, dtype, 0, &rg, &vx, &r))
+    if (dtype != DDF_F64 && tune_int("DDF_TUNE_ROWS", 1) != 0 && rows_plan(p, dtype, &rg, &vx, &r))
         return snprintf(buf, len, "k_rows<VX=%d,R=%d,%s>", vx, r, layout_name(rg));
     if (small_supported(p)) return snprintf(buf, len, "k_small");
     if (wave_geometry(p, dtype, kWaveForward, 0, &wg, &ps, &nv))
@@ -66,7 +67,7 @@ int describe_backward(const Problem &p, int dtype, unsigned need, char *buf, int
                       wave_geometry(p, dtype, kWaveFilters, 0, &gp, &pps, &pnv) && gp.TH == wg.TH &&
                       gp.csplit == wg.csplit;
     if ((need & DDF_NEED_DX) && fneed && dtype != DDF_F64 && tune_int("DDF_TUNE_ROWSF", 1) != 0 &&
-        rows_filters_geometry(p, dtype, true, &rg, &vx, &r)) {
+        rows_filters_plan(p, dtype, true, &rg, &vx, &r)) {
         add("k_rows_filters<dX,VX=%d,R=%d,%s>", vx, r, layout_name(rg));
         add("%s", sums_name(fneed, rg.csplit, rg.nstrips, norm, p.kk));
         return n;
@@ -78,7 +79,7 @@ int describe_backward(const Problem &p, int dtype, unsigned need, char *buf, int
     }
     if (need & DDF_NEED_DX) {
         if (dtype != DDF_F64 && tune_int("DDF_TUNE_ROWS", 1) != 0 &&
-            (p.s == 1 || rows_stride2_feature_gradient(p)) && rows_geometry(p, dtype, 0, &rg, &vx, &r))
+            (p.s == 1 || rows_stride2_feature_gradient(p)) && rows_plan(p, dtype, &rg, &vx, &r))
             add("k_rows<dX,VX=%d,R=%d,%s>", vx, r, layout_name(rg));
         else if (small_supported(p)) add("%s", "k_small<dX>");
         else add("%s", "k_backward_features");
@@ -86,11 +87,11 @@ int describe_backward(const Problem &p, int dtype, unsigned need, char *buf, int
     if (fneed) {
         if (n) add("%s", " + ");
         if (dtype != DDF_F64 && tune_int("DDF_TUNE_ROWSF", 1) != 0 &&
-            rows_taprow_geometry(p, dtype, &rg, &vx, &r)) {
+            rows_taprow_plan(p, dtype, &rg, &vx, &r)) {
             add("k_rows_taprow_filters<VX=%d,%s>", vx, layout_name(rg));
             add("%s", sums_name(fneed, rg.csplit, rg.nstrips, norm, p.kk));
         } else if (dtype != DDF_F64 && tune_int("DDF_TUNE_ROWSF", 1) != 0 &&
-            rows_filters_geometry(p, dtype, false, &rg, &vx, &r)) {
+            rows_filters_plan(p, dtype, false, &rg, &vx, &r)) {
             add("k_rows_filters<VX=%d,R=%d,%s>", vx, r, layout_name(rg));
             add("%s", sums_name(fneed, rg.csplit, rg.nstrips, norm, p.kk));
         } else {

@@ -61,6 +61,10 @@ struct RowsGeom {
     // lp = lpr = seg_out + 2, nstrips = row groups * segs.
     int segs, seg_out;
     unsigned segs_magic;
+    // Rows that are no whole number of vectors (tail > 0: elements of the last vector that
+    // belong to the row; see Ragged): shift: an odd tail of 2-byte elements, whose lane loads
+    // from one element further left.
+    int tail, shift;
 };
 
 // The vectors shifted in from the neighbouring lanes are right as they arrive
@@ -116,10 +120,12 @@ struct Work {
 //             rr (rr = 0 is HY rows above the lane's first row), or -1 when the
 //             row lies outside the image or the lane is idle;
 //   ooff[r]:  the same for the R result rows.
-template <int R, int HY, int VX>
+// RAGGED: rows may end inside a vector (g.tail > 0).
+template <int R, int HY, int VX, bool RAGGED = false>
 struct Lane {
     static constexpr int ROWS = R + 2 * HY;
     bool first, last;         // at the ends of an image row
+    bool ragged;              // the lane's vectors reach past the end of the image row
     int xoff[ROWS];
     int ooff[R];
     // dy: the window rows (xoff) are taken dy image rows further down
@@ -134,10 +140,11 @@ struct Lane {
             const bool reads = lane <= g.seg_out + 1 && x0 >= 0 && x0 < g.W;
             const bool owns = reads && lane >= 1 && lane <= g.seg_out;
             first = last = false;   // (the shifted-in vectors are right as they are)
+            ragged = RAGGED && reads && x0 + VX > g.W;
 #pragma unroll
             for (int rr = 0; rr < ROWS; ++rr) {
                 const int yy = y0 - HY + rr + dy;
-                xoff[rr] = (reads && yy >= 0 && yy < g.H) ? yy * g.W + x0 : -1;
+                xoff[rr] = (reads && yy >= 0 && yy < g.H) ? yy * g.W + x0 - (RAGGED && ragged ? g.shift : 0) : -1;
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) ooff[r] = (owns && y0 + r < g.H) ? (y0 + r) * g.W + x0 : -1;
@@ -150,10 +157,11 @@ struct Lane {
         const int y0 = strip * g.rps + grp * R;
         first = v == 0;
         last = v == g.lpr - 1;
+        ragged = RAGGED && live && last && g.tail > 0;
 #pragma unroll
         for (int rr = 0; rr < ROWS; ++rr) {
             const int yy = y0 - HY + rr + dy;
-            xoff[rr] = (live && yy >= 0 && yy < g.H) ? yy * g.W + x0 : -1;
+            xoff[rr] = (live && yy >= 0 && yy < g.H) ? yy * g.W + x0 - (RAGGED && ragged ? g.shift : 0) : -1;
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) ooff[r] = (live && y0 + r < g.H) ? (y0 + r) * g.W + x0 : -1;
@@ -167,6 +175,7 @@ struct Lane {
 template <int VX>
 struct LaneStride2 {
     static constexpr int ROWS = 3;
+    static constexpr bool ragged = false;
     bool first, last;
     int xoff[ROWS];
     int ooff[1];
@@ -381,6 +390,83 @@ struct ExtRow {
     }
 };
 
+// Rows whose length no vector divides (TAIL > 0).  The last lane of such a row holds `tail`
+// elements of it; the memory unit takes vectors at any element address and checks every
+// 32-bit word of one against the end of the buffer by itself, so what its vectors need is
+// that the elements past the row's end - the next row's - are zero, and that its results
+// go out in pieces.  TAIL == 2: an odd number of 2-byte elements.  The word with the last of
+// them would reach past the row, and on a plane's last row past the buffer, where the whole
+// word reads as zero; such a lane loads from one element further left and shifts.
+template <typename T, int VX, int TAIL>
+struct Ragged {
+    static constexpr int NW = vec_words(VX * sizeof(T)), EPW = 4 / (int)sizeof(T);
+    uint32_t mask[TAIL ? NW : 1];
+    uint32_t sh;
+    bool last;
+    int tail;
+    __device__ __forceinline__ void init(const RowsGeom &g, bool ragged) {
+        if constexpr (TAIL) {
+            static_assert(VX * sizeof(T) >= 8, "vectors of two words at least");
+            last = ragged;
+            tail = g.tail;
+            sh = (TAIL == 2 && ragged) ? 16u : 0u;
+#pragma unroll
+            for (int k = 0; k < NW; ++k) {
+                const int have = ragged ? g.tail - k * EPW : EPW;
+                mask[k] = have >= EPW ? ~0u : (have <= 0 ? 0u : 0xffffu);
+            }
+        }
+    }
+    // a vector as it was loaded -> its elements inside the row
+    __device__ __forceinline__ void fix(uint32_t (&w)[NW]) const {
+        if constexpr (TAIL == 2) {
+#pragma unroll
+            for (int k = 0; k < NW; ++k) w[k] = __builtin_amdgcn_alignbit(k + 1 < NW ? w[k + 1] : 0u, w[k], sh);
+        }
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int k = 0; k < NW; ++k) w[k] &= mask[k];
+        }
+    }
+    // where the lane's own vector is loaded from, given where its results go
+    __device__ __forceinline__ uint32_t load_at(uint32_t off) const {
+        if constexpr (TAIL == 2) return off == kOutside ? kOutside : off - sh / 8u;
+        else return off;
+    }
+    __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, const uint32_t (&w)[NW]) const {
+        store_vec_nt<VX * sizeof(T)>(rsrc, TAIL && last ? kOutside : off, w);
+        if constexpr (TAIL) {
+            // the last lane's elements: four, two and one of them (no branches: the other
+            // lanes' offsets lie outside)
+            const uint32_t at = last ? off : kOutside;
+            if constexpr (VX == 8) {
+                const uint32_t q[2] = {w[0], w[1]};
+                store_words_nt<2>(rsrc, (tail & 4) ? at : kOutside, q);
+            }
+            const int done4 = VX == 8 ? tail & 4 : 0;
+            if constexpr (sizeof(T) == 2) {
+                const uint32_t lo = w[0], hi = w[NW - 2];
+                const uint32_t two[1] = {VX == 8 && done4 ? hi : lo};
+                store_words_nt<1>(rsrc, (tail & 2) && at != kOutside ? at + done4 * 2 : kOutside, two);
+                if constexpr (TAIL == 2) {
+                    // (by value: a choice between array elements would put the array into memory)
+                    const int k = tail >> 1;
+                    const uint32_t e1 = w[1], e2 = w[NW > 2 ? 2 : 0], e3 = w[NW - 1];
+                    const uint32_t one = k == 0 ? lo : k == 1 ? e1 : k == 2 ? e2 : e3;
+                    __builtin_amdgcn_raw_buffer_store_b16((short)one, rsrc,
+                                                          (int)(at != kOutside ? at + (tail & ~1) * 2 : kOutside), 0, 2);
+                }
+            } else {
+                const uint32_t q[2] = {w[0], w[1]};
+                store_words_nt<2>(rsrc, (tail & 2) ? at : kOutside, q);
+                const uint32_t lo = w[0], hi = w[2];
+                const uint32_t one[1] = {(tail & 2) ? hi : lo};
+                store_words_nt<1>(rsrc, (tail & 1) && at != kOutside ? at + (tail & 2) * 4 : kOutside, one);
+            }
+        }
+    }
+};
+
 template <typename A>
 __device__ __forceinline__ A lane_broadcast(A v, int src_lane);
 template <>
@@ -398,8 +484,9 @@ __device__ __forceinline__ double lane_broadcast<double>(double v, int src_lane)
 // WPE: waves per SIMD the register allocation must leave room for.
 // S = 2 (forward, 3 x 3, one row per lane): g describes the result plane, the
 // lane's feature vectors are 2 * VX elements wide (LaneStride2).
+// TAIL: rows that are no whole number of vectors (Ragged).
 template <typename T, int K, int D, bool MUL, bool BWD, int VX, int R, bool PAD, int NST, int WPE,
-          int S = 1>
+          int S = 1, int TAIL = 0>
 __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const T *__restrict__ x,
                                                          const T *__restrict__ cf,
                                                          const T *__restrict__ sf,
@@ -412,6 +499,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     using Row = ExtRow<T, S * VX, HX, PAD>;
     static_assert(KK <= kWave, "one lane per channel-filter tap");
     static_assert(S == 1 || (S == 2 && K == 3 && D == 1 && R == 1), "stride 2: 3 x 3, one row per lane");
+    static_assert(TAIL == 0 || (S == 1 && PAD), "ragged rows: stride 1, padded");
     // Stride-2 feature gradient: the lane of result row y loads dO rows y and y + 1 and
     // writes the feature rows 2y and 2y + 1 of its columns (even feature heights).
     constexpr bool S2B = S == 2 && BWD;
@@ -427,8 +515,10 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     const uint32_t plane_bytes = (uint32_t)plane * (uint32_t)sizeof(T);
     const int64_t xplane = S == 1 ? plane : (int64_t)g.Hi * g.Wi;
     const uint32_t xplane_bytes = S == 1 ? plane_bytes : (uint32_t)xplane * (uint32_t)sizeof(T);
-    std::conditional_t<S == 1, Lane<R, HY, VX>, LaneStride2<VX>> ln;
+    std::conditional_t<S == 1, Lane<R, HY, VX, (TAIL > 0)>, LaneStride2<VX>> ln;
     ln.init(g, wk.strip, lane);
+    Ragged<T, VX, TAIL> rag;
+    rag.init(g, ln.ragged);
 
     // (the tensor read has the result plane's shape in the stride-2 gradient, and the one
     // written the feature plane's)
@@ -496,7 +586,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             for (int t = 0; t < KK; ++t) {
                 const __amdgpu_buffer_rsrc_t sr = plane_rsrc(sfn + t * plane, plane_bytes);
 #pragma unroll
-                for (int r = 0; r < R; ++r) load_vec<kVB>(sr, ob[r], sfw[r][t]);
+                for (int r = 0; r < R; ++r) load_vec<kVB>(sr, rag.load_at(ob[r]), sfw[r][t]);
             }
         } else {
 #pragma unroll
@@ -509,6 +599,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
                     for (int r = 0; r < R; ++r) {
                         Row row;
                         load_vec<kVB>(sr, xb[r + i * D], row.own);
+                        if constexpr (S == 1) rag.fix(row.own);
                         row.sides(ln.first, ln.last);
                         A v[VX];
 #pragma unroll
@@ -550,6 +641,12 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
         for (int t = 0; t < KK; ++t)
 #pragma unroll
             for (int k = 0; k < NW; ++k) asm volatile("" : "+v"(sfw[r][t][k]));
+    if constexpr (TAIL && !BWD) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int t = 0; t < KK; ++t) rag.fix(sfw[r][t]);
+    }
 
     // fp16, 3 x 3 without dilation: the taps of columns 0 and 1 of a filter row go through
     // the two-element dot product (fp32 accumulation), whose operands are pairs of
@@ -666,6 +763,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             if (!row_needed<R, K, D>(rr)) continue;
 #pragma unroll
             for (int k = 0; k < NWX; ++k) row[rr].own[k] = xw[ST][rr][k];
+            if constexpr (TAIL) rag.fix(row[rr].own);
             row[rr].sides(ln.first, ln.last);
         }
         A acc[R][VX];
@@ -752,7 +850,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             }
             uint32_t ow[NW];
             pack<T, VX, A>(acc[r], ow);
-            store_vec_nt<kVB>(orr, ob[r], ow);
+            rag.store(orr, ob[r], ow);
         }
         }   // (not the stride-2 gradient)
     };
@@ -789,5 +887,8 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
 // g->lpr selects the PAD kernels); false when the family does not cover the
 // problem.
 bool rows_geometry(const Problem &p, int dtype, int max_vx, RowsGeom *g, int *vx, int *r);
+// What runs: that geometry, or wide vectors over rows they do not divide (g->tail > 0: the
+// TAIL kernels) where those take fewer instructions or the other covers nothing.
+bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r);
 
 }  // namespace ddf

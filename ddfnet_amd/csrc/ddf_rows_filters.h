@@ -62,7 +62,7 @@ __device__ __forceinline__ void wave_sync() {
 // SEG (with DX): image rows are cut into segments, whose outer lanes hold dO
 // values they do not own; those are kept out of the filter sums.
 template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, bool DX, int NST, int WPE,
-          int S = 1, bool SEG = true>
+          int S = 1, bool SEG = true, int TAIL = 0>
 __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
     RowsGeom g, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,
     const T *__restrict__ sf, T *__restrict__ dx, T *__restrict__ dcf, T *__restrict__ dsf,
@@ -99,8 +99,11 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
     const uint32_t plane_bytes = (uint32_t)plane * (uint32_t)sizeof(T);
     const int64_t xplane = S == 1 ? plane : (int64_t)g.Hi * g.Wi;
     const uint32_t xplane_bytes = S == 1 ? plane_bytes : (uint32_t)xplane * (uint32_t)sizeof(T);
-    std::conditional_t<S == 1, Lane<R, HY, VX>, LaneStride2<VX>> ln;
+    std::conditional_t<S == 1, Lane<R, HY, VX, (TAIL > 0)>, LaneStride2<VX>> ln;
     ln.init(g, wk.strip, lane);
+    static_assert(TAIL == 0 || (S == 1 && PAD), "ragged rows: stride 1, padded");
+    Ragged<T, VX, TAIL> rag;
+    rag.init(g, ln.ragged);
 
     // x_mod != 0: the batch is several groups of x_mod samples that share one set of
     // features (the sub-pixel branches of the up-sampling operator's gradient)
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
         gb[1] = ln.onext < 0 ? kOutside : (uint32_t)ln.onext * (uint32_t)sizeof(T);
     } else {
 #pragma unroll
-        for (int r = 0; r < GROWS; ++r) gb[r] = DX ? xb[r] : ob[r];
+        for (int r = 0; r < GROWS; ++r) gb[r] = DX ? xb[r] : rag.load_at(ob[r]);
     }
     const int tl = lane < KK ? lane : KK - 1;
     const T *cfs = cf + (wk.n * g.C + c_first) * KK;
@@ -215,7 +218,10 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                 for (int rr = 0; rr < ROWS; ++rr) {
                     const bool for_grad = rr >= i * D && rr < i * D + R;
                     const bool for_own = MUL && rr >= HY && rr < HY + R;
-                    if (for_grad || for_own) load_vec<kVB>(sr, xb[rr], pw[rr]);
+                    if (for_grad || for_own) {
+                        load_vec<kVB>(sr, xb[rr], pw[rr]);
+                        rag.fix(pw[rr]);
+                    }
                 }
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
@@ -239,7 +245,7 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
         for (int t = 0; t < KK; ++t) {
             const __amdgpu_buffer_rsrc_t sr = plane_rsrc(sfn + t * plane, plane_bytes);
 #pragma unroll
-            for (int r = 0; r < R; ++r) load_vec<kVB>(sr, ob[r], sfw[r][t]);
+            for (int r = 0; r < R; ++r) load_vec<kVB>(sr, rag.load_at(ob[r]), sfw[r][t]);
         }
     }
     // first channels of the walk; then wait for the spatial taps, which were requested
@@ -255,6 +261,12 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                     if constexpr (MUL) asm volatile("" : "+v"(sfw[r][t][k]));
                     if constexpr (DX) asm volatile("" : "+v"(sfg[r][t][k]));
                 }
+    }
+    if constexpr (TAIL && MUL && !DX) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int t = 0; t < KK; ++t) rag.fix(sfw[r][t]);
     }
     A acc_sf[R][KK][VX];
 #pragma unroll
@@ -314,7 +326,13 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
             if (!row_needed<R, K, D>(rr)) continue;
 #pragma unroll
             for (int k = 0; k < NWX; ++k) row[rr].own[k] = xw[ST][rr][k];
+            if constexpr (TAIL) rag.fix(row[rr].own);
             row[rr].sides(ln.first, ln.last);
+        }
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int r = 0; r < GROWS; ++r)
+                if (!DX || row_needed<R, K, D>(r)) rag.fix(gw[ST][r]);
         }
         // dO at the lane's own pixels.  (DX loads dO through the window offsets, so a
         // lane that only reads for its neighbours - the outer lanes of a row segment -
@@ -482,7 +500,7 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                 }
                 uint32_t ow[NW];
                 pack<T, VX, A>(accx, ow);
-                store_vec_nt<kVB>(dr, ob[r], ow);
+                rag.store(dr, ob[r], ow);
             }
         }
         if (want_cf && ci < nch) {
@@ -545,7 +563,7 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
             if (g.csplit == 1) {
                 uint32_t ow[NW];
                 pack<T, VX, A>(tot, ow);
-                store_vec_nt<kVB>(plane_rsrc(dsf + (wk.n * KK + t) * plane, plane_bytes), off_r, ow);
+                rag.store(plane_rsrc(dsf + (wk.n * KK + t) * plane, plane_bytes), off_r, ow);
             } else {
                 // partial sums in the accumulator type, same plane shape
                 constexpr int AW = VX * sizeof(A) / 4;
@@ -557,12 +575,22 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                                                          : off_r / (uint32_t)sizeof(T) * (uint32_t)sizeof(A);
                 uint32_t aw[AW];
                 pack<A, VX, A>(tot, aw);
+                if constexpr (TAIL) {
+                    // (value by value: the last lane of a row has fewer)
 #pragma unroll
-                for (int h = 0; h < AW; h += CH) {
-                    uint32_t part[CH];
+                    for (int h = 0; h < AW; ++h) {
+                        const uint32_t one[1] = {aw[h]};
+                        store_words_nt<1>(wr, off_a == kOutside || (rag.last && h >= rag.tail) ? kOutside : off_a + h * 4,
+                                          one);
+                    }
+                } else {
 #pragma unroll
-                    for (int q = 0; q < CH; ++q) part[q] = aw[h + q];
-                    store_words_nt<CH>(wr, off_a + h * 4, part);
+                    for (int h = 0; h < AW; h += CH) {
+                        uint32_t part[CH];
+#pragma unroll
+                        for (int q = 0; q < CH; ++q) part[q] = aw[h + q];
+                        store_words_nt<CH>(wr, off_a + h * 4, part);
+                    }
                 }
             }
         }
@@ -578,6 +606,8 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
 // g->cpw * rows::kFilterWaves channels; g->csplit counts those ranges.
 // fused: the geometry of the launch that also writes the feature gradient.
 bool rows_filters_geometry(const Problem &p, int dtype, bool fused, RowsGeom *g, int *vx, int *r);
+// What runs: that geometry or the one for ragged rows (see rows_plan).
+bool rows_filters_plan(const Problem &p, int dtype, bool fused, RowsGeom *g, int *vx, int *r);
 // Workspace the kernel needs (layout as the tile kernels': dSF partials over
 // channel splits, then dCF partials over strips, each 256-byte aligned).
 size_t rows_filters_workspace(const Problem &p, int dtype, unsigned need);

@@ -20,13 +20,17 @@ unsigned magic_of(int d) { return d == 1 ? 0u : (unsigned)((0x100000000ull + d -
 // per wave, strips of even height.  Where it costs no row group, every image
 // row is followed by an idle lane (lane pitch lpr + 1): its loads return zero,
 // which is exactly what the neighbour shift must bring in at the row ends.
+// Rows vx does not divide (the TAIL kernels, which are built padded): ceil(W / vx) lanes,
+// always followed by the idle one.
 void lay_out_lanes(RowsGeom *t, int H, int W, int vx, int R) {
     t->segs = t->seg_out = 0;
     t->segs_magic = 0;
-    if (W / vx > kMaxRowLanes) {
+    t->tail = W % vx;
+    t->shift = 0;
+    const int vectors = (W + vx - 1) / vx;
+    if (vectors > kMaxRowLanes) {
         // an image row is longer than the lanes of a wave take: even segments of at
         // most 62 vectors, each with a vector of its neighbours on either side
-        const int vectors = W / vx;
         t->segs = (vectors + kWave - 3) / (kWave - 2);
         t->seg_out = (vectors + t->segs - 1) / t->segs;
         t->segs_magic = magic_of(t->segs);
@@ -37,13 +41,13 @@ void lay_out_lanes(RowsGeom *t, int H, int W, int vx, int R) {
         t->nstrips = ((H + R - 1) / R) * t->segs;
         return;
     }
-    t->lpr = W / vx;
+    t->lpr = vectors;
     const int row_units = (H + R - 1) / R;                  // lane-sized row groups of the plane
     const int fit_plain = std::min(kWave / t->lpr, row_units);
     const int fit_padded = std::min((kWave + 1) / (t->lpr + 1), row_units);
     auto strips_with = [&](int fit) { return fit > 0 ? (row_units + fit - 1) / fit : 1 << 30; };
-    const bool pad = fit_padded > 0 && strips_with(fit_padded) <= strips_with(fit_plain) &&
-                     tune_int("DDF_TUNE_ROWS_PAD", 1) != 0;
+    const bool pad = t->tail > 0 || (fit_padded > 0 && strips_with(fit_padded) <= strips_with(fit_plain) &&
+                                     tune_int("DDF_TUNE_ROWS_PAD", 1) != 0);
     t->lp = t->lpr + (pad ? 1 : 0);
     t->lp_magic = magic_of(t->lp);
     const int rg_max = pad ? fit_padded : fit_plain;
@@ -181,6 +185,59 @@ bool stride2_geometry(const Problem &p, int dtype, bool filters, int max_vx, Row
     return true;
 }
 
+// Lanes and channel walk of k_rows for vx elements and R rows per lane.
+bool rows_cut(const Problem &p, int vx, int R, RowsGeom *g, int *vx_out, int *r_out) {
+    const int H = (int)p.H, W = (int)p.W, C = (int)p.C;
+    RowsGeom t{};
+    t.C = C; t.H = t.Hi = H; t.W = t.Wi = W;
+    lay_out_lanes(&t, H, W, vx, R);
+
+    // (25 spatial taps per pixel to load before the walk: 32 pixel-channels per lane at least)
+    if (!cut_channels_forward(t, p.N, C, p.k == 5 ? 2 : kRowsStages, (int64_t)H * W, p.k == 5 ? 32 / vx : 0))
+        return false;
+    *g = t;
+    *vx_out = vx;
+    *r_out = R;
+    return true;
+}
+
+// What the ragged-row variants cover.  (Planes of at most 64 pixels that the exact vectors do
+// not cover belong to the kernel that packs several of them into a workgroup.)
+bool ragged_shape(const Problem &p, int dtype, int vx) {
+    if (dtype != DDF_F16 && dtype != DDF_F32) return false;
+    if (p.s != 1 || p.N <= 0 || p.C <= 0 || p.H <= 0 || p.W <= vx || p.W % vx == 0) return false;
+    if (p.H > 16384 || p.W > 16384 || p.C > (1 << 24) || p.N > (1 << 24)) return false;
+    return p.H * p.W > 64 && (int64_t)p.H * p.W * 8 < (1ll << 31) && tune_int("DDF_TUNE_RAGGED", 1) != 0;
+}
+
+constexpr int64_t kSimds = 1024;
+
+// Channels per wave of k_rows_taprow_filters (one wave per filter row).
+bool cut_channels_taprow(RowsGeom &t, const Problem &p) {
+    const int flush = p.k <= 4 ? rows::taprow_flush_channels<3>() : rows::taprow_flush_channels<5>();
+    const int C = (int)p.C, target = tune_int("DDF_TUNE_TAPROW_WAVES", 2048);
+    const int64_t base = p.N * t.nstrips;
+    const int64_t want_split = std::max<int64_t>(1, (target + base * p.k - 1) / (base * p.k));
+    int cpw = (int)((C + want_split - 1) / want_split);
+    cpw = (cpw + flush - 1) / flush * flush;   // whole flush groups (and pipeline rounds)
+    cpw = std::max(cpw, tune_int("DDF_TUNE_TAPROW_MIN_CPW", 2 * flush));
+    const int forced = tune_int("DDF_TUNE_TAPROW_CPW", 0);
+    if (forced) cpw = forced;
+    t.cpw = std::max(1, std::min(cpw, C));
+    t.cpb = t.cpw;
+    t.csplit = (C + t.cpw - 1) / t.cpw;
+    t.wpb = rows::kTaprowWaves;
+    const int64_t nwork = base * t.csplit * p.k;   // one wave per filter row
+    if (nwork > (1 << 30)) return false;
+    if (nwork * std::max(t.csplit, t.nstrips) >= (1ll << 32)) return false;
+    t.csplit_magic = magic_of(t.csplit);
+    t.nstrips_magic = magic_of(t.nstrips);
+    const int64_t ngroups = (nwork + t.wpb - 1) / t.wpb;
+    t.xcd_per = (unsigned)((ngroups + rows::kXcd - 1) / rows::kXcd);
+    t.nwork = (int)nwork;
+    return true;
+}
+
 }  // namespace
 
 // Instantiated (elements per lane and row, rows per lane) per element size.
@@ -201,7 +258,7 @@ bool rows_geometry(const Problem &p, int dtype, int max_vx, RowsGeom *g, int *vx
     if (p.N <= 0 || p.C <= 0 || p.H <= 0 || p.W <= 0) return false;
     if (p.H > 16384 || p.W > 16384 || p.C > (1 << 24) || p.N > (1 << 24)) return false;
     const int esz = dtype == DDF_F16 ? 2 : dtype == DDF_F32 ? 4 : 8;
-    const int H = (int)p.H, W = (int)p.W, C = (int)p.C;
+    const int H = (int)p.H, W = (int)p.W;
     const int hx = p.r * p.d;
     if ((int64_t)H * W * esz >= (1ll << 31)) return false;   // byte offsets inside a plane are 32-bit
     // widest vector the row length allows, at most 32 lanes per image row
@@ -232,17 +289,51 @@ bool rows_geometry(const Problem &p, int dtype, int max_vx, RowsGeom *g, int *vx
     }
     if (!rows_variant_built(esz, vx, R)) return false;
 
-    RowsGeom t{};
-    t.C = C; t.H = t.Hi = H; t.W = t.Wi = W;
-    lay_out_lanes(&t, H, W, vx, R);
+    return rows_cut(p, vx, R, g, vx_out, r_out);
+}
 
-    // (25 spatial taps per pixel to load before the walk: 32 pixel-channels per lane at least)
-    if (!cut_channels_forward(t, p.N, C, p.k == 5 ? 2 : kRowsStages, (int64_t)H * W, p.k == 5 ? 32 / vx : 0))
-        return false;
-    *g = t;
-    *vx_out = vx;
-    *r_out = R;
+// Vectors of vx elements over rows they do not divide (Ragged in ddf_rows.h).
+bool rows_ragged_geometry(const Problem &p, int dtype, int vx, RowsGeom *g, int *r) {
+    const int esz = dtype == DDF_F16 ? 2 : 4;
+    if (!ragged_shape(p, dtype, vx) || !rows_shape_built(p.k, p.d, p.s)) return false;
+    // (two rows per lane: see rows_geometry)
+    const int R = vx * esz == 16 && p.k == 3 && p.d == 1 && p.H * p.W >= 112 * 112 ? 2 : 1;
+    int tvx;
+    if (!rows_cut(p, vx, R, g, &tvx, r)) return false;
+    g->shift = esz == 2 ? g->tail & 1 : 0;
     return true;
+}
+
+bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r) {
+    const bool exact = rows_geometry(p, dtype, 0, g, vx, r);
+    if (dtype != DDF_F16 && dtype != DDF_F32) return exact;
+    // What a launch takes: the instructions of a wave - some 40 per channel and 16 per pixel
+    // of a lane (25 taps: 45), the spatial taps before the walk as much as three channels -
+    // times its waves per SIMD, of which it takes two or three to keep one busy.  Ragged
+    // vectors cost more than their masks: unaligned 16-byte accesses touch a cache line more.
+    // (Fitted over 80 sizes; forward at 12 x 144 x 80 x 87 fp32 28.1 -> 19.9 us, fp16 26.3 ->
+    // 19.3; 5 x 5 at 2 x 48 x 135 x 166, which only the LDS-tile kernels covered, 45 -> 11.3.
+    // Small launches keep vectors that divide their rows: 4 x 256 x 25 x 38 fp16 takes 5.2 us
+    // in vectors of two and 6.7 in eight.)
+    auto cost = [&](const RowsGeom &t, int v, int rows) {
+        const double per_wave = (t.cpw + 3.0) * (40 + (p.k == 5 ? 45 : 16) * v * rows);
+        const double over = t.tail == 0 ? 1.0 : t.shift ? 1.5 : dtype == DDF_F16 ? 1.05 : 1.15;
+        return per_wave * over * std::max(2.5, (double)t.nwork / kSimds);
+    };
+    double best = exact ? cost(*g, *vx, *r) : 1e30;
+    bool found = exact;
+    // (what the shortest ragged walk takes: small launches are decided without laying it out)
+    if (best <= (std::min<int64_t>(p.C, 2 * kRowsStages) + 3.0) * (40 + (p.k == 5 ? 45 : 16) * 4) * 2.5) return true;
+    for (int cand = dtype == DDF_F16 ? 8 : 4; cand >= 4; cand /= 2) {
+        RowsGeom t; int tr;
+        if (!rows_ragged_geometry(p, dtype, cand, &t, &tr) || cost(t, cand, tr) >= best) continue;
+        best = cost(t, cand, tr);
+        found = true;
+        *g = t;
+        *vx = cand;
+        *r = tr;
+    }
+    return found;
 }
 
 // Instantiated (elements per lane and row, rows per lane) of k_rows_filters;
@@ -297,6 +388,31 @@ bool rows_filters_geometry(const Problem &p, int dtype, bool fused, RowsGeom *g,
     return true;
 }
 
+bool rows_filters_plan(const Problem &p, int dtype, bool fused, RowsGeom *g, int *vx, int *r) {
+    const bool exact = rows_filters_geometry(p, dtype, fused, g, vx, r);
+    if (p.k != 3 || (p.d != 1 && p.d != 2) || !ragged_shape(p, dtype, 4)) return exact;
+    if (fused && tune_int("DDF_TUNE_ROWSF_FUSED", 1) == 0) return exact;
+    RowsGeom t{};
+    t.C = (int)p.C; t.H = t.Hi = (int)p.H; t.W = t.Wi = (int)p.W;
+    lay_out_lanes(&t, (int)p.H, (int)p.W, 4, 1);
+    if (!cut_channels_filters(t, p.N, (int)p.C)) return exact;
+    t.shift = dtype == DDF_F16 ? t.tail & 1 : 0;
+    // (as rows_plan; a wave issues some 60 instructions per channel and 50 per pixel of a
+    // lane, and two loads per channel leave a single wave per SIMD busy enough.  All
+    // gradients at 12 x 144 x 80 x 87 fp32: 63 -> 42 us; 3 x 3 with dilation 2 at 4 x 64 x
+    // 60 x 131, which only the LDS-tile kernels covered, 178 -> 18.5; 2 x 256 x 25 x 38 keeps
+    // single pixels, 11.3 us against 12.6.)
+    auto cost = [&](const RowsGeom &u, int px) {
+        const double waves = (double)u.nwork * rows::kFilterWaves;
+        return (u.cpw + 3.0) * (60 + 50 * px) * std::max(1.0, waves / kSimds);
+    };
+    if (exact && cost(t, 4) * 1.1 >= cost(*g, *vx * *r)) return true;
+    *g = t;
+    *vx = 4;
+    *r = 1;
+    return true;
+}
+
 // Built: 5 x 5 filters (and, as a tuning alternative, 3 x 3 without dilation).
 bool rows_taprow_shape_built(int k, int d, int s) {
     if (s != 1) return false;
@@ -329,37 +445,45 @@ bool rows_taprow_geometry(const Problem &p, int dtype, RowsGeom *g, int *vx_out,
         if (p.N * c.nstrips * p.k >= target) break;
     }
     if (vx == 0) return false;
-    const int flush = p.k <= 4 ? rows::taprow_flush_channels<3>() : rows::taprow_flush_channels<5>();
-    const int64_t base = p.N * t.nstrips;
-    const int64_t want_split = std::max<int64_t>(1, (target + base * p.k - 1) / (base * p.k));
-    int cpw = (int)((C + want_split - 1) / want_split);
-    cpw = (cpw + flush - 1) / flush * flush;   // whole flush groups (and pipeline rounds)
-    cpw = std::max(cpw, tune_int("DDF_TUNE_TAPROW_MIN_CPW", 2 * flush));
-    const int forced = tune_int("DDF_TUNE_TAPROW_CPW", 0);
-    if (forced) cpw = forced;
-    t.cpw = std::max(1, std::min(cpw, C));
-    t.cpb = t.cpw;
-    t.csplit = (C + t.cpw - 1) / t.cpw;
-    t.wpb = rows::kTaprowWaves;
-    const int64_t nwork = base * t.csplit * p.k;   // one wave per filter row
-    if (nwork > (1 << 30)) return false;
-    if (nwork * std::max(t.csplit, t.nstrips) >= (1ll << 32)) return false;
-    t.csplit_magic = magic_of(t.csplit);
-    t.nstrips_magic = magic_of(t.nstrips);
-    const int64_t ngroups = (nwork + t.wpb - 1) / t.wpb;
-    t.xcd_per = (unsigned)((ngroups + rows::kXcd - 1) / rows::kXcd);
-    t.nwork = (int)nwork;
+    if (!cut_channels_taprow(t, p)) return false;
     *g = t;
     *vx_out = vx;
     *r_out = 1;
     return true;
 }
 
+bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r) {
+    const bool exact = rows_taprow_geometry(p, dtype, g, vx, r);
+    if (p.k != 5 || (p.d != 1 && p.d != 2)) return exact;
+    // 16-byte vectors, or 8-byte ones of fp16 where those of 16 leave too few workgroups
+    for (int cand = dtype == DDF_F16 ? 8 : 4; cand >= 4; cand /= 2) {
+        if (!ragged_shape(p, dtype, cand)) continue;
+        RowsGeom t{};
+        t.C = (int)p.C; t.H = t.Hi = (int)p.H; t.W = t.Wi = (int)p.W;
+        lay_out_lanes(&t, (int)p.H, (int)p.W, cand, 1);
+        if (cand > 4 && p.N * t.nstrips * p.k < 2048) continue;
+        // (most lanes idle - rows a little too long for one strip of a small plane: the tile
+        // kernel is as fast)
+        if (!exact && p.H * p.W * 2 < (int64_t)t.nstrips * kWave * cand) continue;
+        t.shift = dtype == DDF_F16 ? t.tail & 1 : 0;
+        if (!cut_channels_taprow(t, p)) continue;
+        // (as rows_plan; some 40 instructions per channel and 25 per pixel of a lane.  All
+        // gradients at 2 x 48 x 135 x 166 fp32, 5 x 5: 1056 -> 36 us.)
+        if (exact && (int64_t)t.nstrips * (40 + 25 * cand) * 11 >= (int64_t)g->nstrips * (40 + 25 * *vx) * 10)
+            return true;
+        *g = t;
+        *vx = cand;
+        *r = 1;
+        return true;
+    }
+    return exact;
+}
+
 bool rows_cover_backward(const Problem &p, int dtype) {
     RowsGeom g; int vx, r;
-    return p.s == 1 && rows_geometry(p, dtype, 0, &g, &vx, &r) &&
-           (rows_taprow_geometry(p, dtype, &g, &vx, &r) ||
-            rows_filters_geometry(p, dtype, false, &g, &vx, &r));
+    return p.s == 1 && rows_plan(p, dtype, &g, &vx, &r) &&
+           (rows_taprow_plan(p, dtype, &g, &vx, &r) ||
+            rows_filters_plan(p, dtype, false, &g, &vx, &r));
 }
 
 bool rows_cover_stride2_filters(const Problem &p, int dtype) {
@@ -375,8 +499,8 @@ size_t rows_filters_workspace(const Problem &p, int dtype, unsigned need) {
     for (int cut = 0; cut < 3; ++cut) {
         RowsGeom g; int vx, r;
         if (cut == 1 && !(need & DDF_NEED_DX)) continue;
-        if (cut < 2 ? !rows_filters_geometry(p, dtype, cut != 0, &g, &vx, &r)
-                    : !rows_taprow_geometry(p, dtype, &g, &vx, &r))
+        if (cut < 2 ? !rows_filters_plan(p, dtype, cut != 0, &g, &vx, &r)
+                    : !rows_taprow_plan(p, dtype, &g, &vx, &r))
             continue;
         size_t bytes = 0;
         if ((need & DDF_NEED_DSF) && g.csplit > 1)

@@ -86,6 +86,22 @@ hipError_t launch_v(const Problem &p, const RowsGeom &g, bool backward, const T 
 
 }  // namespace rows
 
+// The kernels for rows that are no whole number of vectors (g.tail > 0), built in files of
+// their own (ddf_rows_ragged.h).
+template <typename T>
+hipError_t rows_ragged_launch(const Problem &p, const RowsGeom &g, int vx, int r, bool backward,
+                              const T *x, const T *cf, const T *sf, T *out, hipStream_t st);
+template <typename T>
+hipError_t rows_ragged_filters_launch(const Problem &p, const RowsGeom &g, const T *go, const T *x,
+                                      const T *cf, const T *sf, T *dx, T *dcf, T *dsf,
+                                      typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf,
+                                      unsigned need, int x_mod, hipStream_t st);
+template <typename T>
+hipError_t rows_ragged_taprow_launch(const Problem &p, const RowsGeom &g, int vx, const T *go,
+                                     const T *x, const T *cf, const T *sf, T *dcf, T *dsf,
+                                     typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf,
+                                     unsigned need, int x_mod, hipStream_t st);
+
 // Forward (backward = false: x -> out) or feature gradient (backward = true:
 // dO -> dX) on the row-register kernels.  hipErrorNotSupported: not covered
 // (shape, or pointers not aligned to the vector the geometry wants); nothing
@@ -96,7 +112,10 @@ hipError_t rows_launch(const Problem &p, bool backward, const T *x, const T *cf,
     const int dtype = sizeof(T) == 2 ? DDF_F16 : sizeof(T) == 4 ? DDF_F32 : DDF_F64;
     RowsGeom g;
     int vx, r;
-    if (!rows_geometry(p, dtype, 0, &g, &vx, &r)) return hipErrorNotSupported;
+    if (!rows_plan(p, dtype, &g, &vx, &r)) return hipErrorNotSupported;
+    if constexpr (sizeof(T) != 8) {
+        if (g.tail > 0) return rows_ragged_launch<T>(p, g, vx, r, backward, x, cf, sf, out, st);
+    }
     const uintptr_t mask = (uintptr_t)(vx * sizeof(T)) - 1;
     if ((((uintptr_t)x | (uintptr_t)sf | (uintptr_t)out) & mask) != 0) return hipErrorNotSupported;
     if (p.s == 2) {
@@ -209,18 +228,24 @@ hipError_t launch_filters_stride2_v(const Problem &p, const RowsGeom &g, const T
     return hipGetLastError();
 }
 
+constexpr int kTaprowStages = 8;   // channels in flight per wave
+// waves per SIMD (5 x 5 'mul' in fp16 vectors of eight holds 40 more registers of spatial taps
+// and would spill some twenty at three)
+template <int K, int VX, bool MUL>
+constexpr int taprow_wpe() { return K == 5 && VX == 8 && MUL ? 2 : 3; }
+
 template <typename T, int K, int D, int VX>
 hipError_t launch_taprow_kdv(const Problem &p, const RowsGeom &g, const T *go, const T *x,
                              const T *cf, const T *sf, T *dcf, T *dsf,
                              typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf,
                              unsigned need, int x_mod, hipStream_t st) {
     using A = typename Acc<T>::type;
-    constexpr int kTaprowStages = 8, kWpe = 3;   // channels in flight per wave; waves per SIMD
     const dim3 grid(g.xcd_per * kXcd), block(kWave * kTaprowWaves);
     const int lds = taprow_lds_bytes<K>((int)sizeof(A));
     const bool pad = rows_shift_in_as_is(g);
 #define DDF_TAPROW_CASE(MUL_, PAD_)                                                              \
-    hipLaunchKernelGGL((k_rows_taprow_filters<T, K, D, MUL_, VX, 1, PAD_, kTaprowStages, kWpe>), \
+    hipLaunchKernelGGL((k_rows_taprow_filters<T, K, D, MUL_, VX, 1, PAD_, kTaprowStages,  \
+                                              taprow_wpe<K, VX, MUL_>()>),               \
                        grid, block, lds, st, g, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod)
     if (p.mul) {
         if (pad) DDF_TAPROW_CASE(true, true);
@@ -266,9 +291,10 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
     RowsGeom g;
     int vx, r;
     // (5 x 5: the tap rows go to the waves of a workgroup)
-    const bool taprow = !fused && rows_taprow_geometry(p, dtype, &g, &vx, &r);
-    if (!taprow && !rows_filters_geometry(p, dtype, fused, &g, &vx, &r)) return hipErrorNotSupported;
-    const uintptr_t mask = (uintptr_t)(vx * sizeof(T)) - 1;
+    const bool taprow = !fused && rows_taprow_plan(p, dtype, &g, &vx, &r);
+    if (!taprow && !rows_filters_plan(p, dtype, fused, &g, &vx, &r)) return hipErrorNotSupported;
+    // (ragged rows take any address of their elements)
+    const uintptr_t mask = g.tail > 0 ? 0 : (uintptr_t)(vx * sizeof(T)) - 1;
     if ((((uintptr_t)x | (uintptr_t)go | (uintptr_t)sf | (uintptr_t)dsf | (uintptr_t)dx) & mask) != 0)
         return hipErrorNotSupported;
     if (p.s == 2 && (x_mod != 0 || (((uintptr_t)x | (uintptr_t)dx) &
@@ -296,6 +322,9 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
                 if (vx == 4) DDF_S2_CASE(4);
             }
 #undef DDF_S2_CASE
+        } else if (g.tail > 0) {
+            err = taprow ? rows_ragged_taprow_launch<T>(p, g, vx, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod, st)
+                         : rows_ragged_filters_launch<T>(p, g, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, x_mod, st);
         } else if (taprow) {
             if (vx == 4)
                 err = rows::launch_taprow_v<T, 4>(p, g, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod, st);
@@ -343,11 +372,11 @@ hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *g
         // every vector access 16-byte aligned, so no launch below can turn the call down
         if ((((uintptr_t)go | (uintptr_t)x | (uintptr_t)sf | (uintptr_t)dx | (uintptr_t)dsf) & 15u) != 0)
             return hipErrorNotSupported;
-        if (want_dx && fneed && rows_filters_geometry(p, dtype, true, &g, &vx, &r))
+        if (want_dx && fneed && rows_filters_plan(p, dtype, true, &g, &vx, &r))
             return rows_filters_launch<T>(p, go, x, cf, sf, dx, dcf, dsf, ws, fneed, st, x_mod);
-        if (want_dx && !rows_geometry(p, dtype, 0, &g, &vx, &r)) return hipErrorNotSupported;
-        if (fneed && !rows_taprow_geometry(p, dtype, &g, &vx, &r) &&
-            !rows_filters_geometry(p, dtype, false, &g, &vx, &r))
+        if (want_dx && !rows_plan(p, dtype, &g, &vx, &r)) return hipErrorNotSupported;
+        if (fneed && !rows_taprow_plan(p, dtype, &g, &vx, &r) &&
+            !rows_filters_plan(p, dtype, false, &g, &vx, &r))
             return hipErrorNotSupported;
         hipError_t err = hipSuccess;
         if (want_dx) {

@@ -36,7 +36,7 @@ constexpr int taprow_lds_bytes(int asz) {
 
 #ifdef __HIPCC__
 
-template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, int NST, int WPE>
+template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, int NST, int WPE, int TAIL = 0>
 __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filters(
     RowsGeom g, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,
     const T *__restrict__ sf, T *__restrict__ dcf, T *__restrict__ dsf,
@@ -62,17 +62,21 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
     const int nch = wk.c_end - c0;
     const int64_t plane = (int64_t)g.H * g.W;
     const uint32_t plane_bytes = (uint32_t)plane * (uint32_t)sizeof(T);
-    Lane<R, 0, VX> ln;
+    Lane<R, 0, VX, (TAIL > 0)> ln;
     ln.init(g, wk.strip, lane, (trow - RAD) * D);
+    static_assert(TAIL == 0 || PAD, "ragged rows: padded");
+    Ragged<T, VX, TAIL> rag;
+    rag.init(g, ln.ragged);
 
     const int64_t xn = x_mod ? wk.n % x_mod : wk.n;   // (see k_rows_filters)
     const T *xs = x + (xn * g.C + c0) * plane;
     const T *gs = go + (wk.n * g.C + c0) * plane;
-    uint32_t xb[R], ob[R];
+    uint32_t xb[R], ob[R], lob[R];   // (lob: where the lane's own vectors are loaded)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         xb[r] = ln.xoff[r] < 0 ? kOutside : (uint32_t)ln.xoff[r] * (uint32_t)sizeof(T);
         ob[r] = ln.ooff[r] < 0 ? kOutside : (uint32_t)ln.ooff[r] * (uint32_t)sizeof(T);
+        lob[r] = rag.load_at(ob[r]);
     }
     const int tl = lane < K ? lane : K - 1;
     const T *cfs = cf + (wk.n * g.C + c0) * KK + trow * K;   // the wave's K taps of a channel
@@ -93,7 +97,7 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
         for (int j = 0; j < K; ++j) {
             const __amdgpu_buffer_rsrc_t sr = plane_rsrc(sfn + j * plane, plane_bytes);
 #pragma unroll
-            for (int r = 0; r < R; ++r) load_words<NW>(sr, ob[r], sfw[r][j]);
+            for (int r = 0; r < R; ++r) load_words<NW>(sr, lob[r], sfw[r][j]);
         }
     }
     // A channel past the last one gets an empty descriptor: it reads zeros and so
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
 #pragma unroll
         for (int r = 0; r < R; ++r) load_words<NW>(pr, xb[r], xw[ST][r]);
 #pragma unroll
-        for (int r = 0; r < R; ++r) load_words<NW>(gr, ob[r], gw[ST][r]);
+        for (int r = 0; r < R; ++r) load_words<NW>(gr, lob[r], gw[ST][r]);
         if constexpr (MUL) {
             const int cc = live ? ci : nch - 1;
             if constexpr (kScalarTaps) {
@@ -130,6 +134,12 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
             for (int j = 0; j < K; ++j)
 #pragma unroll
                 for (int k = 0; k < NW; ++k) asm volatile("" : "+v"(sfw[r][j][k]));
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int j = 0; j < K; ++j) rag.fix(sfw[r][j]);
+        }
     }
 
     A acc_sf[R][K][VX];
@@ -197,6 +207,10 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
         for (int r = 0; r < R; ++r) {
 #pragma unroll
             for (int k = 0; k < NW; ++k) row[r].own[k] = xw[ST][r][k];
+            if constexpr (TAIL) {
+                rag.fix(row[r].own);
+                rag.fix(gw[ST][r]);
+            }
             row[r].sides(ln.first, ln.last);
         }
         A w[K];
@@ -268,7 +282,7 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
             if (g.csplit == 1) {
                 uint32_t ow[NW];
                 pack<T, VX, A>(acc_sf[r][j], ow);
-                store_words_nt<NW>(plane_rsrc(dsf + (wk.n * KK + t) * plane, plane_bytes), ob[r], ow);
+                rag.store(plane_rsrc(dsf + (wk.n * KK + t) * plane, plane_bytes), ob[r], ow);
             } else {
                 // partial sums in the accumulator type, same plane shape
                 constexpr int AW = VX * sizeof(A) / 4;
@@ -280,12 +294,22 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
                                                          : ob[r] / (uint32_t)sizeof(T) * (uint32_t)sizeof(A);
                 uint32_t aw[AW];
                 pack<A, VX, A>(acc_sf[r][j], aw);
+                if constexpr (TAIL) {
+                    // (value by value: the last lane of a row has fewer)
 #pragma unroll
-                for (int h = 0; h < AW; h += CH) {
-                    uint32_t part[CH];
+                    for (int h = 0; h < AW; ++h) {
+                        const uint32_t one[1] = {aw[h]};
+                        store_words_nt<1>(wr, off_a == kOutside || (rag.last && h >= rag.tail) ? kOutside : off_a + h * 4,
+                                          one);
+                    }
+                } else {
 #pragma unroll
-                    for (int q = 0; q < CH; ++q) part[q] = aw[h + q];
-                    store_words_nt<CH>(wr, off_a + h * 4, part);
+                    for (int h = 0; h < AW; h += CH) {
+                        uint32_t part[CH];
+#pragma unroll
+                        for (int q = 0; q < CH; ++q) part[q] = aw[h + q];
+                        store_words_nt<CH>(wr, off_a + h * 4, part);
+                    }
                 }
             }
         }
@@ -300,5 +324,7 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
 // is a wave handling one filter row of one (sample, strip, channel range);
 // g->nwork counts all K of each, g->csplit the ranges of g->cpb = g->cpw channels.
 bool rows_taprow_geometry(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r);
+// What runs: that geometry or the one for ragged rows (see rows_plan).
+bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r);
 
 }  // namespace ddf

@@ -251,7 +251,7 @@ bool tiled_forward_supported(const Problem &p, int dtype) {
     WaveGeom g; int ps, nv;
     RowsGeom rg; int vx, r;
     return wave_geometry(p, dtype, kWaveForward, 0, &g, &ps, &nv) ||
-           (dtype != DDF_F64 && rows_geometry(p, dtype, 0, &rg, &vx, &r));
+           (dtype != DDF_F64 && rows_plan(p, dtype, &rg, &vx, &r));
 }
 
 bool tiled_backward_supported(const Problem &p, int dtype) {

@@ -1,0 +1,50 @@
+"""Row-register kernels over rows that are no whole number of vectors: every length of the last
+vector, both lane layouts, planes whose last row ends a tensor, each gradient on its own."""
+import pytest
+import torch
+
+from ddfnet_amd import _lib
+from ddf_testlib import TOL, check_against_oracle, random_case, rel_err, run_ddf
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _ids(v):
+    return str(v).replace('torch.', '')
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('k,d', [(3, 1), (3, 2), (5, 1), (5, 2)])
+@pytest.mark.parametrize('W', [9, 10, 11, 33, 61, 63, 71, 129, 131, 263, 265])
+def test_every_tail(W, k, d, combine, dtype):
+    """Rows of one vector and a tail up to rows cut into segments; enough channels that the
+    filter gradients go through partial sums."""
+    N, C, H = (5, 67, 23) if W < 100 else (3, 24, 131 if k == 3 and d == 1 and W == 131 else 9)
+    shape = (N, C, H, W)
+    names = _lib.describe(shape, k, d, 1, combine, dtype), _lib.describe(shape, k, d, 1, combine, dtype, need=7)
+    if W % 2 and (d == 2 or k == 5):     # (nothing else covers these)
+        assert all('ragged' in n for n in names), names
+    case = random_case(N, C, H, W, k, 1, dtype, seed=W + k + d)
+    check_against_oracle(*case, k, d, 1, combine, '', what='ragged rows')
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('shape', [(16, 70, 47, 57), (8, 66, 61, 85), (4, 66, 113, 133)], ids=_ids)
+def test_wide_vectors_instead_of_single_pixels(shape, combine, dtype):
+    """Sizes that single-pixel vectors cover too and the wide ones take over; each gradient
+    on its own."""
+    for need in (0, _lib.NEED_DX, 6, 7):
+        name = _lib.describe(shape, 3, 1, 1, combine, dtype, need) if need else \
+            _lib.describe(shape, 3, 1, 1, combine, dtype)
+        assert 'ragged' in name, name
+    x, cf, sf, go = random_case(*shape, 3, 1, dtype, seed=3)
+    want = (oracle.forward(x, cf, sf, 3, 1, 1, combine),) + tuple(oracle.backward(go, x, cf, sf, 3, 1, 1, combine))
+    for need in ((True, False, False), (False, True, True), (True, True, True)):
+        got = run_ddf(x, cf, sf, go, 3, 1, 1, combine, need=need)
+        for g, w in zip(got, want):
+            if g is not None:
+                assert rel_err(g, w) <= TOL[dtype]
