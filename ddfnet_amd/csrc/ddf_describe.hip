@@ -21,6 +21,7 @@ const char *sums_name(unsigned fneed, int csplit, int nstrips, bool norm = false
     return sf && cf ? " + k_sum_partials_pair" : (sf || cf) ? " + k_sum_partials" : "";
 }
 const char *layout_name(const RowsGeom &g) {
+    if (g.cw > 0) return g.segs > 0 ? "ragged segments,stride 2" : "ragged,stride 2";
     if (g.Hi != g.H) return g.lp > g.lpr ? "padded,stride 2" : "plain,stride 2";
     if (g.tail > 0) return g.segs > 0 ? "ragged segments" : "ragged";
     return g.segs > 0 ? "segments" : g.lp > g.lpr ? "padded" : "plain";
@@ -79,7 +80,7 @@ int describe_backward(const Problem &p, int dtype, unsigned need, char *buf, int
     }
     if (need & DDF_NEED_DX) {
         if (dtype != DDF_F64 && tune_int("DDF_TUNE_ROWS", 1) != 0 &&
-            (p.s == 1 || rows_stride2_feature_gradient(p)) && rows_plan(p, dtype, &rg, &vx, &r))
+            rows_plan(p, dtype, &rg, &vx, &r, true))
             add("k_rows<dX,VX=%d,R=%d,%s>", vx, r, layout_name(rg));
         else if (small_supported(p)) add("%s", "k_small<dX>");
         else add("%s", "k_backward_features");

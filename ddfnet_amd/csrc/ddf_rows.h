@@ -65,6 +65,10 @@ struct RowsGeom {
     // belong to the row; see Ragged): shift: an odd tail of 2-byte elements, whose lane loads
     // from one element further left.
     int tail, shift;
+    // Stride 2 on the TAIL kernels: the lanes cover ch x cw result pixels - the result plane
+    // itself or, where every feature pixel is some lane's, half the feature plane rounded up
+    // (the row and column past the result plane hold no results; 0: not such a geometry).
+    int ch, cw;
 };
 
 // The vectors shifted in from the neighbouring lanes are right as they arrive
@@ -195,6 +199,47 @@ struct LaneStride2 {
         }
         ooff[0] = live ? y * g.W + x0 : -1;
         onext = (live && y + 1 < g.H) ? (y + 1) * g.W + x0 : -1;
+    }
+};
+
+// The same over g.ch x g.cw, with rows cut into segments where they are long and a last
+// vector that reaches past the result row (ragged: g.tail of its pixels exist, maybe none).
+//   roff: result rows y and y + 1 as the lane reads them (the outer lanes of a segment too);
+//   ooff: the result pixels the lane owns; soff: its feature rows 2y and 2y + 1.
+template <int VX>
+struct LaneStride2Ragged {
+    static constexpr int ROWS = 3;
+    bool first, last, ragged;
+    int xoff[ROWS];
+    int roff[2], ooff[1], soff[2];
+    __host__ __device__ __forceinline__ void init(const RowsGeom &g, int strip, int lane, int = 0) {
+        int x0, y;
+        bool reads, owns;
+        if (g.segs > 0) {
+            y = magic_div(strip, g.segs_magic);
+            x0 = ((strip - y * g.segs) * g.seg_out + lane - 1) * VX;
+            reads = lane <= g.seg_out + 1 && x0 >= 0 && x0 < g.cw;
+            owns = reads && lane >= 1 && lane <= g.seg_out;
+        } else {
+            const int grp = magic_div(lane, g.lp_magic);
+            const int v = lane - grp * g.lp;
+            y = strip * g.rps + grp;
+            x0 = v * VX;
+            reads = owns = grp < g.rg && v < g.lpr && y < g.ch;
+        }
+        first = last = false;   // (always padded)
+        ragged = reads && x0 + VX > g.W;
+#pragma unroll
+        for (int rr = 0; rr < ROWS; ++rr) {
+            const int yy = 2 * y - 1 + rr;
+            xoff[rr] = (reads && yy >= 0 && yy < g.Hi) ? yy * g.Wi + 2 * x0 : -1;
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            roff[r] = (reads && x0 < g.W && y + r < g.H) ? (y + r) * g.W + x0 : -1;
+            soff[r] = owns ? xoff[1 + r] : -1;
+        }
+        ooff[0] = owns ? roff[0] : -1;
     }
 };
 
@@ -397,6 +442,45 @@ struct ExtRow {
 // go out in pieces.  TAIL == 2: an odd number of 2-byte elements.  The word with the last of
 // them would reach past the row, and on a plane's last row past the buffer, where the whole
 // word reads as zero; such a lane loads from one element further left and shifts.
+template <typename T, int VX, bool ODD>
+struct TailStore {
+    static constexpr int NW = vec_words(VX * sizeof(T));
+    bool last;   // the lane's vector is cut short
+    int tail;    // to this many elements (ODD: maybe an odd number of 2-byte ones)
+    __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, const uint32_t (&w)[NW]) const {
+        static_assert(NW == 2 || NW == 4, "vectors of 8 or 16 bytes");
+        store_vec_nt<VX * sizeof(T)>(rsrc, last ? kOutside : off, w);
+        // the last lane's elements: four, two and one of them (no branches: the other
+        // lanes' offsets lie outside; values are picked by value: a choice between array
+        // elements would put the array into memory)
+        const uint32_t at = last ? off : kOutside;
+        auto piece = [at](bool there, int bytes) { return there && at != kOutside ? at + bytes : kOutside; };
+        if constexpr (sizeof(T) == 2) {
+            if constexpr (VX == 8) {
+                const uint32_t q[2] = {w[0], w[1]};
+                store_words_nt<2>(rsrc, piece(tail & 4, 0), q);
+            }
+            const int done4 = VX == 8 ? tail & 4 : 0;
+            const uint32_t e0 = w[0], e1 = w[1], e2 = w[NW > 2 ? 2 : 0], e3 = w[NW - 1];
+            const uint32_t two[1] = {done4 ? e2 : e0};
+            store_words_nt<1>(rsrc, piece(tail & 2, done4 * 2), two);
+            if constexpr (ODD) {
+                const int k = tail >> 1;
+                const uint32_t one = k == 0 ? e0 : k == 1 ? e1 : k == 2 ? e2 : e3;
+                __builtin_amdgcn_raw_buffer_store_b16((short)one, rsrc, (int)piece(tail & 1, (tail & ~1) * 2), 0, 2);
+            }
+        } else {
+            const uint32_t e0 = w[0], e2 = w[NW > 2 ? 2 : 0];
+            if constexpr (VX == 4) {
+                const uint32_t q[2] = {w[0], w[1]};
+                store_words_nt<2>(rsrc, piece(tail & 2, 0), q);
+            }
+            const uint32_t one[1] = {(tail & 2) ? e2 : e0};
+            store_words_nt<1>(rsrc, piece(tail & 1, (tail & 2) * 4), one);
+        }
+    }
+};
+
 template <typename T, int VX, int TAIL>
 struct Ragged {
     static constexpr int NW = vec_words(VX * sizeof(T)), EPW = 4 / (int)sizeof(T);
@@ -406,7 +490,6 @@ struct Ragged {
     int tail;
     __device__ __forceinline__ void init(const RowsGeom &g, bool ragged) {
         if constexpr (TAIL) {
-            static_assert(VX * sizeof(T) >= 8, "vectors of two words at least");
             last = ragged;
             tail = g.tail;
             sh = (TAIL == 2 && ragged) ? 16u : 0u;
@@ -428,42 +511,29 @@ struct Ragged {
             for (int k = 0; k < NW; ++k) w[k] &= mask[k];
         }
     }
+    // Stride 2: the feature vector of those results, twice as many elements (a whole number
+    // of words, loaded where they are)
+    __device__ __forceinline__ void fix_features(uint32_t (&w)[vec_words(2 * VX * sizeof(T))]) const {
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int k = 0; k < vec_words(2 * VX * (int)sizeof(T)); ++k)
+                w[k] = last && k * EPW >= 2 * tail ? 0u : w[k];
+        }
+    }
     // where the lane's own vector is loaded from, given where its results go
     __device__ __forceinline__ uint32_t load_at(uint32_t off) const {
         if constexpr (TAIL == 2) return off == kOutside ? kOutside : off - sh / 8u;
         else return off;
     }
     __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, const uint32_t (&w)[NW]) const {
-        store_vec_nt<VX * sizeof(T)>(rsrc, TAIL && last ? kOutside : off, w);
-        if constexpr (TAIL) {
-            // the last lane's elements: four, two and one of them (no branches: the other
-            // lanes' offsets lie outside)
-            const uint32_t at = last ? off : kOutside;
-            if constexpr (VX == 8) {
-                const uint32_t q[2] = {w[0], w[1]};
-                store_words_nt<2>(rsrc, (tail & 4) ? at : kOutside, q);
-            }
-            const int done4 = VX == 8 ? tail & 4 : 0;
-            if constexpr (sizeof(T) == 2) {
-                const uint32_t lo = w[0], hi = w[NW - 2];
-                const uint32_t two[1] = {VX == 8 && done4 ? hi : lo};
-                store_words_nt<1>(rsrc, (tail & 2) && at != kOutside ? at + done4 * 2 : kOutside, two);
-                if constexpr (TAIL == 2) {
-                    // (by value: a choice between array elements would put the array into memory)
-                    const int k = tail >> 1;
-                    const uint32_t e1 = w[1], e2 = w[NW > 2 ? 2 : 0], e3 = w[NW - 1];
-                    const uint32_t one = k == 0 ? lo : k == 1 ? e1 : k == 2 ? e2 : e3;
-                    __builtin_amdgcn_raw_buffer_store_b16((short)one, rsrc,
-                                                          (int)(at != kOutside ? at + (tail & ~1) * 2 : kOutside), 0, 2);
-                }
-            } else {
-                const uint32_t q[2] = {w[0], w[1]};
-                store_words_nt<2>(rsrc, (tail & 2) ? at : kOutside, q);
-                const uint32_t lo = w[0], hi = w[2];
-                const uint32_t one[1] = {(tail & 2) ? hi : lo};
-                store_words_nt<1>(rsrc, (tail & 1) && at != kOutside ? at + (tail & 2) * 4 : kOutside, one);
-            }
-        }
+        if constexpr (TAIL) TailStore<T, VX, TAIL == 2>{last, tail}.store(rsrc, off, w);
+        else store_vec_nt<VX * sizeof(T)>(rsrc, off, w);
+    }
+    // (stride 2: a feature row of 2 * VX elements; g.Wi odd: one feature pixel more)
+    __device__ __forceinline__ void store_features(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, const RowsGeom &g,
+                                                   const uint32_t (&w)[vec_words(2 * VX * sizeof(T))]) const {
+        if constexpr (TAIL) TailStore<T, 2 * VX, true>{last, 2 * tail + (g.Wi & 1)}.store(rsrc, off, w);
+        else store_vec_nt<2 * VX * sizeof(T)>(rsrc, off, w);
     }
 };
 
@@ -499,7 +569,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     using Row = ExtRow<T, S * VX, HX, PAD>;
     static_assert(KK <= kWave, "one lane per channel-filter tap");
     static_assert(S == 1 || (S == 2 && K == 3 && D == 1 && R == 1), "stride 2: 3 x 3, one row per lane");
-    static_assert(TAIL == 0 || (S == 1 && PAD), "ragged rows: stride 1, padded");
+    static_assert(TAIL == 0 || PAD, "ragged rows: padded");
     // Stride-2 feature gradient: the lane of result row y loads dO rows y and y + 1 and
     // writes the feature rows 2y and 2y + 1 of its columns (even feature heights).
     constexpr bool S2B = S == 2 && BWD;
@@ -515,7 +585,8 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     const uint32_t plane_bytes = (uint32_t)plane * (uint32_t)sizeof(T);
     const int64_t xplane = S == 1 ? plane : (int64_t)g.Hi * g.Wi;
     const uint32_t xplane_bytes = S == 1 ? plane_bytes : (uint32_t)xplane * (uint32_t)sizeof(T);
-    std::conditional_t<S == 1, Lane<R, HY, VX, (TAIL > 0)>, LaneStride2<VX>> ln;
+    std::conditional_t<S == 1, Lane<R, HY, VX, (TAIL > 0)>,
+                       std::conditional_t<TAIL == 0, LaneStride2<VX>, LaneStride2Ragged<VX>>> ln;
     ln.init(g, wk.strip, lane);
     Ragged<T, VX, TAIL> rag;
     rag.init(g, ln.ragged);
@@ -541,7 +612,14 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     const int tsel = kFlip ? KK - 1 - tl : tl;
     // where the lane's loads are
     uint32_t lb[LROWS];
-    if constexpr (S2B) {
+    if constexpr (S2B && TAIL) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            lb[r] = rag.load_at(ln.roff[r] < 0 ? kOutside : (uint32_t)ln.roff[r] * (uint32_t)sizeof(T));
+            // (and the feature rows it writes)
+            xb[1 + r] = ln.soff[r] < 0 ? kOutside : (uint32_t)ln.soff[r] * (uint32_t)sizeof(T);
+        }
+    } else if constexpr (S2B) {
         lb[0] = ob[0];
         lb[1] = ln.onext < 0 ? kOutside : (uint32_t)ln.onext * (uint32_t)sizeof(T);
     } else {
@@ -570,6 +648,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
                     const __amdgpu_buffer_rsrc_t sr = plane_rsrc(sfn + t * plane, plane_bytes);
                     SRow row;
                     load_vec<kVB>(sr, lb[i == 0 ? 1 : 0], row.own);
+                    rag.fix(row.own);
                     if (j == 0) {
                         row.sides(ln.first, ln.last);
                         A v[VX];
@@ -724,6 +803,8 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             GRow g0, g1;
 #pragma unroll
             for (int k = 0; k < NW; ++k) { g0.own[k] = xw[ST][0][k]; g1.own[k] = xw[ST][1][k]; }
+            rag.fix(g0.own);
+            rag.fix(g1.own);
             g0.sides(ln.first, ln.last);
             g1.sides(ln.first, ln.last);
             // dO * comb(CF[i][j], SF[i][j]) with the spatial tap of slot (i, j)
@@ -753,9 +834,9 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             }
             uint32_t ow[NWX];
             pack<T, 2 * VX, A>(top, ow);
-            store_vec_nt<kXB>(dr, xb[1], ow);
+            rag.store_features(dr, xb[1], g, ow);
             pack<T, 2 * VX, A>(bot, ow);
-            store_vec_nt<kXB>(dr, xb[2], ow);
+            rag.store_features(dr, xb[2], g, ow);
         } else {
         Row row[ROWS];
 #pragma unroll
@@ -763,7 +844,8 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             if (!row_needed<R, K, D>(rr)) continue;
 #pragma unroll
             for (int k = 0; k < NWX; ++k) row[rr].own[k] = xw[ST][rr][k];
-            if constexpr (TAIL) rag.fix(row[rr].own);
+            // (stride 2: what lies past the row reaches no result that is stored)
+            if constexpr (TAIL && S == 1) rag.fix(row[rr].own);
             row[rr].sides(ln.first, ln.last);
         }
         A acc[R][VX];
@@ -889,6 +971,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
 bool rows_geometry(const Problem &p, int dtype, int max_vx, RowsGeom *g, int *vx, int *r);
 // What runs: that geometry, or wide vectors over rows they do not divide (g->tail > 0: the
 // TAIL kernels) where those take fewer instructions or the other covers nothing.
-bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r);
+// backward: of the feature gradient (the same as forward except with stride 2).
+bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r, bool backward = false);
 
 }  // namespace ddf

@@ -99,9 +99,10 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
     const uint32_t plane_bytes = (uint32_t)plane * (uint32_t)sizeof(T);
     const int64_t xplane = S == 1 ? plane : (int64_t)g.Hi * g.Wi;
     const uint32_t xplane_bytes = S == 1 ? plane_bytes : (uint32_t)xplane * (uint32_t)sizeof(T);
-    std::conditional_t<S == 1, Lane<R, HY, VX, (TAIL > 0)>, LaneStride2<VX>> ln;
+    std::conditional_t<S == 1, Lane<R, HY, VX, (TAIL > 0)>,
+                       std::conditional_t<TAIL == 0, LaneStride2<VX>, LaneStride2Ragged<VX>>> ln;
     ln.init(g, wk.strip, lane);
-    static_assert(TAIL == 0 || (S == 1 && PAD), "ragged rows: stride 1, padded");
+    static_assert(TAIL == 0 || PAD, "ragged rows: padded");
     Ragged<T, VX, TAIL> rag;
     rag.init(g, ln.ragged);
 
@@ -119,8 +120,14 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
     for (int r = 0; r < R; ++r)
         ob[r] = ln.ooff[r] < 0 ? kOutside : (uint32_t)ln.ooff[r] * (uint32_t)sizeof(T);
     // where the lane's dO rows are
-    uint32_t gb[GROWS];
-    if constexpr (DX && S == 2) {
+    uint32_t gb[GROWS], sb[2] = {xb[1], xb[ROWS > 2 ? 2 : 1]};   // (sb: feature rows written, stride 2)
+    if constexpr (DX && S == 2 && TAIL) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            gb[r] = rag.load_at(ln.roff[r] < 0 ? kOutside : (uint32_t)ln.roff[r] * (uint32_t)sizeof(T));
+            sb[r] = ln.soff[r] < 0 ? kOutside : (uint32_t)ln.soff[r] * (uint32_t)sizeof(T);
+        }
+    } else if constexpr (DX && S == 2) {
         gb[0] = ob[0];
         gb[1] = ln.onext < 0 ? kOutside : (uint32_t)ln.onext * (uint32_t)sizeof(T);
     } else {
@@ -182,7 +189,10 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                 const int t = i * K + j;
                 const __amdgpu_buffer_rsrc_t sr = plane_rsrc(sfn + t * plane, plane_bytes);
                 uint32_t own[NW];
-                if (MUL || i > 0) load_vec<kVB>(sr, gb[0], own);
+                if (MUL || i > 0) {
+                    load_vec<kVB>(sr, gb[0], own);
+                    rag.fix(own);
+                }
                 if constexpr (MUL) {
 #pragma unroll
                     for (int k = 0; k < NW; ++k) sfw[0][t][k] = own[k];
@@ -190,6 +200,7 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                 SRow row;
                 if (i == 0) {
                     load_vec<kVB>(sr, gb[1], row.own);
+                    rag.fix(row.own);
                 } else {
 #pragma unroll
                     for (int k = 0; k < NW; ++k) row.own[k] = own[k];
@@ -326,13 +337,14 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
             if (!row_needed<R, K, D>(rr)) continue;
 #pragma unroll
             for (int k = 0; k < NWX; ++k) row[rr].own[k] = xw[ST][rr][k];
-            if constexpr (TAIL) rag.fix(row[rr].own);
+            if constexpr (TAIL && S == 1) rag.fix(row[rr].own);
+            if constexpr (TAIL && S == 2) rag.fix_features(row[rr].own);
             row[rr].sides(ln.first, ln.last);
         }
         if constexpr (TAIL) {
 #pragma unroll
             for (int r = 0; r < GROWS; ++r)
-                if (!DX || row_needed<R, K, D>(r)) rag.fix(gw[ST][r]);
+                if (!DX || S == 2 || row_needed<R, K, D>(r)) rag.fix(gw[ST][r]);
         }
         // dO at the lane's own pixels.  (DX loads dO through the window offsets, so a
         // lane that only reads for its neighbours - the outer lanes of a row segment -
@@ -439,9 +451,9 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
             }
             uint32_t ow[NWX];
             pack<T, 2 * VX, A>(top, ow);
-            store_vec_nt<kXB>(dr, xb[1], ow);
+            rag.store_features(dr, sb[0], g, ow);
             pack<T, 2 * VX, A>(bot, ow);
-            store_vec_nt<kXB>(dr, xb[2], ow);
+            rag.store_features(dr, sb[1], g, ow);
         } else if constexpr (DX) {
             // feature gradient of the lane's pixels: dO at the flipped tap offsets
             Row grow[ROWS];

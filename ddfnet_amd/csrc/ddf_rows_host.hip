@@ -22,7 +22,7 @@ unsigned magic_of(int d) { return d == 1 ? 0u : (unsigned)((0x100000000ull + d -
 // which is exactly what the neighbour shift must bring in at the row ends.
 // Rows vx does not divide (the TAIL kernels, which are built padded): ceil(W / vx) lanes,
 // always followed by the idle one.
-void lay_out_lanes(RowsGeom *t, int H, int W, int vx, int R) {
+void lay_out_lanes(RowsGeom *t, int H, int W, int vx, int R, bool padded = false) {
     t->segs = t->seg_out = 0;
     t->segs_magic = 0;
     t->tail = W % vx;
@@ -46,7 +46,7 @@ void lay_out_lanes(RowsGeom *t, int H, int W, int vx, int R) {
     const int fit_plain = std::min(kWave / t->lpr, row_units);
     const int fit_padded = std::min((kWave + 1) / (t->lpr + 1), row_units);
     auto strips_with = [&](int fit) { return fit > 0 ? (row_units + fit - 1) / fit : 1 << 30; };
-    const bool pad = t->tail > 0 || (fit_padded > 0 && strips_with(fit_padded) <= strips_with(fit_plain) &&
+    const bool pad = padded || t->tail > 0 || (fit_padded > 0 && strips_with(fit_padded) <= strips_with(fit_plain) &&
                                      tune_int("DDF_TUNE_ROWS_PAD", 1) != 0);
     t->lp = t->lpr + (pad ? 1 : 0);
     t->lp_magic = magic_of(t->lp);
@@ -238,6 +238,51 @@ bool cut_channels_taprow(RowsGeom &t, const Problem &p) {
     return true;
 }
 
+// Stride 2 with any sizes: 16-byte feature vectors, rows cut into segments where they are
+// long, the last vector of a row cut short (LaneStride2Ragged).  whole: the lanes cover the
+// feature plane (every feature pixel's gradient is written), not only the result plane.
+bool stride2_ragged_geometry(const Problem &p, int dtype, bool filters, bool whole, RowsGeom *g, int *vx_out,
+                             int *r_out) {
+    if (!(p.s == 2 && p.k == 3 && p.d == 1)) return false;
+    if (dtype != DDF_F16 && dtype != DDF_F32) return false;
+    const int vx = dtype == DDF_F16 ? 4 : 2;
+    if (p.N <= 0 || p.C <= 0 || p.Ho <= 0 || p.Wo <= vx) return false;   // (an odd tail loads one pixel to its left)
+    if (p.H > 16384 || p.W > 16384 || p.C > (1 << 24) || p.N > (1 << 24)) return false;
+    if (p.H * p.W * 8 >= (1ll << 31) || tune_int("DDF_TUNE_RAGGED", 1) == 0) return false;
+    RowsGeom t{};
+    t.ch = (int)(whole ? (p.H + 1) / 2 : p.Ho);
+    t.cw = (int)(whole ? (p.W + 1) / 2 : p.Wo);
+    lay_out_lanes(&t, t.ch, t.cw, vx, 1, true);
+    t.C = (int)p.C; t.H = (int)p.Ho; t.W = (int)p.Wo; t.Hi = (int)p.H; t.Wi = (int)p.W;
+    t.tail = t.W % vx;
+    t.shift = dtype == DDF_F16 ? t.tail & 1 : 0;
+    if (filters ? !cut_channels_filters(t, p.N, t.C)
+                : !cut_channels_forward(t, p.N, t.C, kRowsStages, (int64_t)t.H * t.W))
+        return false;
+    *g = t;
+    *vx_out = vx;
+    *r_out = 1;
+    return true;
+}
+
+// What a launch of k_rows takes, for choosing between two cuts of a problem: the instructions
+// of a wave - some 40 per channel and 16 per pixel of a lane (25 taps: 45), the spatial taps
+// before the walk as much as three channels - times its waves per SIMD, of which it takes two
+// or three to keep one busy.  Ragged vectors cost more than their masks: unaligned accesses
+// touch a cache line more.
+double rows_cost(const RowsGeom &g, bool ragged, int k, int esz, int vx, int r) {
+    const double per_wave = (g.cpw + 3.0) * (40 + (k == 5 ? 45 : 16) * vx * r);
+    const double over = !ragged ? 1.0 : g.shift ? 1.5 : esz == 2 ? 1.05 : 1.15;
+    return per_wave * over * std::max(2.5, (double)g.nwork / kSimds);
+}
+
+// The same for k_rows_filters: some 60 instructions per channel and 50 per pixel of a lane;
+// two loads per channel leave a single wave per SIMD busy enough.
+double rows_filters_cost(const RowsGeom &g, bool ragged, int vx, int r) {
+    const double waves = (double)g.nwork * rows::kFilterWaves;
+    return (g.cpw + 3.0) * (60 + 50 * vx * r) * (ragged ? 1.1 : 1.0) * std::max(1.0, waves / kSimds);
+}
+
 }  // namespace
 
 // Instantiated (elements per lane and row, rows per lane) per element size.
@@ -304,35 +349,35 @@ bool rows_ragged_geometry(const Problem &p, int dtype, int vx, RowsGeom *g, int 
     return true;
 }
 
-bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r) {
-    const bool exact = rows_geometry(p, dtype, 0, g, vx, r);
+bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r, bool backward) {
+    // (stride 2: the exact cut writes feature rows 2y and 2y + 1 per result row)
+    const bool exact = (p.s != 2 || !backward || p.H % 2 == 0) && rows_geometry(p, dtype, 0, g, vx, r);
     if (dtype != DDF_F16 && dtype != DDF_F32) return exact;
-    // What a launch takes: the instructions of a wave - some 40 per channel and 16 per pixel
-    // of a lane (25 taps: 45), the spatial taps before the walk as much as three channels -
-    // times its waves per SIMD, of which it takes two or three to keep one busy.  Ragged
-    // vectors cost more than their masks: unaligned 16-byte accesses touch a cache line more.
-    // (Fitted over 80 sizes; forward at 12 x 144 x 80 x 87 fp32 28.1 -> 19.9 us, fp16 26.3 ->
-    // 19.3; 5 x 5 at 2 x 48 x 135 x 166, which only the LDS-tile kernels covered, 45 -> 11.3.
-    // Small launches keep vectors that divide their rows: 4 x 256 x 25 x 38 fp16 takes 5.2 us
-    // in vectors of two and 6.7 in eight.)
-    auto cost = [&](const RowsGeom &t, int v, int rows) {
-        const double per_wave = (t.cpw + 3.0) * (40 + (p.k == 5 ? 45 : 16) * v * rows);
-        const double over = t.tail == 0 ? 1.0 : t.shift ? 1.5 : dtype == DDF_F16 ? 1.05 : 1.15;
-        return per_wave * over * std::max(2.5, (double)t.nwork / kSimds);
-    };
-    double best = exact ? cost(*g, *vx, *r) : 1e30;
+    // Which cut: fitted over 80 sizes.  Forward at 12 x 144 x 80 x 87 fp32 28.1 -> 19.9 us, fp16
+    // 26.3 -> 19.3; 5 x 5 at 2 x 48 x 135 x 166, which only the LDS-tile kernels covered, 45 ->
+    // 11.3.  Small launches keep vectors that divide their rows: 4 x 256 x 25 x 38 fp16 takes
+    // 5.2 us in vectors of two and 6.7 in eight.
+    const int esz = dtype == DDF_F16 ? 2 : 4;
+    double best = exact ? rows_cost(*g, false, p.k, esz, *vx, *r) : 1e30;
     bool found = exact;
-    // (what the shortest ragged walk takes: small launches are decided without laying it out)
-    if (best <= (std::min<int64_t>(p.C, 2 * kRowsStages) + 3.0) * (40 + (p.k == 5 ? 45 : 16) * 4) * 2.5) return true;
-    for (int cand = dtype == DDF_F16 ? 8 : 4; cand >= 4; cand /= 2) {
-        RowsGeom t; int tr;
-        if (!rows_ragged_geometry(p, dtype, cand, &t, &tr) || cost(t, cand, tr) >= best) continue;
-        best = cost(t, cand, tr);
+    RowsGeom t; int tvx, tr;
+    auto consider = [&]() {
+        const double c = rows_cost(t, true, p.k, esz, tvx, tr);
+        if (c >= best) return;
+        best = c;
         found = true;
         *g = t;
-        *vx = cand;
+        *vx = tvx;
         *r = tr;
+    };
+    if (p.s == 2) {
+        if (stride2_ragged_geometry(p, dtype, false, backward, &t, &tvx, &tr)) consider();
+        return found;
     }
+    // (what the shortest ragged walk takes: small launches are decided without laying it out)
+    if (best <= (std::min<int64_t>(p.C, 2 * kRowsStages) + 3.0) * (40 + (p.k == 5 ? 45 : 16) * 4) * 2.5) return true;
+    for (tvx = 16 / esz; tvx >= 4; tvx /= 2)
+        if (rows_ragged_geometry(p, dtype, tvx, &t, &tr)) consider();
     return found;
 }
 
@@ -390,26 +435,25 @@ bool rows_filters_geometry(const Problem &p, int dtype, bool fused, RowsGeom *g,
 
 bool rows_filters_plan(const Problem &p, int dtype, bool fused, RowsGeom *g, int *vx, int *r) {
     const bool exact = rows_filters_geometry(p, dtype, fused, g, vx, r);
-    if (p.k != 3 || (p.d != 1 && p.d != 2) || !ragged_shape(p, dtype, 4)) return exact;
     if (fused && tune_int("DDF_TUNE_ROWSF_FUSED", 1) == 0) return exact;
     RowsGeom t{};
-    t.C = (int)p.C; t.H = t.Hi = (int)p.H; t.W = t.Wi = (int)p.W;
-    lay_out_lanes(&t, (int)p.H, (int)p.W, 4, 1);
-    if (!cut_channels_filters(t, p.N, (int)p.C)) return exact;
-    t.shift = dtype == DDF_F16 ? t.tail & 1 : 0;
-    // (as rows_plan; a wave issues some 60 instructions per channel and 50 per pixel of a
-    // lane, and two loads per channel leave a single wave per SIMD busy enough.  All
-    // gradients at 12 x 144 x 80 x 87 fp32: 63 -> 42 us; 3 x 3 with dilation 2 at 4 x 64 x
+    int tvx = 4, tr = 1;
+    if (p.s == 2) {
+        if (!stride2_ragged_geometry(p, dtype, true, fused, &t, &tvx, &tr)) return exact;
+    } else {
+        if (p.k != 3 || (p.d != 1 && p.d != 2) || !ragged_shape(p, dtype, tvx)) return exact;
+        t.C = (int)p.C; t.H = t.Hi = (int)p.H; t.W = t.Wi = (int)p.W;
+        lay_out_lanes(&t, t.H, t.W, tvx, tr);
+        if (!cut_channels_filters(t, p.N, t.C)) return exact;
+        t.shift = dtype == DDF_F16 ? t.tail & 1 : 0;
+    }
+    // All gradients at 12 x 144 x 80 x 87 fp32: 63 -> 42 us; 3 x 3 with dilation 2 at 4 x 64 x
     // 60 x 131, which only the LDS-tile kernels covered, 178 -> 18.5; 2 x 256 x 25 x 38 keeps
-    // single pixels, 11.3 us against 12.6.)
-    auto cost = [&](const RowsGeom &u, int px) {
-        const double waves = (double)u.nwork * rows::kFilterWaves;
-        return (u.cpw + 3.0) * (60 + 50 * px) * std::max(1.0, waves / kSimds);
-    };
-    if (exact && cost(t, 4) * 1.1 >= cost(*g, *vx * *r)) return true;
+    // single pixels, 11.3 us against 12.6.
+    if (exact && rows_filters_cost(t, true, tvx, tr) >= rows_filters_cost(*g, false, *vx, *r)) return true;
     *g = t;
-    *vx = 4;
-    *r = 1;
+    *vx = tvx;
+    *r = tr;
     return true;
 }
 
@@ -481,14 +525,14 @@ bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r)
 
 bool rows_cover_backward(const Problem &p, int dtype) {
     RowsGeom g; int vx, r;
-    return p.s == 1 && rows_plan(p, dtype, &g, &vx, &r) &&
+    return rows_plan(p, dtype, &g, &vx, &r, true) &&
            (rows_taprow_plan(p, dtype, &g, &vx, &r) ||
             rows_filters_plan(p, dtype, false, &g, &vx, &r));
 }
 
 bool rows_cover_stride2_filters(const Problem &p, int dtype) {
     RowsGeom g; int vx, r;
-    return p.s == 2 && rows_filters_geometry(p, dtype, false, &g, &vx, &r);
+    return p.s == 2 && rows_filters_plan(p, dtype, false, &g, &vx, &r);
 }
 
 size_t rows_filters_workspace(const Problem &p, int dtype, unsigned need) {

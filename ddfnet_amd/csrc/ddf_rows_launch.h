@@ -112,9 +112,9 @@ hipError_t rows_launch(const Problem &p, bool backward, const T *x, const T *cf,
     const int dtype = sizeof(T) == 2 ? DDF_F16 : sizeof(T) == 4 ? DDF_F32 : DDF_F64;
     RowsGeom g;
     int vx, r;
-    if (!rows_plan(p, dtype, &g, &vx, &r)) return hipErrorNotSupported;
+    if (!rows_plan(p, dtype, &g, &vx, &r, backward)) return hipErrorNotSupported;
     if constexpr (sizeof(T) != 8) {
-        if (g.tail > 0) return rows_ragged_launch<T>(p, g, vx, r, backward, x, cf, sf, out, st);
+        if (g.tail > 0 || g.cw > 0) return rows_ragged_launch<T>(p, g, vx, r, backward, x, cf, sf, out, st);
     }
     const uintptr_t mask = (uintptr_t)(vx * sizeof(T)) - 1;
     if ((((uintptr_t)x | (uintptr_t)sf | (uintptr_t)out) & mask) != 0) return hipErrorNotSupported;
@@ -124,7 +124,6 @@ hipError_t rows_launch(const Problem &p, bool backward, const T *x, const T *cf,
         const T *feat = backward ? out : x;
         if (((uintptr_t)feat & (std::min<uintptr_t>(2 * vx * sizeof(T), 16) - 1)) != 0)
             return hipErrorNotSupported;
-        if (backward && !rows_stride2_feature_gradient(p)) return hipErrorNotSupported;
 #define DDF_S2_CASE(VX_)                                                                       \
     return backward ? rows::launch_stride2_v<T, VX_, true>(p, g, x, cf, sf, out, st)           \
                     : rows::launch_stride2_v<T, VX_, false>(p, g, x, cf, sf, out, st)
@@ -294,11 +293,12 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
     const bool taprow = !fused && rows_taprow_plan(p, dtype, &g, &vx, &r);
     if (!taprow && !rows_filters_plan(p, dtype, fused, &g, &vx, &r)) return hipErrorNotSupported;
     // (ragged rows take any address of their elements)
-    const uintptr_t mask = g.tail > 0 ? 0 : (uintptr_t)(vx * sizeof(T)) - 1;
+    const bool ragged = g.tail > 0 || g.cw > 0;
+    const uintptr_t mask = ragged ? 0 : (uintptr_t)(vx * sizeof(T)) - 1;
     if ((((uintptr_t)x | (uintptr_t)go | (uintptr_t)sf | (uintptr_t)dsf | (uintptr_t)dx) & mask) != 0)
         return hipErrorNotSupported;
-    if (p.s == 2 && (x_mod != 0 || (((uintptr_t)x | (uintptr_t)dx) &
-                                    (std::min<uintptr_t>(2 * vx * sizeof(T), 16) - 1)) != 0))
+    if (p.s == 2 && (x_mod != 0 || (!ragged && (((uintptr_t)x | (uintptr_t)dx) &
+                                                (std::min<uintptr_t>(2 * vx * sizeof(T), 16) - 1)) != 0)))
         return hipErrorNotSupported;
     unsigned char *wp = static_cast<unsigned char *>(ws);
     A *ws_sf = nullptr, *ws_cf = nullptr;
@@ -310,7 +310,10 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
     if ((need & DDF_NEED_DCF) && g.nstrips > 1) ws_cf = reinterpret_cast<A *>(wp);
     hipError_t err = hipErrorNotSupported;
     if constexpr (sizeof(T) != 8) {
-        if (p.s == 2) {
+        if (ragged) {
+            err = taprow ? rows_ragged_taprow_launch<T>(p, g, vx, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod, st)
+                         : rows_ragged_filters_launch<T>(p, g, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, x_mod, st);
+        } else if (p.s == 2) {
 #define DDF_S2_CASE(VX_)                                                                          \
     err = fused ? rows::launch_filters_stride2_v<T, VX_, true>(p, g, go, x, cf, sf, dx, dcf, dsf, \
                                                                ws_sf, ws_cf, need, st)            \
@@ -322,9 +325,6 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
                 if (vx == 4) DDF_S2_CASE(4);
             }
 #undef DDF_S2_CASE
-        } else if (g.tail > 0) {
-            err = taprow ? rows_ragged_taprow_launch<T>(p, g, vx, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod, st)
-                         : rows_ragged_filters_launch<T>(p, g, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, x_mod, st);
         } else if (taprow) {
             if (vx == 4)
                 err = rows::launch_taprow_v<T, 4>(p, g, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod, st);
@@ -374,7 +374,7 @@ hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *g
             return hipErrorNotSupported;
         if (want_dx && fneed && rows_filters_plan(p, dtype, true, &g, &vx, &r))
             return rows_filters_launch<T>(p, go, x, cf, sf, dx, dcf, dsf, ws, fneed, st, x_mod);
-        if (want_dx && !rows_plan(p, dtype, &g, &vx, &r)) return hipErrorNotSupported;
+        if (want_dx && !rows_plan(p, dtype, &g, &vx, &r, true)) return hipErrorNotSupported;
         if (fneed && !rows_taprow_plan(p, dtype, &g, &vx, &r) &&
             !rows_filters_plan(p, dtype, false, &g, &vx, &r))
             return hipErrorNotSupported;

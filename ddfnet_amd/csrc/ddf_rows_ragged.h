@@ -42,6 +42,38 @@ hipError_t launch_ragged(const Problem &p, const RowsGeom &g, int r, bool backwa
     return hipErrorNotSupported;
 }
 
+// Stride 2 (LaneStride2Ragged): forward or (BWD) the feature gradient.
+template <typename T, bool BWD, int TAIL>
+hipError_t launch_ragged_stride2(const Problem &p, const RowsGeom &g, const T *x, const T *cf,
+                                 const T *sf, T *out, hipStream_t st) {
+    const dim3 grid(g.xcd_per * kXcd), block(kWave * g.wpb);
+    constexpr int VX = 8 / (int)sizeof(T);
+    if (p.mul)
+        hipLaunchKernelGGL((k_rows<T, 3, 1, true, BWD, VX, 1, true, kStages, 3, 2, TAIL>), grid, block, 0, st,
+                           g, x, cf, sf, out);
+    else
+        hipLaunchKernelGGL((k_rows<T, 3, 1, false, BWD, VX, 1, true, kStages, 3, 2, TAIL>), grid, block, 0, st,
+                           g, x, cf, sf, out);
+    return hipGetLastError();
+}
+
+template <typename T, bool DX, int TAIL>
+hipError_t launch_ragged_filters_stride2(const Problem &p, const RowsGeom &g, const T *go, const T *x,
+                                         const T *cf, const T *sf, T *dx, T *dcf, T *dsf,
+                                         typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf,
+                                         unsigned need, hipStream_t st) {
+    constexpr int VX = 8 / (int)sizeof(T), kStagesS2 = DX ? 2 : 4;   // (as launch_filters_stride2_v)
+    const dim3 grid(g.xcd_per * kXcd), block(kWave * kFilterWaves);
+    const int lds = filters_lds_bytes<9>((int)sizeof(typename Acc<T>::type), 1, VX);
+    if (p.mul)
+        hipLaunchKernelGGL((k_rows_filters<T, 3, 1, true, VX, 1, true, DX, kStagesS2, 2, 2, DX, TAIL>), grid,
+                           block, lds, st, g, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, 0);
+    else
+        hipLaunchKernelGGL((k_rows_filters<T, 3, 1, false, VX, 1, true, DX, kStagesS2, 2, 2, DX, TAIL>), grid,
+                           block, lds, st, g, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, 0);
+    return hipGetLastError();
+}
+
 template <typename T, bool DX, int TAIL>
 hipError_t launch_ragged_filters(const Problem &p, const RowsGeom &g, const T *go, const T *x,
                                  const T *cf, const T *sf, T *dx, T *dcf, T *dsf,
@@ -96,6 +128,16 @@ hipError_t launch_ragged_taprow(const Problem &p, const RowsGeom &g, const T *go
 template <typename T>
 hipError_t rows_ragged_launch(const Problem &p, const RowsGeom &g, int vx, int r, bool backward,
                               const T *x, const T *cf, const T *sf, T *out, hipStream_t st) {
+    if (p.s == 2) {
+        if (vx * sizeof(T) != 8 || r != 1) return hipErrorNotSupported;
+        if constexpr (sizeof(T) == 2) {
+            if (g.shift)
+                return backward ? rows::launch_ragged_stride2<T, true, 2>(p, g, x, cf, sf, out, st)
+                                : rows::launch_ragged_stride2<T, false, 2>(p, g, x, cf, sf, out, st);
+        }
+        return backward ? rows::launch_ragged_stride2<T, true, 1>(p, g, x, cf, sf, out, st)
+                        : rows::launch_ragged_stride2<T, false, 1>(p, g, x, cf, sf, out, st);
+    }
     if constexpr (sizeof(T) == 2) {
         if (vx == 8)
             return g.shift ? rows::launch_ragged<T, 8, 2>(p, g, r, backward, x, cf, sf, out, st)
@@ -111,6 +153,18 @@ hipError_t rows_ragged_filters_launch(const Problem &p, const RowsGeom &g, const
                                       const T *cf, const T *sf, T *dx, T *dcf, T *dsf,
                                       typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf,
                                       unsigned need, int x_mod, hipStream_t st) {
+    if (p.s == 2) {
+#define DDF_RAGGED_CASE(TAIL_)                                                                          \
+    return dx ? rows::launch_ragged_filters_stride2<T, true, TAIL_>(p, g, go, x, cf, sf, dx, dcf, dsf,  \
+                                                                    ws_sf, ws_cf, need, st)             \
+              : rows::launch_ragged_filters_stride2<T, false, TAIL_>(p, g, go, x, cf, sf, dx, dcf, dsf, \
+                                                                     ws_sf, ws_cf, need, st)
+        if constexpr (sizeof(T) == 2) {
+            if (g.shift) DDF_RAGGED_CASE(2);
+        }
+        DDF_RAGGED_CASE(1);
+#undef DDF_RAGGED_CASE
+    }
 #define DDF_RAGGED_CASE(TAIL_)                                                                          \
     return dx ? rows::launch_ragged_filters<T, true, TAIL_>(p, g, go, x, cf, sf, dx, dcf, dsf, ws_sf,   \
                                                             ws_cf, need, x_mod, st)                     \

@@ -48,3 +48,24 @@ def test_wide_vectors_instead_of_single_pixels(shape, combine, dtype):
         for g, w in zip(got, want):
             if g is not None:
                 assert rel_err(g, w) <= TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('H,W', [(9, 10), (8, 11), (7, 12), (10, 13), (31, 15), (24, 18), (13, 30), (12, 63), (11, 131),
+                                 (9, 261), (6, 262), (7, 263), (4, 286), (3, 257), (2, 135)])
+def test_stride_two_of_any_size(H, W, combine, dtype):
+    """Odd heights and widths, every tail, segments: all gradients in one launch, the features'
+    alone, the filters' alone."""
+    shape = (3, 37, H, W)
+    if W % 2:      # (vectors that divide the rows need even ones)
+        assert 'ragged' in _lib.describe(shape, 3, 1, 2, combine, dtype)
+        for need in (_lib.NEED_DX, 6, 7):
+            assert 'ragged' in _lib.describe(shape, 3, 1, 2, combine, dtype, need)
+    x, cf, sf, go = random_case(*shape, 3, 2, dtype, seed=H + W)
+    want = (oracle.forward(x, cf, sf, 3, 1, 2, combine),) + tuple(oracle.backward(go, x, cf, sf, 3, 1, 2, combine))
+    for need in ((True, False, False), (False, True, True), (True, True, True)):
+        got = run_ddf(x, cf, sf, go, 3, 1, 2, combine, need=need)
+        for g, w in zip(got, want):
+            if g is not None:
+                assert rel_err(g, w) <= TOL[dtype]
