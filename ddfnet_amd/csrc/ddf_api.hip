@@ -764,6 +764,23 @@ int ddf_hip_net_conv(const void *features, const void *weight, const ddf_net_nor
     return net_result(ddf::net_conv(a, (hipStream_t)stream), "ddf_hip_net_conv launch");
 }
 
+int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_net_norm_t *norm, int64_t C,
+                          const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
+                          int64_t H, int64_t W, int64_t side_C, int stride, void *output, int64_t N, int64_t O,
+                          int relu, void *stream) {
+    if (N < 0 || H < 1 || W < 1 || C < 1 || side_C < 1 || O < 1 || stride < 1 || C > (1 << 24) ||
+        side_C > (1 << 24) || O > (1 << 24) || H * W >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_conv_pair: bad sizes");
+    if (!features || !weight || !side_features || !side_weight || !output || !net_norm_ok(norm) || !net_norm_ok(side_norm))
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    const int64_t Ho = (H - 1) / stride + 1, Wo = (W - 1) / stride + 1, M = N * Ho * Wo;
+    const ddf::NetConv a{features, weight, nullptr, output, net_norm(norm), M, (int)O, (int)C, relu,
+                         1, (int)Ho, (int)Wo, (int)Wo, (int)(Ho * Wo)};
+    const ddf::NetConv side{side_features, side_weight, nullptr, output, net_norm(side_norm), M, (int)O, (int)side_C, 0,
+                            stride, (int)H, (int)W, (int)Wo, (int)(Ho * Wo)};
+    return net_result(ddf::net_conv_pair(a, side, (hipStream_t)stream), "ddf_hip_net_conv_pair launch");
+}
+
 int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,
                      int64_t H, int64_t W, void *stream) {
     if (N < 0 || H < 1 || W < 1) return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_stem: bad sizes");

@@ -155,6 +155,8 @@ struct NetConv {
 };
 bool net_conv_supported(const NetConv &a);
 hipError_t net_conv(const NetConv &a, hipStream_t st);
+// act(affine(a) + affine'(first)): same pixels and channels, activation and output a's
+hipError_t net_conv_pair(const NetConv &a, const NetConv &first, hipStream_t st);
 hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,
                     hipStream_t st);
 int net_spatial_chunks(int64_t N, int64_t npix);

@@ -88,24 +88,50 @@ struct Affine {
 // pixel under a stride.  Tiles of BM pixels x BN channels; four waves, 2 x 2 over the tile,
 // each in 32x32x16 steps.  W is the A operand, so a lane ends with runs of four channels of
 // one pixel; the tile goes through LDS once more and leaves as whole 16-byte vectors.
-// K comes in steps of 64 (128 bytes of a row per eight lanes), the next step's vectors in
-// registers while this one's are multiplied, LDS double-buffered: one barrier per step.
-// LDS rows of eight 16-byte chunks, chunk number xor row % 8: both the writes and the
-// operand reads (32 rows at one chunk) touch all banks.
-constexpr int kStep = 64, kChunks = kStep / 8;
-
-template <int BM, int BN>
-constexpr int conv_lds_halves(bool two) {
-    const int stage = (BM + BN) * kStep * (two ? 2 : 1), tile = BM * (BN + 8);
-    return stage > tile ? stage : tile;
+// K comes in stages of KST that go from memory straight into a ring of ST LDS buffers, ST - 1
+// of them in flight: no registers hold what is on its way, so WG = 2 to 3 workgroups share a
+// compute unit (staged through registers, the 128 x 128 tile took 230 of them).  One barrier
+// per stage: a wave waits for its own loads of stage k and for its reads of stage k - 1, then
+// the buffer of stage k - 1 is free for k + ST - 1.
+// A stage is rows of KST / 8 16-byte chunks without padding (the loads write LDS in lane
+// order), chunk c of row r in place c ^ turn(r): the sixteen lanes that a 16-byte LDS read
+// serves at once are rows {0-3, 12-15, 20-27} or {4-11, 16-19, 28-31} of 32, and with these
+// turns they meet all sixteen places of the 256 bytes the banks span (r & 7, the turn before,
+// had every second read conflict: 1.76 M conflict cycles at 25088 x 1024 x 256, now 0.15 M).
+// Rate at batch 128, us staged through registers / now: 56 x 56 x 64 -> 256 82 / 65, 28 x 28 x
+// 512 -> 1024 under stride 2 54 / 47, 14 x 14 x 1024 -> 256 28 / 25 (525 TFLOP/s); deeper rings
+// change nothing there, 13 TB/s of tile loads out of the L2s is what bounds them; the wide
+// results of the 56 x 56 layers run at copy rate.
+//
+// With PAIR the tile is act(affine(x w) + affine'(x' w')) of two products, a bottleneck's last
+// convolution and its projection: x' w' goes first, its affine result stays in registers as
+// the fp16 values that a projection of its own would have stored.
+template <int BM, int BN, int KST, int ST>
+constexpr int conv_lds_halves() {
+    const int ring = (BM + BN) * KST * ST, tile = BM * (BN + 8);
+    return ring > tile ? ring : tile;
 }
 
-template <int BM, int BN>
-__global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n, int tiles) {
-    constexpr int RX = BM * kChunks / kThreads, RW = BN * kChunks / kThreads;
+// This wave's loads but the last N have arrived and its LDS reads are done; then all waves'.
+template <int N>
+__device__ __forceinline__ void arrive() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+// 16 bytes per lane to LDS at `lds` + lane * 16.  (Written out because the compiler waits for
+// every such load in flight before any LDS read.)
+__device__ __forceinline__ void load_to_lds(uint32_t lds, const _Float16 *p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+
+template <int BM, int BN, int KST, int ST, int WG, bool PAIR>
+__global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, int tiles_n, int tiles) {
+    constexpr int CH = KST / 8, STAGE = (BM + BN) * KST;
+    constexpr int RX = BM * CH / kThreads, RW = BN * CH / kThreads;
     constexpr int TM = BM / 64, TN = BN / 64;      // 32-wide tiles per wave: pixels, channels
     constexpr int PITCH = BN + 8;
+    static_assert(ST >= 2 && ST <= 4 && (CH == 4 || CH == 8) && RX > 0 && RW > 0);
     extern __shared__ __align__(16) _Float16 net_smem[];
+    __shared__ float affine[PAIR ? 4 : 1][PAIR ? BN : 1];    // scale, shift; of the first product, too
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int block = xcd_block(blockIdx.x, tiles);
@@ -113,66 +139,62 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
     const int tm = block / tiles_n, tn = block - tm * tiles_n;
     const int64_t m0 = (int64_t)tm * BM;
     const int n0 = tn * BN;
-    const _Float16 *x = static_cast<const _Float16 *>(a.x), *w = static_cast<const _Float16 *>(a.w);
+    auto turn = [](int r) { return CH == 8 ? (r >> 1) & 7 : (r >> 2) & 3; };
 
     const _Float16 *xp[RX], *wp[RW];
-    int xs[RX], wsl[RW];                           // LDS positions
+    auto aim = [&](const NetConv &c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < RX; ++i) {
-        const int q = tid + i * kThreads, r = q / kChunks, ch = q % kChunks;
-        int64_t m = m0 + r < a.M ? m0 + r : a.M - 1;
-        if (a.stride > 1) {
-            const int64_t n = m / a.npix;
-            const int p = (int)(m - n * a.npix), y = p / a.Wo, xx = p - y * a.Wo;
-            m = (n * a.H + y * a.stride) * a.W + xx * a.stride;
+        for (int i = 0; i < RX; ++i) {
+            const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+            int64_t m = m0 + r < a.M ? m0 + r : a.M - 1;
+            if (c.stride > 1) {
+                const int64_t n = m / c.npix;
+                const int p = (int)(m - n * c.npix), y = p / c.Wo, xx = p - y * c.Wo;
+                m = (n * c.H + y * c.stride) * c.W + xx * c.stride;
+            }
+            xp[i] = static_cast<const _Float16 *>(c.x) + m * c.K + ch * 8;
         }
-        xp[i] = x + m * a.K + ch * 8;
-        xs[i] = r * kStep + (ch ^ (r & 7)) * 8;
-    }
 #pragma unroll
-    for (int i = 0; i < RW; ++i) {
-        const int q = tid + i * kThreads, r = q / kChunks, ch = q % kChunks;
-        wp[i] = w + (int64_t)min(n0 + r, a.N - 1) * a.K + ch * 8;
-        wsl[i] = BM * kStep + r * kStep + (ch ^ (r & 7)) * 8;
-    }
-    half8_t xr[RX], wr[RW];
-    auto load = [&](int k) {
-#pragma unroll
-        for (int i = 0; i < RX; ++i) xr[i] = *reinterpret_cast<const half8_t *>(xp[i] + k);
-#pragma unroll
-        for (int i = 0; i < RW; ++i) wr[i] = *reinterpret_cast<const half8_t *>(wp[i] + k);
+        for (int i = 0; i < RW; ++i) {
+            const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+            wp[i] = static_cast<const _Float16 *>(c.w) + (int64_t)min(n0 + r, a.N - 1) * c.K + ch * 8;
+        }
     };
-    auto park = [&](int buf) {
-        _Float16 *s = net_smem + buf * (BM + BN) * kStep;
+    const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) _Float16 *)net_smem;
+    auto load = [&](int buf) {
+        const uint32_t at = ring + (uint32_t)(buf * STAGE) * 2 + (uint32_t)wave * (kWave * 16);
 #pragma unroll
-        for (int i = 0; i < RX; ++i) *reinterpret_cast<half8_t *>(s + xs[i]) = xr[i];
+        for (int i = 0; i < RX; ++i, xp[i - 1] += KST) load_to_lds(at + i * kThreads * 16, xp[i]);
 #pragma unroll
-        for (int i = 0; i < RW; ++i) *reinterpret_cast<half8_t *>(s + wsl[i]) = wr[i];
+        for (int i = 0; i < RW; ++i, wp[i - 1] += KST) load_to_lds(at + BM * KST * 2 + i * kThreads * 16, wp[i]);
     };
     const int wm = wave & 1, wn = wave >> 1;
     const int l32 = lane & 31, hi = lane >> 5;
     float16_t acc[TM][TN];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    };
+    clear();
     auto multiply = [&](int buf) {
-        const _Float16 *s = net_smem + buf * (BM + BN) * kStep;
+        const _Float16 *s = net_smem + buf * STAGE;
 #pragma unroll
-        for (int kk = 0; kk < kStep / 16; ++kk) {
+        for (int kk = 0; kk < KST / 16; ++kk) {
             const int ch = kk * 2 + hi;
             half8_t xv[TM], wv[TN];
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 const int r = wm * (BM / 2) + i * 32 + l32;
-                xv[i] = *reinterpret_cast<const half8_t *>(s + r * kStep + (ch ^ (r & 7)) * 8);
+                xv[i] = *reinterpret_cast<const half8_t *>(s + r * KST + (ch ^ turn(r)) * 8);
             }
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int r = wn * (BN / 2) + j * 32 + l32;
-                wv[j] = *reinterpret_cast<const half8_t *>(s + BM * kStep + r * kStep + (ch ^ (r & 7)) * 8);
+                wv[j] = *reinterpret_cast<const half8_t *>(s + BM * KST + r * KST + (ch ^ turn(r)) * 8);
             }
 #pragma unroll
             for (int i = 0; i < TM; ++i)
@@ -181,10 +203,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[j], xv[i], acc[i][j], 0, 0, 0);
         }
     };
-    const int nk = a.K / kStep;
     // what the tile's results meet on their way out: this thread's eight channels, and the
-    // residual of its pixels (requested before the last step, so with everything else where
-    // K is a single step)
+    // residual of its pixels (requested before the last stage is multiplied)
     constexpr int CPR = BN / 8;                     // vectors per pixel
     constexpr int RO = BM * CPR / kThreads;
     const int cq = tid % CPR, c = n0 + cq * 8;
@@ -201,21 +221,77 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
             if (res) rv[i] = *reinterpret_cast<const half8_t *>(res + (m < a.M ? m : a.M - 1) * a.N + (cok ? c : 0));
         }
     };
-    load(0);
-    if (nk == 1) residual();
-    park(0);
-    if (nk > 1) load(kStep);
-    __syncthreads();
-    for (int k = 0; k < nk; ++k) {
-        if (nk > 1 && k == nk - 1) residual();
-        multiply(k & 1);
-        if (k + 1 < nk) park((k + 1) & 1);
-        if (k + 2 < nk) load((k + 2) * kStep);
-        __syncthreads();
-    }
+    // Lane column of a 32x32 step's D = pixel l32, rows (channels) 8 * g + 4 * hi + 0..3 in
+    // registers 4g .. 4g+3.
+    auto channel = [&](int j, int g) { return wn * (BN / 2) + j * 32 + 8 * g + 4 * hi; };
+    half4_t side[PAIR ? TM : 1][PAIR ? TN : 1][PAIR ? 4 : 1];
+    auto affine_of = [&](int which, int i, int j, int g, float (&f)[4]) __attribute__((always_inline)) {
+        const float4_t sc = *reinterpret_cast<const float4_t *>(&affine[which][channel(j, g)]);
+        const float4_t sh = *reinterpret_cast<const float4_t *>(&affine[which + 1][channel(j, g)]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = fmaf((float)(_Float16)acc[i][j][4 * g + e], sc[e], sh[e]);
+    };
 
-    // The tile, rounded to fp16, through LDS: [pixel][channel].  D of a 32x32 step: lane
-    // column = pixel l32, rows (channels) 8 * g + 4 * hi + 0..3 in registers 4g .. 4g+3.
+    const int nk0 = PAIR ? first.K / KST : 0, nk = nk0 + a.K / KST;
+    Affine<1> of[2];
+    if constexpr (PAIR) {
+        if (tid < BN) {
+            of[0].request(a.norm, min(n0 + tid, a.N - 1));
+            of[1].request(first.norm, min(n0 + tid, a.N - 1));
+        }
+        aim(first);
+    } else {
+        aim(a);
+    }
+    auto load_stage = [&](int k, int buf) __attribute__((always_inline)) {
+        if (PAIR && k == nk0) aim(a);
+        load(buf);
+    };
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+        if (s < nk) load_stage(s, s);
+    if constexpr (PAIR) {
+        if (tid < BN) {
+            float sc[1], sh[1];
+            of[0].finish(a.norm, sc, sh);
+            affine[0][tid] = sc[0];
+            affine[1][tid] = sh[0];
+            of[1].finish(first.norm, sc, sh);
+            affine[2][tid] = sc[0];
+            affine[3][tid] = sh[0];
+        }
+    }
+    int buf = 0;
+    for (int k = 0; k < nk; ++k) {
+        // (stages up to k + ST - 2 have been asked for, the last one is nk - 1)
+        if (k + ST - 1 <= nk) arrive<(ST - 2) * (RX + RW)>();
+        else if (ST == 4 && k + 2 == nk) arrive<RX + RW>();
+        else arrive<0>();
+        if (k + ST - 1 < nk) load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+        if (!PAIR && k == nk - 1) residual();
+        multiply(buf);
+        buf = buf == ST - 1 ? 0 : buf + 1;
+        if constexpr (PAIR) {
+            if (k == nk0 - 1) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            float f[4];
+                            affine_of(2, i, j, g, f);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) side[i][j][g][e] = (_Float16)f[e];
+                        }
+                clear();
+            }
+        }
+    }
+    __syncthreads();
+
+    // The tile through LDS as [pixel][channel]: a single product's sums rounded to fp16, a
+    // pair's results.
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -223,14 +299,24 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 half4_t v;
+                if constexpr (PAIR) {
+                    float f[4];
+                    affine_of(0, i, j, g, f);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = (_Float16)acc[i][j][4 * g + e];
-                const int px = wm * (BM / 2) + i * 32 + l32, ch = wn * (BN / 2) + j * 32 + 8 * g + 4 * hi;
-                *reinterpret_cast<half4_t *>(net_smem + px * PITCH + ch) = v;
+                    for (int e = 0; e < 4; ++e) {
+                        f[e] += (float)side[i][j][g][e];
+                        v[e] = (_Float16)(a.relu ? relu(f[e]) : f[e]);
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = (_Float16)acc[i][j][4 * g + e];
+                }
+                const int px = wm * (BM / 2) + i * 32 + l32;
+                *reinterpret_cast<half4_t *>(net_smem + px * PITCH + channel(j, g)) = v;
             }
     __syncthreads();
     float sc[8], sh[8];
-    aff.finish(a.norm, sc, sh);
+    if constexpr (!PAIR) aff.finish(a.norm, sc, sh);
     _Float16 *out = static_cast<_Float16 *>(a.out);
     if (!cok) return;
 #pragma unroll
@@ -238,13 +324,14 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_conv(NetConv a, int tiles_n
         const int r = tid / CPR + i * (kThreads / CPR);
         const int64_t m = m0 + r;
         if (m >= a.M) break;
-        const half8_t v = *reinterpret_cast<const half8_t *>(net_smem + r * PITCH + cq * 8);
-        half8_t o;
+        half8_t o = *reinterpret_cast<const half8_t *>(net_smem + r * PITCH + cq * 8);
+        if constexpr (!PAIR) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            float f = fmaf((float)v[e], sc[e], sh[e]) + (float)rv[i][e];
-            if (a.relu) f = relu(f);
-            o[e] = (_Float16)f;
+            for (int e = 0; e < 8; ++e) {
+                float f = fmaf((float)o[e], sc[e], sh[e]) + (float)rv[i][e];
+                if (a.relu) f = relu(f);
+                o[e] = (_Float16)f;
+            }
         }
         *reinterpret_cast<half8_t *>(out + m * a.N + c) = o;
     }
@@ -797,40 +884,71 @@ __global__ __launch_bounds__(kThreads) void k_net_pool(const _Float16 *__restric
     out[(int64_t)n * C + cc] = (_Float16)(s / (float)plane);
 }
 
-template <int BM, int BN>
-hipError_t launch_conv(const NetConv &a, hipStream_t st) {
+template <int BM, int BN, int KST, int ST, int WG>
+hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     const int tiles_n = (int)cdiv(a.N, BN);
     const int64_t tiles = cdiv(a.M, BM) * tiles_n;
     if (tiles > (1 << 30)) return hipErrorInvalidConfiguration;
-    const int lds = conv_lds_halves<BM, BN>(a.K > kStep) * (int)sizeof(_Float16);
-    hipLaunchKernelGGL((k_net_conv<BM, BN>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a, tiles_n, (int)tiles);
+    const int lds = conv_lds_halves<BM, BN, KST, ST>() * (int)sizeof(_Float16);
+    constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) < 64 * 1024;
+    if (first && !kPair) return hipErrorNotSupported;
+    if (first)
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+                           *first, tiles_n, (int)tiles);
+    else
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+                           a, tiles_n, (int)tiles);
     return hipGetLastError();
+}
+
+// Rows of whole vectors, and not so few tiles of a long K that splitting K is faster (64 tiles
+// at K = 512: 5.2 us in tiles, 5.0 split; 16 at K = 1024: 7.2 and 6.7; 32 at K = 2048: 11.5 and 9.7).
+bool conv_in_tiles(const NetConv &a) {
+    return a.N % 8 == 0 && !(a.K >= 512 && cdiv(a.M, 64) * cdiv(a.N, 64) <= 64);
+}
+
+// The largest tiles that leave somewhat more than a workgroup per compute unit.  Where a unit
+// goes through several, short stages leave room for one workgroup more; where it has one or
+// two, long stages cost fewer barriers (batch 128, us long / short stages: 3136 tiles of
+// 56 x 56 x 64 -> 256 76 / 65, 1568 of 28 x 28 x 512 -> 256 54 / 50, 784 of 14 x 14 x 1024 -> 512
+// 43 / 46, 392 of 14 x 14 x 1024 -> 256 25 / 30).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
+// 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
+hipError_t conv_tiles(const NetConv &a, const NetConv *first, hipStream_t st) {
+    auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
+    constexpr int kMany = 1024, kFew = 320;
+    if (a.N >= 128 && count(128, 128) >= (first ? kFew : kMany)) return launch_conv<128, 128, 32, 3, 3>(a, first, st);
+    if (a.N >= 128 && count(128, 128) >= kFew) return launch_conv<128, 128, 64, 2, 2>(a, nullptr, st);
+    if (count(128, 64) >= kMany) return launch_conv<128, 64, 32, 3, 4>(a, first, st);
+    if (count(128, 64) >= 448) return launch_conv<128, 64, 64, 2, 3>(a, first, st);
+    return launch_conv<64, 64, 64, 3, 3>(a, first, st);
 }
 
 }  // namespace
 
-bool net_conv_supported(const NetConv &a) { return a.K % kStep == 0 && a.K > 0 && a.N > 0; }
+bool net_conv_supported(const NetConv &a) { return a.K % 64 == 0 && a.K > 0 && a.N > 0; }
 
 hipError_t net_conv(const NetConv &a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_conv_supported(a)) return hipErrorNotSupported;
-    // The largest tiles that leave somewhat more than a workgroup per compute unit (measured
-    // over batches of 1 to 128 of the network's twelve products: 128 x 128 from 392 tiles on,
-    // 64 x 64 below); the splitting kernel where even tiles of 64 are few and K is long enough
-    // to split (56 x 64 -> 256 at batch 1: 4.9 us in tiles of 64, 15 split; 14 x 14 x 1024 -> 256:
-    // 9.0 and 7.1), and for odd channel counts.
-    auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
-    constexpr int kEnough = 320;
-    if (a.N % 8 == 0 && !(a.K >= 512 && count(64, 64) <= 64)) {
-        if (a.N >= 128 && count(128, 128) >= kEnough) return launch_conv<128, 128>(a, st);
-        if (count(128, 64) >= kEnough) return launch_conv<128, 64>(a, st);
-        return launch_conv<64, 64>(a, st);
-    }
+    if (conv_in_tiles(a)) return conv_tiles(a, nullptr, st);
     const int tiles_n = (int)cdiv(a.N, 32);
     const int64_t blocks = cdiv(a.M, 32) * tiles_n;
     if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_net_conv_split, dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
     return hipGetLastError();
+}
+
+// One launch where both products are made in tiles; else the projection's results wait in
+// `out`.
+hipError_t net_conv_pair(const NetConv &a, const NetConv &first, hipStream_t st) {
+    if (a.M == 0) return hipSuccess;
+    if (!net_conv_supported(a) || !net_conv_supported(first)) return hipErrorNotSupported;
+    if (conv_in_tiles(a) && conv_in_tiles(first)) return conv_tiles(a, &first, st);
+    hipError_t err = net_conv(first, st);
+    if (err != hipSuccess) return err;
+    NetConv last = a;
+    last.res = a.out;
+    return net_conv(last, st);
 }
 
 hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,

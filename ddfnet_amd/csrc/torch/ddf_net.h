@@ -130,16 +130,17 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
                 DDF_F16, st));
             nm = b.bn2.norm();
             check_status(ddf_hip_net_filter(t1, cf, sf, &nm, t2, n, h, w, width, b.stride, b.combine, st));
-            const void *res = cur;
-            if (b.down.t[0].defined()) {
-                nm = b.down.norm();
-                check_status(ddf_hip_net_conv(cur, b.down.t[0].data_ptr(), &nm, nullptr, other, n, h, w, c, wide_c,
-                                              b.stride, 0, st));
-                std::swap(cur, other);
-                res = cur;
-            }
             nm = b.conv3.norm();
-            check_status(ddf_hip_net_conv(t2, b.conv3.t[0].data_ptr(), &nm, res, cur, n, ho, wo, width, wide_c, 1, 1, st));
+            if (b.down.t[0].defined()) {
+                const ddf_net_norm_t down = b.down.norm();
+                check_status(ddf_hip_net_conv_pair(t2, b.conv3.t[0].data_ptr(), &nm, width, cur,
+                                                   b.down.t[0].data_ptr(), &down, h, w, c, b.stride, other, n, wide_c, 1,
+                                                   st));
+                std::swap(cur, other);
+            } else {
+                check_status(ddf_hip_net_conv(t2, b.conv3.t[0].data_ptr(), &nm, cur, cur, n, ho, wo, width, wide_c, 1, 1,
+                                              st));
+            }
             h = ho; w = wo; c = wide_c;
         }
         check_status(ddf_hip_net_pool(cur, other, n, h * w, c, st));

@@ -356,6 +356,9 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *   conv    out (N, Ho, Wo, O) = act(norm(1x1 convolution of stride `stride`, weight (O, C)) +
  *           residual), residual NULL or shaped like out (which may be the same memory);
  *           C a multiple of 64
+ *   conv_pair out = act(norm(1x1 convolution of features (N, Ho, Wo, C)) + norm'(1x1 convolution of
+ *           stride `stride` of side_features (N, H, W, side_C))): a bottleneck's last convolution
+ *           and its projection; out overlaps neither input; C and side_C multiples of 64
  *   stem    max_pool(relu(norm(7x7 convolution, stride 2, padding 3, weight (64, 3, 7, 7))), 3x3,
  *           stride 2, padding 1) of a planar (N, 3, H, W) image; H and W multiples of 4
  *   spatial the spatial filter branch (3x3 taps, one head): spatial_filter (N, Ho*Wo, 12), nine
@@ -371,6 +374,10 @@ typedef struct {
 int ddf_hip_net_conv(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
                      void *output, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int stride, int relu,
                      void *stream);
+int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_net_norm_t *norm, int64_t C,
+                          const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
+                          int64_t H, int64_t W, int64_t side_C, int stride, void *output, int64_t N, int64_t O,
+                          int relu, void *stream);
 int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,
                      int64_t H, int64_t W, void *stream);
 int ddf_hip_net_spatial(const void *features, const void *weight, const void *bias, void *spatial_filter,

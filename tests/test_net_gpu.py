@@ -57,6 +57,9 @@ def close(got, want, tol):
     (8, 28, 28, 192, 136, 1, 0, 1, 0, 1),      # three steps of K
     (5, 28, 30, 256, 512, 2, 1, 0, 0, 0),      # projection under stride 2
     (40, 56, 56, 256, 512, 2, 1, 0, 0, 0),
+    (16, 28, 28, 128, 264, 1, 1, 0, 1, 1),     # tiles of 128 x 64, channels past the last
+    (42, 56, 56, 64, 136, 1, 1, 1, 0, 1),      # tiles of 128 x 128 in short stages
+    (3, 7, 7, 2112, 520, 1, 1, 0, 1, 1),       # tiles of 64, 33 stages of K
 ])
 def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     torch.manual_seed(c + o)
@@ -70,6 +73,32 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     want = want.clamp_min(0) if relu else want
     out = r if res else torch.empty(n, ho, wo, o, device='cuda', dtype=torch.float16)   # (in place where it may be)
     call('ddf_hip_net_conv', x, wt, norm, r, out, n, h, w, c, o, stride, relu)
+    close(out, want, 3e-3)
+
+
+@pytest.mark.parametrize('n,h,w,c,side,o,stride,relu', [
+    (3, 5, 7, 64, 64, 64, 1, 1),               # a stage of K each, one tile
+    (5, 9, 13, 64, 192, 136, 2, 0),            # rows and channels past a tile
+    (1, 14, 14, 512, 1024, 2048, 2, 1),        # few pixels, long rows: two launches
+    (8, 28, 28, 256, 512, 1024, 2, 1),         # tiles of 64
+    (16, 28, 28, 128, 256, 264, 1, 1),         # 128 x 64
+    (42, 56, 56, 64, 64, 136, 1, 1),           # 128 x 128, many
+    (27, 56, 56, 128, 256, 512, 2, 1),         # 128 x 128, few
+    (42, 56, 56, 128, 64, 64, 1, 1),           # 64 channels, many
+])
+def test_conv_pair(n, h, w, c, side, o, stride, relu):
+    torch.manual_seed(c + o)
+    ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
+    xs = torch.randn(n, h, w, side, device='cuda').half()
+    x = torch.randn(n, ho, wo, c, device='cuda').half()
+    wt, ws = ((torch.randn(o, k, device='cuda') * k ** -0.5).half() for k in (c, side))
+    norm, apply, keep = make_norm(o, 1, 1)
+    norm_s, apply_s, keep_s = make_norm(o, 1, 0)
+    want = apply(x.reshape(-1, c).float() @ wt.float().t()) + \
+        apply_s(xs[:, ::stride, ::stride].reshape(-1, side).float() @ ws.float().t())
+    want = (want.clamp_min(0) if relu else want).reshape(n, ho, wo, o)
+    out = torch.empty(n, ho, wo, o, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_conv_pair', x, wt, norm, c, xs, ws, norm_s, h, w, side, stride, out, n, o, relu)
     close(out, want, 3e-3)
 
 
