@@ -645,6 +645,20 @@ __device__ __forceinline__ float row_sum(float v) {
     return add_permuted<0x140>(v);   // row_mirror
 }
 
+// A value as it lies in memory, in a register of its own (halves that share one load one after
+// the other); zero past the buffer's end.
+template <typename T>
+__device__ __forceinline__ uint32_t ld_bits(__amdgpu_buffer_rsrc_t r, uint32_t index) {
+    const int at = (int)(index * (uint32_t)sizeof(T));
+    if constexpr (sizeof(T) == 2) return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0);
+    else return __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0);
+}
+template <typename T>
+__device__ __forceinline__ float of_bits(uint32_t bits) {
+    if constexpr (sizeof(T) == 2) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
+    else return __builtin_bit_cast(float, bits);
+}
+
 constexpr int kChannelThreads = 1024;  // sixteen waves: the rows of a block's taps are dealt out to them
 constexpr int kChannelWaves = kChannelThreads / kWave;
 
@@ -656,7 +670,7 @@ constexpr int kChannelWaves = kChannelThreads / kWave;
 // workgroup of a sample recomputes the hidden vector, so the blocks are large:
 // smaller ones had all compute units read the same rows of w1 at once, which
 // the L2 serves one after the other.
-template <typename T, int KK, int BLOCK, int NS>
+template <typename T, int KK, int BLOCK, int NS, int AHEAD = 0>
 __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const T *__restrict__ pooled, const T *__restrict__ w1, const T *__restrict__ b1,
     const T *__restrict__ w2, const T *__restrict__ b2, T *__restrict__ cf, int N, int C, int mid,
@@ -670,6 +684,55 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const int64_t n0 = (int64_t)blockIdx.y * NS;
     const int ns = min(NS, N - (int)n0);   // samples of this workgroup (the others: copies of the last)
     const int cb = blockIdx.x * BLOCK;
+    // One sample per workgroup: few workgroups, and their time is the round trips to memory.
+    // What does not depend on the pooled vector is requested along with it: the first 64 * AHEAD
+    // values of the wave's first rows of w1, 16 * AHEAD values of all its rows of w2, the biases,
+    // the gains and offsets; without branches, which would end in a wait each (absent values lie
+    // outside their buffers).  Six round trips, one after the other, become one: 8 samples of 64
+    // channels fp16 6.9 -> 4.9 us, one of 128 9.3 -> 6.3, 128 of 128 9.9 -> 7.0, 32 of 256 fp32
+    // 11.0 -> 9.2 (loads of halves into shared registers, or under branches: 10 to 13 us).
+    constexpr bool kAhead = AHEAD > 0;
+    static_assert(!kAhead || (NS == 1 && KK == 9 && BLOCK == 64));
+    constexpr int RT = NS >= 4 ? 1 : NS == 2 ? 2 : 3;
+    constexpr int GROUPS = kAhead ? BLOCK * KK / (kChannelWaves * 4) : 1, A1 = kAhead ? 4 * AHEAD : 1, A2 = kAhead ? AHEAD : 1;
+    const int seg = lane >> 4, sl = lane & 15;
+    const int rows = min(BLOCK, C - cb) * KK;
+    uint32_t w1a[A1], w2a[GROUPS][A2], b1a = 0, b2a[GROUPS], ga[KK] = {}, oa[KK] = {};
+    float part[kMaxParts];
+    TapParams<T, KK> params;
+    const bool parts_ahead = kAhead && parts && nparts <= kMaxParts;
+    if constexpr (kAhead) {
+        constexpr uint32_t kNone = kOutside / sizeof(T);
+        auto buffer = [](const T *p, int count) { return plane_rsrc(p, p ? (uint32_t)count * (uint32_t)sizeof(T) : 0u); };
+        const int tid = threadIdx.x;
+        const __amdgpu_buffer_rsrc_t pr = plane_rsrc(parts + (parts ? n0 * nparts * C : 0), parts_ahead ? (uint32_t)(nparts * C) * 4u : 0u);
+#pragma unroll
+        for (int q = 0; q < kMaxParts; ++q)
+            part[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr, tid < C ? (q * C + tid) * 4 : (int)kOutside, 0, 0));
+        const __amdgpu_buffer_rsrc_t w1r = buffer(w1, mid * C), b1r = buffer(b1, mid);
+        const int m = wave * 4 + seg;
+#pragma unroll
+        for (int i = 0; i < A1; ++i) w1a[i] = ld_bits<T>(w1r, m < mid && sl + i * 16 < C ? (uint32_t)(m * C + sl + i * 16) : kNone);
+        b1a = ld_bits<T>(b1r, (uint32_t)m);
+        const __amdgpu_buffer_rsrc_t w2r = buffer(w2, C * KK * mid), b2r = buffer(b2, C * KK);
+#pragma unroll
+        for (int t = 0; t < GROUPS; ++t) {
+            const int r = (t * kChannelWaves + wave) * 4 + seg;
+#pragma unroll
+            for (int i = 0; i < A2; ++i)
+                w2a[t][i] = ld_bits<T>(w2r, r < rows && sl + i * 16 < mid ? (uint32_t)((cb * KK + r) * mid + sl + i * 16) : kNone);
+            b2a[t] = ld_bits<T>(b2r, r < rows ? (uint32_t)(cb * KK + r) : kNone);
+        }
+        const __amdgpu_buffer_rsrc_t gr = buffer(gain_vec, C * KK), orr = buffer(offset_vec, C * KK);
+        if (tid < BLOCK) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) {
+                ga[t] = ld_bits<T>(gr, (uint32_t)((cb + tid) * KK + t));
+                oa[t] = ld_bits<T>(orr, (uint32_t)((cb + tid) * KK + t));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     // the pooled vectors: given, or scale * the sum of nparts partial sums per value
     // (parts[(n * nparts + p) * C + c], what k_spatial_stream leaves)
     for (int i = threadIdx.x; i < NS * C; i += kChannelThreads) {
@@ -677,8 +740,13 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         const int64_t n = n0 + min(s, ns - 1);
         if (parts) {
             float a = 0.f;
+            if (parts_ahead && i == (int)threadIdx.x) {
+#pragma unroll
+                for (int q = 0; q < kMaxParts; ++q) a += part[q];
+            } else {
 #pragma unroll 8
-            for (int q = 0; q < nparts; ++q) a += parts[(n * nparts + q) * C + c];
+                for (int q = 0; q < nparts; ++q) a += parts[(n * nparts + q) * C + c];
+            }
             v[i] = a * scale;
         } else {
             v[i] = ld(pooled + n * C + c);
@@ -689,7 +757,6 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     // Dot products with sixteen lanes along a weight row and four rows per wave at a
     // time: each ends in a reduction over a row of 16 lanes (four lane-permute
     // additions for four results; a whole wave per row paid thirteen for one).
-    const int seg = lane >> 4, sl = lane & 15;
     // hidden vectors: rows of w1
     for (int m0 = wave * 4; m0 < mid; m0 += kChannelWaves * 4) {
         const int m = min(m0 + seg, mid - 1);
@@ -697,13 +764,20 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         float p[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) p[s] = 0.f;
+        int c = sl;
+        const bool ahead = kAhead && m0 == wave * 4;
+        if (ahead) {
+#pragma unroll
+            for (int i = 0; i < A1; ++i, c += 16)
+                if (c < C) p[0] = fmaf(of_bits<T>(w1a[i]), v[c], p[0]);
+        }
 #pragma unroll 8
-        for (int c = sl; c < C; c += 16) {
+        for (; c < C; c += 16) {
             const float wv = ld(row + c);
 #pragma unroll
             for (int s = 0; s < NS; ++s) p[s] = fmaf(wv, v[s * C + c], p[s]);
         }
-        const float bias = b1 ? ld(b1 + m) : 0.f;
+        const float bias = ahead ? of_bits<T>(b1a) : b1 ? ld(b1 + m) : 0.f;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const float tot = row_sum(p[s]);
@@ -716,9 +790,26 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     }
     __syncthreads();
     // the block's taps: rows (cb * KK + r) of w2, RT passes of four rows in flight per wave
-    constexpr int RT = NS >= 4 ? 1 : NS == 2 ? 2 : 3;
-    const int rows = min(BLOCK, C - cb) * KK;
-    for (int r0 = wave * 4 * RT; r0 < rows; r0 += kChannelWaves * 4 * RT) {
+    auto emit = [&](int r, int s, float p, float bias) __attribute__((always_inline)) {
+        const float tot = row_sum(p);
+        if (sl == 0 && r < rows) {
+            f[s * BLOCK * KK + r] = tot + bias;
+            if (save.taps && s < ns) save.taps[((n0 + s) * C + cb) * KK + r] = tot + bias;
+        }
+    };
+    if constexpr (kAhead) {
+#pragma unroll
+        for (int t = 0; t < GROUPS; ++t) {
+            const int r = (t * kChannelWaves + wave) * 4 + seg;
+            float p = 0.f;
+            int m = sl;
+#pragma unroll
+            for (int i = 0; i < A2; ++i, m += 16)
+                if (m < mid) p = fmaf(of_bits<T>(w2a[t][i]), h[m], p);
+            for (; m < mid; m += 16) p = fmaf(ld(w2 + ((int64_t)cb * KK + min(r, rows - 1)) * mid + m), h[m], p);
+            emit(r, 0, p, of_bits<T>(b2a[t]));
+        }
+    } else for (int r0 = wave * 4 * RT; r0 < rows; r0 += kChannelWaves * 4 * RT) {
         float p[RT][NS];
         const T *wrow[RT];
 #pragma unroll
@@ -744,13 +835,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
             const int r = r0 + 4 * u + seg;
             const float bias = (b2 && r < rows) ? ld(b2 + (int64_t)cb * KK + r) : 0.f;
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                const float tot = row_sum(p[u][s]);
-                if (sl == 0 && r < rows) {
-                    f[s * BLOCK * KK + r] = tot + bias;
-                    if (save.taps && s < ns) save.taps[((n0 + s) * C + cb) * KK + r] = tot + bias;
-                }
-            }
+            for (int s = 0; s < NS; ++s) emit(r, s, p[u][s], bias);
         }
     }
     __syncthreads();
@@ -761,8 +846,15 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         float u[KK];
 #pragma unroll
         for (int t = 0; t < KK; ++t) u[t] = f[(s * BLOCK + ch) * KK + t];
-        TapParams<T, KK> params;
-        params.load(cb + ch, gain, gain_vec, offset_vec, (const T *)nullptr);   // (b2 is in f already)
+        if constexpr (kAhead) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) {
+                params.gain[t] = gain_vec ? of_bits<T>(ga[t]) : gain;
+                params.offset[t] = of_bits<T>(oa[t]);
+                params.bias[t] = 0.f;
+            }
+        } else
+            params.load(cb + ch, gain, gain_vec, offset_vec, (const T *)nullptr);   // (b2 is in f already)
         normalise<T, KK>(u, params);
         T *op = cf + ((n0 + s) * C + cb + ch) * KK;
 #pragma unroll
@@ -838,10 +930,11 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
     // item (given, or scale * the sum of nparts partial sums per value), and zeros in
     // the last tile of the hidden layer (its overlap with the tile before stays zero).
     auto pooled_vectors = [&]() {
-        const int c4s = C >> 2;
-        for (int i = threadIdx.x; i < kMmaSamples * c4s; i += WAVES * kWave) {
+        // (Only samples there are: a column of the products that belongs to none is read by nothing.)
+        const int c4s = C >> 2, items = min(kMmaSamples, N - n0) * c4s;
+        for (int i = threadIdx.x; i < items; i += WAVES * kWave) {
             const int s = i / c4s, c4 = i - s * c4s;
-            const int64_t n = min(n0 + s, N - 1);
+            const int64_t n = n0 + s;
             half4_t v;
             if (parts) {
                 const float4_t *src = reinterpret_cast<const float4_t *>(parts + n * nparts * C) + c4;
@@ -862,7 +955,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
                 v = load_half4(pooled + n * C + c4 * 4);
             }
             *reinterpret_cast<half4_t *>(pv + ((c4 >> 3) * kMmaSamples + s) * kMmaStep + (c4 & 7) * 4) = v;
-            if (save.pooled && blockIdx.x == 0 && n0 + s < N) {
+            if (save.pooled && blockIdx.x == 0) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) save.pooled[n * C + c4 * 4 + e] = (float)v[e];
             }
@@ -1307,11 +1400,21 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
         else if (ns == 2) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 2);                                    \
         else DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 1);                                                 \
     } while (0)
-    if (k == 3 && block == 64) DDF_CHANNEL_CASE(9, 64);
+#define DDF_CHANNEL_AHEAD(A_)                                                                          \
+    hipLaunchKernelGGL((k_channel_branch<T, 9, 64, 1, A_>), grid, dim3(kChannelThreads), lds, st,     \
+                       pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain, gain_vec,   \
+                       offset_vec, parts, nparts, (float)scale, save)
+    if (k == 3 && block == 64 && ns == 1) {   // (requests for what a layer of this size has)
+        if (C <= 64 && mid <= 16) DDF_CHANNEL_AHEAD(1);
+        else if (C <= 128 && mid <= 32) DDF_CHANNEL_AHEAD(2);
+        else DDF_CHANNEL_AHEAD(4);
+    } else if (k == 3 && block == 64 && ns == 2) DDF_CHANNEL_LAUNCH(9, 64, 2);
+    else if (k == 3 && block == 64) DDF_CHANNEL_LAUNCH(9, 64, 4);
     else if (k == 3) DDF_CHANNEL_CASE(9, 128);
     else if (k == 5 && block == 64) DDF_CHANNEL_CASE(25, 64);
     else if (k == 5) DDF_CHANNEL_CASE(25, 128);
     else return hipErrorNotSupported;
+#undef DDF_CHANNEL_AHEAD
 #undef DDF_CHANNEL_LAUNCH
 #undef DDF_CHANNEL_CASE
     return hipGetLastError();

@@ -217,3 +217,20 @@ def test_channel_branch_parts_matches_fp64(n, c, k, tiles, dtype, tol):
     ref = channel_reference(pooled, *(t.cpu() for t in (w1, b1, w2, b2)), k, 1.0, gv.cpu(), ov.cpu())
     err = ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item()
     assert err < tol, err
+
+
+@pytest.mark.parametrize('dtype,tol', [(torch.float32, 2e-5), (torch.float16, 6e-3)])
+@pytest.mark.parametrize('n,c,mid,tiles', [(1, 64, 16, 1), (3, 64, 17, 8), (2, 65, 16, 9), (3, 128, 31, 8), (2, 129, 32, 3),
+                                           (2, 257, 20, 2), (3, 300, 65, 8), (1, 511, 3, 9), (2, 1, 1, 1)])
+def test_channel_branch_one_sample_per_workgroup(n, c, mid, tiles, dtype, tol):
+    """Few samples: weights requested ahead, to the edges of what is and past them."""
+    torch.manual_seed(c + mid)
+    k = 3
+    parts = torch.randn(n, tiles, c, device='cuda')
+    w1 = (torch.randn(mid, c, device='cuda') * c ** -0.5).to(dtype)
+    w2 = (torch.randn(c * k * k, mid, device='cuda') * mid ** -0.5).to(dtype)
+    b1, b2 = torch.randn(mid, device='cuda').to(dtype), torch.randn(c * k * k, device='cuda').to(dtype)
+    out = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, None, None)
+    ref = channel_reference(parts.double().sum(1).cpu(), *(t.cpu() for t in (w1, b1, w2, b2)), k, 0.7, None, None)
+    err = ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item()
+    assert err < tol, err
