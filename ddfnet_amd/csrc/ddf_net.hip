@@ -99,8 +99,9 @@ struct Affine {
 // turns they meet all sixteen places of the 256 bytes the banks span (r & 7, the turn before,
 // had every second read conflict: 1.76 M conflict cycles at 25088 x 1024 x 256, now 0.15 M).
 // Rate at batch 128, us staged through registers / now: 56 x 56 x 64 -> 256 82 / 65, 28 x 28 x
-// 512 -> 1024 under stride 2 54 / 47, 14 x 14 x 1024 -> 256 28 / 25 (525 TFLOP/s); deeper rings
-// change nothing there, 13 TB/s of tile loads out of the L2s is what bounds them; the wide
+// 512 -> 1024 under stride 2 54 / 47, 14 x 14 x 1024 -> 256 28 / 25 (525 TFLOP/s); deeper rings,
+// larger tiles and a K order turned per tile change nothing there; the matrix cores are busy a
+// third of the time, and 98 tiles for an XCD's 96 places cost 125 -> 128 images 10 %.  The wide
 // results of the 56 x 56 layers run at copy rate.
 //
 // With PAIR the tile is act(affine(x w) + affine'(x' w')) of two products, a bottleneck's last
@@ -337,21 +338,23 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     }
 }
 
-// Few pixels, where tiles of 64 leave most of the chip idle: a workgroup takes 32 pixels x 32
-// channels, its four waves a quarter of K each, operands straight from memory (every value
-// is used by one wave only); the waves' sums meet in LDS.  K goes by in blocks of 64 of which
-// a lane takes one half, 64 contiguous bytes in four loads (the order of the summed
-// dimension is free as long as both operands agree): the 32 rows a load touches are 128-byte
-// lines that are used up at once instead of being fetched again by later steps.
+// Few pixels, where tiles of 64 leave most of the chip idle: a workgroup takes 16 pixels x 16
+// channels, its four waves a quarter of K each, operands straight from memory (every value is
+// used by one wave only); the waves' sums meet in LDS.  K goes by in blocks of 64 of which a lane
+// takes a quarter, 32 contiguous bytes in two loads (the order of the summed dimension is free
+// as long as both operands agree), four blocks of a wave in flight.  What the launch takes is what
+// one compute unit's operands take on their way in, so smaller tiles are faster than larger ones
+// and than more waves (us for 32 x 32, the same with sixteen waves, 16 x 16: 49 x 2048 -> 512 9.7,
+// 9.7, 7.2; 196 x 1024 -> 256 6.7, 9.9, 5.7; 1 x 2048 -> 1000 7.1, 7.1, 5.2).
 __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tiles_n) {
-    constexpr int WAVES = kThreads / kWave, U = 4, P = 33;
-    __shared__ float red[WAVES][32][P];
+    constexpr int WAVES = kThreads / kWave, D = 4, T = 16;
+    __shared__ float red[WAVES][T][T + 1];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
-    const int l32 = lane & 31, hi = lane >> 5;
-    const int n0 = tn * 32;
-    int64_t m = (int64_t)tm * 32 + l32;
+    const int col = lane & 15, quad = lane >> 4;
+    const int n0 = tn * T;
+    int64_t m = (int64_t)tm * T + col;
     if (m >= a.M) m = a.M - 1;
     if (a.stride > 1) {
         const int64_t n = m / a.npix;
@@ -360,74 +363,50 @@ __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tile
     }
     const int blocks = a.K / 64, per = (blocks + WAVES - 1) / WAVES;
     const int b0 = wave * per, b1 = min(b0 + per, blocks);
-    const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + hi * 32;
-    const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + l32, a.N - 1) * a.K + hi * 32;
-    // (a thread finishes one channel of four pixels: 64-byte runs of a pixel's channels)
-    constexpr int PX = 2 * WAVES, RO = 32 / PX;
-    const int oc = n0 + (tid & 31);
-    const bool cok = oc < a.N;
-    const _Float16 *res = static_cast<const _Float16 *>(a.res);
-    Affine<1> aff;
-    _Float16 rv[RO];
-    float16_t acc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    half8_t xv[2][U], wv[2][U];
-    auto request = [&](auto set, int b) __attribute__((always_inline)) {
-        constexpr int B = decltype(set)::value;
+    const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + quad * 16;
+    const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + col, a.N - 1) * a.K + quad * 16;
+    half8_t xv[D][2], wv[D][2];
+    auto request = [&](int set, int b) __attribute__((always_inline)) {
         const int k = min(b, blocks - 1) * 64;    // (past the wave's range: not used)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            xv[B][u] = *reinterpret_cast<const half8_t *>(xp + k + u * 8);
-            wv[B][u] = *reinterpret_cast<const half8_t *>(wp + k + u * 8);
+        for (int u = 0; u < 2; ++u) {
+            xv[set][u] = *reinterpret_cast<const half8_t *>(xp + k + u * 8);
+            wv[set][u] = *reinterpret_cast<const half8_t *>(wp + k + u * 8);
         }
     };
-    auto use = [&](auto set, int b) __attribute__((always_inline)) {
-        constexpr int B = decltype(set)::value;
-        if (b < b1) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[B][u], xv[B][u], acc, 0, 0, 0);
+    for (int d = 0; d < D; ++d) request(d, b0 + d);
+    // (a thread finishes one channel of one pixel)
+    const int oc = n0 + (tid & (T - 1));
+    const int64_t om = (int64_t)tm * T + tid / T;
+    const bool ok = oc < a.N && om < a.M;
+    const _Float16 *res = static_cast<const _Float16 *>(a.res);
+    Affine<1> aff;
+    aff.request(a.norm, oc < a.N ? oc : 0);
+    const _Float16 rv = res ? res[ok ? om * a.N + oc : 0] : (_Float16)0;
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int b = b0; b < b1; b += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (b + d < b1) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[d][u], xv[d][u], acc, 0, 0, 0);
+            }
+            request(d, b + d + D);
         }
-    };
-    using Zero = std::integral_constant<int, 0>;
-    using One = std::integral_constant<int, 1>;
-    if (b0 < b1) {
-        request(Zero{}, b0);
-        request(One{}, b0 + 1);
-    }
-    aff.request(a.norm, cok ? oc : 0);
-#pragma unroll
-    for (int i = 0; i < RO; ++i) {
-        const int64_t mm = (int64_t)tm * 32 + (tid >> 5) + i * PX;
-        rv[i] = res ? res[(mm < a.M ? mm : a.M - 1) * a.N + (cok ? oc : 0)] : (_Float16)0;
-    }
-    for (int b = b0; b < b1; b += 2) {
-        use(Zero{}, b);
-        if (b + 2 < b1) request(Zero{}, b + 2);
-        use(One{}, b + 1);
-        if (b + 3 < b1) request(One{}, b + 3);
     }
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) red[wave][8 * g + 4 * hi + e][l32] = acc[4 * g + e];
+    for (int e = 0; e < 4; ++e) red[wave][4 * quad + e][col] = acc[e];
     __syncthreads();
-    _Float16 *out = static_cast<_Float16 *>(a.out);
     float sc[1], sh[1];
     aff.finish(a.norm, sc, sh);
-    if (!cok) return;
+    if (!ok) return;
+    float f = 0.f;
 #pragma unroll
-    for (int i = 0; i < RO; ++i) {
-        const int px = (tid >> 5) + i * PX;
-        const int64_t mm = (int64_t)tm * 32 + px;
-        if (mm >= a.M) break;
-        float f = 0.f;
-#pragma unroll
-        for (int k = 0; k < WAVES; ++k) f += red[k][tid & 31][px];
-        f = fmaf((float)(_Float16)f, sc[0], sh[0]) + (float)rv[i];
-        if (a.relu) f = relu(f);
-        out[mm * a.N + oc] = (_Float16)f;
-    }
+    for (int k = 0; k < WAVES; ++k) f += red[k][tid & (T - 1)][tid / T];
+    f = fmaf((float)(_Float16)f, sc[0], sh[0]) + (float)rv;
+    if (a.relu) f = relu(f);
+    static_cast<_Float16 *>(a.out)[om * a.N + oc] = (_Float16)f;
 }
 
 // ---- stem: 7x7 convolution of stride 2, BatchNorm, ReLU, 3x3 max-pool of stride 2 ----
@@ -901,10 +880,11 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Rows of whole vectors, and not so few tiles of a long K that splitting K is faster (64 tiles
-// at K = 512: 5.2 us in tiles, 5.0 split; 16 at K = 1024: 7.2 and 6.7; 32 at K = 2048: 11.5 and 9.7).
+// Rows of whole vectors, unless K is long and 16 x 16 results make a workgroup per compute unit
+// at most (us in tiles of 64 / split: 98 x 2048 -> 512, 224 workgroups, 11.7 / 7.4; 196 x 1024 -> 256,
+// 208, 7.4 / 5.7; 392 x 1024 -> 256, 400, 7.4 / 9.2; 128 x 2048 -> 1000, 504, 11.9 / 12.8).
 bool conv_in_tiles(const NetConv &a) {
-    return a.N % 8 == 0 && !(a.K >= 512 && cdiv(a.M, 64) * cdiv(a.N, 64) <= 64);
+    return a.N % 8 == 0 && !(a.K >= 512 && cdiv(a.M, 16) * cdiv(a.N, 16) <= 256);
 }
 
 // The largest tiles that leave somewhat more than a workgroup per compute unit.  Where a unit
@@ -931,8 +911,8 @@ hipError_t net_conv(const NetConv &a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_conv_supported(a)) return hipErrorNotSupported;
     if (conv_in_tiles(a)) return conv_tiles(a, nullptr, st);
-    const int tiles_n = (int)cdiv(a.N, 32);
-    const int64_t blocks = cdiv(a.M, 32) * tiles_n;
+    const int tiles_n = (int)cdiv(a.N, 16);
+    const int64_t blocks = cdiv(a.M, 16) * tiles_n;
     if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(k_net_conv_split, dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
     return hipGetLastError();

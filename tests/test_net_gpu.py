@@ -60,6 +60,9 @@ def close(got, want, tol):
     (16, 28, 28, 128, 264, 1, 1, 0, 1, 1),     # tiles of 128 x 64, channels past the last
     (42, 56, 56, 64, 136, 1, 1, 1, 0, 1),      # tiles of 128 x 128 in short stages
     (3, 7, 7, 2112, 520, 1, 1, 0, 1, 1),       # tiles of 64, 33 stages of K
+    (1, 5, 7, 576, 200, 1, 1, 1, 1, 1),        # K split over the waves: 9 blocks, rows and channels past a tile
+    (17, 1, 1, 64, 33, 1, 0, 1, 0, 1),         # one block of K
+    (1, 13, 9, 1088, 31, 2, 1, 0, 0, 0),       # 17 blocks, under stride 2
 ])
 def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     torch.manual_seed(c + o)
