@@ -547,11 +547,16 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
 
 // ---- spatial filter branch ------------------------------------------------------
 // Pixels are the columns, the nine taps nine of the sixteen rows of 16x16x32 steps over the
-// channels; both operands contiguous.  A wave walks tiles of sixteen pixels of one sample;
-// the same vectors feed the plane sums (KS * 8 fp32 values per lane, brought together at the
-// end).  A pixel's taps end up on four lanes, which normalise them across the wave's
-// rows; they are stored as (pixel, 12), nine taps and padding.  Under stride 2 the three
-// unsampled pixels of a 2 x 2 block only go into the sums.
+// channels; both operands contiguous.  KQ waves share a tile of sixteen pixels, each with its
+// part of the channels (their taps meet in LDS), and walk along one sample; the same vectors feed
+// the plane sums (8 fp32 values per lane and 32 channels, brought together at the end).  With all of
+// 512 channels in one wave, the sums took 256 registers and more, one wave per SIMD, and the loads
+// four dependent rounds: four waves share them (7 x 7, 128 images 9.2 -> 7.6 us, one 8.3 -> 7.1; from
+// 14 x 14 under stride 2 16.5 -> 14.9 and 16.0 -> 13.8).  256 channels over two waves: 14.9 -> 16.6
+// under stride 2, 8.1 -> 8.0 without; not kept.
+// A pixel's taps end up on four lanes, which normalise them across the wave's rows; they are
+// stored as (pixel, 12), nine taps and padding.  Under stride 2 the three unsampled pixels of a
+// 2 x 2 block only go into the sums.
 constexpr int kTapPitch = 12;
 
 __device__ __forceinline__ float rows_total(float v) {
@@ -571,78 +576,82 @@ __device__ __forceinline__ float lanes16_total(float v) {
     return add_permuted<0x140>(v);
 }
 
-template <int KS, int S>
-__global__ __launch_bounds__(kThreads) void k_net_spatial(const _Float16 *__restrict__ x,
+template <int KS, int S, int KQ, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void k_net_spatial(const _Float16 *__restrict__ x,
                                                           const _Float16 *__restrict__ w,
                                                           const _Float16 *__restrict__ bias,
                                                           _Float16 *__restrict__ sf, float *__restrict__ parts,
                                                           int W, int Wo, int npix, int plane, int tiles_per_chunk,
                                                           float gain) {
-    constexpr int C = KS * 32, KK = 9, NPX = S * S;
-    constexpr bool kHold = KS <= 8;               // weights in registers over the walk
-    constexpr int kWaves = kThreads / kWave;
-    __shared__ float red[kWaves][C];
+    constexpr int C = KS * 32, KK = 9, NPX = S * S, KL = KS / KQ, SLOTS = WAVES / KQ;
+    static_assert(KL * KQ == KS && SLOTS * KQ == WAVES);
+    __shared__ float red[SLOTS][C];
+    __shared__ float4_t sums[2][KQ > 1 ? WAVES : 1][kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int kq = wave % KQ, slot = wave / KQ;
     const int col = lane & 15, quad = lane >> 4;
     const int n = blockIdx.y;
     const uint32_t bytes = (uint32_t)plane * C * 2;
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + (int64_t)n * plane * C, bytes);
-    auto weights = [&](int ks) {
-        half8_t v = *reinterpret_cast<const half8_t *>(w + (int64_t)min(col, KK - 1) * C + ks * 32 + quad * 8);
-        if (col >= KK) v = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        return v;
-    };
-    half8_t wv[kHold ? KS : 1];
-    if constexpr (kHold) {
+    half8_t wv[KL];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) wv[ks] = weights(ks);
+    for (int ks = 0; ks < KL; ++ks) {
+        wv[ks] = *reinterpret_cast<const half8_t *>(w + (int64_t)min(col, KK - 1) * C + (kq * KL + ks) * 32 + quad * 8);
+        if (col >= KK) wv[ks] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
     }
     float b[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) b[e] = (bias && quad * 4 + e < KK) ? (float)bias[quad * 4 + e] : 0.f;
-    float pool[KS * 8];
+    float pool[KL * 8];
 #pragma unroll
-    for (int i = 0; i < KS * 8; ++i) pool[i] = 0.f;
+    for (int i = 0; i < KL * 8; ++i) pool[i] = 0.f;
 
     const int tiles = (npix + 15) / 16;
     const int t_end = min((int)(blockIdx.x + 1) * tiles_per_chunk, tiles);
-    for (int t = blockIdx.x * tiles_per_chunk + wave; t < t_end; t += kWaves) {
-        const int p = t * 16 + col;
-        const bool live = p < npix;
+    int buf = 0;
+    for (int t0 = blockIdx.x * tiles_per_chunk; t0 < t_end; t0 += SLOTS) {
+        const int t = t0 + slot, p = t * 16 + col;
+        if (KQ == 1 && t >= t_end) break;
+        const bool live = t < t_end && p < npix;   // (of the others: zeros)
         uint32_t off[NPX];
         if constexpr (S == 1) {
-            off[0] = live ? (uint32_t)p * C * 2 + quad * 16 : kOutside;
+            off[0] = live ? (uint32_t)p * C * 2 + kq * KL * 64 + quad * 16 : kOutside;
         } else {
             const int y = p / Wo, xx = p - y * Wo;
 #pragma unroll
             for (int q = 0; q < NPX; ++q)
-                off[q] = live ? (uint32_t)((2 * y + q / 2) * W + 2 * xx + q % 2) * C * 2 + quad * 16 : kOutside;
+                off[q] = live ? (uint32_t)((2 * y + q / 2) * W + 2 * xx + q % 2) * C * 2 + kq * KL * 64 + quad * 16 : kOutside;
         }
         float4_t acc = {0.f, 0.f, 0.f, 0.f};
-        constexpr int G = KS < 4 ? KS : 4;        // steps requested together
+        constexpr int G = KL < 4 ? KL : S == 2 && WAVES == 16 ? 2 : 4;   // steps requested together
 #pragma unroll
-        for (int k0 = 0; k0 < KS; k0 += G) {
-            half8_t v[NPX][G], wl[kHold ? 1 : G];
+        for (int k0 = 0; k0 < KL; k0 += G) {
+            half8_t v[NPX][G];
 #pragma unroll
             for (int g = 0; g < G; ++g)
 #pragma unroll
                 for (int q = 0; q < NPX; ++q)
                     v[q][g] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
                         xr, (int)off[q], (k0 + g) * 64, 0));
-            if constexpr (!kHold) {
-#pragma unroll
-                for (int g = 0; g < G; ++g) wl[g] = weights(k0 + g);
-            }
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const half8_t a = kHold ? wv[kHold ? k0 + g : 0] : wl[kHold ? 0 : g];
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, v[0][g], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[k0 + g], v[0][g], acc, 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < NPX; ++q)
 #pragma unroll
                     for (int e = 0; e < 8; ++e) pool[(k0 + g) * 8 + e] += (float)v[q][g][e];
             }
+        }
+        if constexpr (KQ > 1) {
+            sums[buf][wave][lane] = acc;
+            __syncthreads();
+            if (kq == 0) {
+#pragma unroll
+                for (int q = 1; q < KQ; ++q) acc += sums[buf][wave + q][lane];
+            }
+            buf ^= 1;
+            if (kq != 0) continue;
         }
         // taps 4 * quad + e of pixel p
         float v[4], s = 0.f;
@@ -665,18 +674,18 @@ __global__ __launch_bounds__(kThreads) void k_net_spatial(const _Float16 *__rest
         if (live && quad < 3) *reinterpret_cast<half4_t *>(sf + ((int64_t)n * npix + p) * kTapPitch + quad * 4) = o;
     }
 #pragma unroll
-    for (int i = 0; i < KS * 8; ++i) pool[i] = lanes16_total(pool[i]);
+    for (int i = 0; i < KL * 8; ++i) pool[i] = lanes16_total(pool[i]);
     if (col == 0) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
+        for (int ks = 0; ks < KL; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) red[wave][ks * 32 + quad * 8 + e] = pool[ks * 8 + e];
+            for (int e = 0; e < 8; ++e) red[slot][(kq * KL + ks) * 32 + quad * 8 + e] = pool[ks * 8 + e];
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < C; c += kThreads) {
+    for (int c = threadIdx.x; c < C; c += WAVES * kWave) {
         float s = 0.f;
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) s += red[k][c];
+        for (int k = 0; k < SLOTS; ++k) s += red[k][c];
         parts[((int64_t)n * gridDim.x + blockIdx.x) * C + c] = s;
     }
 }
@@ -962,15 +971,20 @@ hipError_t net_spatial(const void *x, const void *w, const void *bias, void *sf,
     chunks = (int)cdiv(tiles, per);
     *n_parts = chunks;
     const dim3 grid((unsigned)chunks, (unsigned)N);
-#define DDF_NET_SPATIAL(KS_, S_)                                                                         \
-    if (C == KS_ * 32 && stride == S_) {                                                                 \
-        hipLaunchKernelGGL((k_net_spatial<KS_, S_>), grid, dim3(kThreads), 0, st, (const _Float16 *)x,   \
-                           (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)sf, parts, (int)W,   \
-                           (int)(W / stride), (int)npix, (int)(H * W), per, (float)gain);                \
-        return hipGetLastError();                                                                        \
+    // Sixteen waves per workgroup where there are few workgroups of many tiles (3136 pixels x 64
+    // channels, one image: 7.1 us with four waves, 5.8 with sixteen; 128 and 256 channels, of
+    // which a wave has fewer tiles, 5.4 / 5.8 and 5.6 / 6.8).
+    const bool few = N * chunks <= 256;
+#define DDF_NET_SPATIAL(KS_, S_, KQ_, WAVES_)                                                                       \
+    if (C == KS_ * 32 && stride == S_) {                                                                            \
+        hipLaunchKernelGGL((k_net_spatial<KS_, S_, KQ_, WAVES_>), grid, dim3(WAVES_ * kWave), 0, st,                \
+                           (const _Float16 *)x, (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)sf, parts, \
+                           (int)W, (int)(W / stride), (int)npix, (int)(H * W), per, (float)gain);                   \
+        return hipGetLastError();                                                                                   \
     }
-    DDF_NET_SPATIAL(2, 1) DDF_NET_SPATIAL(4, 1) DDF_NET_SPATIAL(8, 1) DDF_NET_SPATIAL(16, 1)
-    DDF_NET_SPATIAL(2, 2) DDF_NET_SPATIAL(4, 2) DDF_NET_SPATIAL(8, 2) DDF_NET_SPATIAL(16, 2)
+    if (few) DDF_NET_SPATIAL(2, 1, 1, 16)
+    DDF_NET_SPATIAL(2, 1, 1, 4) DDF_NET_SPATIAL(4, 1, 1, 4) DDF_NET_SPATIAL(8, 1, 1, 4) DDF_NET_SPATIAL(16, 1, 4, 16)
+    DDF_NET_SPATIAL(2, 2, 1, 4) DDF_NET_SPATIAL(4, 2, 1, 4) DDF_NET_SPATIAL(8, 2, 1, 4) DDF_NET_SPATIAL(16, 2, 4, 16)
 #undef DDF_NET_SPATIAL
     return hipErrorNotSupported;
 }
