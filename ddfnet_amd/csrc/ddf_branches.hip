@@ -685,9 +685,9 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const int ns = min(NS, N - (int)n0);   // samples of this workgroup (the others: copies of the last)
     const int cb = blockIdx.x * BLOCK;
     // One sample per workgroup: few workgroups, and their time is the round trips to memory.
-    // What does not depend on the pooled vector is requested along with it: the first 64 * AHEAD
-    // values of the wave's first rows of w1, 16 * AHEAD values of all its rows of w2, the biases,
-    // the gains and offsets; without branches, which would end in a wait each (absent values lie
+    // What does not depend on the pooled vector is requested along with it: the wave's rows of w1
+    // (C <= 64 * AHEAD values each) and w2 (mid <= 16 * AHEAD), the biases, the gains and offsets;
+    // without branches, which would end in a wait each (absent values lie
     // outside their buffers).  Six round trips, one after the other, become one: 8 samples of 64
     // channels fp16 6.9 -> 4.9 us, one of 128 9.3 -> 6.3, 128 of 128 9.9 -> 7.0, 32 of 256 fp32
     // 11.0 -> 9.2 (loads of halves into shared registers, or under branches: 10 to 13 us).
@@ -806,7 +806,6 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
 #pragma unroll
             for (int i = 0; i < A2; ++i, m += 16)
                 if (m < mid) p = fmaf(of_bits<T>(w2a[t][i]), h[m], p);
-            for (; m < mid; m += 16) p = fmaf(ld(w2 + ((int64_t)cb * KK + min(r, rows - 1)) * mid + m), h[m], p);
             emit(r, 0, p, of_bits<T>(b2a[t]));
         }
     } else for (int r0 = wave * 4 * RT; r0 < rows; r0 += kChannelWaves * 4 * RT) {
@@ -1404,12 +1403,15 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
     hipLaunchKernelGGL((k_channel_branch<T, 9, 64, 1, A_>), grid, dim3(kChannelThreads), lds, st,     \
                        pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain, gain_vec,   \
                        offset_vec, parts, nparts, (float)scale, save)
-    if (k == 3 && block == 64 && ns == 1) {   // (requests for what a layer of this size has)
+    // Requests ahead of all weights of a layer of up to 256 channels and 64 hidden values, where
+    // every workgroup has a compute unit of its own (their registers leave no room for a second
+    // one: 48 samples x 432 channels, 336 workgroups, layer 61 us ahead, 49 not; 36 x 424, 252
+    // workgroups and weights left over, 38 and 33).
+    if (k == 3 && block == 64 && ns == 1 && C <= 256 && mid <= 64 && (int64_t)grid.x * grid.y <= 256) {
         if (C <= 64 && mid <= 16) DDF_CHANNEL_AHEAD(1);
         else if (C <= 128 && mid <= 32) DDF_CHANNEL_AHEAD(2);
         else DDF_CHANNEL_AHEAD(4);
-    } else if (k == 3 && block == 64 && ns == 2) DDF_CHANNEL_LAUNCH(9, 64, 2);
-    else if (k == 3 && block == 64) DDF_CHANNEL_LAUNCH(9, 64, 4);
+    } else if (k == 3 && block == 64) DDF_CHANNEL_CASE(9, 64);
     else if (k == 3) DDF_CHANNEL_CASE(9, 128);
     else if (k == 5 && block == 64) DDF_CHANNEL_CASE(25, 64);
     else if (k == 5) DDF_CHANNEL_CASE(25, 128);
