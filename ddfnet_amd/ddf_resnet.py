@@ -23,8 +23,8 @@ import torch.nn as nn
 
 from . import functional
 from .functional import ddf  # noqa: F401  (re-exported: callers time the operator through this module)
-from .modules import (DDFPack, FilterNorm, _CONV_CONSTANTS, _PlanSlot, _guard_of, _plain_pointwise_conv,
-                      _unhooked)
+from .modules import (DDFPack, FilterNorm, _CONV_CONSTANTS, _PlanSlot, _guard_of, _holds_own_tensors,
+                      _plain_pointwise_conv, _unhooked)
 
 __all__ = ['DDFBottleneck', 'DDFResNet', 'ddf_mul_resnet50', 'ddf_mul_resnet101',
            'ddf_mul_resnet152', 'ddf_add_resnet50', 'ddf_add_resnet101', 'ddf_add_resnet152',
@@ -170,13 +170,11 @@ class DDFResNet(nn.Module):
     def _native_plan(self, ext):
         """The network's tensors for the extension's native inference, collected once and
         again whenever the network has changed; None where that does not cover it."""
-        slot = self.__dict__.get('_plan')
-        if slot is None:
-            slot = self.__dict__['_plan'] = _PlanSlot()
+        slot = _PlanSlot.of(self)
         if slot.plan is not None and slot.plan.valid():
             return slot.plan
         slot.plan = None
-        if not self._is_stock():
+        if not self._is_stock() or not _holds_own_tensors(self.modules()):
             return None
         own = [self.__dict__[h] for h in ('_forward_hooks', '_forward_pre_hooks', '_backward_hooks',
                                           '_backward_pre_hooks') if h in self.__dict__]
@@ -209,8 +207,7 @@ class DDFResNet(nn.Module):
         # holds, or does not cover the call, answers None)
         ext = functional.extension() if x.is_cuda and x.dtype == torch.float16 and not self.training else None
         if ext is not None:
-            slot = self.__dict__.get('_plan')
-            plan = None if slot is None else slot.plan
+            plan = _PlanSlot.plan_of(self)
             out = None if plan is None else ext.net_forward(plan, x)
             if out is None:
                 fresh = self._native_plan(ext)

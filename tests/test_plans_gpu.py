@@ -1,0 +1,67 @@
+"""Layers and networks around their native plans: what runs is always the module that was
+called, as it is at the time of the call."""
+import copy
+
+import pytest
+import torch
+
+import ddfnet_amd
+from test_plans import replica_of, small_net
+
+pytestmark = pytest.mark.gpu
+
+
+def by_modules(layer, x):
+    """The layer from its branches, run as modules, and the operator."""
+    b, c, h, w = x.shape
+    g, k, s = layer.head, layer.kernel_size, layer.stride
+    cf = layer.channel_branch(x).reshape(b * g, c // g, k, k)
+    sf = layer.spatial_branch(x).reshape(b * g, k * k, h // s, w // s)
+    out = ddfnet_amd.ddf(x.reshape(b * g, c // g, h, w), cf, sf, k, layer.dilation, s, layer.kernel_combine)
+    return out.reshape(b, c, h // s, w // s)
+
+
+def close(got, want, tol=1e-4):
+    assert got.shape == want.shape
+    assert (got - want).abs().max() <= tol * want.abs().max()
+
+
+@pytest.mark.parametrize('grad', [False, True])
+def test_shallow_copy_runs_as_configured(grad):
+    torch.manual_seed(0)
+    layer = ddfnet_amd.DDFPack(16).cuda()
+    x = torch.randn(2, 16, 8, 8, device='cuda')
+    with torch.set_grad_enabled(grad):
+        layer(x)
+        other = copy.copy(layer)
+        other.kernel_combine = 'add'
+        for m in (other, layer, other):
+            close(m(x), by_modules(m, x))
+
+
+@pytest.mark.parametrize('grad', [False, True])
+def test_replicas_run_with_their_own_weights(grad):
+    torch.manual_seed(1)
+    layer = ddfnet_amd.DDFPack(16).cuda()
+    x = torch.randn(2, 16, 8, 8, device='cuda')
+    with torch.set_grad_enabled(grad):
+        layer(x)
+        for scale in (2., 3.):
+            replica = replica_of(layer)
+            replica.channel_branch[4].std.mul_(scale)
+            close(replica(x), scale * by_modules(layer, x))
+            close(layer(x), by_modules(layer, x))
+
+
+def test_replicas_of_a_network_run_with_their_own_weights():
+    torch.manual_seed(2)
+    net = small_net().cuda()
+    x = torch.randn(2, 3, 64, 64, device='cuda').half()
+    with torch.no_grad():
+        want = net(x)
+        for value in (1., 2.):
+            replica = replica_of(net)
+            replica.fc.weight.zero_()
+            replica.fc.bias.fill_(value)
+            assert torch.equal(replica(x), torch.full_like(want, value))
+        assert torch.equal(net(x), want)
