@@ -29,12 +29,12 @@ struct NetBlock {
 using NetLayerArgs = std::pair<std::vector<c10::optional<at::Tensor>>, double>;
 
 struct NetPlan {
-    ModuleGuard guard;
+    std::shared_ptr<ModuleGuard> guard;
     NetLayer stem, fc;
     std::vector<NetBlock> blocks;
     std::vector<at::Tensor> all;
 
-    NetPlan(py::list same, py::list empty) : guard(std::move(same), std::move(empty)) {}
+    explicit NetPlan(std::shared_ptr<ModuleGuard> guard_) : guard(std::move(guard_)) {}
 
     NetLayer layer(const NetLayerArgs &a) {
         NetLayer l;
@@ -74,7 +74,7 @@ struct NetPlan {
 inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
     if (!input.is_cuda() || input.scalar_type() != at::kHalf || input.dim() != 4 || input.size(1) != 3 ||
         input.size(0) < 1 || input.size(0) > 65535 || input.size(2) % 32 || input.size(3) % 32 || input.numel() == 0 ||
-        at::autocast::is_autocast_enabled(at::kCUDA) || !p.guard.holds())
+        at::autocast::is_autocast_enabled(at::kCUDA) || !p.guard->holds())
         return py::none();
     const auto dev = input.device();
     const bool grad = at::GradMode::is_enabled();

@@ -18,7 +18,7 @@ inline size_t aligned_bytes(size_t n) { return (n + kAlign - 1) / kAlign * kAlig
 // What a DDFPack is made of, collected once by DDFPack._native_plan in modules.py (which
 // has checked that both branches are the stock ones).
 struct PackPlan {
-    ModuleGuard guard;
+    std::shared_ptr<ModuleGuard> guard;
     // 1x1 convolutions (weight, bias): spatial branch, first and second of the channel branch
     at::Tensor ws, bs, w1, b1, w2, b2;
     // FilterNorm: learned gains and offsets, or the constant gain
@@ -27,12 +27,12 @@ struct PackPlan {
     int k, d, s, head, combine;
     bool fuse_pool, fuse_norm;
 
-    PackPlan(py::list same, py::list empty, std::vector<at::Tensor> convs,
+    PackPlan(std::shared_ptr<ModuleGuard> guard_, std::vector<at::Tensor> convs,
              c10::optional<at::Tensor> sgain_vec_, c10::optional<at::Tensor> soffset_vec_,
              c10::optional<at::Tensor> cgain_vec_, c10::optional<at::Tensor> coffset_vec_, double sgain_,
              double cgain_, int k_, int d_, int s_, int head_, const std::string &combine_, bool fuse_pool_,
              bool fuse_norm_)
-        : guard(std::move(same), std::move(empty)), sgain_vec(std::move(sgain_vec_)),
+        : guard(std::move(guard_)), sgain_vec(std::move(sgain_vec_)),
           soffset_vec(std::move(soffset_vec_)), cgain_vec(std::move(cgain_vec_)),
           coffset_vec(std::move(coffset_vec_)), sgain(sgain_), cgain(cgain_), k(k_), d(d_), s(s_), head(head_),
           combine(combine_ == "add" ? DDF_ADD : DDF_MUL), fuse_pool(fuse_pool_), fuse_norm(fuse_norm_) {
@@ -224,7 +224,7 @@ public:
 // DDFPack.forward through a plan: the result, or None where the plan does not (any longer)
 // describe the layer or the native path does not cover the call.
 inline py::object pack_forward(const PackPlan &p, const at::Tensor &x) {
-    if (!p.guard.holds() || !x.is_cuda() || x.dim() != 4) return py::none();
+    if (!p.guard->holds() || !x.is_cuda() || x.dim() != 4) return py::none();
     const int dt = dtype_code(x.scalar_type());
     // (a size the stride does not divide fails in the layer's own code, as in the reference
     // at ddf/ddf.py:215-218)

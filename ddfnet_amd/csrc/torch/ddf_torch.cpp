@@ -417,20 +417,28 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("ddf_up", &ddf_up, py::arg("features"), py::arg("channel_filters"),
           py::arg("spatial_filters"), py::arg("kernel_size") = 3, py::arg("dilation") = 1,
           py::arg("scale_factor") = 2, py::arg("kernel_combine") = "mul");
+    py::class_<ModuleGuard::Rules>(m, "GuardRules")
+        .def(py::init([](py::dict classes, py::dict own, py::tuple operators, py::tuple silent) {
+            return ModuleGuard::Rules{classes, own, operators, silent};
+        }));
+    py::class_<ModuleGuard, std::shared_ptr<ModuleGuard>>(m, "ModuleGuard")
+        .def("holds", &ModuleGuard::holds)
+        .def("covers", &ModuleGuard::covers);
+    m.def("guard_of", &ModuleGuard::make, "a guard of modules (the first is the owner), or None");
     py::class_<PackPlan>(m, "PackPlan")
-        .def(py::init<py::list, py::list, std::vector<at::Tensor>, c10::optional<at::Tensor>,
+        .def(py::init<std::shared_ptr<ModuleGuard>, std::vector<at::Tensor>, c10::optional<at::Tensor>,
                       c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>, double, double,
                       int, int, int, int, const std::string &, bool, bool>())
-        .def("valid", [](const PackPlan &p) { return p.guard.holds(); });
+        .def("valid", [](const PackPlan &p) { return p.guard->holds(); });
     m.def("pack_forward", &pack_forward, "DDFPack.forward through a plan, or None");
     m.def("pack_infer", &pack_infer,
           "DDFPack.forward without gradients: spatial branch (pooling on the way where it can), "
           "channel branch, operator");
     py::class_<NetPlan>(m, "NetPlan")
-        .def(py::init<py::list, py::list>())
+        .def(py::init<std::shared_ptr<ModuleGuard>>())
         .def("set_ends", &NetPlan::set_ends)
         .def("add_block", &NetPlan::add_block)
-        .def("valid", [](const NetPlan &p) { return p.guard.holds(); });
+        .def("valid", [](const NetPlan &p) { return p.guard->holds(); });
     m.def("net_forward", &net_forward, "DDFResNet.forward through a plan, or None");
     m.def("library_version", []() { return ddf_hip_version(); });
 }

@@ -23,8 +23,8 @@ import torch.nn as nn
 
 from . import functional
 from .functional import ddf  # noqa: F401  (re-exported: callers time the operator through this module)
-from .modules import (DDFPack, FilterNorm, _CONV_CONSTANTS, _PlanSlot, _guard_of, _holds_own_tensors,
-                      _plain_pointwise_conv, _unhooked)
+from .modules import (DDFPack, _CLASS_RULES, _OWN_METHODS, _PlanSlot, _guard_of, _plain_pointwise_conv, _rule,
+                      _unhooked)
 
 __all__ = ['DDFBottleneck', 'DDFResNet', 'ddf_mul_resnet50', 'ddf_mul_resnet101',
            'ddf_mul_resnet152', 'ddf_add_resnet50', 'ddf_add_resnet101', 'ddf_add_resnet152',
@@ -174,31 +174,33 @@ class DDFResNet(nn.Module):
         if slot.plan is not None and slot.plan.valid():
             return slot.plan
         slot.plan = None
-        if not self._is_stock() or not _holds_own_tensors(self.modules()):
+        if not self._is_stock():
             return None
-        own = [self.__dict__[h] for h in ('_forward_hooks', '_forward_pre_hooks', '_backward_hooks',
-                                          '_backward_pre_hooks') if h in self.__dict__]
-        same, empty = _guard_of(list(self.modules()), {
-            nn.Conv2d: _CONV_CONSTANTS, nn.BatchNorm2d: ('training', 'eps', 'affine', 'track_running_stats'),
-            nn.AdaptiveAvgPool2d: ('output_size',),
-            nn.MaxPool2d: ('kernel_size', 'stride', 'padding', 'dilation', 'ceil_mode', 'return_indices'),
-            FilterNorm: ('in_channels', 'filter_type', 'runing_std', 'runing_mean', 'std'),
-            DDFPack: ('kernel_size', 'stride', 'dilation', 'head', 'kernel_combine')})
-        plan = ext.NetPlan(same, [d for d in empty if not any(d is o for o in own)])
+        guard = _guard_of(ext, list(self.modules()))
+        if guard is None:
+            return None
+        plan, tensors = ext.NetPlan(guard), []
+
+        def layer(conv, norm):
+            args = _layer_args(conv, norm)
+            tensors.extend(args[0])
+            return args
+
         identity = nn.Identity()
-        plan.set_ends(_layer_args(self.conv1, self.bn1), _layer_args(self.fc, identity))
+        plan.set_ends(layer(self.conv1, self.bn1), layer(self.fc, identity))
         for block in self._blocks():
             pack, down = block.conv2, block.downsample
             conv, sp_norm = pack.spatial_branch
             fc1, fc2, ch_norm = pack.channel_branch[1], pack.channel_branch[3], pack.channel_branch[4]
+            branches = [conv.weight, conv.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias,
+                        ch_norm.std if ch_norm.runing_std else None, ch_norm.mean if ch_norm.runing_mean else None]
+            tensors.extend(branches)
             plan.add_block(
-                _layer_args(block.conv1, block.bn1), _layer_args(None, block.bn2),
-                _layer_args(block.conv3, block.bn3),
-                ([None] * 6, 0.0) if down is None else
-                _layer_args(down[0], down[1] if len(down) > 1 else identity),
-                [conv.weight, conv.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias,
-                 ch_norm.std if ch_norm.runing_std else None, ch_norm.mean if ch_norm.runing_mean else None],
+                layer(block.conv1, block.bn1), layer(None, block.bn2), layer(block.conv3, block.bn3),
+                ([None] * 6, 0.0) if down is None else layer(down[0], down[1] if len(down) > 1 else identity), branches,
                 sp_norm.std, 1.0 if ch_norm.runing_std else ch_norm.std, pack.stride, pack.kernel_combine)
+        if not guard.covers(tensors):
+            return None
         slot.plan = plan
         return plan
 
@@ -217,6 +219,11 @@ class DDFResNet(nn.Module):
                 return out
         x = self.global_pool(self.forward_features(x)).flatten(1)
         return self.fc(x)
+
+
+_CLASS_RULES[DDFBottleneck] = _rule(DDFBottleneck)
+_OWN_METHODS[DDFResNet] = ('forward_features', '_blocks', '_is_stock', '_native_plan')
+_CLASS_RULES[DDFResNet] = _rule(DDFResNet, (), ('forward',) + _OWN_METHODS[DDFResNet])
 
 
 def _make(layers, combine):

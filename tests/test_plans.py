@@ -57,3 +57,102 @@ def test_replicas_have_no_plan(make, planned, ext):
     first, second = replica_of(module), replica_of(module)
     assert first._native_plan(ext) is None and second._native_plan(ext) is None
     assert module._native_plan(ext) is not None and (plan is None or module._native_plan(ext) is plan)
+
+
+def _replace_class(m, monkeypatch):
+    m.channel_branch[2].__class__ = torch.nn.LeakyReLU
+
+
+def _class_method(m, monkeypatch):
+    monkeypatch.setattr(torch.nn.Conv2d, 'forward', lambda self, x: x)
+
+
+def _call_of_every_module(m, monkeypatch):
+    monkeypatch.setattr(torch.nn.Module, '__call__', lambda self, *a: None)
+
+
+LAYER_CHANGES = {
+    # (stock: whether a new plan may be made of the changed layer)
+    'module appended': (False, lambda m, mp: m.spatial_branch.append(torch.nn.Tanh())),
+    'module added': (False, lambda m, mp: m.channel_branch.add_module('5', torch.nn.Tanh())),
+    'module replaced': (True, lambda m, mp: m.channel_branch.__setitem__(1, torch.nn.Conv2d(16, 3, 1))),
+    'modules reordered': (False, lambda m, mp: m.channel_branch._modules.__setitem__(
+        '2', m.channel_branch._modules.pop('2'))),
+    'other table': (True, lambda m, mp: setattr(m.spatial_branch, '_modules', dict(m.spatial_branch._modules))),
+    'unused parameter': (True, lambda m, mp: m.spatial_branch.register_parameter(
+        'extra', torch.nn.Parameter(torch.ones(1)))),
+    'parameter replaced': (True, lambda m, mp: setattr(m.spatial_branch[0], 'weight', torch.nn.Parameter(
+        torch.ones(9, 16, 1, 1)))),
+    'parameter hidden': (False, lambda m, mp: m.spatial_branch[0].__dict__.__setitem__('weight', torch.ones(9, 16, 1, 1))),
+    'instance forward': (False, lambda m, mp: setattr(m.spatial_branch[0], 'forward', lambda x: x)),
+    'forward of a branch': (False, lambda m, mp: setattr(m.spatial_branch, 'forward', lambda x: x)),
+    'method of the layer': (False, lambda m, mp: setattr(m, '_channel_filter', lambda x: x)),
+    'class replaced': (False, _replace_class),
+    'class method': (False, _class_method),
+    'calls of all modules': (False, _call_of_every_module),
+    'attribute': (True, lambda m, mp: setattr(m, 'kernel_combine', 'add')),
+    'attribute of a module': (False, lambda m, mp: setattr(m.spatial_branch[0], 'stride', (2, 2))),
+    'hook': (False, lambda m, mp: m.channel_branch[2].register_forward_hook(lambda *a: None)),
+    'hooks of its own dictionary': (False, lambda m, mp: setattr(m.channel_branch[2], '_forward_hooks', {0: lambda *a: None})),
+    'operator': (False, lambda m, mp: mp.setattr(ddfnet_amd.modules, 'ddf', lambda *a: None)),
+}
+
+
+@pytest.mark.parametrize('change', LAYER_CHANGES)
+def test_a_changed_layer_loses_its_plan(change, ext, monkeypatch):
+    m = ddfnet_amd.DDFPack(16)
+    plan = m._native_plan(ext)
+    still_stock, apply = LAYER_CHANGES[change]
+    apply(m, monkeypatch)
+    assert not plan.valid()
+    assert (m._native_plan(ext) is not None) == still_stock
+
+
+def test_what_does_not_matter_keeps_a_plan(ext):
+    m = ddfnet_amd.DDFPack(16)
+    plan = m._native_plan(ext)
+    m.calls = 1                                   # attributes that nothing of a plan reads
+    m.spatial_branch[0].note = torch.ones(1)
+    m.forward = m.forward                         # wrapped: whoever calls this one wants it
+    m.register_forward_hook(lambda *a: None)      # the layer's own hooks run around its forward
+    m.eval()
+    with torch.no_grad():
+        m.spatial_branch[0].weight.mul_(2.)
+    m.half()
+    assert plan.valid() and m._native_plan(ext) is plan
+
+
+class _Widened(ddfnet_amd.DDFPack):
+    def _channel_filter(self, x):
+        return super()._channel_filter(x) * 2
+
+
+def test_subclasses_with_methods_of_their_own_have_no_plan(ext):
+    assert _Widened(16)._native_plan(ext) is None
+    assert type('Named', (ddfnet_amd.DDFPack,), {})(16)._native_plan(ext) is not None
+
+
+NET_CHANGES = {
+    'block appended': lambda m, mp: m.layer1.append(copy.deepcopy(m.layer1[0])),
+    'forward of a block': lambda m, mp: setattr(m.layer1[0], 'forward', lambda x: x),
+    'forward of a layer': lambda m, mp: setattr(m.layer2[0].conv2, 'forward', lambda x: x),
+    'features': lambda m, mp: setattr(m, 'forward_features', lambda x: x),
+    'class of a block': lambda m, mp: setattr(m.layer1[0], '__class__', torch.nn.Identity),
+    'method of a class': lambda m, mp: mp.setattr(torch.nn.BatchNorm2d, 'forward', lambda self, x: x),
+    'class of a norm': lambda m, mp: setattr(m.bn1, '__class__', torch.nn.SyncBatchNorm),
+    'norm in training': lambda m, mp: m.layer3[0].bn2.train(),
+    'hook': lambda m, mp: m.layer4[0].act3.register_forward_pre_hook(lambda *a: None),
+}
+
+
+@pytest.mark.parametrize('before', [False, True])
+@pytest.mark.parametrize('change', NET_CHANGES)
+def test_a_changed_network_has_no_plan(change, before, ext, monkeypatch):
+    """before: the change is there when a plan is first asked for."""
+    m = small_net()
+    plan = None if before else m._native_plan(ext)
+    if not before:
+        assert plan is not None
+    NET_CHANGES[change](m, monkeypatch)
+    assert before or not plan.valid()
+    assert m._native_plan(ext) is None

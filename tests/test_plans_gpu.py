@@ -65,3 +65,23 @@ def test_replicas_of_a_network_run_with_their_own_weights():
             replica.fc.bias.fill_(value)
             assert torch.equal(replica(x), torch.full_like(want, value))
         assert torch.equal(net(x), want)
+
+
+def test_appended_modules_and_replaced_methods_take_part():
+    torch.manual_seed(3)
+    layer = ddfnet_amd.DDFPack(16).cuda()
+    x = torch.randn(2, 16, 8, 8, device='cuda')
+    net = small_net().cuda()
+    image = torch.randn(2, 3, 64, 64, device='cuda').half()
+    with torch.no_grad():
+        layer(x)
+        layer.spatial_branch.append(torch.nn.Tanh())
+        close(layer(x), by_modules(layer, x))
+        want = net(image)
+        net.layer1[0].forward = lambda y: torch.zeros(2, 256, 16, 16, device='cuda', dtype=torch.float16)
+        zeroed = net(image)
+        assert not torch.equal(zeroed, want)
+        del net.layer1[0].forward
+        assert torch.equal(net(image), want)
+        net.layer1[0].act3.forward = lambda y: y * 0
+        close(net(image), zeroed, 2e-2)
