@@ -32,57 +32,79 @@ struct NetPlan {
     std::shared_ptr<ModuleGuard> guard;
     NetLayer stem, fc;
     std::vector<NetBlock> blocks;
-    std::vector<at::Tensor> all;
+    // every tensor and the sizes it must have
+    std::vector<std::pair<at::Tensor, std::vector<int64_t>>> all;
 
     explicit NetPlan(std::shared_ptr<ModuleGuard> guard_) : guard(std::move(guard_)) {}
 
-    NetLayer layer(const NetLayerArgs &a) {
+    void expect(const at::Tensor &t, std::vector<int64_t> sizes) {
+        if (t.defined()) all.emplace_back(t, std::move(sizes));
+    }
+    // A convolution of these sizes (none: only what follows it) with what follows it.
+    NetLayer layer(const NetLayerArgs &a, std::vector<int64_t> sizes, int64_t channels) {
         NetLayer l;
         TORCH_CHECK(a.first.size() == 6, "six tensors per layer expected");
-        for (int i = 0; i < 6; ++i)
-            if (a.first[i].has_value() && a.first[i]->defined()) {
-                l.t[i] = *a.first[i];
-                all.push_back(l.t[i]);
-            }
+        for (int i = 0; i < 6; ++i) {
+            if (a.first[i].has_value()) l.t[i] = *a.first[i];
+            expect(l.t[i], i == 0 ? sizes : std::vector<int64_t>{channels});
+        }
         l.eps = (float)a.second;
         return l;
     }
-    void set_ends(const NetLayerArgs &s, const NetLayerArgs &f) { stem = layer(s); fc = layer(f); }
+    void set_ends(const NetLayerArgs &s, const NetLayerArgs &f, int64_t features, int64_t classes) {
+        stem = layer(s, {64, 3, 7, 7}, 64);
+        fc = layer(f, {classes, features}, classes);
+    }
+    // A bottleneck of `in` -> `width` -> `out` channels with `mid` hidden ones.
     void add_block(const NetLayerArgs &conv1, const NetLayerArgs &bn2, const NetLayerArgs &conv3,
                    const NetLayerArgs &down, std::vector<c10::optional<at::Tensor>> branches, double sgain,
-                   double cgain, int stride, const std::string &combine) {
+                   double cgain, int stride, const std::string &combine, int64_t in, int64_t width, int64_t out,
+                   int64_t mid) {
         NetBlock b;
-        b.conv1 = layer(conv1); b.bn2 = layer(bn2); b.conv3 = layer(conv3); b.down = layer(down);
+        b.conv1 = layer(conv1, {width, in, 1, 1}, width);
+        b.bn2 = layer(bn2, {}, width);
+        b.conv3 = layer(conv3, {out, width, 1, 1}, out);
+        b.down = layer(down, {out, in, 1, 1}, out);
         at::Tensor *const to[8] = {&b.ws, &b.bs, &b.w1, &b.b1, &b.w2, &b.b2, &b.cgain, &b.coffset};
+        const std::vector<int64_t> sizes[8] = {{9, width, 1, 1}, {9}, {mid, width, 1, 1}, {mid}, {9 * width, mid, 1, 1},
+                                               {9 * width}, {9 * width}, {9 * width}};
         TORCH_CHECK(branches.size() == 8, "eight branch tensors expected");
-        for (int i = 0; i < 8; ++i)
-            if (branches[i].has_value() && branches[i]->defined()) {
-                *to[i] = *branches[i];
-                all.push_back(*to[i]);
-            }
+        for (int i = 0; i < 8; ++i) {
+            if (branches[i].has_value()) *to[i] = *branches[i];
+            expect(*to[i], sizes[i]);
+        }
         b.sgain = sgain; b.cgain_const = cgain;
         b.stride = stride;
-        b.combine = combine == "add" ? DDF_ADD : DDF_MUL;
-        b.width = b.conv1.t[0].size(0);
-        b.mid = b.w1.size(0);
+        b.combine = combine_code(combine);
+        b.width = width;
+        b.mid = mid;
         blocks.push_back(b);
+    }
+    // Why the native inference cannot run this input with the network's tensors as they are now
+    // (parameters may have been resized, moved or re-laid in place), or null.
+    const char *misfit(const at::Tensor &x) const {
+        if (x.scalar_type() != at::kHalf || x.dim() != 4 || x.size(1) != 3) return "images in fp16 expected";
+        if (x.size(0) < 1 || x.size(0) > 65535 || x.size(2) % 32 || x.size(3) % 32 || x.numel() == 0)
+            return "image sizes not covered";
+        const bool grad = at::GradMode::is_enabled();
+        if (grad && x.requires_grad()) return "gradients wanted";
+        const auto dev = x.device();
+        for (const auto &[t, sizes] : all) {
+            if (t.scalar_type() != at::kHalf || t.device() != dev) return "parameters must be fp16 and with the images";
+            if (t.sizes() != sizes) return "parameters do not fit each other";
+            if (!t.is_contiguous() || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) return "parameters must be laid out densely";
+            if (grad && t.requires_grad()) return "gradients wanted";
+        }
+        return nullptr;
     }
 };
 
 // Logits, or None where the plan does not (any longer) describe the network or the native
 // path does not cover the call.
 inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
-    if (!input.is_cuda() || input.scalar_type() != at::kHalf || input.dim() != 4 || input.size(1) != 3 ||
-        input.size(0) < 1 || input.size(0) > 65535 || input.size(2) % 32 || input.size(3) % 32 || input.numel() == 0 ||
-        at::autocast::is_autocast_enabled(at::kCUDA) || !p.guard->holds())
+    if (!input.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || !p.guard->holds() || p.misfit(input))
         return py::none();
     const auto dev = input.device();
-    const bool grad = at::GradMode::is_enabled();
-    if (grad && input.requires_grad()) return py::none();
-    for (const at::Tensor &t : p.all)
-        if (t.scalar_type() != at::kHalf || t.device() != dev || !t.is_contiguous() || (grad && t.requires_grad()) ||
-            reinterpret_cast<uintptr_t>(t.data_ptr()) % 16)
-            return py::none();
     const at::Tensor x = input.contiguous();
     const int64_t n = x.size(0), h0 = x.size(2), w0 = x.size(3);
     c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(dev);

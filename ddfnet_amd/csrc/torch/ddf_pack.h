@@ -15,8 +15,9 @@ namespace ddf_torch {
 constexpr size_t kAlign = 256;
 inline size_t aligned_bytes(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
 
-// What a DDFPack is made of, collected once by DDFPack._native_plan in modules.py (which
-// has checked that both branches are the stock ones).
+// What a DDFPack is made of, collected by DDFPack._pack_plan in modules.py (which has
+// checked that both branches are the stock ones): with a guard once, for calls through
+// pack_forward, or without for a single call of pack_infer.
 struct PackPlan {
     std::shared_ptr<ModuleGuard> guard;
     // 1x1 convolutions (weight, bias): spatial branch, first and second of the channel branch
@@ -24,33 +25,48 @@ struct PackPlan {
     // FilterNorm: learned gains and offsets, or the constant gain
     c10::optional<at::Tensor> sgain_vec, soffset_vec, cgain_vec, coffset_vec;
     double sgain, cgain;
+    int64_t channels;     // that the channel filters are normalised by
     int k, d, s, head, combine;
     bool fuse_pool, fuse_norm;
 
     PackPlan(std::shared_ptr<ModuleGuard> guard_, std::vector<at::Tensor> convs,
              c10::optional<at::Tensor> sgain_vec_, c10::optional<at::Tensor> soffset_vec_,
              c10::optional<at::Tensor> cgain_vec_, c10::optional<at::Tensor> coffset_vec_, double sgain_,
-             double cgain_, int k_, int d_, int s_, int head_, const std::string &combine_, bool fuse_pool_,
-             bool fuse_norm_)
+             double cgain_, int64_t channels_, int k_, int d_, int s_, int head_, const std::string &combine_,
+             bool fuse_pool_, bool fuse_norm_)
         : guard(std::move(guard_)), sgain_vec(std::move(sgain_vec_)),
           soffset_vec(std::move(soffset_vec_)), cgain_vec(std::move(cgain_vec_)),
-          coffset_vec(std::move(coffset_vec_)), sgain(sgain_), cgain(cgain_), k(k_), d(d_), s(s_), head(head_),
-          combine(combine_ == "add" ? DDF_ADD : DDF_MUL), fuse_pool(fuse_pool_), fuse_norm(fuse_norm_) {
+          coffset_vec(std::move(coffset_vec_)), sgain(sgain_), cgain(cgain_), channels(channels_), k(k_), d(d_), s(s_),
+          head(head_), combine(combine_code(combine_)), fuse_pool(fuse_pool_), fuse_norm(fuse_norm_) {
         TORCH_CHECK(convs.size() == 6, "six convolution tensors expected");
         ws = convs[0]; bs = convs[1]; w1 = convs[2]; b1 = convs[3]; w2 = convs[4]; b2 = convs[5];
     }
-    // Every tensor lives with the features, in their dtype, laid out densely.
-    bool fits(const at::Tensor &x) const {
+    // Why the branch kernels cannot run these features with the plan's tensors as they are now
+    // (parameters may have been resized, moved or re-laid in place), or null.
+    const char *misfit(const at::Tensor &x) const {
         const auto type = x.scalar_type();
         const auto dev = x.device();
-        for (const at::Tensor *t : {&ws, &bs, &w1, &b1, &w2, &b2})
-            if (t->defined() && (t->scalar_type() != type || t->device() != dev || !t->is_contiguous())) return false;
-        for (const auto *t : {&sgain_vec, &soffset_vec, &cgain_vec, &coffset_vec})
-            if (t->has_value() && ((*t)->scalar_type() != type || (*t)->device() != dev || !(*t)->is_contiguous()))
-                return false;
         const int64_t c = x.size(1), kk = (int64_t)k * k;
-        return ws.size(0) == head * kk && ws.size(1) == c && w1.size(1) == c && w2.size(0) == c * kk &&
-               w2.size(1) == w1.size(0) && c % head == 0;
+        if (head < 1 || c % head != 0) return "channels must divide into heads";
+        if (channels != c) return "the channel filters' normalisation does not fit the features";
+        for (const at::Tensor *t : {&ws, &w1, &w2})
+            if (t->dim() != 4 || t->size(2) != 1 || t->size(3) != 1) return "branch weights do not fit the features";
+        const int64_t mid = w1.size(0);
+        if (ws.size(0) != head * kk || ws.size(1) != c || w1.size(1) != c || w2.size(0) != c * kk || w2.size(1) != mid)
+            return "branch weights do not fit the features";
+        const char *why = nullptr;
+        auto ask = [&](const at::Tensor &t, int64_t count) {
+            if (why || !t.defined()) return;
+            if (t.scalar_type() != type || t.device() != dev) why = "parameters must be of the features' type and device";
+            else if (!t.is_contiguous()) why = "weights must be contiguous";
+            else if (t.numel() != count) why = "branch parameters do not fit the features";
+        };
+        ask(ws, head * kk * c); ask(bs, head * kk);
+        ask(w1, mid * c); ask(b1, mid);
+        ask(w2, c * kk * mid); ask(b2, c * kk);
+        ask(sgain_vec.value_or(at::Tensor()), head * kk); ask(soffset_vec.value_or(at::Tensor()), head * kk);
+        ask(cgain_vec.value_or(at::Tensor()), c * kk); ask(coffset_vec.value_or(at::Tensor()), c * kk);
+        return why;
     }
     bool wants_gradients(const at::Tensor &x) const {
         if (x.requires_grad()) return true;
@@ -68,8 +84,8 @@ inline const void *ptr_or_null(const c10::optional<at::Tensor> &t) {
 inline const void *ptr_or_null(const at::Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 // Without gradients: spatial branch (leaving the planes' partial sums where its kernel
-// can), channel branch, operator.
-inline at::Tensor pack_infer(const PackPlan &p, const at::Tensor &features) {
+// can), channel branch, operator.  (The caller has asked misfit.)
+inline at::Tensor pack_run(const PackPlan &p, const at::Tensor &features) {
     const int dt = dtype_code(features.scalar_type());
     const at::Tensor x = features.contiguous();
     const int64_t b = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3), mid = p.w1.size(0);
@@ -221,15 +237,27 @@ public:
     }
 };
 
+// The same for a caller without a standing plan; refuses with an error what the kernels do not
+// take.
+inline at::Tensor pack_infer(const PackPlan &p, const at::Tensor &x) {
+    TORCH_CHECK(x.is_cuda() && x.dim() == 4, "features must be a 4-d device tensor");
+    const int dt = dtype_code(x.scalar_type());
+    TORCH_CHECK(dt == DDF_F16 || dt == DDF_F32, "the branch kernels cover fp16 and fp32");
+    const char *why = p.misfit(x);
+    TORCH_CHECK(why == nullptr, why);
+    return pack_run(p, x);
+}
+
 // DDFPack.forward through a plan: the result, or None where the plan does not (any longer)
 // describe the layer or the native path does not cover the call.
 inline py::object pack_forward(const PackPlan &p, const at::Tensor &x) {
-    if (!p.guard->holds() || !x.is_cuda() || x.dim() != 4) return py::none();
+    if (!p.guard || !p.guard->holds() || !x.is_cuda() || x.dim() != 4) return py::none();
     const int dt = dtype_code(x.scalar_type());
     // (a size the stride does not divide fails in the layer's own code, as in the reference
     // at ddf/ddf.py:215-218)
-    if ((dt != DDF_F16 && dt != DDF_F32) || x.size(2) % p.s || x.size(3) % p.s || !p.fits(x)) return py::none();
-    if (!(at::GradMode::is_enabled() && p.wants_gradients(x))) return py::cast(pack_infer(p, x));
+    if ((dt != DDF_F16 && dt != DDF_F32) || x.size(2) % p.s || x.size(3) % p.s || p.misfit(x))
+        return py::none();
+    if (!(at::GradMode::is_enabled() && p.wants_gradients(x))) return py::cast(pack_run(p, x));
     // Training: the stock configuration only (constant spatial gain, learned channel gain, no
     // offsets, biases present), everything trained.
     if (!p.fuse_norm || p.sgain_vec || p.soffset_vec || p.coffset_vec || !p.cgain_vec) return py::none();

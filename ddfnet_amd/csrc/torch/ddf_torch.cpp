@@ -56,6 +56,12 @@ inline int dtype_code(at::ScalarType t) {
     }
 }
 
+inline int combine_code(const std::string &kernel_combine) {
+    if (kernel_combine == "mul") return DDF_MUL;
+    if (kernel_combine == "add") return DDF_ADD;
+    assertion_error("only support mul or add combination, instead of " + kernel_combine);
+}
+
 std::string size_string(const at::Tensor &t) {
     // as torch.Size prints: torch.Size([2, 3, 4, 5])
     std::ostringstream os;
@@ -173,10 +179,7 @@ at::Tensor ddf(at::Tensor features, at::Tensor channel_filter, at::Tensor spatia
         assertion_error("spatial_filter size " + size_string(spatial_filter) +
                         " does not match kernel size " + std::to_string(kernel_size));
     if ((kernel_size - 1) % 2 != 0 || kernel_size < 1 || dilation < 1) assertion_error("");
-    int combine;
-    if (kernel_combine == "mul") combine = DDF_MUL;
-    else if (kernel_combine == "add") combine = DDF_ADD;
-    else assertion_error("only support mul or add combination, instead of " + kernel_combine);
+    const int combine = combine_code(kernel_combine);
     int variant;
     if (version.empty()) variant = DDF_VARIANT_AUTO;
     else if (version == "o") variant = DDF_VARIANT_GENERIC;
@@ -317,10 +320,7 @@ at::Tensor ddf_up(at::Tensor features, std::vector<at::Tensor> channel_filters,
         assertion_error("expected " + std::to_string(branches) + " channel filters followed by " +
                         std::to_string(branches) + " spatial filters");
     if (!features.is_cuda()) assertion_error("input feature must be a CUDA tensor.");
-    int combine;
-    if (kernel_combine == "mul") combine = DDF_MUL;
-    else if (kernel_combine == "add") combine = DDF_ADD;
-    else assertion_error("only support mul or add combination, instead of " + kernel_combine);
+    const int combine = combine_code(kernel_combine);
     if ((kernel_size - 1) % 2 != 0 || kernel_size < 1 || dilation < 1) assertion_error("");
     at::ScalarType dtype = features.scalar_type();
     for (const auto *list : {&channel_filters, &spatial_filters})
@@ -428,17 +428,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::class_<PackPlan>(m, "PackPlan")
         .def(py::init<std::shared_ptr<ModuleGuard>, std::vector<at::Tensor>, c10::optional<at::Tensor>,
                       c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>, double, double,
-                      int, int, int, int, const std::string &, bool, bool>())
-        .def("valid", [](const PackPlan &p) { return p.guard->holds(); });
+                      int64_t, int, int, int, int, const std::string &, bool, bool>())
+        .def("valid", [](const PackPlan &p) { return p.guard && p.guard->holds(); })
+        .def("misfit", &PackPlan::misfit, "why the branch kernels cannot run these features, or None");
     m.def("pack_forward", &pack_forward, "DDFPack.forward through a plan, or None");
     m.def("pack_infer", &pack_infer,
-          "DDFPack.forward without gradients: spatial branch (pooling on the way where it can), "
-          "channel branch, operator");
+          "DDFPack.forward without gradients, refusing with an error what the kernels do not take");
     py::class_<NetPlan>(m, "NetPlan")
         .def(py::init<std::shared_ptr<ModuleGuard>>())
         .def("set_ends", &NetPlan::set_ends)
         .def("add_block", &NetPlan::add_block)
-        .def("valid", [](const NetPlan &p) { return p.guard->holds(); });
+        .def("valid", [](const NetPlan &p) { return p.guard->holds(); })
+        .def("misfit", &NetPlan::misfit, "why the native inference cannot run this input, or None");
     m.def("net_forward", &net_forward, "DDFResNet.forward through a plan, or None");
     m.def("library_version", []() { return ddf_hip_version(); });
 }

@@ -145,7 +145,8 @@ class DDFResNet(nn.Module):
                     all(_is_plain_norm(m) for m in (block.bn1, block.bn2, block.bn3)) and
                     all(type(m) is nn.ReLU for m in (block.act1, block.act2, block.act3)) and
                     type(pack) is DDFPack and pack.kernel_size == 3 and pack.dilation == 1 and pack.head == 1 and
-                    pack.stride in (1, 2) and pack._stock_spatial_branch() and pack._stock_channel_branch()):
+                    pack.stride in (1, 2) and pack.kernel_combine in ('mul', 'add') and
+                    pack._stock_spatial_branch() and pack._stock_channel_branch()):
                 return False
             width, norm = block.conv1.out_channels, pack.spatial_branch[1]
             if (norm.runing_std or norm.runing_mean or width not in (64, 128, 256, 512) or
@@ -187,7 +188,8 @@ class DDFResNet(nn.Module):
             return args
 
         identity = nn.Identity()
-        plan.set_ends(layer(self.conv1, self.bn1), layer(self.fc, identity))
+        plan.set_ends(layer(self.conv1, self.bn1), layer(self.fc, identity), self.fc.in_features,
+                      self.fc.out_features)
         for block in self._blocks():
             pack, down = block.conv2, block.downsample
             conv, sp_norm = pack.spatial_branch
@@ -198,7 +200,8 @@ class DDFResNet(nn.Module):
             plan.add_block(
                 layer(block.conv1, block.bn1), layer(None, block.bn2), layer(block.conv3, block.bn3),
                 ([None] * 6, 0.0) if down is None else layer(down[0], down[1] if len(down) > 1 else identity), branches,
-                sp_norm.std, 1.0 if ch_norm.runing_std else ch_norm.std, pack.stride, pack.kernel_combine)
+                sp_norm.std, 1.0 if ch_norm.runing_std else ch_norm.std, pack.stride, pack.kernel_combine,
+                block.conv1.in_channels, block.conv1.out_channels, block.conv3.out_channels, fc1.out_channels)
         if not guard.covers(tensors):
             return None
         slot.plan = plan

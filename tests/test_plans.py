@@ -156,3 +156,80 @@ def test_a_changed_network_has_no_plan(change, before, ext, monkeypatch):
     NET_CHANGES[change](m, monkeypatch)
     assert before or not plan.valid()
     assert m._native_plan(ext) is None
+
+
+def _strided(t):
+    """The same values, every second element of a larger tensor."""
+    wide = torch.zeros(t.shape + (2,), dtype=t.dtype, device=t.device)
+    wide[..., 0] = t.detach()
+    return wide[..., 0]
+
+
+def _set(module, name, value):
+    setattr(module, name, torch.nn.Parameter(value))
+
+
+LAYER_MISFITS = {
+    'heads': (lambda: ddfnet_amd.DDFPack(16, head=3), lambda m: None),
+    'strided weight': (None, lambda m: _set(m.channel_branch[1], 'weight', _strided(m.channel_branch[1].weight))),
+    'strided in place': (None, lambda m: setattr(m.channel_branch[3].weight, 'data', _strided(m.channel_branch[3].weight))),
+    'spatial width': (None, lambda m: _set(m.spatial_branch[0], 'weight', torch.ones(9, 8, 1, 1))),
+    'hidden width': (None, lambda m: _set(m.channel_branch[1], 'weight', torch.ones(5, 16, 1, 1))),
+    'taps': (None, lambda m: _set(m.channel_branch[3], 'weight', torch.ones(9 * 8, 3, 1, 1))),
+    'spatial bias': (None, lambda m: _set(m.spatial_branch[0], 'bias', torch.ones(8))),
+    'hidden bias': (None, lambda m: _set(m.channel_branch[1], 'bias', torch.ones(2))),
+    'taps bias': (None, lambda m: setattr(m.channel_branch[3].bias, 'data', torch.ones(9 * 15))),
+    'gain': (None, lambda m: _set(m.channel_branch[4], 'std', torch.ones(9 * 15))),
+    'normalised channels': (None, lambda m: setattr(m.channel_branch[4], 'in_channels', 8)),
+    'type': (None, lambda m: m.channel_branch[1].half()),
+}
+
+
+@pytest.mark.parametrize('what', LAYER_MISFITS)
+def test_a_plan_does_not_run_what_does_not_fit(what, ext):
+    make, change = LAYER_MISFITS[what]
+    m = make() if make else ddfnet_amd.DDFPack(16)
+    x = torch.ones(2, 16, 6, 6)
+    if make is None:
+        assert m._native_plan(ext).misfit(x) is None
+        assert m._native_plan(ext).misfit(x[:, :8]) is not None
+        assert m._native_plan(ext).misfit(x.double()) is not None
+    change(m)
+    assert m._native_plan(ext).misfit(x) is not None
+
+
+def test_an_unknown_combination_has_no_plan(ext):
+    m = ddfnet_amd.DDFPack(16)
+    m._native_plan(ext)
+    m.kernel_combine = 'max'
+    assert m._native_plan(ext) is None
+    with pytest.raises(AssertionError, match='only support mul or add'):
+        m._pack_plan(ext)
+    net = small_net()
+    net._native_plan(ext)
+    net.layer3[0].conv2.kernel_combine = 'max'
+    assert net._native_plan(ext) is None
+
+
+NET_MISFITS = {
+    'resized in place': lambda m: setattr(m.layer1[0].conv3.weight, 'data', torch.ones(256, 32, 1, 1).half()),
+    'norm': lambda m: _set(m.layer2[0].bn2, 'weight', torch.ones(64).half()),
+    'statistics': lambda m: setattr(m.bn1, 'running_mean', torch.ones(32).half()),
+    'taps': lambda m: _set(m.layer1[0].conv2.spatial_branch[0], 'weight', torch.ones(8, 64, 1, 1).half()),
+    'strided': lambda m: _set(m.layer4[0].conv1, 'weight', _strided(m.layer4[0].conv1.weight)),
+    'classifier': lambda m: _set(m.fc, 'weight', torch.ones(15, 2048).half()),
+    'type': lambda m: m.fc.float(),
+}
+
+
+@pytest.mark.parametrize('what', NET_MISFITS)
+def test_a_network_plan_does_not_run_what_does_not_fit(what, ext):
+    m = small_net()
+    x = torch.ones(1, 3, 64, 64).half()
+    with torch.no_grad():
+        assert m._native_plan(ext).misfit(x) is None
+        for other in (x.float(), x[:, :2], x[:, :, :60], x[:0]):
+            assert m._native_plan(ext).misfit(other) is not None
+        NET_MISFITS[what](m)
+        assert m._native_plan(ext).misfit(x) is not None
+    assert m._native_plan(ext).misfit(x) is not None

@@ -85,3 +85,51 @@ def test_appended_modules_and_replaced_methods_take_part():
         assert torch.equal(net(image), want)
         net.layer1[0].act3.forward = lambda y: y * 0
         close(net(image), zeroed, 2e-2)
+
+
+def test_what_inference_refused_it_refuses():
+    x = torch.randn(2, 64, 8, 8, device='cuda')
+    with torch.no_grad():
+        with pytest.raises(RuntimeError, match='heads'):
+            ddfnet_amd.DDFPack(64, head=3).cuda()(x)
+        layer = ddfnet_amd.DDFPack(64).cuda()
+        layer(x)
+        layer.kernel_combine = 'max'
+        with pytest.raises(AssertionError, match='only support mul or add'):
+            layer(x)
+        layer = ddfnet_amd.DDFPack(64).cuda()
+        layer(x)
+        weight = layer.channel_branch[1].weight
+        weight.data = torch.stack([weight.data, weight.data], -1)[..., 0]
+        with pytest.raises(RuntimeError, match='contiguous'):
+            layer(x)
+        layer = ddfnet_amd.DDFPack(64).cuda()
+        layer(x)
+        layer.spatial_branch[0].weight.data = torch.randn(9, 32, 1, 1, device='cuda')
+        with pytest.raises(RuntimeError, match='fit'):
+            layer(x)
+        layer = ddfnet_amd.DDFPack(64).cuda()
+        layer(x)
+        layer.channel_branch[3].bias.data = torch.randn(9 * 63, device='cuda')
+        with pytest.raises(RuntimeError, match='fit'):
+            layer(x)
+    layer = ddfnet_amd.DDFPack(64).cuda()
+    layer(x)
+    layer.kernel_combine = 'max'
+    with pytest.raises(AssertionError, match='only support mul or add'):
+        layer(x)
+
+
+def test_resized_parameters_of_a_network_are_refused_by_their_modules():
+    net = small_net().cuda()
+    x = torch.randn(1, 3, 64, 64, device='cuda').half()
+    with torch.no_grad():
+        net(x)
+        net.layer1[0].conv3.weight.data = torch.ones(256, 32, 1, 1, device='cuda').half()
+        with pytest.raises(RuntimeError):
+            net(x)
+        net = small_net().cuda()
+        net(x)
+        net.layer1[0].conv2.kernel_combine = 'max'
+        with pytest.raises(AssertionError, match='only support mul or add'):
+            net(x)
