@@ -84,7 +84,10 @@ struct NetPlan {
     // (parameters may have been resized, moved or re-laid in place), or null.
     const char *misfit(const at::Tensor &x) const {
         if (x.scalar_type() != at::kHalf || x.dim() != 4 || x.size(1) != 3) return "images in fp16 expected";
-        if (x.size(0) < 1 || x.size(0) > 65535 || x.size(2) % 32 || x.size(3) % 32 || x.numel() == 0)
+        // (2^27 pixels: 32-bit offsets inside a sample of the stem and of the widest activation
+        // under a 3 x 3, twice the channels at a quarter of the image's rows and columns)
+        if (x.size(0) < 1 || x.size(0) > 65535 || x.size(2) % 32 || x.size(3) % 32 || x.numel() == 0 ||
+            x.size(2) * x.size(3) >= (int64_t(1) << 27))
             return "image sizes not covered";
         const bool grad = at::GradMode::is_enabled();
         if (grad && x.requires_grad()) return "gradients wanted";
@@ -98,6 +101,13 @@ struct NetPlan {
         return nullptr;
     }
 };
+
+// A call whose sizes the library refuses, before or between launches.
+struct NotCovered {};
+inline void covered(int status) {
+    if (status == DDF_ERR_UNSUPPORTED) throw NotCovered();
+    check_status(status);
+}
 
 // Logits, or None where the plan does not (any longer) describe the network or the native
 // path does not cover the call.
@@ -134,41 +144,43 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
     void *sf = q + 2 * wide_b + 2 * narrow_b, *cf = static_cast<char *>(sf) + taps_b;
     float *pp = reinterpret_cast<float *>(static_cast<char *>(cf) + filters_b);
     at::Tensor logits = new_tensor({n, p.fc.t[0].size(0)}, at::kHalf, dev);
-    {
+    try {
         py::gil_scoped_release release;    // (a network's launches take a while)
         ddf_net_norm_t nm = p.stem.norm();
-        check_status(ddf_hip_net_stem(x.data_ptr(), p.stem.t[0].data_ptr(), &nm, cur, n, h0, w0, st));
+        covered(ddf_hip_net_stem(x.data_ptr(), p.stem.t[0].data_ptr(), &nm, cur, n, h0, w0, st));
         int64_t h = h0 / 4, w = w0 / 4, c = 64;
         for (const NetBlock &b : p.blocks) {
             const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0].size(0);
             nm = b.conv1.norm();
-            check_status(ddf_hip_net_conv(cur, b.conv1.t[0].data_ptr(), &nm, nullptr, t1, n, h, w, c, width, 1, 1, st));
+            covered(ddf_hip_net_conv(cur, b.conv1.t[0].data_ptr(), &nm, nullptr, t1, n, h, w, c, width, 1, 1, st));
             int n_parts = 0;
-            check_status(ddf_hip_net_spatial(t1, b.ws.data_ptr(), ptr_or_null(b.bs), sf, pp, &n_parts, n, h, w, width,
+            covered(ddf_hip_net_spatial(t1, b.ws.data_ptr(), ptr_or_null(b.bs), sf, pp, &n_parts, n, h, w, width,
                                              b.stride, b.sgain, st));
-            check_status(ddf_hip_channel_branch_parts(
+            covered(ddf_hip_channel_branch_parts(
                 pp, n_parts, 1.0 / (double)(h * w), b.w1.data_ptr(), ptr_or_null(b.b1), b.w2.data_ptr(),
                 ptr_or_null(b.b2), cf, n, width, b.mid, 3, b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset),
                 DDF_F16, st));
             nm = b.bn2.norm();
-            check_status(ddf_hip_net_filter(t1, cf, sf, &nm, t2, n, h, w, width, b.stride, b.combine, st));
+            covered(ddf_hip_net_filter(t1, cf, sf, &nm, t2, n, h, w, width, b.stride, b.combine, st));
             nm = b.conv3.norm();
             if (b.down.t[0].defined()) {
                 const ddf_net_norm_t down = b.down.norm();
-                check_status(ddf_hip_net_conv_pair(t2, b.conv3.t[0].data_ptr(), &nm, width, cur,
+                covered(ddf_hip_net_conv_pair(t2, b.conv3.t[0].data_ptr(), &nm, width, cur,
                                                    b.down.t[0].data_ptr(), &down, h, w, c, b.stride, other, n, wide_c, 1,
                                                    st));
                 std::swap(cur, other);
             } else {
-                check_status(ddf_hip_net_conv(t2, b.conv3.t[0].data_ptr(), &nm, cur, cur, n, ho, wo, width, wide_c, 1, 1,
+                covered(ddf_hip_net_conv(t2, b.conv3.t[0].data_ptr(), &nm, cur, cur, n, ho, wo, width, wide_c, 1, 1,
                                               st));
             }
             h = ho; w = wo; c = wide_c;
         }
-        check_status(ddf_hip_net_pool(cur, other, n, h * w, c, st));
+        covered(ddf_hip_net_pool(cur, other, n, h * w, c, st));
         nm = p.fc.norm();
-        check_status(ddf_hip_net_conv(other, p.fc.t[0].data_ptr(), &nm, nullptr, logits.data_ptr(), n, 1, 1, c,
+        covered(ddf_hip_net_conv(other, p.fc.t[0].data_ptr(), &nm, nullptr, logits.data_ptr(), n, 1, 1, c,
                                       logits.size(1), 1, 0, st));
+    } catch (const NotCovered &) {
+        return py::none();    // (the modules run; what was written so far is dropped)
     }
     return py::cast(logits);
 }

@@ -233,3 +233,16 @@ def test_a_network_plan_does_not_run_what_does_not_fit(what, ext):
         NET_MISFITS[what](m)
         assert m._native_plan(ext).misfit(x) is not None
     assert m._native_plan(ext).misfit(x) is not None
+
+
+@pytest.mark.parametrize('k', [3, 5, 7, 9])
+def test_a_plan_only_for_filter_sizes_of_the_branch_kernels(k, ext):
+    assert (ddfnet_amd.DDFPack(16, kernel_size=k)._native_plan(ext) is not None) == (k in (3, 5))
+
+
+def test_images_past_the_kernels_limit_do_not_fit(ext):
+    net = small_net()
+    one = torch.zeros(1, dtype=torch.float16)
+    with torch.no_grad():
+        assert net._native_plan(ext).misfit(one.expand(1, 3, 8192, 16384)) is not None
+        assert net._native_plan(ext).misfit(one.expand(1, 3, 8192, 16352)) is None

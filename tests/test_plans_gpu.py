@@ -133,3 +133,25 @@ def test_resized_parameters_of_a_network_are_refused_by_their_modules():
         net.layer1[0].conv2.kernel_combine = 'max'
         with pytest.raises(AssertionError, match='only support mul or add'):
             net(x)
+
+
+@pytest.mark.parametrize('k', [7, 9])
+@pytest.mark.parametrize('dtype,tol', [(torch.float32, 1e-4), (torch.float16, 1e-2)])
+def test_filter_sizes_past_the_branch_kernels_in_inference(k, dtype, tol):
+    torch.manual_seed(4)
+    layer = ddfnet_amd.DDFPack(16, kernel_size=k).cuda().to(dtype)
+    x = torch.randn(2, 16, 12, 10, device='cuda').to(dtype)
+    with torch.no_grad():
+        close(layer(x), by_modules(layer, x), tol)
+
+
+def test_a_network_whose_hidden_layer_no_kernel_takes_runs_by_modules():
+    torch.manual_seed(5)
+    net = small_net().cuda()
+    branch = net.layer1[0].conv2.channel_branch
+    branch[1] = torch.nn.Conv2d(64, 16384, 1).cuda().half()
+    branch[3] = torch.nn.Conv2d(16384, 9 * 64, 1).cuda().half()
+    x = torch.randn(1, 3, 64, 64, device='cuda').half()
+    ext = ddfnet_amd.functional.extension()
+    with torch.no_grad():
+        assert net._native_plan(ext) is not None and ext.net_forward(net._native_plan(ext), x) is None
