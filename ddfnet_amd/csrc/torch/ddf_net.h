@@ -9,10 +9,10 @@ namespace ddf_torch {
 // A convolution with what follows it: (weight, conv bias, BatchNorm weight, bias, running
 // mean, running variance); missing ones undefined.
 struct NetLayer {
-    at::Tensor t[6];
+    TensorRef t[6];
     ddf_net_norm_t norm() const {
-        auto p = [](const at::Tensor &x) -> const void * { return x.defined() ? x.data_ptr() : nullptr; };
-        return ddf_net_norm_t{p(t[2]), p(t[3]), p(t[4]), p(t[5]), p(t[1]), eps};
+        return ddf_net_norm_t{ptr_or_null(t[2]), ptr_or_null(t[3]), ptr_or_null(t[4]), ptr_or_null(t[5]),
+                              ptr_or_null(t[1]), eps};
     }
     float eps = 0.f;
 };
@@ -20,32 +20,42 @@ struct NetLayer {
 struct NetBlock {
     NetLayer conv1, conv3, down;
     NetLayer bn2;                 // (no convolution of its own)
-    at::Tensor ws, bs, w1, b1, w2, b2, cgain, coffset;
+    TensorRef ws, bs, w1, b1, w2, b2, cgain, coffset;
     double sgain, cgain_const;
     int stride, combine;
     int64_t width, mid;
 };
 
-using NetLayerArgs = std::pair<std::vector<c10::optional<at::Tensor>>, double>;
+using NetLayerArgs = std::pair<py::list, double>;
 
 struct NetPlan {
-    std::shared_ptr<ModuleGuard> guard;
+    Refs refs;
+    ModuleGuard *guard;              // (owned by refs)
     NetLayer stem, fc;
     std::vector<NetBlock> blocks;
     // every tensor and the sizes it must have
-    std::vector<std::pair<at::Tensor, std::vector<int64_t>>> all;
+    std::vector<std::pair<TensorRef, std::vector<int64_t>>> all;
 
-    explicit NetPlan(std::shared_ptr<ModuleGuard> guard_) : guard(std::move(guard_)) {}
-
-    void expect(const at::Tensor &t, std::vector<int64_t> sizes) {
+    explicit NetPlan(const py::object &guard_) : guard(guard_.cast<ModuleGuard *>()) { refs.add(guard_.ptr()); }
+    int traverse(visitproc visit, void *arg) const { return refs.traverse(visit, arg); }
+    void clear() {
+        guard = nullptr;
+        stem = fc = NetLayer();
+        blocks.clear();
+        all.clear();
+        refs.clear();
+    }
+    bool holds() const { return guard && guard->holds(); }
+    void expect(const TensorRef &t, std::vector<int64_t> sizes) {
         if (t.defined()) all.emplace_back(t, std::move(sizes));
     }
     // A convolution of these sizes (none: only what follows it) with what follows it.
     NetLayer layer(const NetLayerArgs &a, std::vector<int64_t> sizes, int64_t channels) {
         NetLayer l;
-        TORCH_CHECK(a.first.size() == 6, "six tensors per layer expected");
+        const std::vector<TensorRef> t = tensor_refs(refs, a.first);
+        TORCH_CHECK(t.size() == 6, "six tensors per layer expected");
         for (int i = 0; i < 6; ++i) {
-            if (a.first[i].has_value()) l.t[i] = *a.first[i];
+            l.t[i] = t[i];
             expect(l.t[i], i == 0 ? sizes : std::vector<int64_t>{channels});
         }
         l.eps = (float)a.second;
@@ -57,7 +67,7 @@ struct NetPlan {
     }
     // A bottleneck of `in` -> `width` -> `out` channels with `mid` hidden ones.
     void add_block(const NetLayerArgs &conv1, const NetLayerArgs &bn2, const NetLayerArgs &conv3,
-                   const NetLayerArgs &down, std::vector<c10::optional<at::Tensor>> branches, double sgain,
+                   const NetLayerArgs &down, const py::list &branches, double sgain,
                    double cgain, int stride, const std::string &combine, int64_t in, int64_t width, int64_t out,
                    int64_t mid) {
         NetBlock b;
@@ -65,12 +75,13 @@ struct NetPlan {
         b.bn2 = layer(bn2, {}, width);
         b.conv3 = layer(conv3, {out, width, 1, 1}, out);
         b.down = layer(down, {out, in, 1, 1}, out);
-        at::Tensor *const to[8] = {&b.ws, &b.bs, &b.w1, &b.b1, &b.w2, &b.b2, &b.cgain, &b.coffset};
+        TensorRef *const to[8] = {&b.ws, &b.bs, &b.w1, &b.b1, &b.w2, &b.b2, &b.cgain, &b.coffset};
         const std::vector<int64_t> sizes[8] = {{9, width, 1, 1}, {9}, {mid, width, 1, 1}, {mid}, {9 * width, mid, 1, 1},
                                                {9 * width}, {9 * width}, {9 * width}};
-        TORCH_CHECK(branches.size() == 8, "eight branch tensors expected");
+        const std::vector<TensorRef> t = tensor_refs(refs, branches);
+        TORCH_CHECK(t.size() == 8, "eight branch tensors expected");
         for (int i = 0; i < 8; ++i) {
-            if (branches[i].has_value()) *to[i] = *branches[i];
+            *to[i] = t[i];
             expect(*to[i], sizes[i]);
         }
         b.sgain = sgain; b.cgain_const = cgain;
@@ -92,7 +103,8 @@ struct NetPlan {
         const bool grad = at::GradMode::is_enabled();
         if (grad && x.requires_grad()) return "gradients wanted";
         const auto dev = x.device();
-        for (const auto &[t, sizes] : all) {
+        for (const auto &[ref, sizes] : all) {
+            const at::Tensor &t = *ref;
             if (t.scalar_type() != at::kHalf || t.device() != dev) return "parameters must be fp16 and with the images";
             if (t.sizes() != sizes) return "parameters do not fit each other";
             if (!t.is_contiguous() || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) return "parameters must be laid out densely";
@@ -112,7 +124,7 @@ inline void covered(int status) {
 // Logits, or None where the plan does not (any longer) describe the network or the native
 // path does not cover the call.
 inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
-    if (!input.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || !p.guard->holds() || p.misfit(input))
+    if (!input.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || !p.holds() || p.misfit(input))
         return py::none();
     const auto dev = input.device();
     const at::Tensor x = input.contiguous();
@@ -129,7 +141,7 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
         for (const NetBlock &b : p.blocks) {
             const int64_t ho = h / b.stride, wo = w / b.stride;
             narrow = std::max(narrow, n * h * w * b.width);
-            wide = std::max(wide, n * ho * wo * b.conv3.t[0].size(0));
+            wide = std::max(wide, n * ho * wo * b.conv3.t[0]->size(0));
             taps = std::max(taps, n * ho * wo * 12);
             filters = std::max(filters, n * b.width * 9);
             parts = std::max(parts, n * b.width * 8);
@@ -143,21 +155,21 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
     void *cur = q, *other = q + wide_b, *t1 = q + 2 * wide_b, *t2 = q + 2 * wide_b + narrow_b;
     void *sf = q + 2 * wide_b + 2 * narrow_b, *cf = static_cast<char *>(sf) + taps_b;
     float *pp = reinterpret_cast<float *>(static_cast<char *>(cf) + filters_b);
-    at::Tensor logits = new_tensor({n, p.fc.t[0].size(0)}, at::kHalf, dev);
+    at::Tensor logits = new_tensor({n, p.fc.t[0]->size(0)}, at::kHalf, dev);
     try {
         py::gil_scoped_release release;    // (a network's launches take a while)
         ddf_net_norm_t nm = p.stem.norm();
-        covered(ddf_hip_net_stem(x.data_ptr(), p.stem.t[0].data_ptr(), &nm, cur, n, h0, w0, st));
+        covered(ddf_hip_net_stem(x.data_ptr(), p.stem.t[0]->data_ptr(), &nm, cur, n, h0, w0, st));
         int64_t h = h0 / 4, w = w0 / 4, c = 64;
         for (const NetBlock &b : p.blocks) {
-            const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0].size(0);
+            const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0]->size(0);
             nm = b.conv1.norm();
-            covered(ddf_hip_net_conv(cur, b.conv1.t[0].data_ptr(), &nm, nullptr, t1, n, h, w, c, width, 1, 1, st));
+            covered(ddf_hip_net_conv(cur, b.conv1.t[0]->data_ptr(), &nm, nullptr, t1, n, h, w, c, width, 1, 1, st));
             int n_parts = 0;
-            covered(ddf_hip_net_spatial(t1, b.ws.data_ptr(), ptr_or_null(b.bs), sf, pp, &n_parts, n, h, w, width,
+            covered(ddf_hip_net_spatial(t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, pp, &n_parts, n, h, w, width,
                                              b.stride, b.sgain, st));
             covered(ddf_hip_channel_branch_parts(
-                pp, n_parts, 1.0 / (double)(h * w), b.w1.data_ptr(), ptr_or_null(b.b1), b.w2.data_ptr(),
+                pp, n_parts, 1.0 / (double)(h * w), b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(),
                 ptr_or_null(b.b2), cf, n, width, b.mid, 3, b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset),
                 DDF_F16, st));
             nm = b.bn2.norm();
@@ -165,19 +177,19 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             nm = b.conv3.norm();
             if (b.down.t[0].defined()) {
                 const ddf_net_norm_t down = b.down.norm();
-                covered(ddf_hip_net_conv_pair(t2, b.conv3.t[0].data_ptr(), &nm, width, cur,
-                                                   b.down.t[0].data_ptr(), &down, h, w, c, b.stride, other, n, wide_c, 1,
+                covered(ddf_hip_net_conv_pair(t2, b.conv3.t[0]->data_ptr(), &nm, width, cur,
+                                                   b.down.t[0]->data_ptr(), &down, h, w, c, b.stride, other, n, wide_c, 1,
                                                    st));
                 std::swap(cur, other);
             } else {
-                covered(ddf_hip_net_conv(t2, b.conv3.t[0].data_ptr(), &nm, cur, cur, n, ho, wo, width, wide_c, 1, 1,
+                covered(ddf_hip_net_conv(t2, b.conv3.t[0]->data_ptr(), &nm, cur, cur, n, ho, wo, width, wide_c, 1, 1,
                                               st));
             }
             h = ho; w = wo; c = wide_c;
         }
         covered(ddf_hip_net_pool(cur, other, n, h * w, c, st));
         nm = p.fc.norm();
-        covered(ddf_hip_net_conv(other, p.fc.t[0].data_ptr(), &nm, nullptr, logits.data_ptr(), n, 1, 1, c,
+        covered(ddf_hip_net_conv(other, p.fc.t[0]->data_ptr(), &nm, nullptr, logits.data_ptr(), n, 1, 1, c,
                                       logits.size(1), 1, 0, st));
     } catch (const NotCovered &) {
         return py::none();    // (the modules run; what was written so far is dropped)

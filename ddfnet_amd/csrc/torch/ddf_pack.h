@@ -19,28 +19,39 @@ inline size_t aligned_bytes(size_t n) { return (n + kAlign - 1) / kAlign * kAlig
 // checked that both branches are the stock ones): with a guard once, for calls through
 // pack_forward, or without for a single call of pack_infer.
 struct PackPlan {
-    std::shared_ptr<ModuleGuard> guard;
+    Refs refs;
+    ModuleGuard *guard = nullptr;    // (owned by refs; null: a plan for one call)
     // 1x1 convolutions (weight, bias): spatial branch, first and second of the channel branch
-    at::Tensor ws, bs, w1, b1, w2, b2;
+    TensorRef ws, bs, w1, b1, w2, b2;
     // FilterNorm: learned gains and offsets, or the constant gain
-    c10::optional<at::Tensor> sgain_vec, soffset_vec, cgain_vec, coffset_vec;
+    TensorRef sgain_vec, soffset_vec, cgain_vec, coffset_vec;
     double sgain, cgain;
     int64_t channels;     // that the channel filters are normalised by
     int k, d, s, head, combine;
     bool fuse_pool, fuse_norm;
 
-    PackPlan(std::shared_ptr<ModuleGuard> guard_, std::vector<at::Tensor> convs,
-             c10::optional<at::Tensor> sgain_vec_, c10::optional<at::Tensor> soffset_vec_,
-             c10::optional<at::Tensor> cgain_vec_, c10::optional<at::Tensor> coffset_vec_, double sgain_,
-             double cgain_, int64_t channels_, int k_, int d_, int s_, int head_, const std::string &combine_,
-             bool fuse_pool_, bool fuse_norm_)
-        : guard(std::move(guard_)), sgain_vec(std::move(sgain_vec_)),
-          soffset_vec(std::move(soffset_vec_)), cgain_vec(std::move(cgain_vec_)),
-          coffset_vec(std::move(coffset_vec_)), sgain(sgain_), cgain(cgain_), channels(channels_), k(k_), d(d_), s(s_),
-          head(head_), combine(combine_code(combine_)), fuse_pool(fuse_pool_), fuse_norm(fuse_norm_) {
-        TORCH_CHECK(convs.size() == 6, "six convolution tensors expected");
-        ws = convs[0]; bs = convs[1]; w1 = convs[2]; b1 = convs[3]; w2 = convs[4]; b2 = convs[5];
+    // tensors: those ten
+    PackPlan(const py::object &guard_, const py::list &tensors, double sgain_, double cgain_, int64_t channels_, int k_,
+             int d_, int s_, int head_, const std::string &combine_, bool fuse_pool_, bool fuse_norm_)
+        : sgain(sgain_), cgain(cgain_), channels(channels_), k(k_), d(d_), s(s_), head(head_),
+          combine(combine_code(combine_)), fuse_pool(fuse_pool_), fuse_norm(fuse_norm_) {
+        TORCH_CHECK(tensors.size() == 10, "ten tensors expected");
+        const std::vector<TensorRef> t = tensor_refs(refs, tensors);
+        TORCH_CHECK(t[0].defined() && t[2].defined() && t[4].defined(), "weights expected");
+        ws = t[0]; bs = t[1]; w1 = t[2]; b1 = t[3]; w2 = t[4]; b2 = t[5];
+        sgain_vec = t[6]; soffset_vec = t[7]; cgain_vec = t[8]; coffset_vec = t[9];
+        if (!guard_.is_none()) {
+            guard = guard_.cast<ModuleGuard *>();
+            refs.add(guard_.ptr());
+        }
     }
+    int traverse(visitproc visit, void *arg) const { return refs.traverse(visit, arg); }
+    void clear() {
+        guard = nullptr;
+        for (TensorRef *t : {&ws, &bs, &w1, &b1, &w2, &b2, &sgain_vec, &soffset_vec, &cgain_vec, &coffset_vec}) *t = {};
+        refs.clear();
+    }
+    bool holds() const { return guard && guard->holds(); }
     // Why the branch kernels cannot run these features with the plan's tensors as they are now
     // (parameters may have been resized, moved or re-laid in place), or null.
     const char *misfit(const at::Tensor &x) const {
@@ -49,46 +60,39 @@ struct PackPlan {
         const int64_t c = x.size(1), kk = (int64_t)k * k;
         if (head < 1 || c % head != 0) return "channels must divide into heads";
         if (channels != c) return "the channel filters' normalisation does not fit the features";
-        for (const at::Tensor *t : {&ws, &w1, &w2})
-            if (t->dim() != 4 || t->size(2) != 1 || t->size(3) != 1) return "branch weights do not fit the features";
-        const int64_t mid = w1.size(0);
-        if (ws.size(0) != head * kk || ws.size(1) != c || w1.size(1) != c || w2.size(0) != c * kk || w2.size(1) != mid)
+        for (const TensorRef *t : {&ws, &w1, &w2})
+            if ((*t)->dim() != 4 || (*t)->size(2) != 1 || (*t)->size(3) != 1) return "branch weights do not fit the features";
+        const int64_t mid = w1->size(0);
+        if (ws->size(0) != head * kk || ws->size(1) != c || w1->size(1) != c || w2->size(0) != c * kk || w2->size(1) != mid)
             return "branch weights do not fit the features";
         const char *why = nullptr;
-        auto ask = [&](const at::Tensor &t, int64_t count) {
+        auto ask = [&](const TensorRef &t, int64_t count) {
             if (why || !t.defined()) return;
-            if (t.scalar_type() != type || t.device() != dev) why = "parameters must be of the features' type and device";
-            else if (!t.is_contiguous()) why = "weights must be contiguous";
-            else if (t.numel() != count) why = "branch parameters do not fit the features";
+            if (t->scalar_type() != type || t->device() != dev) why = "parameters must be of the features' type and device";
+            else if (!t->is_contiguous()) why = "weights must be contiguous";
+            else if (t->numel() != count) why = "branch parameters do not fit the features";
         };
         ask(ws, head * kk * c); ask(bs, head * kk);
         ask(w1, mid * c); ask(b1, mid);
         ask(w2, c * kk * mid); ask(b2, c * kk);
-        ask(sgain_vec.value_or(at::Tensor()), head * kk); ask(soffset_vec.value_or(at::Tensor()), head * kk);
-        ask(cgain_vec.value_or(at::Tensor()), c * kk); ask(coffset_vec.value_or(at::Tensor()), c * kk);
+        ask(sgain_vec, head * kk); ask(soffset_vec, head * kk);
+        ask(cgain_vec, c * kk); ask(coffset_vec, c * kk);
         return why;
     }
     bool wants_gradients(const at::Tensor &x) const {
         if (x.requires_grad()) return true;
-        for (const at::Tensor *t : {&ws, &bs, &w1, &b1, &w2, &b2})
-            if (t->defined() && t->requires_grad()) return true;
-        for (const auto *t : {&sgain_vec, &soffset_vec, &cgain_vec, &coffset_vec})
-            if (t->has_value() && (*t)->requires_grad()) return true;
+        for (const TensorRef *t : {&ws, &bs, &w1, &b1, &w2, &b2, &sgain_vec, &soffset_vec, &cgain_vec, &coffset_vec})
+            if (t->defined() && (*t)->requires_grad()) return true;
         return false;
     }
 };
-
-inline const void *ptr_or_null(const c10::optional<at::Tensor> &t) {
-    return t.has_value() && t->defined() ? t->data_ptr() : nullptr;
-}
-inline const void *ptr_or_null(const at::Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 // Without gradients: spatial branch (leaving the planes' partial sums where its kernel
 // can), channel branch, operator.  (The caller has asked misfit.)
 inline at::Tensor pack_run(const PackPlan &p, const at::Tensor &features) {
     const int dt = dtype_code(features.scalar_type());
     const at::Tensor x = features.contiguous();
-    const int64_t b = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3), mid = p.w1.size(0);
+    const int64_t b = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3), mid = p.w1->size(0);
     const int64_t ho = h / p.s, wo = w / p.s, kk = (int64_t)p.k * p.k;
     c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
     hipStream_t st = current_stream(x);
@@ -108,12 +112,12 @@ inline at::Tensor pack_run(const PackPlan &p, const at::Tensor &features) {
         float *parts = reinterpret_cast<float *>(base + cf_bytes + sf_bytes);
         int n_parts = 0;
         const int rc = ddf_hip_spatial_branch_pool(
-            x.data_ptr(), p.ws.data_ptr(), ptr_or_null(p.bs), sf, parts, cap, &n_parts, b, c, h, w, p.head, p.k, p.s,
+            x.data_ptr(), p.ws->data_ptr(), ptr_or_null(p.bs), sf, parts, cap, &n_parts, b, c, h, w, p.head, p.k, p.s,
             p.sgain, ptr_or_null(p.sgain_vec), ptr_or_null(p.soffset_vec), dt, st);
         if (rc != DDF_ERR_UNSUPPORTED) {
             check_status(rc);
             check_status(ddf_hip_channel_branch_parts(
-                parts, n_parts, 1.0 / (double)(h * w), p.w1.data_ptr(), ptr_or_null(p.b1), p.w2.data_ptr(),
+                parts, n_parts, 1.0 / (double)(h * w), p.w1->data_ptr(), ptr_or_null(p.b1), p.w2->data_ptr(),
                 ptr_or_null(p.b2), cf, b, c, mid, p.k, p.cgain, ptr_or_null(p.cgain_vec),
                 ptr_or_null(p.coffset_vec), dt, st));
             pooled_on_the_way = true;
@@ -122,10 +126,10 @@ inline at::Tensor pack_run(const PackPlan &p, const at::Tensor &features) {
     if (!pooled_on_the_way) {
         const at::Tensor pooled = at::mean(x, {2, 3});
         check_status(ddf_hip_channel_branch(
-            pooled.data_ptr(), p.w1.data_ptr(), ptr_or_null(p.b1), p.w2.data_ptr(), ptr_or_null(p.b2), cf, b, c, mid,
+            pooled.data_ptr(), p.w1->data_ptr(), ptr_or_null(p.b1), p.w2->data_ptr(), ptr_or_null(p.b2), cf, b, c, mid,
             p.k, p.cgain, ptr_or_null(p.cgain_vec), ptr_or_null(p.coffset_vec), dt, st));
         check_status(ddf_hip_spatial_branch(
-            x.data_ptr(), p.ws.data_ptr(), ptr_or_null(p.bs), sf, b, c, h, w, p.head, p.k, p.s, p.sgain,
+            x.data_ptr(), p.ws->data_ptr(), ptr_or_null(p.bs), sf, b, c, h, w, p.head, p.k, p.s, p.sgain,
             ptr_or_null(p.sgain_vec), ptr_or_null(p.soffset_vec), dt, st));
     }
     // heads are folded into the batch: (b * head, c / head, h, w)
@@ -251,7 +255,7 @@ inline at::Tensor pack_infer(const PackPlan &p, const at::Tensor &x) {
 // DDFPack.forward through a plan: the result, or None where the plan does not (any longer)
 // describe the layer or the native path does not cover the call.
 inline py::object pack_forward(const PackPlan &p, const at::Tensor &x) {
-    if (!p.guard || !p.guard->holds() || !x.is_cuda() || x.dim() != 4) return py::none();
+    if (!p.holds() || !x.is_cuda() || x.dim() != 4) return py::none();
     const int dt = dtype_code(x.scalar_type());
     // (a size the stride does not divide fails in the layer's own code, as in the reference
     // at ddf/ddf.py:215-218)
@@ -260,18 +264,20 @@ inline py::object pack_forward(const PackPlan &p, const at::Tensor &x) {
     if (!(at::GradMode::is_enabled() && p.wants_gradients(x))) return py::cast(pack_run(p, x));
     // Training: the stock configuration only (constant spatial gain, learned channel gain, no
     // offsets, biases present), everything trained.
-    if (!p.fuse_norm || p.sgain_vec || p.soffset_vec || p.coffset_vec || !p.cgain_vec) return py::none();
-    for (const at::Tensor *t : {&p.ws, &p.bs, &p.w1, &p.b1, &p.w2, &p.b2})
-        if (!t->defined() || !t->requires_grad()) return py::none();
-    if (!p.cgain_vec->requires_grad() || at::autocast::is_autocast_enabled(at::kCUDA)) return py::none();
+    if (!p.fuse_norm || p.sgain_vec.defined() || p.soffset_vec.defined() || p.coffset_vec.defined() ||
+        !p.cgain_vec.defined())
+        return py::none();
+    for (const TensorRef *t : {&p.ws, &p.bs, &p.w1, &p.b1, &p.w2, &p.b2, &p.cgain_vec})
+        if (!t->defined() || !(*t)->requires_grad()) return py::none();
+    if (at::autocast::is_autocast_enabled(at::kCUDA)) return py::none();
     if (x.numel() == 0) return py::none();
     // (the streaming kernel's addresses: weights in whole words, features in whole vectors)
     const bool covered =
-        reinterpret_cast<uintptr_t>(p.ws.data_ptr()) % 4 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-        ddf_hip_pack_backward_workspace_bytes(x.size(0), x.size(1), x.size(2), x.size(3), p.w1.size(0), p.head, p.k,
+        reinterpret_cast<uintptr_t>(p.ws->data_ptr()) % 4 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+        ddf_hip_pack_backward_workspace_bytes(x.size(0), x.size(1), x.size(2), x.size(3), p.w1->size(0), p.head, p.k,
                                               p.s, dt) > 0;
     if (!covered) return py::none();
-    return py::cast(PackAutograd::apply(x.contiguous(), p.ws, p.bs, p.w1, p.b1, p.w2, p.b2, *p.cgain_vec, p.sgain,
+    return py::cast(PackAutograd::apply(x.contiguous(), *p.ws, *p.bs, *p.w1, *p.b1, *p.w2, *p.b2, *p.cgain_vec, p.sgain,
                                         (int64_t)p.k, (int64_t)p.d, (int64_t)p.s, (int64_t)p.head,
                                         (int64_t)p.combine));
 }

@@ -421,24 +421,23 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def(py::init([](py::dict classes, py::dict own, py::tuple operators, py::tuple silent) {
             return ModuleGuard::Rules{classes, own, operators, silent};
         }));
-    py::class_<ModuleGuard, std::shared_ptr<ModuleGuard>>(m, "ModuleGuard")
+    py::class_<ModuleGuard>(m, "ModuleGuard", py::custom_type_setup(collectable<ModuleGuard>))
         .def("holds", &ModuleGuard::holds)
         .def("covers", &ModuleGuard::covers);
     m.def("guard_of", &ModuleGuard::make, "a guard of modules (the first is the owner), or None");
-    py::class_<PackPlan>(m, "PackPlan")
-        .def(py::init<std::shared_ptr<ModuleGuard>, std::vector<at::Tensor>, c10::optional<at::Tensor>,
-                      c10::optional<at::Tensor>, c10::optional<at::Tensor>, c10::optional<at::Tensor>, double, double,
-                      int64_t, int, int, int, int, const std::string &, bool, bool>())
-        .def("valid", [](const PackPlan &p) { return p.guard && p.guard->holds(); })
+    py::class_<PackPlan>(m, "PackPlan", py::custom_type_setup(collectable<PackPlan>))
+        .def(py::init<py::object, py::list, double, double, int64_t, int, int, int, int, const std::string &, bool,
+                      bool>())
+        .def("valid", &PackPlan::holds)
         .def("misfit", &PackPlan::misfit, "why the branch kernels cannot run these features, or None");
     m.def("pack_forward", &pack_forward, "DDFPack.forward through a plan, or None");
     m.def("pack_infer", &pack_infer,
           "DDFPack.forward without gradients, refusing with an error what the kernels do not take");
-    py::class_<NetPlan>(m, "NetPlan")
-        .def(py::init<std::shared_ptr<ModuleGuard>>())
+    py::class_<NetPlan>(m, "NetPlan", py::custom_type_setup(collectable<NetPlan>))
+        .def(py::init<py::object>())
         .def("set_ends", &NetPlan::set_ends)
         .def("add_block", &NetPlan::add_block)
-        .def("valid", [](const NetPlan &p) { return p.guard->holds(); })
+        .def("valid", &NetPlan::holds)
         .def("misfit", &NetPlan::misfit, "why the native inference cannot run this input, or None");
     m.def("net_forward", &net_forward, "DDFResNet.forward through a plan, or None");
     m.def("library_version", []() { return ddf_hip_version(); });

@@ -18,6 +18,8 @@
 
 #include <torch/extension.h>
 
+#include <torch/csrc/autograd/python_variable.h>
+
 #include <algorithm>
 #include <memory>
 #include <unordered_set>
@@ -35,6 +37,75 @@ constexpr bool kDictStamps = false;
 inline uint64_t stamp_of(PyObject *) { return 0; }
 #endif
 
+// Python objects that something native owns, known to the cycle collector by `traverse` and
+// `clear` (see collectable): a module tree may lead back to whoever holds on to it.
+class Refs {
+public:
+    Refs() = default;
+    Refs(const Refs &) = delete;
+    Refs &operator=(const Refs &) = delete;
+    ~Refs() { clear(); }
+    PyObject *add(PyObject *o) {
+        Py_XINCREF(o);
+        if (o) objects_.push_back(o);
+        return o;
+    }
+    int traverse(visitproc visit, void *arg) const {
+        for (PyObject *o : objects_) Py_VISIT(o);
+        return 0;
+    }
+    void clear() {
+        std::vector<PyObject *> gone;
+        gone.swap(objects_);
+        for (PyObject *o : gone) Py_DECREF(o);
+    }
+
+private:
+    std::vector<PyObject *> objects_;
+};
+
+// pybind11::custom_type_setup of a class whose `traverse` and `clear` are those of its Refs.
+template <class T>
+void collectable(PyHeapTypeObject *heap_type) {
+    PyTypeObject *type = &heap_type->ht_type;
+    type->tp_flags |= Py_TPFLAGS_HAVE_GC;
+    type->tp_traverse = [](PyObject *self, visitproc visit, void *arg) -> int {
+        Py_VISIT(Py_TYPE(self));
+        auto at = reinterpret_cast<py::detail::instance *>(self)->get_value_and_holder();
+        return at.holder_constructed() ? static_cast<const T *>(at.value_ptr())->traverse(visit, arg) : 0;
+    };
+    type->tp_clear = [](PyObject *self) -> int {
+        auto at = reinterpret_cast<py::detail::instance *>(self)->get_value_and_holder();
+        if (at.holder_constructed()) static_cast<T *>(at.value_ptr())->clear();
+        return 0;
+    };
+}
+
+// A tensor by its Python object (that some Refs owns; null: none).  The collector sees through
+// an owned Python object, which it does not through an at::Tensor.
+class TensorRef {
+public:
+    TensorRef() = default;
+    explicit TensorRef(PyObject *o) : o_(o) {
+        TORCH_CHECK(!o || THPVariable_Check(o), "tensors expected");
+    }
+    bool defined() const { return o_ != nullptr; }
+    const at::Tensor &operator*() const { return THPVariable_Unpack(o_); }
+    const at::Tensor *operator->() const { return &THPVariable_Unpack(o_); }
+
+private:
+    PyObject *o_ = nullptr;
+};
+// The objects of a list, owned by `refs`; None: no tensor.
+inline std::vector<TensorRef> tensor_refs(Refs &refs, const py::list &objects) {
+    std::vector<TensorRef> out;
+    for (auto o : objects) out.emplace_back(o.is_none() ? nullptr : refs.add(o.ptr()));
+    return out;
+}
+inline const void *ptr_or_null(const TensorRef &t) { return t.defined() ? t->data_ptr() : nullptr; }
+
+// Of the module a plan is made for the guard keeps no more than a weak reference: the plan hangs
+// on that module, and a model goes with its last user, not at some later collection.
 class ModuleGuard {
 public:
     // What is fixed for the package, collected once (modules.py):
@@ -51,12 +122,11 @@ public:
 
     // A guard of `modules` (the first is the plan's owner), or null where they are not plain
     // modules of the classes known, or somebody listens.
-    static std::shared_ptr<ModuleGuard> make(const Rules &rules, const py::list &modules) {
-        std::shared_ptr<ModuleGuard> g(new ModuleGuard());
+    static std::unique_ptr<ModuleGuard> make(const Rules &rules, const py::list &modules) {
+        std::unique_ptr<ModuleGuard> g(new ModuleGuard());
         for (auto item : rules.operators) {
-            py::tuple t = py::reinterpret_borrow<py::tuple>(item);
-            g->keep_.append(t);
-            g->operators_.push_back({t[0].ptr(), t[1].ptr(), t[2].ptr()});
+            PyObject *t = g->keep_.add(item.ptr());
+            g->operators_.push_back({PyTuple_GetItem(t, 0), PyTuple_GetItem(t, 1), PyTuple_GetItem(t, 2)});
         }
         for (auto d : rules.silent) g->add_silent(d.ptr());
         bool first = true;
@@ -64,7 +134,8 @@ public:
             if (!g->add_module(rules, m.ptr(), first)) return nullptr;
             first = false;
         }
-        return g->holds() ? g : nullptr;
+        if (!g->holds()) g.reset();
+        return g;
     }
 
     // Every one of the objects is an entry of a module's tables or an attribute relied on (a
@@ -78,6 +149,10 @@ public:
     }
     // (caller holds the GIL)
     bool holds() const {
+        PyObject *owner = owner_ ? PyWeakref_GetObject(owner_) : Py_None;
+        if (owner == Py_None || Py_TYPE(owner) != owner_type_) return false;
+        PyObject **attributes = _PyObject_GetDictPtr(owner);
+        if (!attributes || *attributes != owner_attributes_) return false;
         for (const Entry &e : operators_)
             if (PyDict_GetItem(e.dict, e.key) != e.value) return false;
         for (PyObject *d : silent_)
@@ -93,6 +168,12 @@ public:
         return true;
     }
 
+    int traverse(visitproc visit, void *arg) const { return keep_.traverse(visit, arg); }
+    void clear() {
+        owner_ = nullptr;     // (never holds again)
+        keep_.clear();
+    }
+
 private:
     enum Kind { kTable, kAttributes, kClass };
     struct Entry { PyObject *dict, *key, *value; };
@@ -101,7 +182,7 @@ private:
         PyObject *dict;
         Kind kind;
         int first, count;            // kTable: pairs_ of its entries; kAttributes: of those relied on
-        int module = 0;              // kAttributes: index into modules_
+        PyTypeObject *type = nullptr;   // kAttributes: the module's class
         PyObject *tables[3] = {nullptr, nullptr, nullptr};
         PyObject *hiding = nullptr;  // kAttributes of the owner: methods not to be hidden (else: any)
         mutable uint64_t stamp;
@@ -112,7 +193,7 @@ private:
     ModuleGuard() = default;
 
     void add_silent(PyObject *d) {
-        keep_.append(py::reinterpret_borrow<py::object>(d));
+        keep_.add(d);
         silent_.push_back(d);
     }
     bool add_module(const Rules &rules, PyObject *m, bool owner) {
@@ -121,21 +202,29 @@ private:
         for (Py_ssize_t i = 0; !rule && i < PyTuple_GET_SIZE(mro); ++i)
             rule = PyDict_GetItem(rules.classes.ptr(), PyTuple_GET_ITEM(mro, i));
         PyObject **slot = _PyObject_GetDictPtr(m);
-        if (!rule || !slot || !*slot) return false;
+        if (!rule || !PyTuple_Check(rule) || !slot || !*slot) return false;
         PyObject *attributes = *slot;
         PyObject *own = nullptr;
         for (Py_ssize_t i = 0; owner && !own && i < PyTuple_GET_SIZE(mro); ++i)
             own = PyDict_GetItem(rules.own.ptr(), PyTuple_GET_ITEM(mro, i));
         if (owner && !own) return false;
-        keep_.append(py::reinterpret_borrow<py::object>(m));
-        keep_.append(py::reinterpret_borrow<py::object>(attributes));
-        modules_.push_back({m, type});
+        if (owner) {
+            py::object ref = py::reinterpret_steal<py::object>(PyWeakref_NewRef(m, nullptr));
+            if (!ref) throw py::error_already_set();
+            owner_ = keep_.add(ref.ptr());
+            owner_type_ = type;
+            owner_attributes_ = attributes;
+        } else {
+            keep_.add(m);
+            keep_.add(attributes);
+            modules_.push_back({m, type});
+        }
         if (!add_class(type, PyTuple_GET_ITEM(rule, 1), own)) return false;
 
         Watch w;
         w.dict = attributes;
         w.kind = kAttributes;
-        w.module = (int)modules_.size() - 1;
+        w.type = type;
         w.hiding = own;
         w.first = (int)pairs_.size();
         auto rely_on = [&](PyObject *key) {
@@ -185,7 +274,7 @@ private:
         for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(methods); ++i) {
             PyObject *pair = PyTuple_GET_ITEM(methods, i), *name = PyTuple_GET_ITEM(pair, 0);
             if (own && PySequence_Contains(own, name) != 1) continue;
-            keep_.append(py::reinterpret_borrow<py::object>(pair));
+            keep_.add(pair);
             methods_.push_back({type, name, PyTuple_GET_ITEM(pair, 1)});
             if (!as_known(methods_.back())) return false;
         }
@@ -195,7 +284,7 @@ private:
             if (t == &PyBaseObject_Type || !t->tp_dict) continue;
             const auto seen = [&](const Watch &w) { return w.dict == t->tp_dict; };
             if (std::any_of(watches_.begin(), watches_.end(), seen)) continue;
-            keep_.append(py::reinterpret_borrow<py::object>(reinterpret_cast<PyObject *>(t)));
+            keep_.add(reinterpret_cast<PyObject *>(t));
             Watch w;
             w.dict = t->tp_dict;
             w.kind = kClass;
@@ -206,8 +295,8 @@ private:
         return true;
     }
     void add_pair(PyObject *key, PyObject *value) {
-        keep_.append(py::reinterpret_borrow<py::object>(key));
-        keep_.append(py::reinterpret_borrow<py::object>(value));
+        keep_.add(key);
+        keep_.add(value);
         pairs_.push_back({key, value});
     }
 
@@ -219,7 +308,7 @@ private:
         for (PyObject *table : w.tables)
             if (PyDict_Contains(table, key) != 0) return true;
         if (w.hiding) return PySequence_Contains(w.hiding, key) != 0;
-        return _PyType_Lookup(modules_[w.module].type, key) != nullptr;
+        return _PyType_Lookup(w.type, key) != nullptr;
     }
     bool same(const Watch &w) const {
         if (w.kind == kClass) return std::all_of(methods_.begin(), methods_.end(), as_known);
@@ -250,7 +339,10 @@ private:
         return *names;
     }
 
-    py::list keep_;                    // owns every reference below
+    Refs keep_;                        // owns what is below, but for the owner's attributes
+    PyObject *owner_ = nullptr;        // weak reference
+    PyTypeObject *owner_type_ = nullptr;
+    PyObject *owner_attributes_ = nullptr;
     std::vector<Entry> operators_;
     std::vector<PyObject *> silent_;
     std::vector<Typed> modules_;

@@ -1,6 +1,8 @@
 """When the native plan of a layer or network may be used: everything that needs no GPU
 (a plan is made of tensors wherever they live; only running it needs the device)."""
 import copy
+import gc
+import weakref
 
 import pytest
 import torch
@@ -246,3 +248,35 @@ def test_images_past_the_kernels_limit_do_not_fit(ext):
     with torch.no_grad():
         assert net._native_plan(ext).misfit(one.expand(1, 3, 8192, 16384)) is not None
         assert net._native_plan(ext).misfit(one.expand(1, 3, 8192, 16352)) is None
+
+
+@pytest.mark.parametrize('make', kinds(), ids=['layer', 'network'])
+def test_a_planned_module_goes_with_its_last_user(make, ext):
+    """... at once, as any module does; and at a collection where its parts lead back to it."""
+    gc.collect()
+    gc.disable()
+    try:
+        module = make()
+        assert module._native_plan(ext).valid()
+        for m in module.modules():
+            if isinstance(m, ddfnet_amd.DDFPack):
+                assert m._native_plan(ext).valid()
+        gone = [weakref.ref(t) for t in list(module.modules()) + list(module.parameters())]
+        m = None
+        del module
+        assert not any(ref() is not None for ref in gone)
+        module = make()
+        plan = module._native_plan(ext)
+        del module
+        assert not plan.valid()
+    finally:
+        gc.enable()
+    module = make()
+    first = next(m for m in module.modules() if isinstance(m, torch.nn.Conv2d))
+    first.owner = module
+    first.weight.owner = module
+    assert module._native_plan(ext).valid()
+    gone = [weakref.ref(t) for t in list(module.modules()) + list(module.parameters())]
+    del module, first
+    gc.collect()
+    assert not any(ref() is not None for ref in gone)
