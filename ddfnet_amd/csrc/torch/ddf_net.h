@@ -101,14 +101,15 @@ struct NetPlan {
             x.size(2) * x.size(3) >= (int64_t(1) << 27))
             return "image sizes not covered";
         const bool grad = at::GradMode::is_enabled();
-        if (grad && x.requires_grad()) return "gradients wanted";
+        if ((grad && x.requires_grad()) || has_tangent(x)) return "gradients wanted";
         const auto dev = x.device();
         for (const auto &[ref, sizes] : all) {
             const at::Tensor &t = *ref;
             if (t.scalar_type() != at::kHalf || t.device() != dev) return "parameters must be fp16 and with the images";
             if (t.sizes() != sizes) return "parameters do not fit each other";
             if (!t.is_contiguous() || reinterpret_cast<uintptr_t>(t.data_ptr()) % 16) return "parameters must be laid out densely";
-            if (grad && t.requires_grad()) return "gradients wanted";
+            if ((grad && t.requires_grad()) || has_tangent(t)) return "gradients wanted";
+            if (t.unsafeGetTensorImpl()->is_python_dispatch()) return "parameters must be plain tensors";
         }
         return nullptr;
     }
@@ -124,7 +125,8 @@ inline void covered(int status) {
 // Logits, or None where the plan does not (any longer) describe the network or the native
 // path does not cover the call.
 inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
-    if (!input.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || !p.holds() || p.misfit(input))
+    if (!input.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || dispatch_watched(input) || !p.holds() ||
+        p.misfit(input))
         return py::none();
     const auto dev = input.device();
     const at::Tensor x = input.contiguous();

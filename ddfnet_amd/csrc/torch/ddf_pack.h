@@ -58,6 +58,7 @@ struct PackPlan {
         const auto type = x.scalar_type();
         const auto dev = x.device();
         const int64_t c = x.size(1), kk = (int64_t)k * k;
+        if (has_tangent(x)) return "the branch kernels have no forward-mode derivative";
         if (head < 1 || c % head != 0) return "channels must divide into heads";
         if (channels != c) return "the channel filters' normalisation does not fit the features";
         for (const TensorRef *t : {&ws, &w1, &w2})
@@ -69,6 +70,8 @@ struct PackPlan {
         auto ask = [&](const TensorRef &t, int64_t count) {
             if (why || !t.defined()) return;
             if (t->scalar_type() != type || t->device() != dev) why = "parameters must be of the features' type and device";
+            else if (t->unsafeGetTensorImpl()->is_python_dispatch()) why = "parameters must be plain tensors";
+            else if (has_tangent(*t)) why = "the branch kernels have no forward-mode derivative";
             else if (!t->is_contiguous()) why = "weights must be contiguous";
             else if (t->numel() != count) why = "branch parameters do not fit the features";
         };
@@ -255,7 +258,7 @@ inline at::Tensor pack_infer(const PackPlan &p, const at::Tensor &x) {
 // DDFPack.forward through a plan: the result, or None where the plan does not (any longer)
 // describe the layer or the native path does not cover the call.
 inline py::object pack_forward(const PackPlan &p, const at::Tensor &x) {
-    if (!p.holds() || !x.is_cuda() || x.dim() != 4) return py::none();
+    if (!p.holds() || !x.is_cuda() || x.dim() != 4 || dispatch_watched(x)) return py::none();
     const int dt = dtype_code(x.scalar_type());
     // (a size the stride does not divide fails in the layer's own code, as in the reference
     // at ddf/ddf.py:215-218)

@@ -9,14 +9,18 @@
 // library calls happen without the interpreter.
 #include <torch/extension.h>
 
+#include <ATen/FuncTorchTLS.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/VariableTypeUtils.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <sstream>
 #include <string>
@@ -82,6 +86,19 @@ inline at::Tensor new_tensor(c10::IntArrayRef sizes, at::ScalarType type, const 
 }
 
 inline bool has_tangent(const at::Tensor &t) { return torch::autograd::isFwGradDefined(t); }
+// No derivative is lost in silence: forward mode (whether or not gradients are recorded) and
+// torch.func's transforms are refused, as a torch::autograd::Function does.
+inline void refuse_transforms() {
+    if (const auto &tls = at::functorch::functorchTLSAccessor()) tls->checkSupportsCppAutogradFunction();
+}
+
+// Somebody takes part in what the dispatcher would see of this call and a launch does not show:
+// a tensor of a subclass with a dispatch of its own, a dispatch mode, torch.func, a tracer.
+inline bool dispatch_watched(const at::Tensor &t) {
+    return t.unsafeGetTensorImpl()->is_python_dispatch() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+           torch::jit::tracer::isTracing();
+}
 
 // The operator's gradient as a node of the autograd graph.  (A torch::autograd::Function
 // does the same through a generic context - argument lists, a dictionary of boxed values,
@@ -186,6 +203,10 @@ at::Tensor ddf(at::Tensor features, at::Tensor channel_filter, at::Tensor spatia
     else if (version == "f") variant = DDF_VARIANT_TILED;
     else assertion_error("version must be '', 'o' or 'f', instead of " + version);
 
+    refuse_transforms();
+    if (has_tangent(features) || has_tangent(channel_filter) || has_tangent(spatial_filter))
+        throw std::runtime_error("ddf has no forward-mode derivative");
+
     at::Tensor out = new_tensor({b, c, out_h, out_w}, dtype, features.device());
     {
         c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(features.device());
@@ -195,8 +216,6 @@ at::Tensor ddf(at::Tensor features, at::Tensor channel_filter, at::Tensor spatia
     }
     if (at::GradMode::is_enabled() &&
         (features.requires_grad() || channel_filter.requires_grad() || spatial_filter.requires_grad())) {
-        if (has_tangent(features) || has_tangent(channel_filter) || has_tangent(spatial_filter))
-            throw std::runtime_error("ddf has no forward-mode derivative");
         auto node = std::shared_ptr<DDFNode>(new DDFNode(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(features, channel_filter, spatial_filter));
         node->k = (int)kernel_size;

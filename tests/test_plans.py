@@ -280,3 +280,24 @@ def test_a_planned_module_goes_with_its_last_user(make, ext):
     del module, first
     gc.collect()
     assert not any(ref() is not None for ref in gone)
+
+
+def _dual(t):
+    return torch.autograd.forward_ad.make_dual(t, torch.ones_like(t))
+
+
+@pytest.mark.parametrize('make,shape', [(kinds()[0], (1, 16, 6, 6)), (kinds()[1], (1, 3, 64, 64))],
+                         ids=['layer', 'network'])
+@torch.no_grad()
+def test_a_plan_leaves_forward_mode_alone(make, shape, ext):
+    module = make()
+    x = torch.ones(shape, dtype=next(module.parameters()).dtype)
+    with torch.autograd.forward_ad.dual_level():
+        plan = module._native_plan(ext)
+        assert plan.misfit(x) is None
+        assert plan.misfit(_dual(x)) is not None
+        conv = next(m for m in module.modules() if isinstance(m, torch.nn.Conv2d))
+        weight = _dual(conv.weight)
+        conv._parameters['weight'] = weight
+        plan = module._native_plan(ext)
+        assert plan is None or plan.misfit(x) is not None

@@ -4,6 +4,7 @@ import copy
 
 import pytest
 import torch
+import torch.utils._python_dispatch
 
 import ddfnet_amd
 from test_plans import replica_of, small_net
@@ -155,3 +156,47 @@ def test_a_network_whose_hidden_layer_no_kernel_takes_runs_by_modules():
     ext = ddfnet_amd.functional.extension()
     with torch.no_grad():
         assert net._native_plan(ext) is not None and ext.net_forward(net._native_plan(ext), x) is None
+
+
+@pytest.mark.parametrize('grad', [False, True])
+def test_forward_mode_is_refused_and_not_dropped(grad):
+    x, cf, sf = (torch.randn(*s, device='cuda') for s in ((2, 16, 6, 6), (2, 16, 3, 3), (2, 9, 6, 6)))
+    layer = ddfnet_amd.DDFPack(16).cuda().requires_grad_(False)
+    net = small_net().cuda().requires_grad_(False)
+    image = torch.randn(1, 3, 64, 64, device='cuda').half()
+    fw = torch.autograd.forward_ad
+    with fw.dual_level(), torch.set_grad_enabled(grad):
+        for i in range(3):
+            ops = [fw.make_dual(t, torch.ones_like(t)) if i == j else t for j, t in enumerate((x, cf, sf))]
+            with pytest.raises(RuntimeError):
+                ddfnet_amd.ddf(*ops)
+        for module, data in ((layer, x), (net, image)):
+            module(data)
+            with pytest.raises(RuntimeError):
+                module(fw.make_dual(data, torch.ones_like(data)))
+
+
+def test_transforms_of_functions_are_refused():
+    x, cf, sf = (torch.randn(*s, device='cuda') for s in ((2, 16, 6, 6), (2, 16, 3, 3), (2, 9, 6, 6)))
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda t: ddfnet_amd.ddf(t, cf, sf))(x[None])
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: ddfnet_amd.ddf(t, cf, sf).sum())(x)
+
+
+def test_a_dispatch_mode_sees_a_networks_operators():
+    class Count(torch.utils._python_dispatch.TorchDispatchMode):
+        convolutions = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.convolutions += 'convolution' in func.name()
+            return func(*args, **(kwargs or {}))
+
+    net = small_net().cuda()
+    image = torch.randn(1, 3, 64, 64, device='cuda').half()
+    with torch.no_grad():
+        want = net(image)
+        with Count() as seen:
+            out = net(image)
+    assert seen.convolutions >= 13
+    close(out, want, 2e-2)
