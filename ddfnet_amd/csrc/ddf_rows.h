@@ -735,7 +735,10 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     // the spatial taps are regrouped once: sfp[r][i][e] = taps (i, 0) and (i, 1) of pixel
     // e, sfs[r][i][k] = tap (i, 2) of pixels 2k and 2k + 1.
     // (Stride 2, forward: result pixel e takes the feature pixels 2e - 1, 2e and 2e + 1.)
-    constexpr bool kDot2 = sizeof(T) == 2 && K == 3 && D == 1 && VX >= 2 && (S == 1 || !BWD);
+    // Not where rows are odd (TAIL == 2) or ragged under stride 2: comb(CF, SF) of those is fp32,
+    // as it is one pixel at a time and in the LDS-tile kernels, which share them.
+    constexpr bool kDot2 = sizeof(T) == 2 && K == 3 && D == 1 && VX >= 2 &&
+                           (TAIL == 0 ? (S == 1 || !BWD) : (TAIL == 1 && S == 1));
     uint32_t sfp[kDot2 ? R : 1][K][kDot2 ? VX : 1], sfs[kDot2 ? R : 1][K][NW];
     if constexpr (kDot2) {
 #pragma unroll

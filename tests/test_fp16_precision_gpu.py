@@ -1,0 +1,56 @@
+"""fp16 storage where every product and sum is fp32: the result is off by its own rounding and
+by fp32 sums, not by a rounded comb(CF, SF).
+
+Bound, per element: half a unit of the stored result, 2^-11 of it (2^-25 below fp16's normal
+range), and for ``terms`` fp32 products and additions 2^-23 of the sum of the terms' magnitudes
+each (a product rounds once, an addition once).  A combination rounded to fp16 is off by 2^-11
+of its term: with terms that cancel it misses the bound by far."""
+import pytest
+import torch
+
+from ddfnet_amd import _lib
+from ddf_testlib import random_case, run_ddf
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _ids(v):
+    return str(v).replace('torch.', '')
+
+
+def within(got, want, magnitude, terms):
+    want, got = want.double(), got.double().cpu()
+    bound = 2.0 ** -11 * want.abs() + 2.0 ** -25 + terms * 2.0 ** -23 * magnitude.double()
+    worst = ((got - want).abs() / bound).max().item()
+    assert worst <= 1, worst
+
+
+def magnitudes(x, cf, sf, go, k, d, s, combine):
+    """The sums with every term's magnitude in its place (CF and SF of 'add' apart)."""
+    a = [t.abs() for t in (x, cf, sf, go)]
+    return (oracle.forward(a[0], a[1], a[2], k, d, s, combine),
+            oracle.backward(a[3], a[0], a[1], a[2], k, d, s, combine)[0])
+
+
+def check(case, k, d, s, combine, need):
+    x, cf, sf, go = case
+    sum_out, sum_dx = magnitudes(x, cf, sf, go, k, d, s, combine)
+    out, dx, _, _ = run_ddf(x, cf, sf, go, k, d, s, combine, need=need)
+    within(out, oracle.forward(x, cf, sf, k, d, s, combine), sum_out, 2 * k * k)
+    if need[0]:
+        within(dx, oracle.backward(go, x, cf, sf, k, d, s, combine)[0], sum_dx, 2 * k * k)
+
+
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('shape,k,d,s', [
+    ((4, 256, 50, 75), 3, 1, 1),       # odd rows in vectors of four
+    ((4, 66, 113, 133), 3, 1, 1),
+    ((4, 64, 113, 265), 3, 1, 1),     # ... and cut into segments
+    ((2, 64, 49, 75), 3, 1, 2),        # stride 2 over odd planes
+    ((2, 64, 50, 78), 3, 1, 2)], ids=_ids)
+def test_forward_and_feature_gradient_alone(shape, k, d, s, combine):
+    if s == 1:
+        assert 'ragged' in _lib.describe(shape, k, d, s, combine, torch.float16)
+    check(random_case(*shape, k, s, torch.float16, seed=sum(shape)), k, d, s, combine, (True, False, False))
