@@ -76,8 +76,10 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
     constexpr int GROWS = DX ? (S == 2 ? 2 : ROWS) : R;
     constexpr int GOWN = DX && S == 1 ? HY : 0;
     constexpr bool kFilters = MUL || DX;       // CF and SF values are needed at all
-    // fp16 feature gradient: comb(CF, SF) of a pixel pair is formed by one packed fp16 operation
-    constexpr bool kPackedComb = sizeof(T) == 2 && DX && S == 1 && VX >= 2;
+    // fp16 feature gradient: comb(CF, SF) of a pixel pair is formed by one packed fp16 operation,
+    // i.e. rounded.  Not over rows that vectors do not divide: comb is fp32 there, as it is one
+    // pixel at a time and in the LDS-tile kernels, which share those rows.
+    constexpr bool kPackedComb = sizeof(T) == 2 && DX && S == 1 && VX >= 2 && TAIL == 0;
     constexpr int kVB = VX * sizeof(T), kXB = S * kVB;   // bytes of a dO / filter vector, of a feature vector
     constexpr int NW = vec_words(kVB), NWX = vec_words(kXB);
     constexpr int G = kFlushChannels;

@@ -54,3 +54,19 @@ def test_forward_and_feature_gradient_alone(shape, k, d, s, combine):
     if s == 1:
         assert 'ragged' in _lib.describe(shape, k, d, s, combine, torch.float16)
     check(random_case(*shape, k, s, torch.float16, seed=sum(shape)), k, d, s, combine, (True, False, False))
+
+
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('shape,d', [
+    ((4, 256, 50, 75), 1),             # odd rows
+    ((16, 64, 57, 58), 1),             # even ones of an odd number of pairs, an odd number of them
+    ((4, 66, 113, 134), 1),            # ... cut into segments
+    ((2, 16, 60, 131), 2),             # dilated
+    ((2, 16, 60, 130), 2)], ids=_ids)
+def test_feature_gradient_with_the_filters(shape, d, combine):
+    assert 'ragged' in _lib.describe(shape, 3, d, 1, combine, torch.float16, need=7)
+    case = random_case(*shape, 3, 1, torch.float16, seed=sum(shape))
+    _, magnitude = magnitudes(*case, 3, d, 1, combine)
+    x, cf, sf, go = case
+    _, dx, _, _ = run_ddf(x, cf, sf, go, 3, d, 1, combine)
+    within(dx, oracle.backward(go, x, cf, sf, 3, d, 1, combine)[0], magnitude, 18)
