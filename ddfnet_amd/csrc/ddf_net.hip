@@ -696,9 +696,10 @@ __global__ __launch_bounds__(WAVES * kWave) void k_net_spatial(const _Float16 *_
 // ahead of use.  The channel taps of the lane's channels stay in registers, tap-major in
 // pairs of channels; a pixel's nine spatial taps come with it.  comb(CF, SF) of two channels
 // is one packed fp16 operation (rounded like the operands), the sums are fp32: 13 vector
-// instructions per pixel and channel quarter.  A row outside the image, a column past its
-// ends and a walk past the last pixel read zeros through the buffer descriptor.
-template <int LP, int S, bool MUL>
+// instructions per pixel and channel quarter.  WIDE: comb in fp32, 18 instructions - for rows
+// of an odd length, where the operator's own kernels have it so.  A row outside the image, a
+// column past its ends and a walk past the last pixel read zeros through the buffer descriptor.
+template <int LP, int S, bool MUL, bool WIDE>
 __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restrict__ x,
                                                          const _Float16 *__restrict__ cf,
                                                          const _Float16 *__restrict__ sf, NetNorm norm,
@@ -785,10 +786,18 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const half2_t cv = __builtin_bit_cast(half2_t, cfp[t][k]);
-                    const half2_t cb = MUL ? cv * sv : cv + sv;
                     const half2_t xv = __builtin_bit_cast(half2_t, col[(A + j) % RING][i][k]);
-                    acc[2 * k] = fmaf((float)xv[0], (float)cb[0], acc[2 * k]);
-                    acc[2 * k + 1] = fmaf((float)xv[1], (float)cb[1], acc[2 * k + 1]);
+                    if constexpr (WIDE) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const float c1 = (float)cv[h], s1 = (float)sv[h];
+                            acc[2 * k + h] = fmaf((float)xv[h], MUL ? c1 * s1 : c1 + s1, acc[2 * k + h]);
+                        }
+                    } else {
+                        const half2_t cb = MUL ? cv * sv : cv + sv;
+                        acc[2 * k] = fmaf((float)xv[0], (float)cb[0], acc[2 * k]);
+                        acc[2 * k + 1] = fmaf((float)xv[1], (float)cb[1], acc[2 * k + 1]);
+                    }
                 }
             }
         half8_t o;
@@ -1019,16 +1028,19 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
         const _Float16 *xn = (const _Float16 *)x + n0 * H * W * C, *cn = (const _Float16 *)cf + n0 * C * 9,
                        *sn = (const _Float16 *)sf + n0 * Ho * Wo * kTapPitch;
         _Float16 *on = (_Float16 *)out + n0 * Ho * Wo * C;
+        const bool wide = Wo % 2 != 0;    // (128 x 7 x 7 x 512 under BatchNorm 7.9 us packed, 8.6 wide)
         bool done = false;
-#define DDF_NET_FILTER_LAUNCH(LP_, S_, MUL_)                                                                     \
-    hipLaunchKernelGGL((k_net_filter<LP_, S_, MUL_>), dim3(xcd_grid(blocks)), dim3(kThreads), 0, st, xn, cn, sn, \
-                       norm, on, (int)H, (int)W, (int)Ho, (int)Wo, (int)runs, run, (int)units, (int)blocks,      \
-                       (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2))
-#define DDF_NET_FILTER(LP_, S_)                            \
-    if (C == LP_ * 8 && stride == S_) {                    \
-        if (mul) DDF_NET_FILTER_LAUNCH(LP_, S_, true);     \
-        else DDF_NET_FILTER_LAUNCH(LP_, S_, false);        \
-        done = true;                                       \
+#define DDF_NET_FILTER_LAUNCH(LP_, S_, MUL_, WIDE_)                                                         \
+    hipLaunchKernelGGL((k_net_filter<LP_, S_, MUL_, WIDE_>), dim3(xcd_grid(blocks)), dim3(kThreads), 0, st, \
+                       xn, cn, sn, norm, on, (int)H, (int)W, (int)Ho, (int)Wo, (int)runs, run, (int)units,  \
+                       (int)blocks, (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2))
+#define DDF_NET_FILTER(LP_, S_)                                     \
+    if (C == LP_ * 8 && stride == S_) {                             \
+        if (wide && mul) DDF_NET_FILTER_LAUNCH(LP_, S_, true, true); \
+        else if (wide) DDF_NET_FILTER_LAUNCH(LP_, S_, false, true); \
+        else if (mul) DDF_NET_FILTER_LAUNCH(LP_, S_, true, false);  \
+        else DDF_NET_FILTER_LAUNCH(LP_, S_, false, false);          \
+        done = true;                                                \
     }
         DDF_NET_FILTER(8, 1) DDF_NET_FILTER(16, 1) DDF_NET_FILTER(32, 1) DDF_NET_FILTER(64, 1)
         DDF_NET_FILTER(8, 2) DDF_NET_FILTER(16, 2) DDF_NET_FILTER(32, 2) DDF_NET_FILTER(64, 2)

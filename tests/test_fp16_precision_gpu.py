@@ -10,6 +10,7 @@ import torch
 
 from ddfnet_amd import _lib
 from ddf_testlib import random_case, run_ddf
+from test_net_gpu import call
 
 import oracle
 
@@ -70,3 +71,20 @@ def test_feature_gradient_with_the_filters(shape, d, combine):
     x, cf, sf, go = case
     _, dx, _, _ = run_ddf(x, cf, sf, go, 3, d, 1, combine)
     within(dx, oracle.backward(go, x, cf, sf, 3, d, 1, combine)[0], magnitude, 18)
+
+
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('n,c,h,w,s', [(8, 512, 7, 7, 1), (8, 512, 14, 14, 2), (2, 64, 5, 9, 1), (3, 128, 11, 3, 1),
+                                       (2, 256, 6, 10, 2)], ids=_ids)
+def test_channels_last_filter_over_odd_rows(n, c, h, w, s, combine):
+    """The network's own kernel of the operator, nothing behind it but its ReLU."""
+    x, cf, sf, _ = random_case(n, c, h, w, 3, s, torch.float16, seed=c + w)
+    ho, wo = h // s, w // s
+    taps = torch.zeros(n, ho * wo, 12, dtype=torch.float16)
+    taps[:, :, :9] = sf.reshape(n, 9, ho * wo).permute(0, 2, 1)
+    out = torch.empty(n, ho, wo, c, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_filter', x.permute(0, 2, 3, 1).contiguous().cuda(), cf.cuda(), taps.cuda(), None, out, n, h, w,
+         c, s, _lib.COMBINE[combine])
+    a = [t.abs() for t in (x, cf, sf)]
+    want, magnitude = oracle.forward(x, cf, sf, 3, 1, s, combine), oracle.forward(*a, 3, 1, s, combine)
+    within(out.permute(0, 3, 1, 2), want.clamp_min(0), magnitude, 18)
