@@ -58,7 +58,8 @@ template <int V>
 struct Affine {
     typedef _Float16 vec __attribute__((ext_vector_type(V)));
     vec w, b, m, v, cb;
-    __device__ __forceinline__ void request(const NetNorm &n, int c) {
+    // bias: the convolution's is part of it.
+    __device__ __forceinline__ void request(const NetNorm &n, int c, bool bias = true) {
         auto get = [&](const void *p, _Float16 other) {
             vec r;
             if (p) __builtin_memcpy(&r, static_cast<const _Float16 *>(p) + c, sizeof(vec));
@@ -71,7 +72,7 @@ struct Affine {
         b = get(n.var ? n.bias : nullptr, (_Float16)0);
         m = get(n.var ? n.mean : nullptr, (_Float16)0);
         v = get(n.var, (_Float16)1);
-        cb = get(n.conv_bias, (_Float16)0);
+        cb = get(bias ? n.conv_bias : nullptr, (_Float16)0);
     }
     __device__ __forceinline__ void finish(const NetNorm &n, float (&scale)[V], float (&shift)[V]) const {
         const float eps = n.var ? n.eps : 0.f;
@@ -171,6 +172,9 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     };
     const int wm = wave & 1, wn = wave >> 1;
     const int l32 = lane & 31, hi = lane >> 5;
+    // Lane column of a 32x32 step's D = pixel l32, rows (channels) 8 * g + 4 * hi + 0..3 in
+    // registers 4g .. 4g+3.
+    auto channel = [&](int j, int g) { return wn * (BN / 2) + j * 32 + 8 * g + 4 * hi; };
     float16_t acc[TM][TN];
     auto clear = [&]() {
 #pragma unroll
@@ -181,6 +185,23 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
     };
     clear();
+    // Without a BatchNorm (the classifier) a bias is part of the sum, which is rounded once;
+    // under one the sum is rounded first, as a convolution's result is.
+    const bool bias_in_sum = !PAIR && !a.norm.var && a.norm.conv_bias;
+    if (bias_in_sum) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int c = n0 + channel(j, g);    // (rows are whole vectors of 8)
+                half4_t b = {0, 0, 0, 0};
+                if (c < a.N) __builtin_memcpy(&b, static_cast<const _Float16 *>(a.norm.conv_bias) + c, sizeof(b));
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)b[e];
+            }
+    }
     auto multiply = [&](int buf) {
         const _Float16 *s = net_smem + buf * STAGE;
 #pragma unroll
@@ -214,7 +235,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     Affine<8> aff;
     half8_t rv[RO];
     auto residual = [&]() {
-        aff.request(a.norm, cok ? c : 0);
+        aff.request(a.norm, cok ? c : 0, !bias_in_sum);
 #pragma unroll
         for (int i = 0; i < RO; ++i) {
             const int64_t m = m0 + tid / CPR + i * (kThreads / CPR);
@@ -222,15 +243,15 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             if (res) rv[i] = *reinterpret_cast<const half8_t *>(res + (m < a.M ? m : a.M - 1) * a.N + (cok ? c : 0));
         }
     };
-    // Lane column of a 32x32 step's D = pixel l32, rows (channels) 8 * g + 4 * hi + 0..3 in
-    // registers 4g .. 4g+3.
-    auto channel = [&](int j, int g) { return wn * (BN / 2) + j * 32 + 8 * g + 4 * hi; };
     half4_t side[PAIR ? TM : 1][PAIR ? TN : 1][PAIR ? 4 : 1];
-    auto affine_of = [&](int which, int i, int j, int g, float (&f)[4]) __attribute__((always_inline)) {
+    auto affine_of = [&](int which, bool bn, int i, int j, int g, float (&f)[4]) __attribute__((always_inline)) {
         const float4_t sc = *reinterpret_cast<const float4_t *>(&affine[which][channel(j, g)]);
         const float4_t sh = *reinterpret_cast<const float4_t *>(&affine[which + 1][channel(j, g)]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = fmaf((float)(_Float16)acc[i][j][4 * g + e], sc[e], sh[e]);
+        for (int e = 0; e < 4; ++e) {
+            const float sum = acc[i][j][4 * g + e];
+            f[e] = fmaf(bn ? (float)(_Float16)sum : sum, sc[e], sh[e]);
+        }
     };
 
     const int nk0 = PAIR ? first.K / KST : 0, nk = nk0 + a.K / KST;
@@ -281,7 +302,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
 #pragma unroll
                         for (int g = 0; g < 4; ++g) {
                             float f[4];
-                            affine_of(2, i, j, g, f);
+                            affine_of(2, first.norm.var != nullptr, i, j, g, f);
 #pragma unroll
                             for (int e = 0; e < 4; ++e) side[i][j][g][e] = (_Float16)f[e];
                         }
@@ -302,7 +323,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 half4_t v;
                 if constexpr (PAIR) {
                     float f[4];
-                    affine_of(0, i, j, g, f);
+                    affine_of(0, a.norm.var != nullptr, i, j, g, f);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         f[e] += (float)side[i][j][g][e];
@@ -404,7 +425,7 @@ __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tile
     float f = 0.f;
 #pragma unroll
     for (int k = 0; k < WAVES; ++k) f += red[k][tid & (T - 1)][tid / T];
-    f = fmaf((float)(_Float16)f, sc[0], sh[0]) + (float)rv;
+    f = fmaf(a.norm.var ? (float)(_Float16)f : f, sc[0], sh[0]) + (float)rv;    // (see k_net_conv)
     if (a.relu) f = relu(f);
     static_cast<_Float16 *>(a.out)[om * a.N + oc] = (_Float16)f;
 }

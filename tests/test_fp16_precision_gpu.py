@@ -10,7 +10,7 @@ import torch
 
 from ddfnet_amd import _lib
 from ddf_testlib import random_case, run_ddf
-from test_net_gpu import call
+from test_net_gpu import Norm, call
 
 import oracle
 
@@ -21,9 +21,10 @@ def _ids(v):
     return str(v).replace('torch.', '')
 
 
-def within(got, want, magnitude, terms):
+def within(got, want, magnitude, terms, stored=0.):
+    """stored: magnitudes of intermediate values that are fp16 by design."""
     want, got = want.double(), got.double().cpu()
-    bound = 2.0 ** -11 * want.abs() + 2.0 ** -25 + terms * 2.0 ** -23 * magnitude.double()
+    bound = 2.0 ** -11 * (want.abs() + stored) + 2.0 ** -25 + terms * 2.0 ** -23 * magnitude.double()
     worst = ((got - want).abs() / bound).max().item()
     assert worst <= 1, worst
 
@@ -88,3 +89,38 @@ def test_channels_last_filter_over_odd_rows(n, c, h, w, s, combine):
     a = [t.abs() for t in (x, cf, sf)]
     want, magnitude = oracle.forward(x, cf, sf, 3, 1, s, combine), oracle.forward(*a, 3, 1, s, combine)
     within(out.permute(0, 3, 1, 2), want.clamp_min(0), magnitude, 18)
+
+
+@pytest.mark.parametrize('n,c,o,residual', [
+    (1, 64, 10, False), (3, 128, 33, True),              # few pixels: 16 x 16 results per workgroup
+    (300, 64, 136, False), (300, 128, 64, True), (6000, 64, 200, False)], ids=_ids)   # tiles
+def test_bias_without_a_norm_is_part_of_the_sum(n, c, o, residual):
+    """The classifier's product: sums that its bias takes back to small values."""
+    g = torch.Generator().manual_seed(n)
+    x, w = torch.rand(n, c, generator=g).half() + 1, torch.rand(o, c, generator=g).half() + 1
+    sums = x.double() @ w.double().t()
+    bias = -sums.mean(0).half()
+    res = torch.randn(n, o, generator=g).half() if residual else None
+    keep = bias.cuda()
+    out = torch.empty(n, o, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_conv', x.cuda(), w.cuda(), Norm(conv_bias=keep.data_ptr()), None if res is None else res.cuda(),
+         out, n, 1, 1, c, o, 1, 0)
+    want = sums + bias.double() + (0 if res is None else res.double())
+    # (with a residual the tiles hand the sum on as fp16: one more rounding, of the sum)
+    within(out, want, (sums + bias.double().abs()), c + 1, (sums + bias.double()).abs() * bool(residual))
+
+
+def test_bias_without_a_norm_beside_a_projection():
+    g = torch.Generator().manual_seed(9)
+    n, c, side, o = 300, 64, 128, 256
+    x, w = torch.rand(n, c, generator=g).half() + 1, torch.rand(o, c, generator=g).half() + 1
+    xs, ws = torch.rand(n, side, generator=g).half() + 1, torch.rand(o, side, generator=g).half() + 1
+    sums, sides = x.double() @ w.double().t(), xs.double() @ ws.double().t()
+    b, bs = -sums.mean(0).half(), -sides.mean(0).half()
+    db, dbs = b.cuda(), bs.cuda()
+    out = torch.empty(n, o, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_conv_pair', x.cuda(), w.cuda(), Norm(conv_bias=db.data_ptr()), c, xs.cuda(), ws.cuda(),
+         Norm(conv_bias=dbs.data_ptr()), 1, 1, side, 1, out, n, o, 0)
+    want_side = sides + bs.double()
+    within(out, sums + b.double() + want_side, sums + sides + b.double().abs() + bs.double().abs(), c + side + 2,
+           want_side.abs())
