@@ -782,7 +782,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         for (int s = 0; s < NS; ++s) {
             const float tot = row_sum(p[s]);
             if (sl == 0 && m0 + seg < mid) {
-                const float hm = fmaxf(tot + bias, 0.f);
+                const float hm = relu(tot + bias);
                 h[s * mid + m0 + seg] = hm;
                 if (save.hidden && blockIdx.x == 0 && s < ns) save.hidden[(n0 + s) * mid + m0 + seg] = hm;
             }
@@ -1020,7 +1020,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
                 if (m < t * 16) continue;    // (the last tile's overlap: those rows belong to the tile before)
                 const float bias = b1 ? ld(b1 + m) : 0.f;
                 const int kt = min(m / kMmaStep, ktiles - 1);
-                const _Float16 hm = (_Float16)fmaxf(acc[e] + bias, 0.f);
+                const _Float16 hm = (_Float16)relu(acc[e] + bias);
                 hv[(kt * kMmaSamples + col) * kMmaStep + m - min(kt * kMmaStep, klast)] = hm;
                 if (save.hidden && blockIdx.x == 0 && n0 + col < N) save.hidden[(int64_t)(n0 + col) * mid + m] = (float)hm;
             }

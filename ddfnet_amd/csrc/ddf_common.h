@@ -43,6 +43,9 @@ __device__ __forceinline__ void st(double *p, double v) { *p = v; }
 template <bool MUL, typename A>
 __device__ __forceinline__ A comb(A a, A b) { return MUL ? a * b : a + b; }
 
+// (NaN stays NaN, as torch's ReLU has it)
+__device__ __forceinline__ float relu(float f) { return f < 0.f ? 0.f : f; }
+
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // The spatial filter normalisation behind the spatial-filter gradient (FilterNorm

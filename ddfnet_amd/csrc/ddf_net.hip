@@ -48,9 +48,6 @@ __device__ __forceinline__ int xcd_block(int block, int blocks) {
 }
 inline unsigned xcd_grid(int64_t blocks) { return (unsigned)(cdiv(blocks, kXcd) * kXcd); }
 
-// (NaN stays NaN, as torch's ReLU has it)
-__device__ __forceinline__ float relu(float f) { return f < 0.f ? 0.f : f; }
-
 // y = scale * x + shift of the convolution's bias and the BatchNorm behind it, for V
 // consecutive channels: requested as vectors early, worked out where they are needed.  (Read
 // channel by channel at the end of a kernel they cost more than small kernels do.)

@@ -316,7 +316,7 @@ __global__ __launch_bounds__(kThreads) void k_pack_hidden(PackDims d, const floa
 #pragma unroll
     for (int k = 1; k < kSumGroups; ++k) a += red[k][col];
     if (hid) {
-        dz1[i] = hidden[i] > 0.f ? a : 0.f;
+        dz1[i] = hidden[i] <= 0.f ? 0.f : a;    // (a hidden NaN passes its gradient on, as torch has it)
     } else {
         const int64_t weights = (int64_t)d.head * KK * d.C;
         if (i < weights) st(dws + i, a);
