@@ -431,8 +431,9 @@ __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tile
 // A workgroup produces 8 x 8 pooled pixels x 64 channels at a time: 17 x 17 convolution
 // results from 39 x 39 image pixels.  The image tile sits in LDS as [row][column][4
 // channels, the last one zero]: for a filter row the eight columns under a result are 32
-// contiguous values, one step of the 16x16x32 matrix instruction (the eighth column and the
-// fourth channel meet zero weights).  The weights stay in registers over the tiles a
+// contiguous values, one step of the 16x16x32 matrix instruction (the fourth channel, zeros,
+// and the eighth column, cleared after the read lest an infinity in it make a NaN, meet zero
+// weights).  The weights stay in registers over the tiles a
 // workgroup walks.  Convolution results never leave LDS (205 MB at batch 128).
 constexpr int kPoolTile = 8, kConvTile = 2 * kPoolTile + 1, kImgRows = 2 * (kConvTile - 1) + 7, kImgCols = kImgRows + 1;
 constexpr int kConvPitch = 64 + 8, kStemOut = 64;
@@ -449,6 +450,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int row = lane & 15, quad = lane >> 4;
     const int Hc = H / 2, Wc = W / 2, Hp = Hc / 2, Wp = Wc / 2;
+    const uint32_t last_column = quad == 3 ? 0u : ~0u;    // (columns 2 * quad and 2 * quad + 1 of eight)
     // weights to LDS as [output][filter row][column * 4 + channel], then to registers
     {
         constexpr int COUNT = kStemOut * 147, R = (COUNT + kThreads - 1) / kThreads;
@@ -523,7 +525,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
             for (int ct = 0; ct < 4; ++ct) acc[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ky = 0; ky < 7; ++ky) {
-                const half8_t b = *reinterpret_cast<const half8_t *>(src + ky * kImgCols * 4);
+                rows_u4 words = *reinterpret_cast<const rows_u4 *>(src + ky * kImgCols * 4);
+                words[2] &= last_column;
+                words[3] &= last_column;
+                const half8_t b = __builtin_bit_cast(half8_t, words);
 #pragma unroll
                 for (int ct = 0; ct < 4; ++ct)
                     acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[ct][ky], b, acc[ct], 0, 0, 0);
