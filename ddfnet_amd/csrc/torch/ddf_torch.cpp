@@ -444,6 +444,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("holds", &ModuleGuard::holds)
         .def("covers", &ModuleGuard::covers);
     m.def("guard_of", &ModuleGuard::make, "a guard of modules (the first is the owner), or None");
+    py::class_<ModuleSnapshot>(m, "ModuleSnapshot", py::custom_type_setup(collectable<ModuleSnapshot>))
+        .def(py::init<const ModuleGuard::Rules &, py::list>())
+        .def("holds", &ModuleSnapshot::holds);
     py::class_<PackPlan>(m, "PackPlan", py::custom_type_setup(collectable<PackPlan>))
         .def(py::init<py::object, py::list, double, double, int64_t, int, int, int, int, const std::string &, bool,
                       bool>())

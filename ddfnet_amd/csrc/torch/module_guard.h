@@ -104,6 +104,12 @@ inline std::vector<TensorRef> tensor_refs(Refs &refs, const py::list &objects) {
 }
 inline const void *ptr_or_null(const TensorRef &t) { return t.defined() ? t->data_ptr() : nullptr; }
 
+inline std::vector<PyObject *> interned(std::initializer_list<const char *> names) {
+    std::vector<PyObject *> out;
+    for (const char *name : names) out.push_back(PyUnicode_InternFromString(name));
+    return out;
+}
+
 // Of the module a plan is made for the guard keeps no more than a weak reference: the plan hangs
 // on that module, and a model goes with its last user, not at some later collection.
 class ModuleGuard {
@@ -235,23 +241,20 @@ private:
         PyObject *names = PyTuple_GET_ITEM(rule, 0);
         for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(names); ++i) rely_on(PyTuple_GET_ITEM(names, i));
         for (int i = 0; i < 3; ++i) {
-            PyObject *table = rely_on(table_names()[i].ptr());
+            PyObject *table = rely_on(table_names()[i]);
             // (an ordered dictionary keeps an order of its own)
             if (!table || !PyDict_CheckExact(table)) return false;
             w.tables[i] = table;
         }
         if (!owner)
-            for (const py::str &name : hook_names()) {
-                PyObject *hooks = rely_on(name.ptr());
+            for (PyObject *name : hook_names()) {
+                PyObject *hooks = rely_on(name);
                 if (!hooks) continue;
                 if (!PyDict_Check(hooks)) return false;
                 add_silent(hooks);
             }
         w.count = (int)pairs_.size() - w.first;
-        Py_ssize_t pos = 0;
-        PyObject *key, *value;
-        while (PyDict_Next(attributes, &pos, &key, &value))
-            if (hides(w, key)) return false;
+        if (hides(w)) return false;
         w.stamp = stamp_of(attributes);
         watches_.push_back(w);
 
@@ -260,7 +263,8 @@ private:
             t.dict = table;
             t.kind = kTable;
             t.first = (int)pairs_.size();
-            pos = 0;
+            Py_ssize_t pos = 0;
+            PyObject *key, *value;
             while (PyDict_Next(table, &pos, &key, &value)) add_pair(key, value);
             t.count = (int)pairs_.size() - t.first;
             t.stamp = stamp_of(table);
@@ -304,11 +308,19 @@ private:
         return _PyType_Lookup(m.type, m.name) == m.value;
     }
     // An attribute by which the module is not the one its class and tables describe.
-    bool hides(const Watch &w, PyObject *key) const {
+    static bool hides(const Watch &w) {
+        PyObject *key, *value;
         for (PyObject *table : w.tables)
-            if (PyDict_Contains(table, key) != 0) return true;
-        if (w.hiding) return PySequence_Contains(w.hiding, key) != 0;
-        return _PyType_Lookup(w.type, key) != nullptr;
+            for (Py_ssize_t pos = 0; PyDict_Next(table, &pos, &key, &value);)
+                if (PyDict_Contains(w.dict, key) != 0) return true;
+        if (w.hiding) {
+            for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(w.hiding); ++i)
+                if (PyDict_Contains(w.dict, PyTuple_GET_ITEM(w.hiding, i)) != 0) return true;
+            return false;
+        }
+        for (Py_ssize_t pos = 0; PyDict_Next(w.dict, &pos, &key, &value);)
+            if (_PyType_Lookup(w.type, key)) return true;
+        return false;
     }
     bool same(const Watch &w) const {
         if (w.kind == kClass) return std::all_of(methods_.begin(), methods_.end(), as_known);
@@ -324,18 +336,16 @@ private:
         }
         for (int i = 0; i < w.count; ++i)
             if (PyDict_GetItem(w.dict, p[i].key) != p[i].value) return false;
-        while (PyDict_Next(w.dict, &pos, &key, &value))
-            if (hides(w, key)) return false;
-        return true;
+        return !hides(w);
     }
 
-    static const std::vector<py::str> &table_names() {
-        static const auto *names = new std::vector<py::str>{"_modules", "_parameters", "_buffers"};
+    static const std::vector<PyObject *> &table_names() {
+        static const auto *names = new std::vector<PyObject *>(interned({"_modules", "_parameters", "_buffers"}));
         return *names;
     }
-    static const std::vector<py::str> &hook_names() {
-        static const auto *names = new std::vector<py::str>{"_forward_hooks", "_forward_pre_hooks", "_backward_hooks",
-                                                            "_backward_pre_hooks"};
+    static const std::vector<PyObject *> &hook_names() {
+        static const auto *names = new std::vector<PyObject *>(
+            interned({"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"}));
         return *names;
     }
 
@@ -350,6 +360,84 @@ private:
     std::vector<Method> methods_;
     std::vector<Pair> pairs_;
     std::vector<Watch> watches_;
+};
+
+// Nothing at all about a tree of modules (the first is its root, held weakly as above) has
+// changed: their classes, attributes, tables, hooks, the operators.  What was found wanting then
+// is still: a network that is not stock is looked through once and not on every call.
+class ModuleSnapshot {
+public:
+    ModuleSnapshot(const ModuleGuard::Rules &rules, const py::list &modules) {
+        static const auto *names = new std::vector<PyObject *>(
+            interned({"_modules", "_parameters", "_buffers", "_forward_hooks", "_forward_pre_hooks", "_backward_hooks",
+                      "_backward_pre_hooks"}));
+        for (auto item : rules.operators) {
+            PyObject *t = keep_.add(item.ptr()), *dict = PyTuple_GetItem(t, 0), *key = PyTuple_GetItem(t, 1);
+            operators_.push_back({dict, key, keep_.add(PyDict_GetItem(dict, key))});
+        }
+        for (auto d : rules.silent) watch(keep_.add(d.ptr()));
+        std::unordered_set<PyObject *> classes;
+        for (auto item : modules) {
+            PyObject *m = item.ptr(), **slot = _PyObject_GetDictPtr(m);
+            if (!slot || !*slot || !kDictStamps) return;    // (never holds)
+            const bool root = owner_ == nullptr;
+            if (root) {
+                py::object ref = py::reinterpret_steal<py::object>(PyWeakref_NewRef(m, nullptr));
+                if (!ref) throw py::error_already_set();
+                owner_ = keep_.add(ref.ptr());
+                owner_type_ = Py_TYPE(m);
+                owner_attributes_ = *slot;
+            } else {
+                modules_.emplace_back(keep_.add(m), Py_TYPE(m));
+                keep_.add(*slot);
+            }
+            watch(*slot);
+            for (PyObject *name : *names) {
+                PyObject *d = PyDict_GetItem(*slot, name);
+                if (d && PyDict_Check(d)) watch(keep_.add(d));
+            }
+            PyObject *mro = Py_TYPE(m)->tp_mro;
+            for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(mro); ++i) {
+                PyTypeObject *t = reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(mro, i));
+                if (t == &PyBaseObject_Type || !t->tp_dict || !classes.insert((PyObject *)t).second) continue;
+                keep_.add(reinterpret_cast<PyObject *>(t));
+                watch(t->tp_dict);
+            }
+        }
+        whole_ = true;
+    }
+    // (caller holds the GIL)
+    bool holds() const {
+        PyObject *owner = whole_ && owner_ ? PyWeakref_GetObject(owner_) : Py_None;
+        if (owner == Py_None || Py_TYPE(owner) != owner_type_) return false;
+        PyObject **attributes = _PyObject_GetDictPtr(owner);
+        if (!attributes || *attributes != owner_attributes_) return false;
+        for (const auto &e : operators_)
+            if (PyDict_GetItem(e.dict, e.key) != e.value) return false;
+        for (const auto &m : modules_)
+            if (Py_TYPE(m.first) != m.second) return false;
+        for (const auto &w : watches_)
+            if (stamp_of(w.first) != w.second) return false;
+        return true;
+    }
+    int traverse(visitproc visit, void *arg) const { return keep_.traverse(visit, arg); }
+    void clear() {
+        whole_ = false;
+        owner_ = nullptr;
+        keep_.clear();
+    }
+
+private:
+    struct Entry { PyObject *dict, *key, *value; };
+    void watch(PyObject *dict) { watches_.emplace_back(dict, stamp_of(dict)); }
+
+    Refs keep_;                        // owns what is below, but for the root's attributes
+    bool whole_ = false;
+    PyObject *owner_ = nullptr, *owner_attributes_ = nullptr;
+    PyTypeObject *owner_type_ = nullptr;
+    std::vector<Entry> operators_;
+    std::vector<std::pair<PyObject *, PyTypeObject *>> modules_;
+    std::vector<std::pair<PyObject *, uint64_t>> watches_;
 };
 
 }  // namespace ddf_torch

@@ -23,8 +23,8 @@ import torch.nn as nn
 
 from . import functional
 from .functional import ddf  # noqa: F401  (re-exported: callers time the operator through this module)
-from .modules import (DDFPack, _CLASS_RULES, _OWN_METHODS, _PlanSlot, _guard_of, _plain_pointwise_conv, _rule,
-                      _unhooked)
+from .modules import (DDFPack, _CLASS_RULES, _OWN_METHODS, _PlanSlot, _guard_of, _module_tree, _plain_pointwise_conv,
+                      _rule)
 
 __all__ = ['DDFBottleneck', 'DDFResNet', 'ddf_mul_resnet50', 'ddf_mul_resnet101',
            'ddf_mul_resnet152', 'ddf_add_resnet50', 'ddf_add_resnet101', 'ddf_add_resnet152',
@@ -121,9 +121,9 @@ class DDFResNet(nn.Module):
 
     def _is_stock(self):
         """The network is what the constructor builds (BatchNorms may have been folded) in
-        eval mode, of the kinds and sizes the native inference covers, and nothing listens
-        on its modules."""
-        if type(self) is not DDFResNet or not all(_unhooked(m) for m in self.modules() if m is not self):
+        eval mode, of the kinds and sizes the native inference covers.  (That nothing
+        listens on its modules and their methods are their classes' is the guard's part.)"""
+        if type(self) is not DDFResNet:
             return False
         conv, pool = self.conv1, self.maxpool
         pair = lambda v: v if isinstance(v, tuple) else (v, v)
@@ -166,19 +166,16 @@ class DDFResNet(nn.Module):
         return channels % 64 == 0 and self.fc.in_features == channels
 
     def _blocks(self):
-        return [b for stage in (self.layer1, self.layer2, self.layer3, self.layer4) for b in stage]
+        return [b for stage in (self.layer1, self.layer2, self.layer3, self.layer4) for b in stage._modules.values()]
 
     def _native_plan(self, ext):
         """The network's tensors for the extension's native inference, collected once and
         again whenever the network has changed; None where that does not cover it."""
-        slot = _PlanSlot.of(self)
-        if slot.plan is not None and slot.plan.valid():
-            return slot.plan
-        slot.plan = None
-        if not self._is_stock():
-            return None
-        guard = _guard_of(ext, list(self.modules()))
-        if guard is None:
+        return _PlanSlot.current(self, ext, self._new_plan)
+
+    def _new_plan(self, ext):
+        guard = _guard_of(ext, _module_tree(self))
+        if guard is None or not self._is_stock():
             return None
         plan, tensors = ext.NetPlan(guard), []
 
@@ -192,8 +189,8 @@ class DDFResNet(nn.Module):
                       self.fc.out_features)
         for block in self._blocks():
             pack, down = block.conv2, block.downsample
-            conv, sp_norm = pack.spatial_branch
-            fc1, fc2, ch_norm = pack.channel_branch[1], pack.channel_branch[3], pack.channel_branch[4]
+            conv, sp_norm = pack.spatial_branch._modules.values()
+            _, fc1, _, fc2, ch_norm = pack.channel_branch._modules.values()
             branches = [conv.weight, conv.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias,
                         ch_norm.std if ch_norm.runing_std else None, ch_norm.mean if ch_norm.runing_mean else None]
             tensors.extend(branches)
@@ -202,10 +199,7 @@ class DDFResNet(nn.Module):
                 ([None] * 6, 0.0) if down is None else layer(down[0], down[1] if len(down) > 1 else identity), branches,
                 sp_norm.std, 1.0 if ch_norm.runing_std else ch_norm.std, pack.stride, pack.kernel_combine,
                 block.conv1.in_channels, block.conv1.out_channels, block.conv3.out_channels, fc1.out_channels)
-        if not guard.covers(tensors):
-            return None
-        slot.plan = plan
-        return plan
+        return plan if guard.covers(tensors) else None
 
     def forward(self, x):
         # fp16 inference natively where the extension covers it (a plan that no longer
@@ -225,7 +219,7 @@ class DDFResNet(nn.Module):
 
 
 _CLASS_RULES[DDFBottleneck] = _rule(DDFBottleneck)
-_OWN_METHODS[DDFResNet] = ('forward_features', '_blocks', '_is_stock', '_native_plan')
+_OWN_METHODS[DDFResNet] = ('forward_features', '_blocks', '_is_stock', '_native_plan', '_new_plan')
 _CLASS_RULES[DDFResNet] = _rule(DDFResNet, (), ('forward',) + _OWN_METHODS[DDFResNet])
 
 

@@ -301,3 +301,28 @@ def test_a_plan_leaves_forward_mode_alone(make, shape, ext):
         conv._parameters['weight'] = weight
         plan = module._native_plan(ext)
         assert plan is None or plan.misfit(x) is not None
+
+
+@pytest.mark.parametrize('make', kinds(), ids=['layer', 'network'])
+def test_a_refusal_stands_until_something_changes(make, ext):
+    module = make()
+    conv = next(m for m in module.modules() if isinstance(m, torch.nn.Conv2d) and m.kernel_size == (1, 1))
+    handle = conv.register_forward_hook(lambda *a: None)
+    assert module._native_plan(ext) is None
+    refused = module.__dict__['_plan'].refused
+    assert refused.holds()
+    with torch.no_grad():
+        conv.weight.mul_(2.)
+    assert module._native_plan(ext) is None and module.__dict__['_plan'].refused is refused
+    conv.note = 1
+    assert not refused.holds() and module._native_plan(ext) is None
+    refused = module.__dict__['_plan'].refused
+    handle.remove()
+    assert not refused.holds() and module._native_plan(ext) is not None
+    assert module.__dict__['_plan'].refused is None
+    # (neither outlives its module)
+    conv.register_forward_hook(lambda *a: None)
+    assert module._native_plan(ext) is None
+    refused, gone = module.__dict__['_plan'].refused, weakref.ref(module)
+    del module
+    assert gone() is None and not refused.holds()
