@@ -117,9 +117,10 @@ __device__ __forceinline__ void arrive() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 // 16 bytes per lane to LDS at `lds` + lane * 16.  (Written out because the compiler waits for
-// every such load in flight before any LDS read.)
+// every such load in flight before any LDS read.  The address is an operand in m0, so that the
+// compiler itself writes m0 and knows it; the load must not follow that write at once.)
 __device__ __forceinline__ void load_to_lds(uint32_t lds, const _Float16 *p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
 
 template <int BM, int BN, int KST, int ST, int WG, bool PAIR>
