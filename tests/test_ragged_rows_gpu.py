@@ -3,6 +3,7 @@ vector, both lane layouts, planes whose last row ends a tensor, each gradient on
 import pytest
 import torch
 
+import ddfnet_amd
 from ddfnet_amd import _lib
 from ddf_testlib import TOL, check_against_oracle, random_case, rel_err, run_ddf
 
@@ -69,3 +70,32 @@ def test_stride_two_of_any_size(H, W, combine, dtype):
         for g, w in zip(got, want):
             if g is not None:
                 assert rel_err(g, w) <= TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('shape,k,d,s', [((8, 66, 61, 85), 3, 1, 1), ((4, 66, 113, 134), 3, 1, 1),
+                                         ((2, 16, 60, 131), 3, 2, 1), ((2, 16, 23, 71), 5, 2, 1),
+                                         ((3, 37, 11, 131), 3, 1, 2), ((3, 37, 10, 13), 3, 1, 2)], ids=_ids)
+def test_operands_at_odd_element_addresses(shape, k, d, s, combine, dtype):
+    """Every operand and result one element into its buffer: these launches take any address."""
+    def odd(t):
+        view = torch.empty(t.numel() + 1, dtype=t.dtype, device='cuda')[1:].view(t.shape)
+        return view.copy_(t)
+    assert 'ragged' in _lib.describe(shape, k, d, s, combine, dtype)
+    x, cf, sf, go = random_case(*shape, k, s, dtype, seed=k + s)
+    xd, cfd, sfd, god = (odd(t) for t in (x, cf, sf, go))
+    out, dx = odd(torch.zeros_like(go)), odd(torch.zeros_like(x))
+    _lib.forward(xd, cfd, sfd, out, k, d, s, combine)
+    assert rel_err(out, oracle.forward(x, cf, sf, k, d, s, combine)) <= TOL[dtype]
+    need = _lib.NEED_DX
+    ws = torch.empty(max(1, _lib.backward_workspace_bytes(shape, k, d, s, combine, dtype, need)), dtype=torch.uint8,
+                     device='cuda')
+    _lib.backward(god, xd, cfd, sfd, dx, None, None, k, d, s, combine, need, ws)
+    want = oracle.backward(go, x, cf, sf, k, d, s, combine)
+    assert rel_err(dx, want[0]) <= TOL[dtype]
+    # (all gradients, by the public operator; its results are fresh tensors)
+    leaves = [t.requires_grad_(True) for t in (xd, cfd, sfd)]
+    got = torch.autograd.grad(ddfnet_amd.ddf(*leaves, k, d, s, combine), leaves, god)
+    for g, w in zip(got, want):
+        assert rel_err(g, w) <= TOL[dtype]
