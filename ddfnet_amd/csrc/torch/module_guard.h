@@ -144,14 +144,16 @@ public:
         return g;
     }
 
-    // Every one of the objects is an entry of a module's tables or an attribute relied on (a
+    // Every one of the tensors is an entry of a module's tables or an attribute relied on (a
     // tensor assigned as a plain attribute, as on the replicas of nn.DataParallel, is not: the
-    // guard does not see it replaced).
-    bool covers(const py::list &objects) const {
+    // guard does not see it replaced), and none is the result of other operations: a plan that
+    // holds it would hold its graph (the weights torch.func.functional_call puts in for one call).
+    bool covers(const py::list &tensors) const {
         std::unordered_set<PyObject *> mine;
         for (const Pair &p : pairs_) mine.insert(p.value);
-        return std::all_of(objects.begin(), objects.end(),
-                           [&](py::handle o) { return o.is_none() || mine.count(o.ptr()); });
+        return std::all_of(tensors.begin(), tensors.end(), [&](py::handle o) {
+            return o.is_none() || (mine.count(o.ptr()) && THPVariable_Check(o.ptr()) && THPVariable_Unpack(o.ptr()).is_leaf());
+        });
     }
     // (caller holds the GIL)
     bool holds() const {

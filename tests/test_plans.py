@@ -326,3 +326,18 @@ def test_a_refusal_stands_until_something_changes(make, ext):
     refused, gone = module.__dict__['_plan'].refused, weakref.ref(module)
     del module
     assert gone() is None and not refused.holds()
+
+
+@pytest.mark.parametrize('make', kinds(), ids=['layer', 'network'])
+def test_no_plan_holds_on_to_the_graph_of_weights_put_in_for_a_call(make, ext):
+    module = make()
+    assert module._native_plan(ext) is not None
+    conv = next(m for m in module.modules() if isinstance(m, torch.nn.Conv2d))
+    own = conv.weight
+    conv._parameters['weight'] = fast = own * 2
+    gone = weakref.ref(fast)
+    assert module._native_plan(ext) is None
+    conv._parameters['weight'] = own
+    del fast
+    assert gone() is None
+    assert module._native_plan(ext) is not None
