@@ -214,6 +214,8 @@ class DDFResNet(nn.Module):
                     out = ext.net_forward(fresh, x)
             if out is not None:
                 return out
+        else:
+            _PlanSlot.drop(self)
         x = self.global_pool(self.forward_features(x)).flatten(1)
         return self.fc(x)
 

@@ -341,3 +341,13 @@ def test_no_plan_holds_on_to_the_graph_of_weights_put_in_for_a_call(make, ext):
     del fast
     assert gone() is None
     assert module._native_plan(ext) is not None
+
+
+def test_a_network_that_trains_lets_replaced_parts_go(ext):
+    net = small_net().float()
+    assert net._native_plan(ext) is not None
+    gone = weakref.ref(net.fc)
+    net.fc = torch.nn.Linear(2048, 4)
+    with pytest.raises((AssertionError, RuntimeError)):      # (no device: the operator refuses)
+        net.train()(torch.zeros(2, 3, 64, 64))
+    assert gone() is None
