@@ -354,9 +354,9 @@ bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r, bool b
     const bool exact = (p.s != 2 || !backward || p.H % 2 == 0) && rows_geometry(p, dtype, 0, g, vx, r);
     if (dtype != DDF_F16 && dtype != DDF_F32) return exact;
     // Which cut: fitted over 80 sizes.  Forward at 12 x 144 x 80 x 87 fp32 28.1 -> 19.9 us, fp16
-    // 26.3 -> 19.3; 5 x 5 at 2 x 48 x 135 x 166, which only the LDS-tile kernels covered, 45 ->
-    // 11.3.  Small launches keep vectors that divide their rows: 4 x 256 x 25 x 38 fp16 takes
-    // 5.2 us in vectors of two and 6.7 in eight.
+    // 26.1 -> 22.1 (odd rows: taps combined in fp32 on either); 5 x 5 at 2 x 48 x 135 x 166,
+    // which only the LDS-tile kernels covered, 45 -> 11.3.  Small launches keep vectors that
+    // divide their rows: 4 x 256 x 25 x 38 fp16 takes 5.2 us in vectors of two and 6.7 in eight.
     const int esz = dtype == DDF_F16 ? 2 : 4;
     double best = exact ? rows_cost(*g, false, p.k, esz, *vx, *r) : 1e30;
     bool found = exact;
