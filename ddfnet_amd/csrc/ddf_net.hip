@@ -183,17 +183,18 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
     };
     clear();
-    // Without a BatchNorm (the classifier) a bias is part of the sum, which is rounded once;
-    // under one the sum is rounded first, as a convolution's result is.
+    // Without a BatchNorm (the classifier) a bias is part of the sum, which is rounded once, as
+    // nn.Linear has it.  Elsewhere, and in a pair, the sum is rounded first, as a convolution's
+    // result is.  (A bias in a pair's accumulators had the 128 x 128 tiles spill: 86 -> 117 us.)
     const bool bias_in_sum = !PAIR && !a.norm.var && a.norm.conv_bias;
     if (bias_in_sum) {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int c = n0 + channel(j, g);    // (rows are whole vectors of 8)
+                const int o = n0 + channel(j, g);    // (rows are whole vectors of 8)
                 half4_t b = {0, 0, 0, 0};
-                if (c < a.N) __builtin_memcpy(&b, static_cast<const _Float16 *>(a.norm.conv_bias) + c, sizeof(b));
+                if (o < a.N) __builtin_memcpy(&b, static_cast<const _Float16 *>(a.norm.conv_bias) + o, sizeof(b));
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -242,14 +243,11 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
     };
     half4_t side[PAIR ? TM : 1][PAIR ? TN : 1][PAIR ? 4 : 1];
-    auto affine_of = [&](int which, bool bn, int i, int j, int g, float (&f)[4]) __attribute__((always_inline)) {
+    auto affine_of = [&](int which, int i, int j, int g, float (&f)[4]) __attribute__((always_inline)) {
         const float4_t sc = *reinterpret_cast<const float4_t *>(&affine[which][channel(j, g)]);
         const float4_t sh = *reinterpret_cast<const float4_t *>(&affine[which + 1][channel(j, g)]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float sum = acc[i][j][4 * g + e];
-            f[e] = fmaf(bn ? (float)(_Float16)sum : sum, sc[e], sh[e]);
-        }
+        for (int e = 0; e < 4; ++e) f[e] = fmaf((float)(_Float16)acc[i][j][4 * g + e], sc[e], sh[e]);
     };
 
     const int nk0 = PAIR ? first.K / KST : 0, nk = nk0 + a.K / KST;
@@ -300,7 +298,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
 #pragma unroll
                         for (int g = 0; g < 4; ++g) {
                             float f[4];
-                            affine_of(2, first.norm.var != nullptr, i, j, g, f);
+                            affine_of(2, i, j, g, f);
 #pragma unroll
                             for (int e = 0; e < 4; ++e) side[i][j][g][e] = (_Float16)f[e];
                         }
@@ -321,7 +319,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 half4_t v;
                 if constexpr (PAIR) {
                     float f[4];
-                    affine_of(0, a.norm.var != nullptr, i, j, g, f);
+                    affine_of(0, i, j, g, f);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         f[e] += (float)side[i][j][g][e];

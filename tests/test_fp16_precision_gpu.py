@@ -121,6 +121,8 @@ def test_bias_without_a_norm_beside_a_projection():
     out = torch.empty(n, o, device='cuda', dtype=torch.float16)
     call('ddf_hip_net_conv_pair', x.cuda(), w.cuda(), Norm(conv_bias=db.data_ptr()), c, xs.cuda(), ws.cuda(),
          Norm(conv_bias=dbs.data_ptr()), 1, 1, side, 1, out, n, o, 0)
-    want_side = sides + bs.double()
-    within(out, sums + b.double() + want_side, sums + sides + b.double().abs() + bs.double().abs(), c + side + 2,
-           want_side.abs())
+    want, want_side = sums + b.double(), sides + bs.double()
+    # (both sums are fp16 before their biases, as two convolutions' results are, and the projection's
+    # result is)
+    within(out, want + want_side, sums + sides + b.double().abs() + bs.double().abs(), c + side + 2,
+           sums + sides + want_side.abs())
