@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "ddf_channel.h"
 #include "ddf_common.h"
 #include "ddf_rows.h"
 
@@ -36,56 +37,6 @@ using rows::store_vec_nt;
 using rows::vec_words;
 
 constexpr int kChunk = 256;   // channels whose weights sit in LDS at a time (64 per wave)
-
-// Gains, offsets and biases of the KK taps of filter group `g`, read once (all
-// loads go out together; read tap by tap where they are used, every one of
-// them is a round trip of its own at the end of the kernel).
-template <typename T, int KK>
-struct TapParams {
-    float gain[KK], offset[KK], bias[KK];
-    __device__ __forceinline__ void load(int64_t g, float scalar_gain, const T *gain_vec,
-                                         const T *offset_vec, const T *bias_vec) {
-#pragma unroll
-        for (int t = 0; t < KK; ++t) {
-            gain[t] = scalar_gain;
-            offset[t] = 0.f;
-            bias[t] = 0.f;
-        }
-        if (gain_vec) {
-#pragma unroll
-            for (int t = 0; t < KK; ++t) gain[t] = ld(gain_vec + g * KK + t);
-        }
-        if (offset_vec) {
-#pragma unroll
-            for (int t = 0; t < KK; ++t) offset[t] = ld(offset_vec + g * KK + t);
-        }
-        if (bias_vec) {
-#pragma unroll
-            for (int t = 0; t < KK; ++t) bias[t] = ld(bias_vec + g * KK + t);
-        }
-    }
-};
-
-// v[0..KK) + bias, standardised in place, times gain plus offset.
-template <typename T, int KK>
-__device__ __forceinline__ void normalise(float (&v)[KK], const TapParams<T, KK> &p) {
-    float sum = 0;
-#pragma unroll
-    for (int t = 0; t < KK; ++t) {
-        v[t] += p.bias[t];
-        sum += v[t];
-    }
-    const float mean = sum / (float)KK;
-    float sq = 0;
-#pragma unroll
-    for (int t = 0; t < KK; ++t) {
-        v[t] -= mean;
-        sq += v[t] * v[t];
-    }
-    const float inv = 1.f / (sqrtf(sq / (float)(KK - 1)) + 1e-10f);
-#pragma unroll
-    for (int t = 0; t < KK; ++t) v[t] = v[t] * inv * p.gain[t] + p.offset[t];
-}
 
 // VP storage-type values at p (aligned to VP * sizeof(T)), widened.
 template <typename T, int VP>
@@ -862,276 +813,10 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
 }
 
 
-// ---- the channel branch on the matrix cores (fp16) ---------------------------
-//
-// Both 1x1 convolutions are matrix products with the batch as one dimension:
-//   hidden[m, n] = relu(b1[m] + sum_c w1[m, c] * v[n, c])           (mid x C) . (C x N)
-//   taps[r, n]   = b2[r] + sum_m w2[r, m] * hidden[m, n]            (C*KK x mid) . (mid x N)
-// v_mfma_f32_16x16x32_f16 takes, per lane l of a wave, eight values of a row of A
-// (row l % 16, positions 8 * (l / 16) + 0..7 of the 32 the step covers: one
-// 16-byte load from a row-major weight matrix) and the eight values of column
-// l % 16 of B at the same positions, and leaves D[4 * (l / 16) + 0..3][l % 16].
-// A workgroup takes sixteen samples (the columns) and `block` channels:
-//   * the pooled vectors go to LDS as [32 channels][sample][32], rounded to fp16
-//     (what the reference's half-precision pooling returns);
-//   * the hidden layer goes to LDS as [32 values][sample][32], rounded to fp16 (as
-//     the reference's first convolution does);
-//   * the rows of tile j of the second product are (channel c0 + i, tap j), so a
-//     lane ends up with all KK taps of four channels of one sample and
-//     normalises them in registers: 4 * KK contiguous values to store.
-// mid is no multiple of 32 (nor of 16): the last tile of hidden values starts at
-// mid - 32 (mid - 16 for the rows of the first product) and overlaps the one
-// before it; the overlapping positions of its B operand are zero (they are
-// counted in the tile before), so every weight that is read is a weight of the
-// row it is used for.  Rows of w2 start at any even byte address: its loads are
-// 16 bytes at 2-byte alignment.
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ half8_t load_half8_any(const __half *p) {
-    half8_t v;
-    __builtin_memcpy(&v, p, sizeof(v));
-    return v;
-}
-__device__ __forceinline__ half8_t load_half8(const __half *p) {
-    return *reinterpret_cast<const half8_t *>(p);
-}
-__device__ __forceinline__ half4_t load_half4(const __half *p) {
-    return *reinterpret_cast<const half4_t *>(p);
-}
-
-constexpr int kMmaSamples = 16;
-constexpr int kMmaStep = 32;                          // values of the summed dimension per instruction
-constexpr int kMmaTile = kMmaSamples * kMmaStep;      // halves of one [sample][32] tile in LDS
-
-template <int KK, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void k_channel_branch_mma(
-    const __half *__restrict__ pooled, const __half *__restrict__ w1, const __half *__restrict__ b1,
-    const __half *__restrict__ w2, const __half *__restrict__ b2, __half *__restrict__ cf, int N, int C,
-    int mid, int block, float gain, const __half *__restrict__ gain_vec,
-    const __half *__restrict__ offset_vec, const float *__restrict__ parts, int nparts, float scale,
-    ChannelSave save) {
-    extern __shared__ __align__(16) _Float16 mma_smem[];
-    _Float16 *pv = mma_smem;                        // [C / 32][16 samples][32]: pooled vectors
-    _Float16 *hv = pv + (C / kMmaStep) * kMmaTile;  // [tiles of mid][16 samples][32]: hidden vectors
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int col = lane & 15, quad = lane >> 4;
-    const int n0 = blockIdx.y * kMmaSamples;
-    const int cb = blockIdx.x * block;
-    const int rtiles = (mid + 15) >> 4;             // tiles of sixteen rows of w1
-    const int ktiles = (mid + kMmaStep - 1) / kMmaStep;   // steps of the second product
-    const int klast = mid - kMmaStep;               // where the last of them starts
-    const int nk = C / kMmaStep;                    // steps of the first product
-
-    // All waves: the pooled vectors of the sixteen samples into LDS, four channels per
-    // item (given, or scale * the sum of nparts partial sums per value), and zeros in
-    // the last tile of the hidden layer (its overlap with the tile before stays zero).
-    auto pooled_vectors = [&]() {
-        // (Only samples there are: a column of the products that belongs to none is read by nothing.)
-        const int c4s = C >> 2, items = min(kMmaSamples, N - n0) * c4s;
-        for (int i = threadIdx.x; i < items; i += WAVES * kWave) {
-            const int s = i / c4s, c4 = i - s * c4s;
-            const int64_t n = n0 + s;
-            half4_t v;
-            if (parts) {
-                const float4_t *src = reinterpret_cast<const float4_t *>(parts + n * nparts * C) + c4;
-                float4_t a = {0.f, 0.f, 0.f, 0.f};
-                // four partial sums requested together (the fence keeps the compiler from
-                // taking them one round trip at a time to save registers)
-                int q = 0;
-                for (; q + 4 <= nparts; q += 4) {
-                    const float4_t x0 = src[(int64_t)q * c4s], x1 = src[(int64_t)(q + 1) * c4s],
-                                   x2 = src[(int64_t)(q + 2) * c4s], x3 = src[(int64_t)(q + 3) * c4s];
-                    __builtin_amdgcn_sched_barrier(0);
-                    a += (x0 + x1) + (x2 + x3);
-                }
-                for (; q < nparts; ++q) a += src[(int64_t)q * c4s];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = (_Float16)(a[e] * scale);
-            } else {
-                v = load_half4(pooled + n * C + c4 * 4);
-            }
-            *reinterpret_cast<half4_t *>(pv + ((c4 >> 3) * kMmaSamples + s) * kMmaStep + (c4 & 7) * 4) = v;
-            if (save.pooled && blockIdx.x == 0) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) save.pooled[n * C + c4 * 4 + e] = (float)v[e];
-            }
-        }
-        for (int i = threadIdx.x; i < kMmaTile / 2; i += WAVES * kWave)
-            reinterpret_cast<uint32_t *>(hv + (ktiles - 1) * kMmaTile)[i] = 0u;
-    };
-
-    // The first waves compute taps (a tile of sixteen channels at a time), the others
-    // the hidden layer; each kind asks for the first weights it will need before
-    // anything else (they depend on nothing, and are there by the time the operand
-    // from LDS is).  The two kinds run separate code, so each has the whole register
-    // file for what it keeps in flight; both pass the same two barriers.
-    const int tap_waves = min(min(block, C - cb) >> 4, WAVES - 1);
-    if (wave >= tap_waves) {
-        // ---- hidden layer: tiles of sixteen rows of w1 ----
-        constexpr int kPre1 = 16;
-        const int hidden_waves = WAVES - tap_waves;
-        const int t0 = wave - tap_waves;
-        half8_t apre[kPre1];
-        auto request = [&](int t) {
-            const __half *arow = w1 + (int64_t)(min(t * 16, mid - 16) + col) * C + quad * 8;
-#pragma unroll
-            for (int u = 0; u < kPre1; ++u) apre[u] = load_half8(arow + min(u, nk - 1) * kMmaStep);
-        };
-        if (t0 < rtiles) request(t0);
-        pooled_vectors();
-        __syncthreads();
-        for (int t = t0; t < rtiles; t += hidden_waves) {
-            if (t != t0) request(t);
-            const int mbase = min(t * 16, mid - 16);
-            const __half *arow = w1 + (int64_t)(mbase + col) * C + quad * 8;
-            const _Float16 *brow = pv + col * kMmaStep + quad * 8;
-            float4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int u = 0; u < kPre1; ++u) {
-                if (u < nk)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                        apre[u], *reinterpret_cast<const half8_t *>(brow + u * kMmaTile), acc, 0, 0, 0);
-            }
-            // (the matrix instruction is convergent, which rules out unrolling with a
-            // remainder: chunks of a fixed number of steps, all loads of a chunk first)
-            int kb = kPre1;
-            auto chunk = [&](auto steps) {
-                constexpr int U = decltype(steps)::value;
-                half8_t a[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) a[u] = load_half8(arow + (kb + u) * kMmaStep);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                        a[u], *reinterpret_cast<const half8_t *>(brow + (kb + u) * kMmaTile), acc, 0, 0, 0);
-                kb += U;
-            };
-            while (nk - kb >= 16) chunk(std::integral_constant<int, 16>());
-            if (nk - kb >= 8) chunk(std::integral_constant<int, 8>());
-            if (nk - kb >= 4) chunk(std::integral_constant<int, 4>());
-            while (kb < nk) chunk(std::integral_constant<int, 1>());
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = mbase + quad * 4 + e;
-                if (m < t * 16) continue;    // (the last tile's overlap: those rows belong to the tile before)
-                const float bias = b1 ? ld(b1 + m) : 0.f;
-                const int kt = min(m / kMmaStep, ktiles - 1);
-                const _Float16 hm = (_Float16)relu(acc[e] + bias);
-                hv[(kt * kMmaSamples + col) * kMmaStep + m - min(kt * kMmaStep, klast)] = hm;
-                if (save.hidden && blockIdx.x == 0 && n0 + col < N) save.hidden[(int64_t)(n0 + col) * mid + m] = (float)hm;
-            }
-        }
-        __syncthreads();
-        return;
-    }
-
-    // ---- taps: per wave sixteen channels x KK taps x sixteen samples ----
-    constexpr int kPre = KK <= 9 ? 2 : 1;           // steps of the second product requested up front
-    half4_t pg[KK], po[KK], pb[KK];
-    half8_t apre[kPre][KK];
-    auto request = [&](int c0) {
-        // gains, offsets and biases of this lane's four channels: 4 * KK contiguous values each
-        const int64_t pbase = (int64_t)(c0 + quad * 4) * KK;
-#pragma unroll
-        for (int j = 0; j < KK; ++j) pg[j] = po[j] = pb[j] = half4_t{0, 0, 0, 0};
-        if (gain_vec) {
-#pragma unroll
-            for (int j = 0; j < KK; ++j) pg[j] = load_half4(gain_vec + pbase + 4 * j);
-        }
-        if (offset_vec) {
-#pragma unroll
-            for (int j = 0; j < KK; ++j) po[j] = load_half4(offset_vec + pbase + 4 * j);
-        }
-        if (b2) {
-#pragma unroll
-            for (int j = 0; j < KK; ++j) pb[j] = load_half4(b2 + pbase + 4 * j);
-        }
-        const __half *arow = w2 + (int64_t)(c0 + col) * KK * mid + quad * 8;
-#pragma unroll
-        for (int u = 0; u < kPre; ++u) {
-            const int kbase = min(u * kMmaStep, klast);    // (steps past the last one: the last one again, unused)
-#pragma unroll
-            for (int j = 0; j < KK; ++j) apre[u][j] = load_half8_any(arow + j * mid + kbase);
-        }
-    };
-    request(cb + wave * 16);
-    pooled_vectors();
-    __syncthreads();
-    __syncthreads();
-    const int n = n0 + col;
-    for (int ct = wave; ct * 16 < block && cb + ct * 16 < C; ct += tap_waves) {
-        const int c0 = cb + ct * 16;
-        if (ct != wave) request(c0);
-        float4_t acc[KK];
-#pragma unroll
-        for (int j = 0; j < KK; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
-        const __half *arow = w2 + (int64_t)(c0 + col) * KK * mid + quad * 8;
-        const _Float16 *brow = hv + col * kMmaStep + quad * 8;
-#pragma unroll
-        for (int u = 0; u < kPre; ++u) {
-            if (u < ktiles) {
-                const half8_t b = *reinterpret_cast<const half8_t *>(brow + u * kMmaTile);
-#pragma unroll
-                for (int j = 0; j < KK; ++j)
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(apre[u][j], b, acc[j], 0, 0, 0);
-            }
-        }
-        int t = kPre;
-        auto tiles = [&](auto count) {
-            constexpr int U = decltype(count)::value;
-            half8_t a[U][KK];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int kbase = min((t + u) * kMmaStep, klast);
-#pragma unroll
-                for (int j = 0; j < KK; ++j) a[u][j] = load_half8_any(arow + j * mid + kbase);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const half8_t b = *reinterpret_cast<const half8_t *>(brow + (t + u) * kMmaTile);
-#pragma unroll
-                for (int j = 0; j < KK; ++j)
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[u][j], b, acc[j], 0, 0, 0);
-            }
-            t += U;
-        };
-        while (ktiles - t >= kPre) tiles(std::integral_constant<int, kPre>());
-        if (kPre > 1 && t < ktiles) tiles(std::integral_constant<int, 1>());
-        if (n >= N) continue;
-        half4_t out[KK];   // channel e of the lane's four: values [e * KK, (e + 1) * KK) of the 4 * KK
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float u[KK];
-            TapParams<__half, KK> params;
-#pragma unroll
-            for (int j = 0; j < KK; ++j) {
-                const int at = e * KK + j;
-                u[j] = acc[j][e];
-                params.gain[j] = gain_vec ? (float)pg[at >> 2][at & 3] : gain;
-                params.offset[j] = offset_vec ? (float)po[at >> 2][at & 3] : 0.f;
-                params.bias[j] = b2 ? (float)pb[at >> 2][at & 3] : 0.f;
-            }
-            if (save.taps) {
-                float *zp = save.taps + ((int64_t)n * C + c0 + quad * 4 + e) * KK;
-#pragma unroll
-                for (int j = 0; j < KK; ++j) zp[j] = u[j] + params.bias[j];
-            }
-            normalise<__half, KK>(u, params);
-#pragma unroll
-            for (int j = 0; j < KK; ++j) {
-                const int at = e * KK + j;
-                out[at >> 2][at & 3] = (_Float16)u[j];
-            }
-        }
-        half4_t *op = reinterpret_cast<half4_t *>(cf + ((int64_t)n * C + c0 + quad * 4) * KK);
-#pragma unroll
-        for (int j = 0; j < KK; ++j) op[j] = out[j];
-    }
+template <int KK, bool SAVE>
+__global__ __launch_bounds__(kMmaThreads) void k_channel_branch_mma(ChannelMma a) {
+    extern __shared__ __align__(16) unsigned char mma_smem[];
+    channel_mma<KK, SAVE>(a, blockIdx.x, blockIdx.y, mma_smem);
 }
 
 }  // namespace
@@ -1344,26 +1029,20 @@ hipError_t channel_branch_mma<__half>(const __half *pooled, const __half *w1, co
                                       int nparts, double scale, const ChannelSave &save) {
     if (tune_int("DDF_TUNE_CHANNEL_MMA", 1) == 0) return hipErrorNotSupported;
     auto aligned = [](const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
-    const size_t lds = (size_t)(C / kMmaStep + cdiv(mid, kMmaStep)) * kMmaTile * sizeof(__half);
-    if ((k != 3 && k != 5) || mid < kMmaStep || C % kMmaStep != 0 || lds > 64 * 1024 ||
-        N > (int64_t)65535 * kMmaSamples || C * k * k * mid >= ((int64_t)1 << 31))
+    if ((k != 3 && k != 5) || !channel_mma_covers(C, mid, k * k) || N > (int64_t)65535 * kMmaSamples)
         return hipErrorNotSupported;
     if (!aligned(w1, 16) || !aligned(cf, 8) || !aligned(b2, 8) || !aligned(gain_vec, 8) ||
         !aligned(offset_vec, 8) || !aligned(w2, 2) || (parts ? !aligned(parts, 16) : !aligned(pooled, 8)))
         return hipErrorNotSupported;
-    // (25 taps: the accumulators and parameters of a tile need the registers of a wave alone on its SIMD)
-    const int waves = k == 3 && tune_int("DDF_TUNE_CHANNEL_MMA_WAVES", 8) == 8 ? 8 : 4;
-    int block = tune_int("DDF_TUNE_CHANNEL_MMA_BLOCK", 16);
-    block = std::max(16, block / 16 * 16);
-    const dim3 grid((unsigned)cdiv(C, block), (unsigned)cdiv(N, kMmaSamples));
-#define DDF_MMA_LAUNCH(KK_, WAVES_)                                                                  \
-    hipLaunchKernelGGL((k_channel_branch_mma<KK_, WAVES_>), grid, dim3(WAVES_ * kWave), lds, st, pooled, \
-                       w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, block, (float)gain, gain_vec,      \
-                       offset_vec, parts, nparts, (float)scale, save)
-    if (k == 3 && waves == 8) DDF_MMA_LAUNCH(9, 8);
-    else if (k == 3) DDF_MMA_LAUNCH(9, 4);
-    else DDF_MMA_LAUNCH(25, 4);
-#undef DDF_MMA_LAUNCH
+    const ChannelMma a{pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain, gain_vec, offset_vec,
+                       parts, nparts, (float)scale, save, channel_mma_lds(C, mid, k * k)};
+    const dim3 grid((unsigned)cdiv(C, kMmaChannels), (unsigned)cdiv(N, kMmaSamples));
+    const size_t lds = a.lds.total;
+    const bool saves = save.pooled || save.hidden || save.taps;
+    if (k == 3 && saves) hipLaunchKernelGGL((k_channel_branch_mma<9, true>), grid, dim3(kMmaThreads), lds, st, a);
+    else if (k == 3) hipLaunchKernelGGL((k_channel_branch_mma<9, false>), grid, dim3(kMmaThreads), lds, st, a);
+    else if (saves) hipLaunchKernelGGL((k_channel_branch_mma<25, true>), grid, dim3(kMmaThreads), lds, st, a);
+    else hipLaunchKernelGGL((k_channel_branch_mma<25, false>), grid, dim3(kMmaThreads), lds, st, a);
     return hipGetLastError();
 }
 

@@ -1,0 +1,530 @@
+// The channel filter branch of DDFPack on the matrix cores (fp16), as a device function: the
+// layer's kernel (ddf_branches.hip) is nothing else, a network's runs it beside the spatial
+// branch (ddf_net.hip).
+#pragma once
+
+#include <algorithm>
+
+#include "ddf_common.h"
+#include "ddf_rows.h"
+
+namespace ddf {
+
+// Both 1x1 convolutions are matrix products with the batch as one dimension:
+//   hidden[m, n] = relu(b1[m] + sum_c w1[m, c] * v[n, c])           (mid x C) . (C x N)
+//   taps[r, n]   = b2[r] + sum_m w2[r, m] * hidden[m, n]            (C*KK x mid) . (mid x N)
+// v_mfma_f32_16x16x32_f16 takes, per lane l of a wave, eight values of a row of A
+// (row l % 16, positions 8 * (l / 16) + 0..7 of the 32 the step covers: one
+// 16-byte load from a row-major weight matrix) and the eight values of column
+// l % 16 of B at the same positions, and leaves D[4 * (l / 16) + 0..3][l % 16].
+// A workgroup takes sixteen samples (the columns) and sixteen channels:
+//   * the pooled vectors go to LDS as [32 channels][sample][32], rounded to fp16
+//     (what the reference's half-precision pooling returns);
+//   * the hidden layer goes to LDS as [32 values][sample][32], rounded to fp16 (as
+//     the reference's first convolution does);
+//   * the rows of tile j of the second product are (channel c0 + i, tap j); the taps meet in
+//     LDS as fp32, and a thread per sample and pair of channels normalises and stores them.
+// mid is no multiple of 16 or 32: rows of w1 past the last are whatever lies in LDS and make
+// hidden values that are set to zero; the last step of a row of w2 is cut at its end.
+//
+// There is no arithmetic to speak of: the launch is a chain of round trips and the way the
+// weights come in.  An operand read straight from memory is sixteen rows of 64 bytes per load
+// instruction, which a compute unit takes 70 (aligned rows) to 110 clocks for, where 1 KB in a
+// row takes 20 (eight waves, from L2); a workgroup of 256 channels has 68 such loads.  So w1
+// and the block's part of w2 - one run of bytes each - come in as they lie, straight into
+// LDS, before anything else, and operands are read from there; biases, gains and offsets
+// are requested along with them by the other half of the waves.  Eight waves take the hidden
+// tiles, five the nine taps, four the normalisation (one wave had taps and normalisation).  us a
+// launch, before / now: 1 sample x 256 channels 8.2 / 4.7, 1 x 512 9.2 / 6.2, 128 x 256 9.9 / 5.8,
+// 128 x 512 13.2 / 8.5, 4 x 1024 24.3 / 22.2 (an empty launch: 1.6).
+constexpr int kMmaSamples = 16, kMmaChannels = 16;
+constexpr int kMmaStep = 32;                          // values of the summed dimension per instruction
+constexpr int kMmaTile = kMmaSamples * kMmaStep;      // halves of one [sample][32] tile in LDS
+constexpr int kMmaWaves = 8, kMmaThreads = kMmaWaves * kWave;
+constexpr int kMmaSpread = 4 * kWave;                 // channels up to which waves share a value's partial sums
+constexpr int kMmaRound = 8;                          // partial sums requested together
+constexpr int kMmaLds = 160 * 1024;
+
+// LDS, bytes: pooled vectors | rows of w1 | the block's rows of w2 | hidden vectors | partial
+// sums on their way to the pooled vectors.  All rows of w1 and w2 where they fit; else w1 by
+// `chunk` rows and w2 in the same place after it, or (chunk_w2 false) from memory.  The block's
+// taps go where w1 and the pooled vectors were.
+struct ChannelMmaLds {
+    int pitch;                  // bytes of a row of w1
+    int chunk;                  // rows of w1 at a time, whole tiles
+    int w1, w2, hidden, sums, total;
+    bool stage_w2, shared;      // shared: the taps reach into the rows of w2
+};
+inline int mma_round(int64_t v) { return (int)((v + 15) / 16 * 16); }
+inline ChannelMmaLds channel_mma_lds(int64_t C, int64_t mid, int kk) {
+    ChannelMmaLds l{};
+    // (a wave's load is 1 KB: two rows of up to 256 channels, or one in pieces of 512)
+    l.pitch = C <= 256 ? 512 : (int)((C + 511) / 512 * 1024);
+    const int64_t pooled = C * kMmaSamples * 2, rows = (mid + 15) / 16 * 16;
+    const int64_t w2 = (int64_t)kMmaChannels * kk * mid * 2;
+    const int64_t hidden = (mid + kMmaStep - 1) / kMmaStep * kMmaTile * 2, sums = C <= kMmaSpread ? kMmaThreads * 16 : 0;
+    const int64_t taps = kMmaSamples * (kMmaChannels * kk + 1) * 4;
+    const int64_t left = kMmaLds - pooled - hidden - sums;
+    l.w1 = (int)pooled;
+    int64_t space;
+    if (rows * l.pitch + w2 <= left) {
+        l.chunk = (int)rows;
+        l.stage_w2 = true;
+        l.w2 = l.w1 + (int)rows * l.pitch;
+        space = rows * l.pitch + w2;
+    } else {
+        l.chunk = (int)std::min<int64_t>(rows, std::max<int64_t>(left / l.pitch / 16 * 16, 0));
+        l.stage_w2 = w2 <= left;
+        l.w2 = l.w1;
+        space = std::max<int64_t>((int64_t)l.chunk * l.pitch, l.stage_w2 ? w2 : 0);
+    }
+    space = std::max(space, taps - pooled);
+    l.shared = l.stage_w2 && l.w2 < taps;
+    l.hidden = mma_round(l.w1 + space);
+    l.sums = l.hidden + (int)hidden;
+    l.total = l.sums + (int)sums;
+    return l;
+}
+inline bool channel_mma_covers(int64_t C, int64_t mid, int kk) {
+    if (mid < kMmaStep || C % kMmaStep != 0 || C * kk * mid >= ((int64_t)1 << 31)) return false;
+    if (C / kMmaStep + (mid + kMmaStep - 1) / kMmaStep > 64) return false;
+    const ChannelMmaLds l = channel_mma_lds(C, mid, kk);
+    return l.chunk > 0 && l.total <= kMmaLds;
+}
+
+struct ChannelMma {
+    const __half *pooled, *w1, *b1, *w2, *b2;
+    __half *cf;
+    int N, C, mid;
+    float gain;
+    const __half *gain_vec, *offset_vec;
+    const float *parts;    // (nparts per sample; null: `pooled`)
+    int nparts;
+    float scale;
+    ChannelSave save;
+    ChannelMmaLds lds;
+};
+
+#ifdef __HIPCC__
+
+// Gains, offsets and biases of the KK taps of filter group `g`, read once (all
+// loads go out together; read tap by tap where they are used, every one of
+// them is a round trip of its own at the end of the kernel).
+template <typename T, int KK>
+struct TapParams {
+    float gain[KK], offset[KK], bias[KK];
+    __device__ __forceinline__ void load(int64_t g, float scalar_gain, const T *gain_vec,
+                                         const T *offset_vec, const T *bias_vec) {
+#pragma unroll
+        for (int t = 0; t < KK; ++t) {
+            gain[t] = scalar_gain;
+            offset[t] = 0.f;
+            bias[t] = 0.f;
+        }
+        if (gain_vec) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) gain[t] = ld(gain_vec + g * KK + t);
+        }
+        if (offset_vec) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) offset[t] = ld(offset_vec + g * KK + t);
+        }
+        if (bias_vec) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) bias[t] = ld(bias_vec + g * KK + t);
+        }
+    }
+};
+
+// v[0..KK) + bias, standardised in place, times gain plus offset.
+template <typename T, int KK>
+__device__ __forceinline__ void normalise(float (&v)[KK], const TapParams<T, KK> &p) {
+    float sum = 0;
+#pragma unroll
+    for (int t = 0; t < KK; ++t) {
+        v[t] += p.bias[t];
+        sum += v[t];
+    }
+    const float mean = sum / (float)KK;
+    float sq = 0;
+#pragma unroll
+    for (int t = 0; t < KK; ++t) {
+        v[t] -= mean;
+        sq += v[t] * v[t];
+    }
+    const float inv = 1.f / (sqrtf(sq / (float)(KK - 1)) + 1e-10f);
+#pragma unroll
+    for (int t = 0; t < KK; ++t) v[t] = v[t] * inv * p.gain[t] + p.offset[t];
+}
+
+
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane to LDS at `lds` + lane * 16.  (Written out because the compiler waits for
+// every such load in flight before any LDS read.  The address is an operand in m0, so that the
+// compiler itself writes m0 and knows it; the load must not follow that write at once.)
+__device__ __forceinline__ void load_to_lds(uint32_t lds, const void *p) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
+}
+// The same from a uniform address and a lane's offset.
+__device__ __forceinline__ void load_to_lds(uint32_t lds, const char *base, int offset) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
+}
+// This wave's are there.
+__device__ __forceinline__ void loads_to_lds_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Block (bx, by) of (C / 16, samples / 16), kMmaThreads threads.  SAVE: a.save is wanted
+// (compiled in, as a branch around every store has the loads before it wait one by one).
+template <int KK, bool SAVE>
+__device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by, unsigned char *smem) {
+    constexpr int TPW = KK <= 9 ? 2 : 4, TAP_WAVES = (KK + TPW - 1) / TPW;      // taps per wave
+    constexpr int NORM_WAVES = kMmaSamples * kMmaChannels / kWave;
+    static_assert(TAP_WAVES <= kMmaWaves && NORM_WAVES <= kMmaWaves && KK % 8 == 1);
+    constexpr int ZP = kMmaChannels * KK + 1;            // (odd: samples in different banks)
+    const int C = a.C, mid = a.mid;
+    _Float16 *pv = reinterpret_cast<_Float16 *>(smem);   // [C / 32][16 samples][32]: pooled vectors
+    float *z = reinterpret_cast<float *>(smem);          // [sample][channel][tap], in their place and w1's
+    const unsigned char *w1s = smem + a.lds.w1, *w2s = smem + a.lds.w2;
+    _Float16 *hv = reinterpret_cast<_Float16 *>(smem + a.lds.hidden);   // [steps of mid][16 samples][32]: hidden vectors
+    float4_t *ps = reinterpret_cast<float4_t *>(smem + a.lds.sums);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int col = lane & 15, quad = lane >> 4;
+    const int n0 = by * kMmaSamples, ns = min(kMmaSamples, a.N - n0);
+    const int c0 = bx * kMmaChannels;
+    const int ktiles = (mid + kMmaStep - 1) / kMmaStep;  // steps of the second product
+    const int nk = C / kMmaStep;                         // steps of the first product
+    const int c4s = C >> 2;                              // vectors of four pooled values per sample
+    const bool together = a.lds.w2 != a.lds.w1;
+
+    // ---- weights, as they lie in memory, by `loaders` waves of which this is number w ----
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    // Rows r0 .. r0 + chunk of w1; row r's 16-byte chunk c in place c ^ (r & 15), so that the
+    // sixteen rows of an operand spread over the banks.  (A wave's rows are `loaders`, four or
+    // eight, loads apart: r & 15 comes round after four or two, the lanes' offsets are constants.)
+    auto stage_w1 = [&](int r0, int w, auto loader_waves) __attribute__((always_inline)) {
+        constexpr int LOADERS = decltype(loader_waves)::value;
+        const int rows = min(a.lds.chunk, mid - r0), chunks = C >> 3;
+        const char *base = reinterpret_cast<const char *>(a.w1 + (int64_t)r0 * C);
+        const uint32_t to = lds0 + a.lds.w1;
+        if (C <= 256) {
+            // two rows per load
+            constexpr int ROUND = 8 / LOADERS;
+            const int hi = lane >> 5;
+            int c[ROUND];
+#pragma unroll
+            for (int i = 0; i < ROUND; ++i) c[i] = (lane & 31) ^ (2 * (w + i * LOADERS) + hi);
+            for (int q0 = w; 2 * q0 < rows; q0 += 8)
+#pragma unroll
+                for (int i = 0; i < ROUND; ++i) {
+                    const int q = q0 + i * LOADERS;
+                    if (2 * q + hi < rows && c[i] < chunks)
+                        load_to_lds(to + q * 1024, base + q * (C * 4), (hi * chunks + c[i]) * 16);
+                }
+        } else {
+            constexpr int ROUND = 16 / LOADERS;
+            const int pieces = a.lds.pitch >> 10;
+            for (int piece = 0; piece < pieces; ++piece) {
+                int c[ROUND];
+#pragma unroll
+                for (int i = 0; i < ROUND; ++i) c[i] = (piece * kWave + lane) ^ (w + i * LOADERS);
+                for (int q0 = w; q0 < rows; q0 += 16)
+#pragma unroll
+                    for (int i = 0; i < ROUND; ++i) {
+                        const int r = q0 + i * LOADERS;
+                        if (r < rows && c[i] < chunks)
+                            load_to_lds(to + (r * pieces + piece) * 1024, base + r * (C * 2), c[i] * 16);
+                    }
+            }
+        }
+    };
+    // The KK rows of each of the block's channels: one run of bytes.
+    auto stage_w2 = [&](int w, int loaders) __attribute__((always_inline)) {
+        const int chunks = kMmaChannels * KK * mid / 8;
+        const char *base = reinterpret_cast<const char *>(a.w2 + (int64_t)c0 * KK * mid);
+        for (int q = w; q * kWave < chunks; q += loaders)
+            if (q * kWave + lane < chunks) load_to_lds(lds0 + a.lds.w2 + q * 1024, base + q * 1024, lane * 16);
+    };
+    // Half of the waves fetch the weights, the others the pooled vectors and what the threads
+    // that normalise will need (the first NORM_WAVES waves, a sample's channel per thread).
+    constexpr int kPoolWaves = 4;
+    static_assert(kPoolWaves == NORM_WAVES);
+    const int zs = tid / kMmaChannels, zc = tid % kMmaChannels;
+    struct Values { half8_t v[KK / 8]; _Float16 last; };    // a channel's KK contiguous values of a parameter
+    Values gain, offset, bias;
+    uint16_t b1v[4];    // biases of a wave's first tile of hidden values
+    auto request_bias = [&](int t) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t r = rows::plane_rsrc(a.b1, a.b1 ? (uint32_t)mid * 2u : 0u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            b1v[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, (t * 16 + quad * 4 + e) * 2, 0, 0);
+    };
+    // (hidden values past the last are zero)
+    if (tid < kMmaTile / 2) reinterpret_cast<uint32_t *>(hv + (ktiles - 1) * kMmaTile)[tid] = 0u;
+    static_assert(kMmaTile / 2 <= kMmaThreads);
+    if (wave >= kPoolWaves) {
+        stage_w1(0, wave - kPoolWaves, std::integral_constant<int, kMmaWaves - kPoolWaves>{});
+        if (together) stage_w2(wave - kPoolWaves, kMmaWaves - kPoolWaves);
+        request_bias(wave);
+    }
+
+    // ---- the pooled vectors: given, or scale * the sum of nparts partial sums per value ----
+    // A wave takes a sample, a lane four channels; where there are fewer samples than waves,
+    // several waves share a sample's partial sums, which meet in LDS.  (Samples there are only:
+    // the other columns of the products are read by nothing.)
+    auto put_pooled = [&](int s, int c4, half4_t v) __attribute__((always_inline)) {
+        *reinterpret_cast<half4_t *>(pv + ((c4 >> 3) * kMmaSamples + s) * kMmaStep + (c4 & 7) * 4) = v;
+        if constexpr (SAVE) {
+            if (a.save.pooled && bx == 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a.save.pooled[(int64_t)(n0 + s) * C + c4 * 4 + e] = (float)v[e];
+            }
+        }
+    };
+    auto scaled = [&](float4_t sum) __attribute__((always_inline)) {
+        half4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (_Float16)(sum[e] * a.scale);
+        return v;
+    };
+    const int share = !a.parts || C > kMmaSpread || a.nparts <= kMmaRound ? 1 : ns == 1 ? 4 : ns == 2 ? 2 : 1;
+    const int g = wave & (share - 1);    // (this wave's part of a sample's)
+    if (wave < kPoolWaves) {
+        const int stride = kPoolWaves / share;    // samples at a time
+        if (a.parts) {
+            // (a sample at a time behind a descriptor: beyond its partial sums there are zeros)
+            const uint32_t bytes = (uint32_t)(a.nparts * C) * 4u;
+            auto sample = [&](int s) __attribute__((always_inline)) {
+                return rows::plane_rsrc(a.parts + (int64_t)(n0 + min(s, ns - 1)) * a.nparts * C, s < ns ? bytes : 0u);
+            };
+            for (int s = wave / share; s < ns; s += 2 * stride) {
+                const __amdgpu_buffer_rsrc_t r[2] = {sample(s), sample(s + stride)};
+                for (int c4 = lane; c4 < c4s; c4 += kWave) {
+                    float4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                    for (int q0 = g; q0 < a.nparts; q0 += kMmaRound * share) {
+                        float4_t x[2][kMmaRound];
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+#pragma unroll
+                            for (int u = 0; u < kMmaRound; ++u)
+                                x[i][u] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                    r[i], c4 * 16, (q0 + u * share) * C * 4, 0));
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            sum[i] += ((x[i][0] + x[i][1]) + (x[i][2] + x[i][3])) + ((x[i][4] + x[i][5]) + (x[i][6] + x[i][7]));
+                    }
+                    if (share > 1) {    // (one sample per wave, one round of channels at most)
+                        ps[wave * kWave + lane] = sum[0];
+                    } else {
+                        put_pooled(s, c4, scaled(sum[0]));
+                        if (s + stride < ns) put_pooled(s + stride, c4, scaled(sum[1]));
+                    }
+                }
+            }
+        } else {
+            for (int s = wave; s < ns; s += kPoolWaves)
+                for (int c4 = lane; c4 < c4s; c4 += kWave)
+                    put_pooled(s, c4, *reinterpret_cast<const half4_t *>(a.pooled + (int64_t)(n0 + s) * C + c4 * 4));
+        }
+        auto get = [&](const __half *p, Values &to) __attribute__((always_inline)) {
+            // (no such parameter: anything that is there, C * KK values of it at least)
+            const __half *at = (p ? p : a.w2) + (int64_t)c0 * KK + (uint32_t)(zc * KK);
+#pragma unroll
+            for (int k = 0; k < KK / 8; ++k) __builtin_memcpy(&to.v[k], at + k * 8, sizeof(half8_t));
+            __builtin_memcpy(&to.last, at + KK - 1, 2);
+        };
+        request_bias(wave);
+        get(a.gain_vec, gain);
+        get(a.offset_vec, offset);
+        get(a.b2, bias);
+    }
+    if (share > 1) {
+        __syncthreads();
+        if (wave < kPoolWaves && g == 0 && wave / share < ns && lane < c4s) {
+            float4_t sum = ps[wave * kWave + lane];
+            for (int k = 1; k < share; ++k) sum += ps[(wave + k) * kWave + lane];
+            put_pooled(wave / share, lane, scaled(sum));
+        }
+    }
+    if (wave >= kPoolWaves) loads_to_lds_done();
+    __syncthreads();
+
+    // ---- hidden layer: tiles of sixteen rows of w1 dealt out to the waves ----
+    for (int r0 = 0; r0 < mid; r0 += a.lds.chunk) {
+        if (r0 > 0) {
+            __syncthreads();
+            stage_w1(r0, wave, std::integral_constant<int, kMmaWaves>{});
+            loads_to_lds_done();
+            __syncthreads();
+        }
+        const int rend = min(r0 + a.lds.chunk, mid);
+        for (int t = r0 / 16 + wave; t * 16 < rend; t += kMmaWaves) {
+            if (t != wave) request_bias(t);
+            const unsigned char *arow = w1s + (t * 16 + col - r0) * a.lds.pitch;
+            const _Float16 *brow = pv + col * kMmaStep + quad * 8;
+            float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            constexpr int U = 8;
+#pragma unroll 1
+            for (int k0 = 0; k0 < nk; k0 += U) {
+                half8_t av[U], bv[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int k = min(k0 + u, nk - 1);
+                    av[u] = *reinterpret_cast<const half8_t *>(arow + ((k * 4 + quad) ^ col) * 16);
+                    bv[u] = *reinterpret_cast<const half8_t *>(brow + k * kMmaTile);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (k0 + u < nk) acc[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[u], bv[u], acc[u & 1], 0, 0, 0);
+            }
+            // (rows past the last: zero)
+            half4_t h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = relu(acc[0][e] + acc[1][e] + (float)__builtin_bit_cast(_Float16, b1v[e]));
+                h[e] = t * 16 + quad * 4 + e < mid ? (_Float16)v : (_Float16)0;
+            }
+            *reinterpret_cast<half4_t *>(hv + ((t >> 1) * kMmaSamples + col) * kMmaStep + (t & 1) * 16 + quad * 4) = h;
+            if constexpr (SAVE) {
+                if (a.save.hidden && bx == 0 && col < ns) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int m = t * 16 + quad * 4 + e;
+                        if (m < mid) a.save.hidden[(int64_t)(n0 + col) * mid + m] = (float)h[e];
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (!together && a.lds.stage_w2) {
+        stage_w2(wave, kMmaWaves);
+        loads_to_lds_done();
+        __syncthreads();
+    }
+
+    // ---- taps: TPW taps of sixteen channels and samples per wave ----
+    float4_t acc[TPW];
+    if (wave < TAP_WAVES) {
+#pragma unroll
+        for (int j = 0; j < TPW; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+        const _Float16 *brow = hv + col * kMmaStep + quad * 8;
+        // (a tap past the last: the last again, not used)
+        uint32_t at[TPW];    // first of the lane's values in the row of channel col, tap j: halves
+#pragma unroll
+        for (int j = 0; j < TPW; ++j) at[j] = (uint32_t)((col * KK + min(wave * TPW + j, KK - 1)) * mid + quad * 8);
+        // Values t * 32 .. + 8 of them.  The row's last step ends with values of the next row
+        // (staged: whatever follows), which are made zero: times zero a NaN would stay one.
+        auto cut = [&](half8_t &v, int t) __attribute__((always_inline)) {
+            const int left = mid - t * kMmaStep - quad * 8;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (e >= left) v[e] = (_Float16)0;
+        };
+        auto staged = [&](int j, int t) __attribute__((always_inline)) {
+            // eight values from any even byte on: five words, shifted by half a word or not
+            const uint32_t *p = reinterpret_cast<const uint32_t *>(w2s + (at[j] * 2u & ~3u)) + t * (kMmaStep / 2);
+            const uint32_t by = (at[j] & 1u) * 16u;
+            uint4 q;
+            q.x = __builtin_amdgcn_alignbit(p[1], p[0], by);
+            q.y = __builtin_amdgcn_alignbit(p[2], p[1], by);
+            q.z = __builtin_amdgcn_alignbit(p[3], p[2], by);
+            q.w = __builtin_amdgcn_alignbit(p[4], p[3], by);
+            return __builtin_bit_cast(half8_t, q);
+        };
+        auto step = [&](int t, half8_t (&w)[TPW]) __attribute__((always_inline)) {
+            const half8_t b = *reinterpret_cast<const half8_t *>(brow + t * kMmaTile);
+#pragma unroll
+            for (int j = 0; j < TPW; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[j], b, acc[j], 0, 0, 0);
+        };
+        if (a.lds.stage_w2) {
+            int t = 0;
+#pragma unroll 1
+            for (; t + 2 < ktiles; t += 2) {
+                half8_t w[2][TPW];
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < TPW; ++j) w[i][j] = staged(j, t + i);
+                step(t, w[0]);
+                step(t + 1, w[1]);
+            }
+            if (t + 1 < ktiles) {
+                half8_t w[TPW];
+#pragma unroll
+                for (int j = 0; j < TPW; ++j) w[j] = staged(j, t);
+                step(t++, w);
+            }
+            half8_t w[TPW];
+#pragma unroll
+            for (int j = 0; j < TPW; ++j) {
+                w[j] = staged(j, t);
+                cut(w[j], t);
+            }
+            step(t, w);
+        } else {
+            const __half *base = a.w2 + (int64_t)c0 * KK * mid;
+#pragma unroll 1
+            for (int t = 0; t < ktiles; ++t) {
+                half8_t w[TPW];
+#pragma unroll
+                for (int j = 0; j < TPW; ++j) {
+                    if (t + 1 < ktiles) {
+                        __builtin_memcpy(&w[j], base + at[j] + t * kMmaStep, sizeof(w[j]));
+                    } else {
+                        const int left = mid - t * kMmaStep - quad * 8;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            w[j][e] = e < left ? *reinterpret_cast<const _Float16 *>(base + at[j] + t * kMmaStep + e) : (_Float16)0;
+                    }
+                }
+                step(t, w);
+            }
+        }
+    }
+    if (a.lds.shared) __syncthreads();
+    if (wave < TAP_WAVES) {
+#pragma unroll
+        for (int j = 0; j < TPW; ++j)
+            if (wave * TPW + j < KK) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) z[col * ZP + (quad * 4 + e) * KK + wave * TPW + j] = acc[j][e];
+            }
+    }
+    __syncthreads();
+    if (wave >= NORM_WAVES || zs >= ns) return;
+    float u[KK];
+    TapParams<__half, KK> params;
+#pragma unroll
+    for (int j = 0; j < KK; ++j) {
+        auto value = [&](const Values &p) __attribute__((always_inline)) { return (float)(j < KK - 1 ? p.v[j / 8][j % 8] : p.last); };
+        u[j] = z[zs * ZP + zc * KK + j];
+        params.gain[j] = a.gain_vec ? value(gain) : a.gain;
+        params.offset[j] = a.offset_vec ? value(offset) : 0.f;
+        params.bias[j] = a.b2 ? value(bias) : 0.f;
+    }
+    const int64_t to = ((int64_t)(n0 + zs) * C + c0 + zc) * KK;
+    if constexpr (SAVE) {
+        if (a.save.taps) {
+#pragma unroll
+            for (int j = 0; j < KK; ++j) a.save.taps[to + j] = u[j] + params.bias[j];
+        }
+    }
+    normalise<__half, KK>(u, params);
+    __half *op = a.cf + to;
+#pragma unroll
+    for (int k = 0; k < KK / 8; ++k) {
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)u[k * 8 + e];
+        __builtin_memcpy(op + k * 8, &o, sizeof(o));
+    }
+    st(op + KK - 1, u[KK - 1]);
+}
+
+#endif  // __HIPCC__
+
+}  // namespace ddf

@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "ddf_channel.h"
 #include "ddf_common.h"
 #include "ddf_rows.h"
 
@@ -32,9 +33,6 @@ using rows::kOutside;
 using rows::load_words;
 using rows::plane_rsrc;
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t rows_u4 __attribute__((ext_vector_type(4)));
 
@@ -116,13 +114,6 @@ template <int N>
 __device__ __forceinline__ void arrive() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
-// 16 bytes per lane to LDS at `lds` + lane * 16.  (Written out because the compiler waits for
-// every such load in flight before any LDS read.  The address is an operand in m0, so that the
-// compiler itself writes m0 and knows it; the load must not follow that write at once.)
-__device__ __forceinline__ void load_to_lds(uint32_t lds, const _Float16 *p) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
-}
-
 template <int BM, int BN, int KST, int ST, int WG, bool PAIR>
 __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, int tiles_n, int tiles) {
     constexpr int CH = KST / 8, STAGE = (BM + BN) * KST;

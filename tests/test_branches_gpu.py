@@ -234,3 +234,29 @@ def test_channel_branch_one_sample_per_workgroup(n, c, mid, tiles, dtype, tol):
     ref = channel_reference(parts.double().sum(1).cpu(), *(t.cpu() for t in (w1, b1, w2, b2)), k, 0.7, None, None)
     err = ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item()
     assert err < tol, err
+
+
+@pytest.mark.parametrize('n,c,mid,tiles,k', [
+    (1, 256, 51, 13, 3), (2, 256, 64, 9, 3), (3, 192, 33, 17, 3),   # a sample's partial sums over four waves, two, one
+    (1, 32, 32, 33, 3), (1, 32, 129, 5, 3),                         # one step of channels; more tiles than waves
+    (2, 288, 57, 3, 3), (17, 544, 108, 4, 3),                       # rows of w1 in one piece of 1 KB, in two
+    (1, 1024, 204, 2, 3), (1, 1664, 332, 1, 3),                     # w1 in parts, then w2 in its place
+    (1, 512, 512, 2, 3), (2, 1024, 204, 2, 5),                      # w2 from memory
+    (18, 64, 96, 9, 5), (1, 32, 32, 1, 5),                          # taps where rows of w2 were
+])
+def test_channel_branch_weights_through_lds(n, c, mid, tiles, k):
+    """fp16 on the matrix cores: every way the weights take into LDS; and an infinite weight
+    reaches the taps of its own channel only (rows end inside a step)."""
+    torch.manual_seed(c + mid)
+    parts = torch.randn(n, tiles, c, device='cuda')
+    w1 = (torch.randn(mid, c, device='cuda') * c ** -0.5).half()
+    w2 = (torch.randn(c * k * k, mid, device='cuda') * mid ** -0.5).half()
+    b1, b2 = torch.randn(mid, device='cuda').half(), torch.randn(c * k * k, device='cuda').half()
+    out = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, None, None)
+    ref = channel_reference(parts.double().sum(1).cpu(), *(t.cpu() for t in (w1, b1, w2, b2)), k, 0.7, None, None)
+    err = ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item()
+    assert err < 6e-3, err      # (pooled and hidden values rounded to 11 bits, see above)
+    w2[(c // 2) * k * k, 0] = float('inf')
+    got = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, None, None).view(n, c, -1)
+    rest = [i for i in range(c) if i != c // 2]
+    assert torch.equal(got[:, rest], out.view(n, c, -1)[:, rest])
