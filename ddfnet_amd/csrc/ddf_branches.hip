@@ -10,10 +10,11 @@
 //   average pool:
 //     cf[n, c, t] = norm_t( b2[c*KK + t] + sum_m w2[c*KK + t, m] * relu(b1[m] + sum_c' w1[m, c'] * v[n, c']) )
 //   the two 1x1 convolutions on the pooled (n, c) vector are small matrix
-//   products; one workgroup computes the hidden vector of its sample and 64
-//   (wide layers: 128) channels' filters, and normalises them in place
-//   (k_channel_branch), or, in fp16 with a hidden layer of 32 values or more,
-//   sixteen samples x sixteen channels on the matrix cores (k_channel_branch_mma).
+//   products (ddf_channel.h): one workgroup computes the hidden vector of its sample and 16
+//   to 64 channels' filters out of LDS (k_channel_branch_rows), or, in fp16 with a hidden
+//   layer of 32 values or more, sixteen samples x sixteen channels on the matrix cores
+//   (k_channel_branch_mma); large batches, 5 x 5 taps and unaligned weights go through
+//   k_channel_branch, whose loads serve several samples.
 //
 // norm_t(u) = gain_t * (u_t - mean(u)) / (std(u) + 1e-10) + offset_t with the
 // unbiased standard deviation over the KK taps, as in ddf_filter_norm.hip.
@@ -558,8 +559,14 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
 // out[n * C + c] = sum of parts[(n * nparts + p) * C + c] over p.  Every workgroup of the
 // channel branch starts from the pooled vectors; with dozens of partial sums per value each
 // of them would spend longer adding up than on its own work (8 x 64 x 200 x 300 fp16: 472
-// sums per value then, 37 of the layer's 107 us), so planes of many tiles pay for one launch.
-constexpr int kMaxParts = 8;             // partial sums the channel branch reads in one round trip
+// sums per value then, 37 of the layer's 107 us), so planes of many tiles pay for one launch,
+// unless a sample's few channels leave the workgroup waves enough to share a value's sums.
+constexpr int kMaxParts = 8;             // partial sums per value the channel branch is left at least
+// (two rounds of requests; 118 sums of 64 channels 5.1 us, 4.1 with few, and the launch 4.7)
+inline int64_t channel_parts_left(int64_t N, int64_t C) {
+    const int64_t width = cdiv(C, kWave);
+    return N * width <= 256 && width <= 4 ? 2 * kMaxParts * (kRowsPoolWaves / width) : kMaxParts;
+}
 constexpr int kCollapseChannels = 64, kCollapseGroups = 8;
 __global__ __launch_bounds__(kCollapseChannels * kCollapseGroups) void k_collapse_parts(
     const float *__restrict__ parts, float *__restrict__ out, int C, int nparts) {
@@ -582,34 +589,6 @@ __global__ __launch_bounds__(kCollapseChannels * kCollapseGroups) void k_collaps
     }
 }
 
-// Butterfly steps through the VALU's lane-permute path.  (Shuffles through the
-// LDS crossbar cost a round trip each and made these kernels several times slower.)
-template <int CTRL>
-__device__ __forceinline__ float add_permuted(float x) {
-    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-// Sum over each row of 16 lanes (the same value in every lane of the row).
-__device__ __forceinline__ float row_sum(float v) {
-    v = add_permuted<0xB1>(v);    // quad_perm [1,0,3,2]
-    v = add_permuted<0x4E>(v);    // quad_perm [2,3,0,1]
-    v = add_permuted<0x141>(v);   // row_half_mirror
-    return add_permuted<0x140>(v);   // row_mirror
-}
-
-// A value as it lies in memory, in a register of its own (halves that share one load one after
-// the other); zero past the buffer's end.
-template <typename T>
-__device__ __forceinline__ uint32_t ld_bits(__amdgpu_buffer_rsrc_t r, uint32_t index) {
-    const int at = (int)(index * (uint32_t)sizeof(T));
-    if constexpr (sizeof(T) == 2) return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0);
-    else return __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0);
-}
-template <typename T>
-__device__ __forceinline__ float of_bits(uint32_t bits) {
-    if constexpr (sizeof(T) == 2) return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
-    else return __builtin_bit_cast(float, bits);
-}
-
 constexpr int kChannelThreads = 1024;  // sixteen waves: the rows of a block's taps are dealt out to them
 constexpr int kChannelWaves = kChannelThreads / kWave;
 
@@ -621,7 +600,7 @@ constexpr int kChannelWaves = kChannelThreads / kWave;
 // workgroup of a sample recomputes the hidden vector, so the blocks are large:
 // smaller ones had all compute units read the same rows of w1 at once, which
 // the L2 serves one after the other.
-template <typename T, int KK, int BLOCK, int NS, int AHEAD = 0>
+template <typename T, int KK, int BLOCK, int NS>
 __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const T *__restrict__ pooled, const T *__restrict__ w1, const T *__restrict__ b1,
     const T *__restrict__ w2, const T *__restrict__ b2, T *__restrict__ cf, int N, int C, int mid,
@@ -635,55 +614,10 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const int64_t n0 = (int64_t)blockIdx.y * NS;
     const int ns = min(NS, N - (int)n0);   // samples of this workgroup (the others: copies of the last)
     const int cb = blockIdx.x * BLOCK;
-    // One sample per workgroup: few workgroups, and their time is the round trips to memory.
-    // What does not depend on the pooled vector is requested along with it: the wave's rows of w1
-    // (C <= 64 * AHEAD values each) and w2 (mid <= 16 * AHEAD), the biases, the gains and offsets;
-    // without branches, which would end in a wait each (absent values lie
-    // outside their buffers).  Six round trips, one after the other, become one: 8 samples of 64
-    // channels fp16 6.9 -> 4.9 us, one of 128 9.3 -> 6.3, 128 of 128 9.9 -> 7.0, 32 of 256 fp32
-    // 11.0 -> 9.2 (loads of halves into shared registers, or under branches: 10 to 13 us).
-    constexpr bool kAhead = AHEAD > 0;
-    static_assert(!kAhead || (NS == 1 && KK == 9 && BLOCK == 64));
     constexpr int RT = NS >= 4 ? 1 : NS == 2 ? 2 : 3;
-    constexpr int GROUPS = kAhead ? BLOCK * KK / (kChannelWaves * 4) : 1, A1 = kAhead ? 4 * AHEAD : 1, A2 = kAhead ? AHEAD : 1;
     const int seg = lane >> 4, sl = lane & 15;
     const int rows = min(BLOCK, C - cb) * KK;
-    uint32_t w1a[A1], w2a[GROUPS][A2], b1a = 0, b2a[GROUPS], ga[KK] = {}, oa[KK] = {};
-    float part[kMaxParts];
     TapParams<T, KK> params;
-    const bool parts_ahead = kAhead && parts && nparts <= kMaxParts;
-    if constexpr (kAhead) {
-        constexpr uint32_t kNone = kOutside / sizeof(T);
-        auto buffer = [](const T *p, int count) { return plane_rsrc(p, p ? (uint32_t)count * (uint32_t)sizeof(T) : 0u); };
-        const int tid = threadIdx.x;
-        const __amdgpu_buffer_rsrc_t pr = plane_rsrc(parts + (parts ? n0 * nparts * C : 0), parts_ahead ? (uint32_t)(nparts * C) * 4u : 0u);
-#pragma unroll
-        for (int q = 0; q < kMaxParts; ++q)
-            part[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr, tid < C ? (q * C + tid) * 4 : (int)kOutside, 0, 0));
-        const __amdgpu_buffer_rsrc_t w1r = buffer(w1, mid * C), b1r = buffer(b1, mid);
-        const int m = wave * 4 + seg;
-#pragma unroll
-        for (int i = 0; i < A1; ++i) w1a[i] = ld_bits<T>(w1r, m < mid && sl + i * 16 < C ? (uint32_t)(m * C + sl + i * 16) : kNone);
-        b1a = ld_bits<T>(b1r, (uint32_t)m);
-        const __amdgpu_buffer_rsrc_t w2r = buffer(w2, C * KK * mid), b2r = buffer(b2, C * KK);
-#pragma unroll
-        for (int t = 0; t < GROUPS; ++t) {
-            const int r = (t * kChannelWaves + wave) * 4 + seg;
-#pragma unroll
-            for (int i = 0; i < A2; ++i)
-                w2a[t][i] = ld_bits<T>(w2r, r < rows && sl + i * 16 < mid ? (uint32_t)((cb * KK + r) * mid + sl + i * 16) : kNone);
-            b2a[t] = ld_bits<T>(b2r, r < rows ? (uint32_t)(cb * KK + r) : kNone);
-        }
-        const __amdgpu_buffer_rsrc_t gr = buffer(gain_vec, C * KK), orr = buffer(offset_vec, C * KK);
-        if (tid < BLOCK) {
-#pragma unroll
-            for (int t = 0; t < KK; ++t) {
-                ga[t] = ld_bits<T>(gr, (uint32_t)((cb + tid) * KK + t));
-                oa[t] = ld_bits<T>(orr, (uint32_t)((cb + tid) * KK + t));
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
     // the pooled vectors: given, or scale * the sum of nparts partial sums per value
     // (parts[(n * nparts + p) * C + c], what k_spatial_stream leaves)
     for (int i = threadIdx.x; i < NS * C; i += kChannelThreads) {
@@ -691,13 +625,8 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         const int64_t n = n0 + min(s, ns - 1);
         if (parts) {
             float a = 0.f;
-            if (parts_ahead && i == (int)threadIdx.x) {
-#pragma unroll
-                for (int q = 0; q < kMaxParts; ++q) a += part[q];
-            } else {
 #pragma unroll 8
-                for (int q = 0; q < nparts; ++q) a += parts[(n * nparts + q) * C + c];
-            }
+            for (int q = 0; q < nparts; ++q) a += parts[(n * nparts + q) * C + c];
             v[i] = a * scale;
         } else {
             v[i] = ld(pooled + n * C + c);
@@ -716,19 +645,13 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
 #pragma unroll
         for (int s = 0; s < NS; ++s) p[s] = 0.f;
         int c = sl;
-        const bool ahead = kAhead && m0 == wave * 4;
-        if (ahead) {
-#pragma unroll
-            for (int i = 0; i < A1; ++i, c += 16)
-                if (c < C) p[0] = fmaf(of_bits<T>(w1a[i]), v[c], p[0]);
-        }
 #pragma unroll 8
         for (; c < C; c += 16) {
             const float wv = ld(row + c);
 #pragma unroll
             for (int s = 0; s < NS; ++s) p[s] = fmaf(wv, v[s * C + c], p[s]);
         }
-        const float bias = ahead ? of_bits<T>(b1a) : b1 ? ld(b1 + m) : 0.f;
+        const float bias = b1 ? ld(b1 + m) : 0.f;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const float tot = row_sum(p[s]);
@@ -748,18 +671,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
             if (save.taps && s < ns) save.taps[((n0 + s) * C + cb) * KK + r] = tot + bias;
         }
     };
-    if constexpr (kAhead) {
-#pragma unroll
-        for (int t = 0; t < GROUPS; ++t) {
-            const int r = (t * kChannelWaves + wave) * 4 + seg;
-            float p = 0.f;
-            int m = sl;
-#pragma unroll
-            for (int i = 0; i < A2; ++i, m += 16)
-                if (m < mid) p = fmaf(of_bits<T>(w2a[t][i]), h[m], p);
-            emit(r, 0, p, of_bits<T>(b2a[t]));
-        }
-    } else for (int r0 = wave * 4 * RT; r0 < rows; r0 += kChannelWaves * 4 * RT) {
+    for (int r0 = wave * 4 * RT; r0 < rows; r0 += kChannelWaves * 4 * RT) {
         float p[RT][NS];
         const T *wrow[RT];
 #pragma unroll
@@ -796,15 +708,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         float u[KK];
 #pragma unroll
         for (int t = 0; t < KK; ++t) u[t] = f[(s * BLOCK + ch) * KK + t];
-        if constexpr (kAhead) {
-#pragma unroll
-            for (int t = 0; t < KK; ++t) {
-                params.gain[t] = gain_vec ? of_bits<T>(ga[t]) : gain;
-                params.offset[t] = of_bits<T>(oa[t]);
-                params.bias[t] = 0.f;
-            }
-        } else
-            params.load(cb + ch, gain, gain_vec, offset_vec, (const T *)nullptr);   // (b2 is in f already)
+        params.load(cb + ch, gain, gain_vec, offset_vec, (const T *)nullptr);   // (b2 is in f already)
         normalise<T, KK>(u, params);
         T *op = cf + ((n0 + s) * C + cb + ch) * KK;
 #pragma unroll
@@ -812,6 +716,11 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     }
 }
 
+template <typename T, bool SAVE>
+__global__ __launch_bounds__(kRowsThreads) void k_channel_branch_rows(ChannelRows<T> a) {
+    extern __shared__ __align__(16) unsigned char rows_smem[];
+    channel_rows<T, SAVE>(a, blockIdx.x, blockIdx.y, rows_smem);
+}
 
 template <int KK, bool SAVE>
 __global__ __launch_bounds__(kMmaThreads) void k_channel_branch_mma(ChannelMma a) {
@@ -889,9 +798,9 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     if (N > 65535 || head > 65535) return hipErrorNotSupported;
     bool collapse = false;
     if (pool) {
-        // (more tiles than kMaxParts: their sums go behind the N * C totals that
-        // k_collapse_parts then makes of them)
-        collapse = tiles > kMaxParts;
+        // (more tiles than the channel branch is left: their sums go behind the N * C totals
+        // that k_collapse_parts then makes of them)
+        collapse = tiles > tune_int("DDF_TUNE_COLLAPSE", (int)channel_parts_left(N, C));
         if (N * (tiles + (collapse ? 1 : 0)) * C > pool_capacity) return hipErrorInvalidValue;
         *pool_parts = collapse ? 1 : tiles;
     }
@@ -1057,6 +966,18 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
                                           offset_vec, st, parts, nparts, scale, save);
         e != hipErrorNotSupported)
         return e;
+    if (k == 3) {
+        ChannelRows<T> a{pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain, gain_vec, offset_vec,
+                         parts, nparts, (float)scale, save};
+        if (channel_rows_plan(a) && N * cdiv(C, a.block) <= tune_int("DDF_TUNE_CHANNEL_ROWS", 1 << 30)) {
+            const dim3 grid((unsigned)cdiv(C, a.block), (unsigned)N);
+            if (save.pooled || save.hidden || save.taps)
+                hipLaunchKernelGGL((k_channel_branch_rows<T, true>), grid, dim3(kRowsThreads), a.total, st, a);
+            else
+                hipLaunchKernelGGL((k_channel_branch_rows<T, false>), grid, dim3(kRowsThreads), a.total, st, a);
+            return hipGetLastError();
+        }
+    }
     // (wide layers: fewer, larger blocks, as every block of a sample recomputes the hidden vector)
     const int block = C >= 512 ? 128 : 64;
     // samples per workgroup: as many as keep every compute unit busy and fit the LDS
@@ -1078,24 +999,11 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
         else if (ns == 2) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 2);                                    \
         else DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 1);                                                 \
     } while (0)
-#define DDF_CHANNEL_AHEAD(A_)                                                                          \
-    hipLaunchKernelGGL((k_channel_branch<T, 9, 64, 1, A_>), grid, dim3(kChannelThreads), lds, st,     \
-                       pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain, gain_vec,   \
-                       offset_vec, parts, nparts, (float)scale, save)
-    // Requests ahead of all weights of a layer of up to 256 channels and 64 hidden values, where
-    // every workgroup has a compute unit of its own (their registers leave no room for a second
-    // one: 48 samples x 432 channels, 336 workgroups, layer 61 us ahead, 49 not; 36 x 424, 252
-    // workgroups and weights left over, 38 and 33).
-    if (k == 3 && block == 64 && ns == 1 && C <= 256 && mid <= 64 && (int64_t)grid.x * grid.y <= 256) {
-        if (C <= 64 && mid <= 16) DDF_CHANNEL_AHEAD(1);
-        else if (C <= 128 && mid <= 32) DDF_CHANNEL_AHEAD(2);
-        else DDF_CHANNEL_AHEAD(4);
-    } else if (k == 3 && block == 64) DDF_CHANNEL_CASE(9, 64);
+    if (k == 3 && block == 64) DDF_CHANNEL_CASE(9, 64);
     else if (k == 3) DDF_CHANNEL_CASE(9, 128);
     else if (k == 5 && block == 64) DDF_CHANNEL_CASE(25, 64);
     else if (k == 5) DDF_CHANNEL_CASE(25, 128);
     else return hipErrorNotSupported;
-#undef DDF_CHANNEL_AHEAD
 #undef DDF_CHANNEL_LAUNCH
 #undef DDF_CHANNEL_CASE
     return hipGetLastError();

@@ -1,6 +1,7 @@
-// The channel filter branch of DDFPack on the matrix cores (fp16), as a device function: the
-// layer's kernel (ddf_branches.hip) is nothing else, a network's runs it beside the spatial
-// branch (ddf_net.hip).
+// The channel filter branch of DDFPack with its weights in LDS, as device functions: on the
+// matrix cores (channel_mma, fp16) and on the vector ALU (channel_rows).  A layer's kernels
+// (ddf_branches.hip) are nothing else, a network's run them beside the spatial branch
+// (ddf_net.hip).
 #pragma once
 
 #include <algorithm>
@@ -23,7 +24,7 @@ namespace ddf {
 //   * the hidden layer goes to LDS as [32 values][sample][32], rounded to fp16 (as
 //     the reference's first convolution does);
 //   * the rows of tile j of the second product are (channel c0 + i, tap j); the taps meet in
-//     LDS as fp32, and a thread per sample and pair of channels normalises and stores them.
+//     LDS as fp32, and a thread per sample and channel normalises and stores them.
 // mid is no multiple of 16 or 32: rows of w1 past the last are whatever lies in LDS and make
 // hidden values that are set to zero; the last step of a row of w2 is cut at its end.
 //
@@ -47,7 +48,7 @@ constexpr int kMmaLds = 160 * 1024;
 
 // LDS, bytes: pooled vectors | rows of w1 | the block's rows of w2 | hidden vectors | partial
 // sums on their way to the pooled vectors.  All rows of w1 and w2 where they fit; else w1 by
-// `chunk` rows and w2 in the same place after it, or (chunk_w2 false) from memory.  The block's
+// `chunk` rows and w2 in the same place after it, or (stage_w2 false) from memory.  The block's
 // taps go where w1 and the pooled vectors were.
 struct ChannelMmaLds {
     int pitch;                  // bytes of a row of w1
@@ -523,6 +524,297 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by,
         __builtin_memcpy(op + k * 8, &o, sizeof(o));
     }
     st(op + KK - 1, u[KK - 1]);
+}
+
+#endif  // __HIPCC__
+
+// ---- one sample per workgroup, on the vector ALU (3 x 3 taps) ----------------------------
+// A workgroup of sixteen waves takes one sample and `block` channels.  All of w1 and the block's
+// rows of w2 come into LDS as runs of bytes, requested by one half of the waves while the other
+// adds up the pooled vector; sixteen lanes then take a row, four rows a wave at a time.  Read
+// straight from memory by those lanes, a row is 32 or 64 bytes per load: 880 loads of a quarter
+// KB for 256 fp32 channels, which is what the launch waited for, where 110 of 1 KB do.  Sums
+// and what passes between the layers are fp32.  us a launch, straight from memory / now: fp32,
+// samples x channels, 32 x 256 7.9 / 5.1, 8 x 512 24.5 / 8.6, 64 x 128 6.1 / 4.2; fp16, 128 x 128
+// 6.3 / 5.1, 32 x 432 16.8 / 9.1; 8 x 64 with 118 partial sums per value 15.2 / 5.1.
+constexpr int kRowsKK = 9;
+constexpr int kRowsThreads = 1024, kRowsWaves = kRowsThreads / kWave, kRowsPoolWaves = kRowsWaves / 2;
+constexpr int kRowsMaxBlock = 64;
+
+template <typename T>
+struct ChannelRows {
+    const T *pooled, *w1, *b1, *w2, *b2;
+    T *cf;
+    int N, C, mid;
+    float gain;
+    const T *gain_vec, *offset_vec;
+    const float *parts;    // (nparts per sample; null: `pooled`)
+    int nparts;
+    float scale;
+    ChannelSave save;
+    // LDS, bytes: pooled vector, hidden vector, taps, partial sums | w1 by `chunk` rows | the
+    // first `early` of the block's rows of w2, the others where w1 was
+    int block, chunk, early, w1_at, w2_at, total;
+};
+// The layout for blocks of `block` channels; false: rows too long.
+template <typename T>
+inline bool channel_rows_lds(ChannelRows<T> &a, int block) {
+    const int64_t row1 = (int64_t)a.C * sizeof(T), row2 = (int64_t)a.mid * sizeof(T), rows = (int64_t)block * kRowsKK;
+    a.block = block;
+    a.w1_at = mma_round(((int64_t)a.C + a.mid + rows + kRowsPoolWaves * kWave) * 4);
+    const int64_t left = kMmaLds - a.w1_at - 32;
+    if (left < 8 * row1) return false;
+    // (parts of eight rows are whole 16 bytes)
+    a.chunk = a.mid * row1 <= left ? a.mid : (int)(left / row1 / 8 * 8);
+    const int64_t w1 = mma_round(a.chunk * row1);
+    a.early = (int)std::min(rows, std::max<int64_t>((left - w1) / row2, 0) / 8 * 8);
+    a.w2_at = a.w1_at + (int)w1;
+    a.total = a.w2_at + mma_round(a.early * row2);
+    return (rows - a.early) * row2 <= w1;
+}
+// Blocks of 16, 32 or 64 channels: the smallest that give every compute unit one workgroup at
+// most.  False: not covered.  (Where there are more workgroups, loads that serve several samples
+// are faster: 512 x 64 fp32 6.4 us and 9.6 here, 128 x 256 12.8 and 16.2, 48 x 432 fp16 20.5 and
+// 19.3.  Weights must be whole 16 bytes from their start on.)
+template <typename T>
+inline bool channel_rows_plan(ChannelRows<T> &a) {
+    auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    if (!aligned(a.w1) || !aligned(a.w2) || a.mid < 1 || a.C < 1) return false;
+    if ((int64_t)a.C * a.mid * kRowsKK * (int64_t)sizeof(T) >= ((int64_t)1 << 31)) return false;
+    for (int block = 16; block <= kRowsMaxBlock; block *= 2)
+        if ((int64_t)a.N * ((a.C + block - 1) / block) <= 256) return channel_rows_lds(a, block);
+    return false;
+}
+
+#ifdef __HIPCC__
+
+// Butterfly steps through the VALU's lane-permute path.  (Shuffles through the
+// LDS crossbar cost a round trip each and made these kernels several times slower.)
+template <int CTRL>
+__device__ __forceinline__ float add_permuted(float x) {
+    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+// Sum over each row of 16 lanes (the same value in every lane of the row).
+__device__ __forceinline__ float row_sum(float v) {
+    v = add_permuted<0xB1>(v);    // quad_perm [1,0,3,2]
+    v = add_permuted<0x4E>(v);    // quad_perm [2,3,0,1]
+    v = add_permuted<0x141>(v);   // row_half_mirror
+    return add_permuted<0x140>(v);   // row_mirror
+}
+
+
+// Block (bx, by) of (channel blocks, samples), kRowsThreads threads.
+template <typename T, bool SAVE>
+__device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, int by, unsigned char *smem) {
+    constexpr int KK = kRowsKK, VE = 16 / sizeof(T);
+    const int C = a.C, mid = a.mid;
+    float *v = reinterpret_cast<float *>(smem);     // [C]
+    float *h = v + C;                               // [mid]
+    float *f = h + mid;                             // [block * KK]
+    float *sums = f + a.block * KK;                 // [pool waves][64]
+    const T *w1s = reinterpret_cast<const T *>(smem + a.w1_at), *w2s = reinterpret_cast<const T *>(smem + a.w2_at);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int64_t n = by;
+    const int cb = bx * a.block, channels = min(a.block, C - cb), rows = channels * KK;
+    const int early = min(a.early, rows);           // rows of w2 that come in with w1
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+
+    // `count` values from `from` (whole 16 bytes into its tensor) on to LDS, by `loaders` waves
+    // of which this is number w; the last ones that fill no 16 bytes one by one.
+    auto stage = [&](const T *from, int count, int to, int w, int loaders) __attribute__((always_inline)) {
+        const char *base = reinterpret_cast<const char *>(from);
+        const int chunks = count / VE, whole = chunks / kWave;
+        int q = w;
+        for (; q < whole; q += loaders) load_to_lds(lds0 + to + q * 1024, base + q * 1024, lane * 16);
+        if (q == whole) {
+            if (q * kWave + lane < chunks) load_to_lds(lds0 + to + q * 1024, base + q * 1024, lane * 16);
+            const int at = chunks * VE + lane;
+            if (at < count) *reinterpret_cast<T *>(smem + to + at * (int)sizeof(T)) = from[at];
+        }
+    };
+    T gain[KK] = {}, offset[KK] = {}, bias[KK] = {};
+    // (a lane of the first waves takes a channel of the pooled vector; of many partial sums several
+    // waves share a channel's; the others fetch the weights)
+    const int width = (C + kWave - 1) / kWave;      // waves side by side
+    const int share = a.parts && a.nparts > kMmaRound && width <= kRowsPoolWaves / 2 ? kRowsPoolWaves / width : 1;
+    const int pool_waves = min(width * share, kRowsPoolWaves);
+    if (wave >= pool_waves) {
+        stage(a.w1, min(a.chunk, mid) * C, a.w1_at, wave - pool_waves, kRowsWaves - pool_waves);
+        stage(a.w2 + (int64_t)cb * KK * mid, early * mid, a.w2_at, wave - pool_waves, kRowsWaves - pool_waves);
+    }
+
+    const int seg = lane >> 4, sl = lane & 15;
+    const float b1_first = a.b1 ? ld(a.b1 + min(wave * 4 + seg, mid - 1)) : 0.f;
+
+    // The pooled vector: given, or scale * the sum of nparts partial sums per value.
+    const int g = wave / width;
+    if (wave < pool_waves) {
+        auto put = [&](int c, float x) __attribute__((always_inline)) {
+            v[c] = x;
+            if constexpr (SAVE) {
+                if (a.save.pooled && bx == 0) a.save.pooled[n * C + c] = x;
+            }
+        };
+        if (a.parts) {
+            const __amdgpu_buffer_rsrc_t r = rows::plane_rsrc(a.parts + n * a.nparts * C, (uint32_t)(a.nparts * C) * 4u);
+            for (int c = (share > 1 ? wave - g * width : wave) * kWave + lane; c < width * kWave;
+                 c += kRowsPoolWaves * kWave) {
+                float sum = 0.f;
+                for (int q0 = share > 1 ? g : 0; q0 < a.nparts; q0 += kMmaRound * share) {
+                    float x[kMmaRound];    // (beyond the last: zeros)
+#pragma unroll
+                    for (int u = 0; u < kMmaRound; ++u) {
+                        const int q = q0 + u * share;
+                        x[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                            r, c < C && q < a.nparts ? c * 4 : (int)rows::kOutside, q * C * 4, 0));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    sum += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+                }
+                if (share > 1) sums[wave * kWave + lane] = sum;
+                else if (c < C) put(c, sum * a.scale);
+            }
+        } else {
+            for (int c = tid; c < C; c += pool_waves * kWave) put(c, ld(a.pooled + n * C + c));
+        }
+        // gains, offsets and biases of the channel that the thread normalises
+        if (tid < channels) {
+            const int64_t at = (int64_t)(cb + tid) * KK;
+            auto get = [&](const T *p, T (&to)[KK]) __attribute__((always_inline)) {
+                if (p) __builtin_memcpy(to, p + at, sizeof(to));
+            };
+            get(a.gain_vec, gain);
+            get(a.offset_vec, offset);
+            get(a.b2, bias);
+        }
+    }
+    if (share > 1) {
+        __syncthreads();
+        if (wave < width && tid < C) {
+            float sum = sums[tid];
+            for (int k = 1; k < share; ++k) sum += sums[(k * width + wave) * kWave + lane];
+            v[tid] = sum * a.scale;
+            if constexpr (SAVE) {
+                if (a.save.pooled && bx == 0) a.save.pooled[n * C + tid] = sum * a.scale;
+            }
+        }
+    }
+    if (wave >= pool_waves) loads_to_lds_done();
+    __syncthreads();
+
+    // ---- hidden vector: rows of w1, sixteen lanes each ----
+    for (int r0 = 0; r0 < mid; r0 += a.chunk) {
+        if (r0 > 0) {
+            __syncthreads();
+            stage(a.w1 + (int64_t)r0 * C, min(a.chunk, mid - r0) * C, a.w1_at, wave, kRowsWaves);
+            loads_to_lds_done();
+            __syncthreads();
+        }
+        const int rend = min(r0 + a.chunk, mid);
+        for (int m0 = r0 + wave * 4; m0 < rend; m0 += kRowsWaves * 4) {
+            const int m = min(m0 + seg, rend - 1);
+            const float b = m0 == wave * 4 ? b1_first : a.b1 ? ld(a.b1 + m) : 0.f;
+            const T *row = w1s + (m - r0) * C;
+            float p = 0.f;
+            if (C % VE == 0) {
+                const int vectors = C / VE;
+#pragma unroll 2
+                for (int j = sl; j < vectors; j += 16) {
+                    T w[VE];
+                    float x[VE];
+                    __builtin_memcpy(w, __builtin_assume_aligned(row + j * VE, 16), sizeof(w));
+#pragma unroll
+                    for (int e = 0; e < VE; e += 4)
+                        __builtin_memcpy(x + e, __builtin_assume_aligned(v + j * VE + e, 16), 16);
+#pragma unroll
+                    for (int e = 0; e < VE; ++e) p = fmaf(ld(&w[e]), x[e], p);
+                }
+            } else {
+#pragma unroll 4
+                for (int c = sl; c < C; c += 16) p = fmaf(ld(row + c), v[c], p);
+            }
+            const float hm = relu(row_sum(p) + b);
+            if (sl == 0 && m0 + seg < rend) {
+                h[m] = hm;
+                if constexpr (SAVE) {
+                    if (a.save.hidden && bx == 0) a.save.hidden[n * mid + m] = hm;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (early < rows) stage(a.w2 + ((int64_t)cb * KK + early) * mid, (rows - early) * mid, a.w1_at, wave, kRowsWaves);
+
+    // ---- taps: rows of w2, the lane's values of the hidden vector in registers ----
+    // NI: values per lane, G: rows at a time (no value is read under a branch: it would be waited
+    // for alone)
+    auto taps_of = [&](auto ni, const T *first, int from, int to) __attribute__((always_inline)) {
+        constexpr int NI = decltype(ni)::value, G = NI >= 8 ? 1 : 8 / NI;
+        float hm[NI];
+        int at[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            at[i] = min(sl + i * 16, mid - 1);
+            hm[i] = h[at[i]];
+        }
+        for (int r0 = from + wave * 4; r0 < to; r0 += G * kRowsWaves * 4) {
+            float x[G][NI];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const T *row = first + (min(r0 + k * kRowsWaves * 4 + seg, to - 1) - from) * mid;
+#pragma unroll
+                for (int i = 0; i < NI; ++i) x[k][i] = ld(row + at[i]);
+            }
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                float p = 0.f;
+#pragma unroll
+                for (int i = 0; i < NI; ++i) p = fmaf(sl + i * 16 < mid ? x[k][i] : 0.f, hm[i], p);
+                if (NI == 8)
+                    for (int m = sl + NI * 16; m < mid; m += 16)
+                        p = fmaf(ld(first + (min(r0 + seg, to - 1) - from) * mid + m), h[m], p);
+                const float tot = row_sum(p);
+                const int r = r0 + k * kRowsWaves * 4 + seg;
+                if (sl == 0 && r < to) f[r] = tot;
+            }
+        }
+    };
+    auto taps = [&](const T *first, int from, int to) __attribute__((always_inline)) {
+        if (mid <= 16) taps_of(std::integral_constant<int, 1>{}, first, from, to);
+        else if (mid <= 32) taps_of(std::integral_constant<int, 2>{}, first, from, to);
+        else if (mid <= 64) taps_of(std::integral_constant<int, 4>{}, first, from, to);
+        else taps_of(std::integral_constant<int, 8>{}, first, from, to);
+    };
+    taps(w2s, 0, early);
+    if (early < rows) {
+        loads_to_lds_done();
+        __syncthreads();
+        taps(w1s, early, rows);
+    }
+    __syncthreads();
+    if (tid >= channels) return;
+    float u[KK];
+    TapParams<T, KK> params;
+#pragma unroll
+    for (int j = 0; j < KK; ++j) {
+        u[j] = f[tid * KK + j];
+        params.gain[j] = a.gain_vec ? ld(&gain[j]) : a.gain;
+        params.offset[j] = ld(&offset[j]);
+        params.bias[j] = ld(&bias[j]);
+    }
+    const int64_t to = (n * C + cb + tid) * KK;
+    if constexpr (SAVE) {
+        if (a.save.taps) {
+#pragma unroll
+            for (int j = 0; j < KK; ++j) a.save.taps[to + j] = u[j] + params.bias[j];
+        }
+    }
+    normalise<T, KK>(u, params);
+    T o[KK];
+#pragma unroll
+    for (int j = 0; j < KK; ++j) st(&o[j], u[j]);
+    __builtin_memcpy(a.cf + to, o, sizeof(o));
 }
 
 #endif  // __HIPCC__

@@ -9,7 +9,7 @@
 // five launches, each activation is written once:
 //   k_net_conv     1x1 convolution (+ BatchNorm, residual, ReLU)
 //   k_net_spatial  spatial filter branch, planes' partial sums for the pooling on the way
-//   (k_channel_branch / _mma, ddf_branches.hip)
+//   (the channel branch, ddf_branches.hip)
 //   k_net_filter   dynamic filter + BatchNorm + ReLU
 //   k_net_conv
 // and k_net_stem is the 7x7 convolution, BatchNorm, ReLU and max-pool in one.

@@ -260,3 +260,31 @@ def test_channel_branch_weights_through_lds(n, c, mid, tiles, k):
     got = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, None, None).view(n, c, -1)
     rest = [i for i in range(c) if i != c // 2]
     assert torch.equal(got[:, rest], out.view(n, c, -1)[:, rest])
+
+
+@pytest.mark.parametrize('dtype,tol', [(torch.float32, 2e-5), (torch.float16, 6e-3)])
+@pytest.mark.parametrize('n,c,mid,tiles', [
+    (1, 64, 12, 118), (4, 65, 13, 64), (2, 129, 25, 33), (1, 200, 31, 17),    # partial sums shared by 8, 4, 2 waves
+    (31, 16, 3, 9), (1, 1, 1, 40), (256, 16, 16, 2),                          # blocks of 16, up to 256 workgroups
+    (33, 100, 20, 3), (100, 70, 17, 2),                                       # blocks of 32 and 64, the last one short
+    (64, 256, 51, 4), (9, 300, 129, 3),                                       # rows of w2 that come in late
+    (3, 513, 30, 2), (1, 1030, 206, 5), (2, 20, 300, 1),                      # w1 in parts (fp32), long and short rows
+])
+def test_channel_branch_rows_through_lds(n, c, mid, tiles, dtype, tol):
+    """One sample per workgroup on the vector ALU: every split of the weights over LDS.  (fp16 with
+    whole steps of channels and values goes to the matrix cores.)"""
+    torch.manual_seed(c + mid)
+    k = 3
+    parts = torch.randn(n, tiles, c, device='cuda')
+    w1 = (torch.randn(mid, c, device='cuda') * c ** -0.5).to(dtype)
+    w2 = (torch.randn(c * k * k, mid, device='cuda') * mid ** -0.5).to(dtype)
+    b1, b2 = torch.randn(mid, device='cuda').to(dtype), torch.randn(c * k * k, device='cuda').to(dtype)
+    gv, ov = (torch.rand(c * k * k, device='cuda') + 0.5).to(dtype), torch.randn(c * k * k, device='cuda').to(dtype)
+    out = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, gv, ov)
+    ref = channel_reference(parts.double().sum(1).cpu(), *(t.cpu() for t in (w1, b1, w2, b2)), k, 0.7, gv.cpu(), ov.cpu())
+    err = ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item()
+    assert err < tol, err
+    w2[(c // 2) * k * k, mid - 1] = float('inf')     # (reaches its own channel only)
+    got = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, gv, ov).view(n, c, -1)
+    rest = [i for i in range(c) if i != c // 2]
+    assert torch.equal(got[:, rest], out.view(n, c, -1)[:, rest])
