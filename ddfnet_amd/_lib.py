@@ -50,9 +50,13 @@ SYMBOLS = {
     'ddf_hip_pack_backward': (_i, [_vp] * 10 + [ctypes.c_double] + [_vp] * 9 + [_sz] + [_i64] * 5 + [_i] * 4 +
                               [_vp]),
     'ddf_hip_net_conv': (_i, [_vp] * 5 + [_i64] * 5 + [_i] * 2 + [_vp]),
+    'ddf_hip_net_conv_pool_parts': (_i64, [_i64] * 5),
+    'ddf_hip_net_conv_pool': (_i, [_vp] * 5 + [_i64] * 5 + [_i, _vp]),
     'ddf_hip_net_conv_pair': (_i, [_vp] * 3 + [_i64] + [_vp] * 3 + [_i64] * 3 + [_i, _vp] + [_i64] * 2 + [_i, _vp]),
     'ddf_hip_net_stem': (_i, [_vp] * 4 + [_i64] * 3 + [_vp]),
     'ddf_hip_net_spatial': (_i, [_vp] * 5 + [ctypes.POINTER(ctypes.c_int)] + [_i64] * 4 + [_i, ctypes.c_double, _vp]),
+    'ddf_hip_net_branches': (_i, [_vp] * 4 + [ctypes.c_double, _vp, _i] + [_vp] * 5 + [_i64, ctypes.c_double] + [_vp] * 2 +
+                             [_i64] * 4 + [_i, _vp]),
     'ddf_hip_net_filter': (_i, [_vp] * 5 + [_i64] * 4 + [_i] * 2 + [_vp]),
     'ddf_hip_net_pool': (_i, [_vp] * 2 + [_i64] * 3 + [_vp]),
     'ddf_hip_up_forward': (_i, [_vp] * 4 + [_i64] * 4 + [_i] * 5 + [_vp]),

@@ -760,8 +760,28 @@ int ddf_hip_net_conv(const void *features, const void *weight, const ddf_net_nor
     if (!features || !weight || !output || !net_norm_ok(norm)) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
     const int64_t Ho = (H - 1) / stride + 1, Wo = (W - 1) / stride + 1;
     const ddf::NetConv a{features, weight, residual, output, net_norm(norm), N * Ho * Wo, (int)O, (int)C, relu,
-                         stride, (int)H, (int)W, (int)Wo, (int)(Ho * Wo)};
+                         stride, (int)H, (int)W, (int)Wo, (int)(Ho * Wo), nullptr, 0};
     return net_result(ddf::net_conv(a, (hipStream_t)stream), "ddf_hip_net_conv launch");
+}
+
+int64_t ddf_hip_net_conv_pool_parts(int64_t N, int64_t H, int64_t W, int64_t C, int64_t O) {
+    if (N < 1 || H < 1 || W < 1 || C < 1 || O < 1 || C > (1 << 24) || O > (1 << 24) || H * W >= (1ll << 31)) return 0;
+    const ddf::NetConv a{nullptr, nullptr, nullptr, nullptr, {}, N * H * W, (int)O, (int)C, 0, 1, (int)H, (int)W, (int)W,
+                         (int)(H * W), nullptr, 0};
+    return ddf::net_conv_pool_slots(a);
+}
+
+int ddf_hip_net_conv_pool(const void *features, const void *weight, const ddf_net_norm_t *norm, void *output,
+                          float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int relu,
+                          void *stream) {
+    if (N < 0 || H < 1 || W < 1 || C < 1 || O < 1 || C > (1 << 24) || O > (1 << 24) || H * W >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_conv_pool: bad sizes");
+    if (!features || !weight || !output || !pool_parts || !net_norm_ok(norm))
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    ddf::NetConv a{features, weight, nullptr, output, net_norm(norm), N * H * W, (int)O, (int)C, relu, 1, (int)H, (int)W,
+                   (int)W, (int)(H * W), pool_parts, 0};
+    a.pool_slots = ddf::net_conv_pool_slots(a);
+    return net_result(ddf::net_conv(a, (hipStream_t)stream), "ddf_hip_net_conv_pool launch");
 }
 
 int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_net_norm_t *norm, int64_t C,
@@ -775,9 +795,9 @@ int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_ne
         return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
     const int64_t Ho = (H - 1) / stride + 1, Wo = (W - 1) / stride + 1, M = N * Ho * Wo;
     const ddf::NetConv a{features, weight, nullptr, output, net_norm(norm), M, (int)O, (int)C, relu,
-                         1, (int)Ho, (int)Wo, (int)Wo, (int)(Ho * Wo)};
+                         1, (int)Ho, (int)Wo, (int)Wo, (int)(Ho * Wo), nullptr, 0};
     const ddf::NetConv side{side_features, side_weight, nullptr, output, net_norm(side_norm), M, (int)O, (int)side_C, 0,
-                            stride, (int)H, (int)W, (int)Wo, (int)(Ho * Wo)};
+                            stride, (int)H, (int)W, (int)Wo, (int)(Ho * Wo), nullptr, 0};
     return net_result(ddf::net_conv_pair(a, side, (hipStream_t)stream), "ddf_hip_net_conv_pair launch");
 }
 
@@ -799,6 +819,23 @@ int ddf_hip_net_spatial(const void *features, const void *weight, const void *bi
     return net_result(ddf::net_spatial(features, weight, bias, spatial_filter, pool_parts, n_parts, N, H, W, C, stride,
                                        gain, (hipStream_t)stream),
                       "ddf_hip_net_spatial launch");
+}
+
+int ddf_hip_net_branches(const void *features, const void *spatial_weight, const void *spatial_bias,
+                         void *spatial_filter, double spatial_gain, const float *pool_parts, int n_parts,
+                         const void *weight1, const void *bias1, const void *weight2, const void *bias2,
+                         void *channel_filter, int64_t mid, double channel_gain, const void *gain_vec,
+                         const void *offset_vec, int64_t N, int64_t H, int64_t W, int64_t C, int stride, void *stream) {
+    if (N < 1 || H < 1 || W < 1 || C < 1 || C > (1 << 24) || mid < 1 || mid > (1 << 24) || stride < 1 || n_parts < 1 ||
+        H / stride < 1 || W / stride < 1 || (int64_t)n_parts * C * 4 >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_branches: bad sizes");
+    if (!features || !spatial_weight || !spatial_filter || !pool_parts || !weight1 || !weight2 || !channel_filter)
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    const ddf::NetChannel channel{pool_parts, n_parts, weight1, bias1, weight2, bias2, gain_vec, offset_vec,
+                                  channel_filter, mid, channel_gain};
+    return net_result(ddf::net_branches(features, spatial_weight, spatial_bias, spatial_filter, spatial_gain, &channel, N,
+                                        H, W, C, stride, (hipStream_t)stream),
+                      "ddf_hip_net_branches launch");
 }
 
 int ddf_hip_net_filter(const void *features, const void *channel_filter, const void *spatial_filter,

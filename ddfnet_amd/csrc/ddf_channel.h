@@ -57,7 +57,7 @@ struct ChannelMmaLds {
     bool stage_w2, shared;      // shared: the taps reach into the rows of w2
 };
 inline int mma_round(int64_t v) { return (int)((v + 15) / 16 * 16); }
-inline ChannelMmaLds channel_mma_lds(int64_t C, int64_t mid, int kk) {
+inline ChannelMmaLds channel_mma_lds(int64_t C, int64_t mid, int kk, int64_t most = kMmaLds) {
     ChannelMmaLds l{};
     // (a wave's load is 1 KB: two rows of up to 256 channels, or one in pieces of 512)
     l.pitch = C <= 256 ? 512 : (int)((C + 511) / 512 * 1024);
@@ -65,7 +65,7 @@ inline ChannelMmaLds channel_mma_lds(int64_t C, int64_t mid, int kk) {
     const int64_t w2 = (int64_t)kMmaChannels * kk * mid * 2;
     const int64_t hidden = (mid + kMmaStep - 1) / kMmaStep * kMmaTile * 2, sums = C <= kMmaSpread ? kMmaThreads * 16 : 0;
     const int64_t taps = kMmaSamples * (kMmaChannels * kk + 1) * 4;
-    const int64_t left = kMmaLds - pooled - hidden - sums;
+    const int64_t left = most - pooled - hidden - sums;
     l.w1 = (int)pooled;
     int64_t space;
     if (rows * l.pitch + w2 <= left) {

@@ -155,14 +155,30 @@ struct NetConv {
     NetNorm norm;
     int64_t M;
     int N, K, relu, stride, H, W, Wo, npix;
+    // nullable: also the results' sums over the pixels of each sample, fp32, in parts:
+    // [(sample * pool_slots + slot) * N + channel]
+    float *pool;
+    int pool_slots;
 };
 bool net_conv_supported(const NetConv &a);
+int net_conv_pool_slots(const NetConv &a);    // as many as the launch leaves
 hipError_t net_conv(const NetConv &a, hipStream_t st);
 // act(affine(a) + affine'(first)): same pixels and channels, activation and output a's
 hipError_t net_conv_pair(const NetConv &a, const NetConv &first, hipStream_t st);
 hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,
                     hipStream_t st);
-int net_spatial_chunks(int64_t N, int64_t npix);
+// Both filter branches (channel null: the spatial one), the channel one from the pooled vectors'
+// partial sums.
+struct NetChannel {
+    const float *parts;
+    int n_parts;
+    const void *w1, *b1, *w2, *b2, *gain_vec, *offset_vec;
+    void *cf;
+    int64_t mid;
+    double gain;
+};
+hipError_t net_branches(const void *x, const void *w, const void *bias, void *sf, double gain, const NetChannel *channel,
+                        int64_t N, int64_t H, int64_t W, int64_t C, int stride, hipStream_t st);
 hipError_t net_spatial(const void *x, const void *w, const void *bias, void *sf, float *parts, int *n_parts, int64_t N,
                        int64_t H, int64_t W, int64_t C, int stride, double gain, hipStream_t st);
 hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNorm &norm, void *out, int64_t N,

@@ -6,11 +6,10 @@
 // what the matrix cores read; a lane of the dynamic filter owns eight channels of a pixel
 // and its neighbours are whole vectors, whatever the row length; and BatchNorm, ReLU and
 // the residual addition ride on the kernel that produces the values.  A bottleneck is
-// five launches, each activation is written once:
-//   k_net_conv     1x1 convolution (+ BatchNorm, residual, ReLU)
-//   k_net_spatial  spatial filter branch, planes' partial sums for the pooling on the way
-//   (the channel branch, ddf_branches.hip)
-//   k_net_filter   dynamic filter + BatchNorm + ReLU
+// four launches, each activation is written once:
+//   k_net_conv      1x1 convolution (+ BatchNorm, residual, ReLU), sums over its pixels on the way
+//   k_net_branches  spatial and channel filter branch
+//   k_net_filter    dynamic filter + BatchNorm + ReLU
 //   k_net_conv
 // and k_net_stem is the 7x7 convolution, BatchNorm, ReLU and max-pool in one.
 // At batch 128 the network took 8.85 ms as torch modules around the operator: 3.2 ms of
@@ -19,6 +18,7 @@
 // fp16 where the modules round it, and less often (not between convolution and BatchNorm's
 // ReLU).
 #include <algorithm>
+#include <numeric>
 #include <type_traits>
 
 #include "ddf_channel.h"
@@ -79,6 +79,78 @@ struct Affine {
     }
 };
 
+// Sum over the wave's four rows of sixteen lanes (the same value in every lane of a column).
+__device__ __forceinline__ float rows_total(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float add_permuted(float x) {
+    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+// Lanes of the lower half of the wave: a over both halves; of the upper half: b.
+__device__ __forceinline__ float add_swapped32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Lanes of even rows of sixteen: a over the row and the next; of odd rows: b over the row before, too.
+__device__ __forceinline__ float add_swapped16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// ---- spatial filter branch of sixteen pixels ------------------------------------------
+// Pixels are the columns, the nine taps nine of the sixteen rows of 16x16x32 steps over the
+// channels; both operands contiguous.  A pixel's taps end up on four lanes, which normalise them
+// across the wave's rows; they are stored as (pixel, 12), nine taps and padding.
+constexpr int kTapPitch = 12;
+
+template <int KS>
+struct TapWeights {
+    static constexpr int KK = 9;
+    half8_t w[KS];
+    float b[4];
+    __device__ __forceinline__ void request(const _Float16 *weight, const _Float16 *bias, int lane) {
+        const int col = lane & 15, quad = lane >> 4;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            w[ks] = *reinterpret_cast<const half8_t *>(weight + min(col, KK - 1) * KS * 32 + ks * 32 + quad * 8);
+            if (col >= KK) w[ks] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = (bias && quad * 4 + e < KK) ? (float)bias[quad * 4 + e] : 0.f;
+    }
+    // v: channels ks * 32 + quad * 8 .. + 7 of the lane's pixel; `at`: where its taps go
+    __device__ __forceinline__ void taps(const half8_t (&v)[KS], float gain, bool there, _Float16 *sf, int64_t at, int lane) const {
+        const int quad = lane >> 4;
+        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[ks], v[ks], acc, 0, 0, 0);
+        // taps 4 * quad + e of the pixel (rows past the ninth: zero weights, zero bias)
+        float f[4], s = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[e] = acc[e] + b[e];
+            s += f[e];
+        }
+        const float mean = rows_total(s) / (float)KK;
+        float sq = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[e] -= mean;
+            if (quad * 4 + e < KK) sq += f[e] * f[e];
+        }
+        const float inv = gain / (sqrtf(rows_total(sq) / (float)(KK - 1)) + 1e-10f);
+        half4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (_Float16)(f[e] * inv);
+        if (there && quad < 3) *reinterpret_cast<half4_t *>(sf + at * kTapPitch + quad * 4) = o;
+    }
+};
+
 // ---- 1x1 convolution ----------------------------------------------------------
 // out[m, o] = act(affine(sum_k x[row(m), k] w[o, k]) (+ res[m, o])), row(m) the sampled
 // pixel under a stride.  Tiles of BM pixels x BN channels; four waves, 2 x 2 over the tile,
@@ -105,7 +177,8 @@ struct Affine {
 // the fp16 values that a projection of its own would have stored.
 template <int BM, int BN, int KST, int ST>
 constexpr int conv_lds_halves() {
-    const int ring = (BM + BN) * KST * ST, tile = BM * (BN + 8);
+    // (behind the tile: the waves' sums over its pixels)
+    const int ring = (BM + BN) * KST * ST, tile = BM * (BN + 8) + kThreads / kWave * BN * 2;
     return ring > tile ? ring : tile;
 }
 
@@ -114,7 +187,7 @@ template <int N>
 __device__ __forceinline__ void arrive() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
-template <int BM, int BN, int KST, int ST, int WG, bool PAIR>
+template <int BM, int BN, int KST, int ST, int WG, bool PAIR, bool POOL>
 __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, int tiles_n, int tiles) {
     constexpr int CH = KST / 8, STAGE = (BM + BN) * KST;
     constexpr int RX = BM * CH / kThreads, RW = BN * CH / kThreads;
@@ -327,12 +400,13 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     float sc[8], sh[8];
     if constexpr (!PAIR) aff.finish(a.norm, sc, sh);
     _Float16 *out = static_cast<_Float16 *>(a.out);
-    if (!cok) return;
+    if (!POOL && !cok) return;
+    rows_u4 results[POOL ? RO : 1];
 #pragma unroll
     for (int i = 0; i < RO; ++i) {
         const int r = tid / CPR + i * (kThreads / CPR);
         const int64_t m = m0 + r;
-        if (m >= a.M) break;
+        if (!POOL && m >= a.M) break;
         half8_t o = *reinterpret_cast<const half8_t *>(net_smem + r * PITCH + cq * 8);
         if constexpr (!PAIR) {
 #pragma unroll
@@ -342,7 +416,60 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 o[e] = (_Float16)f;
             }
         }
-        *reinterpret_cast<half8_t *>(out + m * a.N + c) = o;
+        if (!POOL || (cok && m < a.M)) *reinterpret_cast<half8_t *>(out + m * a.N + c) = o;
+        if constexpr (POOL) results[i] = __builtin_bit_cast(rows_u4, o);
+    }
+    if constexpr (POOL) {
+        // Sums over the tile's pixels of each sample it touches, to the sample's slot for this
+        // tile; the tile with a sample's last pixel clears the slots that sample does not use.
+        float *red = reinterpret_cast<float *>(net_smem + BM * PITCH);    // [waves][BN]
+        const int first = (int)m0, end = (int)min(m0 + BM, a.M);
+        const int n_last = (end - 1) / a.npix;
+        float one = 1.f;
+        asm volatile("" : "+v"(one));    // (value * one + sum: a conversion less than value + sum)
+        for (int n = first / a.npix; n <= n_last; ++n) {
+            const int lo = n * a.npix - first, hi = lo + a.npix;
+            float sum[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+            auto add = [&](auto whole) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < RO; ++i) {
+                    const int r = tid / CPR + i * (kThreads / CPR);
+                    rows_u4 v = results[i];
+                    if (!decltype(whole)::value && (r < lo || r >= hi)) v = rows_u4{0, 0, 0, 0};
+                    const half8_t f = __builtin_bit_cast(half8_t, v);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) sum[e] = fmaf((float)f[e], one, sum[e]);
+                }
+            };
+            if (lo <= 0 && hi >= BM) add(std::true_type{});
+            else add(std::false_type{});
+            // over the lanes that share this one's channels: from eight sums to the two of
+            // channels 2 * row of lanes + 0..1
+            if constexpr (CPR == 8) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sum[e] = add_permuted<0x128 /* row_ror:8 */>(sum[e]);
+            }
+            float half[4], pair[2];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) half[e] = add_swapped32(sum[e], sum[e + 4]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) pair[e] = add_swapped16(half[e], half[e + 2]);
+            if (CPR == 16 || !(lane & 8)) {
+                typedef float float2_t __attribute__((ext_vector_type(2)));
+                *reinterpret_cast<float2_t *>(red + wave * BN + (lane % CPR) * 8 + (lane >> 4) * 2) = float2_t{pair[0], pair[1]};
+            }
+            __syncthreads();
+            if (tid < BN && n0 + tid < a.N) {
+                float *to = a.pool + (int64_t)n * a.pool_slots * a.N + n0 + tid;
+                int slot = tm - (int)((int64_t)n * a.npix / BM);
+                to[(int64_t)slot * a.N] = (red[tid] + red[BN + tid]) + (red[2 * BN + tid] + red[3 * BN + tid]);
+                if (hi <= end - first)
+                    while (++slot < a.pool_slots) to[(int64_t)slot * a.N] = 0.f;
+            }
+            if (n < n_last) __syncthreads();
+        }
     }
 }
 
@@ -354,6 +481,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
 // one compute unit's operands take on their way in, so smaller tiles are faster than larger ones
 // and than more waves (us for 32 x 32, the same with sixteen waves, 16 x 16: 49 x 2048 -> 512 9.7,
 // 9.7, 7.2; 196 x 1024 -> 256 6.7, 9.9, 5.7; 1 x 2048 -> 1000 7.1, 7.1, 5.2).
+template <bool POOL>
 __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tiles_n) {
     constexpr int WAVES = kThreads / kWave, D = 4, T = 16;
     __shared__ float red[WAVES][T][T + 1];
@@ -408,13 +536,35 @@ __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tile
     __syncthreads();
     float sc[1], sh[1];
     aff.finish(a.norm, sc, sh);
-    if (!ok) return;
+    if (!POOL && !ok) return;
     float f = 0.f;
 #pragma unroll
     for (int k = 0; k < WAVES; ++k) f += red[k][tid & (T - 1)][tid / T];
     f = fmaf(a.norm.var ? (float)(_Float16)f : f, sc[0], sh[0]) + (float)rv;    // (see k_net_conv)
     if (a.relu) f = relu(f);
-    static_cast<_Float16 *>(a.out)[om * a.N + oc] = (_Float16)f;
+    if (!POOL || ok) static_cast<_Float16 *>(a.out)[om * a.N + oc] = (_Float16)f;
+    if constexpr (POOL) {
+        // (see k_net_conv: a channel's sums by one thread)
+        __shared__ float results[T][T + 1];
+        results[tid / T][tid & (T - 1)] = (float)(_Float16)f;
+        __syncthreads();
+        if (tid >= T || n0 + tid >= a.N) return;
+        const int first = tm * T, end = (int)min((int64_t)first + T, a.M), n_last = (end - 1) / a.npix;
+        float v[T];
+#pragma unroll
+        for (int r = 0; r < T; ++r) v[r] = results[r][tid];
+        for (int n = first / a.npix; n <= n_last; ++n) {
+            const int lo = n * a.npix - first, hi = lo + a.npix;
+            float sum = 0.f;
+#pragma unroll
+            for (int r = 0; r < T; ++r) sum += r >= lo && r < hi ? v[r] : 0.f;
+            float *to = a.pool + (int64_t)n * a.pool_slots * a.N + n0 + tid;
+            int slot = tm - (int)((int64_t)n * a.npix / T);
+            to[(int64_t)slot * a.N] = sum;
+            if (hi <= end - first)
+                while (++slot < a.pool_slots) to[(int64_t)slot * a.N] = 0.f;
+        }
+    }
 }
 
 // ---- stem: 7x7 convolution of stride 2, BatchNorm, ReLU, 3x3 max-pool of stride 2 ----
@@ -558,149 +708,77 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
     }
 }
 
-// ---- spatial filter branch ------------------------------------------------------
-// Pixels are the columns, the nine taps nine of the sixteen rows of 16x16x32 steps over the
-// channels; both operands contiguous.  KQ waves share a tile of sixteen pixels, each with its
-// part of the channels (their taps meet in LDS), and walk along one sample; the same vectors feed
-// the plane sums (8 fp32 values per lane and 32 channels, brought together at the end).  With all of
-// 512 channels in one wave, the sums took 256 registers and more, one wave per SIMD, and the loads
-// four dependent rounds: four waves share them (7 x 7, 128 images 9.2 -> 7.6 us, one 8.3 -> 7.1; from
-// 14 x 14 under stride 2 16.5 -> 14.9 and 16.0 -> 13.8).  256 channels over two waves: 14.9 -> 16.6
-// under stride 2, 8.1 -> 8.0 without; not kept.
-// A pixel's taps end up on four lanes, which normalise them across the wave's rows; they are
-// stored as (pixel, 12), nine taps and padding.  Under stride 2 the three unsampled pixels of a
-// 2 x 2 block only go into the sums.
-constexpr int kTapPitch = 12;
+// ---- filter branches --------------------------------------------------------------
+// Both branches depend on the first convolution only - the spatial one on its results, the
+// channel one on their sums, which the convolution leaves - so one launch has them both: its first
+// workgroups are the channel branch (ddf_channel.h), a chain of round trips, the others the
+// spatial one.  A wave of the spatial branch takes
+// tiles of sixteen pixels, as many at a time as make eight loads, its weights in registers; under
+// stride 2 only the sampled pixels are read.  us for both branches, as two launches with the pooling
+// in the spatial one (which then read every pixel under stride 2, too) / now, batch 128: 56 x 56 x 64
+// 21.0 / 20.5, 28 x 28 x 128 16.8 / 14.0, from 56 x 56 under stride 2 31.5 / 12.9, 14 x 14 x 256
+// 17.0 / 7.6, from 14 x 14 x 512 under stride 2 28.5 / 13.6; one image, 56 x 56 x 64 10.5 / 5.3,
+// 14 x 14 x 256 13.4 / 5.8, 7 x 7 x 512 16.2 / 6.9.  (The spatial taps in the first convolution,
+// where its tile has all channels: 8 us more there, 8 less here, and a slower filter, whose
+// operands this launch leaves in the caches.)
+struct NetTaps {
+    const _Float16 *x, *w, *bias;
+    _Float16 *sf;
+    int W, Wo, npix, plane, pixels, tiles;    // npix, plane: results, pixels of a sample; pixels: results of all
+    float gain;
+};
 
-__device__ __forceinline__ float rows_total(float v) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
-}
-template <int CTRL>
-__device__ __forceinline__ float add_permuted(float x) {
-    return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lanes16_total(float v) {
-    v = add_permuted<0xB1>(v);
-    v = add_permuted<0x4E>(v);
-    v = add_permuted<0x141>(v);
-    return add_permuted<0x140>(v);
+template <int KS, int S, int U>
+__device__ __forceinline__ void net_taps(const NetTaps &a, int wave, int waves) {
+    constexpr int C = KS * 32;
+    const int lane = threadIdx.x & (kWave - 1), col = lane & 15, quad = lane >> 4;
+    TapWeights<KS> weights;
+    weights.request(a.w, a.bias, lane);
+    for (int t0 = wave * U; t0 < a.tiles; t0 += waves * U) {
+        half8_t v[U][KS];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int p = min((t0 + u) * 16 + col, a.pixels - 1);    // (past the last: not stored)
+            int64_t at = p;
+            if constexpr (S == 2) {
+                const int n = p / a.npix, q = p - n * a.npix, y = q / a.Wo, xx = q - y * a.Wo;
+                at = (int64_t)n * a.plane + 2 * y * a.W + 2 * xx;
+            }
+            const _Float16 *src = a.x + at * C + quad * 8;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) v[u][ks] = *reinterpret_cast<const half8_t *>(src + ks * 32);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int p = (t0 + u) * 16 + col;
+            weights.taps(v[u], a.gain, p < a.pixels, a.sf, p, lane);
+        }
+    }
 }
 
-template <int KS, int S, int KQ, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void k_net_spatial(const _Float16 *__restrict__ x,
-                                                          const _Float16 *__restrict__ w,
-                                                          const _Float16 *__restrict__ bias,
-                                                          _Float16 *__restrict__ sf, float *__restrict__ parts,
-                                                          int W, int Wo, int npix, int plane, int tiles_per_chunk,
-                                                          float gain) {
-    constexpr int C = KS * 32, KK = 9, NPX = S * S, KL = KS / KQ, SLOTS = WAVES / KQ;
-    static_assert(KL * KQ == KS && SLOTS * KQ == WAVES);
-    __shared__ float red[SLOTS][C];
-    __shared__ float4_t sums[2][KQ > 1 ? WAVES : 1][kWave];
-    const int lane = threadIdx.x & (kWave - 1);
+// Workgroups of the channel branch in front of those of the spatial one.
+enum { kNoChannels, kChannelsRows, kChannelsMma };
+template <int CH> struct ChannelArgs { };
+template <> struct ChannelArgs<kChannelsRows> { ChannelRows<__half> a; };
+template <> struct ChannelArgs<kChannelsMma> { ChannelMma a; };
+constexpr int branch_threads(int ch) { return ch == kChannelsRows ? kRowsThreads : kMmaThreads; }
+
+template <int KS, int S, int U, int CH>
+__global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps taps, ChannelArgs<CH> channels, int blocks_x,
+                                                                     int blocks) {
+    extern __shared__ __align__(16) unsigned char branch_smem[];
+    const int block = blockIdx.x;
+    if constexpr (CH != kNoChannels) {
+        if (block < blocks) {
+            const int by = block / blocks_x, bx = block - by * blocks_x;
+            if constexpr (CH == kChannelsRows) channel_rows<__half, false>(channels.a, bx, by, branch_smem);
+            else channel_mma<9, false>(channels.a, bx, by, branch_smem);
+            return;
+        }
+    }
+    constexpr int WAVES = branch_threads(CH) / kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int kq = wave % KQ, slot = wave / KQ;
-    const int col = lane & 15, quad = lane >> 4;
-    const int n = blockIdx.y;
-    const uint32_t bytes = (uint32_t)plane * C * 2;
-    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + (int64_t)n * plane * C, bytes);
-    half8_t wv[KL];
-#pragma unroll
-    for (int ks = 0; ks < KL; ++ks) {
-        wv[ks] = *reinterpret_cast<const half8_t *>(w + (int64_t)min(col, KK - 1) * C + (kq * KL + ks) * 32 + quad * 8);
-        if (col >= KK) wv[ks] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-    float b[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) b[e] = (bias && quad * 4 + e < KK) ? (float)bias[quad * 4 + e] : 0.f;
-    float pool[KL * 8];
-#pragma unroll
-    for (int i = 0; i < KL * 8; ++i) pool[i] = 0.f;
-
-    const int tiles = (npix + 15) / 16;
-    const int t_end = min((int)(blockIdx.x + 1) * tiles_per_chunk, tiles);
-    int buf = 0;
-    for (int t0 = blockIdx.x * tiles_per_chunk; t0 < t_end; t0 += SLOTS) {
-        const int t = t0 + slot, p = t * 16 + col;
-        if (KQ == 1 && t >= t_end) break;
-        const bool live = t < t_end && p < npix;   // (of the others: zeros)
-        uint32_t off[NPX];
-        if constexpr (S == 1) {
-            off[0] = live ? (uint32_t)p * C * 2 + kq * KL * 64 + quad * 16 : kOutside;
-        } else {
-            const int y = p / Wo, xx = p - y * Wo;
-#pragma unroll
-            for (int q = 0; q < NPX; ++q)
-                off[q] = live ? (uint32_t)((2 * y + q / 2) * W + 2 * xx + q % 2) * C * 2 + kq * KL * 64 + quad * 16 : kOutside;
-        }
-        float4_t acc = {0.f, 0.f, 0.f, 0.f};
-        constexpr int G = KL < 4 ? KL : S == 2 && WAVES == 16 ? 2 : 4;   // steps requested together
-#pragma unroll
-        for (int k0 = 0; k0 < KL; k0 += G) {
-            half8_t v[NPX][G];
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-#pragma unroll
-                for (int q = 0; q < NPX; ++q)
-                    v[q][g] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
-                        xr, (int)off[q], (k0 + g) * 64, 0));
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[k0 + g], v[0][g], acc, 0, 0, 0);
-#pragma unroll
-                for (int q = 0; q < NPX; ++q)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) pool[(k0 + g) * 8 + e] += (float)v[q][g][e];
-            }
-        }
-        if constexpr (KQ > 1) {
-            sums[buf][wave][lane] = acc;
-            __syncthreads();
-            if (kq == 0) {
-#pragma unroll
-                for (int q = 1; q < KQ; ++q) acc += sums[buf][wave + q][lane];
-            }
-            buf ^= 1;
-            if (kq != 0) continue;
-        }
-        // taps 4 * quad + e of pixel p
-        float v[4], s = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = acc[e] + b[e];
-            s += v[e];                             // (rows past the ninth: zero weights, zero bias)
-        }
-        const float mean = rows_total(s) / (float)KK;
-        float sq = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] -= mean;
-            if (quad * 4 + e < KK) sq += v[e] * v[e];
-        }
-        const float inv = gain / (sqrtf(rows_total(sq) / (float)(KK - 1)) + 1e-10f);
-        half4_t o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (_Float16)(v[e] * inv);
-        if (live && quad < 3) *reinterpret_cast<half4_t *>(sf + ((int64_t)n * npix + p) * kTapPitch + quad * 4) = o;
-    }
-#pragma unroll
-    for (int i = 0; i < KL * 8; ++i) pool[i] = lanes16_total(pool[i]);
-    if (col == 0) {
-#pragma unroll
-        for (int ks = 0; ks < KL; ++ks)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) red[slot][(kq * KL + ks) * 32 + quad * 8 + e] = pool[ks * 8 + e];
-    }
-    __syncthreads();
-    for (int c = threadIdx.x; c < C; c += WAVES * kWave) {
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < SLOTS; ++k) s += red[k][c];
-        parts[((int64_t)n * gridDim.x + blockIdx.x) * C + c] = s;
-    }
+    net_taps<KS, S, U>(taps, (block - blocks) * WAVES + wave, (gridDim.x - blocks) * WAVES);
 }
 
 // ---- dynamic filter + BatchNorm + ReLU ---------------------------------------------
@@ -864,8 +942,9 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 #undef DDF_I
 }
 
-// ---- mean over the pixels -----------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_net_pool(const _Float16 *__restrict__ x, _Float16 *__restrict__ out,
+// ---- mean (fp16) or sum (fp32) over the pixels ---------------------------------------------
+template <typename O>
+__global__ __launch_bounds__(kThreads) void k_net_pool(const _Float16 *__restrict__ x, O *__restrict__ out,
                                                        int plane, int C) {
     constexpr int LANES = 32, GROUPS = kThreads / LANES;
     __shared__ float red[GROUPS][LANES * 8];
@@ -891,7 +970,8 @@ __global__ __launch_bounds__(kThreads) void k_net_pool(const _Float16 *__restric
     float s = 0.f;
 #pragma unroll
     for (int k = 0; k < GROUPS; ++k) s += red[k][i];
-    out[(int64_t)n * C + cc] = (_Float16)(s / (float)plane);
+    if constexpr (sizeof(O) == 2) out[(int64_t)n * C + cc] = (O)(s / (float)plane);
+    else out[(int64_t)n * C + cc] = s;
 }
 
 template <int BM, int BN, int KST, int ST, int WG>
@@ -903,10 +983,13 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) < 64 * 1024;
     if (first && !kPair) return hipErrorNotSupported;
     if (first)
-        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
                            *first, tiles_n, (int)tiles);
+    else if (a.pool)
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, true>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+                           a, tiles_n, (int)tiles);
     else
-        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
                            a, tiles_n, (int)tiles);
     return hipGetLastError();
 }
@@ -924,28 +1007,52 @@ bool conv_in_tiles(const NetConv &a) {
 // 56 x 56 x 64 -> 256 76 / 65, 1568 of 28 x 28 x 512 -> 256 54 / 50, 784 of 14 x 14 x 1024 -> 512
 // 43 / 46, 392 of 14 x 14 x 1024 -> 256 25 / 30).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
 // 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
-hipError_t conv_tiles(const NetConv &a, const NetConv *first, hipStream_t st) {
+enum ConvTile { kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64, kTileSplit };
+ConvTile conv_tile(const NetConv &a, bool pair) {
     auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
     constexpr int kMany = 1024, kFew = 320;
-    if (a.N >= 128 && count(128, 128) >= (first ? kFew : kMany)) return launch_conv<128, 128, 32, 3, 3>(a, first, st);
-    if (a.N >= 128 && count(128, 128) >= kFew) return launch_conv<128, 128, 64, 2, 2>(a, nullptr, st);
-    if (count(128, 64) >= kMany) return launch_conv<128, 64, 32, 3, 4>(a, first, st);
-    if (count(128, 64) >= 448) return launch_conv<128, 64, 64, 2, 3>(a, first, st);
-    return launch_conv<64, 64, 64, 3, 3>(a, first, st);
+    if (!conv_in_tiles(a)) return kTileSplit;
+    if (a.N >= 128 && count(128, 128) >= (pair ? kFew : kMany)) return kTile128;
+    if (a.N >= 128 && count(128, 128) >= kFew) return kTile128Long;
+    if (count(128, 64) >= kMany) return kTile128x64;
+    if (count(128, 64) >= 448) return kTile128x64Long;
+    return kTile64;
+}
+int tile_rows(ConvTile t) { return t == kTileSplit ? 16 : t == kTile64 ? 64 : 128; }
+
+hipError_t conv_tiles(ConvTile tile, const NetConv &a, const NetConv *first, hipStream_t st) {
+    switch (tile) {
+        case kTile128: return launch_conv<128, 128, 32, 3, 3>(a, first, st);
+        case kTile128Long: return launch_conv<128, 128, 64, 2, 2>(a, first, st);
+        case kTile128x64: return launch_conv<128, 64, 32, 3, 4>(a, first, st);
+        case kTile128x64Long: return launch_conv<128, 64, 64, 2, 3>(a, first, st);
+        default: return launch_conv<64, 64, 64, 3, 3>(a, first, st);
+    }
 }
 
 }  // namespace
 
 bool net_conv_supported(const NetConv &a) { return a.K % 64 == 0 && a.K > 0 && a.N > 0; }
 
+// Slots of a sample in a convolution's sums over its pixels: one per tile of rows that a sample
+// can touch (samples start at multiples of the common divisor of their pixels and the tile).
+int net_conv_pool_slots(const NetConv &a) {
+    const int rows = tile_rows(conv_tile(a, false)), start = a.M > a.npix ? rows - std::gcd(rows, a.npix) : 0;
+    return (start + a.npix - 1) / rows + 1;
+}
+
 hipError_t net_conv(const NetConv &a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
-    if (!net_conv_supported(a)) return hipErrorNotSupported;
-    if (conv_in_tiles(a)) return conv_tiles(a, nullptr, st);
+    if (!net_conv_supported(a) || (a.pool && a.M > INT32_MAX - 256)) return hipErrorNotSupported;
+    const ConvTile tile = conv_tile(a, false);
+    if (tile != kTileSplit) return conv_tiles(tile, a, nullptr, st);
     const int tiles_n = (int)cdiv(a.N, 16);
     const int64_t blocks = cdiv(a.M, 16) * tiles_n;
     if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k_net_conv_split, dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
+    if (a.pool)
+        hipLaunchKernelGGL((k_net_conv_split<true>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
+    else
+        hipLaunchKernelGGL((k_net_conv_split<false>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
     return hipGetLastError();
 }
 
@@ -954,7 +1061,7 @@ hipError_t net_conv(const NetConv &a, hipStream_t st) {
 hipError_t net_conv_pair(const NetConv &a, const NetConv &first, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_conv_supported(a) || !net_conv_supported(first)) return hipErrorNotSupported;
-    if (conv_in_tiles(a) && conv_in_tiles(first)) return conv_tiles(a, &first, st);
+    if (conv_in_tiles(a) && conv_in_tiles(first)) return conv_tiles(conv_tile(a, true), a, &first, st);
     hipError_t err = net_conv(first, st);
     if (err != hipSuccess) return err;
     NetConv last = a;
@@ -975,40 +1082,90 @@ hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *o
     return hipGetLastError();
 }
 
-// Chunks of a sample's tiles: enough workgroups, at most kMaxChunks partial sums.
-constexpr int kMaxChunks = 8;
-int net_spatial_chunks(int64_t N, int64_t npix) {
-    const int64_t tiles = cdiv(npix, 16);
-    const int64_t want = std::min<int64_t>(std::max<int64_t>(1, cdiv(1024, N)), kMaxChunks);
-    return (int)std::min<int64_t>(want, cdiv(tiles, 4));   // (a tile per wave at least)
+// Waves of the spatial branch at most: the weights a wave loads first are paid for once per walk.
+constexpr int kMaxTapWaves = 8192;
+// Several tiles at a time from this many waves on (us, one / several: 8 x 56 x 56 x 64, 392 waves,
+// 5.7 / 7.5; 40 x 28 x 28 x 128, 980, 8.6 / 7.6).
+constexpr int kManyTapWaves = 512;
+
+// The spatial branch, and before it in the same launch the channel branch where `channel` is
+// given and its kernels cover it; else in a launch of its own.
+hipError_t net_branches(const void *x, const void *w, const void *bias, void *sf, double gain, const NetChannel *channel,
+                        int64_t N, int64_t H, int64_t W, int64_t C, int stride, hipStream_t st) {
+    if ((stride != 1 && stride != 2) || (stride == 2 && (H % 2 || W % 2)) || N * H * W >= (1ll << 31) - 256)
+        return hipErrorNotSupported;
+    const int64_t pixels = N * (H / stride) * (W / stride);
+    const NetTaps taps{(const _Float16 *)x, (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)sf, (int)W,
+                       (int)(W / stride), (int)((H / stride) * (W / stride)), (int)(H * W), (int)pixels,
+                       (int)cdiv(pixels, 16), (float)gain};
+    ChannelArgs<kChannelsMma> mma{};
+    ChannelArgs<kChannelsRows> rows{};
+    int kind = kNoChannels, blocks_x = 1, blocks = 0, lds = 0;
+    if (channel) {
+        const NetChannel &c = *channel;
+        auto half = [](const void *p) { return static_cast<const __half *>(p); };
+        const float scale = 1.f / (float)(H * W);
+        auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+        const bool vectors = aligned(c.w1) && aligned(c.w2) && aligned(c.parts) && N <= 65535;
+        rows.a = {nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2), (__half *)c.cf, (int)N, (int)C, (int)c.mid,
+                  (float)c.gain, half(c.gain_vec), half(c.offset_vec), c.parts, c.n_parts, scale, ChannelSave()};
+        if (C >= 256 && vectors && channel_mma_covers(C, c.mid, 9)) {
+            blocks_x = (int)(C / kMmaChannels);
+            blocks = blocks_x * (int)cdiv(N, kMmaSamples);
+            // (a channel block on every compute unit: half of the LDS, so that there is room for
+            // spatial ones beside it.  128 x 7 x 7 x 512 16.1 -> 13.4 us, w1 by 48 rows.)
+            const int64_t most = blocks > 128 ? kMmaLds / 2 : kMmaLds;
+            mma.a = {nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2), (__half *)c.cf, (int)N, (int)C, (int)c.mid,
+                     (float)c.gain, half(c.gain_vec), half(c.offset_vec), c.parts, c.n_parts, scale, ChannelSave(),
+                     channel_mma_lds(C, c.mid, 9, most)};
+            if (mma.a.lds.chunk == 0) mma.a.lds = channel_mma_lds(C, c.mid, 9);
+            kind = kChannelsMma;
+            lds = mma.a.lds.total;
+        } else if (C <= 128 && vectors && c.mid < kMmaStep && channel_rows_plan(rows.a)) {
+            kind = kChannelsRows;
+            blocks_x = (int)cdiv(C, rows.a.block);
+            blocks = blocks_x * (int)N;
+            lds = rows.a.total;
+        } else {
+            const hipError_t err = channel_branch<__half>(nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2),
+                                                          (__half *)c.cf, N, C, c.mid, 3, c.gain, half(c.gain_vec),
+                                                          half(c.offset_vec), st, c.parts, c.n_parts, scale);
+            if (err != hipSuccess) return err;
+        }
+    }
+    bool done = false;
+#define DDF_NET_BRANCHES(KS_, S_, U_, CH_, ARGS_)                                                                   \
+    if (!done && C == KS_ * 32 && stride == S_ && kind == CH_ && (U_ == 1 || cdiv(taps.tiles, U_) >= kManyTapWaves)) { \
+        constexpr int kWaves = branch_threads(CH_) / kWave;                                                         \
+        const int64_t most = kMaxTapWaves / kWaves;                                                                 \
+        const unsigned grid = (unsigned)(blocks + std::min(cdiv(cdiv(taps.tiles, U_), kWaves), most));              \
+        hipLaunchKernelGGL((k_net_branches<KS_, S_, U_, CH_>), dim3(grid), dim3(branch_threads(CH_)), lds, st, taps, \
+                           ARGS_, blocks_x, blocks);                                                                \
+        done = true;                                                                                                \
+    }
+#define DDF_NET_BRANCHES_S(KS_, U_, CH_, ARGS_) \
+    DDF_NET_BRANCHES(KS_, 1, U_, CH_, ARGS_) DDF_NET_BRANCHES(KS_, 2, U_, CH_, ARGS_)
+    const ChannelArgs<kNoChannels> none{};
+    DDF_NET_BRANCHES_S(2, 4, kChannelsRows, rows) DDF_NET_BRANCHES_S(2, 1, kChannelsRows, rows)
+    DDF_NET_BRANCHES_S(4, 2, kChannelsRows, rows) DDF_NET_BRANCHES_S(4, 1, kChannelsRows, rows)
+    DDF_NET_BRANCHES_S(8, 1, kChannelsMma, mma) DDF_NET_BRANCHES_S(16, 1, kChannelsMma, mma)
+    DDF_NET_BRANCHES_S(2, 1, kNoChannels, none) DDF_NET_BRANCHES_S(4, 1, kNoChannels, none)
+    DDF_NET_BRANCHES_S(8, 1, kNoChannels, none) DDF_NET_BRANCHES_S(16, 1, kNoChannels, none)
+#undef DDF_NET_BRANCHES_S
+#undef DDF_NET_BRANCHES
+    return done ? hipGetLastError() : hipErrorNotSupported;
 }
 
+// The spatial branch alone, and the planes' sums.
 hipError_t net_spatial(const void *x, const void *w, const void *bias, void *sf, float *parts, int *n_parts, int64_t N,
                        int64_t H, int64_t W, int64_t C, int stride, double gain, hipStream_t st) {
-    if (N > 65535 || H * W * C * 2 >= (1ll << 31) || (stride == 2 && (H % 2 || W % 2))) return hipErrorNotSupported;
-    const int64_t npix = (H / stride) * (W / stride);
-    const int tiles = (int)cdiv(npix, 16);
-    int chunks = net_spatial_chunks(N, npix);
-    const int per = (int)cdiv(tiles, chunks);
-    chunks = (int)cdiv(tiles, per);
-    *n_parts = chunks;
-    const dim3 grid((unsigned)chunks, (unsigned)N);
-    // Sixteen waves per workgroup where there are few workgroups of many tiles (3136 pixels x 64
-    // channels, one image: 7.1 us with four waves, 5.8 with sixteen; 128 and 256 channels, of
-    // which a wave has fewer tiles, 5.4 / 5.8 and 5.6 / 6.8).
-    const bool few = N * chunks <= 256;
-#define DDF_NET_SPATIAL(KS_, S_, KQ_, WAVES_)                                                                       \
-    if (C == KS_ * 32 && stride == S_) {                                                                            \
-        hipLaunchKernelGGL((k_net_spatial<KS_, S_, KQ_, WAVES_>), grid, dim3(WAVES_ * kWave), 0, st,                \
-                           (const _Float16 *)x, (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)sf, parts, \
-                           (int)W, (int)(W / stride), (int)npix, (int)(H * W), per, (float)gain);                   \
-        return hipGetLastError();                                                                                   \
-    }
-    if (few) DDF_NET_SPATIAL(2, 1, 1, 16)
-    DDF_NET_SPATIAL(2, 1, 1, 4) DDF_NET_SPATIAL(4, 1, 1, 4) DDF_NET_SPATIAL(8, 1, 1, 4) DDF_NET_SPATIAL(16, 1, 4, 16)
-    DDF_NET_SPATIAL(2, 2, 1, 4) DDF_NET_SPATIAL(4, 2, 1, 4) DDF_NET_SPATIAL(8, 2, 1, 4) DDF_NET_SPATIAL(16, 2, 4, 16)
-#undef DDF_NET_SPATIAL
-    return hipErrorNotSupported;
+    if (N > 65535) return hipErrorNotSupported;
+    const hipError_t err = net_branches(x, w, bias, sf, gain, nullptr, N, H, W, C, stride, st);
+    if (err != hipSuccess) return err;
+    *n_parts = 1;
+    hipLaunchKernelGGL((k_net_pool<float>), dim3((unsigned)cdiv(C, 256), (unsigned)N), dim3(kThreads), 0, st,
+                       (const _Float16 *)x, parts, (int)(H * W), (int)C);
+    return hipGetLastError();
 }
 
 hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNorm &norm, void *out, int64_t N,
@@ -1067,8 +1224,8 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
 hipError_t net_pool(const void *x, void *out, int64_t N, int64_t plane, int64_t C, hipStream_t st) {
     if (N * plane * C == 0) return hipSuccess;
     if (N > 65535 || C % 8 != 0) return hipErrorNotSupported;
-    hipLaunchKernelGGL(k_net_pool, dim3((unsigned)cdiv(C, 256), (unsigned)N), dim3(kThreads), 0, st, (const _Float16 *)x,
-                       (_Float16 *)out, (int)plane, (int)C);
+    hipLaunchKernelGGL((k_net_pool<_Float16>), dim3((unsigned)cdiv(C, 256), (unsigned)N), dim3(kThreads), 0, st,
+                       (const _Float16 *)x, (_Float16 *)out, (int)plane, (int)C);
     return hipGetLastError();
 }
 

@@ -138,7 +138,7 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
     // adds its result in place), between them the narrow activations and the filters.
     int64_t wide = 0, narrow = 0, taps = 0, filters = 0, parts = 0;
     {
-        int64_t h = h0 / 4, w = w0 / 4;
+        int64_t h = h0 / 4, w = w0 / 4, c = 64;
         wide = n * h * w * 64;
         for (const NetBlock &b : p.blocks) {
             const int64_t ho = h / b.stride, wo = w / b.stride;
@@ -146,7 +146,8 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             wide = std::max(wide, n * ho * wo * b.conv3.t[0]->size(0));
             taps = std::max(taps, n * ho * wo * 12);
             filters = std::max(filters, n * b.width * 9);
-            parts = std::max(parts, n * b.width * 8);
+            parts = std::max(parts, n * b.width * ddf_hip_net_conv_pool_parts(n, h, w, c, b.width));
+            c = b.conv3.t[0]->size(0);
             h = ho; w = wo;
         }
     }
@@ -166,14 +167,12 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
         for (const NetBlock &b : p.blocks) {
             const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0]->size(0);
             nm = b.conv1.norm();
-            covered(ddf_hip_net_conv(cur, b.conv1.t[0]->data_ptr(), &nm, nullptr, t1, n, h, w, c, width, 1, 1, st));
-            int n_parts = 0;
-            covered(ddf_hip_net_spatial(t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, pp, &n_parts, n, h, w, width,
-                                             b.stride, b.sgain, st));
-            covered(ddf_hip_channel_branch_parts(
-                pp, n_parts, 1.0 / (double)(h * w), b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(),
-                ptr_or_null(b.b2), cf, n, width, b.mid, 3, b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset),
-                DDF_F16, st));
+            covered(ddf_hip_net_conv_pool(cur, b.conv1.t[0]->data_ptr(), &nm, t1, pp, n, h, w, c, width, 1, st));
+            covered(ddf_hip_net_branches(
+                t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pp,
+                (int)ddf_hip_net_conv_pool_parts(n, h, w, c, width), b.w1->data_ptr(), ptr_or_null(b.b1),
+                b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid, b.cgain_const, ptr_or_null(b.cgain),
+                ptr_or_null(b.coffset), n, h, w, width, b.stride, st));
             nm = b.bn2.norm();
             covered(ddf_hip_net_filter(t1, cf, sf, &nm, t2, n, h, w, width, b.stride, b.combine, st));
             nm = b.conv3.norm();

@@ -364,6 +364,11 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *   spatial the spatial filter branch (3x3 taps, one head): spatial_filter (N, Ho*Wo, 12), nine
  *           taps and three of padding, and partial sums of the channels over the pixels as
  *           ddf_hip_spatial_branch_pool's; at most 8 parts; C 64, 128, 256 or 512
+ *   conv_pool  conv (stride 1, no residual) that also leaves the sums of its results over the
+ *           pixels of each sample in ddf_hip_net_conv_pool_parts parts (such partial sums)
+ *   branches  both filter branches in one launch: the spatial one, and the channel one of
+ *           ddf_hip_channel_branch_parts (3x3 taps) from the partial sums of conv_pool; sizes as
+ *           spatial's
  *   filter  relu(norm(the operator)) with the filters of `spatial` and ddf_hip_channel_branch_parts
  *   pool    mean over the pixels, (N, C)
  */
@@ -374,6 +379,10 @@ typedef struct {
 int ddf_hip_net_conv(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
                      void *output, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int stride, int relu,
                      void *stream);
+int64_t ddf_hip_net_conv_pool_parts(int64_t N, int64_t H, int64_t W, int64_t C, int64_t O);
+int ddf_hip_net_conv_pool(const void *features, const void *weight, const ddf_net_norm_t *norm, void *output,
+                          float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int relu,
+                          void *stream);
 int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_net_norm_t *norm, int64_t C,
                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
                           int64_t H, int64_t W, int64_t side_C, int stride, void *output, int64_t N, int64_t O,
@@ -383,6 +392,11 @@ int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t
 int ddf_hip_net_spatial(const void *features, const void *weight, const void *bias, void *spatial_filter,
                         float *pool_parts, int *n_parts, int64_t N, int64_t H, int64_t W, int64_t C, int stride,
                         double gain, void *stream);
+int ddf_hip_net_branches(const void *features, const void *spatial_weight, const void *spatial_bias,
+                         void *spatial_filter, double spatial_gain, const float *pool_parts, int n_parts,
+                         const void *weight1, const void *bias1, const void *weight2, const void *bias2,
+                         void *channel_filter, int64_t mid, double channel_gain, const void *gain_vec,
+                         const void *offset_vec, int64_t N, int64_t H, int64_t W, int64_t C, int stride, void *stream);
 int ddf_hip_net_filter(const void *features, const void *channel_filter, const void *spatial_filter,
                        const ddf_net_norm_t *norm, void *output, int64_t N, int64_t H, int64_t W, int64_t C,
                        int stride, int combine, void *stream);

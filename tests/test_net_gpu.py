@@ -184,3 +184,53 @@ def test_network_matches_its_modules(build, n, size, classes):
         model(x)
         handle.remove()
         assert calls == [1]
+
+
+@pytest.mark.parametrize('n,h,w,c,o', [
+    (1, 1, 1, 64, 64),                          # one pixel
+    (5, 7, 7, 64, 64), (3, 5, 7, 512, 512),     # samples that end inside tiles of 64 rows, of 16
+    (1, 14, 14, 1024, 256), (2, 14, 14, 1024, 256),
+    (9, 28, 28, 64, 128), (33, 28, 28, 256, 64), (16, 28, 28, 128, 264), (42, 56, 56, 64, 136),
+    (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64),
+])
+def test_conv_pool(n, h, w, c, o):
+    """The results of conv, and their sums over the pixels, slot by slot of the tiles."""
+    torch.manual_seed(c + o)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    wt = (torch.randn(o, c, device='cuda') * c ** -0.5).half()
+    norm, apply, keep = make_norm(o, 1, 1)
+    want, out = (torch.empty(n, h, w, o, device='cuda', dtype=torch.float16) for _ in range(2))
+    call('ddf_hip_net_conv', x, wt, norm, None, want, n, h, w, c, o, 1, 1)
+    count = _lib.lib().ddf_hip_net_conv_pool_parts(n, h, w, c, o)
+    parts = torch.full((n, count + 1, o), float('nan'), device='cuda')
+    call('ddf_hip_net_conv_pool', x, wt, norm, out, parts, n, h, w, c, o, 1)
+    assert torch.equal(out, want) and parts.view(-1)[n * count * o:].isnan().all()
+    total = parts.view(-1)[:n * count * o].view(n, count, o).double().sum(1)
+    # (fp32 sums of at most h * w terms of one sign)
+    assert (total - want.double().sum((1, 2))).abs().max() <= 1e-6 * want.double().abs().sum((1, 2)).max() + 1e-30
+
+
+@pytest.mark.parametrize('n,h,w,c,s,mid,n_parts', [
+    (1, 56, 56, 64, 1, 12, 49), (70, 6, 10, 64, 2, 12, 3), (300, 4, 4, 64, 1, 12, 1),     # samples past one per compute unit
+    (3, 9, 13, 128, 1, 25, 8), (2, 4, 6, 128, 2, 25, 9),
+    (1, 14, 14, 256, 1, 51, 13), (17, 3, 5, 256, 1, 51, 2), (3, 28, 28, 256, 2, 51, 7),
+    (5, 7, 7, 512, 1, 102, 2), (1, 14, 14, 512, 2, 102, 4),
+    (2, 5, 5, 64, 1, 40, 2), (2, 5, 5, 256, 1, 20, 3), (1, 1, 1, 512, 1, 512, 1),         # channel branch of its own
+])
+def test_both_branches(n, h, w, c, s, mid, n_parts):
+    from test_branches_gpu import channel_reference
+    torch.manual_seed(h * w + c)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    ws, bs = (torch.randn(9, c, device='cuda') * c ** -0.5).half(), torch.randn(9, device='cuda').half()
+    parts = torch.randn(n, n_parts, c, device='cuda')
+    w1, w2 = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((mid, c), (9 * c, mid)))
+    b1, b2, gv, ov = (torch.randn(k, device='cuda').half() for k in (mid, 9 * c, 9 * c, 9 * c))
+    ho, wo = h // s, w // s
+    sf = torch.empty(n, ho * wo, 12, device='cuda', dtype=torch.float16)
+    cf = torch.empty(n, c, 9, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_branches', x, ws, bs, sf, 0.6, parts, n_parts, w1, b1, w2, b2, cf, mid, 0.7, gv, ov, n, h, w, c, s)
+    raw = F.conv2d(x.float().permute(0, 3, 1, 2), ws.float().view(9, c, 1, 1), bs.float(), stride=s)
+    want = (raw - raw.mean(1, keepdim=True)) / (raw.std(1, keepdim=True) + 1e-10) * 0.6
+    close(sf[:, :, :9].permute(0, 2, 1).reshape(n, 9, ho, wo), want, 4e-3)
+    ref = channel_reference(parts.double().sum(1).cpu() / (h * w), *(t.cpu() for t in (w1, b1, w2, b2)), 3, 0.7, gv.cpu(), ov.cpu())
+    close(cf.cpu(), ref.view(n, c, 9), 6e-3)
