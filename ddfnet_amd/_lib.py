@@ -58,6 +58,8 @@ SYMBOLS = {
     'ddf_hip_net_branches': (_i, [_vp] * 4 + [ctypes.c_double, _vp, _i] + [_vp] * 5 + [_i64, ctypes.c_double] + [_vp] * 2 +
                              [_i64] * 4 + [_i, _vp]),
     'ddf_hip_net_filter': (_i, [_vp] * 5 + [_i64] * 4 + [_i] * 2 + [_vp]),
+    'ddf_hip_net_ddf': (_i, [_vp] * 4 + [ctypes.c_double, _vp, _i] + [_vp] * 5 + [_i64, ctypes.c_double] + [_vp] * 4 +
+                        [_i64] * 4 + [_i] * 2 + [_vp]),
     'ddf_hip_net_pool': (_i, [_vp] * 2 + [_i64] * 3 + [_vp]),
     'ddf_hip_up_forward': (_i, [_vp] * 4 + [_i64] * 4 + [_i] * 5 + [_vp]),
     'ddf_hip_up_backward_workspace_bytes': (_sz, [_i64] * 4 + [_i] * 5 + [_u]),

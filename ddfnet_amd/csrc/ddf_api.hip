@@ -850,6 +850,25 @@ int ddf_hip_net_filter(const void *features, const void *channel_filter, const v
                       "ddf_hip_net_filter launch");
 }
 
+int ddf_hip_net_ddf(const void *features, const void *spatial_weight, const void *spatial_bias, void *spatial_filter,
+                    double spatial_gain, const float *pool_parts, int n_parts, const void *weight1, const void *bias1,
+                    const void *weight2, const void *bias2, void *channel_filter, int64_t mid, double channel_gain,
+                    const void *gain_vec, const void *offset_vec, const ddf_net_norm_t *norm, void *output, int64_t N,
+                    int64_t H, int64_t W, int64_t C, int stride, int combine, void *stream) {
+    if (N < 1 || H < 1 || W < 1 || C < 1 || C > (1 << 24) || mid < 1 || mid > (1 << 24) || stride < 1 || n_parts < 1 ||
+        H / stride < 1 || W / stride < 1 || H > (1 << 24) || W > (1 << 24) || (int64_t)n_parts * C * 4 >= (1ll << 31) ||
+        (combine != DDF_MUL && combine != DDF_ADD))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_ddf: bad sizes");
+    if (!features || !spatial_weight || !spatial_filter || !pool_parts || !weight1 || !weight2 || !channel_filter ||
+        !output || !net_norm_ok(norm))
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    const ddf::NetChannel channel{pool_parts, n_parts, weight1, bias1, weight2, bias2, gain_vec, offset_vec,
+                                  channel_filter, mid, channel_gain};
+    return net_result(ddf::net_ddf(features, spatial_weight, spatial_bias, spatial_filter, spatial_gain, channel,
+                                   net_norm(norm), output, N, H, W, C, stride, combine == DDF_MUL, (hipStream_t)stream),
+                      "ddf_hip_net_ddf launch");
+}
+
 int ddf_hip_net_pool(const void *features, void *output, int64_t N, int64_t pixels, int64_t C, void *stream) {
     if (N < 0 || pixels < 1 || C < 1 || C > (1 << 24) || pixels >= (1ll << 31))
         return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_pool: bad sizes");

@@ -176,10 +176,28 @@ __device__ __forceinline__ void load_to_lds(uint32_t lds, const char *base, int 
 // This wave's are there.
 __device__ __forceinline__ void loads_to_lds_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Block (bx, by) of (C / 16, samples / 16), kMmaThreads threads.  SAVE: a.save is wanted
-// (compiled in, as a branch around every store has the loads before it wait one by one).
-template <int KK, bool SAVE>
-__device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by, unsigned char *smem) {
+// What a workgroup does beside the branch - while its first requests are on their way; once a
+// wave's hidden values are made - and where a channel's taps go.
+struct Nothing {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <typename T, int KK>
+struct ToFilter {    // (sample, channel, taps) to a tensor
+    T *cf;
+    int C;
+    __device__ __forceinline__ void operator()(int64_t n, int c, const float (&u)[KK]) const {
+        T o[KK];
+#pragma unroll
+        for (int j = 0; j < KK; ++j) st(&o[j], u[j]);
+        __builtin_memcpy(cf + (n * C + c) * KK, o, sizeof(o));
+    }
+};
+
+// Channels 16 * bx on of the ns (up to 16) samples from n0 on, kMmaThreads threads.  SAVE: a.save
+// is wanted (compiled in, as a branch around every store has the loads before it wait one by one).
+template <int KK, bool SAVE, typename Meanwhile, typename After, typename Sink>
+__device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0, int ns, unsigned char *smem,
+                                            const Meanwhile &meanwhile, const After &after, const Sink &sink) {
     constexpr int TPW = KK <= 9 ? 2 : 4, TAP_WAVES = (KK + TPW - 1) / TPW;      // taps per wave
     constexpr int NORM_WAVES = kMmaSamples * kMmaChannels / kWave;
     static_assert(TAP_WAVES <= kMmaWaves && NORM_WAVES <= kMmaWaves && KK % 8 == 1);
@@ -193,7 +211,6 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by,
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int col = lane & 15, quad = lane >> 4;
-    const int n0 = by * kMmaSamples, ns = min(kMmaSamples, a.N - n0);
     const int c0 = bx * kMmaChannels;
     const int ktiles = (mid + kMmaStep - 1) / kMmaStep;  // steps of the second product
     const int nk = C / kMmaStep;                         // steps of the first product
@@ -350,6 +367,7 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by,
             put_pooled(wave / share, lane, scaled(sum));
         }
     }
+    meanwhile();
     if (wave >= kPoolWaves) loads_to_lds_done();
     __syncthreads();
 
@@ -400,6 +418,7 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by,
             }
         }
     }
+    after();
     __syncthreads();
     if (!together && a.lds.stage_w2) {
         stage_w2(wave, kMmaWaves);
@@ -515,15 +534,7 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int by,
         }
     }
     normalise<__half, KK>(u, params);
-    __half *op = a.cf + to;
-#pragma unroll
-    for (int k = 0; k < KK / 8; ++k) {
-        half8_t o;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (_Float16)u[k * 8 + e];
-        __builtin_memcpy(op + k * 8, &o, sizeof(o));
-    }
-    st(op + KK - 1, u[KK - 1]);
+    sink(n0 + zs, c0 + zc, u);
 }
 
 #endif  // __HIPCC__
@@ -603,9 +614,10 @@ __device__ __forceinline__ float row_sum(float v) {
 }
 
 
-// Block (bx, by) of (channel blocks, samples), kRowsThreads threads.
-template <typename T, bool SAVE>
-__device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, int by, unsigned char *smem) {
+// Block bx of sample n's channels, kRowsThreads threads.
+template <typename T, bool SAVE, typename Meanwhile, typename After, typename Sink>
+__device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, int64_t n, unsigned char *smem,
+                                             const Meanwhile &meanwhile, const After &after, const Sink &sink) {
     constexpr int KK = kRowsKK, VE = 16 / sizeof(T);
     const int C = a.C, mid = a.mid;
     float *v = reinterpret_cast<float *>(smem);     // [C]
@@ -615,7 +627,6 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
     const T *w1s = reinterpret_cast<const T *>(smem + a.w1_at), *w2s = reinterpret_cast<const T *>(smem + a.w2_at);
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int64_t n = by;
     const int cb = bx * a.block, channels = min(a.block, C - cb), rows = channels * KK;
     const int early = min(a.early, rows);           // rows of w2 that come in with w1
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
@@ -700,6 +711,7 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
             }
         }
     }
+    meanwhile();
     if (wave >= pool_waves) loads_to_lds_done();
     __syncthreads();
 
@@ -743,6 +755,7 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
             }
         }
     }
+    after();
     __syncthreads();
     if (early < rows) stage(a.w2 + ((int64_t)cb * KK + early) * mid, (rows - early) * mid, a.w1_at, wave, kRowsWaves);
 
@@ -811,10 +824,7 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
         }
     }
     normalise<T, KK>(u, params);
-    T o[KK];
-#pragma unroll
-    for (int j = 0; j < KK; ++j) st(&o[j], u[j]);
-    __builtin_memcpy(a.cf + to, o, sizeof(o));
+    sink(n, cb + tid, u);
 }
 
 #endif  // __HIPCC__

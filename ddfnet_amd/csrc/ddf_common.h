@@ -183,6 +183,9 @@ hipError_t net_spatial(const void *x, const void *w, const void *bias, void *sf,
                        int64_t H, int64_t W, int64_t C, int stride, double gain, hipStream_t st);
 hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNorm &norm, void *out, int64_t N,
                       int64_t H, int64_t W, int64_t C, int stride, bool mul, hipStream_t st);
+hipError_t net_ddf(const void *x, const void *w, const void *bias, void *sf, double gain, const NetChannel &channel,
+                   const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W, int64_t C, int stride, bool mul,
+                   hipStream_t st);
 hipError_t net_pool(const void *x, void *out, int64_t N, int64_t plane, int64_t C, hipStream_t st);
 
 // All scale*scale sub-pixel branches of an up-sampling DDF in one launch,

@@ -112,16 +112,16 @@ template <int KS>
 struct TapWeights {
     static constexpr int KK = 9;
     half8_t w[KS];
-    float b[4];
+    uint16_t b[4];
+    // (rows past the ninth, and a bias that is not there, lie outside their buffers: zeros)
     __device__ __forceinline__ void request(const _Float16 *weight, const _Float16 *bias, int lane) {
         const int col = lane & 15, quad = lane >> 4;
+        const __amdgpu_buffer_rsrc_t wr = plane_rsrc(weight, KK * KS * 64), br = plane_rsrc(bias, bias ? KK * 2 : 0);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            w[ks] = *reinterpret_cast<const half8_t *>(weight + min(col, KK - 1) * KS * 32 + ks * 32 + quad * 8);
-            if (col >= KK) w[ks] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        }
+        for (int ks = 0; ks < KS; ++ks)
+            w[ks] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(wr, col * KS * 64 + quad * 16, ks * 64, 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) b[e] = (bias && quad * 4 + e < KK) ? (float)bias[quad * 4 + e] : 0.f;
+        for (int e = 0; e < 4; ++e) b[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, (quad * 4 + e) * 2, 0, 0);
     }
     // v: channels ks * 32 + quad * 8 .. + 7 of the lane's pixel; `at`: where its taps go
     __device__ __forceinline__ void taps(const half8_t (&v)[KS], float gain, bool there, _Float16 *sf, int64_t at, int lane) const {
@@ -133,7 +133,7 @@ struct TapWeights {
         float f[4], s = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            f[e] = acc[e] + b[e];
+            f[e] = acc[e] + (float)__builtin_bit_cast(_Float16, b[e]);
             s += f[e];
         }
         const float mean = rows_total(s) / (float)KK;
@@ -771,8 +771,13 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps tap
     if constexpr (CH != kNoChannels) {
         if (block < blocks) {
             const int by = block / blocks_x, bx = block - by * blocks_x;
-            if constexpr (CH == kChannelsRows) channel_rows<__half, false>(channels.a, bx, by, branch_smem);
-            else channel_mma<9, false>(channels.a, bx, by, branch_smem);
+            const ToFilter<__half, 9> sink{channels.a.cf, channels.a.C};
+            if constexpr (CH == kChannelsRows) {
+                channel_rows<__half, false>(channels.a, bx, by, branch_smem, Nothing(), Nothing(), sink);
+            } else {
+                const int n0 = by * kMmaSamples;
+                channel_mma<9, false>(channels.a, bx, n0, min(kMmaSamples, channels.a.N - n0), branch_smem, Nothing(), Nothing(), sink);
+            }
             return;
         }
     }
@@ -790,6 +795,19 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps tap
 // instructions per pixel and channel quarter.  WIDE: comb in fp32, 18 instructions - for rows
 // of an odd length, where the operator's own kernels have it so.  A row outside the image, a
 // column past its ends and a walk past the last pixel read zeros through the buffer descriptor.
+template <bool MUL, bool WIDE>
+__device__ __forceinline__ void filter_pair(half2_t cv, half2_t sv, half2_t xv, float &a0, float &a1) {
+    if constexpr (WIDE) {
+        const float c0 = (float)cv[0], c1 = (float)cv[1], s0 = (float)sv[0], s1 = (float)sv[1];
+        a0 = fmaf((float)xv[0], MUL ? c0 * s0 : c0 + s0, a0);
+        a1 = fmaf((float)xv[1], MUL ? c1 * s1 : c1 + s1, a1);
+    } else {
+        const half2_t cb = MUL ? cv * sv : cv + sv;
+        a0 = fmaf((float)xv[0], (float)cb[0], a0);
+        a1 = fmaf((float)xv[1], (float)cb[1], a1);
+    }
+}
+
 template <int LP, int S, bool MUL, bool WIDE>
 __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restrict__ x,
                                                          const _Float16 *__restrict__ cf,
@@ -876,19 +894,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                 const half2_t sv = {sp[t & 1], sp[t & 1]};
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const half2_t cv = __builtin_bit_cast(half2_t, cfp[t][k]);
-                    const half2_t xv = __builtin_bit_cast(half2_t, col[(A + j) % RING][i][k]);
-                    if constexpr (WIDE) {
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const float c1 = (float)cv[h], s1 = (float)sv[h];
-                            acc[2 * k + h] = fmaf((float)xv[h], MUL ? c1 * s1 : c1 + s1, acc[2 * k + h]);
-                        }
-                    } else {
-                        const half2_t cb = MUL ? cv * sv : cv + sv;
-                        acc[2 * k] = fmaf((float)xv[0], (float)cb[0], acc[2 * k]);
-                        acc[2 * k + 1] = fmaf((float)xv[1], (float)cb[1], acc[2 * k + 1]);
-                    }
+                    filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, cfp[t][k]), sv,
+                                           __builtin_bit_cast(half2_t, col[(A + j) % RING][i][k]), acc[2 * k], acc[2 * k + 1]);
                 }
             }
         half8_t o;
@@ -940,6 +947,129 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
         }
     }
 #undef DDF_I
+}
+
+// ---- branches and dynamic filter in one launch, few pixels ---------------------------------
+// Where the two launches are latency, a workgroup computes sixteen channels' taps, the spatial
+// taps of `rows` result rows and those rows' results of its channels: every workgroup of a sample
+// recomputes the hidden vector, every one of a row its spatial taps, and neither goes through
+// memory.  The rows it reads (and zeros around them) come into LDS as [pixel][16 channels] while
+// the channel branch waits for its weights, the spatial taps are computed meanwhile; then a
+// thread takes eight channels of a pixel.  Arithmetic and rounding are k_net_filter's.  us, two
+// launches / this: one image 56 x 56 x 64 10.3 / 7.7, 28 x 28 x 128 10.4 / 6.9, 14 x 14 x 256 10.6 /
+// 6.9, 7 x 7 x 512 11.9 / 9.6; most of it is the channel branch's chain and the instructions in front
+// of the first barrier (divisions by runtime values there cost 1 us).
+struct NetFew {
+    const _Float16 *x, *tap_w, *tap_bias;
+    _Float16 *out;
+    NetNorm norm;
+    int H, W, Ho, Wo, rows;
+    int per_row;                               // 64 vectors of a row of W + 2 pixels
+    uint32_t per_row_magic;                    // 2^16 / per_row, rounded up
+    uint32_t wo_magic;                         // 2^20 / Wo, rounded up
+    float tap_gain;
+    int sf, tile, channels;                    // where in LDS (bytes): spatial taps, rows, the channel branch's
+};
+constexpr int kFewItems = 3;
+constexpr int kFewCf = 9 * kMmaChannels * 2;   // the channels' taps [tap][channel], at LDS 0
+
+template <int KS, int S, bool MUL, bool WIDE, int CH>
+__global__ __launch_bounds__(branch_threads(CH)) void k_net_filter_few(NetFew a, ChannelArgs<CH> channels) {
+    constexpr int C = KS * 32, KK = 9, GROUPS = C / kMmaChannels, THREADS = branch_threads(CH), WAVES = THREADS / kWave;
+    constexpr int ITEMS = kFewItems;           // 16-byte vectors of the rows per thread at most
+    extern __shared__ __align__(16) unsigned char few_smem[];
+    _Float16 *cfs = reinterpret_cast<_Float16 *>(few_smem), *sfs = reinterpret_cast<_Float16 *>(few_smem + a.sf);
+    rows_u4 *tile = reinterpret_cast<rows_u4 *>(few_smem + a.tile);
+    const int g = blockIdx.x % GROUPS, chunk = blockIdx.x / GROUPS, n = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int y0 = chunk * a.rows, rows = min(a.rows, a.Ho - y0), pixels = rows * a.Wo;
+    const uint32_t sample_bytes = (uint32_t)(a.H * a.W) * C * 2;
+    const _Float16 *xn = a.x + (int64_t)n * a.H * a.W * C;
+
+    // Rows S * y0 - 1 .. S * (y0 + rows - 1) + 1, columns -1 .. W, both halves of a pixel: a wave
+    // takes 64 vectors of a row at a time (no division per lane: with sixteen waves that alone was
+    // 1 us).
+    const int pitch = a.W + 2, waves_of = (S * (rows - 1) + 3) * a.per_row;
+    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(xn, sample_bytes);
+    rows_u4 part[ITEMS];
+    int to[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const int i = wave + k * WAVES, yy = (int)((uint32_t)i * a.per_row_magic >> 16), at = (i - yy * a.per_row) * kWave + lane;
+        const int y = S * y0 - 1 + yy, x = (at >> 1) - 1;
+        to[k] = i < waves_of && at < 2 * pitch ? yy * 2 * pitch + at : -1;
+        const bool in = to[k] >= 0 && y >= 0 && y < a.H && x >= 0 && x < a.W;
+        part[k] = __builtin_bit_cast(rows_u4, __builtin_amdgcn_raw_buffer_load_b128(
+            xr, in ? ((y * a.W + x) * C + g * kMmaChannels + (at & 1) * 8) * 2 : (int)kOutside, 0, 0));
+    }
+    // (row of a result pixel of the workgroup: below 512, as Wo is)
+    auto row_of = [&](int q) __attribute__((always_inline)) { return (int)(((uint32_t)q * a.wo_magic) >> 20); };
+    const int o = tid & 1, p = tid >> 1;
+    const int c = g * kMmaChannels + o * 8;
+    Affine<8> aff;
+    aff.request(a.norm, c);
+    // Spatial taps by the last waves first, which have nothing to do when the hidden values are
+    // made: the pixels of a wave's first tile are requested early, its taps are worked out then.
+    TapWeights<KS> weights;
+    half8_t v[KS];
+    auto pixels_of = [&](int t) __attribute__((always_inline)) {
+        const int q = min(t * 16 + (lane & 15), pixels - 1), y = row_of(q), x = q - y * a.Wo;
+        const _Float16 *src = xn + (int64_t)(S * (y0 + y) * a.W + S * x) * C + (lane >> 4) * 8;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) v[ks] = *reinterpret_cast<const half8_t *>(src + ks * 32);
+    };
+    const int t_first = WAVES - 1 - wave;
+    constexpr bool kEarly = KS <= 8;           // (512 channels: no registers for that)
+    auto meanwhile = [&]() __attribute__((always_inline)) {
+        if (kEarly && t_first * 16 < pixels) {
+            pixels_of(t_first);
+            weights.request(a.tap_w, a.tap_bias, lane);
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k)
+            if (to[k] >= 0) tile[to[k]] = part[k];
+    };
+    float sc[8], sh[8];
+    auto after = [&]() __attribute__((always_inline)) {
+        aff.finish(a.norm, sc, sh);
+        for (int t = t_first; t * 16 < pixels; t += WAVES) {
+            if (!kEarly || t != t_first) pixels_of(t);
+            if (!kEarly) weights.request(a.tap_w, a.tap_bias, lane);
+            weights.taps(v, a.tap_gain, t * 16 + (lane & 15) < pixels, sfs, t * 16 + (lane & 15), lane);
+        }
+    };
+    auto sink = [&](int64_t, int c, const float (&u)[KK]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < KK; ++t) cfs[t * kMmaChannels + (c & (kMmaChannels - 1))] = (_Float16)u[t];
+    };
+    if constexpr (CH == kChannelsRows) channel_rows<__half, false>(channels.a, g, n, few_smem + a.channels, meanwhile, after, sink);
+    else channel_mma<KK, false>(channels.a, g, n, 1, few_smem + a.channels, meanwhile, after, sink);
+    __syncthreads();
+    if (p >= pixels) return;
+    const int y = row_of(p), x = p - y * a.Wo;
+    uint32_t tap[6];
+    __builtin_memcpy(tap, __builtin_assume_aligned(sfs + p * kTapPitch, 8), sizeof(tap));
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int t = i * 3 + j;
+            const half2_t sp = __builtin_bit_cast(half2_t, tap[t / 2]);
+            const half2_t sv = {sp[t & 1], sp[t & 1]};
+            const rows_u4 xw = tile[((S * y + i) * pitch + S * x + j) * 2 + o];
+            const rows_u4 cw = *reinterpret_cast<const rows_u4 *>(cfs + t * kMmaChannels + o * 8);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, (uint32_t)cw[k]), sv,
+                                       __builtin_bit_cast(half2_t, (uint32_t)xw[k]), acc[2 * k], acc[2 * k + 1]);
+        }
+    half8_t r;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = (_Float16)relu(fmaf((float)(_Float16)acc[e], sc[e], sh[e]));
+    *reinterpret_cast<half8_t *>(a.out + (((int64_t)n * a.Ho + y0 + y) * a.Wo + x) * C + c) = r;
 }
 
 // ---- mean (fp16) or sum (fp32) over the pixels ---------------------------------------------
@@ -1082,11 +1212,31 @@ hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *o
     return hipGetLastError();
 }
 
+// One workgroup per compute unit, of up to this many pixels: a pixel is a thread's pair, and with
+// more of them the launch takes longer than the two it replaces (ResNet-50, us, at most 256 or 512 /
+// at most 128 / two launches: 1 image 342 / 340 / 385, 8 471 / 458 / 468, 16 596 / 573 / 570).
+constexpr int kFewBlocks = 256, kFewPixels = 128;
+
 // Waves of the spatial branch at most: the weights a wave loads first are paid for once per walk.
 constexpr int kMaxTapWaves = 8192;
 // Several tiles at a time from this many waves on (us, one / several: 8 x 56 x 56 x 64, 392 waves,
 // 5.7 / 7.5; 40 x 28 x 28 x 128, 980, 8.6 / 7.6).
 constexpr int kManyTapWaves = 512;
+
+// Which of the channel branch's device functions has these sizes (both would: the same one as in
+// a launch of its own); its arguments but for the split over LDS.
+int channel_kind(const NetChannel &c, int64_t N, int64_t H, int64_t W, int64_t C, ChannelMma *mma, ChannelRows<__half> *rows) {
+    auto half = [](const void *p) { return static_cast<const __half *>(p); };
+    auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const float scale = 1.f / (float)(H * W);
+    *rows = {nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2), (__half *)c.cf, (int)N, (int)C, (int)c.mid,
+             (float)c.gain, half(c.gain_vec), half(c.offset_vec), c.parts, c.n_parts, scale, ChannelSave()};
+    *mma = {nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2), (__half *)c.cf, (int)N, (int)C, (int)c.mid,
+            (float)c.gain, half(c.gain_vec), half(c.offset_vec), c.parts, c.n_parts, scale, ChannelSave()};
+    if (!aligned(c.w1) || !aligned(c.w2) || !aligned(c.parts) || N > 65535) return kNoChannels;
+    if (C >= 256 && channel_mma_covers(C, c.mid, 9)) return kChannelsMma;
+    return C <= 128 && c.mid < kMmaStep ? kChannelsRows : kNoChannels;
+}
 
 // The spatial branch, and before it in the same launch the channel branch where `channel` is
 // given and its kernels cover it; else in a launch of its own.
@@ -1102,34 +1252,24 @@ hipError_t net_branches(const void *x, const void *w, const void *bias, void *sf
     ChannelArgs<kChannelsRows> rows{};
     int kind = kNoChannels, blocks_x = 1, blocks = 0, lds = 0;
     if (channel) {
-        const NetChannel &c = *channel;
-        auto half = [](const void *p) { return static_cast<const __half *>(p); };
-        const float scale = 1.f / (float)(H * W);
-        auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-        const bool vectors = aligned(c.w1) && aligned(c.w2) && aligned(c.parts) && N <= 65535;
-        rows.a = {nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2), (__half *)c.cf, (int)N, (int)C, (int)c.mid,
-                  (float)c.gain, half(c.gain_vec), half(c.offset_vec), c.parts, c.n_parts, scale, ChannelSave()};
-        if (C >= 256 && vectors && channel_mma_covers(C, c.mid, 9)) {
+        kind = channel_kind(*channel, N, H, W, C, &mma.a, &rows.a);
+        if (kind == kChannelsMma) {
             blocks_x = (int)(C / kMmaChannels);
             blocks = blocks_x * (int)cdiv(N, kMmaSamples);
             // (a channel block on every compute unit: half of the LDS, so that there is room for
             // spatial ones beside it.  128 x 7 x 7 x 512 16.1 -> 13.4 us, w1 by 48 rows.)
-            const int64_t most = blocks > 128 ? kMmaLds / 2 : kMmaLds;
-            mma.a = {nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2), (__half *)c.cf, (int)N, (int)C, (int)c.mid,
-                     (float)c.gain, half(c.gain_vec), half(c.offset_vec), c.parts, c.n_parts, scale, ChannelSave(),
-                     channel_mma_lds(C, c.mid, 9, most)};
-            if (mma.a.lds.chunk == 0) mma.a.lds = channel_mma_lds(C, c.mid, 9);
-            kind = kChannelsMma;
+            mma.a.lds = channel_mma_lds(C, channel->mid, 9, blocks > 128 ? kMmaLds / 2 : kMmaLds);
+            if (mma.a.lds.chunk == 0) mma.a.lds = channel_mma_lds(C, channel->mid, 9);
             lds = mma.a.lds.total;
-        } else if (C <= 128 && vectors && c.mid < kMmaStep && channel_rows_plan(rows.a)) {
-            kind = kChannelsRows;
+        } else if (kind == kChannelsRows && channel_rows_plan(rows.a)) {
             blocks_x = (int)cdiv(C, rows.a.block);
             blocks = blocks_x * (int)N;
             lds = rows.a.total;
         } else {
-            const hipError_t err = channel_branch<__half>(nullptr, half(c.w1), half(c.b1), half(c.w2), half(c.b2),
-                                                          (__half *)c.cf, N, C, c.mid, 3, c.gain, half(c.gain_vec),
-                                                          half(c.offset_vec), st, c.parts, c.n_parts, scale);
+            kind = kNoChannels;
+            const ChannelRows<__half> &c = rows.a;
+            const hipError_t err = channel_branch<__half>(nullptr, c.w1, c.b1, c.w2, c.b2, c.cf, N, C, c.mid, 3, c.gain,
+                                                          c.gain_vec, c.offset_vec, st, c.parts, c.nparts, c.scale);
             if (err != hipSuccess) return err;
         }
     }
@@ -1219,6 +1359,67 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
         if (!done) return hipErrorNotSupported;
     }
     return hipGetLastError();
+}
+
+// Both branches and the filter behind them: one launch where a compute unit has one workgroup of
+// sixteen channels of some rows at most; else two.
+hipError_t net_ddf(const void *x, const void *w, const void *bias, void *sf, double gain, const NetChannel &channel,
+                   const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W, int64_t C, int stride, bool mul,
+                   hipStream_t st) {
+    const int64_t Ho = H / stride, Wo = W / stride;
+    ChannelArgs<kChannelsMma> mma{};
+    ChannelArgs<kChannelsRows> rows{};
+    const int kind = channel_kind(channel, N, H, W, C, &mma.a, &rows.a);
+    const int threads = branch_threads(kind);
+    const int64_t groups = C / kMmaChannels, most = kFewBlocks / std::max<int64_t>(groups * N, 1);    // chunks of a sample
+    const int64_t per = most > 0 ? cdiv(Ho, most) : Ho;
+    const int64_t tile = (stride * (per - 1) + 3) * (W + 2) * 2, per_row = cdiv(2 * (W + 2), kWave);
+    bool few = kind != kNoChannels && (stride == 1 || (stride == 2 && H % 2 == 0 && W % 2 == 0)) && most > 0 &&
+               per * Wo <= kFewPixels && per_row * (stride * (per - 1) + 3) <= kFewItems * (threads / kWave) && H * W * C * 2 < (1ll << 31);
+    if (few) {
+        NetFew a{(const _Float16 *)x, (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)out, norm, (int)H, (int)W,
+                 (int)Ho, (int)Wo, (int)per, (int)per_row, (uint32_t)cdiv(1 << 16, per_row), (uint32_t)cdiv(1 << 20, Wo),
+                 (float)gain, kFewCf, 0, 0};
+        const dim3 grid((unsigned)(groups * cdiv(Ho, per)), (unsigned)N);
+        a.tile = mma_round(a.sf + per * Wo * kTapPitch * 2);
+        a.channels = a.tile + (int)tile * 16;
+        int lds = 0;
+        if (kind == kChannelsMma) {
+            mma.a.lds = channel_mma_lds(C, channel.mid, 9, kMmaLds - a.channels);
+            few = mma.a.lds.chunk > 0;
+            lds = a.channels + mma.a.lds.total;
+        } else {
+            few = channel_rows_lds(rows.a, kMmaChannels);
+            lds = a.channels + rows.a.total;
+        }
+        few = few && lds <= kMmaLds;
+        if (few) {
+            const bool wide = Wo % 2 != 0;
+            bool done = false;
+#define DDF_NET_FEW_LAUNCH(KS_, S_, MUL_, WIDE_, CH_, ARGS_)                                                          \
+    hipLaunchKernelGGL((k_net_filter_few<KS_, S_, MUL_, WIDE_, CH_>), grid, dim3(threads), lds, st, a, ARGS_)
+#define DDF_NET_FEW(KS_, S_, CH_, ARGS_)                                         \
+    if (C == KS_ * 32 && stride == S_) {                                         \
+        if (wide && mul) DDF_NET_FEW_LAUNCH(KS_, S_, true, true, CH_, ARGS_);    \
+        else if (wide) DDF_NET_FEW_LAUNCH(KS_, S_, false, true, CH_, ARGS_);     \
+        else if (mul) DDF_NET_FEW_LAUNCH(KS_, S_, true, false, CH_, ARGS_);      \
+        else DDF_NET_FEW_LAUNCH(KS_, S_, false, false, CH_, ARGS_);              \
+        done = true;                                                             \
+    }
+            if (kind == kChannelsRows) {
+                DDF_NET_FEW(2, 1, kChannelsRows, rows) DDF_NET_FEW(4, 1, kChannelsRows, rows)
+                DDF_NET_FEW(2, 2, kChannelsRows, rows) DDF_NET_FEW(4, 2, kChannelsRows, rows)
+            } else {
+                DDF_NET_FEW(8, 1, kChannelsMma, mma) DDF_NET_FEW(16, 1, kChannelsMma, mma)
+                DDF_NET_FEW(8, 2, kChannelsMma, mma) DDF_NET_FEW(16, 2, kChannelsMma, mma)
+            }
+#undef DDF_NET_FEW
+#undef DDF_NET_FEW_LAUNCH
+            if (done) return hipGetLastError();
+        }
+    }
+    const hipError_t err = net_branches(x, w, bias, sf, gain, &channel, N, H, W, C, stride, st);
+    return err == hipSuccess ? net_filter(x, channel.cf, sf, norm, out, N, H, W, C, stride, mul, st) : err;
 }
 
 hipError_t net_pool(const void *x, void *out, int64_t N, int64_t plane, int64_t C, hipStream_t st) {

@@ -168,13 +168,12 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0]->size(0);
             nm = b.conv1.norm();
             covered(ddf_hip_net_conv_pool(cur, b.conv1.t[0]->data_ptr(), &nm, t1, pp, n, h, w, c, width, 1, st));
-            covered(ddf_hip_net_branches(
+            nm = b.bn2.norm();
+            covered(ddf_hip_net_ddf(
                 t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pp,
                 (int)ddf_hip_net_conv_pool_parts(n, h, w, c, width), b.w1->data_ptr(), ptr_or_null(b.b1),
                 b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid, b.cgain_const, ptr_or_null(b.cgain),
-                ptr_or_null(b.coffset), n, h, w, width, b.stride, st));
-            nm = b.bn2.norm();
-            covered(ddf_hip_net_filter(t1, cf, sf, &nm, t2, n, h, w, width, b.stride, b.combine, st));
+                ptr_or_null(b.coffset), &nm, t2, n, h, w, width, b.stride, b.combine, st));
             nm = b.conv3.norm();
             if (b.down.t[0].defined()) {
                 const ddf_net_norm_t down = b.down.norm();

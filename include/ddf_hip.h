@@ -370,6 +370,8 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *           ddf_hip_channel_branch_parts (3x3 taps) from the partial sums of conv_pool; sizes as
  *           spatial's
  *   filter  relu(norm(the operator)) with the filters of `spatial` and ddf_hip_channel_branch_parts
+ *   ddf     branches and filter: spatial_filter and channel_filter are work space (the launch may
+ *           be one that keeps them to itself)
  *   pool    mean over the pixels, (N, C)
  */
 typedef struct {
@@ -400,6 +402,11 @@ int ddf_hip_net_branches(const void *features, const void *spatial_weight, const
 int ddf_hip_net_filter(const void *features, const void *channel_filter, const void *spatial_filter,
                        const ddf_net_norm_t *norm, void *output, int64_t N, int64_t H, int64_t W, int64_t C,
                        int stride, int combine, void *stream);
+int ddf_hip_net_ddf(const void *features, const void *spatial_weight, const void *spatial_bias, void *spatial_filter,
+                    double spatial_gain, const float *pool_parts, int n_parts, const void *weight1, const void *bias1,
+                    const void *weight2, const void *bias2, void *channel_filter, int64_t mid, double channel_gain,
+                    const void *gain_vec, const void *offset_vec, const ddf_net_norm_t *norm, void *output, int64_t N,
+                    int64_t H, int64_t W, int64_t C, int stride, int combine, void *stream);
 int ddf_hip_net_pool(const void *features, void *output, int64_t N, int64_t pixels, int64_t C, void *stream);
 
 /*

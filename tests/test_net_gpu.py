@@ -234,3 +234,34 @@ def test_both_branches(n, h, w, c, s, mid, n_parts):
     close(sf[:, :, :9].permute(0, 2, 1).reshape(n, 9, ho, wo), want, 4e-3)
     ref = channel_reference(parts.double().sum(1).cpu() / (h * w), *(t.cpu() for t in (w1, b1, w2, b2)), 3, 0.7, gv.cpu(), ov.cpu())
     close(cf.cpu(), ref.view(n, c, 9), 6e-3)
+
+
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('n,h,w,c,s,mid,n_parts', [
+    (1, 56, 56, 64, 1, 12, 49), (3, 56, 56, 64, 1, 12, 25), (8, 56, 56, 64, 1, 12, 25),    # a row, 2 rows, two launches
+    (1, 1, 1, 64, 1, 12, 1), (3, 5, 9, 64, 1, 12, 2), (2, 10, 18, 64, 2, 12, 3),
+    (1, 28, 28, 128, 1, 25, 13), (3, 56, 30, 128, 2, 25, 9), (1, 3, 200, 128, 1, 25, 5),
+    (1, 14, 14, 256, 1, 51, 13), (8, 14, 14, 256, 1, 51, 2), (1, 28, 28, 256, 2, 51, 13), (5, 13, 11, 256, 1, 51, 3),
+    (1, 7, 7, 512, 1, 102, 4), (8, 7, 7, 512, 1, 102, 2), (3, 14, 14, 512, 2, 102, 3), (2, 4, 70, 512, 1, 102, 2),
+    (1, 6, 6, 512, 1, 300, 2),                                                              # w1 and w2 in parts
+    (2, 5, 5, 256, 1, 20, 3),                                                               # not covered
+])
+def test_ddf_layer(n, h, w, c, s, mid, n_parts, combine):
+    """Branches and filter of one call: what the two calls leave."""
+    torch.manual_seed(h * w + c)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    ws, bs = (torch.randn(9, c, device='cuda') * c ** -0.5).half(), torch.randn(9, device='cuda').half()
+    parts = torch.randn(n, n_parts, c, device='cuda')
+    w1, w2 = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((mid, c), (9 * c, mid)))
+    b1, b2, gv, ov = (torch.randn(k, device='cuda').half() for k in (mid, 9 * c, 9 * c, 9 * c))
+    ho, wo = h // s, w // s
+    sf = torch.empty(n, ho * wo, 12, device='cuda', dtype=torch.float16)
+    cf = torch.empty(n, c, 9, device='cuda', dtype=torch.float16)
+    want, got = (torch.full((n, ho, wo, c), float('nan'), device='cuda').half() for _ in range(2))
+    norm, apply, keep = make_norm(c, 1, 0)
+    branches = (x, ws, bs, sf, 0.6, parts, n_parts, w1, b1, w2, b2, cf, mid, 0.7, gv, ov)
+    call('ddf_hip_net_branches', *branches, n, h, w, c, s)
+    call('ddf_hip_net_filter', x, cf, sf, norm, want, n, h, w, c, s, _lib.COMBINE[combine])
+    call('ddf_hip_net_ddf', *branches, norm, got, n, h, w, c, s, _lib.COMBINE[combine])
+    assert torch.isfinite(want).all()
+    close(got, want, 2e-3)      # (order of the sums over the partial sums)
