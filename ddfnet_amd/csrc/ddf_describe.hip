@@ -23,6 +23,7 @@ const char *sums_name(unsigned fneed, int csplit, int nstrips, bool norm = false
 const char *layout_name(const RowsGeom &g) {
     if (g.cw > 0) return g.segs > 0 ? "ragged segments,stride 2" : "ragged,stride 2";
     if (g.Hi != g.H) return g.lp > g.lpr ? "padded,stride 2" : "plain,stride 2";
+    if (g.halo > 0) return g.tail > 0 ? "ragged run" : "run";
     if (g.tail > 0) return g.segs > 0 ? "ragged segments" : "ragged";
     return g.segs > 0 ? "segments" : g.lp > g.lpr ? "padded" : "plain";
 }

@@ -61,6 +61,10 @@ struct RowsGeom {
     // lp = lpr = seg_out + 2, nstrips = row groups * segs.
     int segs, seg_out;
     unsigned segs_magic;
+    // The plane's row groups one after the other, lp lanes each, are a run of lanes; a strip is
+    // `run` lanes of it (whole row groups, run = rg * lp; or, with halo = 1, as many as a wave has
+    // between one lane of the neighbouring strips on either side that it only reads).
+    int run, halo;
     // Rows that are no whole number of vectors (tail > 0: elements of the last vector that
     // belong to the row; see Ragged): shift: an odd tail of 2-byte elements, whose lane loads
     // from one element further left.
@@ -154,11 +158,13 @@ struct Lane {
             for (int r = 0; r < R; ++r) ooff[r] = (owns && y0 + r < g.H) ? (y0 + r) * g.W + x0 : -1;
             return;
         }
-        const int grp = magic_div(lane, g.lp_magic);
-        const int v = lane - grp * g.lp;
-        const bool live = grp < g.rg && v < g.lpr;
+        const int at = strip * g.run + lane - g.halo, slot = at < 0 ? 0 : at;
+        const int grp = magic_div(slot, g.lp_magic);
+        const int v = slot - grp * g.lp;
+        const bool live = at >= 0 && lane < g.run + 2 * g.halo && v < g.lpr;
+        const bool owns = live && lane >= g.halo && lane < g.run + g.halo;
         const int x0 = v * VX;
-        const int y0 = strip * g.rps + grp * R;
+        const int y0 = grp * R;
         first = v == 0;
         last = v == g.lpr - 1;
         ragged = RAGGED && live && last && g.tail > 0;
@@ -168,7 +174,7 @@ struct Lane {
             xoff[rr] = (live && yy >= 0 && yy < g.H) ? yy * g.W + x0 - (RAGGED && ragged ? g.shift : 0) : -1;
         }
 #pragma unroll
-        for (int r = 0; r < R; ++r) ooff[r] = (live && y0 + r < g.H) ? (y0 + r) * g.W + x0 : -1;
+        for (int r = 0; r < R; ++r) ooff[r] = (owns && y0 + r < g.H) ? (y0 + r) * g.W + x0 : -1;
     }
 };
 

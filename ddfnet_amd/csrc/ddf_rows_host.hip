@@ -54,6 +54,8 @@ void lay_out_lanes(RowsGeom *t, int H, int W, int vx, int R, bool padded = false
     t->nstrips = (row_units + rg_max - 1) / rg_max;
     t->rg = (row_units + t->nstrips - 1) / t->nstrips;      // even strips
     t->rps = t->rg * R;
+    t->run = t->rg * t->lp;
+    t->halo = 0;
 }
 
 // Channels per wave of k_rows: enough waves to fill the machine (and to even out
@@ -199,6 +201,39 @@ bool rows_cut(const Problem &p, int vx, int R, RowsGeom *g, int *vx_out, int *r_
     *vx_out = vx;
     *r_out = R;
     return true;
+}
+
+// The plane as one run of lanes (RowsGeom::halo) instead of strips of whole rows, in vectors of vx
+// and R rows per lane; false where that takes no strip less.  A strip of whole rows leaves up to
+// half of a wave's lanes idle (38 vectors of a 300-pixel row, 26 of a 101-pixel one); a run
+// leaves two, and one per row.  Forward, strips -> run: fp16 8 x 64 x 200 x 300 39.7 -> 34.9 us,
+// 5 x 5 at 8 x 64 x 90 x 100 18.8 -> 15.9, 3 x 77 x 140 x 190 12.1 -> 11.0; fp32 8 x 64 x 100 x
+// 150 17.0 -> 15.9, 12 x 144 x 80 x 87 27.2 -> 25.5; the feature gradient alone at 8 x 128 x 64 x
+// 88 with dilation 2 12.9 -> 11.6.  Launches that are over in a few microseconds keep the strips
+// (the run is not laid out for them): they wait for memory, whatever their lanes do.
+bool lay_out_run(const Problem &p, int vx, int R, const RowsGeom &rows, RowsGeom *g) {
+    if (tune_int("DDF_TUNE_ROWS_RUN", 1) == 0) return false;
+    RowsGeom t{};
+    t.C = (int)p.C; t.H = t.Hi = (int)p.H; t.W = t.Wi = (int)p.W;
+    t.tail = rows.tail;
+    t.shift = rows.shift;
+    t.lpr = (t.W + vx - 1) / vx;
+    t.lp = t.lpr + 1;
+    t.lp_magic = magic_of(t.lp);
+    t.rg = 1;
+    t.rps = R;
+    t.run = kWave - 2;
+    t.halo = 1;
+    const int64_t slots = (int64_t)((t.H + R - 1) / R) * t.lp;
+    if (slots * t.lp >= (1ll << 32) || slots >= (1ll << 30)) return false;    // (divisions by multiplication; see magic_div)
+    t.nstrips = (int)((slots + t.run - 1) / t.run);
+    if (t.nstrips >= rows.nstrips) return false;
+    *g = t;
+    return true;
+}
+bool rows_run_geometry(const Problem &p, int vx, int R, const RowsGeom &rows, RowsGeom *g) {
+    return lay_out_run(p, vx, R, rows, g) &&
+           cut_channels_forward(*g, p.N, g->C, p.k == 5 ? 2 : kRowsStages, p.H * p.W, p.k == 5 ? 32 / vx : 0);
 }
 
 // What the ragged-row variants cover.  (Planes of at most 64 pixels that the exact vectors do
@@ -361,8 +396,8 @@ bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r, bool b
     double best = exact ? rows_cost(*g, false, p.k, esz, *vx, *r) : 1e30;
     bool found = exact;
     RowsGeom t; int tvx, tr;
-    auto consider = [&]() {
-        const double c = rows_cost(t, true, p.k, esz, tvx, tr);
+    auto consider = [&](bool ragged) {
+        const double c = rows_cost(t, ragged, p.k, esz, tvx, tr);
         if (c >= best) return;
         best = c;
         found = true;
@@ -371,13 +406,23 @@ bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r, bool b
         *r = tr;
     };
     if (p.s == 2) {
-        if (stride2_ragged_geometry(p, dtype, false, backward, &t, &tvx, &tr)) consider();
+        if (stride2_ragged_geometry(p, dtype, false, backward, &t, &tvx, &tr)) consider(true);
         return found;
     }
     // (what the shortest ragged walk takes: small launches are decided without laying it out)
     if (best <= (std::min<int64_t>(p.C, 2 * kRowsStages) + 3.0) * (40 + (p.k == 5 ? 45 : 16) * 4) * 2.5) return true;
+    const RowsGeom whole = *g;
+    const int exact_vx = *vx, exact_r = *r;
     for (tvx = 16 / esz; tvx >= 4; tvx /= 2)
-        if (rows_ragged_geometry(p, dtype, tvx, &t, &tr)) consider();
+        if (rows_ragged_geometry(p, dtype, tvx, &t, &tr)) consider(true);
+    // (ragged rows take operands at any address: such a launch stays one, as a run or not)
+    tvx = exact_vx;
+    tr = exact_r;
+    if (exact && g->tail == 0 && rows_run_geometry(p, tvx, tr, whole, &t)) consider(false);
+    for (tvx = 16 / esz; tvx >= 4; tvx /= 2) {
+        RowsGeom rows;
+        if (rows_ragged_geometry(p, dtype, tvx, &rows, &tr) && rows_run_geometry(p, tvx, tr, rows, &t)) consider(true);
+    }
     return found;
 }
 

@@ -53,6 +53,28 @@ def test_wide_vectors_instead_of_single_pixels(shape, combine, dtype):
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
 @pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('shape,k,d', [((4, 40, 113, 150), 3, 1), ((4, 33, 50, 263), 3, 1), ((2, 33, 140, 301), 3, 1),
+                                       ((5, 36, 200, 296), 3, 1), ((4, 40, 113, 150), 3, 2), ((2, 33, 140, 301), 3, 2),
+                                       ((2, 33, 140, 301), 5, 1), ((4, 66, 113, 133), 5, 1), ((2, 33, 140, 301), 5, 2),
+                                       ((4, 66, 113, 133), 5, 2)], ids=_ids)
+def test_planes_as_one_run_of_lanes(shape, k, d, combine, dtype):
+    """Strips that end inside an image row: every vector width, with and without a tail; the
+    result, each gradient on its own and all of them."""
+    for need in (0, _lib.NEED_DX):
+        name = _lib.describe(shape, k, d, 1, combine, dtype, need) if need else \
+            _lib.describe(shape, k, d, 1, combine, dtype)
+        assert 'run>' in name, name
+    x, cf, sf, go = random_case(*shape, k, 1, dtype, seed=k + d)
+    want = (oracle.forward(x, cf, sf, k, d, 1, combine),) + tuple(oracle.backward(go, x, cf, sf, k, d, 1, combine))
+    for need in ((True, False, False), (False, True, True), (True, True, True)):
+        got = run_ddf(x, cf, sf, go, k, d, 1, combine, need=need)
+        for g, w in zip(got, want):
+            if g is not None:
+                assert rel_err(g, w) <= TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
+@pytest.mark.parametrize('combine', ['mul', 'add'])
 @pytest.mark.parametrize('H,W', [(9, 10), (8, 11), (7, 12), (10, 13), (31, 15), (24, 18), (13, 30), (12, 63), (11, 131),
                                  (9, 261), (6, 262), (7, 263), (4, 286), (3, 257), (2, 135)])
 def test_stride_two_of_any_size(H, W, combine, dtype):
