@@ -59,8 +59,8 @@ __device__ __forceinline__ void wave_sync() {
 // S = 2 (3 x 3, one row per lane): g describes the dO plane, the lane's feature
 // vectors are 2 * VX elements wide (LaneStride2).  With DX the lane of result
 // row y also writes the feature gradient of feature rows 2y and 2y + 1.
-// SEG (with DX): image rows are cut into segments, whose outer lanes hold dO
-// values they do not own; those are kept out of the filter sums.
+// SEG (with DX): strips end inside image rows (segments, or a plane as one run of lanes), whose
+// outer lanes hold dO values they do not own; those are kept out of the filter sums.
 template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, bool DX, int NST, int WPE,
           int S = 1, bool SEG = true, int TAIL = 0>
 __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
@@ -349,9 +349,9 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
                 if (!DX || S == 2 || row_needed<R, K, D>(r)) rag.fix(gw[ST][r]);
         }
         // dO at the lane's own pixels.  (DX loads dO through the window offsets, so a
-        // lane that only reads for its neighbours - the outer lanes of a row segment -
-        // holds real values here: they must not enter the filter sums twice.  Without
-        // segments every lane that owns nothing reads zeros anyway.)
+        // lane that only reads for its neighbours - the outer lanes of a row segment or a
+        // run - holds real values here: they must not enter the filter sums twice.  In strips
+        // of whole rows every lane that owns nothing reads zeros anyway.)
         A gval[R][VX];
 #pragma unroll
         for (int r = 0; r < R; ++r)

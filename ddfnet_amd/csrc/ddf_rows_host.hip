@@ -236,6 +236,20 @@ bool rows_run_geometry(const Problem &p, int vx, int R, const RowsGeom &rows, Ro
            cut_channels_forward(*g, p.N, g->C, p.k == 5 ? 2 : kRowsStages, p.H * p.W, p.k == 5 ? 32 / vx : 0);
 }
 
+// Channels split as for another cut of the same problem; `items`: waves or workgroups per strip
+// and channel range.
+void cut_channels_like(RowsGeom &t, const RowsGeom &g, int64_t items) {
+    t.cpw = g.cpw;
+    t.cpb = g.cpb;
+    t.csplit = g.csplit;
+    t.wpb = g.wpb;
+    t.csplit_magic = g.csplit_magic;
+    t.nstrips_magic = magic_of(t.nstrips);
+    t.nwork = (int)(items * t.nstrips * t.csplit);
+    const int64_t ngroups = (t.nwork + t.wpb - 1) / t.wpb;
+    t.xcd_per = (unsigned)((ngroups + rows::kXcd - 1) / rows::kXcd);
+}
+
 // What the ragged-row variants cover.  (Planes of at most 64 pixels that the exact vectors do
 // not cover belong to the kernel that packs several of them into a workgroup.)
 bool ragged_shape(const Problem &p, int dtype, int vx) {
@@ -245,7 +259,7 @@ bool ragged_shape(const Problem &p, int dtype, int vx) {
     return p.H * p.W > 64 && (int64_t)p.H * p.W * 8 < (1ll << 31) && tune_int("DDF_TUNE_RAGGED", 1) != 0;
 }
 
-constexpr int64_t kSimds = 1024;
+constexpr int64_t kCus = 256, kSimds = 4 * kCus;
 
 // Channels per wave of k_rows_taprow_filters (one wave per filter row).
 bool cut_channels_taprow(RowsGeom &t, const Problem &p) {
@@ -316,6 +330,17 @@ double rows_cost(const RowsGeom &g, bool ragged, int k, int esz, int vx, int r) 
 double rows_filters_cost(const RowsGeom &g, bool ragged, int vx, int r) {
     const double waves = (double)g.nwork * rows::kFilterWaves;
     return (g.cpw + 3.0) * (60 + 50 * vx * r) * (ragged ? 1.1 : 1.0) * std::max(1.0, waves / kSimds);
+}
+
+// The same in whole workgroups per CU.
+double rows_filters_steps(const RowsGeom &g, bool ragged, int vx, int r) {
+    return (g.cpw + 3.0) * (60 + 50 * vx * r) * (ragged ? 1.1 : 1.0) * ((g.nwork + kCus - 1) / kCus);
+}
+
+// And of k_rows_taprow_filters (some 40 instructions per channel and 25 per pixel of a lane) in
+// whole waves per SIMD.
+double taprow_steps(const RowsGeom &g, int vx) {
+    return (g.cpw + 3.0) * (40 + 25 * vx) * (g.tail > 0 ? 1.1 : 1.0) * ((g.nwork + kSimds - 1) / kSimds);
 }
 
 }  // namespace
@@ -482,23 +507,58 @@ bool rows_filters_plan(const Problem &p, int dtype, bool fused, RowsGeom *g, int
     const bool exact = rows_filters_geometry(p, dtype, fused, g, vx, r);
     if (fused && tune_int("DDF_TUNE_ROWSF_FUSED", 1) == 0) return exact;
     RowsGeom t{};
-    int tvx = 4, tr = 1;
-    if (p.s == 2) {
-        if (!stride2_ragged_geometry(p, dtype, true, fused, &t, &tvx, &tr)) return exact;
-    } else {
-        if (p.k != 3 || (p.d != 1 && p.d != 2) || !ragged_shape(p, dtype, tvx)) return exact;
-        t.C = (int)p.C; t.H = t.Hi = (int)p.H; t.W = t.Wi = (int)p.W;
-        lay_out_lanes(&t, t.H, t.W, tvx, tr);
-        if (!cut_channels_filters(t, p.N, t.C)) return exact;
-        t.shift = dtype == DDF_F16 ? t.tail & 1 : 0;
-    }
     // All gradients at 12 x 144 x 80 x 87 fp32: 63 -> 42 us; 3 x 3 with dilation 2 at 4 x 64 x
     // 60 x 131, which only the LDS-tile kernels covered, 178 -> 18.5; 2 x 256 x 25 x 38 keeps
     // single pixels, 11.3 us against 12.6.
-    if (exact && rows_filters_cost(t, true, tvx, tr) >= rows_filters_cost(*g, false, *vx, *r)) return true;
-    *g = t;
-    *vx = tvx;
-    *r = tr;
+    bool found = exact;
+    double best = exact ? rows_filters_cost(*g, false, *vx, *r) : 1e30;
+    auto consider = [&](bool ragged, int tvx, int tr) {
+        const double c = rows_filters_cost(t, ragged, tvx, tr);
+        if (c >= best) return;
+        best = c;
+        found = true;
+        *g = t;
+        *vx = tvx;
+        *r = tr;
+    };
+    if (p.s == 2) {
+        int tvx, tr;
+        if (stride2_ragged_geometry(p, dtype, true, fused, &t, &tvx, &tr)) consider(true, tvx, tr);
+        return found;
+    }
+    const RowsGeom whole = *g;
+    const int exact_vx = *vx, exact_r = *r;
+    const bool any_tail = p.k == 3 && (p.d == 1 || p.d == 2) && ragged_shape(p, dtype, 4);
+    RowsGeom rows{};
+    if (any_tail) {
+        rows.C = (int)p.C; rows.H = rows.Hi = (int)p.H; rows.W = rows.Wi = (int)p.W;
+        lay_out_lanes(&rows, rows.H, rows.W, 4, 1);
+        rows.shift = dtype == DDF_F16 ? rows.tail & 1 : 0;
+        t = rows;
+        if (cut_channels_filters(t, p.N, t.C)) consider(true, 4, 1);
+    }
+    // The plane as one run of lanes, with the channels split as before if that leaves a workgroup
+    // per CU: where it takes three
+    // tenths of the strips away, or leaves the fullest CU fewer workgroups to walk.  (A CU holds
+    // two: 360 of them at 12 x 144 x 80 x 87 take what 480 do, and 4 % more.)  All gradients,
+    // strips -> run: fp16 8 x 64 x 200 x 300 106 -> 75 us, 1 x 128 x 180 x 260 34.0 -> 25.8; fp32
+    // 4 x 64 x 200 x 300 71 -> 58, 8 x 64 x 100 x 150 47 -> 39, 2 x 100 x 130 x 140 32.1 -> 22.5.
+    // (A ragged cut stays one: see rows_plan.)
+    if (!found) return false;
+    const RowsGeom strips = *g;
+    best = rows_filters_steps(strips, strips.tail > 0, *vx, *r);
+    auto consider_run = [&](bool ragged, int tvx, int tr) {
+        cut_channels_like(t, strips, p.N);
+        if (t.nwork < kCus && !cut_channels_filters(t, p.N, t.C)) return;   // (too few workgroups)
+        const double c = rows_filters_steps(t, ragged, tvx, tr);
+        if (c > best || (c == best && t.nstrips * 10 > strips.nstrips * 7)) return;
+        best = c;
+        *g = t;
+        *vx = tvx;
+        *r = tr;
+    };
+    if (exact && strips.tail == 0 && lay_out_run(p, exact_vx, exact_r, whole, &t)) consider_run(false, exact_vx, exact_r);
+    if (any_tail && lay_out_run(p, 4, 1, rows, &t)) consider_run(true, 4, 1);
     return true;
 }
 
@@ -544,6 +604,7 @@ bool rows_taprow_geometry(const Problem &p, int dtype, RowsGeom *g, int *vx_out,
 bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r) {
     const bool exact = rows_taprow_geometry(p, dtype, g, vx, r);
     if (p.k != 5 || (p.d != 1 && p.d != 2)) return exact;
+    bool found = exact;
     // 16-byte vectors, or 8-byte ones of fp16 where those of 16 leave too few workgroups
     for (int cand = dtype == DDF_F16 ? 8 : 4; cand >= 4; cand /= 2) {
         if (!ragged_shape(p, dtype, cand)) continue;
@@ -559,13 +620,42 @@ bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r)
         // (as rows_plan; some 40 instructions per channel and 25 per pixel of a lane.  All
         // gradients at 2 x 48 x 135 x 166 fp32, 5 x 5: 1056 -> 36 us.)
         if (exact && (int64_t)t.nstrips * (40 + 25 * cand) * 11 >= (int64_t)g->nstrips * (40 + 25 * *vx) * 10)
-            return true;
+            break;
         *g = t;
         *vx = cand;
         *r = 1;
-        return true;
+        found = true;
+        break;
     }
-    return exact;
+    if (!found) return false;
+    // The plane as one run of lanes (a ragged cut stays one: see rows_plan), the channels split as
+    // before or anew.  Ragged rows are not split for it: their partial sums are stored value by
+    // value (4 x 64 x 113 x 150 fp32 29 us, in two channel ranges 36).  Filter gradients, strips ->
+    // run: fp32 8 x 64 x 90 x 100 40.5 -> 28.6 us, 2 x 96 x 140 x 301 48.7 -> 41.0, 4 x 128 x 60 x
+    // 131 37.7 -> 29.9; fp16 8 x 64 x 200 x 304 162 -> 108.
+    const RowsGeom strips = *g;
+    RowsGeom rows{}, t{};
+    rows.C = (int)p.C; rows.H = rows.Hi = (int)p.H; rows.W = rows.Wi = (int)p.W;
+    double best = taprow_steps(strips, *vx);
+    for (int cand = dtype == DDF_F16 ? 8 : 4; cand >= std::max(2, p.r * p.d); cand /= 2) {
+        const bool ragged = p.W % cand != 0;
+        if (ragged ? cand < 4 || !ragged_shape(p, dtype, cand) : strips.tail > 0) continue;
+        lay_out_lanes(&rows, rows.H, rows.W, cand, 1);
+        if (cand > 4 && p.N * rows.nstrips * p.k < 2048) continue;
+        rows.shift = dtype == DDF_F16 ? rows.tail & 1 : 0;
+        if (!lay_out_run(p, cand, 1, rows, &t)) continue;
+        for (int anew = 0; anew < 2; ++anew) {
+            if (anew && ragged && strips.csplit == 1 && t.nwork >= kSimds) break;
+            if (!anew) cut_channels_like(t, strips, p.N * p.k);
+            else if (!cut_channels_taprow(t, p)) break;
+            const double c = taprow_steps(t, cand);
+            if (c >= best) continue;
+            best = c;
+            *g = t;
+            *vx = cand;
+        }
+    }
+    return true;
 }
 
 bool rows_cover_backward(const Problem &p, int dtype) {

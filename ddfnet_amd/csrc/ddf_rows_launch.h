@@ -173,8 +173,8 @@ hipError_t launch_filters_v(const Problem &p, const RowsGeom &g, const T *go, co
     const int lds = filters_lds_bytes<9>((int)sizeof(A), R, VX);
     if (p.k != 3 || (p.d != 1 && p.d != 2)) return hipErrorNotSupported;
     const bool pad = rows_shift_in_as_is(g);
-    // (row segments: only the launch that also writes the feature gradient tells them apart)
-    const bool seg = DX && g.segs > 0;
+    // (lanes that only read: only the launch that also writes the feature gradient tells them apart)
+    const bool seg = DX && (g.segs > 0 || g.halo > 0);
 #define DDF_ROWSF_CASE(D_, MUL_, PAD_, SEG_)                                                     \
     hipLaunchKernelGGL((k_rows_filters<T, 3, D_, MUL_, VX, R, PAD_, DX, kFilterStages,           \
                                        MUL_ ? WPE_MUL : WPE_ADD, 1, SEG_>),                      \

@@ -335,15 +335,16 @@ static void check_rows(long N, long C, long H, long W, int k, int d, int dtype, 
 
 // A plane's row groups as one run of lanes (RowsGeom::halo): every lane of every strip loads its
 // own rows or nothing, every pixel belongs to one lane, and that lane's neighbours in the wave
-// hold the vectors left and right of it, or nothing where its image row ends.
+// hold the vectors left and right of it, or nothing where its image row ends.  dy: the window's
+// rows are taken dy rows further down (kind 2, once per filter row).
 template <int R, int HY, int VX>
-static void replay_rows_run(const RowsGeom &g, long N, long C, bool filters) {
+static void replay_rows_run(const RowsGeom &g, long N, long C, int kind, int taps, int dy) {
     std::vector<int> owner((size_t)g.H * g.W, 0);
     CHECK(g.segs == 0 && g.run >= 1 && g.run + 2 <= 64 && g.lp == g.lpr + 1 && g.lpr == (g.W + VX - 1) / VX &&
           g.tail == g.W % VX, "lanes of a run");
     for (int strip = 0; strip < g.nstrips; ++strip) {
         rows::Lane<R, HY, VX, true> wave[64];
-        for (int lane = 0; lane < 64; ++lane) wave[lane].init(g, strip, lane);
+        for (int lane = 0; lane < 64; ++lane) wave[lane].init(g, strip, lane, dy);
         for (int lane = 0; lane < 64; ++lane) {
             const rows::Lane<R, HY, VX, true> &ln = wave[lane];
             const long at = (long)strip * g.run + lane - 1;
@@ -352,55 +353,62 @@ static void replay_rows_run(const RowsGeom &g, long N, long C, bool filters) {
             CHECK(!live || (ln.first == (v == 0) && ln.last == (v == g.lpr - 1)), "row ends");
             CHECK(ln.ragged == (live && v == g.lpr - 1 && g.tail > 0), "last vector of a row");
             for (int rr = 0; rr < R + 2 * HY; ++rr) {
-                const int yy = y0 - HY + rr;
-                CHECK(ln.xoff[rr] == (live && yy >= 0 && yy < g.H ? yy * g.W + x0 - (ln.ragged ? g.shift : 0) : -1),
+                const int yy = y0 - HY + rr + dy;
+                const bool reads = yy >= 0 && yy < g.H;
+                CHECK(ln.xoff[rr] == (live && reads ? yy * g.W + x0 - (ln.ragged ? g.shift : 0) : -1),
                       "lane %d window row %d", lane, rr);
+                if (!owns) continue;
+                for (int side : {-1, 1}) {
+                    const rows::Lane<R, HY, VX, true> &by = wave[lane + side];
+                    const bool inside = reads && (side < 0 ? v > 0 : v < g.lpr - 1);
+                    CHECK(by.xoff[rr] == (inside ? yy * g.W + x0 + side * VX - (by.ragged ? g.shift : 0) : -1),
+                          "lane %d's neighbour %d", lane, side);
+                }
             }
             for (int r = 0; r < R; ++r) {
                 CHECK(ln.ooff[r] == (owns && y0 + r < g.H ? (y0 + r) * g.W + x0 : -1), "lane %d result row %d", lane, r);
-                if (ln.ooff[r] < 0) continue;
-                for (int x = x0; x < std::min(x0 + VX, g.W); ++x) ++owner[(size_t)(y0 + r) * g.W + x];
-                for (int side : {-1, 1}) {
-                    const rows::Lane<R, HY, VX, true> &by = wave[lane + side];
-                    const bool inside = side < 0 ? v > 0 : v < g.lpr - 1;
-                    CHECK(by.xoff[HY + r] == (inside ? (y0 + r) * g.W + x0 + side * VX - (by.ragged ? g.shift : 0) : -1),
-                          "lane %d's neighbour %d", lane, side);
-                }
+                if (ln.ooff[r] >= 0)
+                    for (int x = x0; x < std::min(x0 + VX, g.W); ++x) ++owner[(size_t)(y0 + r) * g.W + x];
             }
         }
     }
     for (size_t i = 0; i < owner.size(); ++i)
         if (owner[i] != 1) { CHECK(false, "pixel %zu owned %d times", i, owner[i]); break; }
-    check_work_items(g, N, C, filters ? 1 : 0, 0);
+    check_work_items(g, N, C, kind, taps);
 }
 
-// Whether the cut of a problem is such a run.
-static bool check_rows_run(long N, long C, long H, long W, int k, int d, int dtype, bool filters, bool fused) {
+// kind 0: k_rows, 1: k_rows_filters (`fused`: with the feature gradient), 2: k_rows_taprow_filters.
+static void check_rows_run(long N, long C, long H, long W, int k, int d, int dtype, int kind, bool fused = false) {
     const Problem p = make_problem(N, C, H, W, k, d, 1, 0);
     RowsGeom g{};
     int vx, r;
-    if (!(filters ? rows_filters_plan(p, dtype, fused, &g, &vx, &r) : rows_plan(p, dtype, &g, &vx, &r)) || g.halo == 0) {
-        printf("kind rows-run %ldx%ldx%ldx%ld k%d d%d dt%d f%d: unsupported\n", N, C, H, W, k, d, dtype, filters + fused);
-        return false;
+    const bool ok = kind == 2   ? rows_taprow_plan(p, dtype, &g, &vx, &r)
+                    : kind == 1 ? rows_filters_plan(p, dtype, fused, &g, &vx, &r)
+                                : rows_plan(p, dtype, &g, &vx, &r);
+    if (!ok || g.halo == 0) {
+        printf("kind rows-run%d %ldx%ldx%ldx%ld k%d d%d dt%d: unsupported\n", kind, N, C, H, W, k, d, dtype);
+        return;
     }
-    printf("kind rows-run %ldx%ldx%ldx%ld k%d d%d dt%d f%d: vx=%d r=%d tail=%d nstrips=%d cpw=%d csplit=%d wpb=%d nwork=%d\n",
-           N, C, H, W, k, d, dtype, filters + fused, vx, r, g.tail, g.nstrips, g.cpw, g.csplit, g.wpb, g.nwork);
+    printf("kind rows-run%d %ldx%ldx%ldx%ld k%d d%d dt%d: vx=%d r=%d tail=%d nstrips=%d cpw=%d csplit=%d wpb=%d nwork=%d\n",
+           kind, N, C, H, W, k, d, dtype, vx, r, g.tail, g.nstrips, g.cpw, g.csplit, g.wpb, g.nwork);
     CHECK(dtype != 2 && (k / 2) * d <= vx && g.halo == 1, "taps reach beyond the neighbouring lane");
-    if (filters) {
+    if (kind == 1) {
         CHECK(rows::filters_lds_bytes<9>(4, r, vx) <= 64 * 1024, "filter kernel LDS");
         CHECK(g.cpw % rows::kFlushChannels == 0, "channels per wave %d not whole flush groups", g.cpw);
     }
-    const int hy = (k / 2) * d;
+    const int hy = kind == 2 ? 0 : (k / 2) * d;
     bool done = false;
-#define RUN_CASE(R_, HY_, VX_) if (r == R_ && hy == HY_ && vx == VX_) { replay_rows_run<R_, HY_, VX_>(g, N, C, filters); done = true; }
-    RUN_CASE(1, 1, 1) RUN_CASE(1, 1, 2) RUN_CASE(1, 1, 4) RUN_CASE(1, 1, 8) RUN_CASE(2, 1, 2) RUN_CASE(2, 1, 4) RUN_CASE(2, 1, 8)
-    RUN_CASE(1, 2, 2) RUN_CASE(1, 2, 4) RUN_CASE(1, 2, 8) RUN_CASE(2, 2, 2) RUN_CASE(2, 2, 4) RUN_CASE(2, 2, 8)
-    RUN_CASE(1, 4, 4) RUN_CASE(1, 4, 8)
+    for (int i = 0; i < (kind == 2 ? k : 1); ++i) {
+        const int dy = kind == 2 ? (i - k / 2) * d : 0;
+#define RUN_CASE(R_, HY_, VX_) if (r == R_ && hy == HY_ && vx == VX_) { replay_rows_run<R_, HY_, VX_>(g, N, C, kind, kind == 2 ? k : 0, dy); done = true; }
+        RUN_CASE(1, 1, 1) RUN_CASE(1, 1, 2) RUN_CASE(1, 1, 4) RUN_CASE(1, 1, 8) RUN_CASE(2, 1, 2) RUN_CASE(2, 1, 4)
+        RUN_CASE(2, 1, 8) RUN_CASE(1, 2, 2) RUN_CASE(1, 2, 4) RUN_CASE(1, 2, 8) RUN_CASE(2, 2, 2) RUN_CASE(2, 2, 4)
+        RUN_CASE(2, 2, 8) RUN_CASE(1, 4, 4) RUN_CASE(1, 4, 8) RUN_CASE(1, 0, 2) RUN_CASE(1, 0, 4) RUN_CASE(1, 0, 8)
 #undef RUN_CASE
+    }
     CHECK(done, "no replay for r=%d hy=%d vx=%d", r, hy, vx);
     if (g_fails) printf("  -> %d violations\n", g_fails);
     g_fails = 0;
-    return true;
 }
 
 // Stride 2 (3 x 3) on the row-register kernels: lanes are laid out over the result plane;
@@ -624,8 +632,14 @@ int main() {
     // planes as one run of lanes, in every vector width, with and without a tail
     for (long H : {17l, 90l, 113l, 140l})
         for (long W : {45l, 47l, 58l, 61l, 85l, 87l, 90l, 100l, 101l, 150l, 166l, 263l, 300l, 301l, 312l, 600l, 1001l})
-            for (int i = 0; i < 24; ++i)
-                check_rows_run(8, 96, H, W, i & 1 ? 5 : 3, i & 2 ? 2 : 1, i >> 2 & 1, i >= 8, i >= 16);
+            for (int dtype = 0; dtype < 2; ++dtype)
+                for (int d = 1; d <= 2; ++d) {
+                    check_rows_run(8, 96, H, W, 3, d, dtype, 0);
+                    check_rows_run(8, 96, H, W, 5, d, dtype, 0);
+                    check_rows_run(8, 96, H, W, 3, d, dtype, 1);
+                    check_rows_run(8, 96, H, W, 3, d, dtype, 1, true);
+                    check_rows_run(8, 96, H, W, 5, d, dtype, 2);
+                }
     // seeded random shapes on top of the fixed list
     unsigned long long state = 0x9E3779B97F4A7C15ull;
     auto next = [&](int lo, int hi) {

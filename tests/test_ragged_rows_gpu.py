@@ -75,6 +75,28 @@ def test_planes_as_one_run_of_lanes(shape, k, d, combine, dtype):
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
 @pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('shape,k,d', [((2, 100, 130, 140), 3, 1), ((8, 33, 100, 150), 3, 1), ((4, 70, 45, 90), 3, 1),
+                                       ((2, 33, 140, 301), 3, 1), ((3, 37, 90, 130), 3, 2), ((2, 33, 140, 301), 3, 2),
+                                       ((3, 66, 60, 100), 5, 1), ((8, 70, 40, 44), 5, 1), ((4, 66, 113, 133), 5, 1),
+                                       ((2, 40, 200, 304), 5, 1), ((3, 66, 60, 100), 5, 2), ((2, 33, 140, 301), 5, 2)],
+                         ids=_ids)
+def test_filter_gradients_in_one_run_of_lanes(shape, k, d, combine, dtype):
+    """The same for the filter gradients, whose read-only lanes must stay out of the sums: with
+    the feature gradient and without, with and without a channel split, each filter alone."""
+    for need in (6, 7):
+        name = _lib.describe(shape, k, d, 1, combine, dtype, need).split('filters')[-1]
+        assert 'run>' in name, name
+    x, cf, sf, go = random_case(*shape, k, 1, dtype, seed=k + d)
+    want = (oracle.forward(x, cf, sf, k, d, 1, combine),) + tuple(oracle.backward(go, x, cf, sf, k, d, 1, combine))
+    for need in ((False, True, False), (False, False, True), (False, True, True), (True, True, True)):
+        got = run_ddf(x, cf, sf, go, k, d, 1, combine, need=need)
+        for g, w in zip(got, want):
+            if g is not None:
+                assert rel_err(g, w) <= TOL[dtype]
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=_ids)
+@pytest.mark.parametrize('combine', ['mul', 'add'])
 @pytest.mark.parametrize('H,W', [(9, 10), (8, 11), (7, 12), (10, 13), (31, 15), (24, 18), (13, 30), (12, 63), (11, 131),
                                  (9, 261), (6, 262), (7, 263), (4, 286), (3, 257), (2, 135)])
 def test_stride_two_of_any_size(H, W, combine, dtype):
