@@ -528,7 +528,11 @@ __global__ __launch_bounds__(kWave * kFilterWaves, WPE) void k_rows_filters(
     // whole rounds of NST channels (see k_rows)
     auto step = [&](auto st_tag, int ci) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_tag)::value;
-        // (loads first, and nothing moves between steps: see k_rows)
+        // (loads first, and nothing moves between steps; taps before the next ones: see k_rows)
+        if constexpr (kScalarTaps && kFilters) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) asm volatile("" : "+s"(cfu[ST][t]));
+        }
         issue(std::integral_constant<int, (ST + NST - 1) % NST>{}, ci + NST - 1);
         __builtin_amdgcn_sched_barrier(0);
         compute(st_tag, ci);
