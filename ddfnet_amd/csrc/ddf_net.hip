@@ -171,6 +171,11 @@ struct TapWeights {
 // larger tiles and a K order turned per tile change nothing there; the matrix cores are busy a
 // third of the time, and 98 tiles for an XCD's 96 places cost 125 -> 128 images 10 %.  The wide
 // results of the 56 x 56 layers run at copy rate.
+// On the way out the vector ALU counts as much as memory (half of its time at 56 x 56): all of a
+// thread's vectors come from LDS at once, and eight results take 24 instructions instead of 57 -
+// fp16 operands inside the multiply-adds, ReLU two at a time after the rounding.  Batch 128, us:
+// 56 x 56 x 64 -> 256 with a residual 91.9 -> 85.0, 28 x 28 x 128 -> 512 54.4 -> 48.3, 14 x 14 x
+// 256 -> 1024 38.4 -> 34.2; pairs 95 -> 81 (28 x 28 x 128 + 256 -> 512), 80 -> 67 (7 x 7).
 //
 // With PAIR the tile is act(affine(x w) + affine'(x' w')) of two products, a bottleneck's last
 // convolution and its projection: x' w' goes first, its affine result stays in registers as
@@ -187,13 +192,13 @@ template <int N>
 __device__ __forceinline__ void arrive() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
-template <int BM, int BN, int KST, int ST, int WG, bool PAIR, bool POOL>
+template <int BM, int BN, int KST, int ST, int WG, bool PAIR, bool POOL, bool RES>
 __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, int tiles_n, int tiles) {
     constexpr int CH = KST / 8, STAGE = (BM + BN) * KST;
     constexpr int RX = BM * CH / kThreads, RW = BN * CH / kThreads;
     constexpr int TM = BM / 64, TN = BN / 64;      // 32-wide tiles per wave: pixels, channels
     constexpr int PITCH = BN + 8;
-    static_assert(ST >= 2 && ST <= 4 && (CH == 4 || CH == 8) && RX > 0 && RW > 0);
+    static_assert((ST == 2 || ST == 3) && (CH == 4 || CH == 8) && RX > 0 && RW > 0 && !(RES && PAIR));
     extern __shared__ __align__(16) _Float16 net_smem[];
     __shared__ float affine[PAIR ? 4 : 1][PAIR ? BN : 1];    // scale, shift; of the first product, too
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -203,25 +208,34 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     const int tm = block / tiles_n, tn = block - tm * tiles_n;
     const int64_t m0 = (int64_t)tm * BM;
     const int n0 = tn * BN;
+    const int rows = (int)min((int64_t)BM, a.M - m0);    // pixels of the tile
     auto turn = [](int r) { return CH == 8 ? (r >> 1) & 7 : (r >> 2) & 3; };
 
     const _Float16 *xp[RX], *wp[RW];
     auto aim = [&](const NetConv &c) __attribute__((always_inline)) {
+        const _Float16 *x = static_cast<const _Float16 *>(c.x), *w = static_cast<const _Float16 *>(c.w) + (int64_t)n0 * c.K;
+        if (c.stride > 1) {
+            const int64_t sample = m0 / c.npix;
+            const int at = (int)(m0 - sample * c.npix);
 #pragma unroll
-        for (int i = 0; i < RX; ++i) {
-            const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
-            int64_t m = m0 + r < a.M ? m0 + r : a.M - 1;
-            if (c.stride > 1) {
-                const int64_t n = m / c.npix;
-                const int p = (int)(m - n * c.npix), y = p / c.Wo, xx = p - y * c.Wo;
-                m = (n * c.H + y * c.stride) * c.W + xx * c.stride;
+            for (int i = 0; i < RX; ++i) {
+                const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+                const unsigned pix = (unsigned)(at + min(r, rows - 1)), n = pix / (unsigned)c.npix, p = pix - n * c.npix;
+                const unsigned y = p / (unsigned)c.Wo, xx = p - y * c.Wo;
+                xp[i] = x + (((sample + n) * c.H + y * c.stride) * c.W + xx * c.stride) * c.K + ch * 8;
             }
-            xp[i] = static_cast<const _Float16 *>(c.x) + m * c.K + ch * 8;
+        } else {
+            x += m0 * c.K;
+#pragma unroll
+            for (int i = 0; i < RX; ++i) {
+                const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+                xp[i] = x + ((int64_t)min(r, rows - 1) * c.K + ch * 8);
+            }
         }
 #pragma unroll
         for (int i = 0; i < RW; ++i) {
             const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
-            wp[i] = static_cast<const _Float16 *>(c.w) + (int64_t)min(n0 + r, a.N - 1) * c.K + ch * 8;
+            wp[i] = w + ((int64_t)min(r, a.N - 1 - n0) * c.K + ch * 8);
         }
     };
     const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) _Float16 *)net_smem;
@@ -265,7 +279,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                     for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)b[e];
             }
     }
-    auto multiply = [&](int buf) {
+    auto multiply = [&](int buf) __attribute__((always_inline)) {
         const _Float16 *s = net_smem + buf * STAGE;
 #pragma unroll
         for (int kk = 0; kk < KST / 16; ++kk) {
@@ -289,23 +303,23 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
     };
     // what the tile's results meet on their way out: this thread's eight channels, and the
-    // residual of its pixels (requested before the last stage is multiplied)
+    // residual of its pixels
     constexpr int CPR = BN / 8;                     // vectors per pixel
-    constexpr int RO = BM * CPR / kThreads;
-    const int cq = tid % CPR, c = n0 + cq * 8;
+    constexpr int RO = BM * CPR / kThreads, STEP = kThreads / CPR;
+    const int cq = tid % CPR, r0 = tid / CPR, c = n0 + cq * 8;
     const bool cok = c < a.N;
-    const _Float16 *res = static_cast<const _Float16 *>(a.res);
-    Affine<8> aff;
-    half8_t rv[RO];
-    auto residual = [&]() {
-        aff.request(a.norm, cok ? c : 0, !bias_in_sum);
+    Affine<PAIR ? 1 : 8> aff;
+    half8_t rv[RES ? RO : 1];
+    auto residual = [&]() __attribute__((always_inline)) {
+        if constexpr (RES) {
+            const _Float16 *res = static_cast<const _Float16 *>(a.res) + m0 * a.N + (cok ? c : 0);
 #pragma unroll
-        for (int i = 0; i < RO; ++i) {
-            const int64_t m = m0 + tid / CPR + i * (kThreads / CPR);
-            rv[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-            if (res) rv[i] = *reinterpret_cast<const half8_t *>(res + (m < a.M ? m : a.M - 1) * a.N + (cok ? c : 0));
+            for (int i = 0; i < RO; ++i)
+                rv[i] = *reinterpret_cast<const half8_t *>(res + (int64_t)min(r0 + i * STEP, rows - 1) * a.N);
         }
     };
+    // ReLU of rounded results, which a NaN passes: the larger of them and this
+    const _Float16 least = a.relu ? (_Float16)0.f : -(_Float16)__builtin_inff();
     half4_t side[PAIR ? TM : 1][PAIR ? TN : 1][PAIR ? 4 : 1];
     auto affine_of = [&](int which, int i, int j, int g, float (&f)[4]) __attribute__((always_inline)) {
         const float4_t sc = *reinterpret_cast<const float4_t *>(&affine[which][channel(j, g)]);
@@ -323,6 +337,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
         aim(first);
     } else {
+        aff.request(a.norm, cok ? c : 0, !bias_in_sum);
         aim(a);
     }
     auto load_stage = [&](int k, int buf) __attribute__((always_inline)) {
@@ -344,13 +359,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
     }
     int buf = 0;
-    for (int k = 0; k < nk; ++k) {
-        // (stages up to k + ST - 2 have been asked for, the last one is nk - 1)
-        if (k + ST - 1 <= nk) arrive<(ST - 2) * (RX + RW)>();
-        else if (ST == 4 && k + 2 == nk) arrive<RX + RW>();
-        else arrive<0>();
-        if (k + ST - 1 < nk) load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
-        if (!PAIR && k == nk - 1) residual();
+    auto multiply_stage = [&](int k) __attribute__((always_inline)) {
         multiply(buf);
         buf = buf == ST - 1 ? 0 : buf + 1;
         if constexpr (PAIR) {
@@ -369,8 +378,40 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 clear();
             }
         }
+    };
+    // A stage's loads are followed by those of the ST - 2 after it, the last stage's by the
+    // residual's RO, which are asked for a stage earlier than they were and in one go (a branch for
+    // each and a wait between them took a memory latency per tile).  No load moves across arrive().
+    if constexpr (PAIR) {
+        for (int k = 0; k < nk; ++k) {
+            if (k + 1 < nk) arrive<(ST - 2) * (RX + RW)>();
+            else arrive<0>();
+            if (k + ST - 1 < nk) load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+            multiply_stage(k);
+        }
+    } else {
+        int k = 0;
+        for (; k < nk - 2; ++k) {
+            arrive<(ST - 2) * (RX + RW)>();
+            load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+            multiply_stage(k);
+        }
+        if (nk > 1) {
+            arrive<(ST - 2) * (RX + RW)>();
+            if (ST == 2) load_stage(k + 1, buf ^ 1);
+        } else {
+            arrive<0>();
+        }
+        residual();
+        if (nk > 1) {
+            multiply_stage(k);
+            arrive<RES ? RO : 0>();
+        }
+        multiply_stage(nk - 1);
     }
     __syncthreads();
+    float one = 1.f;
+    asm volatile("" : "+v"(one));    // (value * one + f: a conversion less than value + f)
 
     // The tile through LDS as [pixel][channel]: a single product's sums rounded to fp16, a
     // pair's results.
@@ -386,9 +427,11 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                     affine_of(0, i, j, g, f);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        f[e] += (float)side[i][j][g][e];
-                        v[e] = (_Float16)(a.relu ? relu(f[e]) : f[e]);
+                        f[e] = fmaf((float)side[i][j][g][e], one, f[e]);
+                        asm volatile("" : "+v"(f[e]));
+                        v[e] = (_Float16)f[e];
                     }
+                    v = __builtin_elementwise_maximum(v, half4_t{least, least, least, least});
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = (_Float16)acc[i][j][4 * g + e];
@@ -397,36 +440,35 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                 *reinterpret_cast<half4_t *>(net_smem + px * PITCH + channel(j, g)) = v;
             }
     __syncthreads();
-    float sc[8], sh[8];
-    if constexpr (!PAIR) aff.finish(a.norm, sc, sh);
-    _Float16 *out = static_cast<_Float16 *>(a.out);
-    if (!POOL && !cok) return;
-    rows_u4 results[POOL ? RO : 1];
+    half8_t results[RO];
 #pragma unroll
-    for (int i = 0; i < RO; ++i) {
-        const int r = tid / CPR + i * (kThreads / CPR);
-        const int64_t m = m0 + r;
-        if (!POOL && m >= a.M) break;
-        half8_t o = *reinterpret_cast<const half8_t *>(net_smem + r * PITCH + cq * 8);
-        if constexpr (!PAIR) {
+    for (int i = 0; i < RO; ++i)
+        results[i] = *reinterpret_cast<const half8_t *>(net_smem + (r0 + i * STEP) * PITCH + cq * 8);
+    if constexpr (!PAIR) {
+        float sc[8], sh[8];
+        aff.finish(a.norm, sc, sh);
+#pragma unroll
+        for (int i = 0; i < RO; ++i) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float f = fmaf((float)o[e], sc[e], sh[e]) + (float)rv[i][e];
-                if (a.relu) f = relu(f);
-                o[e] = (_Float16)f;
+                float f = fmaf((float)results[i][e], sc[e], sh[e]);
+                if constexpr (RES) f = fmaf((float)rv[i][e], one, f);
+                asm volatile("" : "+v"(f));    // (rounded to fp32 first in every instance)
+                results[i][e] = (_Float16)f;
             }
+            results[i] = __builtin_elementwise_maximum(results[i], half8_t{least, least, least, least, least, least, least, least});
         }
-        if (!POOL || (cok && m < a.M)) *reinterpret_cast<half8_t *>(out + m * a.N + c) = o;
-        if constexpr (POOL) results[i] = __builtin_bit_cast(rows_u4, o);
     }
+    _Float16 *out = static_cast<_Float16 *>(a.out) + (m0 * a.N + (int64_t)r0 * a.N + c);
+#pragma unroll
+    for (int i = 0; i < RO; ++i, out += (int64_t)STEP * a.N)
+        if (cok && r0 + i * STEP < rows) *reinterpret_cast<half8_t *>(out) = results[i];
     if constexpr (POOL) {
         // Sums over the tile's pixels of each sample it touches, to the sample's slot for this
         // tile; the tile with a sample's last pixel clears the slots that sample does not use.
         float *red = reinterpret_cast<float *>(net_smem + BM * PITCH);    // [waves][BN]
         const int first = (int)m0, end = (int)min(m0 + BM, a.M);
         const int n_last = (end - 1) / a.npix;
-        float one = 1.f;
-        asm volatile("" : "+v"(one));    // (value * one + sum: a conversion less than value + sum)
         for (int n = first / a.npix; n <= n_last; ++n) {
             const int lo = n * a.npix - first, hi = lo + a.npix;
             float sum[8];
@@ -435,8 +477,8 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             auto add = [&](auto whole) __attribute__((always_inline)) {
 #pragma unroll
                 for (int i = 0; i < RO; ++i) {
-                    const int r = tid / CPR + i * (kThreads / CPR);
-                    rows_u4 v = results[i];
+                    const int r = r0 + i * STEP;
+                    rows_u4 v = __builtin_bit_cast(rows_u4, results[i]);
                     if (!decltype(whole)::value && (r < lo || r >= hi)) v = rows_u4{0, 0, 0, 0};
                     const half8_t f = __builtin_bit_cast(half8_t, v);
 #pragma unroll
@@ -1113,13 +1155,16 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) < 64 * 1024;
     if (first && !kPair) return hipErrorNotSupported;
     if (first)
-        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
                            *first, tiles_n, (int)tiles);
     else if (a.pool)
-        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, true>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, true, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+                           a, tiles_n, (int)tiles);
+    else if (a.res)
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, false, true>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
                            a, tiles_n, (int)tiles);
     else
-        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
                            a, tiles_n, (int)tiles);
     return hipGetLastError();
 }
