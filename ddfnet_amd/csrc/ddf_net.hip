@@ -831,12 +831,16 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps tap
 // ---- dynamic filter + BatchNorm + ReLU ---------------------------------------------
 // C / 8 lanes own a pixel, eight channels each, and walk along a row: the window slides, so
 // a step loads one new column (three 16-byte vectors; two columns under stride 2), a step
-// ahead of use.  The channel taps of the lane's channels stay in registers, tap-major in
-// pairs of channels; a pixel's nine spatial taps come with it.  comb(CF, SF) of two channels
-// is one packed fp16 operation (rounded like the operands), the sums are fp32: 13 vector
-// instructions per pixel and channel quarter.  WIDE: comb in fp32, 18 instructions - for rows
-// of an odd length, where the operator's own kernels have it so.  A row outside the image, a
-// column past its ends and a walk past the last pixel read zeros through the buffer descriptor.
+// ahead of use.  The channel taps of the lane's channels stay in registers; a pixel's nine spatial
+// taps come with it.  comb(CF, SF) is one packed fp16 operation for two (rounded like the
+// operands), the sums are fp32.  Filter rows 0 and 1 of a channel are a pair, so the two-element
+// dot product takes both (a column's eight words are paired once for the three results it is
+// under); row 2 goes two channels at a time.  With ReLU on rounded pairs a result takes 140 vector
+// instructions where it took 175: 56 x 56 x 64 at batch 128 26.2 -> 25.3 us, 28 x 28 x 128 17.5 ->
+// 16.4; what is left is the latency of a column, at two to three waves per SIMD.  WIDE: comb in
+// fp32 - for rows of an odd length, where the operator's own kernels have it so.  A row outside the
+// image, a column past its ends and a walk past the last pixel read zeros through the buffer
+// descriptor.
 template <bool MUL, bool WIDE>
 __device__ __forceinline__ void filter_pair(half2_t cv, half2_t sv, half2_t xv, float &a0, float &a1) {
     if constexpr (WIDE) {
@@ -856,7 +860,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                                                          const _Float16 *__restrict__ sf, NetNorm norm,
                                                          _Float16 *__restrict__ out, int H, int W, int Ho, int Wo,
                                                          int runs, int run, int units, int blocks, uint32_t x_bytes,
-                                                         uint32_t out_bytes) {
+                                                         uint32_t out_bytes, uint32_t tap_bytes) {
     constexpr int C = LP * 8, SLOTS = kWave / LP, KK = 9;
     const int block = xcd_block(blockIdx.x, blocks);
     if (block >= blocks) return;
@@ -871,13 +875,15 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     const int x1 = live ? min(x0 + run, Wo) : x0;
     // (lanes of a wave may belong to different samples: one descriptor over all of them)
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x, x_bytes);
-    const _Float16 *sn = sf + ((int64_t)n * Ho + y) * Wo * kTapPitch;
+    const __amdgpu_buffer_rsrc_t tr = plane_rsrc(sf, tap_bytes);
+    const uint32_t tap_row = (uint32_t)((n * Ho + y) * Wo) * (kTapPitch * 2);
     const __amdgpu_buffer_rsrc_t orr = plane_rsrc(out, out_bytes);
     const uint32_t oo = (uint32_t)(((n * Ho + y) * Wo) * C + cl * 8) * 2;
 
     Affine<8> aff;
     aff.request(norm, cl * 8);
-    uint32_t cfp[KK][4];
+    // channel taps: of filter rows 0 and 1 as a channel's pair, of row 2 as two channels'
+    uint32_t cfa[3][8], cfb[3][4];
     {
         const uint4 *src = reinterpret_cast<const uint4 *>(cf + ((int64_t)n * C + cl * 8) * KK);
         uint32_t wd[36];
@@ -888,9 +894,12 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
         }
         auto half_at = [&](int i) { return (i & 1) ? wd[i / 2] >> 16 : wd[i / 2] & 0xffffu; };
 #pragma unroll
-        for (int t = 0; t < KK; ++t)
+        for (int j = 0; j < 3; ++j) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) cfp[t][k] = half_at(18 * k + t) | (half_at(18 * k + 9 + t) << 16);
+            for (int e = 0; e < 8; ++e) cfa[j][e] = half_at(9 * e + j) | (half_at(9 * e + 3 + j) << 16);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cfb[j][k] = half_at(18 * k + 6 + j) | (half_at(18 * k + 15 + j) << 16);
+        }
     }
     uint32_t rowo[3];
 #pragma unroll
@@ -906,47 +915,73 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     uint32_t col[RING][3][4], tap[2][6];
     auto column = [&](auto slot, int xx) __attribute__((always_inline)) {
         constexpr int J = decltype(slot)::value % RING;
-        const bool in = xx >= 0 && xx < W;
+        // (a column outside, a row outside or both: past the descriptor's end and short of 2^32)
+        const uint32_t at = (unsigned)xx < (unsigned)W ? (uint32_t)xx * C * 2 : kOutside - 16;
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-            load_words<4>(xr, in && rowo[i] != kOutside ? rowo[i] + (uint32_t)xx * C * 2 : kOutside, col[J][i]);
+        for (int i = 0; i < 3; ++i) load_words<4>(xr, rowo[i] + at, col[J][i]);
     };
     auto taps = [&](auto slot, int xx) __attribute__((always_inline)) {
         constexpr int J = decltype(slot)::value % 2;
-        const uint2 *p = reinterpret_cast<const uint2 *>(sn + (int64_t)min(xx, Wo - 1) * kTapPitch);
+        const uint32_t at = tap_row + (uint32_t)min(xx, Wo - 1) * (kTapPitch * 2);
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            const uint2 q = p[i];
-            tap[J][2 * i] = q.x;
-            tap[J][2 * i + 1] = q.y;
+            uint32_t q[2];
+            load_words<2>(tr, at + i * 8, q);
+            tap[J][2 * i] = q[0];
+            tap[J][2 * i + 1] = q[1];
+        }
+    };
+    // Rows 0 and 1 of a column as a channel's pair each, once for the three results it is under.
+    auto pair_rows = [&](auto slot) __attribute__((always_inline)) {
+        constexpr int J = decltype(slot)::value % RING;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t top = col[J][0][k], low = col[J][1][k];
+            col[J][0][k] = __builtin_amdgcn_perm(low, top, 0x05040100);
+            col[J][1][k] = __builtin_amdgcn_perm(low, top, 0x07060302);
         }
     };
     // result xx from the columns in slots A, A + 1 and A + 2 and the taps in slot J
     auto emit = [&](auto first, auto slot, int xx) __attribute__((always_inline)) {
         constexpr int A = decltype(first)::value, J = decltype(slot)::value % 2;
+        const uint32_t *tp = tap[J];
+        // spatial taps j and 3 + j
+        const uint32_t sa[3] = {__builtin_amdgcn_perm(tp[1], tp[0], 0x07060100), __builtin_amdgcn_perm(tp[2], tp[0], 0x05040302),
+                                __builtin_amdgcn_perm(tp[2], tp[1], 0x07060100)};
         float acc[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = 0.f;
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+        for (int j = 0; j < 3; ++j) {
+            const uint32_t(&at)[3][4] = col[(A + j) % RING];
+            const half2_t sp = __builtin_bit_cast(half2_t, sa[j]);
+            const half2_t sb = __builtin_bit_cast(half2_t, tp[(6 + j) / 2]);
+            const half2_t sv = {sb[j & 1], sb[j & 1]};
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int t = i * 3 + j;
-                const half2_t sp = __builtin_bit_cast(half2_t, tap[J][t / 2]);
-                const half2_t sv = {sp[t & 1], sp[t & 1]};
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, cfp[t][k]), sv,
-                                           __builtin_bit_cast(half2_t, col[(A + j) % RING][i][k]), acc[2 * k], acc[2 * k + 1]);
+            for (int e = 0; e < 8; ++e) {
+                const half2_t xv = __builtin_bit_cast(half2_t, at[e & 1][e / 2]), cv = __builtin_bit_cast(half2_t, cfa[j][e]);
+                if constexpr (WIDE) {
+                    const float c0 = (float)cv[0], c1 = (float)cv[1], s0 = (float)sp[0], s1 = (float)sp[1];
+                    acc[e] = fmaf((float)xv[0], MUL ? c0 * s0 : c0 + s0, acc[e]);
+                    acc[e] = fmaf((float)xv[1], MUL ? c1 * s1 : c1 + s1, acc[e]);
+                } else {
+                    acc[e] = __builtin_amdgcn_fdot2(xv, MUL ? cv * sp : cv + sp, acc[e], false);
                 }
             }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, cfb[j][k]), sv, __builtin_bit_cast(half2_t, at[2][k]),
+                                       acc[2 * k], acc[2 * k + 1]);
+        }
         half8_t o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             // (the complete sum is rounded as the operator's result is)
-            const float f = fmaf((float)(_Float16)acc[e], sc[e], sh[e]);
-            o[e] = (_Float16)relu(f);
+            float f = fmaf((float)(_Float16)acc[e], sc[e], sh[e]);
+            asm volatile("" : "+v"(f));
+            o[e] = (_Float16)f;
         }
+        o = __builtin_elementwise_maximum(o, half8_t{0, 0, 0, 0, 0, 0, 0, 0});
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, o), orr,
                                                (int)(xx < x1 ? oo + (uint32_t)xx * C * 2 : kOutside), 0, 0);
     };
@@ -957,6 +992,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
         column(DDF_I(2), x0 + 1);
         taps(DDF_I(0), x0);
         aff.finish(norm, sc, sh);
+        pair_rows(DDF_I(0));
+        pair_rows(DDF_I(1));
         for (int j = 0; j < run; j += 4) {
             rows::static_for<0, 4>([&](auto q) __attribute__((always_inline)) {
                 constexpr int Q = decltype(q)::value;
@@ -964,6 +1001,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                 column(DDF_I(Q + 3), xx + 2);
                 taps(DDF_I(Q + 1), xx + 1);
                 __builtin_amdgcn_sched_barrier(0);
+                pair_rows(DDF_I(Q + 2));
                 emit(DDF_I(Q), q, xx);
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -975,6 +1013,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
         column(DDF_I(1), 2 * x0 + 1);
         taps(DDF_I(0), x0);
         aff.finish(norm, sc, sh);
+        pair_rows(DDF_I(5));
         for (int j = 0; j < run; j += 6) {
             rows::static_for<0, 6>([&](auto q) __attribute__((always_inline)) {
                 constexpr int Q = decltype(q)::value;
@@ -983,6 +1022,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                 column(DDF_I(2 * Q + 3), 2 * xx + 3);
                 taps(DDF_I(Q + 1), xx + 1);
                 __builtin_amdgcn_sched_barrier(0);
+                pair_rows(DDF_I(2 * Q));
+                pair_rows(DDF_I(2 * Q + 1));
                 emit(DDF_I(2 * Q + 5), q, xx);
                 __builtin_amdgcn_sched_barrier(0);
             });
@@ -997,7 +1038,7 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 // recomputes the hidden vector, every one of a row its spatial taps, and neither goes through
 // memory.  The rows it reads (and zeros around them) come into LDS as [pixel][16 channels] while
 // the channel branch waits for its weights, the spatial taps are computed meanwhile; then a
-// thread takes eight channels of a pixel.  Arithmetic and rounding are k_net_filter's.  us, two
+// thread takes eight channels of a pixel.  Rounding is k_net_filter's.  us, two
 // launches / this: one image 56 x 56 x 64 10.3 / 7.7, 28 x 28 x 128 10.4 / 6.9, 14 x 14 x 256 10.6 /
 // 6.9, 7 x 7 x 512 11.9 / 9.6; most of it is the channel branch's chain and the instructions in front
 // of the first barrier (divisions by runtime values there cost 1 us).
@@ -1360,8 +1401,8 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
     const int step = stride == 1 ? 4 : 6;
     if (C < 8 || C > kWave * 8) return hipErrorNotSupported;
     const int slots = (int)(kWave * 8 / C);
-    // (32-bit offsets: as many samples at a time as stay below 2 GiB)
-    const int64_t sample = H * W * C * 2, most = ((1ll << 31) - 1) / sample;
+    // (32-bit offsets: as many samples at a time as stay below 2 GiB; a pixel is 16 bytes or more)
+    const int64_t sample = H * W * C * 2, most = ((1ll << 31) - 16) / sample;
     if (most < 1) return hipErrorNotSupported;
     for (int64_t n0 = 0; n0 < N; n0 += most) {
         const int64_t cnt = std::min(most, N - n0);
@@ -1388,7 +1429,8 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
 #define DDF_NET_FILTER_LAUNCH(LP_, S_, MUL_, WIDE_)                                                         \
     hipLaunchKernelGGL((k_net_filter<LP_, S_, MUL_, WIDE_>), dim3(xcd_grid(blocks)), dim3(kThreads), 0, st, \
                        xn, cn, sn, norm, on, (int)H, (int)W, (int)Ho, (int)Wo, (int)runs, run, (int)units,  \
-                       (int)blocks, (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2))
+                       (int)blocks, (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2),        \
+                       (uint32_t)(cnt * Ho * Wo * kTapPitch * 2))
 #define DDF_NET_FILTER(LP_, S_)                                     \
     if (C == LP_ * 8 && stride == S_) {                             \
         if (wide && mul) DDF_NET_FILTER_LAUNCH(LP_, S_, true, true); \
