@@ -556,6 +556,177 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     }
 }
 
+// Spatial branch of fp16 planes on the matrix cores, 3 x 3 taps, stride 1: the taps are a product
+// of nine weight rows with the pixels' channels.  A wave owns 16 * VP neighbouring pixels, its lane
+// (l & 15) VP of them, and its quarter (l >> 4) of the lanes eight of 32 channels: eight loads
+// of a vector of pixels, which pairs of channels turn into VP operands of 16 pixels x 32 channels
+// in the order that the 16x16x32 step wants (VP / 2 * 8 permutes; the product itself is VP
+// steps).  Pixel e of every lane is column l & 15 of result e, taps 4 * quarter + 0..3 in its four
+// registers, so a pixel's nine taps are spread over three quarters, which meet in the
+// normalisation; a tap's VP pixels lie in one lane and leave as a vector.  A workgroup is four such
+// waves next to each other, their sums over the pixels (see k_spatial_stream) meet in LDS.
+// k_spatial_stream spends nine dot products on a pixel's pair of channels, 1230 vector
+// instructions per 128 pixels of 64 channels, where this takes half of it and memory is what bounds
+// it: 8 x 64 x 200 x 300 in 17.4 us, 13.5 at copy rate (the line in the dispatch has the sizes).
+typedef uint32_t rows_u4 __attribute__((ext_vector_type(4)));
+constexpr int kSpatialMmaWaves = 4, kSpatialMmaStages = 2, kSpatialMmaChannels = 2048;
+
+template <int VP, bool POOL>
+__global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 3 : 4) void k_spatial_mma(
+    SpatialGeom g, const __half *__restrict__ x, const __half *__restrict__ w, const __half *__restrict__ bias,
+    __half *__restrict__ sf, float gain, const __half *__restrict__ gain_vec, const __half *__restrict__ offset_vec,
+    float *__restrict__ pool_part, __half *__restrict__ raw) {
+    constexpr int KK = 9, NST = kSpatialMmaStages, NW = VP / 2, kVB = VP * 2;
+    extern __shared__ __align__(16) float pool_sums[];             // [waves][C]
+    const int lane = threadIdx.x & (kWave - 1), col = lane & 15, quarter = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int head = blockIdx.y, heads = gridDim.y;
+    const int64_t n = blockIdx.z;
+    const int v = (blockIdx.x * kSpatialMmaWaves + wave) * 16 + col;
+    const bool live = v < g.nvec;
+    const uint32_t plane_bytes = (uint32_t)g.plane * 2u;
+    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + n * g.C * (int64_t)g.plane, (uint32_t)g.C * plane_bytes);
+    const uint32_t xb = live ? (uint32_t)v * kVB + (uint32_t)(quarter * 8) * plane_bytes : kOutside;
+    const __amdgpu_buffer_rsrc_t wr = plane_rsrc(w + (int64_t)head * KK * g.C, (uint32_t)(KK * g.C) * 2u);
+    const uint32_t wb = col < KK ? (uint32_t)(col * g.C + quarter * 8) * 2u : kOutside;
+
+    uint32_t xw[NST][8][NW], ww[NST][4];
+    auto issue = [&](auto st_tag, int i) __attribute__((always_inline)) {
+        constexpr int ST = decltype(st_tag)::value;
+        const bool have = i < g.ngroups;
+        const uint32_t at = have ? xb : kOutside, cb = (uint32_t)(have ? i * 32 : 0) * plane_bytes;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if constexpr (VP == 8) {
+                const auto q = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)at, (int)(cb + (uint32_t)u * plane_bytes), 0);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) xw[ST][u][k] = q[k];
+            } else {
+                const auto q = __builtin_amdgcn_raw_buffer_load_b64(xr, (int)at, (int)(cb + (uint32_t)u * plane_bytes), 0);
+                xw[ST][u][0] = q[0];
+                xw[ST][u][1] = q[1];
+            }
+        }
+        rows::load_words<4>(wr, have ? wb + (uint32_t)i * 64u : kOutside, ww[ST]);
+    };
+    float4_t acc[VP];
+#pragma unroll
+    for (int e = 0; e < VP; ++e) acc[e] = float4_t{0.f, 0.f, 0.f, 0.f};
+    float *const sums = pool_sums + wave * g.C + quarter * 8 + (lane & 3);
+    auto compute = [&](auto st_tag, int i) __attribute__((always_inline)) {
+        constexpr int ST = decltype(st_tag)::value;
+        if constexpr (POOL) {
+            if (head == 0) {
+                const rows::half2_t ones = {(_Float16)1, (_Float16)1};
+                float ps[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    float part[NW];
+#pragma unroll
+                    for (int k = 0; k < NW; ++k)
+                        part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, xw[ST][u][k]), ones, 0.f, false);
+                    ps[u] = NW == 4 ? (part[0] + part[1]) + (part[NW - 2] + part[NW - 1]) : part[0] + part[1];
+                }
+                // over the row of sixteen lanes: channel 4 * h + (lane & 3) in each (see wave_sums)
+                const bool b0 = lane & 1, b1 = lane & 2;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float *q = ps + 4 * h;
+                    const float k0 = (b0 ? q[1] : q[0]) + from_permuted<0xB1>(b0 ? q[0] : q[1]);
+                    const float k1 = (b0 ? q[3] : q[2]) + from_permuted<0xB1>(b0 ? q[2] : q[3]);
+                    float k = (b1 ? k1 : k0) + from_permuted<0x4E>(b1 ? k0 : k1);
+                    k += from_permuted<0x124 /* row_ror:4 */>(k);
+                    k += from_permuted<0x128 /* row_ror:8 */>(k);
+                    if (col < 4) sums[i * 32 + 4 * h] = k;
+                }
+            }
+        }
+        const half8_t wv = __builtin_bit_cast(half8_t, rows_u4{ww[ST][0], ww[ST][1], ww[ST][2], ww[ST][3]});
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            rows_u4 low, high;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                low[c] = __builtin_amdgcn_perm(xw[ST][2 * c + 1][k], xw[ST][2 * c][k], 0x05040100u);
+                high[c] = __builtin_amdgcn_perm(xw[ST][2 * c + 1][k], xw[ST][2 * c][k], 0x07060302u);
+            }
+            acc[2 * k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, __builtin_bit_cast(half8_t, low), acc[2 * k], 0, 0, 0);
+            acc[2 * k + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, __builtin_bit_cast(half8_t, high), acc[2 * k + 1], 0, 0, 0);
+        }
+    };
+    issue(std::integral_constant<int, 0>{}, 0);
+    // this lane's four taps
+    float gains[4], offsets[4], biases[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int t = quarter * 4 + r;
+        const int at = head * KK + min(t, KK - 1);
+        gains[r] = gain_vec ? ld(gain_vec + at) : gain;
+        offsets[r] = offset_vec ? ld(offset_vec + at) : 0.f;
+        biases[r] = bias && t < KK ? ld(bias + at) : 0.f;
+    }
+    for (int i = 0; i < g.ngroups; i += 2) {
+        issue(std::integral_constant<int, 1>{}, i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(std::integral_constant<int, 0>{}, i);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 1 >= g.ngroups) break;
+        issue(std::integral_constant<int, 0>{}, i + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(std::integral_constant<int, 1>{}, i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    const int64_t taps_at = ((n * heads + head) * KK) * (int64_t)g.npix;
+    const uint32_t tap_bytes = (uint32_t)g.npix * 2u, all_bytes = KK * tap_bytes;
+    uint32_t ob[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int t = quarter * 4 + r;
+        ob[r] = live && t < KK ? (uint32_t)v * kVB + (uint32_t)t * tap_bytes : kOutside;
+    }
+    // (taps past the ninth: zero weights, zero bias)
+#pragma unroll
+    for (int e = 0; e < VP; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[e][r] += biases[r];
+    auto leave = [&](__half *to) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rr = plane_rsrc(to + taps_at, all_bytes);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float f[VP];
+#pragma unroll
+            for (int e = 0; e < VP; ++e) f[e] = acc[e][r];
+            uint32_t ow[NW];
+            rows::pack<__half, VP, float>(f, ow);
+            store_vec_nt<kVB>(rr, ob[r], ow);
+        }
+    };
+    if (raw) leave(raw);
+    // as normalise() has it, the sums over the taps across the quarters
+#pragma unroll
+    for (int e = 0; e < VP; ++e) {
+        const float mean = rows_total((acc[e][0] + acc[e][1]) + (acc[e][2] + acc[e][3])) / (float)KK;
+        float sq = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            acc[e][r] -= mean;
+            if (quarter * 4 + r < KK) sq += acc[e][r] * acc[e][r];
+        }
+        const float inv = 1.f / (sqrtf(rows_total(sq) / (float)(KK - 1)) + 1e-10f);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[e][r] = acc[e][r] * inv * gains[r] + offsets[r];
+    }
+    leave(sf);
+    if constexpr (POOL) {
+        if (head != 0) return;
+        __syncthreads();
+        float *out = pool_part + (n * gridDim.x + blockIdx.x) * g.C;
+        for (int c = threadIdx.x; c < g.C; c += kSpatialMmaWaves * kWave)
+            out[c] = (pool_sums[c] + pool_sums[g.C + c]) + (pool_sums[2 * g.C + c] + pool_sums[3 * g.C + c]);
+    }
+}
+
 // out[n * C + c] = sum of parts[(n * nparts + p) * C + c] over p.  Every workgroup of the
 // channel branch starts from the pooled vectors; with dozens of partial sums per value each
 // of them would spend longer adding up than on its own work (8 x 64 x 200 x 300 fp16: 472
@@ -785,6 +956,28 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     const int fvp = tune_int("DDF_TUNE_SPATIAL_VP", 0), fwv = tune_int("DDF_TUNE_SPATIAL_WAVES", 0);
     if (fvp > 0 && fvp <= vp_max && fits(fvp)) vp = fvp;
     if (fwv > 0) waves = fwv;
+    // fp16, stride 1: on the matrix cores where vectors of eight pixels make a workgroup per CU, or
+    // of four a quarter of that (up to 256 channels, whose walk is eight steps).  Eight from 64
+    // workgroups on where four leave more partial sums than the channel branch takes.  us with the
+    // pooled sums, k_spatial_stream (and k_collapse_parts) / here: 8 x 64 x 200 x 300 21.0 / 17.4,
+    // 1 x 64 x 200 x 300 11.6 / 6.3, 8 x 256 x 50 x 76 11.1 / 7.9, 16 x 64 x 56 x 56 9.4 / 5.0,
+    // 64 x 128 x 28 x 28 7.9 / 6.5, 32 x 256 x 28 x 28 8.1 / 7.7, 6 x 160 x 44 x 46 9.1 / 6.5;
+    // 24 x 512 x 28 x 28 10.9 / 11.1 in 96 workgroups, 1 x 96 x 80 x 96 8.0 / 8.1 in 30.
+    bool mma = false;
+    if constexpr (esz == 2) {
+        if (stride == 1 && C % 32 == 0 && C <= kSpatialMmaChannels && (uintptr_t)w % 16 == 0 &&
+            tune_int("DDF_TUNE_SPATIAL_MMA", 1) != 0) {
+            const int64_t tiles8 = cdiv(npix / 8, kWave), tiles4 = cdiv(npix / 4, kWave), left = channel_parts_left(N, C);
+            const bool narrow = fits(4) && tiles4 * N * head >= (C <= 256 ? 64 : 256);
+            const bool wide = fits(8) && (tiles8 * N * head >= 256 ||
+                                          (narrow && pool && tiles4 > left && tiles8 <= left && tiles8 * N * head >= 64));
+            if (wide || narrow) {
+                mma = true;
+                vp = wide ? 8 : 4;
+                waves = 1;
+            }
+        }
+    }
     if (vp == 0) return hipErrorNotSupported;
     if (vp * waves > 32 || (waves & (waves - 1)) != 0 || waves > 16) return hipErrorNotSupported;   // (the variants built)
     SpatialGeom g;
@@ -794,7 +987,7 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     g.nvec = (int)(npix / vp);
     const int tiles = (int)cdiv(g.nvec, kWave);
     g.lpt = (int)cdiv(g.nvec, tiles);                   // (tiles of equal size)
-    g.ngroups = (int)(C / U);
+    g.ngroups = (int)(mma ? C / 32 : C / U);
     g.gpw = (int)cdiv(g.ngroups, waves);
     g.steps = (int)cdiv(g.gpw, NST) * NST;
     if (N > 65535 || head > 65535) return hipErrorNotSupported;
@@ -808,6 +1001,23 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     }
     float *parts_out = collapse ? pool_part + N * C : pool_part;
     const dim3 grid((unsigned)tiles, (unsigned)head, (unsigned)N);
+    if constexpr (esz == 2) {
+        if (mma) {
+            const int lds = pool ? kSpatialMmaWaves * g.C * (int)sizeof(float) : 0;
+#define DDF_SPATIAL_MMA(VP_, POOL_)                                                               \
+    hipLaunchKernelGGL((k_spatial_mma<VP_, POOL_>), grid, dim3(kSpatialMmaWaves * kWave), lds, st, g, x, w, bias, sf, \
+                       (float)gain, gain_vec, offset_vec, parts_out, raw)
+            if (vp == 8 && pool) DDF_SPATIAL_MMA(8, true);
+            else if (vp == 8) DDF_SPATIAL_MMA(8, false);
+            else if (pool) DDF_SPATIAL_MMA(4, true);
+            else DDF_SPATIAL_MMA(4, false);
+#undef DDF_SPATIAL_MMA
+            if (collapse)
+                hipLaunchKernelGGL(k_collapse_parts, dim3((unsigned)cdiv(C, kCollapseChannels), (unsigned)N),
+                                   dim3(kCollapseChannels * kCollapseGroups), 0, st, parts_out, pool_part, (int)C, tiles);
+            return hipGetLastError();
+        }
+    }
 #define DDF_STREAM_LAUNCH(VP_, S_, WAVES_)                                                        \
     do {                                                                                          \
         if (pool) {                                                                               \

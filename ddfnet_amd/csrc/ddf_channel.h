@@ -163,6 +163,14 @@ typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
+// Sum over the wave's four rows of sixteen lanes (the same value in every lane of a column).
+__device__ __forceinline__ float rows_total(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+}
+
 // 16 bytes per lane to LDS at `lds` + lane * 16.  (Written out because the compiler waits for
 // every such load in flight before any LDS read.  The address is an operand in m0, so that the
 // compiler itself writes m0 and knows it; the load must not follow that write at once.)

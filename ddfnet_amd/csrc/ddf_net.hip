@@ -79,14 +79,6 @@ struct Affine {
     }
 };
 
-// Sum over the wave's four rows of sixteen lanes (the same value in every lane of a column).
-__device__ __forceinline__ float rows_total(float v) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
-}
-
 template <int CTRL>
 __device__ __forceinline__ float add_permuted(float x) {
     return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));

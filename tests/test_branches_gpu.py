@@ -186,6 +186,37 @@ def test_spatial_branch_pool(case, dtype):
     assert ((parts.double().sum(1).cpu() - sums).abs().max() / scale).item() < 1e-6
 
 
+# vectors of four and of eight pixels, whole and partly filled tiles, odd and even numbers of
+# 32-channel groups, several heads
+MMA_CASES = [(11, 32, 40, 44, 1), (70, 64, 8, 13, 1), (3, 96, 60, 100, 3), (40, 320, 36, 52, 1), (34, 256, 33, 64, 1),
+             (2, 64, 240, 300, 1), (1, 64, 200, 300, 1)]
+
+
+@pytest.mark.parametrize('vectors', [False, True])
+@pytest.mark.parametrize('case', MMA_CASES, ids=lambda c: 'x'.join(map(str, c)))
+def test_spatial_branch_on_the_matrix_cores(case, vectors):
+    n, c, h, w_, head = case
+    torch.manual_seed(c + h)
+    x = torch.randn(n, c, h, w_, device='cuda').half()
+    w = (torch.randn(head * 9, c, device='cuda') * 0.2).half()
+    b, gv, ov = (torch.randn(3, head * 9, device='cuda').half() if vectors else (None, None, None))
+    sf, parts = _lib.spatial_branch_pool(x, w, b, head, 3, 1, 0.7, gv, ov)
+    assert torch.equal(sf, _lib.spatial_branch(x, w, b, head, 3, 1, 0.7, gv, ov))
+    ref = spatial_reference(*(None if t is None else t.cpu() for t in (x, w, b)), head, 3, 1, 0.7,
+                            None if gv is None else gv.cpu(), None if ov is None else ov.cpu())
+    assert ((sf.double().cpu() - ref).abs().max() / ref.abs().max()).item() < 4e-3
+    sums, scale = x.double().sum((2, 3)), x.double().abs().sum((2, 3)).max()
+    assert ((parts.double().sum(1) - sums).abs().max() / scale).item() < 1e-6
+    # what is not finite stays with its pixel and its channel
+    x[0, 5, h - 1, w_ - 1] = float('inf')
+    sf2, parts2 = _lib.spatial_branch_pool(x, w, b, head, 3, 1, 0.7, gv, ov)
+    last = sf2.reshape(n, head * 9, -1)[0, :, -1]
+    assert torch.isnan(last).all()
+    sf2.reshape(n, head * 9, -1)[0, :, -1] = sf.reshape(n, head * 9, -1)[0, :, -1]
+    assert torch.equal(sf2, sf)
+    assert torch.isinf(parts2[0, :, 5].sum()) and torch.isfinite(parts2.sum(1)).sum().item() == n * c - 1
+
+
 def test_spatial_branch_pool_turns_down_what_it_cannot_cover():
     x = torch.randn(2, 16, 9, 8, device='cuda')
     w5 = torch.randn(25, 16, device='cuda')
