@@ -504,23 +504,27 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     }
 
     if constexpr (WAVES > 1) {
-        // the other waves' sums reach wave 0 through LDS, [wave][tap][lane][pixel]
+        // The waves' sums meet in LDS, [slot][tap][lane][pixel], half of the waves handing theirs to
+        // the other half at a time (each round has slots of its own, so one barrier will do):
+        // wave 0 alone adding up fifteen others waited for LDS fifteen times.
         __shared__ __align__(16) float red[WAVES - 1][KK][kWave][VP];
-        if (wave > 0) {
+        rows::static_for<0, WAVES == 2 ? 1 : WAVES == 4 ? 2 : WAVES == 8 ? 3 : 4>([&](auto round) __attribute__((always_inline)) {
+            constexpr int HALF = WAVES >> (decltype(round)::value + 1), FIRST = WAVES - 2 * HALF;
+            if (wave >= HALF && wave < 2 * HALF) {
 #pragma unroll
-            for (int t = 0; t < KK; ++t)
+                for (int t = 0; t < KK; ++t)
 #pragma unroll
-                for (int k = 0; k < VP; ++k) red[wave - 1][t][lane][k] = acc[t][k];
-        }
-        __syncthreads();
+                    for (int k = 0; k < VP; ++k) red[FIRST + wave - HALF][t][lane][k] = acc[t][k];
+            }
+            __syncthreads();
+            if (wave < HALF) {
+#pragma unroll
+                for (int t = 0; t < KK; ++t)
+#pragma unroll
+                    for (int k = 0; k < VP; ++k) acc[t][k] += red[FIRST + wave][t][lane][k];
+            }
+        });
         if (wave > 0) return;
-        // (one wave's sums at a time: unrolled, all of them would be in registers at once)
-#pragma unroll 1
-        for (int q = 0; q < WAVES - 1; ++q)
-#pragma unroll
-            for (int t = 0; t < KK; ++t)
-#pragma unroll
-                for (int k = 0; k < VP; ++k) acc[t][k] += red[q][t][lane][k];
     }
     TapParams<T, KK> params;
     params.load(head, gain, gain_vec, offset_vec, bias);
