@@ -555,16 +555,22 @@ __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tile
     aff.request(a.norm, oc < a.N ? oc : 0);
     const _Float16 rv = res ? res[ok ? om * a.N + oc : 0] : (_Float16)0;
     float4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int b = b0; b < b1; b += D) {
+    auto multiply = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[d][u], xv[d][u], acc, 0, 0, 0);
+    };
+    // (the last round asks for nothing: its loads would be as many again as K = 1024 has)
+    int b = b0;
+    for (; b + D < b1; b += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            if (b + d < b1) {
-#pragma unroll
-                for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[d][u], xv[d][u], acc, 0, 0, 0);
-            }
+            multiply(d);
             request(d, b + d + D);
         }
     }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (b + d < b1) multiply(d);
 #pragma unroll
     for (int e = 0; e < 4; ++e) red[wave][4 * quad + e][col] = acc[e];
     __syncthreads();
@@ -1216,8 +1222,9 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
 }
 
 // Rows of whole vectors, unless K is long and 16 x 16 results make a workgroup per compute unit
-// at most (us in tiles of 64 / split: 98 x 2048 -> 512, 224 workgroups, 11.7 / 7.4; 196 x 1024 -> 256,
-// 208, 7.4 / 5.7; 392 x 1024 -> 256, 400, 7.4 / 9.2; 128 x 2048 -> 1000, 504, 11.9 / 12.8).
+// at most (us in tiles of 64 / split: 392 x 1024 -> 256, 400 workgroups, 6.1 / 6.1; 392 x 512 -> 256,
+// 400, 4.5 / 5.8; 784 x 1024 -> 256, 784, 6.4 / 9.4; split below that, 196 x 1024 -> 256, 208, takes
+// 4.2 and 98 x 2048 -> 512, 224, 6.1).
 bool conv_in_tiles(const NetConv &a) {
     return a.N % 8 == 0 && !(a.K >= 512 && cdiv(a.M, 16) * cdiv(a.N, 16) <= 256);
 }
