@@ -118,6 +118,26 @@ def test_stem(n, h, w):
     close(out, want, 3e-3)
 
 
+def test_stem_takes_images_at_any_address_and_keeps_what_is_not_finite_local():
+    """Pairs of columns from an odd element on; the window's idle column holds an infinity."""
+    torch.manual_seed(0)
+    x = torch.randn(2, 3, 36, 44, device='cuda').half()
+    wt = (torch.randn(64, 3, 7, 7, device='cuda') * 0.1).half()
+    norm, apply, keep = make_norm(64, 1, 1)
+    out, odd_out = (torch.empty(2, 9, 11, 64, device='cuda', dtype=torch.float16) for _ in range(2))
+    call('ddf_hip_net_stem', x, wt, norm, out, 2, 36, 44)
+    odd = torch.empty(x.numel() + 1, device='cuda', dtype=torch.float16)[1:].view(x.shape).copy_(x)
+    call('ddf_hip_net_stem', odd, wt, norm, odd_out, 2, 36, 44)
+    assert torch.equal(odd_out, out)
+    x[0, 1, 17, 20] = float('inf')     # under the convolution results of columns 9 .. 11
+    reached = torch.zeros(2, 1, 36, 44)
+    reached[0, 0, 17, 20] = 1
+    reached = F.max_pool2d(F.max_pool2d(F.pad(reached, (3, 3, 3, 3)), 7, 2), 3, 2, 1)[:, 0] > 0
+    call('ddf_hip_net_stem', x, wt, norm, odd_out, 2, 36, 44)
+    same = (odd_out == out).all(-1).cpu()
+    assert same[~reached].all() and not same[reached].any()
+
+
 @pytest.mark.parametrize('combine', ['mul', 'add'])
 @pytest.mark.parametrize('n,h,w,c,s', [(2, 56, 56, 64, 1), (1, 2, 2, 512, 1), (3, 7, 7, 512, 1), (5, 9, 13, 128, 1),
                                        (2, 14, 14, 256, 1), (2, 4, 6, 256, 2), (1, 28, 28, 128, 2), (3, 14, 14, 512, 2),
