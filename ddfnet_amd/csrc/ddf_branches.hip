@@ -562,25 +562,25 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
 
 // Spatial branch of fp16 planes on the matrix cores, 3 x 3 taps, stride 1: the taps are a product
 // of nine weight rows with the pixels' channels.  A wave owns 16 * VP neighbouring pixels, its lane
-// (l & 15) VP of them, and its quarter (l >> 4) of the lanes eight of 32 channels: eight loads
-// of a vector of pixels, which pairs of channels turn into VP operands of 16 pixels x 32 channels
-// in the order that the 16x16x32 step wants (VP / 2 * 8 permutes; the product itself is VP
-// steps).  Pixel e of every lane is column l & 15 of result e, taps 4 * quarter + 0..3 in its four
-// registers, so a pixel's nine taps are spread over three quarters, which meet in the
-// normalisation; a tap's VP pixels lie in one lane and leave as a vector.  A workgroup is four such
-// waves next to each other, their sums over the pixels (see k_spatial_stream) meet in LDS.
+// (l & 15) VP of them, and its quarter (l >> 4) of the lanes four of 16 channels: four loads of a
+// vector of pixels, which pairs of channels turn into VP operands of 16 pixels x 16 channels in the
+// order that the 16x16x16 step wants (4 * VP / 2 permutes; the product itself is VP steps).  Pixel e
+// of every lane is column l & 15 of result e, taps 4 * quarter + 0..3 in its four registers, so a
+// pixel's nine taps are spread over three quarters, which meet in the normalisation; a tap's VP
+// pixels lie in one lane and leave as a vector.  A workgroup is four such waves next to each other,
+// their sums over the pixels (see k_spatial_stream) meet in LDS.
 // k_spatial_stream spends nine dot products on a pixel's pair of channels, 1230 vector
 // instructions per 128 pixels of 64 channels, where this takes half of it and memory is what bounds
-// it: 8 x 64 x 200 x 300 in 17.4 us, 13.5 at copy rate (the line in the dispatch has the sizes).
-typedef uint32_t rows_u4 __attribute__((ext_vector_type(4)));
-constexpr int kSpatialMmaWaves = 4, kSpatialMmaStages = 2, kSpatialMmaChannels = 2048;
+// it: 8 x 64 x 200 x 300 in 16.4 us, 13.5 at copy rate.  Groups of 32 channels (the 16x16x32 step)
+// took 155 registers, three waves per SIMD and 17.4 us; three groups of 16 in flight 19.0.
+constexpr int kSpatialMmaWaves = 4, kSpatialMmaStages = 2, kSpatialMmaGroup = 16, kSpatialMmaChannels = 2048;
 
 template <int VP, bool POOL>
-__global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 3 : 4) void k_spatial_mma(
+__global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_spatial_mma(
     SpatialGeom g, const __half *__restrict__ x, const __half *__restrict__ w, const __half *__restrict__ bias,
     __half *__restrict__ sf, float gain, const __half *__restrict__ gain_vec, const __half *__restrict__ offset_vec,
     float *__restrict__ pool_part, __half *__restrict__ raw) {
-    constexpr int KK = 9, NST = kSpatialMmaStages, NW = VP / 2, kVB = VP * 2;
+    constexpr int KK = 9, NST = kSpatialMmaStages, G = kSpatialMmaGroup, NW = VP / 2, kVB = VP * 2;
     extern __shared__ __align__(16) float pool_sums[];             // [waves][C]
     const int lane = threadIdx.x & (kWave - 1), col = lane & 15, quarter = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -590,17 +590,17 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 3 : 4) void k_s
     const bool live = v < g.nvec;
     const uint32_t plane_bytes = (uint32_t)g.plane * 2u;
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + n * g.C * (int64_t)g.plane, (uint32_t)g.C * plane_bytes);
-    const uint32_t xb = live ? (uint32_t)v * kVB + (uint32_t)(quarter * 8) * plane_bytes : kOutside;
+    const uint32_t xb = live ? (uint32_t)v * kVB + (uint32_t)(quarter * 4) * plane_bytes : kOutside;
     const __amdgpu_buffer_rsrc_t wr = plane_rsrc(w + (int64_t)head * KK * g.C, (uint32_t)(KK * g.C) * 2u);
-    const uint32_t wb = col < KK ? (uint32_t)(col * g.C + quarter * 8) * 2u : kOutside;
+    const uint32_t wb = col < KK ? (uint32_t)(col * g.C + quarter * 4) * 2u : kOutside;
 
-    uint32_t xw[NST][8][NW], ww[NST][4];
+    uint32_t xw[NST][4][NW], ww[NST][2];
     auto issue = [&](auto st_tag, int i) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_tag)::value;
         const bool have = i < g.ngroups;
-        const uint32_t at = have ? xb : kOutside, cb = (uint32_t)(have ? i * 32 : 0) * plane_bytes;
+        const uint32_t at = have ? xb : kOutside, cb = (uint32_t)(have ? i * G : 0) * plane_bytes;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < 4; ++u) {
             if constexpr (VP == 8) {
                 const auto q = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)at, (int)(cb + (uint32_t)u * plane_bytes), 0);
 #pragma unroll
@@ -611,75 +611,69 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 3 : 4) void k_s
                 xw[ST][u][1] = q[1];
             }
         }
-        rows::load_words<4>(wr, have ? wb + (uint32_t)i * 64u : kOutside, ww[ST]);
+        rows::load_words<2>(wr, have ? wb + (uint32_t)i * (G * 2u) : kOutside, ww[ST]);
     };
     float4_t acc[VP];
 #pragma unroll
     for (int e = 0; e < VP; ++e) acc[e] = float4_t{0.f, 0.f, 0.f, 0.f};
-    float *const sums = pool_sums + wave * g.C + quarter * 8 + (lane & 3);
+    float *const sums = pool_sums + wave * g.C + quarter * 4 + (lane & 3);
     auto compute = [&](auto st_tag, int i) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_tag)::value;
         if constexpr (POOL) {
             if (head == 0) {
                 const rows::half2_t ones = {(_Float16)1, (_Float16)1};
-                float ps[8];
+                float ps[4];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
+                for (int u = 0; u < 4; ++u) {
                     float part[NW];
 #pragma unroll
                     for (int k = 0; k < NW; ++k)
                         part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, xw[ST][u][k]), ones, 0.f, false);
                     ps[u] = NW == 4 ? (part[0] + part[1]) + (part[NW - 2] + part[NW - 1]) : part[0] + part[1];
                 }
-                // over the row of sixteen lanes: channel 4 * h + (lane & 3) in each (see wave_sums)
+                // over the row of sixteen lanes: channel (lane & 3) in each (see wave_sums)
                 const bool b0 = lane & 1, b1 = lane & 2;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float *q = ps + 4 * h;
-                    const float k0 = (b0 ? q[1] : q[0]) + from_permuted<0xB1>(b0 ? q[0] : q[1]);
-                    const float k1 = (b0 ? q[3] : q[2]) + from_permuted<0xB1>(b0 ? q[2] : q[3]);
-                    float k = (b1 ? k1 : k0) + from_permuted<0x4E>(b1 ? k0 : k1);
-                    k += from_permuted<0x124 /* row_ror:4 */>(k);
-                    k += from_permuted<0x128 /* row_ror:8 */>(k);
-                    if (col < 4) sums[i * 32 + 4 * h] = k;
-                }
+                const float k0 = (b0 ? ps[1] : ps[0]) + from_permuted<0xB1>(b0 ? ps[0] : ps[1]);
+                const float k1 = (b0 ? ps[3] : ps[2]) + from_permuted<0xB1>(b0 ? ps[2] : ps[3]);
+                float k = (b1 ? k1 : k0) + from_permuted<0x4E>(b1 ? k0 : k1);
+                k += from_permuted<0x124 /* row_ror:4 */>(k);
+                k += from_permuted<0x128 /* row_ror:8 */>(k);
+                if (col < 4 && i < g.ngroups) sums[i * G] = k;
             }
         }
-        const half8_t wv = __builtin_bit_cast(half8_t, rows_u4{ww[ST][0], ww[ST][1], ww[ST][2], ww[ST][3]});
+        typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
+        const half4_t wv = __builtin_bit_cast(half4_t, pair_t{ww[ST][0], ww[ST][1]});
 #pragma unroll
         for (int k = 0; k < NW; ++k) {
-            rows_u4 low, high;
+            pair_t low, high;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < 2; ++c) {
                 low[c] = __builtin_amdgcn_perm(xw[ST][2 * c + 1][k], xw[ST][2 * c][k], 0x05040100u);
                 high[c] = __builtin_amdgcn_perm(xw[ST][2 * c + 1][k], xw[ST][2 * c][k], 0x07060302u);
             }
-            acc[2 * k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, __builtin_bit_cast(half8_t, low), acc[2 * k], 0, 0, 0);
-            acc[2 * k + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, __builtin_bit_cast(half8_t, high), acc[2 * k + 1], 0, 0, 0);
+            acc[2 * k] = __builtin_amdgcn_mfma_f32_16x16x16f16(wv, __builtin_bit_cast(half4_t, low), acc[2 * k], 0, 0, 0);
+            acc[2 * k + 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(wv, __builtin_bit_cast(half4_t, high), acc[2 * k + 1], 0, 0, 0);
         }
     };
-    issue(std::integral_constant<int, 0>{}, 0);
-    // this lane's four taps
-    float gains[4], offsets[4], biases[4];
+    rows::static_for<0, NST - 1>([&](auto q) __attribute__((always_inline)) { issue(q, decltype(q)::value); });
+    // this lane's four taps, as stored: they wait for the end of the walk
+    _Float16 taps_of[3][4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int t = quarter * 4 + r;
-        const int at = head * KK + min(t, KK - 1);
-        gains[r] = gain_vec ? ld(gain_vec + at) : gain;
-        offsets[r] = offset_vec ? ld(offset_vec + at) : 0.f;
-        biases[r] = bias && t < KK ? ld(bias + at) : 0.f;
+        const int at = head * KK + min(quarter * 4 + r, KK - 1);
+        taps_of[0][r] = gain_vec ? *reinterpret_cast<const _Float16 *>(gain_vec + at) : (_Float16)0;
+        taps_of[1][r] = offset_vec ? *reinterpret_cast<const _Float16 *>(offset_vec + at) : (_Float16)0;
+        taps_of[2][r] = bias ? *reinterpret_cast<const _Float16 *>(bias + at) : (_Float16)0;
     }
-    for (int i = 0; i < g.ngroups; i += 2) {
-        issue(std::integral_constant<int, 1>{}, i + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(std::integral_constant<int, 0>{}, i);
-        __builtin_amdgcn_sched_barrier(0);
-        if (i + 1 >= g.ngroups) break;
-        issue(std::integral_constant<int, 0>{}, i + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(std::integral_constant<int, 1>{}, i + 1);
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    // (whole rounds: a group past the last one reads zeros)
+    for (int i = 0; i < g.ngroups; i += NST)
+        rows::static_for<0, NST>([&](auto q) __attribute__((always_inline)) {
+            constexpr int Q = decltype(q)::value;
+            issue(std::integral_constant<int, (Q + NST - 1) % NST>{}, i + Q + NST - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(q, i + Q);
+            __builtin_amdgcn_sched_barrier(0);
+        });
 
     const int64_t taps_at = ((n * heads + head) * KK) * (int64_t)g.npix;
     const uint32_t tap_bytes = (uint32_t)g.npix * 2u, all_bytes = KK * tap_bytes;
@@ -690,10 +684,15 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 3 : 4) void k_s
         ob[r] = live && t < KK ? (uint32_t)v * kVB + (uint32_t)t * tap_bytes : kOutside;
     }
     // (taps past the ninth: zero weights, zero bias)
+    float gains[4], offsets[4];
 #pragma unroll
-    for (int e = 0; e < VP; ++e)
+    for (int r = 0; r < 4; ++r) {
+        gains[r] = gain_vec ? (float)taps_of[0][r] : gain;
+        offsets[r] = (float)taps_of[1][r];
+        const float b = quarter * 4 + r < KK ? (float)taps_of[2][r] : 0.f;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[e][r] += biases[r];
+        for (int e = 0; e < VP; ++e) acc[e][r] += b;
+    }
     auto leave = [&](__half *to) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t rr = plane_rsrc(to + taps_at, all_bytes);
 #pragma unroll
@@ -961,15 +960,16 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     if (fvp > 0 && fvp <= vp_max && fits(fvp)) vp = fvp;
     if (fwv > 0) waves = fwv;
     // fp16, stride 1: on the matrix cores where vectors of eight pixels make a workgroup per CU, or
-    // of four a quarter of that (up to 256 channels, whose walk is eight steps).  Eight from 64
+    // of four a quarter of that (up to 256 channels, whose walk is sixteen steps).  Eight from 64
     // workgroups on where four leave more partial sums than the channel branch takes.  us with the
-    // pooled sums, k_spatial_stream (and k_collapse_parts) / here: 8 x 64 x 200 x 300 21.0 / 17.4,
-    // 1 x 64 x 200 x 300 11.6 / 6.3, 8 x 256 x 50 x 76 11.1 / 7.9, 16 x 64 x 56 x 56 9.4 / 5.0,
-    // 64 x 128 x 28 x 28 7.9 / 6.5, 32 x 256 x 28 x 28 8.1 / 7.7, 6 x 160 x 44 x 46 9.1 / 6.5;
+    // pooled sums, k_spatial_stream (and k_collapse_parts) / here: 8 x 64 x 200 x 300 20.2 / 16.4,
+    // 1 x 64 x 200 x 300 11.6 / 6.3, 8 x 256 x 50 x 76 11.4 / 8.3, 16 x 64 x 56 x 56 9.4 / 5.6,
+    // 64 x 128 x 28 x 28 8.2 / 6.5, 32 x 256 x 28 x 28 8.3 / 8.2, 6 x 160 x 44 x 46 9.7 / 7.0;
+    // without them 15.6 / 15.5, 5.9 / 5.4, 7.8 / 7.4, 6.2 / 5.2, 7.2 / 6.2, 7.3 / 7.4, 6.1 / 6.1;
     // 24 x 512 x 28 x 28 10.9 / 11.1 in 96 workgroups, 1 x 96 x 80 x 96 8.0 / 8.1 in 30.
     bool mma = false;
     if constexpr (esz == 2) {
-        if (stride == 1 && C % 32 == 0 && C <= kSpatialMmaChannels && (uintptr_t)w % 16 == 0 &&
+        if (stride == 1 && C % kSpatialMmaGroup == 0 && C <= kSpatialMmaChannels && (uintptr_t)w % 16 == 0 &&
             tune_int("DDF_TUNE_SPATIAL_MMA", 1) != 0) {
             const int64_t tiles8 = cdiv(npix / 8, kWave), tiles4 = cdiv(npix / 4, kWave), left = channel_parts_left(N, C);
             const bool narrow = fits(4) && tiles4 * N * head >= (C <= 256 ? 64 : 256);
@@ -991,7 +991,7 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     g.nvec = (int)(npix / vp);
     const int tiles = (int)cdiv(g.nvec, kWave);
     g.lpt = (int)cdiv(g.nvec, tiles);                   // (tiles of equal size)
-    g.ngroups = (int)(mma ? C / 32 : C / U);
+    g.ngroups = (int)(mma ? C / kSpatialMmaGroup : C / U);
     g.gpw = (int)cdiv(g.ngroups, waves);
     g.steps = (int)cdiv(g.gpw, NST) * NST;
     if (N > 65535 || head > 65535) return hipErrorNotSupported;

@@ -187,8 +187,8 @@ def test_spatial_branch_pool(case, dtype):
 
 
 # vectors of four and of eight pixels, whole and partly filled tiles, odd and even numbers of
-# 32-channel groups, several heads
-MMA_CASES = [(11, 32, 40, 44, 1), (70, 64, 8, 13, 1), (3, 96, 60, 100, 3), (40, 320, 36, 52, 1), (34, 256, 33, 64, 1),
+# 16-channel groups, several heads
+MMA_CASES = [(11, 32, 40, 44, 1), (11, 16, 40, 44, 1), (9, 48, 64, 36, 2), (70, 64, 8, 13, 1), (3, 96, 60, 100, 3), (40, 320, 36, 52, 1), (34, 256, 33, 64, 1),
              (2, 64, 240, 300, 1), (1, 64, 200, 300, 1)]
 
 
