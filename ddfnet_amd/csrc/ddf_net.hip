@@ -158,8 +158,8 @@ struct TapWeights {
 // serves at once are rows {0-3, 12-15, 20-27} or {4-11, 16-19, 28-31} of 32, and with these
 // turns they meet all sixteen places of the 256 bytes the banks span (r & 7, the turn before,
 // had every second read conflict: 1.76 M conflict cycles at 25088 x 1024 x 256, now 0.15 M).
-// Rate at batch 128, us staged through registers / now: 56 x 56 x 64 -> 256 82 / 65, 28 x 28 x
-// 512 -> 1024 under stride 2 54 / 47, 14 x 14 x 1024 -> 256 28 / 25 (525 TFLOP/s); deeper rings,
+// Rate at batch 128, us staged through registers / through the ring: 56 x 56 x 64 -> 256 82 / 65, 28 x 28 x
+// 512 -> 1024 under stride 2 54 / 47, 14 x 14 x 1024 -> 256 28 / 24 (545 TFLOP/s); deeper rings,
 // larger tiles and a K order turned per tile change nothing there; the matrix cores are busy a
 // third of the time, and 98 tiles for an XCD's 96 places cost 125 -> 128 images 10 %.  The wide
 // results of the 56 x 56 layers run at copy rate.
@@ -514,7 +514,8 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
 // as long as both operands agree), four blocks of a wave in flight.  What the launch takes is what
 // one compute unit's operands take on their way in, so smaller tiles are faster than larger ones
 // and than more waves (us for 32 x 32, the same with sixteen waves, 16 x 16: 49 x 2048 -> 512 9.7,
-// 9.7, 7.2; 196 x 1024 -> 256 6.7, 9.9, 5.7; 1 x 2048 -> 1000 7.1, 7.1, 5.2).
+// 9.7, 7.2; 196 x 1024 -> 256 6.7, 9.9, 5.7; 1 x 2048 -> 1000 7.1, 7.1, 5.2; without a last round of
+// loads that nothing used 16 x 16 takes 5.7, 4.2 and 4.3).
 template <bool POOL>
 __global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tiles_n) {
     constexpr int WAVES = kThreads / kWave, D = 4, T = 16;
@@ -1233,7 +1234,7 @@ bool conv_in_tiles(const NetConv &a) {
 // goes through several, short stages leave room for one workgroup more; where it has one or
 // two, long stages cost fewer barriers (batch 128, us long / short stages: 3136 tiles of
 // 56 x 56 x 64 -> 256 76 / 65, 1568 of 28 x 28 x 512 -> 256 54 / 50, 784 of 14 x 14 x 1024 -> 512
-// 43 / 46, 392 of 14 x 14 x 1024 -> 256 25 / 30).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
+// 42.2 / 43.4, 392 of 14 x 14 x 1024 -> 256 24.1 / 28.5).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
 // 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
 enum ConvTile { kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64, kTileSplit };
 ConvTile conv_tile(const NetConv &a, bool pair) {
