@@ -2,6 +2,7 @@
 // rows per lane, how lanes are laid over a strip and how many channels a wave
 // walks.
 #include <algorithm>
+#include <cmath>
 
 #include "ddf_rows_taprow.h"
 
@@ -204,7 +205,8 @@ bool rows_cut(const Problem &p, int vx, int R, RowsGeom *g, int *vx_out, int *r_
 }
 
 // The plane as one run of lanes (RowsGeom::halo) instead of strips of whole rows, in vectors of vx
-// and R rows per lane; false where that takes no strip less.  A strip of whole rows leaves up to
+// and R rows per lane; false where that takes no strip less.  (Whether the forward pass and the
+// feature gradient take it: rows_layout_cost.)  A strip of whole rows leaves up to
 // half of a wave's lanes idle (38 vectors of a 300-pixel row, 26 of a 101-pixel one); a run
 // leaves two, and one per row.  Forward, strips -> run: fp16 8 x 64 x 200 x 300 39.7 -> 34.9 us,
 // 5 x 5 at 8 x 64 x 90 x 100 18.8 -> 15.9, 3 x 77 x 140 x 190 12.1 -> 11.0; fp32 8 x 64 x 100 x
@@ -319,10 +321,38 @@ bool stride2_ragged_geometry(const Problem &p, int dtype, bool filters, bool who
 // before the walk as much as three channels - times its waves per SIMD, of which it takes two
 // or three to keep one busy.  Ragged vectors cost more than their masks: unaligned accesses
 // touch a cache line more.
-double rows_cost(const RowsGeom &g, bool ragged, int k, int esz, int vx, int r) {
+double rows_cost(const RowsGeom &g, bool ragged, int k, int esz, int vx, int r, double odd_tail = 1.5,
+                 double busy = 2.5) {
     const double per_wave = (g.cpw + 3.0) * (40 + (k == 5 ? 45 : 16) * vx * r);
-    const double over = !ragged ? 1.0 : g.shift ? 1.5 : esz == 2 ? 1.05 : 1.15;
-    return per_wave * over * std::max(2.5, (double)g.nwork / kSimds);
+    const double over = !ragged ? 1.0 : g.shift ? odd_tail : esz == 2 ? 1.05 : 1.15;
+    return per_wave * over * std::max(busy, (double)g.nwork / kSimds);
+}
+
+// For choosing between whole rows and a run of lanes: the same beside the memory the launch moves
+// (an instruction of a wave takes 1.1 ns, in which a large copy moves 5.8 kB), as two sides of a
+// right angle.  Whole rows end on memory lines, or in one that the next strip shares; a run ends
+// anywhere, and lanes of two rows end in two lines per strip, whose parts two compute units read
+// and store (32 x 256 x 112 x 112 fp32: 13.5 % more cache accesses, 5 % more requests to L2, 360 000 of
+// 6.8 million writes to memory shorter than 64 bytes).  In a launch that waits for memory that costs
+// more than idle lanes do: 3 x 3, strips -> run, fp32 32 x 256 x 112 x 112 168.6 -> 194.8 us (28 strips
+// -> 27), 32 x 256 x 224 x 224 727 -> 806 (112 -> 103), 32 x 192 x 139 x 145 252 -> 284 (70 -> 43); fp16
+// 51 x 170 x 108 x 162 172 -> 191 (27 -> 20).  Lanes of one row: 22 x 456 x 100 x 72 fp32 130.6 -> 138.9, elsewhere within 2 %.  Rows in
+// several segments end inside lines as well (fp32 12 x 112 x 238 x 331 252 -> 236, 238 strips -> 162;
+// 8 x 64 x 200 x 300 68.8 -> 66.0), and what fits L2 is put together there (3 x 56 x 221 x 133 15.2
+// -> 13.1, 111 -> 63).  Vectors of less than 16 bytes ask more often for the same (8 x 64 x 100 x 150
+// fp16: 11.7 us in strips of 16-byte vectors, 12.3 in a run of 8-byte ones); those of an odd tail,
+// which start at odd elements, are dearer the longer they are.  The shares are fitted over 1434 calls
+// between 0.6 and 1600 MB: their choices are 0.7 % over the better one's time on average, counting
+// instructions alone 3.5 %, whole rows throughout 3.8 %.  25 taps never wait for memory.
+double rows_layout_cost(const Problem &p, const RowsGeom &g, int esz, int vx, int r) {
+    const bool wide = vx * esz >= 16;
+    const double instructions = rows_cost(g, g.tail > 0, p.k, esz, vx, r, !wide ? 1.3 : p.d == 1 ? 1.8 : 1.5, 2.0);
+    if (p.k == 5) return instructions;
+    const bool on_lines = g.segs <= 1 || (g.seg_out * vx * esz % 128 == 0 && p.W * esz % 128 == 0);
+    const double parted = g.halo ? (r == 2 ? 0.35 : 0.02) : on_lines ? 0.0 : 0.3;
+    const double bytes = 2.0 * p.N * p.C * p.H * p.W * esz, beyond_l2 = std::max(0.0, 1 - 30e6 / bytes);
+    const double memory = bytes / 5800 * ((wide ? 1.1 : esz == 2 ? 1.2 : 1.4) + parted * beyond_l2);
+    return std::sqrt(instructions * instructions + memory * memory);
 }
 
 // The same for k_rows_filters: some 60 instructions per channel and 50 per pixel of a lane;
@@ -440,15 +470,28 @@ bool rows_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r, bool b
     const int exact_vx = *vx, exact_r = *r;
     for (tvx = 16 / esz; tvx >= 4; tvx /= 2)
         if (rows_ragged_geometry(p, dtype, tvx, &t, &tr)) consider(true);
+    if (!found) return false;
+    // The plane as one run of lanes; 3 x 3 taps with no less than half the pixels per lane (fp16
+    // 12 x 72 x 245 x 369 100 us with sixteen, 118 with four)
     // (ragged rows take operands at any address: such a launch stays one, as a run or not)
-    tvx = exact_vx;
-    tr = exact_r;
-    if (exact && g->tail == 0 && rows_run_geometry(p, tvx, tr, whole, &t)) consider(false);
+    const bool rows_ragged = g->tail > 0;
+    const int pixels = *vx * *r;
+    best = rows_layout_cost(p, *g, esz, *vx, *r);
+    auto consider_run = [&](int rvx, int rr) {
+        if (p.k == 3 && rvx * rr * 2 < pixels) return;
+        const double c = rows_layout_cost(p, t, esz, rvx, rr);
+        if (c >= best) return;
+        best = c;
+        *g = t;
+        *vx = rvx;
+        *r = rr;
+    };
+    if (exact && !rows_ragged && rows_run_geometry(p, exact_vx, exact_r, whole, &t)) consider_run(exact_vx, exact_r);
     for (tvx = 16 / esz; tvx >= 4; tvx /= 2) {
         RowsGeom rows;
-        if (rows_ragged_geometry(p, dtype, tvx, &rows, &tr) && rows_run_geometry(p, tvx, tr, rows, &t)) consider(true);
+        if (rows_ragged_geometry(p, dtype, tvx, &rows, &tr) && rows_run_geometry(p, tvx, tr, rows, &t)) consider_run(tvx, tr);
     }
-    return found;
+    return true;
 }
 
 // Instantiated (elements per lane and row, rows per lane) of k_rows_filters;

@@ -50,3 +50,25 @@ def test_every_launch_geometry_stays_in_bounds(tmp_path):
         assert sum(l.startswith('kind') and 'unsupported' not in l for l in lines) > 500
         bad = [l for l in lines if 'VIOLATION' in l]
         assert not bad, '\n'.join(bad[:10])
+
+
+@pytest.mark.parametrize('dtype,shape,k,run', [
+    # launches that wait for memory: whole rows, in full vectors
+    ('float32', (32, 256, 112, 112), 3, False), ('float32', (32, 256, 224, 224), 3, False),
+    ('float32', (64, 64, 112, 112), 3, False), ('float32', (32, 192, 139, 145), 3, False),
+    ('float16', (51, 170, 108, 162), 3, False), ('float16', (8, 64, 100, 150), 3, False),
+    # rows cut into segments, results that fit L2, 25 taps, lanes of one row
+    ('float16', (8, 64, 200, 300), 3, True), ('float32', (12, 112, 238, 331), 3, True),
+    ('float32', (3, 56, 221, 133), 3, True), ('float16', (26, 64, 65, 85), 5, True),
+    ('float32', (8, 64, 90, 100), 5, True), ('float32', (12, 144, 80, 87), 3, True),
+])
+def test_a_plane_is_a_run_of_lanes_where_that_pays(dtype, shape, k, run):
+    """Strips of whole rows against one run of lanes: each as it was measured to be faster."""
+    import torch
+    from ddfnet_amd import _lib
+    dtype = getattr(torch, dtype)
+    for need in (0, _lib.NEED_DX):
+        name = _lib.describe(shape, k, 1, 1, 'mul', dtype, need)
+        assert ('run>' in name) == run, name
+        if not run:
+            assert 'VX=%d,R=2' % (16 // dtype.itemsize) in name, name
