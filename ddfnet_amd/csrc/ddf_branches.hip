@@ -959,25 +959,35 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     const int fvp = tune_int("DDF_TUNE_SPATIAL_VP", 0), fwv = tune_int("DDF_TUNE_SPATIAL_WAVES", 0);
     if (fvp > 0 && fvp <= vp_max && fits(fvp)) vp = fvp;
     if (fwv > 0) waves = fwv;
-    // fp16, stride 1: on the matrix cores where vectors of eight pixels make a workgroup per CU, or
-    // of four a quarter of that (up to 256 channels, whose walk is sixteen steps).  Eight from 64
-    // workgroups on where four leave more partial sums than the channel branch takes.  us with the
-    // pooled sums, k_spatial_stream (and k_collapse_parts) / here: 8 x 64 x 200 x 300 20.2 / 16.4,
-    // 1 x 64 x 200 x 300 11.6 / 6.3, 8 x 256 x 50 x 76 11.4 / 8.3, 16 x 64 x 56 x 56 9.4 / 5.6,
-    // 64 x 128 x 28 x 28 8.2 / 6.5, 32 x 256 x 28 x 28 8.3 / 8.2, 6 x 160 x 44 x 46 9.7 / 7.0;
-    // without them 15.6 / 15.5, 5.9 / 5.4, 7.8 / 7.4, 6.2 / 5.2, 7.2 / 6.2, 7.3 / 7.4, 6.1 / 6.1;
-    // 24 x 512 x 28 x 28 10.9 / 11.1 in 96 workgroups, 1 x 96 x 80 x 96 8.0 / 8.1 in 30.
+    // fp16, stride 1: on the matrix cores where that leaves enough workgroups at work: its four waves
+    // walk all channels of their pixels, so few of them are one long walk behind another, which
+    // k_spatial_stream splits over waves.  Counted in workgroups full of pixels: 64 at up to 80
+    // channels, 128 at up to 256, 256 beyond; 32 at up to 128 where k_spatial_stream leaves more partial sums
+    // than the channel branch takes and a launch more would add them up.  Vectors of eight pixels from
+    // 256 on, of four below, or of eight where those of four leave too many partial sums.  An odd
+    // number of 16-channel groups walks one more: of three that is too much for the largest planes.
+    // (With the sums or without: the same kernel, so the same bits.)  us without the pooled sums /
+    // with them and the channel branch behind, operands from memory, k_spatial_stream -> here: 128 x 64 x
+    // 56 x 56 13.6 / 20.7 -> 14.2 / 20.2, 128 x 128 x 28 x 28 10.9 / 17.8 -> 9.6 / 15.8, 8 x 64 x 200 x 300 16.0 /
+    // 22.2 -> 15.5 / 21.8, 1 x 64 x 200 x 300 6.4 / 16.6 -> 6.0 / 13.0, 21 x 320 x 48 x 68 18.4 / 28 -> 14.6 / 24;
+    // left to it: 128 x 256 x 14 x 14 (98 full ones) 8.0 / 15.7, here 9.5 / 16.4; 64 x 256 x 14 x 14 7.3 / 14.9,
+    // 9.3 / 16.4; 32 x 256 x 28 x 28 8.0 / 15.6, 9.6 / 16.9; 24 x 512 x 28 x 28 9.9 / 20.5, 14.6 / 25.4; 54 x 48 x 106 x
+    // 84 12.8 / 18.9, 14.0 / 20.9.  (1096 sizes: 1.5 / 0.9 % over the best of the three on average,
+    // k_spatial_stream throughout 2.8 / 4.7 %.)
     bool mma = false;
     if constexpr (esz == 2) {
         if (stride == 1 && C % kSpatialMmaGroup == 0 && C <= kSpatialMmaChannels && (uintptr_t)w % 16 == 0 &&
             tune_int("DDF_TUNE_SPATIAL_MMA", 1) != 0) {
+            constexpr int kPixels = 4 * kWave;     // of a workgroup, four per lane
             const int64_t tiles8 = cdiv(npix / 8, kWave), tiles4 = cdiv(npix / 4, kWave), left = channel_parts_left(N, C);
-            const bool narrow = fits(4) && tiles4 * N * head >= (C <= 256 ? 64 : 256);
-            const bool wide = fits(8) && (tiles8 * N * head >= 256 ||
-                                          (narrow && pool && tiles4 > left && tiles8 <= left && tiles8 * N * head >= 64));
+            const int64_t full = head * (C <= 64 ? N * tiles4 : N * npix / kPixels);
+            const bool collapses = vp > 0 && C <= 128 && cdiv(npix / vp, kWave) > left && tiles4 <= left;
+            const bool odd = (C / kSpatialMmaGroup) % 2 != 0 && C < 64;
+            const bool wide = fits(8) && full >= (odd ? 2048 : 256);
+            const bool narrow = fits(4) && full >= (collapses ? 32 : C <= 80 ? 64 : C <= 256 ? 128 : 256) && !(odd && full >= 512);
             if (wide || narrow) {
                 mma = true;
-                vp = wide ? 8 : 4;
+                vp = wide || (pool && fits(8) && tiles4 > left && tiles8 <= left) ? 8 : 4;
                 waves = 1;
             }
         }

@@ -319,3 +319,22 @@ def test_channel_branch_rows_through_lds(n, c, mid, tiles, dtype, tol):
     got = _lib.channel_branch_parts(parts, 1.0, w1, b1, w2, b2, k, 0.7, gv, ov).view(n, c, -1)
     rest = [i for i in range(c) if i != c // 2]
     assert torch.equal(got[:, rest], out.view(n, c, -1)[:, rest])
+
+
+@pytest.mark.parametrize('case,tiles', [
+    # few workgroups, or not full of pixels: k_spatial_stream's vectors of two, a pixel
+    ((128, 256, 14, 14), 2), ((64, 256, 14, 14), 2), ((32, 256, 28, 28), 7), ((24, 512, 28, 28), 7), ((8, 256, 50, 76), 30),
+    # the matrix cores, in vectors of eight (where those of four leave too many sums, too) and of four
+    ((128, 128, 28, 28), 2), ((21, 320, 48, 68), 7), ((1, 64, 200, 300), 118), ((16, 64, 56, 56), 13), ((64, 128, 28, 28), 4),
+    ((2, 128, 92, 144), 52),
+], ids=lambda c: str(c).replace(' ', ''))
+def test_spatial_branch_takes_the_faster_kernel(case, tiles):
+    """Which kernel ran, by the pixels its tiles cover: each as it was measured to be faster."""
+    n, c, h, w_ = case
+    x = torch.randn(n, c, h, w_, device='cuda').half()
+    w = (torch.randn(9, c, device='cuda') * 0.2).half()
+    sf, parts = _lib.spatial_branch_pool(x, w, None, 1, 3, 1, 0.7)
+    assert parts.shape[1] == tiles
+    assert torch.equal(sf, _lib.spatial_branch(x, w, None, 1, 3, 1, 0.7))
+    sums, scale = x.double().sum((2, 3)), x.double().abs().sum((2, 3)).max()
+    assert ((parts.double().sum(1) - sums).abs().max() / scale).item() < 1e-6
