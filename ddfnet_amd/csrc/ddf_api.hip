@@ -784,6 +784,20 @@ int ddf_hip_net_conv_pool(const void *features, const void *weight, const ddf_ne
     return net_result(ddf::net_conv(a, (hipStream_t)stream), "ddf_hip_net_conv_pool launch");
 }
 
+int ddf_hip_net_parts_left(int64_t N, int64_t C, int64_t mid) {
+    if (N < 1 || C < 1 || mid < 1 || C > (1 << 24) || mid > (1 << 24)) return 1;
+    return (int)ddf::parts_left(N, C, mid, 2);
+}
+
+int ddf_hip_net_sum_parts(const float *pool_parts, int n_parts, float *totals, int64_t N, int64_t C, void *stream) {
+    if (N < 0 || N > 65535 || C < 1 || C > (1 << 24) || n_parts < 1 || (int64_t)n_parts * C * 4 >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_sum_parts: bad sizes");
+    if (!pool_parts || !totals) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    if (N == 0) return DDF_OK;
+    return net_result(ddf::collapse_parts(pool_parts, n_parts, totals, N, C, (hipStream_t)stream),
+                      "ddf_hip_net_sum_parts launch");
+}
+
 int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_net_norm_t *norm, int64_t C,
                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
                           int64_t H, int64_t W, int64_t side_C, int stride, void *output, int64_t N, int64_t O,

@@ -730,37 +730,47 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_s
     }
 }
 
-// out[n * C + c] = sum of parts[(n * nparts + p) * C + c] over p.  Every workgroup of the
-// channel branch starts from the pooled vectors; with dozens of partial sums per value each
-// of them would spend longer adding up than on its own work (8 x 64 x 200 x 300 fp16: 472
-// sums per value then, 37 of the layer's 107 us), so planes of many tiles pay for one launch,
-// unless a sample's few channels leave the workgroup waves enough to share a value's sums.
-constexpr int kMaxParts = 8;             // partial sums per value the channel branch is left at least
-// (two rounds of requests; 118 sums of 64 channels 5.1 us, 4.1 with few, and the launch 4.7)
-inline int64_t channel_parts_left(int64_t N, int64_t C) {
-    const int64_t width = cdiv(C, kWave);
-    return N * width <= 256 && width <= 4 ? 2 * kMaxParts * (kRowsPoolWaves / width) : kMaxParts;
-}
-constexpr int kCollapseChannels = 64, kCollapseGroups = 8;
-__global__ __launch_bounds__(kCollapseChannels * kCollapseGroups) void k_collapse_parts(
-    const float *__restrict__ parts, float *__restrict__ out, int C, int nparts) {
-    __shared__ float red[kCollapseGroups][kCollapseChannels];
-    const int i = threadIdx.x % kCollapseChannels, grp = threadIdx.x / kCollapseChannels;
-    const int c = blockIdx.x * kCollapseChannels + i;
+// out[n * C + c] = sum of parts[(n * nparts + p) * C + c] over p, for 64 channels of a sample: a
+// lane loads V of them, eight partial sums at a time, so that 512 of them (V = 4) are one round trip.
+constexpr int kCollapseChannels = 64, kCollapseThreads = 1024, kCollapseWaves = kCollapseThreads / kWave;
+template <int V>
+__global__ __launch_bounds__(kCollapseThreads) void k_collapse_parts(const float *__restrict__ parts,
+                                                                     float *__restrict__ out, int C, int nparts) {
+    constexpr int LANES = kCollapseChannels / V, GROUPS = kCollapseThreads / LANES, ROUND = 8;
+    __shared__ float red[kCollapseWaves][kCollapseChannels];
+    const int at = threadIdx.x % LANES * V, grp = threadIdx.x / LANES;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int c = blockIdx.x * kCollapseChannels + at;
     const int64_t n = blockIdx.y;
-    float a = 0.f;
-    if (c < C) {
-        const float *src = parts + n * nparts * C + c;
-#pragma unroll 8
-        for (int q = grp; q < nparts; q += kCollapseGroups) a += src[(int64_t)q * C];
-    }
-    red[grp][i] = a;
-    __syncthreads();
-    if (grp == 0 && c < C) {
+    const __amdgpu_buffer_rsrc_t r = plane_rsrc(parts + n * nparts * C, (uint32_t)(nparts * C) * 4u);
+    float sum[V];
 #pragma unroll
-        for (int k = 1; k < kCollapseGroups; ++k) a += red[k][i];
-        out[n * C + c] = a;
+    for (int v = 0; v < V; ++v) sum[v] = 0.f;
+    for (int q0 = grp; q0 < nparts; q0 += GROUPS * ROUND) {
+        uint32_t x[ROUND][V];
+#pragma unroll
+        for (int u = 0; u < ROUND; ++u) {
+            const int q = q0 + u * GROUPS;
+            load_vec<V * 4>(r, c < C && q < nparts ? (uint32_t)(q * C + c) * 4u : kOutside, x[u]);
+        }
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            auto y = [&](int u) __attribute__((always_inline)) { return __uint_as_float(x[u][v]); };
+            sum[v] += ((y(0) + y(1)) + (y(2) + y(3))) + ((y(4) + y(5)) + (y(6) + y(7)));
+        }
     }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        if constexpr (V == 4) sum[v] = rows_total(sum[v]);    // (four groups a wave)
+        if (lane < LANES) red[wave][at + v] = sum[v];
+    }
+    __syncthreads();
+    const int i = threadIdx.x, to = blockIdx.x * kCollapseChannels + i;
+    if (i >= kCollapseChannels || to >= C) return;
+    float total = 0.f;
+#pragma unroll
+    for (int k = 0; k < kCollapseWaves; ++k) total += red[k][i];
+    out[n * C + to] = total;
 }
 
 constexpr int kChannelThreads = 1024;  // sixteen waves: the rows of a block's taps are dealt out to them
@@ -793,19 +803,35 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const int rows = min(BLOCK, C - cb) * KK;
     TapParams<T, KK> params;
     // the pooled vectors: given, or scale * the sum of nparts partial sums per value
-    // (parts[(n * nparts + p) * C + c], what k_spatial_stream leaves)
-    for (int i = threadIdx.x; i < NS * C; i += kChannelThreads) {
+    // (parts[(n * nparts + p) * C + c], what k_spatial_stream leaves); of many of them as many
+    // threads share a value's as there are
+    const int values = NS * C, share = parts && nparts > kMmaRound ? kChannelThreads / values : 1;
+    const int g = threadIdx.x / values;
+    auto part_sum = [&](int i, int first, int step) __attribute__((always_inline)) {
         const int s = i / C, c = i - s * C;
-        const int64_t n = n0 + min(s, ns - 1);
-        if (parts) {
-            float a = 0.f;
+        const float *src = parts + (n0 + min(s, ns - 1)) * nparts * C + c;
+        float a = 0.f;
 #pragma unroll 8
-            for (int q = 0; q < nparts; ++q) a += parts[(n * nparts + q) * C + c];
-            v[i] = a * scale;
-        } else {
-            v[i] = ld(pooled + n * C + c);
+        for (int q = first; q < nparts; q += step) a += src[(int64_t)q * C];
+        return a;
+    };
+    auto put_pooled = [&](int i, float a) __attribute__((always_inline)) {
+        v[i] = a;
+        const int s = i / C;
+        if (save.pooled && blockIdx.x == 0 && s < ns) save.pooled[n0 * C + i] = a;
+    };
+    if (share > 1) {
+        __shared__ float red[kChannelThreads];
+        if (g < share) red[threadIdx.x] = part_sum(threadIdx.x - g * values, g, share);
+        __syncthreads();
+        if (g == 0) {
+            float a = red[threadIdx.x];
+            for (int k = 1; k < share; ++k) a += red[k * values + threadIdx.x];
+            put_pooled(threadIdx.x, a * scale);
         }
-        if (save.pooled && blockIdx.x == 0 && s < ns) save.pooled[n * C + c] = v[i];
+    } else {
+        for (int i = threadIdx.x; i < values; i += kChannelThreads)
+            put_pooled(i, parts ? part_sum(i, 0, 1) * scale : ld(pooled + (n0 + min(i / C, ns - 1)) * C + i % C));
     }
     __syncthreads();
     // Dot products with sixteen lanes along a weight row and four rows per wave at a
@@ -908,6 +934,16 @@ __global__ __launch_bounds__(kMmaThreads) void k_channel_branch_mma(ChannelMma a
 
 bool branch_kernel_size_built(int k) { return k == 3 || k == 5; }
 
+int64_t parts_left(int64_t N, int64_t C, int64_t mid, int esz) { return channel_parts_left(N, C, mid, esz); }
+hipError_t collapse_parts(const float *parts, int nparts, float *totals, int64_t N, int64_t C, hipStream_t st) {
+    const dim3 grid((unsigned)cdiv(C, kCollapseChannels), (unsigned)N);
+    if (C % 4 == 0 && (uintptr_t)parts % 16 == 0)
+        hipLaunchKernelGGL((k_collapse_parts<4>), grid, dim3(kCollapseThreads), 0, st, parts, totals, (int)C, nparts);
+    else
+        hipLaunchKernelGGL((k_collapse_parts<1>), grid, dim3(kCollapseThreads), 0, st, parts, totals, (int)C, nparts);
+    return hipGetLastError();
+}
+
 // Launch of k_spatial_stream; hipErrorNotSupported where it does not cover the problem
 // (the caller then takes the kernels above).
 template <typename T>
@@ -962,29 +998,27 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     // fp16, stride 1: on the matrix cores where that leaves enough workgroups at work: its four waves
     // walk all channels of their pixels, so few of them are one long walk behind another, which
     // k_spatial_stream splits over waves.  Counted in workgroups full of pixels: 64 at up to 80
-    // channels, 128 at up to 256, 256 beyond; 32 at up to 128 where k_spatial_stream leaves more partial sums
-    // than the channel branch takes and a launch more would add them up.  Vectors of eight pixels from
-    // 256 on, of four below, or of eight where those of four leave too many partial sums.  An odd
-    // number of 16-channel groups walks one more: of three that is too much for the largest planes.
-    // (With the sums or without: the same kernel, so the same bits.)  us without the pooled sums /
-    // with them and the channel branch behind, operands from memory, k_spatial_stream -> here: 128 x 64 x
-    // 56 x 56 13.6 / 20.7 -> 14.2 / 20.2, 128 x 128 x 28 x 28 10.9 / 17.8 -> 9.6 / 15.8, 8 x 64 x 200 x 300 16.0 /
-    // 22.2 -> 15.5 / 21.8, 1 x 64 x 200 x 300 6.4 / 16.6 -> 6.0 / 13.0, 21 x 320 x 48 x 68 18.4 / 28 -> 14.6 / 24;
-    // left to it: 128 x 256 x 14 x 14 (98 full ones) 8.0 / 15.7, here 9.5 / 16.4; 64 x 256 x 14 x 14 7.3 / 14.9,
-    // 9.3 / 16.4; 32 x 256 x 28 x 28 8.0 / 15.6, 9.6 / 16.9; 24 x 512 x 28 x 28 9.9 / 20.5, 14.6 / 25.4; 54 x 48 x 106 x
-    // 84 12.8 / 18.9, 14.0 / 20.9.  (1096 sizes: 1.5 / 0.9 % over the best of the three on average,
-    // k_spatial_stream throughout 2.8 / 4.7 %.)
+    // channels, 128 at up to 256, 256 beyond.  Vectors of eight pixels from 256 on (768 at up to 64
+    // channels), of four below, or of eight where those of four leave too many partial sums.  An odd
+    // number of 16-channel groups walks one more: of three that is too much for large planes.  (With
+    // the sums or without: the same kernel, so the same bits.)  us without the pooled sums / with them
+    // and the channel branch behind, operands from memory, k_spatial_stream -> here: 128 x 64 x 56 x 56
+    // 13.6 / 20.7 -> 14.2 / 20.2, 128 x 128 x 28 x 28 10.9 / 17.8 -> 9.6 / 15.8, 8 x 64 x 200 x 300 16.0 / 22.2 ->
+    // 15.5 / 21.8, 16 x 64 x 56 x 56 6.7 / 13.2 -> 5.8 / 12.0, 21 x 320 x 48 x 68 18.4 / 28 -> 14.6 / 24; left to
+    // it: 128 x 256 x 14 x 14 (98 full ones) 8.0 / 15.7, here 9.5 / 16.4; 64 x 256 x 14 x 14 7.3 / 14.9, 9.3 /
+    // 16.4; 32 x 256 x 28 x 28 8.0 / 15.6, 9.6 / 16.9; 24 x 512 x 28 x 28 9.9 / 20.5, 14.6 / 25.4; 54 x 48 x 106 x 84
+    // 12.8 / 18.9, 14.0 / 20.9.  (943 sizes: 1.6 / 0.8 % over the best of the three on average,
+    // k_spatial_stream throughout 2.9 / 4.3 %.)
     bool mma = false;
     if constexpr (esz == 2) {
         if (stride == 1 && C % kSpatialMmaGroup == 0 && C <= kSpatialMmaChannels && (uintptr_t)w % 16 == 0 &&
             tune_int("DDF_TUNE_SPATIAL_MMA", 1) != 0) {
             constexpr int kPixels = 4 * kWave;     // of a workgroup, four per lane
-            const int64_t tiles8 = cdiv(npix / 8, kWave), tiles4 = cdiv(npix / 4, kWave), left = channel_parts_left(N, C);
+            const int64_t tiles8 = cdiv(npix / 8, kWave), tiles4 = cdiv(npix / 4, kWave), left = channel_parts_left(N, C, C / 5, esz);
             const int64_t full = head * (C <= 64 ? N * tiles4 : N * npix / kPixels);
-            const bool collapses = vp > 0 && C <= 128 && cdiv(npix / vp, kWave) > left && tiles4 <= left;
             const bool odd = (C / kSpatialMmaGroup) % 2 != 0 && C < 64;
-            const bool wide = fits(8) && full >= (odd ? 2048 : 256);
-            const bool narrow = fits(4) && full >= (collapses ? 32 : C <= 80 ? 64 : C <= 256 ? 128 : 256) && !(odd && full >= 512);
+            const bool wide = fits(8) && full >= (odd ? 2048 : C <= 64 ? 768 : 256);
+            const bool narrow = fits(4) && full >= (C <= 80 ? 64 : C <= 256 ? 128 : 256) && !(odd && full >= 512);
             if (wide || narrow) {
                 mma = true;
                 vp = wide || (pool && fits(8) && tiles4 > left && tiles8 <= left) ? 8 : 4;
@@ -1007,9 +1041,10 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     if (N > 65535 || head > 65535) return hipErrorNotSupported;
     bool collapse = false;
     if (pool) {
-        // (more tiles than the channel branch is left: their sums go behind the N * C totals
-        // that k_collapse_parts then makes of them)
-        collapse = tiles > tune_int("DDF_TUNE_COLLAPSE", (int)channel_parts_left(N, C));
+        // (more tiles than the channel branch is left - with the hidden layer that a layer has unless
+        // it is told otherwise, a fifth of the channels: their sums go behind the N * C totals that
+        // k_collapse_parts then makes of them)
+        collapse = tiles > tune_int("DDF_TUNE_COLLAPSE", (int)std::min<int64_t>(channel_parts_left(N, C, C / 5, esz), 1 << 30));
         if (N * (tiles + (collapse ? 1 : 0)) * C > pool_capacity) return hipErrorInvalidValue;
         *pool_parts = collapse ? 1 : tiles;
     }
@@ -1026,9 +1061,7 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
             else if (pool) DDF_SPATIAL_MMA(4, true);
             else DDF_SPATIAL_MMA(4, false);
 #undef DDF_SPATIAL_MMA
-            if (collapse)
-                hipLaunchKernelGGL(k_collapse_parts, dim3((unsigned)cdiv(C, kCollapseChannels), (unsigned)N),
-                                   dim3(kCollapseChannels * kCollapseGroups), 0, st, parts_out, pool_part, (int)C, tiles);
+            if (collapse) return collapse_parts(parts_out, tiles, pool_part, N, C, st);
             return hipGetLastError();
         }
     }
@@ -1065,9 +1098,7 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     }
 #undef DDF_STREAM_WAVES
 #undef DDF_STREAM_LAUNCH
-    if (collapse)
-        hipLaunchKernelGGL(k_collapse_parts, dim3((unsigned)cdiv(C, kCollapseChannels), (unsigned)N),
-                           dim3(kCollapseChannels * kCollapseGroups), 0, st, parts_out, pool_part, (int)C, tiles);
+    if (collapse) return collapse_parts(parts_out, tiles, pool_part, N, C, st);
     return hipGetLastError();
 }
 

@@ -605,6 +605,34 @@ inline bool channel_rows_plan(ChannelRows<T> &a) {
     return false;
 }
 
+// Partial sums per pooled value that the channel branch is left (3 x 3 taps).  Every workgroup adds
+// up those of its samples, in rounds of kMmaRound requests per lane with a round trip to memory
+// each; `spare` rounds more than one value takes are cheaper than a launch that makes totals of them.
+// us, kept as they are less totals first, medians over 668 sizes: matrix cores 4 rounds more -0.5, 6
+// -0.1, 8 +1.2, 16 +5.9; rows 4 -0.9, 6 0.0, 8 +1.5, 16 +5.3; k_channel_branch 2 -0.9, 3 +0.4, 6 +1.8.
+// (8 x 64 x 200 x 300 fp16, 118 sums: 21.8 kept, 24.9 with totals.)
+inline int64_t channel_parts_left(int64_t N, int64_t C, int64_t mid, int esz) {
+    auto div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+    const int64_t width = div(C, kWave);
+    int64_t share = 1, trips, spare;           // waves that share a value's sums, round trips per round
+    if (esz == 2 && channel_mma_covers(C, mid, kRowsKK)) {
+        const int64_t ns = std::min<int64_t>(N, kMmaSamples);
+        share = C > kMmaSpread || ns > 2 ? 1 : 4 / ns;
+        trips = div(C, 4 * kWave) * div(div(ns * share, 4), 2);
+        spare = 5;
+    } else if (N * div(C, kRowsMaxBlock) <= 256) {
+        share = width <= kRowsPoolWaves / 2 ? kRowsPoolWaves / width : 1;
+        trips = div(width * share, kRowsPoolWaves);
+        spare = 6;
+    } else {
+        const int64_t values = std::max<int64_t>(std::min<int64_t>(N * width / 256, 4), 1) * C;
+        share = std::max<int64_t>(kRowsThreads / values, 1);
+        trips = div(values, kRowsThreads);
+        spare = 3;
+    }
+    return kMmaRound * share * ((spare + trips) / trips);
+}
+
 #ifdef __HIPCC__
 
 // Butterfly steps through the VALU's lane-permute path.  (Shuffles through the

@@ -118,6 +118,10 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
                           const T *gain_vec, const T *offset_vec, hipStream_t st,
                           const float *parts = nullptr, int nparts = 0, double scale = 1.0,
                           ChannelSave save = ChannelSave());
+// Partial sums of the pooled vectors ([sample][part][channel]) to totals; more of them than the
+// second says (3 x 3 taps) are better added up before the channel branch (channel_parts_left).
+hipError_t collapse_parts(const float *parts, int nparts, float *totals, int64_t N, int64_t C, hipStream_t st);
+int64_t parts_left(int64_t N, int64_t C, int64_t mid, int esz);
 
 // Gradients of both branches (ddf_pack_backward.hip; 3 x 3 taps): from dcf and draw (the
 // gradients of the channel filter and of the un-normalised spatial taps) and what the

@@ -136,7 +136,13 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
 
     // One workspace: a block's input and output trade places (a block without a projection
     // adds its result in place), between them the narrow activations and the filters.
-    int64_t wide = 0, narrow = 0, taps = 0, filters = 0, parts = 0;
+    int64_t wide = 0, narrow = 0, taps = 0, filters = 0, parts = 0, totals = 0;
+    // (more partial sums of the pooled vectors than the channel branch is left become totals)
+    struct Parts { int count; bool summed; };
+    auto parts_of = [n](const NetBlock &b, int64_t h, int64_t w, int64_t c) {
+        const int64_t count = ddf_hip_net_conv_pool_parts(n, h, w, c, b.width);
+        return Parts{(int)count, count > ddf_hip_net_parts_left(n, b.width, b.mid)};
+    };
     {
         int64_t h = h0 / 4, w = w0 / 4, c = 64;
         wide = n * h * w * 64;
@@ -146,18 +152,22 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             wide = std::max(wide, n * ho * wo * b.conv3.t[0]->size(0));
             taps = std::max(taps, n * ho * wo * 12);
             filters = std::max(filters, n * b.width * 9);
-            parts = std::max(parts, n * b.width * ddf_hip_net_conv_pool_parts(n, h, w, c, b.width));
+            const Parts of = parts_of(b, h, w, c);
+            parts = std::max(parts, n * b.width * of.count);
+            if (of.summed) totals = std::max(totals, n * b.width);
             c = b.conv3.t[0]->size(0);
             h = ho; w = wo;
         }
     }
     const size_t wide_b = aligned_bytes(wide * 2), narrow_b = aligned_bytes(narrow * 2), taps_b = aligned_bytes(taps * 2),
-                 filters_b = aligned_bytes(filters * 2), parts_b = aligned_bytes(parts * 4);
-    at::Tensor work = new_tensor({(int64_t)(2 * wide_b + 2 * narrow_b + taps_b + filters_b + parts_b)}, at::kByte, x.device());
+                 filters_b = aligned_bytes(filters * 2), parts_b = aligned_bytes(parts * 4),
+                 totals_b = aligned_bytes(totals * 4);
+    at::Tensor work = new_tensor({(int64_t)(2 * wide_b + 2 * narrow_b + taps_b + filters_b + parts_b + totals_b)},
+                                 at::kByte, x.device());
     char *q = static_cast<char *>(work.data_ptr());
     void *cur = q, *other = q + wide_b, *t1 = q + 2 * wide_b, *t2 = q + 2 * wide_b + narrow_b;
     void *sf = q + 2 * wide_b + 2 * narrow_b, *cf = static_cast<char *>(sf) + taps_b;
-    float *pp = reinterpret_cast<float *>(static_cast<char *>(cf) + filters_b);
+    float *pp = reinterpret_cast<float *>(static_cast<char *>(cf) + filters_b), *pt = pp + parts_b / sizeof(float);
     at::Tensor logits = new_tensor({n, p.fc.t[0]->size(0)}, at::kHalf, dev);
     try {
         py::gil_scoped_release release;    // (a network's launches take a while)
@@ -168,12 +178,14 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0]->size(0);
             nm = b.conv1.norm();
             covered(ddf_hip_net_conv_pool(cur, b.conv1.t[0]->data_ptr(), &nm, t1, pp, n, h, w, c, width, 1, st));
+            const Parts of = parts_of(b, h, w, c);
+            if (of.summed) covered(ddf_hip_net_sum_parts(pp, of.count, pt, n, width, st));
             nm = b.bn2.norm();
             covered(ddf_hip_net_ddf(
-                t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pp,
-                (int)ddf_hip_net_conv_pool_parts(n, h, w, c, width), b.w1->data_ptr(), ptr_or_null(b.b1),
-                b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid, b.cgain_const, ptr_or_null(b.cgain),
-                ptr_or_null(b.coffset), &nm, t2, n, h, w, width, b.stride, b.combine, st));
+                t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, of.summed ? pt : pp,
+                of.summed ? 1 : of.count, b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(), ptr_or_null(b.b2),
+                cf, b.mid, b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset), &nm, t2, n, h, w, width,
+                b.stride, b.combine, st));
             nm = b.conv3.norm();
             if (b.down.t[0].defined()) {
                 const ddf_net_norm_t down = b.down.norm();

@@ -362,10 +362,13 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *   stem    max_pool(relu(norm(7x7 convolution, stride 2, padding 3, weight (64, 3, 7, 7))), 3x3,
  *           stride 2, padding 1) of a planar (N, 3, H, W) image; H and W multiples of 4
  *   spatial the spatial filter branch (3x3 taps, one head): spatial_filter (N, Ho*Wo, 12), nine
- *           taps and three of padding, and partial sums of the channels over the pixels as
- *           ddf_hip_spatial_branch_pool's; at most 8 parts; C 64, 128, 256 or 512
+ *           taps and three of padding, and the sums of the channels over the pixels as
+ *           ddf_hip_spatial_branch_pool's, in one part; C 64, 128, 256 or 512
  *   conv_pool  conv (stride 1, no residual) that also leaves the sums of its results over the
- *           pixels of each sample in ddf_hip_net_conv_pool_parts parts (such partial sums)
+ *           pixels of each sample in ddf_hip_net_conv_pool_parts parts (such partial sums): one
+ *           or so per 16, 64 or 128 pixels.  Of more than ddf_hip_net_parts_left(N, C, mid) the
+ *           branches are faster from their totals
+ *   sum_parts  totals (N, C) of n_parts such partial sums per sample and channel
  *   branches  both filter branches in one launch: the spatial one, and the channel one of
  *           ddf_hip_channel_branch_parts (3x3 taps) from the partial sums of conv_pool; sizes as
  *           spatial's
@@ -385,6 +388,8 @@ int64_t ddf_hip_net_conv_pool_parts(int64_t N, int64_t H, int64_t W, int64_t C, 
 int ddf_hip_net_conv_pool(const void *features, const void *weight, const ddf_net_norm_t *norm, void *output,
                           float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int relu,
                           void *stream);
+int ddf_hip_net_parts_left(int64_t N, int64_t C, int64_t mid);
+int ddf_hip_net_sum_parts(const float *pool_parts, int n_parts, float *totals, int64_t N, int64_t C, void *stream);
 int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_net_norm_t *norm, int64_t C,
                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
                           int64_t H, int64_t W, int64_t side_C, int stride, void *output, int64_t N, int64_t O,

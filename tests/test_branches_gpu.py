@@ -4,6 +4,8 @@ the reference modules they replace: the 1x1 convolution with the operator's
 stride followed by FilterNorm('spatial') (ddf/ddf.py:176-180, :145-157), and
 the bottleneck MLP on the pooled features followed by FilterNorm('channel')
 (ddf/ddf.py:183-192, :158-170)."""
+import math
+
 import pytest
 import torch
 
@@ -324,9 +326,9 @@ def test_channel_branch_rows_through_lds(n, c, mid, tiles, dtype, tol):
 @pytest.mark.parametrize('case,tiles', [
     # few workgroups, or not full of pixels: k_spatial_stream's vectors of two, a pixel
     ((128, 256, 14, 14), 2), ((64, 256, 14, 14), 2), ((32, 256, 28, 28), 7), ((24, 512, 28, 28), 7), ((8, 256, 50, 76), 30),
-    # the matrix cores, in vectors of eight (where those of four leave too many sums, too) and of four
-    ((128, 128, 28, 28), 2), ((21, 320, 48, 68), 7), ((1, 64, 200, 300), 118), ((16, 64, 56, 56), 13), ((64, 128, 28, 28), 4),
-    ((2, 128, 92, 144), 52),
+    # the matrix cores, in vectors of eight and of four; of eight where those of four leave too many sums
+    ((128, 128, 28, 28), 2), ((21, 320, 48, 68), 7), ((1, 64, 200, 300), 235), ((16, 64, 56, 56), 13), ((64, 128, 28, 28), 4),
+    ((10, 128, 64, 152), 19), ((2, 256, 120, 144), 68), ((3, 256, 120, 120), 29),
 ], ids=lambda c: str(c).replace(' ', ''))
 def test_spatial_branch_takes_the_faster_kernel(case, tiles):
     """Which kernel ran, by the pixels its tiles cover: each as it was measured to be faster."""
@@ -338,3 +340,47 @@ def test_spatial_branch_takes_the_faster_kernel(case, tiles):
     assert torch.equal(sf, _lib.spatial_branch(x, w, None, 1, 3, 1, 0.7))
     sums, scale = x.double().sum((2, 3)), x.double().abs().sum((2, 3)).max()
     assert ((parts.double().sum(1) - sums).abs().max() / scale).item() < 1e-6
+
+
+@pytest.mark.parametrize('dtype,tol', [(torch.float32, 2e-5), (torch.float16, 6e-3)])
+@pytest.mark.parametrize('n,c,h,w_,tiles', [
+    (1, 64, 480, 520, None), (2, 36, 480, 520, None), (3, 132, 250, 250, None), (20, 512, 130, 140, None),   # totals of many sums
+    (2, 34, 480, 520, None),                                                                                # channel by channel
+    (1, 64, 200, 300, 235), (8, 32, 100, 100, 40),                                                          # left as they are
+])
+def test_partial_sums_that_the_channel_branch_is_left(n, c, h, w_, tiles, dtype, tol):
+    """Few enough rounds for the kernel that will add them up, else totals in a launch of their own."""
+    if dtype == torch.float16 and c % 4:
+        return      # (pooled by a launch of its own)
+    torch.manual_seed(c + h)
+    x = torch.randn(n, c, h, w_, device='cuda').relu_().to(dtype)
+    w = (torch.randn(9, c, device='cuda') * 0.2).to(dtype)
+    sf, parts = _lib.spatial_branch_pool(x, w, None, 1, 3, 1, 0.7)
+    if tiles is None:
+        assert parts.shape[1] == 1
+    elif dtype == torch.float16:
+        assert parts.shape[1] == tiles
+    sums = x.double().sum((2, 3))
+    assert ((parts.double().sum(1) - sums).abs().max() / sums.abs().max()).item() < 1e-6
+    mid, k = max(c // 5, 1), 3
+    w1 = (torch.randn(mid, c, device='cuda') * c ** -0.5).to(dtype)
+    w2 = (torch.randn(c * 9, mid, device='cuda') * mid ** -0.5).to(dtype)
+    b1, b2 = torch.randn(mid, device='cuda').to(dtype), torch.randn(c * 9, device='cuda').to(dtype)
+    got = _lib.channel_branch_parts(parts, 1 / (h * w_), w1, b1, w2, b2, k, 0.7, None, None)
+    ref = channel_reference(sums.cpu() / (h * w_), *(t.cpu() for t in (w1, b1, w2, b2)), k, 0.7, None, None)
+    assert ((got.double().cpu() - ref).abs().max() / ref.abs().max()).item() < tol
+
+
+@pytest.mark.parametrize('n,c,mid,tiles', [(1, 64, 12, 237), (3, 100, 20, 33), (300, 64, 12, 9), (600, 32, 6, 12), (2, 1000, 30, 9),
+                                           (1, 1, 1, 1000), (1, 1024, 20, 10)])
+def test_channel_branch_of_unaligned_weights_and_many_sums(n, c, mid, tiles):
+    """k_channel_branch: the threads of a workgroup share a value's partial sums, one sample or several."""
+    torch.manual_seed(c + mid)
+    parts = torch.randn(n, tiles, c, device='cuda')
+    odd = lambda *size: torch.randn(math.prod(size) + 1, device='cuda')[1:].view(size)
+    w1, w2 = odd(mid, c).mul_(c ** -0.5), odd(c * 9, mid).mul_(mid ** -0.5)
+    assert w1.data_ptr() % 16 and w2.data_ptr() % 16
+    b1, b2 = torch.randn(mid, device='cuda'), torch.randn(c * 9, device='cuda')
+    out = _lib.channel_branch_parts(parts, 0.25, w1, b1, w2, b2, 3, 0.7, None, None)
+    ref = channel_reference(parts.double().sum(1).cpu() * 0.25, *(t.cpu() for t in (w1, b1, w2, b2)), 3, 0.7, None, None)
+    assert ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item() < 2e-5

@@ -285,3 +285,37 @@ def test_ddf_layer(n, h, w, c, s, mid, n_parts, combine):
     call('ddf_hip_net_ddf', *branches, norm, got, n, h, w, c, s, _lib.COMBINE[combine])
     assert torch.isfinite(want).all()
     close(got, want, 2e-3)      # (order of the sums over the partial sums)
+
+
+@pytest.mark.parametrize('n,c,mid,n_parts', [(1, 64, 12, 512), (2, 128, 25, 513), (1, 512, 102, 33), (33, 256, 51, 9),
+                                             (3, 20, 4, 1030), (2, 70, 14, 17), (70, 64, 12, 1)])
+def test_sum_parts(n, c, mid, n_parts):
+    parts = torch.randn(n, n_parts, c, device='cuda')
+    totals = torch.empty(n, c, device='cuda')
+    call('ddf_hip_net_sum_parts', parts, n_parts, totals, n, c)
+    want = parts.double().sum(1)
+    # (fp32 sums of n_parts values: at most n_parts roundings of the values' absolute sum, a tree's few)
+    assert (totals - want).abs().max() <= 1e-6 * parts.double().abs().sum(1).max()
+    assert 8 <= _lib.lib().ddf_hip_net_parts_left(n, c, mid) <= 1024
+
+
+@pytest.mark.parametrize('n,h,w', [(1, 1024, 1024), (3, 1024, 768), (1, 2048, 512)])
+def test_network_of_large_images(n, h, w):
+    """Hundreds of partial sums per pooled value: some are left to the channel branch, some become
+    totals first."""
+    lib, left = _lib.lib(), []
+    for k, (c, width) in enumerate(((256, 64), (256, 128), (512, 256), (1024, 512))):
+        hw = [v >> (2 + max(k - 1, 0)) for v in (h, w)]
+        left.append(lib.ddf_hip_net_conv_pool_parts(n, *hw, c, width) <= lib.ddf_hip_net_parts_left(n, width, int(.2 * width)))
+    assert True in left and False in left
+    torch.manual_seed(n)
+    model = ddf_resnet.ddf_mul_resnet50(num_classes=10, zero_init_last_bn=False).cuda().half().eval()
+    x = torch.randn(n, 3, h, w, device='cuda').half()
+    with torch.no_grad():
+        out = ddfnet_amd.functional.extension().net_forward(
+            model._native_plan(ddfnet_amd.functional.extension()), x)
+        modules = lambda net, y: net.fc(net.global_pool(net.forward_features(y)).flatten(1))
+        by_modules = modules(model, x).float()
+        want = modules(model.float(), x.float())
+    off = lambda y: ((y.float() - want).norm() / want.norm()).item()
+    assert off(out) <= max(4e-3, 1.3 * off(by_modules))
