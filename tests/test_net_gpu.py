@@ -287,6 +287,40 @@ def test_ddf_layer(n, h, w, c, s, mid, n_parts, combine):
     close(got, want, 2e-3)      # (order of the sums over the partial sums)
 
 
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('n,h,w,c,s,mid,n_parts', [
+    (1, 56, 56, 64, 1, 12, 49), (2, 10, 18, 64, 2, 12, 3), (8, 56, 56, 64, 1, 12, 25), (1, 28, 28, 128, 1, 25, 13),
+    (3, 56, 30, 128, 2, 25, 200), (1, 14, 14, 256, 1, 51, 13), (5, 13, 11, 256, 1, 51, 60), (1, 7, 7, 512, 1, 102, 4),
+    (3, 14, 14, 512, 2, 102, 30), (1, 6, 6, 512, 1, 300, 2), (2, 5, 5, 256, 1, 20, 3),
+])
+def test_ddf_layer_matches_pytorch(n, h, w, c, s, mid, n_parts, combine):
+    """The same against plain PyTorch on the same fp16 values, many partial sums among them."""
+    from test_branches_gpu import channel_reference
+    torch.manual_seed(h * w + c)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    ws, bs = (torch.randn(9, c, device='cuda') * c ** -0.5).half(), torch.randn(9, device='cuda').half()
+    parts = torch.randn(n, n_parts, c, device='cuda') * (h * w / n_parts ** 0.5)
+    w1, w2 = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((mid, c), (9 * c, mid)))
+    b1, b2, gv, ov = (torch.randn(k, device='cuda').half() for k in (mid, 9 * c, 9 * c, 9 * c))
+    ho, wo = h // s, w // s
+    sf = torch.empty(n, ho * wo, 12, device='cuda', dtype=torch.float16)
+    cf = torch.empty(n, c, 9, device='cuda', dtype=torch.float16)
+    got = torch.full((n, ho, wo, c), float('nan'), device='cuda').half()
+    norm, apply, keep = make_norm(c, 1, 0)
+    call('ddf_hip_net_ddf', x, ws, bs, sf, 0.6, parts, n_parts, w1, b1, w2, b2, cf, mid, 0.7, gv, ov, norm, got, n, h, w, c, s,
+         _lib.COMBINE[combine])
+    xc = x.float().permute(0, 3, 1, 2)
+    raw = F.conv2d(xc, ws.float().view(9, c, 1, 1), bs.float(), stride=s)
+    sf_want = (raw - raw.mean(1, keepdim=True)) / (raw.std(1, keepdim=True) + 1e-10) * 0.6
+    cf_want = channel_reference(parts.double().sum(1).cpu() / (h * w), *(t.cpu() for t in (w1, b1, w2, b2)), 3, 0.7, gv.cpu(),
+                                ov.cpu()).float().cuda().view(n, c, 9, 1, 1)
+    taps = sf_want.view(n, 1, 9, ho, wo)
+    comb = cf_want * taps if combine == 'mul' else cf_want + taps
+    window = F.unfold(xc, 3, padding=1, stride=s).view(n, c, 9, (h - 1) // s + 1, (w - 1) // s + 1)[..., :ho, :wo]
+    want = apply((window * comb).sum(2).permute(0, 2, 3, 1)).clamp_min(0)
+    close(got, want, 4e-3 + 4e-3 + 6e-3)     # (what the filter, its spatial and its channel taps may be off)
+
+
 @pytest.mark.parametrize('n,c,mid,n_parts', [(1, 64, 12, 512), (2, 128, 25, 513), (1, 512, 102, 33), (33, 256, 51, 9),
                                              (3, 20, 4, 1030), (2, 70, 14, 17), (70, 64, 12, 1)])
 def test_sum_parts(n, c, mid, n_parts):
