@@ -341,14 +341,15 @@ double rows_cost(const RowsGeom &g, bool ragged, int k, int esz, int vx, int r, 
 // 8 x 64 x 200 x 300 68.8 -> 66.0), and what fits L2 is put together there (3 x 56 x 221 x 133 15.2
 // -> 13.1, 111 -> 63).  Vectors of less than 16 bytes ask more often for the same (8 x 64 x 100 x 150
 // fp16: 11.7 us in strips of 16-byte vectors, 12.3 in a run of 8-byte ones); those of an odd tail,
-// which start at odd elements, are dearer the longer they are.  The shares are fitted over 1434 calls
-// between 0.6 and 1600 MB: their choices are 0.7 % over the better one's time on average, counting
+// which start at odd elements, are dearer the longer they are.  The shares are fitted over 2738 calls
+// between 0.6 and 1600 MB: their choices are 1 % over the best one's time on average, counting
 // instructions alone 3.5 %, whole rows throughout 3.8 %.  25 taps never wait for memory.
 double rows_layout_cost(const Problem &p, const RowsGeom &g, int esz, int vx, int r) {
     const bool wide = vx * esz >= 16;
-    const double instructions = rows_cost(g, g.tail > 0, p.k, esz, vx, r, !wide ? 1.3 : p.d == 1 ? 1.8 : 1.5, 2.0);
+    const double instructions = rows_cost(g, g.tail > 0, p.k, esz, vx, r, !wide ? 1.2 : p.d == 1 ? 1.8 : 1.5, 2.0);
     if (p.k == 5) return instructions;
-    const bool on_lines = g.segs <= 1 || (g.seg_out * vx * esz % 128 == 0 && p.W * esz % 128 == 0);
+    // (64 bytes: what a write to memory holds)
+    const bool on_lines = g.segs <= 1 || (g.seg_out * vx * esz % 64 == 0 && p.W * esz % 64 == 0);
     const double parted = g.halo ? (r == 2 ? 0.35 : 0.02) : on_lines ? 0.0 : 0.3;
     const double bytes = 2.0 * p.N * p.C * p.H * p.W * esz, beyond_l2 = std::max(0.0, 1 - 30e6 / bytes);
     const double memory = bytes / 5800 * ((wide ? 1.1 : esz == 2 ? 1.2 : 1.4) + parted * beyond_l2);
