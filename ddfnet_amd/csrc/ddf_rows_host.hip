@@ -342,8 +342,8 @@ double rows_cost(const RowsGeom &g, bool ragged, int k, int esz, int vx, int r, 
 // -> 13.1, 111 -> 63).  Vectors of less than 16 bytes ask more often for the same (8 x 64 x 100 x 150
 // fp16: 11.7 us in strips of 16-byte vectors, 12.3 in a run of 8-byte ones); those of an odd tail,
 // which start at odd elements, are dearer the longer they are.  The shares are fitted over 2738 calls
-// between 0.6 and 1600 MB: their choices are 1 % over the best one's time on average, counting
-// instructions alone 3.5 %, whole rows throughout 3.8 %.  25 taps never wait for memory.
+// between 0.6 and 1600 MB: their choices are 0.6 % over the best one's time on average, counting
+// instructions alone 3.5 %, whole rows throughout 4.9 %.  25 taps never wait for memory.
 double rows_layout_cost(const Problem &p, const RowsGeom &g, int esz, int vx, int r) {
     const bool wide = vx * esz >= 16;
     const double instructions = rows_cost(g, g.tail > 0, p.k, esz, vx, r, !wide ? 1.2 : p.d == 1 ? 1.8 : 1.5, 2.0);
