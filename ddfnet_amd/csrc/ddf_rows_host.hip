@@ -582,20 +582,29 @@ bool rows_filters_plan(const Problem &p, int dtype, bool fused, RowsGeom *g, int
         if (cut_channels_filters(t, p.N, t.C)) consider(true, 4, 1);
     }
     // The plane as one run of lanes, with the channels split as before if that leaves a workgroup
-    // per CU: where it takes three
-    // tenths of the strips away, or leaves the fullest CU fewer workgroups to walk.  (A CU holds
+    // per CU: where it takes three tenths of the strips away, or leaves the fullest CU fewer
+    // workgroups to walk.  (A CU holds
     // two: 360 of them at 12 x 144 x 80 x 87 take what 480 do, and 4 % more.)  All gradients,
     // strips -> run: fp16 8 x 64 x 200 x 300 106 -> 75 us, 1 x 128 x 180 x 260 34.0 -> 25.8; fp32
     // 4 x 64 x 200 x 300 71 -> 58, 8 x 64 x 100 x 150 47 -> 39, 2 x 100 x 130 x 140 32.1 -> 22.5.
-    // (A ragged cut stays one: see rows_plan.)
+    // Strips of fp32 vectors that end with a line part none of dX's and the features' lines, which
+    // such launches wait for where the features are larger than the L2s: there a run has to take a
+    // quarter of the strips away.  (8 x 96 x 72 x 96 fits: 29.8 us as rows, 24.2 as a run.  32 x 256 x
+    // 224 x 224, 203 strips for 224: 1161 us as rows, 1206 as a run; 4 x 128 x 445 x 448 323 and
+    // 333; 16 x 64 x 88 x 176, 63 for 88: 63.1 and 52.8.  In fp16, at the vector ALU's bound, 16 x
+    // 192 x 221 x 224 takes 328 and 319.)  (A ragged cut stays one: see rows_plan.)
     if (!found) return false;
     const RowsGeom strips = *g;
     best = rows_filters_steps(strips, strips.tail > 0, *vx, *r);
+    const bool on_lines = dtype == DDF_F32 && strips.tail == 0 && p.W * 4 % 64 == 0 &&
+                          p.N * p.C * p.H * p.W * 4 > 32 << 20 &&
+                          (strips.segs <= 1 || strips.seg_out * *vx * 4 % 64 == 0);
     auto consider_run = [&](bool ragged, int tvx, int tr) {
         cut_channels_like(t, strips, p.N);
         if (t.nwork < kCus && !cut_channels_filters(t, p.N, t.C)) return;   // (too few workgroups)
         const double c = rows_filters_steps(t, ragged, tvx, tr);
         if (c > best || (c == best && t.nstrips * 10 > strips.nstrips * 7)) return;
+        if (on_lines && t.nstrips * 4 > strips.nstrips * 3) return;
         best = c;
         *g = t;
         *vx = tvx;

@@ -72,3 +72,19 @@ def test_a_plane_is_a_run_of_lanes_where_that_pays(dtype, shape, k, run):
         assert ('run>' in name) == run, name
         if not run:
             assert 'VX=%d,R=2' % (16 // dtype.itemsize) in name, name
+
+
+@pytest.mark.parametrize('dtype,shape,run', [
+    ('float32', (32, 256, 224, 224), False), ('float32', (4, 128, 445, 448), False),
+    ('float32', (16, 192, 156, 208), False), ('float32', (8, 96, 72, 96), True),
+    ('float32', (16, 64, 88, 176), True),
+    ('float32', (8, 64, 200, 300), True), ('float32', (32, 64, 240, 320), True),
+    ('float16', (16, 192, 221, 224), True), ('float16', (8, 64, 200, 300), True),
+])
+def test_filter_gradients_of_whole_lines_stay_rows(dtype, shape, run):
+    """Strips that end with a line are left for a run of lanes where it takes a quarter of them away, or in cache."""
+    import torch
+    from ddfnet_amd import _lib
+    for need in (_lib.NEED_DCF | _lib.NEED_DSF, _lib.NEED_DX | _lib.NEED_DCF | _lib.NEED_DSF):
+        name = _lib.describe(shape, 3, 1, 1, 'mul', getattr(torch, dtype), need)
+        assert ('run>' in name) == run, name
