@@ -177,9 +177,11 @@ __device__ __forceinline__ float rows_total(float v) {
 __device__ __forceinline__ void load_to_lds(uint32_t lds, const void *p) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
-// The same from a uniform address and a lane's offset.
+// The same from a uniform address and a lane's offset.  (A scalar register that a vector instruction
+// has written - a spilled one that comes back by v_readlane - may be read by a vector memory instruction
+// five wait states later; the compiler does not see one in here.)
 __device__ __forceinline__ void load_to_lds(uint32_t lds, const char *base, int offset) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
 // This wave's are there.
 __device__ __forceinline__ void loads_to_lds_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
