@@ -815,6 +815,32 @@ int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_ne
     return net_result(ddf::net_conv_pair(a, side, (hipStream_t)stream), "ddf_hip_net_conv_pair launch");
 }
 
+int64_t ddf_hip_net_conv_chain_parts(int64_t N, int64_t H, int64_t W, int64_t C, int64_t side_C, int64_t O, int64_t next_O) {
+    if (N < 1 || H < 1 || W < 1 || C < 1 || side_C < 0 || O < 1 || next_O < 1 || H * W >= (1ll << 31)) return 0;
+    if (!ddf::net_chain_covers(N * H * W, C, side_C, O, next_O)) return 0;
+    return ddf::net_chain_pool_slots(N * H * W, (int)(H * W));
+}
+
+int ddf_hip_net_conv_chain(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
+                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
+                           int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm,
+                           void *next, float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O,
+                           int64_t next_O, void *stream) {
+    if (N < 0 || H < 1 || W < 1 || C < 1 || side_C < 0 || O < 1 || next_O < 1 || H * W >= (1ll << 31))
+        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_conv_chain: bad sizes");
+    if (!features || !weight || !output || !next_weight || !next || !pool_parts || !net_norm_ok(norm) || !net_norm_ok(next_norm) ||
+        !net_norm_ok(side_norm) || (side_C ? !side_features || !side_weight : !residual))
+        return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    if (N == 0) return DDF_OK;
+    const int64_t M = N * H * W;
+    if (!ddf::net_chain_covers(M, C, side_C, O, next_O))
+        return fail(DDF_ERR_UNSUPPORTED, "ddf_hip_net_conv_chain: sizes not covered");
+    const ddf::NetChain a{features, weight, residual, side_features, side_weight, next_weight, output, next, pool_parts,
+                          net_norm(norm), net_norm(side_norm), net_norm(next_norm), M, (int)C, (int)side_C, (int)O,
+                          (int)next_O, (int)(H * W), 0, 0};
+    return net_result(ddf::net_chain(a, (hipStream_t)stream), "ddf_hip_net_conv_chain launch");
+}
+
 int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,
                      int64_t H, int64_t W, void *stream) {
     if (N < 0 || H < 1 || W < 1) return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_stem: bad sizes");

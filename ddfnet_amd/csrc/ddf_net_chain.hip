@@ -1,0 +1,404 @@
+// A bottleneck's last 1x1 convolution and the next one's first in one launch (DDF-ResNet
+// inference, fp16, channels-last; ddf_resnet.py:34-111 of the reference composes them).
+#include <numeric>
+
+#include "ddf_net_device.h"
+
+namespace ddf {
+namespace {
+using namespace net;
+using rows::plane_rsrc;
+
+// out (M, N) = relu(norm(x . w) + res), or relu(norm(x . w) + norm'(side . side_w));
+// next (M, N2) = relu(norm''(out . w2)), and next's sums over its pixels.
+//
+// The wide result is written once and not read back: a workgroup takes 32 * P pixels of all channels,
+// goes over the wide channels by kChunk, and each chunk is the next block of the summed dimension of
+// the second product, whose sums stay in registers.  A wave has 32 pixels: their x in registers as the
+// operand of every chunk, a tile of LDS for the chunk's results, which are rounded, meet the residual
+// and leave as whole 128-byte lines from there, and are read as the second product's operand.  The
+// weights of a chunk are shared: w's rows come in while the second product of the chunk before is
+// made, w2's during the first product, straight to LDS, two barriers a chunk.
+// Memory bounds it at 56 x 56: 514 MB in 84 us behind the filter's launch (6.1 TB/s, the last-level cache
+// has part of the residual; 103 us, a copy's rate, with everything from memory).  us, two launches /
+// this, batch 128: 56 x 56 x 64 -> 256 -> 64 122 / 84, with the projection 141 / 95, -> 128 140 / 105, 28 x 28 x
+// 128 -> 512 -> 128 68 / 62; batch 16: 24.0 / 16.0, 26.5 / 20.4, 24.2 / 18.4.  Tried there and no faster: the first product of the
+// next chunk beside the second one of this, one barrier's work (65 -> 68 us at 28 x 28), waves in
+// pairs that split the channels (66), 64 pixels a workgroup (73); at 14 x 14 x 256 -> 1024 -> 256 such pairs take
+// 48 us where the two launches take 51, LDS bound (each weight fragment feeds one product of a wave).
+constexpr int kChunk = 64, kTilePitch = kChunk + 8;
+constexpr int kChainWaves = kThreads / kWave, kChainRows = 32 * kChainWaves;    // a wave: 32 pixels
+
+template <int K, int K2, int N2>
+struct ChainLds {    // halves; K2: channels of the side product, 0: none
+    static constexpr int w = 0, wd = w + kChunk * K, w2 = wd + kChunk * K2, tile = w2 + N2 * kChunk,
+                         norms = tile + kChainRows * kTilePitch;
+    // at the end: a wave's tile of next's results, and the sums over its pixels
+    static constexpr int red = kChainRows * kTilePitch;
+    static_assert(red + kChainWaves * N2 * 2 <= norms, "next's results fit in front of the norms");
+    // scale, shift, what a sum starts with; of the wide channels (and of the side product), of next's
+    static constexpr int bytes(int N) { return norms * 2 + (N * (K2 ? 5 : 3) + N2 * 3) * 4; }
+};
+
+// chunk c of row r of a weight tile sits in place c ^ turn (see k_net_conv: sixteen lanes that LDS serves at
+// once meet all of its banks)
+template <int CH>
+__device__ __forceinline__ int turn(int r) { return CH == 8 ? (r >> 1) & 7 : r & 15; }
+
+// ROWS rows of LEN halves, `pitch` halves apart in memory, to LDS by all threads.
+template <int ROWS, int LEN>
+struct StageRows {
+    static constexpr int CH = LEN / 8, STEP = kThreads / CH, COUNT = ROWS / STEP;
+    static_assert(kThreads % CH == 0 && ROWS % STEP == 0 && STEP % 16 == 0);
+    int offset;
+    __device__ __forceinline__ StageRows(int tid, int pitch) {
+        const int r = tid / CH, c = (tid % CH) ^ turn<CH>(r);
+        offset = (r * pitch + c * 8) * 2;
+    }
+    __device__ __forceinline__ void load(uint32_t lds, int wave, const _Float16 *base, int pitch) const {
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i)
+            load_to_lds(lds + wave * (kWave * 16) + i * (kThreads * 16), reinterpret_cast<const char *>(base + (int64_t)i * STEP * pitch), offset);
+    }
+};
+
+template <int K, int K2, int N2, int WPS>
+__global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
+    typedef ChainLds<K, K2, N2> L;
+    constexpr int BM = kChainRows;
+    constexpr int TA = kChunk / 32, TB = N2 / 32, SB = N2 / kChunk;    // tiles of 32 channels; chunks of next's channels
+    constexpr int RV = 4;                          // vectors of a chunk that a lane takes on their way out
+    extern __shared__ __align__(16) _Float16 chain_smem[];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int l32 = lane & 31, hi = lane >> 5;
+    const int block = xcd_block(blockIdx.x, a.tiles);
+    if (block >= a.tiles) return;
+    const int64_t m0 = (int64_t)block * BM;
+    const int rows = (int)min((int64_t)BM, a.M - m0), N = a.N, chunks = N / kChunk;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) _Float16 *)chain_smem;
+    float *const norms = reinterpret_cast<float *>(chain_smem + L::norms);
+    float *const scale = norms, *const shift = norms + N, *const start = norms + 2 * N;
+    float *const side_scale = norms + 3 * N, *const side_shift = norms + 4 * N;
+    float *const scale2 = norms + (K2 ? 5 : 3) * N, *const shift2 = scale2 + N2, *const start2 = shift2 + N2;
+
+    // (rows past the last pixel read zeros and are not stored: every one of these loads and stores is
+    // issued whatever the tile, the waits below count them)
+    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(static_cast<const _Float16 *>(a.x) + m0 * K, rows * K * 2);
+    const __amdgpu_buffer_rsrc_t rr = plane_rsrc(K2 ? nullptr : static_cast<const _Float16 *>(a.res) + m0 * N, K2 ? 0 : rows * N * 2);
+    const __amdgpu_buffer_rsrc_t orr = plane_rsrc(static_cast<_Float16 *>(a.out) + m0 * N, rows * N * 2);
+    half8_t xv[K / 16], dv[K2 ? K2 / 16 : 1];
+#pragma unroll
+    for (int k = 0; k < K / 16; ++k)
+        xv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(xr, ((wave * 32 + l32) * K + hi * 8) * 2, k * 32, 0));
+    if constexpr (K2 > 0) {
+        const __amdgpu_buffer_rsrc_t dr = plane_rsrc(static_cast<const _Float16 *>(a.side) + m0 * K2, rows * K2 * 2);
+#pragma unroll
+        for (int k = 0; k < K2 / 16; ++k)
+            dv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(dr, ((wave * 32 + l32) * K2 + hi * 8) * 2, k * 32, 0));
+    }
+    // Without a BatchNorm a bias is part of the sum, elsewhere the sum is rounded first (see k_net_conv).
+    auto put_norm = [&](const NetNorm &n, bool in_sum, int c, float *sc, float *sh, float *st) __attribute__((always_inline)) {
+        Affine<1> aff;
+        aff.request(n, c, !in_sum);
+        float s1[1], s2[1];
+        aff.finish(n, s1, s2);
+        sc[c] = s1[0];
+        sh[c] = s2[0];
+        if (st) st[c] = in_sum ? (float)static_cast<const _Float16 *>(n.conv_bias)[c] : 0.f;
+    };
+    const bool in_sum = !K2 && !a.norm.var && a.norm.conv_bias, in_sum2 = !a.norm2.var && a.norm2.conv_bias;
+    for (int c = tid; c < N; c += kThreads) {
+        put_norm(a.norm, in_sum, c, scale, shift, start);
+        if constexpr (K2 > 0) put_norm(a.side_norm, false, c, side_scale, side_shift, nullptr);
+    }
+    for (int c = tid; c < N2; c += kThreads) put_norm(a.norm2, in_sum2, c, scale2, shift2, start2);
+
+    const StageRows<kChunk, K> sw(tid, K);
+    const StageRows<kChunk, K2 ? K2 : K> sd(tid, K2);
+    const StageRows<N2, kChunk> sw2(tid, N);
+    const _Float16 *const w = static_cast<const _Float16 *>(a.w), *const wd = static_cast<const _Float16 *>(a.side_w),
+                   *const w2 = static_cast<const _Float16 *>(a.w2);
+    auto stage_w = [&](int j) __attribute__((always_inline)) {
+        sw.load(lds0 + L::w * 2, wave, w + (int64_t)j * kChunk * K, K);
+        if constexpr (K2 > 0) sd.load(lds0 + L::wd * 2, wave, wd + (int64_t)j * kChunk * K2, K2);
+    };
+    // a lane's vectors on their way out: eight channels of every eighth pixel
+    const int c8 = lane & 7, px0 = wave * 32 + (lane >> 3);
+    rows_u4 rv[RV];
+    auto residual = [&](int j) __attribute__((always_inline)) {
+        if constexpr (K2 == 0) {
+#pragma unroll
+            for (int i = 0; i < RV; ++i)
+                rv[i] = __builtin_amdgcn_raw_buffer_load_b128(rr, (px0 * N + c8 * 8) * 2, (i * 8 * N + j * kChunk) * 2, 0);
+        }
+    };
+    stage_w(0);
+    residual(0);
+
+    // a lane's column of a 32 x 32 step's result is pixel l32, rows (channels) 8 * q + 4 * hi + 0..3 in
+    // registers 4 * q ..
+    auto channel = [&](int t, int q) { return t * 32 + 8 * q + 4 * hi; };
+    _Float16 *const tile = chain_smem + L::tile + wave * 32 * kTilePitch;
+    float16_t sum2[TB];
+    auto clear = [](float16_t &s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = 0.f;
+    };
+#pragma unroll
+    for (int t = 0; t < TB; ++t) clear(sum2[t]);
+    auto product = [&](const _Float16 *weights, auto len, const auto &v, float16_t(&s)[TA]) __attribute__((always_inline)) {
+        constexpr int LEN = decltype(len)::value;
+#pragma unroll
+        for (int k = 0; k < LEN / 16; ++k)
+#pragma unroll
+            for (int t = 0; t < TA; ++t) {
+                const int r = t * 32 + l32;
+                const half8_t wv = *reinterpret_cast<const half8_t *>(weights + r * LEN + ((k * 2 + hi) ^ turn<LEN / 8>(r)) * 8);
+                s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv, v[k], s[t], 0, 0, 0);
+            }
+    };
+    float one = 1.f;
+    asm volatile("" : "+v"(one));    // (value * one + f: a conversion less than value + f)
+
+    for (int j = 0; j < chunks; ++j) {
+        // w's rows are there (the residual may be on its way); everybody is done with w2's
+        arrive<K2 ? 0 : RV>();
+        sw2.load(lds0 + L::w2 * 2, wave, w2 + j * kChunk, N);
+        half4_t side[K2 ? TA : 1][4];
+        float16_t sum[TA];
+        if constexpr (K2 > 0) {
+#pragma unroll
+            for (int t = 0; t < TA; ++t) clear(sum[t]);
+            product(chain_smem + L::wd, std::integral_constant<int, K2 ? K2 : 16>{}, dv, sum);
+#pragma unroll
+            for (int t = 0; t < TA; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4_t sc = *reinterpret_cast<const float4_t *>(side_scale + j * kChunk + channel(t, q));
+                    const float4_t sh = *reinterpret_cast<const float4_t *>(side_shift + j * kChunk + channel(t, q));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) side[t][q][e] = (_Float16)fmaf((float)(_Float16)sum[t][4 * q + e], sc[e], sh[e]);
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < TA; ++t) clear(sum[t]);
+        if (in_sum) {
+#pragma unroll
+            for (int t = 0; t < TA; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4_t b = *reinterpret_cast<const float4_t *>(start + j * kChunk + channel(t, q));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[t][4 * q + e] = b[e];
+                }
+        }
+        product(chain_smem + L::w, std::integral_constant<int, K>{}, xv, sum);
+        // to the tile: sums rounded to fp16, with a side product the results
+#pragma unroll
+        for (int t = 0; t < TA; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                half4_t v;
+                if constexpr (K2 > 0) {
+                    const float4_t sc = *reinterpret_cast<const float4_t *>(scale + j * kChunk + channel(t, q));
+                    const float4_t sh = *reinterpret_cast<const float4_t *>(shift + j * kChunk + channel(t, q));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float f = fmaf((float)(_Float16)sum[t][4 * q + e], sc[e], sh[e]);
+                        f = fmaf((float)side[t][q][e], one, f);
+                        asm volatile("" : "+v"(f));
+                        v[e] = (_Float16)f;
+                    }
+                    v = __builtin_elementwise_maximum(v, half4_t{0, 0, 0, 0});
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = (_Float16)sum[t][4 * q + e];
+                }
+                *reinterpret_cast<half4_t *>(tile + l32 * kTilePitch + channel(t, q)) = v;
+            }
+        asm volatile("" ::: "memory");    // (a wave's LDS operations keep their order)
+        float sc[8], sh[8];
+        if constexpr (K2 == 0) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4_t s = *reinterpret_cast<const float4_t *>(scale + j * kChunk + c8 * 8 + h * 4);
+                const float4_t o = *reinterpret_cast<const float4_t *>(shift + j * kChunk + c8 * 8 + h * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sc[4 * h + e] = s[e];
+                    sh[4 * h + e] = o[e];
+                }
+            }
+        }
+        half8_t v[RV];
+#pragma unroll
+        for (int i = 0; i < RV; ++i)
+            v[i] = *reinterpret_cast<const half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8);
+#pragma unroll
+        for (int i = 0; i < RV; ++i) {
+            if constexpr (K2 == 0) {
+                const half8_t r = __builtin_bit_cast(half8_t, rv[i]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float f = fmaf((float)v[i][e], sc[e], sh[e]);
+                    f = fmaf((float)r[e], one, f);
+                    asm volatile("" : "+v"(f));    // (rounded to fp32 first in every instance)
+                    v[i][e] = (_Float16)f;
+                }
+                v[i] = __builtin_elementwise_maximum(v[i], half8_t{0, 0, 0, 0, 0, 0, 0, 0});
+                *reinterpret_cast<half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8) = v[i];
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, v[i]), orr, (px0 * N + c8 * 8) * 2,
+                                                   (i * 8 * N + j * kChunk) * 2, 0);
+        }
+        // w2's rows are there; everybody is done with w's
+        arrive<RV>();
+        if (j + 1 < chunks) {
+            stage_w(j + 1);
+            residual(j + 1);
+        }
+#pragma unroll
+        for (int k = 0; k < kChunk / 16; ++k) {
+            const half8_t pv = *reinterpret_cast<const half8_t *>(tile + l32 * kTilePitch + (k * 2 + hi) * 8);
+#pragma unroll
+            for (int t = 0; t < TB; ++t) {
+                const int r = t * 32 + l32;
+                const half8_t wv = *reinterpret_cast<const half8_t *>(chain_smem + L::w2 + r * kChunk + ((k * 2 + hi) ^ turn<kChunk / 8>(r)) * 8);
+                sum2[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv, pv, sum2[t], 0, 0, 0);
+            }
+        }
+    }
+
+    // next's results, kChunk channels of the wave's pixels at a time, through a tile of its own
+    __syncthreads();
+    _Float16 *const last = chain_smem + wave * 32 * kTilePitch;
+    const __amdgpu_buffer_rsrc_t nr = plane_rsrc(static_cast<_Float16 *>(a.next) + m0 * N2, rows * N2 * 2);
+    half8_t v[SB][4];
+#pragma unroll
+    for (int s = 0; s < SB; ++s) {
+        const int c0 = s * kChunk;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float4_t b = {0.f, 0.f, 0.f, 0.f};
+                if (in_sum2) b = *reinterpret_cast<const float4_t *>(start2 + c0 + t * 32 + 8 * q + 4 * hi);
+                half4_t h;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[e] = (_Float16)(sum2[s * 2 + t][4 * q + e] + b[e]);
+                *reinterpret_cast<half4_t *>(last + l32 * kTilePitch + t * 32 + 8 * q + 4 * hi) = h;
+            }
+        asm volatile("" ::: "memory");
+        float sc[8], sh[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            sc[e] = scale2[c0 + c8 * 8 + e];
+            sh[e] = shift2[c0 + c8 * 8 + e];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int px = i * 8 + (lane >> 3);
+            v[s][i] = *reinterpret_cast<const half8_t *>(last + px * kTilePitch + c8 * 8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float f = fmaf((float)v[s][i][e], sc[e], sh[e]);
+                asm volatile("" : "+v"(f));
+                v[s][i][e] = (_Float16)f;
+            }
+            v[s][i] = __builtin_elementwise_maximum(v[s][i], half8_t{0, 0, 0, 0, 0, 0, 0, 0});
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, v[s][i]), nr, ((wave * 32 + px) * N2 + c0 + c8 * 8) * 2, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    }
+    // Sums over the tile's pixels of each sample it touches, to the sample's slot for this tile; the
+    // tile with a sample's last pixel clears the slots that sample does not use (as k_net_conv's).
+    float *const red = reinterpret_cast<float *>(chain_smem + L::red);    // [wave][N2]
+    const int first = (int)m0, end = (int)min(m0 + BM, a.M), n_last = (end - 1) / a.npix;
+    for (int n = first / a.npix; n <= n_last; ++n) {
+        const int lo = n * a.npix - first, up = lo + a.npix;
+#pragma unroll
+        for (int s = 0; s < SB; ++s) {
+            float sum[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = wave * 32 + i * 8 + (lane >> 3);
+                const bool in = r >= lo && r < up && r < rows;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sum[e] += in ? (float)v[s][i][e] : 0.f;
+            }
+            float half[4], pair[2];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[e] = add_permuted<0x128 /* row_ror:8 */>(sum[e]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) half[e] = add_swapped32(sum[e], sum[e + 4]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) pair[e] = add_swapped16(half[e], half[e + 2]);
+            if (!(lane & 8)) {
+                typedef float float2_t __attribute__((ext_vector_type(2)));
+                *reinterpret_cast<float2_t *>(red + wave * N2 + s * kChunk + c8 * 8 + (lane >> 4) * 2) = float2_t{pair[0], pair[1]};
+            }
+        }
+        __syncthreads();
+        for (int c = tid; c < N2; c += kThreads) {
+            float *to = a.pool + (int64_t)n * a.pool_slots * N2 + c;
+            int slot = block - (int)((int64_t)n * a.npix / BM);
+            float total = red[c];
+#pragma unroll
+            for (int k = 1; k < kChainWaves; ++k) total += red[k * N2 + c];
+            to[(int64_t)slot * N2] = total;
+            if (up <= end - first)
+                while (++slot < a.pool_slots) to[(int64_t)slot * N2] = 0.f;
+        }
+        if (n < n_last) __syncthreads();
+    }
+}
+
+template <int K, int K2, int N2, int WPS>
+hipError_t launch_chain(const NetChain &a, hipStream_t st) {
+    const int lds = ChainLds<K, K2, N2>::bytes(a.N);
+    hipLaunchKernelGGL((k_net_chain<K, K2, N2, WPS>), dim3(xcd_grid(a.tiles)), dim3(kThreads), lds, st, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// Whether the two convolutions are one launch: three quarters of a workgroup per compute unit at least (us, two
+// launches / one: 8 x 56 x 56, 196 workgroups, 14.5 / 14.0 and 18.7 / 17.0 with the projection; 16 x 28 x 28, 98 of
+// them, 15.8 / 23.3; 32 x 28 x 28, 196, 26 / 23); where 256 channels follow, two workgroups at most, which
+// then run side by side (28 x 28 x 128 -> 512 -> 256: 32 images 30.1 / 28.9, 64 47.8 / 43.8, 96, 588 workgroups, 63.9 / 70.3).
+bool net_chain_covers(int64_t M, int64_t K, int64_t side, int64_t N, int64_t N2) {
+    constexpr int kFew = 192, kSideBySide = 512;
+    if (N % kChunk || N < kChunk || N > 2048 || M > INT32_MAX - 256) return false;
+    const int64_t tiles = cdiv(M, kChainRows);
+    if (tiles < kFew) return false;
+    if (side) return K == 64 && side == 64 && N2 == 64;
+    if (K == 64) return N2 == 64 || N2 == 128;
+    return K == 128 && (N2 == 128 || (N2 == 256 && tiles <= kSideBySide));
+}
+
+int net_chain_pool_slots(int64_t M, int npix) {
+    const int start = M > npix ? kChainRows - std::gcd(kChainRows, npix) : 0;
+    return (start + npix - 1) / kChainRows + 1;
+}
+
+// (the waves per SIMD are what registers and LDS leave room for)
+hipError_t net_chain(NetChain a, hipStream_t st) {
+    if (a.M == 0) return hipSuccess;
+    if (!net_chain_covers(a.M, a.K, a.side_K, a.N, a.N2)) return hipErrorNotSupported;
+    a.tiles = (int)cdiv(a.M, kChainRows);
+    a.pool_slots = net_chain_pool_slots(a.M, a.npix);
+#define DDF_CHAIN(K_, SIDE_, N2_, WPS_) \
+    if (a.K == K_ && a.side_K == SIDE_ && a.N2 == N2_) return launch_chain<K_, SIDE_, N2_, WPS_>(a, st);
+    DDF_CHAIN(64, 64, 64, 3)
+    DDF_CHAIN(64, 0, 64, 4)
+    DDF_CHAIN(64, 0, 128, 3)
+    DDF_CHAIN(128, 0, 128, 2)
+    DDF_CHAIN(128, 0, 256, 2)
+#undef DDF_CHAIN
+    return hipErrorNotSupported;
+}
+
+}  // namespace ddf

@@ -139,20 +139,30 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
     int64_t wide = 0, narrow = 0, taps = 0, filters = 0, parts = 0, totals = 0;
     // (more partial sums of the pooled vectors than the channel branch is left become totals)
     struct Parts { int count; bool summed; };
-    auto parts_of = [n](const NetBlock &b, int64_t h, int64_t w, int64_t c) {
-        const int64_t count = ddf_hip_net_conv_pool_parts(n, h, w, c, b.width);
+    // (0: b's last convolution and the first one of the block behind it are launches of their own)
+    auto chain_parts = [n, &p](size_t i, int64_t ho, int64_t wo, int64_t c) -> int64_t {
+        const NetBlock &b = p.blocks[i];
+        const bool down = b.down.t[0].defined();
+        if (i + 1 == p.blocks.size() || (down && b.stride != 1)) return 0;
+        return ddf_hip_net_conv_chain_parts(n, ho, wo, b.width, down ? c : 0, b.conv3.t[0]->size(0), p.blocks[i + 1].width);
+    };
+    // chained: what the launch that made b's first results has left, 0 where that is one of its own
+    auto parts_of = [n](const NetBlock &b, int64_t h, int64_t w, int64_t c, int64_t chained) {
+        const int64_t count = chained ? chained : ddf_hip_net_conv_pool_parts(n, h, w, c, b.width);
         return Parts{(int)count, count > ddf_hip_net_parts_left(n, b.width, b.mid)};
     };
     {
-        int64_t h = h0 / 4, w = w0 / 4, c = 64;
+        int64_t h = h0 / 4, w = w0 / 4, c = 64, chained = 0;
         wide = n * h * w * 64;
-        for (const NetBlock &b : p.blocks) {
+        for (size_t i = 0; i < p.blocks.size(); ++i) {
+            const NetBlock &b = p.blocks[i];
             const int64_t ho = h / b.stride, wo = w / b.stride;
             narrow = std::max(narrow, n * h * w * b.width);
             wide = std::max(wide, n * ho * wo * b.conv3.t[0]->size(0));
             taps = std::max(taps, n * ho * wo * 12);
             filters = std::max(filters, n * b.width * 9);
-            const Parts of = parts_of(b, h, w, c);
+            const Parts of = parts_of(b, h, w, c, chained);
+            chained = chain_parts(i, ho, wo, c);
             parts = std::max(parts, n * b.width * of.count);
             if (of.summed) totals = std::max(totals, n * b.width);
             c = b.conv3.t[0]->size(0);
@@ -173,12 +183,16 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
         py::gil_scoped_release release;    // (a network's launches take a while)
         ddf_net_norm_t nm = p.stem.norm();
         covered(ddf_hip_net_stem(x.data_ptr(), p.stem.t[0]->data_ptr(), &nm, cur, n, h0, w0, st));
-        int64_t h = h0 / 4, w = w0 / 4, c = 64;
-        for (const NetBlock &b : p.blocks) {
+        int64_t h = h0 / 4, w = w0 / 4, c = 64, chained = 0;
+        for (size_t i = 0; i < p.blocks.size(); ++i) {
+            const NetBlock &b = p.blocks[i];
             const int64_t ho = h / b.stride, wo = w / b.stride, width = b.width, wide_c = b.conv3.t[0]->size(0);
-            nm = b.conv1.norm();
-            covered(ddf_hip_net_conv_pool(cur, b.conv1.t[0]->data_ptr(), &nm, t1, pp, n, h, w, c, width, 1, st));
-            const Parts of = parts_of(b, h, w, c);
+            if (!chained) {
+                nm = b.conv1.norm();
+                covered(ddf_hip_net_conv_pool(cur, b.conv1.t[0]->data_ptr(), &nm, t1, pp, n, h, w, c, width, 1, st));
+            }
+            const Parts of = parts_of(b, h, w, c, chained);
+            chained = chain_parts(i, ho, wo, c);
             if (of.summed) covered(ddf_hip_net_sum_parts(pp, of.count, pt, n, width, st));
             nm = b.bn2.norm();
             covered(ddf_hip_net_ddf(
@@ -187,8 +201,17 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
                 cf, b.mid, b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset), &nm, t2, n, h, w, width,
                 b.stride, b.combine, st));
             nm = b.conv3.norm();
-            if (b.down.t[0].defined()) {
-                const ddf_net_norm_t down = b.down.norm();
+            const ddf_net_norm_t down = b.down.norm();
+            if (chained) {
+                const NetBlock &next = p.blocks[i + 1];
+                const ddf_net_norm_t nm1 = next.conv1.norm();
+                const bool side = b.down.t[0].defined();
+                void *to = side ? other : cur;
+                covered(ddf_hip_net_conv_chain(t2, b.conv3.t[0]->data_ptr(), &nm, side ? nullptr : cur, side ? cur : nullptr,
+                                               ptr_or_null(b.down.t[0]), &down, side ? c : 0, to, next.conv1.t[0]->data_ptr(),
+                                               &nm1, t1, pp, n, ho, wo, width, wide_c, next.width, st));
+                if (side) std::swap(cur, other);
+            } else if (b.down.t[0].defined()) {
                 covered(ddf_hip_net_conv_pair(t2, b.conv3.t[0]->data_ptr(), &nm, width, cur,
                                                    b.down.t[0]->data_ptr(), &down, h, w, c, b.stride, other, n, wide_c, 1,
                                                    st));

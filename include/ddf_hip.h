@@ -368,6 +368,10 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *           pixels of each sample in ddf_hip_net_conv_pool_parts parts (such partial sums): one
  *           or so per 16, 64 or 128 pixels.  Of more than ddf_hip_net_parts_left(N, C, mid) the
  *           branches are faster from their totals
+ *   conv_chain  conv (stride 1, residual; side_C > 0: conv_pair of stride 1 instead) and conv_pool of its
+ *           results with next_weight (next_O, O), both with ReLU, in one launch that leaves
+ *           ddf_hip_net_conv_chain_parts partial sums (0: sizes that want the two calls).  residual may
+ *           be output; next overlaps neither, and no input
  *   sum_parts  totals (N, C) of n_parts such partial sums per sample and channel
  *   branches  both filter branches in one launch: the spatial one, and the channel one of
  *           ddf_hip_channel_branch_parts (3x3 taps) from the partial sums of conv_pool; sizes as
@@ -394,6 +398,12 @@ int ddf_hip_net_conv_pair(const void *features, const void *weight, const ddf_ne
                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
                           int64_t H, int64_t W, int64_t side_C, int stride, void *output, int64_t N, int64_t O,
                           int relu, void *stream);
+int64_t ddf_hip_net_conv_chain_parts(int64_t N, int64_t H, int64_t W, int64_t C, int64_t side_C, int64_t O, int64_t next_O);
+int ddf_hip_net_conv_chain(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
+                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
+                           int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm,
+                           void *next, float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O,
+                           int64_t next_O, void *stream);
 int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,
                      int64_t H, int64_t W, void *stream);
 int ddf_hip_net_spatial(const void *features, const void *weight, const void *bias, void *spatial_filter,

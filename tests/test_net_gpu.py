@@ -230,6 +230,47 @@ def test_conv_pool(n, h, w, c, o):
     assert (total - want.double().sum((1, 2))).abs().max() <= 1e-6 * want.double().abs().sum((1, 2)).max() + 1e-30
 
 
+@pytest.mark.parametrize('n,h,w,c,side,o,next_o,bn', [
+    (8, 56, 56, 64, 0, 256, 64, 1), (29, 47, 49, 64, 0, 256, 64, 1),       # samples that end inside tiles
+    (21, 56, 56, 64, 64, 256, 64, 1), (3, 151, 149, 64, 64, 64, 64, 1),    # a projection; one chunk
+    (70, 31, 31, 64, 0, 192, 128, 1), (84, 28, 28, 128, 0, 512, 128, 1),
+    (60, 28, 28, 128, 0, 512, 256, 1), (1, 199, 199, 128, 0, 128, 256, 1),
+    (1100, 8, 8, 64, 0, 256, 64, 0), (70000, 1, 1, 128, 0, 128, 128, 0),   # folded BatchNorm; samples of a tile, of a pixel
+    (700, 6, 6, 64, 64, 128, 64, 0),
+])
+def test_conv_chain(n, h, w, c, side, o, next_o, bn):
+    """The two convolutions of one launch: what the two calls leave, and the sums over the pixels."""
+    torch.manual_seed(c + o + next_o)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    wt, ws, wn = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((o, c), (o, side or 1), (next_o, o)))
+    norm, _, keep = make_norm(o, bn, 1)
+    norm_s, _, keep_s = make_norm(o, bn, 1)
+    norm_n, _, keep_n = make_norm(next_o, bn, 1)
+    xs = torch.randn(n, h, w, side, device='cuda').half() if side else None
+    res = None if side else torch.randn(n, h, w, o, device='cuda').half()
+    want = torch.empty(n, h, w, o, device='cuda', dtype=torch.float16)
+    if side:
+        call('ddf_hip_net_conv_pair', x, wt, norm, c, xs, ws, norm_s, h, w, side, 1, want, n, o, 1)
+    else:
+        call('ddf_hip_net_conv', x, wt, norm, res, want, n, h, w, c, o, 1, 1)
+    want_next = torch.empty(n, h, w, next_o, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_conv', want, wn, norm_n, None, want_next, n, h, w, o, next_o, 1, 1)
+    count = _lib.lib().ddf_hip_net_conv_chain_parts(n, h, w, c, side, o, next_o)
+    assert count > 0
+    parts = torch.full((n, count + 1, next_o), float('nan'), device='cuda')
+    out = torch.empty_like(want) if side else res     # (in place where it may be)
+    got_next = torch.empty_like(want_next)
+    call('ddf_hip_net_conv_chain', x, wt, norm, res, xs, ws if side else None, norm_s if side else None, side, out, wn, norm_n,
+         got_next, parts, n, h, w, c, o, next_o)
+    assert torch.equal(out, want)
+    # (a bias without a BatchNorm joins the sum last instead of first: a rounding of fp32 below one of fp16)
+    close(got_next, want_next, 0 if bn else 1e-3)
+    assert parts.view(-1)[n * count * next_o:].isnan().all()
+    total = parts.view(-1)[:n * count * next_o].view(n, count, next_o).double().sum(1)
+    # (fp32 sums of at most h * w terms of one sign)
+    assert (total - got_next.double().sum((1, 2))).abs().max() <= 1e-6 * got_next.double().abs().sum((1, 2)).max() + 1e-30
+
+
 @pytest.mark.parametrize('n,h,w,c,s,mid,n_parts', [
     (1, 56, 56, 64, 1, 12, 49), (70, 6, 10, 64, 2, 12, 3), (300, 4, 4, 64, 1, 12, 1),     # samples past one per compute unit
     (3, 9, 13, 128, 1, 25, 8), (2, 4, 6, 128, 2, 25, 9),
