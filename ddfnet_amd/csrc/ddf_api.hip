@@ -225,8 +225,8 @@ int up_backward_typed(const ddf::Problem &p, int scale, const void *go, const vo
     T *parts = reinterpret_cast<T *>(base + w.lattices);
     const int64_t n_x = p.N * p.C * p.H * p.W;
     const int branches = scale * scale;
-    hipError_t err = ddf::up_split_lattices<T>((const T *)go, lat, p.N * p.C, p.H, p.W, scale, stream);
-    if (err != hipSuccess) return fail_hip(err, "ddf_hip_up_backward split launch");
+    hipError_t err;
+    bool split = false;
 
     // All branches as one batch of scale*scale * N samples that share the features:
     // a handful of launches that fill the machine, instead of three or four small
@@ -238,21 +238,27 @@ int up_backward_typed(const ddf::Problem &p, int scale, const void *go, const vo
         T *dcf_all = w.dcf_all ? reinterpret_cast<T *>(q) : nullptr; q += w.dcf_all;
         T *dsf_all = w.dsf_all ? reinterpret_cast<T *>(q) : nullptr; q += w.dsf_all;
         const int64_t n_cf = p.N * p.C * p.kk, n_sf = p.N * p.kk * p.H * p.W;
-        err = ddf::up_gather_filters<T>(cfs, sfs, cf_all, sf_all, n_cf, n_sf, branches, stream);
-        if (err != hipSuccess) return fail_hip(err, "ddf_hip_up_backward gather launch");
+        err = ddf::up_prepare<T>((const T *)go, lat, p.N * p.C, p.H, p.W, scale, cfs, sfs, cf_all, sf_all, n_cf, n_sf, stream);
+        if (err != hipSuccess) return fail_hip(err, "ddf_hip_up_backward split launch");
         const ddf::Problem pb = ddf::make_problem(p.N * branches, p.C, p.H, p.W, p.k, p.d, 1,
                                                   p.mul ? DDF_MUL : DDF_ADD);
+        ddf::FilterParts<T> left;
         err = ddf::rows_backward_shared_features<T>(
             pb, (int)p.N, lat, (const T *)x, cf_all, sf_all, (need & DDF_NEED_DX) ? parts : nullptr,
-            dcf_all, dsf_all, w.batch_ws ? q : nullptr, need, stream);
+            dcf_all, dsf_all, w.batch_ws ? q : nullptr, need, stream, &left);
         if (err == hipSuccess) {
             err = ddf::up_finish<T>((need & DDF_NEED_DX) ? parts : nullptr, (T *)dx, n_x, branches,
-                                    dcf_all, dsf_all, dcfs, dsfs, n_cf, n_sf, stream);
+                                    dcf_all, dsf_all, left, dcfs, dsfs, p.N, p.C, p.kk, p.H * p.W, stream);
             if (err != hipSuccess) return fail_hip(err, "ddf_hip_up_backward finish launch");
             return DDF_OK;
         }
-        // (e.g. features not 16-byte aligned: nothing was launched, take the other route)
+        // (e.g. features not 16-byte aligned: take the other route, the lattices are there)
         if (err != hipErrorNotSupported) return fail_hip(err, "ddf_hip_up_backward batch launch");
+        split = true;
+    }
+    if (!split) {
+        err = ddf::up_prepare<T>((const T *)go, lat, p.N * p.C, p.H, p.W, scale, cfs, sfs, (T *)nullptr, (T *)nullptr, 0, 0, stream);
+        if (err != hipSuccess) return fail_hip(err, "ddf_hip_up_backward split launch");
     }
 
     void *branch_ws = w.branch ? base + w.lattices + w.dx_parts : nullptr;

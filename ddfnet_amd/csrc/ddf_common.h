@@ -216,26 +216,30 @@ hipError_t up_forward(int64_t N, int64_t C, int64_t H, int64_t W, int k, int d, 
                       bool mul, const T *x, const void *const *cf, const void *const *sf, T *out,
                       hipStream_t st);
 
+// What a filter-gradient launch leaves in its workspace where the caller adds it up itself: partial sums
+// of dSF over csplit channel splits, of dCF over nstrips strips (null: the result is complete).
+template <typename T>
+struct FilterParts {
+    const typename Acc<T>::type *sf = nullptr, *cf = nullptr;
+    int csplit = 1, nstrips = 1;
+};
+
 // Helpers of the up-sampling backward: the gradient of the pixel shuffle (dO
-// split into its scale*scale sub-pixel lattices, stored back to back) and the
+// split into its scale*scale sub-pixel lattices, stored back to back) and, with cf_all, the branches'
+// filters copied back to back (cf / sf: host arrays of device pointers); the
 // sum of `parts` equally sized tensors stored back to back.
 template <typename T>
-hipError_t up_split_lattices(const T *go, T *lat, int64_t planes, int64_t H, int64_t W, int scale,
-                             hipStream_t st);
+hipError_t up_prepare(const T *go, T *lat, int64_t planes, int64_t H, int64_t W, int scale, const void *const *cf,
+                      const void *const *sf, T *cf_all, T *sf_all, int64_t n_cf, int64_t n_sf, hipStream_t st);
 template <typename T>
 hipError_t up_sum_parts(const T *in, T *out, int64_t count, int parts, hipStream_t st);
-// For the backward pass of all branches as one batch: the branches' filters
-// copied back to back (cf / sf: host arrays of `branches` device pointers), and
-// afterwards dX summed from the branches' parts (parts may be null) together
-// with the batch's filter gradients copied out to the branches' tensors (null
-// destinations are skipped; dcf_all / dsf_all may be null).
+// After the backward pass of all branches as one batch: dX summed from the branches' parts (parts may be
+// null), and the batch's filter gradients (complete where `left` names no partial sums of them) to
+// the branches' tensors (null destinations are skipped; dcf_all / dsf_all null: not asked for).
 template <typename T>
-hipError_t up_gather_filters(const void *const *cf, const void *const *sf, T *cf_all, T *sf_all,
-                             int64_t n_cf, int64_t n_sf, int branches, hipStream_t st);
-template <typename T>
-hipError_t up_finish(const T *parts, T *dx, int64_t n_x, int branches, const T *dcf_all,
-                     const T *dsf_all, void *const *dcfs, void *const *dsfs, int64_t n_cf,
-                     int64_t n_sf, hipStream_t st);
+hipError_t up_finish(const T *parts, T *dx, int64_t n_x, int branches, const T *dcf_all, const T *dsf_all,
+                     const FilterParts<T> &left, void *const *dcfs, void *const *dsfs, int64_t N, int64_t C, int64_t kk,
+                     int64_t plane, hipStream_t st);
 
 // Tiny planes (H*W <= 64), 3x3, stride 1: forward (backward = false: x -> out)
 // and feature gradient (backward = true: dO -> dX), G = 256 / (H*W) channel
@@ -266,17 +270,18 @@ bool rows_cover_backward(const Problem &p, int dtype);
 bool rows_cover_stride2_filters(const Problem &p, int dtype);
 // x_mod != 0: the batch p.N is several groups of x_mod samples sharing one set
 // of features x (x_mod samples long); everything else is indexed by the sample.
+// left != null: partial sums are not added up but named there.
 template <typename T>
 hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const T *cf, const T *sf,
                                T *dx, T *dcf, T *dsf, void *ws, unsigned need, hipStream_t st,
-                               int x_mod = 0, NormTail<T> *norm = nullptr);
+                               int x_mod = 0, NormTail<T> *norm = nullptr, FilterParts<T> *left = nullptr);
 // The whole backward pass of such a batch on the row-register kernels, or
 // hipErrorNotSupported before anything is launched (shape or alignment not
 // covered).  `ws`: rows_filters_workspace(p) bytes.
 template <typename T>
 hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *go, const T *x,
                                          const T *cf, const T *sf, T *dx, T *dcf, T *dsf, void *ws,
-                                         unsigned need, hipStream_t st);
+                                         unsigned need, hipStream_t st, FilterParts<T> *left);
 
 // Names of the kernels a forward / backward call on the tiled families would
 // launch, written into buf (at most len bytes); returns snprintf's count.

@@ -283,7 +283,7 @@ hipError_t launch_taprow_v(const Problem &p, const RowsGeom &g, const T *go, con
 template <typename T>
 hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const T *cf, const T *sf,
                                T *dx, T *dcf, T *dsf, void *ws, unsigned need, hipStream_t st,
-                               int x_mod, NormTail<T> *norm) {
+                               int x_mod, NormTail<T> *norm, FilterParts<T> *left) {
     using A = typename Acc<T>::type;
     const int dtype = sizeof(T) == 2 ? DDF_F16 : sizeof(T) == 4 ? DDF_F32 : DDF_F64;
     const bool fused = dx != nullptr;
@@ -352,6 +352,10 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
         }
     }
     if (err != hipSuccess) return err;
+    if (left) {
+        *left = FilterParts<T>{ws_sf, ws_cf, (int)g.csplit, (int)g.nstrips};
+        return hipSuccess;
+    }
     return wave::sum_filter_partials<T>(ws_sf, dsf, p.N, g.csplit, p.kk * p.Ho * p.Wo, ws_cf, dcf,
                                         p.N * p.C, g.nstrips, (int64_t)p.kk, st,
                                         (need & DDF_NEED_DSF) ? norm : nullptr);
@@ -360,7 +364,7 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
 template <typename T>
 hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *go, const T *x,
                                          const T *cf, const T *sf, T *dx, T *dcf, T *dsf, void *ws,
-                                         unsigned need, hipStream_t st) {
+                                         unsigned need, hipStream_t st, FilterParts<T> *left) {
     if constexpr (sizeof(T) == 8) {
         return hipErrorNotSupported;
     } else {
@@ -373,7 +377,7 @@ hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *g
         if ((((uintptr_t)go | (uintptr_t)x | (uintptr_t)sf | (uintptr_t)dx | (uintptr_t)dsf) & 15u) != 0)
             return hipErrorNotSupported;
         if (want_dx && fneed && rows_filters_plan(p, dtype, true, &g, &vx, &r))
-            return rows_filters_launch<T>(p, go, x, cf, sf, dx, dcf, dsf, ws, fneed, st, x_mod);
+            return rows_filters_launch<T>(p, go, x, cf, sf, dx, dcf, dsf, ws, fneed, st, x_mod, nullptr, left);
         if (want_dx && !rows_plan(p, dtype, &g, &vx, &r, true)) return hipErrorNotSupported;
         if (fneed && !rows_taprow_plan(p, dtype, &g, &vx, &r) &&
             !rows_filters_plan(p, dtype, false, &g, &vx, &r))
@@ -384,7 +388,7 @@ hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *g
             if (err != hipSuccess) return err;
         }
         if (fneed) {
-            err = rows_filters_launch<T>(p, go, x, cf, sf, (T *)nullptr, dcf, dsf, ws, fneed, st, x_mod);
+            err = rows_filters_launch<T>(p, go, x, cf, sf, (T *)nullptr, dcf, dsf, ws, fneed, st, x_mod, nullptr, left);
             if (err == hipErrorNotSupported) err = hipErrorUnknown;   // (ruled out above)
         }
         return err;
@@ -394,11 +398,11 @@ hipError_t rows_backward_shared_features(const Problem &p, int x_mod, const T *g
 #define DDF_INSTANTIATE_ROWS(T)                                                              \
     template hipError_t rows_filters_launch<T>(const Problem &, const T *, const T *, const T *, \
                                                const T *, T *, T *, T *, void *, unsigned,   \
-                                               hipStream_t, int, NormTail<T> *);              \
+                                               hipStream_t, int, NormTail<T> *, FilterParts<T> *); \
     template hipError_t rows_launch<T>(const Problem &, bool, const T *, const T *, const T *, \
                                        T *, hipStream_t);                                     \
     template hipError_t rows_backward_shared_features<T>(const Problem &, int, const T *,    \
                                                          const T *, const T *, const T *, T *, \
-                                                         T *, T *, void *, unsigned, hipStream_t);
+                                                         T *, T *, void *, unsigned, hipStream_t, FilterParts<T> *);
 
 }  // namespace ddf

@@ -16,6 +16,7 @@
 #include <atomic>
 
 #include "ddf_chunks.h"
+#include "ddf_wave.h"
 
 namespace ddf {
 int tune_int(const char *name, int fallback);
@@ -227,24 +228,73 @@ hipError_t launch(bool mul, const UpFilters<T> &f, const T *x, T *out, int64_t N
     return hipGetLastError();
 }
 
+template <typename T, int V>
+struct alignas(sizeof(T) * V) UpVec {
+    T e[V];
+};
+
+// The branches' filters, back to back: cf_all[b] = cf of branch b (n_cf elements),
+// sf_all[b] = sf of branch b (n_sf elements); V elements a thread.
+template <typename T, int V>
+__device__ __forceinline__ void up_gather(const UpFilters<T> &f, T *__restrict__ cf_all, T *__restrict__ sf_all,
+                                          int64_t n_cf, int64_t n_sf, int branches, int64_t idx) {
+    using Vec = UpVec<T, V>;
+    const int64_t per = n_cf + n_sf;
+    idx *= V;
+    if (idx >= per * branches) return;
+    const int b = (int)(idx / per);
+    const int64_t e = idx - b * per;
+    if (e < n_cf) *reinterpret_cast<Vec *>(cf_all + b * n_cf + e) = *reinterpret_cast<const Vec *>(f.cf[b] + e);
+    else *reinterpret_cast<Vec *>(sf_all + b * n_sf + (e - n_cf)) = *reinterpret_cast<const Vec *>(f.sf[b] + (e - n_cf));
+}
+
 // Gradient of the pixel shuffle: lat[b][nc][y][x] = dO[nc][y*R + i][x*R + j],
-// b = i*R + j.  One thread per (nc, y, x): it reads R runs of R neighbouring
-// elements and writes one element to each of the R*R lattices (neighbouring
-// lanes write neighbouring elements).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_up_split(const T *__restrict__ go,
-                                                       T *__restrict__ lat, int64_t planes, int H,
-                                                       int W, int R) {
+// b = i*R + j, in the first split_blocks workgroups, and in the same launch the branches' filters
+// back to back.  V == 1: one thread per (nc, y, x) reads R runs of R neighbouring
+// elements and writes one element to each of the R*R lattices.  V > 1 (R == 2, rows of whole 16-byte
+// vectors): V neighbouring pixels a thread, 16 bytes per access.  8 x 64 x 64 x 64 fp32, 67 MB and
+// 9 of filters: 22.5 us as two launches of V = 1, now 15.5 (a copy's rate: 14.6).
+template <typename T, int V>
+__global__ __launch_bounds__(kThreads) void k_up_prepare(const T *__restrict__ go, T *__restrict__ lat, int64_t planes,
+                                                         int H, int W, int R, unsigned split_blocks, UpFilters<T> f,
+                                                         T *__restrict__ cf_all, T *__restrict__ sf_all, int64_t n_cf,
+                                                         int64_t n_sf, bool wide) {
+    if (blockIdx.x >= split_blocks) {
+        const int64_t idx = (int64_t)(blockIdx.x - split_blocks) * kThreads + threadIdx.x;
+        constexpr int F = 16 / sizeof(T);
+        if (wide) up_gather<T, F>(f, cf_all, sf_all, n_cf, n_sf, R * R, idx);
+        else up_gather<T, 1>(f, cf_all, sf_all, n_cf, n_sf, R * R, idx);
+        return;
+    }
     const int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    const int64_t plane = (int64_t)H * W;
-    if (idx >= planes * plane) return;
-    const int64_t nc = idx / plane;
-    const int pix = (int)(idx - nc * plane);
-    const int y = pix / W, x = pix - y * W;
+    const int wv = W / V;
+    const int64_t plane = (int64_t)H * W, vectors = (int64_t)H * wv;
+    if (idx >= planes * vectors) return;
+    const int64_t nc = idx / vectors;
+    const int v = (int)(idx - nc * vectors), y = v / wv, x = (v - y * wv) * V;
     const T *src = go + (nc * H * R + (int64_t)y * R) * W * R + (int64_t)x * R;
-    for (int i = 0; i < R; ++i)
-        for (int j = 0; j < R; ++j)
-            lat[(int64_t)(i * R + j) * planes * plane + idx] = src[(int64_t)i * W * R + j];
+    T *dst = lat + nc * plane + (int64_t)y * W + x;
+    if constexpr (V == 1) {
+        for (int i = 0; i < R; ++i)
+            for (int j = 0; j < R; ++j)
+                dst[(int64_t)(i * R + j) * planes * plane] = src[(int64_t)i * W * R + j];
+    } else {
+        using Vec = UpVec<T, V>;
+        Vec in[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) in[i][h] = reinterpret_cast<const Vec *>(src + (int64_t)i * W * 2)[h];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                Vec out;
+#pragma unroll
+                for (int e = 0; e < V; ++e) out.e[e] = in[i][(2 * e + j) / V].e[(2 * e + j) % V];
+                *reinterpret_cast<Vec *>(dst + (int64_t)(i * 2 + j) * planes * plane) = out;
+            }
+    }
 }
 
 // out[e] = sum over `parts` tensors of `count` elements stored back to back.
@@ -260,105 +310,139 @@ __global__ __launch_bounds__(kThreads) void k_up_sum(const T *__restrict__ in,
     st(out + idx, acc);
 }
 
-// The branches' filters, back to back: cf_all[b] = cf of branch b (n_cf elements),
-// sf_all[b] = sf of branch b (n_sf elements).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_up_gather(UpFilters<T> f, T *__restrict__ cf_all,
-                                                        T *__restrict__ sf_all, int64_t n_cf,
-                                                        int64_t n_sf, int branches) {
-    const int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    const int64_t per = n_cf + n_sf;
-    if (idx >= per * branches) return;
-    const int b = (int)(idx / per);
-    const int64_t e = idx - b * per;
-    if (e < n_cf) cf_all[b * n_cf + e] = f.cf[b][e];
-    else sf_all[b * n_sf + (e - n_cf)] = f.sf[b][e - n_cf];
-}
-
 template <typename T>
 struct UpGrads {
     T *dcf[DDF_UP_MAX_BRANCHES];
     T *dsf[DDF_UP_MAX_BRANCHES];
 };
 
-// dX = sum of the branches' parts (parts != null); the branches' filter
-// gradients from where the batched kernels left them back to back to the
-// tensors they belong to (a null destination was not asked for).
+// A filter gradient of all branches: complete and back to back (`all`, n elements a branch), or partial
+// sums (`sum`, the job of branch 0; those of a branch follow the ones of the branch before).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_up_finish(
-    const T *__restrict__ parts, T *__restrict__ dx, int64_t n_x, int branches,
-    const T *__restrict__ dcf_all, const T *__restrict__ dsf_all, UpGrads<T> g, int64_t n_cf,
-    int64_t n_sf) {
+struct UpFilterGrad {
+    const T *all;
+    int64_t n;
+    wave::SumJob<T> sum;
+    unsigned blocks;    // workgroups of a branch, 0: not asked for
+};
+template <typename T, int V, bool SPLIT>
+__device__ __forceinline__ void up_filter_grad(const UpFilterGrad<T> &f, T *const (&to)[DDF_UP_MAX_BRANCHES], unsigned block) {
+    const int b = (int)(block / f.blocks);
+    const unsigned at = block - b * f.blocks;
+    T *const out = to[b];
+    if (!out) return;    // (not asked for)
+    const wave::SumJob<T> &j = f.sum;
+    if (!j.part) {
+        using Vec = UpVec<T, V>;
+        const int64_t e = ((int64_t)at * kThreads + threadIdx.x) * V;
+        if (e < f.n) *reinterpret_cast<Vec *>(out + e) = *reinterpret_cast<const Vec *>(f.all + b * f.n + e);
+    } else {
+        const auto *part = j.part + (int64_t)b * j.outer * j.parts * j.inner;
+        if (j.wide) wave::sum_partials_block<T, 4, SPLIT>(part, out, j.outer, j.parts, j.inner, j.split, at);
+        else wave::sum_partials_block<T, 1, SPLIT>(part, out, j.outer, j.parts, j.inner, j.split, at);
+    }
+}
+
+// The branches' filter gradients, added up or from where the batched kernels left them, to the tensors
+// they belong to (a null destination was not asked for); dX = sum of the branches' parts.  V elements
+// a thread: 16 bytes where every count and address allows.  8 x 64 x 64 x 64 fp32: 21.6 us as two
+// launches of single elements (the partial sums first), now 11.0 (52 MB, a copy's rate 10).
+template <typename T, int V, bool SPLIT>
+__global__ __launch_bounds__(kThreads) void k_up_finish(UpFilterGrad<T> cf, UpFilterGrad<T> sf, UpGrads<T> g, int branches,
+                                                        const T *__restrict__ parts, T *__restrict__ dx, int64_t n_x) {
     using A = typename Acc<T>::type;
-    int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    const int64_t n_dx = parts ? n_x : 0;
-    if (idx < n_dx) {
-        A acc = 0;
-        for (int b = 0; b < branches; ++b) acc += (A)ld(parts + (int64_t)b * n_x + idx);
-        st(dx + idx, acc);
-        return;
+    using Vec = UpVec<T, V>;
+    unsigned block = blockIdx.x;
+    if (block < cf.blocks * branches) return up_filter_grad<T, V, SPLIT>(cf, g.dcf, block);
+    block -= cf.blocks * branches;
+    if (block < sf.blocks * branches) return up_filter_grad<T, V, SPLIT>(sf, g.dsf, block);
+    block -= sf.blocks * branches;
+    const int64_t idx = ((int64_t)block * kThreads + threadIdx.x) * V;
+    if (idx >= n_x) return;
+    A acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = 0;
+    // (four branches' loads in flight)
+    for (int b0 = 0; b0 < branches; b0 += 4) {
+        Vec v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const Vec *>(parts + (int64_t)min(b0 + q, branches - 1) * n_x + idx);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc[e] += b0 + q < branches ? (A)ld(&v[q].e[e]) : A(0);
     }
-    idx -= n_dx;
-    const int64_t all_cf = dcf_all ? n_cf * branches : 0;
-    if (idx < all_cf) {
-        const int b = (int)(idx / n_cf);
-        if (g.dcf[b]) g.dcf[b][idx - b * n_cf] = dcf_all[idx];
-        return;
-    }
-    idx -= all_cf;
-    if (dsf_all && idx < n_sf * branches) {
-        const int b = (int)(idx / n_sf);
-        if (g.dsf[b]) g.dsf[b][idx - b * n_sf] = dsf_all[idx];
-    }
+    Vec out;
+#pragma unroll
+    for (int e = 0; e < V; ++e) st(&out.e[e], acc[e]);
+    *reinterpret_cast<Vec *>(dx + idx) = out;
 }
 
 }  // namespace
 
 template <typename T>
-hipError_t up_gather_filters(const void *const *cf, const void *const *sf, T *cf_all, T *sf_all,
-                             int64_t n_cf, int64_t n_sf, int branches, hipStream_t stream) {
-    const int64_t total = (n_cf + n_sf) * branches;
-    if (total == 0) return hipSuccess;
+hipError_t up_prepare(const T *go, T *lat, int64_t planes, int64_t H, int64_t W, int scale, const void *const *cf,
+                      const void *const *sf, T *cf_all, T *sf_all, int64_t n_cf, int64_t n_sf, hipStream_t stream) {
+    constexpr int V = 16 / sizeof(T);
+    const int branches = scale * scale;
     UpFilters<T> f;
+    uintptr_t any = 0;
     for (int b = 0; b < DDF_UP_MAX_BRANCHES; ++b) {
-        f.cf[b] = b < branches ? (const T *)cf[b] : nullptr;
-        f.sf[b] = b < branches ? (const T *)sf[b] : nullptr;
+        f.cf[b] = cf_all && b < branches ? (const T *)cf[b] : nullptr;
+        f.sf[b] = cf_all && b < branches ? (const T *)sf[b] : nullptr;
+        any |= (uintptr_t)f.cf[b] | (uintptr_t)f.sf[b];
     }
-    const int64_t grid = cdiv(total, kThreads);
-    if (grid > 2147483647) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_up_gather<T>), dim3((unsigned)grid), dim3(kThreads), 0, stream, f, cf_all,
-                       sf_all, n_cf, n_sf, branches);
+    const bool vec = scale == 2 && W % V == 0 && (uintptr_t)go % 16 == 0;
+    const bool wide = any % 16 == 0 && n_cf % V == 0 && n_sf % V == 0;
+    const int64_t split = cdiv(planes * H * (vec ? W / V : W), kThreads);
+    const int64_t gather = cf_all ? cdiv((n_cf + n_sf) * branches / (wide ? V : 1), kThreads) : 0;
+    if (split + gather == 0) return hipSuccess;
+    if (split + gather > 2147483647) return hipErrorInvalidConfiguration;
+#define DDF_UP_PREPARE(V_)                                                                                           \
+    hipLaunchKernelGGL((k_up_prepare<T, V_>), dim3((unsigned)(split + gather)), dim3(kThreads), 0, stream, go, lat, planes, \
+                       (int)H, (int)W, scale, (unsigned)split, f, cf_all, sf_all, n_cf, n_sf, wide)
+    if (vec) DDF_UP_PREPARE(V);
+    else DDF_UP_PREPARE(1);
+#undef DDF_UP_PREPARE
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t up_finish(const T *parts, T *dx, int64_t n_x, int branches, const T *dcf_all,
-                     const T *dsf_all, void *const *dcfs, void *const *dsfs, int64_t n_cf,
-                     int64_t n_sf, hipStream_t stream) {
-    const int64_t total = (parts ? n_x : 0) + (dcf_all ? n_cf * branches : 0) +
-                          (dsf_all ? n_sf * branches : 0);
-    if (total == 0) return hipSuccess;
+hipError_t up_finish(const T *parts, T *dx, int64_t n_x, int branches, const T *dcf_all, const T *dsf_all,
+                     const FilterParts<T> &left, void *const *dcfs, void *const *dsfs, int64_t N, int64_t C, int64_t kk,
+                     int64_t plane, hipStream_t stream) {
+    constexpr int V = 16 / sizeof(T);
+    const int64_t n_cf = N * C * kk, n_sf = N * kk * plane;
     UpGrads<T> g;
+    uintptr_t any = (uintptr_t)dx;
     for (int b = 0; b < DDF_UP_MAX_BRANCHES; ++b) {
-        g.dcf[b] = (b < branches && dcfs) ? (T *)dcfs[b] : nullptr;
-        g.dsf[b] = (b < branches && dsfs) ? (T *)dsfs[b] : nullptr;
+        g.dcf[b] = (b < branches && dcfs && dcf_all) ? (T *)dcfs[b] : nullptr;
+        g.dsf[b] = (b < branches && dsfs && dsf_all) ? (T *)dsfs[b] : nullptr;
+        any |= (uintptr_t)g.dcf[b] | (uintptr_t)g.dsf[b];
     }
-    const int64_t grid = cdiv(total, kThreads);
+    const bool vec = any % 16 == 0 && n_x % V == 0 && n_cf % V == 0 && n_sf % V == 0;
+    const int per = kThreads * (vec ? V : 1);
+    UpFilterGrad<T> cf{dcf_all, n_cf, {}, 0}, sf{dsf_all, n_sf, {}, 0};
+    if (dcf_all) {
+        if (left.cf) cf.sum = wave::sum_job<T>(left.cf, nullptr, N * C, left.nstrips, kk);
+        cf.blocks = left.cf ? cf.sum.blocks : (unsigned)cdiv(n_cf, per);
+    }
+    if (dsf_all) {
+        if (left.sf) sf.sum = wave::sum_job<T>(left.sf, nullptr, N, left.csplit, kk * plane);
+        sf.blocks = left.sf ? sf.sum.blocks : (unsigned)cdiv(n_sf, per);
+    }
+    const int64_t grid = (int64_t)(cf.blocks + sf.blocks) * branches + (parts ? cdiv(n_x, per) : 0);
+    if (grid == 0) return hipSuccess;
     if (grid > 2147483647) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_up_finish<T>), dim3((unsigned)grid), dim3(kThreads), 0, stream, parts, dx,
-                       n_x, branches, dcf_all, dsf_all, g, n_cf, n_sf);
-    return hipGetLastError();
-}
-
-template <typename T>
-hipError_t up_split_lattices(const T *go, T *lat, int64_t planes, int64_t H, int64_t W, int scale,
-                             hipStream_t stream) {
-    const int64_t total = planes * H * W;
-    if (total == 0) return hipSuccess;
-    const int64_t grid = cdiv(total, kThreads);
-    if (grid > 2147483647) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((k_up_split<T>), dim3((unsigned)grid), dim3(kThreads), 0, stream, go, lat,
-                       planes, (int)H, (int)W, scale);
+#define DDF_UP_FINISH(V_, SPLIT_)                                                                                    \
+    hipLaunchKernelGGL((k_up_finish<T, V_, SPLIT_>), dim3((unsigned)grid), dim3(kThreads), 0, stream, cf, sf, g, branches, \
+                       parts, dx, parts ? n_x : 0)
+    const bool split = cf.sum.split || sf.sum.split;
+    if (vec && split) DDF_UP_FINISH(V, true);
+    else if (vec) DDF_UP_FINISH(V, false);
+    else if (split) DDF_UP_FINISH(1, true);
+    else DDF_UP_FINISH(1, false);
+#undef DDF_UP_FINISH
     return hipGetLastError();
 }
 
@@ -405,13 +489,12 @@ hipError_t up_forward(int64_t N, int64_t C, int64_t H, int64_t W, int k, int d, 
     template hipError_t up_forward<T>(int64_t, int64_t, int64_t, int64_t, int, int, int, bool,  \
                                       const T *, const void *const *, const void *const *, T *, \
                                       hipStream_t);                                             \
-    template hipError_t up_split_lattices<T>(const T *, T *, int64_t, int64_t, int64_t, int,    \
-                                             hipStream_t);                                      \
+    template hipError_t up_prepare<T>(const T *, T *, int64_t, int64_t, int64_t, int, const void *const *, \
+                                      const void *const *, T *, T *, int64_t, int64_t, hipStream_t); \
     template hipError_t up_sum_parts<T>(const T *, T *, int64_t, int, hipStream_t);             \
-    template hipError_t up_gather_filters<T>(const void *const *, const void *const *, T *, T *, \
-                                             int64_t, int64_t, int, hipStream_t);              \
     template hipError_t up_finish<T>(const T *, T *, int64_t, int, const T *, const T *,        \
-                                     void *const *, void *const *, int64_t, int64_t, hipStream_t);
+                                     const FilterParts<T> &, void *const *, void *const *,      \
+                                     int64_t, int64_t, int64_t, int64_t, hipStream_t);
 DDF_UP_INSTANCE(__half)
 DDF_UP_INSTANCE(float)
 DDF_UP_INSTANCE(double)

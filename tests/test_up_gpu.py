@@ -70,6 +70,33 @@ def test_shapes(N, C, H, W):
     check_up(N, C, H, W, 3, 1, 2, 'mul', torch.float32)
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('N,C,H,W,k', [
+    (2, 8, 10, 8, 3), (1, 16, 12, 24, 5),    # 16 bytes per access throughout
+    (1, 3, 6, 16, 3),                        # filters of a length that 16 bytes do not divide
+    (1, 4, 5, 12, 3),                        # fp16: rows that they do not
+    (1, 8, 260, 64, 3), (2, 4, 200, 40, 3),  # partial sums of many strips
+    (1, 520, 8, 8, 3),                       # partial sums over channel ranges
+])
+def test_gradient_vectors(N, C, H, W, k, dtype):
+    check_up(N, C, H, W, k, 1, 2, 'mul', dtype)
+
+
+def test_gradients_of_filters_at_any_address():
+    """Filters and their gradients one element past an aligned address."""
+    x, cfs, sfs, go = up_case(2, 8, 8, 16, 3, 2, torch.float16, seed=3)
+    want_x, want_cf, want_sf = oracle.up_backward(go, x, cfs, sfs, 3, 1, 2, 'mul')
+    odd = lambda t: torch.zeros(t.numel() + 1, device='cuda', dtype=t.dtype)[1:].view(t.shape).copy_(t)
+    for shift_in, shift_out in ((True, False), (False, True)):
+        cfd, sfd = ([odd(t) if shift_in else t.cuda() for t in l] for l in (cfs, sfs))
+        gx = torch.empty(x.shape, device='cuda', dtype=x.dtype)
+        gcf, gsf = ([odd(t) if shift_out else torch.empty_like(t, device='cuda') for t in l] for l in (cfs, sfs))
+        _lib.up_backward(go.cuda(), x.cuda(), cfd, sfd, gx, gcf, gsf, 3, 1, 2, 'mul')
+        torch.cuda.synchronize()
+        for got, want in zip([gx] + gcf + gsf, [want_x] + list(want_cf) + list(want_sf)):
+            assert rel_err(got, want) <= TOL[torch.float16]
+
+
 def test_empty_tensors():
     for shape in ((0, 4, 5, 5), (2, 0, 5, 5), (2, 4, 0, 5)):
         N, C, H, W = shape
