@@ -827,24 +827,55 @@ int64_t ddf_hip_net_conv_chain_parts(int64_t N, int64_t H, int64_t W, int64_t C,
     return ddf::net_chain_pool_slots(N * H * W, (int)(H * W));
 }
 
-int ddf_hip_net_conv_chain(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
-                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
-                           int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm,
-                           void *next, float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O,
-                           int64_t next_O, void *stream) {
+int64_t ddf_hip_net_filter_chain_parts(int64_t N, int64_t H, int64_t W, int64_t C, int64_t side_C, int64_t O, int64_t next_O) {
+    return W > 0 && ddf::net_chain_filters(W, C) ? ddf_hip_net_conv_chain_parts(N, H, W, C, side_C, O, next_O) : 0;
+}
+
+namespace {
+// (spatial_filter null: no filter in front)
+int net_chain_impl(const char *name, const void *features, const void *channel_filter, const void *spatial_filter,
+                   const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
+                   const void *residual, const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
+                   int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm, void *next,
+                   float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int64_t next_O, void *stream) {
     if (N < 0 || H < 1 || W < 1 || C < 1 || side_C < 0 || O < 1 || next_O < 1 || H * W >= (1ll << 31))
-        return fail(DDF_ERR_BAD_ARG, "ddf_hip_net_conv_chain: bad sizes");
+        return fail(DDF_ERR_BAD_ARG, "%s: bad sizes", name);
     if (!features || !weight || !output || !next_weight || !next || !pool_parts || !net_norm_ok(norm) || !net_norm_ok(next_norm) ||
         !net_norm_ok(side_norm) || (side_C ? !side_features || !side_weight : !residual))
         return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
     if (N == 0) return DDF_OK;
     const int64_t M = N * H * W;
-    if (!ddf::net_chain_covers(M, C, side_C, O, next_O))
-        return fail(DDF_ERR_UNSUPPORTED, "ddf_hip_net_conv_chain: sizes not covered");
+    if (!ddf::net_chain_covers(M, C, side_C, O, next_O) || (spatial_filter && !ddf::net_chain_filters(W, C)))
+        return fail(DDF_ERR_UNSUPPORTED, "%s: sizes not covered", name);
     const ddf::NetChain a{features, weight, residual, side_features, side_weight, next_weight, output, next, pool_parts,
                           net_norm(norm), net_norm(side_norm), net_norm(next_norm), M, (int)C, (int)side_C, (int)O,
-                          (int)next_O, (int)(H * W), 0, 0};
-    return net_result(ddf::net_chain(a, (hipStream_t)stream), "ddf_hip_net_conv_chain launch");
+                          (int)next_O, (int)(H * W), channel_filter, spatial_filter, net_norm(filter_norm), (int)W,
+                          combine == DDF_MUL, 0, 0};
+    return net_result(ddf::net_chain(a, (hipStream_t)stream), name);
+}
+}  // namespace
+
+int ddf_hip_net_conv_chain(const void *features, const void *weight, const ddf_net_norm_t *norm, const void *residual,
+                           const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
+                           int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm,
+                           void *next, float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O,
+                           int64_t next_O, void *stream) {
+    return net_chain_impl("ddf_hip_net_conv_chain", features, nullptr, nullptr, nullptr, DDF_MUL, weight, norm, residual,
+                          side_features, side_weight, side_norm, side_C, output, next_weight, next_norm, next, pool_parts, N,
+                          H, W, C, O, next_O, stream);
+}
+
+int ddf_hip_net_filter_chain(const void *features, const void *channel_filter, const void *spatial_filter,
+                             const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
+                             const void *residual, const void *side_features, const void *side_weight,
+                             const ddf_net_norm_t *side_norm, int64_t side_C, void *output, const void *next_weight,
+                             const ddf_net_norm_t *next_norm, void *next, float *pool_parts, int64_t N, int64_t H, int64_t W,
+                             int64_t C, int64_t O, int64_t next_O, void *stream) {
+    if (combine != DDF_MUL && combine != DDF_ADD) return fail(DDF_ERR_BAD_ARG, "unknown combine %d", combine);
+    if (!channel_filter || !spatial_filter || !net_norm_ok(filter_norm)) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    return net_chain_impl("ddf_hip_net_filter_chain", features, channel_filter, spatial_filter, filter_norm, combine, weight,
+                          norm, residual, side_features, side_weight, side_norm, side_C, output, next_weight, next_norm, next,
+                          pool_parts, N, H, W, C, O, next_O, stream);
 }
 
 int ddf_hip_net_stem(const void *image, const void *weight, const ddf_net_norm_t *norm, void *output, int64_t N,

@@ -11,6 +11,7 @@
 //   k_net_branches  spatial and channel filter branch
 //   k_net_filter    dynamic filter + BatchNorm + ReLU
 //   k_net_conv
+// (with many pixels the last two and the next one's first are one, k_net_chain of ddf_net_chain.hip)
 // and k_net_stem is the 7x7 convolution, BatchNorm, ReLU and max-pool in one.
 // At batch 128 the network took 8.85 ms as torch modules around the operator: 3.2 ms of
 // BatchNorm, 1.6 ms of ReLU and additions, 3 ms of convolutions (ddf_resnet.py:34-111 of
@@ -30,7 +31,6 @@ namespace ddf {
 namespace {
 using namespace net;
 using rows::from_left;
-using rows::half2_t;
 using rows::kOutside;
 using rows::load_words;
 using rows::plane_rsrc;
@@ -38,8 +38,7 @@ using rows::plane_rsrc;
 // ---- spatial filter branch of sixteen pixels ------------------------------------------
 // Pixels are the columns, the nine taps nine of the sixteen rows of 16x16x32 steps over the
 // channels; both operands contiguous.  A pixel's taps end up on four lanes, which normalise them
-// across the wave's rows; they are stored as (pixel, 12), nine taps and padding.
-constexpr int kTapPitch = 12;
+// across the wave's rows; they are stored as (pixel, kTapPitch), nine taps and padding.
 
 template <int KS>
 struct TapWeights {
@@ -789,19 +788,6 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps tap
 // fp32 - for rows of an odd length, where the operator's own kernels have it so.  A row outside the
 // image, a column past its ends and a walk past the last pixel read zeros through the buffer
 // descriptor.
-template <bool MUL, bool WIDE>
-__device__ __forceinline__ void filter_pair(half2_t cv, half2_t sv, half2_t xv, float &a0, float &a1) {
-    if constexpr (WIDE) {
-        const float c0 = (float)cv[0], c1 = (float)cv[1], s0 = (float)sv[0], s1 = (float)sv[1];
-        a0 = fmaf((float)xv[0], MUL ? c0 * s0 : c0 + s0, a0);
-        a1 = fmaf((float)xv[1], MUL ? c1 * s1 : c1 + s1, a1);
-    } else {
-        const half2_t cb = MUL ? cv * sv : cv + sv;
-        a0 = fmaf((float)xv[0], (float)cb[0], a0);
-        a1 = fmaf((float)xv[1], (float)cb[1], a1);
-    }
-}
-
 template <int LP, int S, bool MUL, bool WIDE>
 __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restrict__ x,
                                                          const _Float16 *__restrict__ cf,
@@ -830,25 +816,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 
     Affine<8> aff;
     aff.request(norm, cl * 8);
-    // channel taps: of filter rows 0 and 1 as a channel's pair, of row 2 as two channels'
     uint32_t cfa[3][8], cfb[3][4];
-    {
-        const uint4 *src = reinterpret_cast<const uint4 *>(cf + ((int64_t)n * C + cl * 8) * KK);
-        uint32_t wd[36];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) {
-            const uint4 q = src[i];
-            wd[4 * i] = q.x; wd[4 * i + 1] = q.y; wd[4 * i + 2] = q.z; wd[4 * i + 3] = q.w;
-        }
-        auto half_at = [&](int i) { return (i & 1) ? wd[i / 2] >> 16 : wd[i / 2] & 0xffffu; };
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) cfa[j][e] = half_at(9 * e + j) | (half_at(9 * e + 3 + j) << 16);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) cfb[j][k] = half_at(18 * k + 6 + j) | (half_at(18 * k + 15 + j) << 16);
-        }
-    }
+    channel_taps(cf + ((int64_t)n * C + cl * 8) * KK, cfa, cfb);
     uint32_t rowo[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -879,48 +848,12 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
             tap[J][2 * i + 1] = q[1];
         }
     };
-    // Rows 0 and 1 of a column as a channel's pair each, once for the three results it is under.
-    auto pair_rows = [&](auto slot) __attribute__((always_inline)) {
-        constexpr int J = decltype(slot)::value % RING;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t top = col[J][0][k], low = col[J][1][k];
-            col[J][0][k] = __builtin_amdgcn_perm(low, top, 0x05040100);
-            col[J][1][k] = __builtin_amdgcn_perm(low, top, 0x07060302);
-        }
-    };
+    auto pair_rows = [&](auto slot) __attribute__((always_inline)) { pair_column(col[decltype(slot)::value % RING]); };
     // result xx from the columns in slots A, A + 1 and A + 2 and the taps in slot J
     auto emit = [&](auto first, auto slot, int xx) __attribute__((always_inline)) {
         constexpr int A = decltype(first)::value, J = decltype(slot)::value % 2;
-        const uint32_t *tp = tap[J];
-        // spatial taps j and 3 + j
-        const uint32_t sa[3] = {__builtin_amdgcn_perm(tp[1], tp[0], 0x07060100), __builtin_amdgcn_perm(tp[2], tp[0], 0x05040302),
-                                __builtin_amdgcn_perm(tp[2], tp[1], 0x07060100)};
         float acc[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const uint32_t(&at)[3][4] = col[(A + j) % RING];
-            const half2_t sp = __builtin_bit_cast(half2_t, sa[j]);
-            const half2_t sb = __builtin_bit_cast(half2_t, tp[(6 + j) / 2]);
-            const half2_t sv = {sb[j & 1], sb[j & 1]};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const half2_t xv = __builtin_bit_cast(half2_t, at[e & 1][e / 2]), cv = __builtin_bit_cast(half2_t, cfa[j][e]);
-                if constexpr (WIDE) {
-                    const float c0 = (float)cv[0], c1 = (float)cv[1], s0 = (float)sp[0], s1 = (float)sp[1];
-                    acc[e] = fmaf((float)xv[0], MUL ? c0 * s0 : c0 + s0, acc[e]);
-                    acc[e] = fmaf((float)xv[1], MUL ? c1 * s1 : c1 + s1, acc[e]);
-                } else {
-                    acc[e] = __builtin_amdgcn_fdot2(xv, MUL ? cv * sp : cv + sp, acc[e], false);
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, cfb[j][k]), sv, __builtin_bit_cast(half2_t, at[2][k]),
-                                       acc[2 * k], acc[2 * k + 1]);
-        }
+        filter_sums<MUL, WIDE>(cfa, cfb, col[A % RING], col[(A + 1) % RING], col[(A + 2) % RING], tap[J], acc);
         half8_t o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {

@@ -1,12 +1,15 @@
-// A bottleneck's last 1x1 convolution and the next one's first in one launch (DDF-ResNet
-// inference, fp16, channels-last; ddf_resnet.py:34-111 of the reference composes them).
+// A bottleneck's dynamic filter, its last 1x1 convolution and the next one's first in one launch
+// (DDF-ResNet inference, fp16, channels-last; ddf_resnet.py:34-111 of the reference composes them).
 #include <numeric>
+#include <type_traits>
 
 #include "ddf_net_device.h"
 
 namespace ddf {
 namespace {
 using namespace net;
+using rows::kOutside;
+using rows::load_words;
 using rows::plane_rsrc;
 
 // out (M, N) = relu(norm(x . w) + res), or relu(norm(x . w) + norm'(side . side_w));
@@ -36,9 +39,107 @@ struct ChainLds {    // halves; K2: channels of the side product, 0: none
     // at the end: a wave's tile of next's results, and the sums over its pixels
     static constexpr int red = kChainRows * kTilePitch;
     static_assert(red + kChainWaves * N2 * 2 <= norms, "next's results fit in front of the norms");
+    static constexpr int filtered = norms - kChainRows * (K + 8);    // at the start: a wave's filtered pixels
+    static_assert(filtered >= wd + kChunk * K2, "and do not meet the first weights");
     // scale, shift, what a sum starts with; of the wide channels (and of the side product), of next's
     static constexpr int bytes(int N) { return norms * 2 + (N * (K2 ? 5 : 3) + N2 * 3) * 4; }
 };
+
+// ---- the dynamic filter in front --------------------------------------------------------
+// A wave's 32 pixels of x, filtered, normalised and rounded as k_net_filter does it, to its part of LDS
+// (rows of K + 8).  K / 8 lanes own four neighbouring pixels at a time, eight channels each, so a channel's
+// taps are paired once for all of a lane's pixels and six columns serve four results; rows of images are
+// whole runs of four (W % 4 == 0), as tiles are.  Pixels past the last are made from zeros.
+// The filter's results, 103 MB of a batch of 128 at 56 x 56, never reach memory; what is left of its time is a chain of
+// round trips in front of each tile's products, which the compute unit's other workgroups cover in part (44
+// registers more than four of them leave spill: 150 us where three take 105).  us, filter and the launch behind it / this, batch
+// 128: 56 x 56 x 64 -> 256 -> 64 125 / 106, with the projection 128 / 116, -> 128 144 / 125, 28 x 28 x 128 -> 512 -> 128 72 /
+// 63; batch 16: 22.4 / 18.4, 27.1 / 22.4, 24.6 / 20.6; batch 8 20 / 14, 20.6 / 17.9, 20.2 / 15.9.
+constexpr int kRun = 4;
+template <int K, bool MUL>
+__device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int wave, int lane, _Float16 *to) {
+    constexpr int LP = K / 8, SLOTS = kWave / LP, PER = 32 / SLOTS, RING = 5;
+    static_assert(PER % kRun == 0);
+    const int cl = lane % LP, H = a.npix / a.W, W = a.W;
+    // (all offsets from a pixel in front of the tile's neighbours: a tile's are 32-bit ones)
+    const int64_t base = m0 - W - 1 > 0 ? m0 - W - 1 : 0;
+    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(static_cast<const _Float16 *>(a.x) + base * K,
+                                                 (uint32_t)(min(a.M - base, (int64_t)(2 * W + 2 + kChainRows)) * K * 2));
+    const __amdgpu_buffer_rsrc_t tr = plane_rsrc(static_cast<const _Float16 *>(a.sf) + m0 * kTapPitch,
+                                                 (uint32_t)(min(a.M - m0, (int64_t)kChainRows) * kTapPitch * 2));
+    const bool bn = a.filter_norm.var;
+    auto parameter = [&](bool there, const void *p) __attribute__((always_inline)) {    // (zeros where there is none)
+        return __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(plane_rsrc(p, there && p ? K * 2 : 0), cl * 16, 0, 0));
+    };
+    const half8_t nw = parameter(bn, a.filter_norm.weight), nb = parameter(bn, a.filter_norm.bias), nm = parameter(bn, a.filter_norm.mean),
+                  nv = parameter(bn, a.filter_norm.var), nc = parameter(true, a.filter_norm.conv_bias);
+    uint32_t cfa[3][8], cfb[3][4];
+    float sc[8], sh[8];
+#pragma unroll
+    for (int run = 0; run < PER / kRun; ++run) {
+        const int px = wave * 32 + lane / LP * PER + run * kRun;    // in the tile
+        const bool live = m0 + px < a.M;
+        const unsigned pix = live ? (unsigned)m0 + px : (unsigned)m0, row = pix / (unsigned)W;
+        const int xx = (int)(pix - row * W), n = (int)(row / (unsigned)H), y = (int)(row - (unsigned)n * H);
+        uint32_t rowo[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int yy = y - 1 + i;
+            rowo[i] = live && yy >= 0 && yy < H ? (uint32_t)(((int)((int64_t)pix - base) + (i - 1) * W) * K + cl * 8) * 2 : kOutside;
+        }
+        uint32_t col[RING][3][4], tap[kRun][6];
+        auto column = [&](auto slot) __attribute__((always_inline)) {
+            constexpr int Q = decltype(slot)::value;    // column xx - 1 + Q
+            const bool in = (Q > 0 || xx > 0) && (Q < kRun + 1 || xx + kRun < W);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                load_words<4>(xr, in && rowo[i] != kOutside ? rowo[i] + (uint32_t)((Q - 1) * K * 2) : kOutside, col[Q % RING][i]);
+        };
+        auto taps = [&](auto slot) __attribute__((always_inline)) {
+            constexpr int Q = decltype(slot)::value;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(tr, (px + Q) * kTapPitch * 2 + i * 8, 0, 0);
+                tap[Q][2 * i] = v[0];
+                tap[Q][2 * i + 1] = v[1];
+            }
+        };
+        if (run == 0 || a.npix % PER) channel_taps(static_cast<const _Float16 *>(a.cf) + ((int64_t)n * K + cl * 8) * 9, cfa, cfb);
+        rows::static_for<0, RING - 1>(column);
+        rows::static_for<0, 2>(taps);
+        if (run == 0) {
+            const float eps = bn ? a.filter_norm.eps : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                sc[e] = (bn ? (float)nw[e] : 1.f) * rsqrtf((bn ? (float)nv[e] : 1.f) + eps);
+                sh[e] = (float)nb[e] + ((float)nc[e] - (float)nm[e]) * sc[e];
+            }
+        }
+        rows::static_for<0, kRun>([&](auto q) __attribute__((always_inline)) {
+            constexpr int Q = decltype(q)::value;
+            if constexpr (Q + RING - 1 < kRun + 2) column(std::integral_constant<int, Q + RING - 1>{});
+            if constexpr (Q + 2 < kRun) taps(std::integral_constant<int, Q + 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (Q == 0) {
+                pair_column(col[0]);
+                pair_column(col[1]);
+            }
+            pair_column(col[(Q + 2) % RING]);
+            float acc[8];
+            filter_sums<MUL, false>(cfa, cfb, col[Q % RING], col[(Q + 1) % RING], col[(Q + 2) % RING], tap[Q], acc);
+            half8_t o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float f = fmaf((float)(_Float16)acc[e], sc[e], sh[e]);    // (the sum is rounded as the operator's result is)
+                asm volatile("" : "+v"(f));
+                o[e] = (_Float16)f;
+            }
+            o = __builtin_elementwise_maximum(o, half8_t{0, 0, 0, 0, 0, 0, 0, 0});
+            *reinterpret_cast<half8_t *>(to + (px - wave * 32 + Q) * (K + 8) + cl * 8) = o;
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
+}
 
 // chunk c of row r of a weight tile sits in place c ^ turn (see k_net_conv: sixteen lanes that LDS serves at
 // once meet all of its banks)
@@ -62,7 +163,53 @@ struct StageRows {
     }
 };
 
-template <int K, int K2, int N2, int WPS>
+// Scale, shift and what a sum starts with, of all channels of a norm: four channels per thread and pass, asked for
+// through descriptors that hold nothing where a parameter is not there (under a branch each, the loads
+// waited for one another: 0.7 us of 16 at 16 x 56 x 56, 2 of 50 with 1024 channels).  Without a BatchNorm a bias is part of the sum, elsewhere the
+// sum is rounded first (see k_net_conv).
+template <int PASSES>
+struct Norms {
+    uint32_t w[PASSES][2], b[PASSES][2], m[PASSES][2], v[PASSES][2], cb[PASSES][2];
+    __device__ __forceinline__ void request(const NetNorm &n, int channels, int tid) {
+        const void *const p[5] = {n.var ? n.weight : nullptr, n.var ? n.bias : nullptr, n.var ? n.mean : nullptr, n.var, n.conv_bias};
+        uint32_t(*const to[5])[2] = {w, b, m, v, cb};
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const __amdgpu_buffer_rsrc_t r = plane_rsrc(p[k], p[k] ? channels * 2 : 0);
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) rows::load_words<2>(r, (uint32_t)(i * kThreads + tid) * 8, to[k][i]);
+        }
+    }
+    __device__ __forceinline__ void put(const NetNorm &n, int channels, int tid, float *scale, float *shift, float *start) const {
+        const bool bn = n.var, in_sum = start && !bn;
+        const float eps = bn ? n.eps : 0.f;
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) {
+            const int c = (i * kThreads + tid) * 4;
+            const half4_t wv = __builtin_bit_cast(half4_t, w[i]), bv = __builtin_bit_cast(half4_t, b[i]), mv = __builtin_bit_cast(half4_t, m[i]),
+                          vv = __builtin_bit_cast(half4_t, v[i]), cv = __builtin_bit_cast(half4_t, cb[i]);
+            float4_t sc, sh, st;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float conv = (float)cv[e];
+                sc[e] = (bn && n.weight ? (float)wv[e] : 1.f) * rsqrtf((bn ? (float)vv[e] : 1.f) + eps);
+                sh[e] = (float)bv[e] + ((in_sum ? 0.f : conv) - (float)mv[e]) * sc[e];
+                st[e] = in_sum ? conv : 0.f;
+            }
+            if (c < channels) {
+                *reinterpret_cast<float4_t *>(scale + c) = sc;
+                *reinterpret_cast<float4_t *>(shift + c) = sh;
+                if (start) *reinterpret_cast<float4_t *>(start + c) = st;
+            }
+        }
+    }
+};
+// (passes of the wide channels: what a launch takes)
+constexpr int kMaxWide = 2048, kWidePasses = kMaxWide / (4 * kThreads);
+
+enum { kNoFilter, kFilterMul, kFilterAdd };
+
+template <int K, int K2, int N2, int WPS, int FILTER>
 __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
     typedef ChainLds<K, K2, N2> L;
     constexpr int BM = kChainRows;
@@ -84,36 +231,8 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
 
     // (rows past the last pixel read zeros and are not stored: every one of these loads and stores is
     // issued whatever the tile, the waits below count them)
-    const __amdgpu_buffer_rsrc_t xr = plane_rsrc(static_cast<const _Float16 *>(a.x) + m0 * K, rows * K * 2);
     const __amdgpu_buffer_rsrc_t rr = plane_rsrc(K2 ? nullptr : static_cast<const _Float16 *>(a.res) + m0 * N, K2 ? 0 : rows * N * 2);
     const __amdgpu_buffer_rsrc_t orr = plane_rsrc(static_cast<_Float16 *>(a.out) + m0 * N, rows * N * 2);
-    half8_t xv[K / 16], dv[K2 ? K2 / 16 : 1];
-#pragma unroll
-    for (int k = 0; k < K / 16; ++k)
-        xv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(xr, ((wave * 32 + l32) * K + hi * 8) * 2, k * 32, 0));
-    if constexpr (K2 > 0) {
-        const __amdgpu_buffer_rsrc_t dr = plane_rsrc(static_cast<const _Float16 *>(a.side) + m0 * K2, rows * K2 * 2);
-#pragma unroll
-        for (int k = 0; k < K2 / 16; ++k)
-            dv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(dr, ((wave * 32 + l32) * K2 + hi * 8) * 2, k * 32, 0));
-    }
-    // Without a BatchNorm a bias is part of the sum, elsewhere the sum is rounded first (see k_net_conv).
-    auto put_norm = [&](const NetNorm &n, bool in_sum, int c, float *sc, float *sh, float *st) __attribute__((always_inline)) {
-        Affine<1> aff;
-        aff.request(n, c, !in_sum);
-        float s1[1], s2[1];
-        aff.finish(n, s1, s2);
-        sc[c] = s1[0];
-        sh[c] = s2[0];
-        if (st) st[c] = in_sum ? (float)static_cast<const _Float16 *>(n.conv_bias)[c] : 0.f;
-    };
-    const bool in_sum = !K2 && !a.norm.var && a.norm.conv_bias, in_sum2 = !a.norm2.var && a.norm2.conv_bias;
-    for (int c = tid; c < N; c += kThreads) {
-        put_norm(a.norm, in_sum, c, scale, shift, start);
-        if constexpr (K2 > 0) put_norm(a.side_norm, false, c, side_scale, side_shift, nullptr);
-    }
-    for (int c = tid; c < N2; c += kThreads) put_norm(a.norm2, in_sum2, c, scale2, shift2, start2);
-
     const StageRows<kChunk, K> sw(tid, K);
     const StageRows<kChunk, K2 ? K2 : K> sd(tid, K2);
     const StageRows<N2, kChunk> sw2(tid, N);
@@ -123,6 +242,37 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
         sw.load(lds0 + L::w * 2, wave, w + (int64_t)j * kChunk * K, K);
         if constexpr (K2 > 0) sd.load(lds0 + L::wd * 2, wave, wd + (int64_t)j * kChunk * K2, K2);
     };
+    stage_w(0);
+    {
+        Norms<kWidePasses> norm, side_norm;
+        Norms<1> norm2;
+        norm.request(a.norm, N, tid);
+        if constexpr (K2 > 0) side_norm.request(a.side_norm, N, tid);
+        norm2.request(a.norm2, N2, tid);
+        norm.put(a.norm, N, tid, scale, shift, K2 ? nullptr : start);
+        if constexpr (K2 > 0) side_norm.put(a.side_norm, N, tid, side_scale, side_shift, nullptr);
+        norm2.put(a.norm2, N2, tid, scale2, shift2, start2);
+    }
+    half8_t xv[K / 16], dv[K2 ? K2 / 16 : 1];
+    if constexpr (FILTER) {
+        _Float16 *const mine = chain_smem + L::filtered + wave * 32 * (K + 8);
+        filter_pixels<K, FILTER == kFilterMul>(a, m0, wave, lane, mine);
+        asm volatile("" ::: "memory");    // (a wave's LDS operations keep their order)
+#pragma unroll
+        for (int k = 0; k < K / 16; ++k) xv[k] = *reinterpret_cast<const half8_t *>(mine + l32 * (K + 8) + k * 16 + hi * 8);
+    } else {
+        const __amdgpu_buffer_rsrc_t xr = plane_rsrc(static_cast<const _Float16 *>(a.x) + m0 * K, rows * K * 2);
+#pragma unroll
+        for (int k = 0; k < K / 16; ++k)
+            xv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(xr, ((wave * 32 + l32) * K + hi * 8) * 2, k * 32, 0));
+    }
+    if constexpr (K2 > 0) {
+        const __amdgpu_buffer_rsrc_t dr = plane_rsrc(static_cast<const _Float16 *>(a.side) + m0 * K2, rows * K2 * 2);
+#pragma unroll
+        for (int k = 0; k < K2 / 16; ++k)
+            dv[k] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(dr, ((wave * 32 + l32) * K2 + hi * 8) * 2, k * 32, 0));
+    }
+    const bool in_sum = !K2 && !a.norm.var && a.norm.conv_bias, in_sum2 = !a.norm2.var && a.norm2.conv_bias;
     // a lane's vectors on their way out: eight channels of every eighth pixel
     const int c8 = lane & 7, px0 = wave * 32 + (lane >> 3);
     rows_u4 rv[RV];
@@ -133,7 +283,6 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
                 rv[i] = __builtin_amdgcn_raw_buffer_load_b128(rr, (px0 * N + c8 * 8) * 2, (i * 8 * N + j * kChunk) * 2, 0);
         }
     };
-    stage_w(0);
     residual(0);
 
     // a lane's column of a 32 x 32 step's result is pixel l32, rows (channels) 8 * q + 4 * hi + 0..3 in
@@ -356,10 +505,10 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
     }
 }
 
-template <int K, int K2, int N2, int WPS>
+template <int K, int K2, int N2, int WPS, int FILTER>
 hipError_t launch_chain(const NetChain &a, hipStream_t st) {
     const int lds = ChainLds<K, K2, N2>::bytes(a.N);
-    hipLaunchKernelGGL((k_net_chain<K, K2, N2, WPS>), dim3(xcd_grid(a.tiles)), dim3(kThreads), lds, st, a);
+    hipLaunchKernelGGL((k_net_chain<K, K2, N2, WPS, FILTER>), dim3(xcd_grid(a.tiles)), dim3(kThreads), lds, st, a);
     return hipGetLastError();
 }
 
@@ -371,13 +520,17 @@ hipError_t launch_chain(const NetChain &a, hipStream_t st) {
 // then run side by side (28 x 28 x 128 -> 512 -> 256: 32 images 30.1 / 28.9, 64 47.8 / 43.8, 96, 588 workgroups, 63.9 / 70.3).
 bool net_chain_covers(int64_t M, int64_t K, int64_t side, int64_t N, int64_t N2) {
     constexpr int kFew = 192, kSideBySide = 512;
-    if (N % kChunk || N < kChunk || N > 2048 || M > INT32_MAX - 256) return false;
+    if (N % kChunk || N < kChunk || N > kMaxWide || M > INT32_MAX - 256) return false;
     const int64_t tiles = cdiv(M, kChainRows);
     if (tiles < kFew) return false;
     if (side) return K == 64 && side == 64 && N2 == 64;
     if (K == 64) return N2 == 64 || N2 == 128;
     return K == 128 && (N2 == 128 || (N2 == 256 && tiles <= kSideBySide));
 }
+
+// (runs of four pixels; rows of 4096, far more than an image has, keep a tile's neighbours within 2 MB.  No
+// size was found where the two launches are faster.)
+bool net_chain_filters(int64_t W, int64_t K) { return W % kRun == 0 && W <= 4096 && (K == 64 || K == 128); }
 
 int net_chain_pool_slots(int64_t M, int npix) {
     const int start = M > npix ? kChainRows - std::gcd(kChainRows, npix) : 0;
@@ -388,15 +541,19 @@ int net_chain_pool_slots(int64_t M, int npix) {
 hipError_t net_chain(NetChain a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_chain_covers(a.M, a.K, a.side_K, a.N, a.N2)) return hipErrorNotSupported;
+    if (a.sf && !net_chain_filters(a.W, a.K)) return hipErrorNotSupported;
     a.tiles = (int)cdiv(a.M, kChainRows);
     a.pool_slots = net_chain_pool_slots(a.M, a.npix);
-#define DDF_CHAIN(K_, SIDE_, N2_, WPS_) \
-    if (a.K == K_ && a.side_K == SIDE_ && a.N2 == N2_) return launch_chain<K_, SIDE_, N2_, WPS_>(a, st);
-    DDF_CHAIN(64, 64, 64, 3)
-    DDF_CHAIN(64, 0, 64, 4)
-    DDF_CHAIN(64, 0, 128, 3)
-    DDF_CHAIN(128, 0, 128, 2)
-    DDF_CHAIN(128, 0, 256, 2)
+#define DDF_CHAIN(K_, SIDE_, N2_, WPS_, FWPS_) \
+    if (a.K == K_ && a.side_K == SIDE_ && a.N2 == N2_) {                                            \
+        if (!a.sf) return launch_chain<K_, SIDE_, N2_, WPS_, kNoFilter>(a, st);                     \
+        return a.mul ? launch_chain<K_, SIDE_, N2_, FWPS_, kFilterMul>(a, st) : launch_chain<K_, SIDE_, N2_, FWPS_, kFilterAdd>(a, st); \
+    }
+    DDF_CHAIN(64, 64, 64, 3, 3)
+    DDF_CHAIN(64, 0, 64, 4, 3)
+    DDF_CHAIN(64, 0, 128, 3, 3)
+    DDF_CHAIN(128, 0, 128, 2, 2)
+    DDF_CHAIN(128, 0, 256, 2, 2)
 #undef DDF_CHAIN
     return hipErrorNotSupported;
 }

@@ -10,6 +10,7 @@ namespace net {
 
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t rows_u4 __attribute__((ext_vector_type(4)));
+using rows::half2_t;
 
 constexpr int kThreads = 256;
 constexpr int kXcd = 8;
@@ -63,6 +64,86 @@ __device__ __forceinline__ float add_swapped32(float a, float b) {
 __device__ __forceinline__ float add_swapped16(float a, float b) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+constexpr int kTapPitch = 12;    // a pixel's spatial taps: nine and padding
+
+// The dynamic filter of eight channels of a pixel (k_net_filter's comment has the reasons).
+template <bool MUL, bool WIDE>
+__device__ __forceinline__ void filter_pair(half2_t cv, half2_t sv, half2_t xv, float &a0, float &a1) {
+    if constexpr (WIDE) {
+        const float c0 = (float)cv[0], c1 = (float)cv[1], s0 = (float)sv[0], s1 = (float)sv[1];
+        a0 = fmaf((float)xv[0], MUL ? c0 * s0 : c0 + s0, a0);
+        a1 = fmaf((float)xv[1], MUL ? c1 * s1 : c1 + s1, a1);
+    } else {
+        const half2_t cb = MUL ? cv * sv : cv + sv;
+        a0 = fmaf((float)xv[0], (float)cb[0], a0);
+        a1 = fmaf((float)xv[1], (float)cb[1], a1);
+    }
+}
+
+// The channel taps of eight channels: of filter rows 0 and 1 as a channel's pair, of row 2 as two channels'.
+__device__ __forceinline__ void channel_taps(const _Float16 *cf, uint32_t (&cfa)[3][8], uint32_t (&cfb)[3][4]) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(cf);
+    uint32_t wd[36];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const uint4 q = src[i];
+        wd[4 * i] = q.x; wd[4 * i + 1] = q.y; wd[4 * i + 2] = q.z; wd[4 * i + 3] = q.w;
+    }
+    auto half_at = [&](int i) { return (i & 1) ? wd[i / 2] >> 16 : wd[i / 2] & 0xffffu; };
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) cfa[j][e] = half_at(9 * e + j) | (half_at(9 * e + 3 + j) << 16);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) cfb[j][k] = half_at(18 * k + 6 + j) | (half_at(18 * k + 15 + j) << 16);
+    }
+}
+
+// Rows 0 and 1 of a column as a channel's pair each, once for the three results it is under.
+__device__ __forceinline__ void pair_column(uint32_t (&col)[3][4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t top = col[0][k], low = col[1][k];
+        col[0][k] = __builtin_amdgcn_perm(low, top, 0x05040100);
+        col[1][k] = __builtin_amdgcn_perm(low, top, 0x07060302);
+    }
+}
+
+// The sums of a result from its three (paired) columns and the pixel's taps.
+template <bool MUL, bool WIDE>
+__device__ __forceinline__ void filter_sums(const uint32_t (&cfa)[3][8], const uint32_t (&cfb)[3][4], const uint32_t (&c0)[3][4],
+                                            const uint32_t (&c1)[3][4], const uint32_t (&c2)[3][4], const uint32_t (&tp)[6],
+                                            float (&acc)[8]) {
+    // spatial taps j and 3 + j
+    const uint32_t sa[3] = {__builtin_amdgcn_perm(tp[1], tp[0], 0x07060100), __builtin_amdgcn_perm(tp[2], tp[0], 0x05040302),
+                            __builtin_amdgcn_perm(tp[2], tp[1], 0x07060100)};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    // (all indices constants: a loop over j was unrolled too late in larger kernels, its taps went through memory)
+    rows::static_for<0, 3>([&](auto column) __attribute__((always_inline)) {
+        constexpr int j = decltype(column)::value;
+        const uint32_t(&at)[3][4] = j == 0 ? c0 : j == 1 ? c1 : c2;
+        const half2_t sp = __builtin_bit_cast(half2_t, sa[j]);
+        const half2_t sb = __builtin_bit_cast(half2_t, tp[(6 + j) / 2]);
+        const half2_t sv = {sb[j & 1], sb[j & 1]};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const half2_t xv = __builtin_bit_cast(half2_t, at[e & 1][e / 2]), cv = __builtin_bit_cast(half2_t, cfa[j][e]);
+            if constexpr (WIDE) {
+                const float f0 = (float)cv[0], f1 = (float)cv[1], s0 = (float)sp[0], s1 = (float)sp[1];
+                acc[e] = fmaf((float)xv[0], MUL ? f0 * s0 : f0 + s0, acc[e]);
+                acc[e] = fmaf((float)xv[1], MUL ? f1 * s1 : f1 + s1, acc[e]);
+            } else {
+                acc[e] = __builtin_amdgcn_fdot2(xv, MUL ? cv * sp : cv + sp, acc[e], false);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, cfb[j][k]), sv, __builtin_bit_cast(half2_t, at[2][k]),
+                                   acc[2 * k], acc[2 * k + 1]);
+    });
 }
 
 // This wave's loads but the last N have arrived and its LDS reads are done; then all waves'.

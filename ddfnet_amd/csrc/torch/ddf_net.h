@@ -146,6 +146,12 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
         if (i + 1 == p.blocks.size() || (down && b.stride != 1)) return 0;
         return ddf_hip_net_conv_chain_parts(n, ho, wo, b.width, down ? c : 0, b.conv3.t[0]->size(0), p.blocks[i + 1].width);
     };
+    // (whether that launch makes block i's dynamic filter, too)
+    auto filtered = [n, &p](size_t i, int64_t ho, int64_t wo, int64_t c) {
+        const NetBlock &b = p.blocks[i];
+        return b.stride == 1 && ddf_hip_net_filter_chain_parts(n, ho, wo, b.width, b.down.t[0].defined() ? c : 0,
+                                                               b.conv3.t[0]->size(0), p.blocks[i + 1].width) > 0;
+    };
     // chained: what the launch that made b's first results has left, 0 where that is one of its own
     auto parts_of = [n](const NetBlock &b, int64_t h, int64_t w, int64_t c, int64_t chained) {
         const int64_t count = chained ? chained : ddf_hip_net_conv_pool_parts(n, h, w, c, b.width);
@@ -194,12 +200,20 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             const Parts of = parts_of(b, h, w, c, chained);
             chained = chain_parts(i, ho, wo, c);
             if (of.summed) covered(ddf_hip_net_sum_parts(pp, of.count, pt, n, width, st));
+            const float *const pooled = of.summed ? pt : pp;
+            const int count = of.summed ? 1 : of.count;
+            const bool fused = chained && filtered(i, ho, wo, c);
             nm = b.bn2.norm();
-            covered(ddf_hip_net_ddf(
-                t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, of.summed ? pt : pp,
-                of.summed ? 1 : of.count, b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(), ptr_or_null(b.b2),
-                cf, b.mid, b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset), &nm, t2, n, h, w, width,
-                b.stride, b.combine, st));
+            if (fused)
+                covered(ddf_hip_net_branches(t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pooled, count,
+                                             b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid,
+                                             b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset), n, h, w, width, 1, st));
+            else
+                covered(ddf_hip_net_ddf(t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pooled, count,
+                                        b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid,
+                                        b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset), &nm, t2, n, h, w, width,
+                                        b.stride, b.combine, st));
+            const ddf_net_norm_t nm2 = nm;
             nm = b.conv3.norm();
             const ddf_net_norm_t down = b.down.norm();
             if (chained) {
@@ -207,9 +221,17 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
                 const ddf_net_norm_t nm1 = next.conv1.norm();
                 const bool side = b.down.t[0].defined();
                 void *to = side ? other : cur;
-                covered(ddf_hip_net_conv_chain(t2, b.conv3.t[0]->data_ptr(), &nm, side ? nullptr : cur, side ? cur : nullptr,
-                                               ptr_or_null(b.down.t[0]), &down, side ? c : 0, to, next.conv1.t[0]->data_ptr(),
-                                               &nm1, t1, pp, n, ho, wo, width, wide_c, next.width, st));
+                const void *const res = side ? nullptr : cur, *const side_x = side ? cur : nullptr;
+                if (fused) {
+                    covered(ddf_hip_net_filter_chain(t1, cf, sf, &nm2, b.combine, b.conv3.t[0]->data_ptr(), &nm, res, side_x,
+                                                     ptr_or_null(b.down.t[0]), &down, side ? c : 0, to, next.conv1.t[0]->data_ptr(),
+                                                     &nm1, t2, pp, n, ho, wo, width, wide_c, next.width, st));
+                    std::swap(t1, t2);
+                } else {
+                    covered(ddf_hip_net_conv_chain(t2, b.conv3.t[0]->data_ptr(), &nm, res, side_x, ptr_or_null(b.down.t[0]),
+                                                   &down, side ? c : 0, to, next.conv1.t[0]->data_ptr(), &nm1, t1, pp, n, ho, wo,
+                                                   width, wide_c, next.width, st));
+                }
                 if (side) std::swap(cur, other);
             } else if (b.down.t[0].defined()) {
                 covered(ddf_hip_net_conv_pair(t2, b.conv3.t[0]->data_ptr(), &nm, width, cur,

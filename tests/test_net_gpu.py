@@ -271,6 +271,44 @@ def test_conv_chain(n, h, w, c, side, o, next_o, bn):
     assert (total - got_next.double().sum((1, 2))).abs().max() <= 1e-6 * got_next.double().abs().sum((1, 2)).max() + 1e-30
 
 
+@pytest.mark.parametrize('n,h,w,c,side,o,next_o,combine,bn', [
+    (8, 56, 56, 64, 0, 256, 64, 0, 1), (9, 55, 52, 64, 0, 256, 64, 1, 1),          # samples that end inside tiles
+    (21, 56, 56, 64, 64, 256, 64, 0, 1), (70, 33, 28, 64, 0, 192, 128, 1, 0),      # a projection; no BatchNorm
+    (84, 28, 28, 128, 0, 512, 128, 0, 1), (32, 28, 28, 128, 0, 128, 256, 1, 1),
+    (1, 1, 24804, 64, 0, 64, 64, 0, 1), (2, 4100, 4, 64, 64, 64, 64, 0, 1),        # one row (no fused launch: None), rows of one run
+    (3100, 2, 4, 128, 0, 64, 128, 0, 1), (1, 7, 4096, 64, 0, 64, 128, 1, 1),       # samples of a lane's pixels; the widest rows
+])
+def test_filter_chain(n, h, w, c, side, o, next_o, combine, bn):
+    """The filter in front of the chain's launch: what the two calls leave, to the bit."""
+    torch.manual_seed(c + o + next_o + w)
+    x = torch.randn(n, h, w, c, device='cuda').half()
+    cf = torch.randn(n, c, 9, device='cuda').half()
+    sf = torch.randn(n, h * w, 12, device='cuda').half()
+    sf[..., 9:] = float('nan')       # (padding)
+    wt, ws, wn = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((o, c), (o, side or 1), (next_o, o)))
+    (norm_f, _, keep_f), (norm, _, keep), (norm_s, _, keep_s), (norm_n, _, keep_n) = (make_norm(k, bn, 1) for k in (c, o, o, next_o))
+    xs = torch.randn(n, h, w, side, device='cuda').half() if side else None
+    res = None if side else torch.randn(n, h, w, o, device='cuda').half()
+    count = _lib.lib().ddf_hip_net_filter_chain_parts(n, h, w, c, side, o, next_o)
+    assert (count > 0) == (w <= 4096) and _lib.lib().ddf_hip_net_filter_chain_parts(n, h, w + 2, c, side, o, next_o) == 0
+    if not count:
+        return
+    filtered = torch.empty_like(x)
+    call('ddf_hip_net_filter', x, cf, sf, norm_f, filtered, n, h, w, c, 1, combine)
+
+    def outputs():
+        return (res.clone() if res is not None else torch.empty(n, h, w, o, device='cuda', dtype=torch.float16),
+                torch.empty(n, h, w, next_o, device='cuda', dtype=torch.float16),
+                torch.full((n, count + 1, next_o), float('nan'), device='cuda'))
+    want, got = outputs(), outputs()
+    for (out, nxt, parts), filters in ((want, None), (got, (cf, sf, norm_f, combine))):
+        call('ddf_hip_net_filter_chain' if filters else 'ddf_hip_net_conv_chain', x if filters else filtered, *(filters or ()), wt,
+             norm, None if side else out, xs, ws if side else None, norm_s if side else None, side, out, wn, norm_n, nxt, parts,
+             n, h, w, c, o, next_o)
+    for g, v in zip(got, want):
+        assert torch.equal(g.nan_to_num(nan=-7.), v.nan_to_num(nan=-7.))
+
+
 @pytest.mark.parametrize('n,h,w,c,s,mid,n_parts', [
     (1, 56, 56, 64, 1, 12, 49), (70, 6, 10, 64, 2, 12, 3), (300, 4, 4, 64, 1, 12, 1),     # samples past one per compute unit
     (3, 9, 13, 128, 1, 25, 8), (2, 4, 6, 128, 2, 25, 9),
