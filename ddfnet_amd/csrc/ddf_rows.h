@@ -557,6 +557,10 @@ __device__ __forceinline__ double lane_broadcast<double>(double v, int src_lane)
 }
 
 // BWD = false: out = forward(x, cf, sf).  BWD = true: x is dO and out is dX.
+// Whether a lane's feature rows are taken one after another (see compute()).
+template <typename T, int K, int VX, int R, int TAIL>
+constexpr bool by_row() { return K == 5 && R == 1 && VX * sizeof(T) == 16 && (sizeof(T) == 4 || TAIL == 0); }
+
 // WPE: waves per SIMD the register allocation must leave room for.
 // S = 2 (forward, 3 x 3, one row per lane): g describes the result plane, the
 // lane's feature vectors are 2 * VX elements wide (LaneStride2).
@@ -848,14 +852,25 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
             rag.store_features(dr, xb[2], g, ow);
         } else {
         Row row[ROWS];
-#pragma unroll
-        for (int rr = 0; rr < ROWS; ++rr) {
-            if (!row_needed<R, K, D>(rr)) continue;
+        auto prepare = [&](int rr) __attribute__((always_inline)) {
 #pragma unroll
             for (int k = 0; k < NWX; ++k) row[rr].own[k] = xw[ST][rr][k];
             // (stride 2: what lies past the row reaches no result that is stored)
             if constexpr (TAIL && S == 1) rag.fix(row[rr].own);
             row[rr].sides(ln.first, ln.last);
+        };
+        // 25 taps, vectors of 16 bytes: one row after another, each with its neighbours and sums before the next
+        // begins.  Left to itself the compiler fetches the neighbours of all five rows first: 210 registers, two
+        // waves per SIMD, where this takes 158.  us, forward, before / now: fp32 32 x 128 x 56 x 56, taps two apart,
+        // 33.3 / 31.1, 'add' 32.5 / 29.1, taps one apart 27.9 / 25.6, 32 x 256 x 28 x 28 18.9 / 17.0, 8 x 64 x 200 x 300
+        // 66 / 62; fp16 32 x 128 x 56 x 56 29.9 / 27.7, 8 x 64 x 200 x 300 60.8 / 55.2.  (The channel's taps moved to vector
+        // registers as well, whose multiply-adds issue faster: 34.0.)  Not over fp16's ragged rows, which spill at
+        // three waves (15 registers) and take 1 % longer at two, and not with shorter vectors, which have the room anyway.
+        constexpr bool kByRow = by_row<T, K, VX, R, TAIL>();
+        if constexpr (!kByRow) {
+#pragma unroll
+            for (int rr = 0; rr < ROWS; ++rr)
+                if (row_needed<R, K, D>(rr)) prepare(rr);
         }
         A acc[R][VX];
 #pragma unroll
@@ -911,7 +926,13 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
         // mul: x * sf is exact in the accumulator type for fp16 storage and goes
         // into one mixed-precision multiply; add: two multiply-adds
 #pragma unroll
-        for (int i = 0; i < K; ++i)
+        for (int i = 0; i < K; ++i) {
+            if constexpr (kByRow) {
+#pragma unroll
+                for (int e = 0; e < VX; ++e) asm volatile("" : "+v"(acc[0][e]));
+                __builtin_amdgcn_sched_barrier(0);
+                prepare(i * D);
+            }
 #pragma unroll
             for (int j = 0; j < K; ++j)
 #pragma unroll
@@ -927,6 +948,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
                             acc[r][e] = fma_(xv, sv, acc[r][e]);
                         }
                     }
+        }
         }   // (not the dot-product path)
         const __amdgpu_buffer_rsrc_t orr = plane_rsrc(os + (int64_t)ci * out_plane, ci < nch ? out_bytes : 0u);
 #pragma unroll

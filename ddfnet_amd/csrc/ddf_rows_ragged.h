@@ -14,7 +14,7 @@ hipError_t launch_ragged_kd(const Problem &p, const RowsGeom &g, bool backward, 
     const dim3 grid(g.xcd_per * kXcd), block(kWave * g.wpb);
 #define DDF_ROWS_CASE(MUL_, BWD_)                                                               \
     hipLaunchKernelGGL((k_rows<T, K, D, MUL_, BWD_, VX, R, true, stages<K>(),                   \
-                               waves_per_simd<T, K, VX, R>(), 1, TAIL>),                        \
+                               waves_per_simd<T, K, VX, R, TAIL>(), 1, TAIL>),                  \
                        grid, block, 0, st, g, x, cf, sf, out)
     if (p.mul) {
         if (backward) DDF_ROWS_CASE(true, true);
