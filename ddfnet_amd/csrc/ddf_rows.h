@@ -558,8 +558,8 @@ __device__ __forceinline__ double lane_broadcast<double>(double v, int src_lane)
 
 // BWD = false: out = forward(x, cf, sf).  BWD = true: x is dO and out is dX.
 // Whether a lane's feature rows are taken one after another (see compute()).
-template <typename T, int K, int VX, int R, int TAIL>
-constexpr bool by_row() { return K == 5 && R == 1 && VX * sizeof(T) == 16 && (sizeof(T) == 4 || TAIL == 0); }
+template <typename T, int K, int VX, int R>
+constexpr bool by_row() { return K == 5 && R == 1 && VX * sizeof(T) == 16; }
 
 // WPE: waves per SIMD the register allocation must leave room for.
 // S = 2 (forward, 3 x 3, one row per lane): g describes the result plane, the
@@ -863,10 +863,11 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
         // begins.  Left to itself the compiler fetches the neighbours of all five rows first: 210 registers, two
         // waves per SIMD, where this takes 158.  us, forward, before / now: fp32 32 x 128 x 56 x 56, taps two apart,
         // 33.3 / 31.1, 'add' 32.5 / 29.1, taps one apart 27.9 / 25.6, 32 x 256 x 28 x 28 18.9 / 17.0, 8 x 64 x 200 x 300
-        // 66 / 62; fp16 32 x 128 x 56 x 56 29.9 / 27.7, 8 x 64 x 200 x 300 60.8 / 55.2.  (The channel's taps moved to vector
-        // registers as well, whose multiply-adds issue faster: 34.0.)  Not over fp16's ragged rows, which spill at
-        // three waves (15 registers) and take 1 % longer at two, and not with shorter vectors, which have the room anyway.
-        constexpr bool kByRow = by_row<T, K, VX, R, TAIL>();
+        // 66 / 62; fp16 32 x 128 x 56 x 56 29.9 / 27.7, ragged rows, two waves all the same (15 registers spill at three),
+        // 8 x 64 x 200 x 300 60.8 / 55.2, 8 x 96 x 92 x 130 22.7 / 22.9.  (The channel's taps moved to vector registers as
+        // well, whose multiply-adds issue faster: 34.0 where this takes 31.1.)  Shorter vectors have the room anyway and
+        // are 1 % faster without it.
+        constexpr bool kByRow = by_row<T, K, VX, R>();
         if constexpr (!kByRow) {
 #pragma unroll
             for (int rr = 0; rr < ROWS; ++rr)

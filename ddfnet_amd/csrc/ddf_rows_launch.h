@@ -13,7 +13,8 @@ constexpr int kStages = 3;   // channels in flight per wave (one computed, two l
 // waves per SIMD the registers are budgeted for (fp16 with 16 pixels per lane needs the room)
 template <typename T, int K, int VX, int R, int TAIL = 0>
 constexpr int waves_per_simd() {
-    if (K == 5) return by_row<T, K, VX, R, TAIL>() ? 3 : 2;   // 25 taps of 4 or 8 pixels in registers
+    // (25 taps of 4 or 8 pixels in registers)
+    if (K == 5) return by_row<T, K, VX, R>() && (sizeof(T) == 4 || TAIL == 0) ? 3 : 2;
     return sizeof(T) == 2 && VX * R >= 16 ? 2 : 3;
 }
 template <int K>
