@@ -238,7 +238,7 @@ __global__ __launch_bounds__(4 * kWave) void k_spatial_branch_tiles(
 // launcher prefers).  A lane owns VP neighbouring result pixels of one sample
 // (stride 1: the plane is one run of pixels, so a vector may cross image rows;
 // stride 2: the 2 * VP feature pixels under VP result pixels of one row come in
-// as one vector) and adds up KK taps for each.  The WAVES waves of a workgroup
+// as one vector; see vector_of) and adds up KK taps for each.  The WAVES waves of a workgroup
 // cover the same pixels and a range of channels each, U at a time; their sums
 // meet in LDS at the end.  Like the operator's own kernels it has
 //   * every channel plane behind a buffer descriptor (an idle lane's offset and
@@ -249,12 +249,40 @@ struct SpatialGeom {
     int C, W, Wo;
     int plane;      // H * W
     int npix;       // Ho * Wo
-    int nvec;       // npix / VP
+    int nvec;       // vectors of VP result pixels (see vector_of)
+    int vrow;       // stride 2: vectors of a row
     int lpt;        // lanes of a workgroup's pixel tile that have a vector
     int ngroups;    // C / U
     int gpw;        // channel groups per wave
     int steps;      // gpw rounded up to a multiple of NST
 };
+
+// Where vector v of a sample's begins: its first result pixel, its first feature element.  The last vector of
+// the run (stride 2: of a row) ends with it: it begins further left where VP does not divide the
+// run, and its first `again` pixels are the vector's before, too - made twice, alike, and counted once
+// in the planes' sums.  So planes of any size have full vectors (at any element address), no
+// tails and no branches.
+struct VectorAt { int p, in, again; };
+template <int VP, int S>
+__device__ __forceinline__ VectorAt vector_of(const SpatialGeom &g, int v) {
+    if constexpr (S == 1) {
+        const int p = min(v * VP, g.npix - VP);
+        return {p, p, v * VP - p};
+    } else {
+        const int yo = v / g.vrow, at = (v - yo * g.vrow) * VP, xo = min(at, g.Wo - VP);
+        return {yo * g.Wo + xo, 2 * yo * g.W + 2 * xo, at - xo};
+    }
+}
+// Masks of the words of a vector without its first `again` elements (bitwise: an infinity among
+// those must not reach the sums).
+template <typename T, int NW>
+__device__ __forceinline__ void words_from(int again, uint32_t (&mask)[NW]) {
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+        if constexpr (sizeof(T) == 4) mask[k] = k >= again ? ~0u : 0u;
+        else mask[k] = (2 * k >= again ? 0xffffu : 0u) | (2 * k + 1 >= again ? 0xffff0000u : 0u);
+    }
+}
 
 // Sums of U (2 or 4) values per lane over the wave: every lane ends up with the total of
 // value number (lane % U).  The first steps halve the
@@ -292,7 +320,8 @@ __device__ __forceinline__ float wave_sums(const float (&v)[U], int lane) {
 // has in registers anyway.  Under stride 2 (even H and W) the lane also loads the
 // feature row below its own, and both columns where it otherwise takes one; those lines
 // come in with their neighbours in any case.
-template <typename T, int KK, int VP, int S, int WAVES, int U, int NST, bool POOL = false>
+// RAGGED: VP does not divide the run (or the row) of pixels.
+template <typename T, int KK, int VP, int S, int WAVES, int U, int NST, bool POOL = false, bool RAGGED = false>
 __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     SpatialGeom g, const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
     T *__restrict__ sf, float gain, const T *__restrict__ gain_vec, const T *__restrict__ offset_vec,
@@ -309,13 +338,13 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     const int64_t n = blockIdx.z;
     const int v = blockIdx.x * g.lpt + lane;
     const bool live = lane < g.lpt && v < g.nvec;
-    const int p = v * VP;                                      // first of the lane's result pixels
-    int in_off = p;
-    if constexpr (S == 2) {
-        const int yo = p / g.Wo, xo = p - yo * g.Wo;
-        in_off = 2 * yo * g.W + 2 * xo;
-    }
-    const uint32_t xb = live ? (uint32_t)in_off * (uint32_t)sizeof(T) : kOutside;
+    const VectorAt at = vector_of<VP, S>(g, v);
+    const int p = at.p;                                        // first of the lane's result pixels
+    const uint32_t xb = live ? (uint32_t)at.in * (uint32_t)sizeof(T) : kOutside;
+    constexpr bool kMasked = POOL && RAGGED && VP > 1;
+    uint32_t mask[NWX];
+    if constexpr (kMasked) words_from<T, NWX>(S * at.again, mask);
+    auto counted = [&](uint32_t word, int k) __attribute__((always_inline)) { return kMasked ? word & mask[k] : word; };
     const uint32_t plane_bytes = (uint32_t)g.plane * (uint32_t)sizeof(T);
     // the sample's C planes behind one descriptor; a channel is a scalar offset into it
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + n * g.C * (int64_t)g.plane, (uint32_t)g.C * plane_bytes);
@@ -420,9 +449,9 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
                         float part[NWX];
 #pragma unroll
                         for (int k = 0; k < NWX; ++k) {
-                            part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, xw[ST][u][k]), ones, 0.f, false);
+                            part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, counted(xw[ST][u][k], k)), ones, 0.f, false);
                             if constexpr (S == 2)
-                                part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, xlow[ST][u][k]), ones, part[k], false);
+                                part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, counted(xlow[ST][u][k], k)), ones, part[k], false);
                         }
                         if constexpr (NWX == 4) ps = (part[0] + part[1]) + (part[2] + part[3]);
                         else if constexpr (NWX == 2) ps = part[0] + part[1];
@@ -430,8 +459,8 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
                     } else {
 #pragma unroll
                         for (int k = 0; k < NWX; ++k) {
-                            ps += __uint_as_float(xw[ST][u][k]);
-                            if constexpr (S == 2) ps += __uint_as_float(xlow[ST][u][k]);
+                            ps += __uint_as_float(counted(xw[ST][u][k], k));
+                            if constexpr (S == 2) ps += __uint_as_float(counted(xlow[ST][u][k], k));
                         }
                     }
                     psum[u] = ps;
@@ -575,7 +604,7 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
 // took 155 registers, three waves per SIMD and 17.4 us; three groups of 16 in flight 19.0.
 constexpr int kSpatialMmaWaves = 4, kSpatialMmaStages = 2, kSpatialMmaGroup = 16, kSpatialMmaChannels = 2048;
 
-template <int VP, bool POOL>
+template <int VP, bool POOL, bool RAGGED>
 __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_spatial_mma(
     SpatialGeom g, const __half *__restrict__ x, const __half *__restrict__ w, const __half *__restrict__ bias,
     __half *__restrict__ sf, float gain, const __half *__restrict__ gain_vec, const __half *__restrict__ offset_vec,
@@ -590,7 +619,11 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_s
     const bool live = v < g.nvec;
     const uint32_t plane_bytes = (uint32_t)g.plane * 2u;
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(x + n * g.C * (int64_t)g.plane, (uint32_t)g.C * plane_bytes);
-    const uint32_t xb = live ? (uint32_t)v * kVB + (uint32_t)(quarter * 4) * plane_bytes : kOutside;
+    const VectorAt at = vector_of<VP, 1>(g, v);
+    const uint32_t xb = live ? (uint32_t)at.in * 2u + (uint32_t)(quarter * 4) * plane_bytes : kOutside;
+    constexpr bool kMasked = POOL && RAGGED;
+    uint32_t mask[NW];
+    if constexpr (kMasked) words_from<__half, NW>(at.again, mask);
     const __amdgpu_buffer_rsrc_t wr = plane_rsrc(w + (int64_t)head * KK * g.C, (uint32_t)(KK * g.C) * 2u);
     const uint32_t wb = col < KK ? (uint32_t)(col * g.C + quarter * 4) * 2u : kOutside;
 
@@ -598,15 +631,15 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_s
     auto issue = [&](auto st_tag, int i) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_tag)::value;
         const bool have = i < g.ngroups;
-        const uint32_t at = have ? xb : kOutside, cb = (uint32_t)(have ? i * G : 0) * plane_bytes;
+        const uint32_t vb = have ? xb : kOutside, cb = (uint32_t)(have ? i * G : 0) * plane_bytes;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             if constexpr (VP == 8) {
-                const auto q = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)at, (int)(cb + (uint32_t)u * plane_bytes), 0);
+                const auto q = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)vb, (int)(cb + (uint32_t)u * plane_bytes), 0);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) xw[ST][u][k] = q[k];
             } else {
-                const auto q = __builtin_amdgcn_raw_buffer_load_b64(xr, (int)at, (int)(cb + (uint32_t)u * plane_bytes), 0);
+                const auto q = __builtin_amdgcn_raw_buffer_load_b64(xr, (int)vb, (int)(cb + (uint32_t)u * plane_bytes), 0);
                 xw[ST][u][0] = q[0];
                 xw[ST][u][1] = q[1];
             }
@@ -628,7 +661,8 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_s
                     float part[NW];
 #pragma unroll
                     for (int k = 0; k < NW; ++k)
-                        part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, xw[ST][u][k]), ones, 0.f, false);
+                        part[k] = __builtin_amdgcn_fdot2(__builtin_bit_cast(rows::half2_t, kMasked ? xw[ST][u][k] & mask[k] : xw[ST][u][k]),
+                                                         ones, 0.f, false);
                     ps[u] = NW == 4 ? (part[0] + part[1]) + (part[NW - 2] + part[NW - 1]) : part[0] + part[1];
                 }
                 // over the row of sixteen lanes: channel (lane & 3) in each (see wave_sums)
@@ -660,10 +694,10 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_s
     _Float16 taps_of[3][4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int at = head * KK + min(quarter * 4 + r, KK - 1);
-        taps_of[0][r] = gain_vec ? *reinterpret_cast<const _Float16 *>(gain_vec + at) : (_Float16)0;
-        taps_of[1][r] = offset_vec ? *reinterpret_cast<const _Float16 *>(offset_vec + at) : (_Float16)0;
-        taps_of[2][r] = bias ? *reinterpret_cast<const _Float16 *>(bias + at) : (_Float16)0;
+        const int tap = head * KK + min(quarter * 4 + r, KK - 1);
+        taps_of[0][r] = gain_vec ? *reinterpret_cast<const _Float16 *>(gain_vec + tap) : (_Float16)0;
+        taps_of[1][r] = offset_vec ? *reinterpret_cast<const _Float16 *>(offset_vec + tap) : (_Float16)0;
+        taps_of[2][r] = bias ? *reinterpret_cast<const _Float16 *>(bias + tap) : (_Float16)0;
     }
     // (whole rounds: a group past the last one reads zeros)
     for (int i = 0; i < g.ngroups; i += NST)
@@ -681,7 +715,7 @@ __global__ __launch_bounds__(kSpatialMmaWaves * kWave, VP == 8 ? 4 : 6) void k_s
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int t = quarter * 4 + r;
-        ob[r] = live && t < KK ? (uint32_t)v * kVB + (uint32_t)t * tap_bytes : kOutside;
+        ob[r] = live && t < KK ? (uint32_t)at.p * 2u + (uint32_t)t * tap_bytes : kOutside;
     }
     // (taps past the ninth: zero weights, zero bias)
     float gains[4], offsets[4];
@@ -962,13 +996,13 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     // pixels per lane: the widest vector the shapes and addresses allow ...
     const bool pool = pool_part != nullptr;
     if (pool && stride == 2 && (H % 2 != 0 || W % 2 != 0)) return hipErrorNotSupported;   // (pixels no lane covers)
+    // (vectors lie at any element address; a run or a row as long as one has them, see vector_of)
     auto fits = [&](int vp) {
-        if (npix % vp != 0 || ((uintptr_t)sf % (vp * esz)) != 0) return false;
         if (pool && stride == 2 && vp == 1) return ((uintptr_t)x % (2 * esz)) == 0;   // (pairs of columns)
-        if (stride == 1) return ((uintptr_t)x % (vp * esz)) == 0 && (H * W) % vp == 0;
-        if (vp == 1) return true;
-        return Wo % vp == 0 && W % vp == 0 && (H * W) % (2 * vp) == 0 && ((uintptr_t)x % (2 * vp * esz)) == 0;
+        return (stride == 1 ? npix : Wo) >= vp;
     };
+    auto divides = [&](int vp) { return (stride == 1 ? npix : Wo) % vp == 0; };
+    auto vectors = [&](int vp) { return stride == 1 ? cdiv(npix, (int64_t)vp) : Ho * cdiv(Wo, (int64_t)vp); };
     const int vp_max = (stride == 1 ? 16 : 8) / esz;
     // ... that still leaves enough waves to fill the machine: the waves of a workgroup
     // share its pixels and split the channels, at least two pipeline rounds each
@@ -981,13 +1015,23 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     int vp = 0, waves = 1;
     for (int cand = vp_max; cand >= 1; cand /= 2) {
         if (!fits(cand)) continue;
-        const int64_t nvec = npix / cand;
+        const int64_t nvec = vectors(cand);
         const int64_t tiles = cdiv(nvec, kWave) * N * head;
         int wv = 1;
         // (nearly a wave per SIMD with whole channel walks: better than splitting them)
         if (tiles < tune_int("DDF_TUNE_SPATIAL_WHOLE", 768))
             while (wv < 16 && wv * 2 * cand <= 32 && tiles * wv < want && (C / U) / (wv * 2) >= 2 * NST)
                 wv *= 2;
+        // Vectors that do not divide the run, where half as wide ones do not either (or are single pixels): where they
+        // fill the machine, with a quarter to spare where a workgroup is sixteen waves, whose sums meet in
+        // four rounds, or from 1 280 whole walks on, and leave a fifth of the lanes idle at most.  us of a layer's
+        // inference, single pixels (or pairs) / such vectors: fp32 11 x 184 x 79 x 77 56.4 / 43.9, 16 x 128 x 57 x 55 37.9 /
+        // 27.2, 26 x 48 x 65 x 145 41.9 / 39.4, stride 2 8 x 256 x 98 x 98 45.2 / 40.2, fp16 8 x 64 x 199 x 301 71.8 / 60.4,
+        // 16 x 176 x 57 x 55 39.3 / 30.6; left alone 64 x 256 x 15 x 15 26.7 / 27.3, 32 x 256 x 7 x 7 17.1 / 18.1, two heads of
+        // 48 x 432 x 15 x 19 48.0 / 49.8 and 1 x 324 x 165 x 238 52.4 / 56.0, stride 2 32 x 256 x 26 x 30 23.2 / 26.5.
+        if (!divides(cand) && ((cand > 2 && divides(cand / 2)) || nvec * 5 < cdiv(nvec, kWave) * kWave * 4 ||
+                               tiles * wv < (wv == 16 ? want + want / 4 : wv == 1 ? 1280 : want)))
+            continue;
         vp = cand;
         waves = wv;
         if (tiles * wv >= enough(cand) || wv == 1) break;
@@ -1014,7 +1058,7 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
         if (stride == 1 && C % kSpatialMmaGroup == 0 && C <= kSpatialMmaChannels && (uintptr_t)w % 16 == 0 &&
             tune_int("DDF_TUNE_SPATIAL_MMA", 1) != 0) {
             constexpr int kPixels = 4 * kWave;     // of a workgroup, four per lane
-            const int64_t tiles8 = cdiv(npix / 8, kWave), tiles4 = cdiv(npix / 4, kWave), left = channel_parts_left(N, C, C / 5, esz);
+            const int64_t tiles8 = cdiv(vectors(8), kWave), tiles4 = cdiv(vectors(4), kWave), left = channel_parts_left(N, C, C / 5, esz);
             const int64_t full = head * (C <= 64 ? N * tiles4 : N * npix / kPixels);
             const bool odd = (C / kSpatialMmaGroup) % 2 != 0 && C < 64;
             const bool wide = fits(8) && full >= (odd ? 2048 : C <= 64 ? 768 : 256);
@@ -1032,7 +1076,9 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     g.C = (int)C; g.W = (int)W; g.Wo = (int)Wo;
     g.plane = (int)(H * W);
     g.npix = (int)npix;
-    g.nvec = (int)(npix / vp);
+    g.nvec = (int)vectors(vp);
+    g.vrow = (int)cdiv(Wo, (int64_t)vp);
+    const bool ragged = !divides(vp);
     const int tiles = (int)cdiv(g.nvec, kWave);
     g.lpt = (int)cdiv(g.nvec, tiles);                   // (tiles of equal size)
     g.ngroups = (int)(mma ? C / kSpatialMmaGroup : C / U);
@@ -1053,13 +1099,15 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     if constexpr (esz == 2) {
         if (mma) {
             const int lds = pool ? kSpatialMmaWaves * g.C * (int)sizeof(float) : 0;
-#define DDF_SPATIAL_MMA(VP_, POOL_)                                                               \
-    hipLaunchKernelGGL((k_spatial_mma<VP_, POOL_>), grid, dim3(kSpatialMmaWaves * kWave), lds, st, g, x, w, bias, sf, \
-                       (float)gain, gain_vec, offset_vec, parts_out, raw)
-            if (vp == 8 && pool) DDF_SPATIAL_MMA(8, true);
-            else if (vp == 8) DDF_SPATIAL_MMA(8, false);
-            else if (pool) DDF_SPATIAL_MMA(4, true);
-            else DDF_SPATIAL_MMA(4, false);
+#define DDF_SPATIAL_MMA(VP_, POOL_, RAGGED_)                                                      \
+    hipLaunchKernelGGL((k_spatial_mma<VP_, POOL_, RAGGED_>), grid, dim3(kSpatialMmaWaves * kWave), lds, st, g, x, w, bias, \
+                       sf, (float)gain, gain_vec, offset_vec, parts_out, raw)
+            if (vp == 8 && pool && ragged) DDF_SPATIAL_MMA(8, true, true);
+            else if (vp == 8 && pool) DDF_SPATIAL_MMA(8, true, false);
+            else if (vp == 8) DDF_SPATIAL_MMA(8, false, false);
+            else if (pool && ragged) DDF_SPATIAL_MMA(4, true, true);
+            else if (pool) DDF_SPATIAL_MMA(4, true, false);
+            else DDF_SPATIAL_MMA(4, false, false);
 #undef DDF_SPATIAL_MMA
             if (collapse) return collapse_parts(parts_out, tiles, pool_part, N, C, st);
             return hipGetLastError();
@@ -1067,6 +1115,12 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
     }
 #define DDF_STREAM_LAUNCH(VP_, S_, WAVES_)                                                        \
     do {                                                                                          \
+        if (pool && ragged) {                                                                     \
+            hipLaunchKernelGGL((k_spatial_stream<T, KK, VP_, S_, WAVES_, U, NST, true, (VP_ > 1)>), grid, \
+                               dim3(WAVES_ * kWave), 0, st, g, x, w, bias, sf, (float)gain,       \
+                               gain_vec, offset_vec, parts_out, raw);                             \
+            break;                                                                                \
+        }                                                                                         \
         if (pool) {                                                                               \
             hipLaunchKernelGGL((k_spatial_stream<T, KK, VP_, S_, WAVES_, U, NST, true>), grid,    \
                                dim3(WAVES_ * kWave), 0, st, g, x, w, bias, sf, (float)gain,       \

@@ -219,6 +219,56 @@ def test_spatial_branch_on_the_matrix_cores(case, vectors):
     assert torch.isinf(parts2[0, :, 5].sum()) and torch.isfinite(parts2.sum(1)).sum().item() == n * c - 1
 
 
+# runs (stride 2: rows) that end inside a vector, by 1 to VP - 1 pixels: of four and two pixels in fp32, of eight, four
+# and two in fp16, under stride 2, on the matrix cores (16-channel groups); a run one pixel longer than a vector
+RAGGED_CASES = [
+    (80, 12, 17, 55, 1, 2, 'f', 2), (26, 48, 27, 43, 1, 2, 'f', 2), (22, 100, 51, 13, 1, 2, 'f', 2), (9, 200, 45, 23, 1, 2, 'f', 2),
+    (46, 12, 63, 53, 1, 2, 'f', 4), (53, 48, 31, 37, 1, 2, 'f', 4), (45, 100, 15, 41, 1, 2, 'f', 4), (80, 12, 90, 38, 2, 2, 'f', 2),
+    (64, 48, 110, 14, 2, 2, 'f', 2), (68, 100, 110, 6, 2, 2, 'f', 2), (16, 200, 90, 22, 2, 2, 'f', 2),
+    (74, 12, 19, 55, 1, 2, 'h', 2), (64, 100, 7, 61, 1, 2, 'h', 2), (26, 200, 9, 57, 1, 2, 'h', 2), (80, 12, 65, 29, 1, 2, 'h', 4),
+    (54, 100, 41, 25, 1, 2, 'h', 4), (46, 200, 41, 15, 1, 2, 'h', 4), (65, 12, 75, 63, 1, 2, 'h', 8), (65, 100, 75, 22, 1, 2, 'h', 8),
+    (80, 12, 38, 94, 2, 2, 'h', 2), (64, 200, 106, 6, 2, 2, 'h', 2), (59, 12, 118, 82, 2, 2, 'h', 4),
+    (32, 64, 7, 6, 1, 2, 'h', 4), (40, 48, 51, 53, 1, 1, 'h', 4), (12, 64, 151, 149, 1, 2, 'h', 8), (40, 256, 45, 47, 1, 1, 'h', 8),
+    (65000, 16, 1, 9, 1, 1, 'h', 8),
+]
+
+
+@pytest.mark.parametrize('shift', [0, 1])
+@pytest.mark.parametrize('case', RAGGED_CASES, ids=lambda c: 'x'.join(map(str, c)))
+def test_spatial_branch_whose_runs_end_inside_a_vector(case, shift):
+    """Every pixel once in the sums, all taps; what is not finite stays with its pixel and its channel, also
+    where it is one that two vectors hold; tensors at odd element addresses."""
+    n, c, h, w_, s, head, kind, vp = case
+    dtype = {'f': torch.float32, 'h': torch.float16}[kind]
+    torch.manual_seed(c + h)
+    store = torch.randn(n * c * h * w_ + shift, device='cuda').to(dtype)
+    x = store[shift:].view(n, c, h, w_)
+    w = (torch.randn(head * 9, c, device='cuda') * 0.2).to(dtype)
+    b = torch.randn(head * 9, device='cuda').to(dtype)
+    sf, parts = _lib.spatial_branch_pool(x, w, b, head, 3, s, 0.7, None, None)
+    run, lines = (h // s * (w_ // s), 1) if s == 1 else (w_ // s, h // s)
+    assert run % vp and parts.shape[1] in (1, -(-(lines * -(-run // vp)) // 64)), parts.shape
+    again = _lib.spatial_branch_pool(x, w, b, head, 3, s, 0.7, None, None)
+    assert torch.equal(sf, again[0]) and torch.equal(parts, again[1])
+    assert torch.equal(sf, _lib.spatial_branch(x, w, b, head, 3, s, 0.7, None, None))
+    few = slice(0, min(n, 64))
+    ref = spatial_reference(x[few].cpu(), w.cpu(), b.cpu(), head, 3, s, 0.7, None, None)
+    # (as the other tests of this kernel: a tap's spread of nine values divides its rounding)
+    assert ((sf[few].double().cpu() - ref).abs().max() / ref.abs().max()).item() < {'f': 2e-5, 'h': 4e-3}[kind]
+    sums, scale = x.double().sum((2, 3)), x.double().abs().sum((2, 3)).max()
+    assert ((parts.double().sum(1) - sums).abs().max() / scale).item() < 1e-6
+    yl, xl = (h // s - 1) * s, (w_ // s - 1) * s
+    x[n - 1, 5, yl, xl - s] = float('inf')       # (held by the last vector and the one before it, or the last only)
+    sf2, parts2 = _lib.spatial_branch_pool(x, w, b, head, 3, s, 0.7, None, None)
+    at = torch.zeros(h // s, w_ // s, dtype=torch.bool, device='cuda')
+    at[-1, -2] = True
+    assert torch.isnan(sf2[n - 1][:, at]).all()
+    sf2[n - 1][:, at] = sf[n - 1][:, at]
+    assert torch.equal(sf2, sf)
+    total = parts2.sum(1)
+    assert torch.isposinf(total[n - 1, 5]) and torch.isfinite(total).sum().item() == n * c - 1
+
+
 def test_spatial_branch_pool_turns_down_what_it_cannot_cover():
     x = torch.randn(2, 16, 9, 8, device='cuda')
     w5 = torch.randn(25, 16, device='cuda')
