@@ -166,12 +166,12 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
     };
     const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) _Float16 *)net_smem;
-    auto load = [&](int buf) {
+    // (load i of a stage; first those of x)
+    auto load_one = [&](int i, int buf) __attribute__((always_inline)) {
         const uint32_t at = ring + (uint32_t)(buf * STAGE) * 2 + (uint32_t)wave * (kWave * 16);
-#pragma unroll
-        for (int i = 0; i < RX; ++i, xp[i - 1] += KST) load_to_lds(at + i * kThreads * 16, xp[i]);
-#pragma unroll
-        for (int i = 0; i < RW; ++i, wp[i - 1] += KST) load_to_lds(at + BM * KST * 2 + i * kThreads * 16, wp[i]);
+        const _Float16 *&p = i < RX ? xp[i < RX ? i : 0] : wp[i < RX ? 0 : i - RX];
+        load_to_lds(at + (i < RX ? i * kThreads * 16 : BM * KST * 2 + (i - RX) * kThreads * 16), p);
+        p += KST;
     };
     const int wm = wave & 1, wn = wave >> 1;
     const int l32 = lane & 31, hi = lane >> 5;
@@ -206,27 +206,40 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                     for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)b[e];
             }
     }
-    auto multiply = [&](int buf) __attribute__((always_inline)) {
+    // `meanwhile`: what goes out behind the products of a step, the stage's loads spread over its steps.  The
+    // next step's operands are asked for in front of a step's products: left to itself the compiler keeps one set of
+    // registers for operands, and every step waits out LDS.  Batch 128, us before / now: 14 x 14 x 1024 -> 256 24.2 / 22.5,
+    // -> 512 43.5 / 38.0, 7 x 7 x 512 -> 2048 25.5 / 23.1, 2048 -> 512 30.4 / 29.4, 28 x 28 x 512 -> 256 42.2 / 41.0.  (All loads
+    // behind the first step 23.1 and 41.3; a raised priority around the products 23.9 and 42.2.)
+    constexpr int STEPS = KST / 16;
+    auto multiply = [&](int buf, auto meanwhile) __attribute__((always_inline)) {
         const _Float16 *s = net_smem + buf * STAGE;
-#pragma unroll
-        for (int kk = 0; kk < KST / 16; ++kk) {
+        half8_t xv[2][TM], wv[2][TN];
+        auto operands = [&](int kk) __attribute__((always_inline)) {
             const int ch = kk * 2 + hi;
-            half8_t xv[TM], wv[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                const int r = wm * (BM / 2) + i * 32 + l32;
-                xv[i] = *reinterpret_cast<const half8_t *>(s + r * KST + (ch ^ turn(r)) * 8);
-            }
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int r = wn * (BN / 2) + j * 32 + l32;
-                wv[j] = *reinterpret_cast<const half8_t *>(s + BM * KST + r * KST + (ch ^ turn(r)) * 8);
+                wv[kk & 1][j] = *reinterpret_cast<const half8_t *>(s + BM * KST + r * KST + (ch ^ turn(r)) * 8);
             }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int r = wm * (BM / 2) + i * 32 + l32;
+                xv[kk & 1][i] = *reinterpret_cast<const half8_t *>(s + r * KST + (ch ^ turn(r)) * 8);
+            }
+        };
+        operands(0);
+#pragma unroll
+        for (int kk = 0; kk < STEPS; ++kk) {
+            if (kk + 1 < STEPS) operands(kk + 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[j], xv[i], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[kk & 1][j], xv[kk & 1][i], acc[i][j], 0, 0, 0);
+            meanwhile(kk);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     // what the tile's results meet on their way out: this thread's eight channels, and the
@@ -269,7 +282,8 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     }
     auto load_stage = [&](int k, int buf) __attribute__((always_inline)) {
         if (PAIR && k == nk0) aim(a);
-        load(buf);
+#pragma unroll
+        for (int i = 0; i < RX + RW; ++i) load_one(i, buf);
     };
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
@@ -286,8 +300,9 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
     }
     int buf = 0;
-    auto multiply_stage = [&](int k) __attribute__((always_inline)) {
-        multiply(buf);
+    auto nothing = [](int) __attribute__((always_inline)) {};
+    auto multiply_stage = [&](int k, auto meanwhile) __attribute__((always_inline)) {
+        multiply(buf, meanwhile);
         buf = buf == ST - 1 ? 0 : buf + 1;
         if constexpr (PAIR) {
             if (k == nk0 - 1) {
@@ -314,14 +329,17 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             if (k + 1 < nk) arrive<(ST - 2) * (RX + RW)>();
             else arrive<0>();
             if (k + ST - 1 < nk) load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
-            multiply_stage(k);
+            multiply_stage(k, nothing);
         }
     } else {
         int k = 0;
         for (; k < nk - 2; ++k) {
             arrive<(ST - 2) * (RX + RW)>();
-            load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
-            multiply_stage(k);
+            const int to = buf == 0 ? ST - 1 : buf - 1;
+            multiply_stage(k, [&](int kk) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = kk * (RX + RW) / STEPS; i < (kk + 1) * (RX + RW) / STEPS; ++i) load_one(i, to);
+            });
         }
         if (nk > 1) {
             arrive<(ST - 2) * (RX + RW)>();
@@ -331,10 +349,10 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         }
         residual();
         if (nk > 1) {
-            multiply_stage(k);
+            multiply_stage(k, nothing);
             arrive<RES ? RO : 0>();
         }
-        multiply_stage(nk - 1);
+        multiply_stage(nk - 1, nothing);
     }
     __syncthreads();
     float one = 1.f;
