@@ -58,7 +58,7 @@ SYMBOLS = {
     'ddf_hip_net_conv_chain_parts': (_i64, [_i64] * 7),
     'ddf_hip_net_conv_chain': (_i, [_vp] * 7 + [_i64] + [_vp] * 5 + [_i64] * 6 + [_vp]),
     'ddf_hip_net_filter_chain_parts': (_i64, [_i64] * 7),
-    'ddf_hip_net_filter_chain': (_i, [_vp] * 4 + [_i] + [_vp] * 6 + [_i64] + [_vp] * 5 + [_i64] * 6 + [_vp]),
+    'ddf_hip_net_filter_chain': (_i, [_vp] * 4 + [ctypes.c_double, _vp, _i] + [_vp] * 6 + [_i64] + [_vp] * 5 + [_i64] * 6 + [_vp]),
     'ddf_hip_net_stem': (_i, [_vp] * 4 + [_i64] * 3 + [_vp]),
     'ddf_hip_net_spatial': (_i, [_vp] * 5 + [ctypes.POINTER(ctypes.c_int)] + [_i64] * 4 + [_i, ctypes.c_double, _vp]),
     'ddf_hip_net_branches': (_i, [_vp] * 4 + [ctypes.c_double, _vp, _i] + [_vp] * 5 + [_i64, ctypes.c_double] + [_vp] * 2 +

@@ -832,9 +832,9 @@ int64_t ddf_hip_net_filter_chain_parts(int64_t N, int64_t H, int64_t W, int64_t 
 }
 
 namespace {
-// (spatial_filter null: no filter in front)
-int net_chain_impl(const char *name, const void *features, const void *channel_filter, const void *spatial_filter,
-                   const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
+// (channel_filter null: no filter in front)
+int net_chain_impl(const char *name, const void *features, const void *channel_filter, const void *spatial_weight,
+                   const void *spatial_bias, double spatial_gain, const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
                    const void *residual, const void *side_features, const void *side_weight, const ddf_net_norm_t *side_norm,
                    int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm, void *next,
                    float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O, int64_t next_O, void *stream) {
@@ -845,12 +845,12 @@ int net_chain_impl(const char *name, const void *features, const void *channel_f
         return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
     if (N == 0) return DDF_OK;
     const int64_t M = N * H * W;
-    if (!ddf::net_chain_covers(M, C, side_C, O, next_O) || (spatial_filter && !ddf::net_chain_filters(W, C)))
+    if (!ddf::net_chain_covers(M, C, side_C, O, next_O) || (channel_filter && !ddf::net_chain_filters(W, C)))
         return fail(DDF_ERR_UNSUPPORTED, "%s: sizes not covered", name);
     const ddf::NetChain a{features, weight, residual, side_features, side_weight, next_weight, output, next, pool_parts,
                           net_norm(norm), net_norm(side_norm), net_norm(next_norm), M, (int)C, (int)side_C, (int)O,
-                          (int)next_O, (int)(H * W), channel_filter, spatial_filter, net_norm(filter_norm), (int)W,
-                          combine == DDF_MUL, 0, 0};
+                          (int)next_O, (int)(H * W), channel_filter, spatial_weight, spatial_bias, (float)spatial_gain,
+                          net_norm(filter_norm), (int)W, combine == DDF_MUL, 0, 0};
     return net_result(ddf::net_chain(a, (hipStream_t)stream), name);
 }
 }  // namespace
@@ -860,20 +860,21 @@ int ddf_hip_net_conv_chain(const void *features, const void *weight, const ddf_n
                            int64_t side_C, void *output, const void *next_weight, const ddf_net_norm_t *next_norm,
                            void *next, float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O,
                            int64_t next_O, void *stream) {
-    return net_chain_impl("ddf_hip_net_conv_chain", features, nullptr, nullptr, nullptr, DDF_MUL, weight, norm, residual,
+    return net_chain_impl("ddf_hip_net_conv_chain", features, nullptr, nullptr, nullptr, 0.0, nullptr, DDF_MUL, weight, norm, residual,
                           side_features, side_weight, side_norm, side_C, output, next_weight, next_norm, next, pool_parts, N,
                           H, W, C, O, next_O, stream);
 }
 
-int ddf_hip_net_filter_chain(const void *features, const void *channel_filter, const void *spatial_filter,
-                             const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
+int ddf_hip_net_filter_chain(const void *features, const void *channel_filter, const void *spatial_weight,
+                             const void *spatial_bias, double spatial_gain, const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
                              const void *residual, const void *side_features, const void *side_weight,
                              const ddf_net_norm_t *side_norm, int64_t side_C, void *output, const void *next_weight,
                              const ddf_net_norm_t *next_norm, void *next, float *pool_parts, int64_t N, int64_t H, int64_t W,
                              int64_t C, int64_t O, int64_t next_O, void *stream) {
     if (combine != DDF_MUL && combine != DDF_ADD) return fail(DDF_ERR_BAD_ARG, "unknown combine %d", combine);
-    if (!channel_filter || !spatial_filter || !net_norm_ok(filter_norm)) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
-    return net_chain_impl("ddf_hip_net_filter_chain", features, channel_filter, spatial_filter, filter_norm, combine, weight,
+    if (!channel_filter || !spatial_weight || !net_norm_ok(filter_norm)) return fail(DDF_ERR_BAD_ARG, "null tensor pointer");
+    return net_chain_impl("ddf_hip_net_filter_chain", features, channel_filter, spatial_weight, spatial_bias, spatial_gain,
+                          filter_norm, combine, weight,
                           norm, residual, side_features, side_weight, side_norm, side_C, output, next_weight, next_norm, next,
                           pool_parts, N, H, W, C, O, next_O, stream);
 }

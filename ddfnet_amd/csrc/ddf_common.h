@@ -171,8 +171,9 @@ hipError_t net_conv(const NetConv &a, hipStream_t st);
 hipError_t net_conv_pair(const NetConv &a, const NetConv &first, hipStream_t st);
 // out (M, N) = relu(norm(x (M, K) . w (N, K)) + res), with side_K > 0 relu(norm(..) + side_norm(side (M, side_K)
 // . side_w (N, side_K))); next (M, N2) = relu(norm2(out . w2 (N2, N))) and its sums over the pixels of
-// each sample (npix), in net_chain_pool_slots parts.  With sf, x holds the features of images W wide and what is
-// multiplied is relu(filter_norm(the operator)) with the filters cf and sf, as net_filter makes it.
+// each sample (npix), in net_chain_pool_slots parts.  With cf, x holds the features of images W wide and what is
+// multiplied is relu(filter_norm(the operator)) with the filters cf and the spatial branch's (tap_w, tap_bias,
+// tap_gain), as net_branches and net_filter make it.
 struct NetChain {
     const void *x, *w, *res, *side, *side_w, *w2;
     void *out, *next;
@@ -180,13 +181,14 @@ struct NetChain {
     NetNorm norm, side_norm, norm2;
     int64_t M;
     int K, side_K, N, N2, npix;
-    const void *cf, *sf;
+    const void *cf, *tap_w, *tap_bias;
+    float tap_gain;
     NetNorm filter_norm;
     int W, mul;
     int tiles, pool_slots;    // (net_chain's own)
 };
 bool net_chain_covers(int64_t M, int64_t K, int64_t side_K, int64_t N, int64_t N2);
-// whether the filter is made in front of it by the same launch
+// whether the spatial branch and the filter are made in front of it by the same launch
 bool net_chain_filters(int64_t W, int64_t K);
 int net_chain_pool_slots(int64_t M, int npix);
 hipError_t net_chain(NetChain a, hipStream_t st);

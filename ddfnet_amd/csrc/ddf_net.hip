@@ -11,7 +11,8 @@
 //   k_net_branches  spatial and channel filter branch
 //   k_net_filter    dynamic filter + BatchNorm + ReLU
 //   k_net_conv
-// (with many pixels the last two and the next one's first are one, k_net_chain of ddf_net_chain.hip)
+// (with many pixels all but the channel branch are one with the next one's first, k_net_chain of
+// ddf_net_chain.hip)
 // and k_net_stem is the 7x7 convolution, BatchNorm, ReLU and max-pool in one.
 // At batch 128 the network took 8.85 ms as torch modules around the operator: 3.2 ms of
 // BatchNorm, 1.6 ms of ReLU and additions, 3 ms of convolutions (ddf_resnet.py:34-111 of
@@ -34,54 +35,6 @@ using rows::from_left;
 using rows::kOutside;
 using rows::load_words;
 using rows::plane_rsrc;
-
-// ---- spatial filter branch of sixteen pixels ------------------------------------------
-// Pixels are the columns, the nine taps nine of the sixteen rows of 16x16x32 steps over the
-// channels; both operands contiguous.  A pixel's taps end up on four lanes, which normalise them
-// across the wave's rows; they are stored as (pixel, kTapPitch), nine taps and padding.
-
-template <int KS>
-struct TapWeights {
-    static constexpr int KK = 9;
-    half8_t w[KS];
-    uint16_t b[4];
-    // (rows past the ninth, and a bias that is not there, lie outside their buffers: zeros)
-    __device__ __forceinline__ void request(const _Float16 *weight, const _Float16 *bias, int lane) {
-        const int col = lane & 15, quad = lane >> 4;
-        const __amdgpu_buffer_rsrc_t wr = plane_rsrc(weight, KK * KS * 64), br = plane_rsrc(bias, bias ? KK * 2 : 0);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-            w[ks] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(wr, col * KS * 64 + quad * 16, ks * 64, 0));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) b[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, (quad * 4 + e) * 2, 0, 0);
-    }
-    // v: channels ks * 32 + quad * 8 .. + 7 of the lane's pixel; `at`: where its taps go
-    __device__ __forceinline__ void taps(const half8_t (&v)[KS], float gain, bool there, _Float16 *sf, int64_t at, int lane) const {
-        const int quad = lane >> 4;
-        float4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[ks], v[ks], acc, 0, 0, 0);
-        // taps 4 * quad + e of the pixel (rows past the ninth: zero weights, zero bias)
-        float f[4], s = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            f[e] = acc[e] + (float)__builtin_bit_cast(_Float16, b[e]);
-            s += f[e];
-        }
-        const float mean = rows_total(s) / (float)KK;
-        float sq = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            f[e] -= mean;
-            if (quad * 4 + e < KK) sq += f[e] * f[e];
-        }
-        const float inv = gain / (sqrtf(rows_total(sq) / (float)(KK - 1)) + 1e-10f);
-        half4_t o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (_Float16)(f[e] * inv);
-        if (there && quad < 3) *reinterpret_cast<half4_t *>(sf + at * kTapPitch + quad * 4) = o;
-    }
-};
 
 // ---- 1x1 convolution ----------------------------------------------------------
 // out[m, o] = act(affine(sum_k x[row(m), k] w[o, k]) (+ res[m, o])), row(m) the sampled

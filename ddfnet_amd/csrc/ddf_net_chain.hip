@@ -1,5 +1,5 @@
-// A bottleneck's dynamic filter, its last 1x1 convolution and the next one's first in one launch
-// (DDF-ResNet inference, fp16, channels-last; ddf_resnet.py:34-111 of the reference composes them).
+// A bottleneck's spatial filter branch and dynamic filter, its last 1x1 convolution and the next one's
+// first in one launch (DDF-ResNet inference, fp16, channels-last; ddf_resnet.py:34-111 of the reference composes them).
 #include <numeric>
 #include <type_traits>
 
@@ -42,31 +42,45 @@ struct ChainLds {    // halves; K2: channels of the side product, 0: none
     static constexpr int filtered = norms - kChainRows * (K + 8);    // at the start: a wave's filtered pixels
     static_assert(filtered >= wd + kChunk * K2, "and do not meet the first weights");
     // scale, shift, what a sum starts with; of the wide channels (and of the side product), of next's
-    static constexpr int bytes(int N) { return norms * 2 + (N * (K2 ? 5 : 3) + N2 * 3) * 4; }
+    static constexpr int floats(int N) { return N * (K2 ? 5 : 3) + N2 * 3; }
+    // with a filter: behind them the spatial taps of the tile's pixels
+    static constexpr int bytes(int N, bool filter) { return norms * 2 + floats(N) * 4 + (filter ? kChainRows * kTapPitch * 2 : 0); }
 };
 
-// ---- the dynamic filter in front --------------------------------------------------------
+// ---- spatial branch and dynamic filter in front -----------------------------------------------
 // A wave's 32 pixels of x, filtered, normalised and rounded as k_net_filter does it, to its part of LDS
 // (rows of K + 8).  K / 8 lanes own four neighbouring pixels at a time, eight channels each, so a channel's
 // taps are paired once for all of a lane's pixels and six columns serve four results; rows of images are
-// whole runs of four (W % 4 == 0), as tiles are.  Pixels past the last are made from zeros.
-// The filter's results, 103 MB of a batch of 128 at 56 x 56, never reach memory; what is left of its time is a chain of
-// round trips in front of each tile's products, which the compute unit's other workgroups cover in part (44
-// registers more than four of them leave spill: 150 us where three take 105).  us, filter and the launch behind it / this, batch
-// 128: 56 x 56 x 64 -> 256 -> 64 125 / 106, with the projection 128 / 116, -> 128 144 / 125, 28 x 28 x 128 -> 512 -> 128 72 /
-// 63; batch 16: 22.4 / 18.4, 27.1 / 22.4, 24.6 / 20.6; batch 8 20 / 14, 20.6 / 17.9, 20.2 / 15.9.
+// whole runs of four (W % 4 == 0), as tiles are.  Pixels past the last are made from zeros.  The pixels' spatial
+// taps are made from their channels, which the filter reads in any case (TapWeights: the same bits as
+// k_net_branches), and stay in LDS.
+// Neither the filter's results, 103 MB of a batch of 128 at 56 x 56, nor the taps reach memory, and the features are
+// read once instead of twice; what is left is a chain of round trips in front of each tile's products, which the
+// compute unit's other workgroups cover in part (44 registers more than four of them leave spill: 150 us where
+// three take 105).  us, filter and the launch behind it / those in one, batch 128: 56 x 56 x 64 -> 256 -> 64 125 / 106, with
+// the projection 128 / 116, -> 128 144 / 125, 28 x 28 x 128 -> 512 -> 128 72 / 63.  Both branches, filter and that
+// launch / the channel branch and this, batch 128: 139 / 113, 143 / 127, 157 / 130, 84 / 72; batch 64: 69 / 57, 77 / 64, 76 / 64,
+// 50 / 42; batch 8: 30 / 22 (as are all at 56 x 56).
 constexpr int kRun = 4;
 template <int K, bool MUL>
-__device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int wave, int lane, _Float16 *to) {
-    constexpr int LP = K / 8, SLOTS = kWave / LP, PER = 32 / SLOTS, RING = 5;
+__device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int wave, int lane, _Float16 *to, _Float16 *sf) {
+    constexpr int KS = K / 32, LP = K / 8, SLOTS = kWave / LP, PER = 32 / SLOTS, RING = 5;
     static_assert(PER % kRun == 0);
     const int cl = lane % LP, H = a.npix / a.W, W = a.W;
     // (all offsets from a pixel in front of the tile's neighbours: a tile's are 32-bit ones)
     const int64_t base = m0 - W - 1 > 0 ? m0 - W - 1 : 0;
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(static_cast<const _Float16 *>(a.x) + base * K,
                                                  (uint32_t)(min(a.M - base, (int64_t)(2 * W + 2 + kChainRows)) * K * 2));
-    const __amdgpu_buffer_rsrc_t tr = plane_rsrc(static_cast<const _Float16 *>(a.sf) + m0 * kTapPitch,
-                                                 (uint32_t)(min(a.M - m0, (int64_t)kChainRows) * kTapPitch * 2));
+    // the spatial taps of the wave's pixels, sixteen at a time
+    TapWeights<KS> weights;
+    weights.request(static_cast<const _Float16 *>(a.tap_w), static_cast<const _Float16 *>(a.tap_bias), lane);
+    half8_t own[2][KS];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            own[i][ks] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                xr, (int)(((int)(m0 - base) + wave * 32 + i * 16 + (lane & 15)) * K + (lane >> 4) * 8) * 2, ks * 64, 0));
     const bool bn = a.filter_norm.var;
     auto parameter = [&](bool there, const void *p) __attribute__((always_inline)) {    // (zeros where there is none)
         return __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(plane_rsrc(p, there && p ? K * 2 : 0), cl * 16, 0, 0));
@@ -99,15 +113,17 @@ __device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int
             constexpr int Q = decltype(slot)::value;
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                const auto v = __builtin_amdgcn_raw_buffer_load_b64(tr, (px + Q) * kTapPitch * 2 + i * 8, 0, 0);
-                tap[Q][2 * i] = v[0];
-                tap[Q][2 * i + 1] = v[1];
+                const uint2 v = *reinterpret_cast<const uint2 *>(sf + (px - wave * 32 + Q) * kTapPitch + i * 4);
+                tap[Q][2 * i] = v.x;
+                tap[Q][2 * i + 1] = v.y;
             }
         };
         if (run == 0 || a.npix % PER) channel_taps(static_cast<const _Float16 *>(a.cf) + ((int64_t)n * K + cl * 8) * 9, cfa, cfb);
         rows::static_for<0, RING - 1>(column);
-        rows::static_for<0, 2>(taps);
         if (run == 0) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) weights.taps(own[i], a.tap_gain, true, sf, i * 16 + (lane & 15), lane);
+            asm volatile("" ::: "memory");    // (a wave's LDS operations keep their order)
             const float eps = bn ? a.filter_norm.eps : 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -115,6 +131,7 @@ __device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int
                 sh[e] = (float)nb[e] + ((float)nc[e] - (float)nm[e]) * sc[e];
             }
         }
+        rows::static_for<0, 2>(taps);
         rows::static_for<0, kRun>([&](auto q) __attribute__((always_inline)) {
             constexpr int Q = decltype(q)::value;
             if constexpr (Q + RING - 1 < kRun + 2) column(std::integral_constant<int, Q + RING - 1>{});
@@ -256,7 +273,8 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
     half8_t xv[K / 16], dv[K2 ? K2 / 16 : 1];
     if constexpr (FILTER) {
         _Float16 *const mine = chain_smem + L::filtered + wave * 32 * (K + 8);
-        filter_pixels<K, FILTER == kFilterMul>(a, m0, wave, lane, mine);
+        _Float16 *const taps = reinterpret_cast<_Float16 *>(norms + L::floats(N)) + wave * 32 * kTapPitch;
+        filter_pixels<K, FILTER == kFilterMul>(a, m0, wave, lane, mine, taps);
         asm volatile("" ::: "memory");    // (a wave's LDS operations keep their order)
 #pragma unroll
         for (int k = 0; k < K / 16; ++k) xv[k] = *reinterpret_cast<const half8_t *>(mine + l32 * (K + 8) + k * 16 + hi * 8);
@@ -507,7 +525,7 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
 
 template <int K, int K2, int N2, int WPS, int FILTER>
 hipError_t launch_chain(const NetChain &a, hipStream_t st) {
-    const int lds = ChainLds<K, K2, N2>::bytes(a.N);
+    const int lds = ChainLds<K, K2, N2>::bytes(a.N, FILTER);
     hipLaunchKernelGGL((k_net_chain<K, K2, N2, WPS, FILTER>), dim3(xcd_grid(a.tiles)), dim3(kThreads), lds, st, a);
     return hipGetLastError();
 }
@@ -541,12 +559,12 @@ int net_chain_pool_slots(int64_t M, int npix) {
 hipError_t net_chain(NetChain a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_chain_covers(a.M, a.K, a.side_K, a.N, a.N2)) return hipErrorNotSupported;
-    if (a.sf && !net_chain_filters(a.W, a.K)) return hipErrorNotSupported;
+    if (a.cf && !net_chain_filters(a.W, a.K)) return hipErrorNotSupported;
     a.tiles = (int)cdiv(a.M, kChainRows);
     a.pool_slots = net_chain_pool_slots(a.M, a.npix);
 #define DDF_CHAIN(K_, SIDE_, N2_, WPS_, FWPS_) \
     if (a.K == K_ && a.side_K == SIDE_ && a.N2 == N2_) {                                            \
-        if (!a.sf) return launch_chain<K_, SIDE_, N2_, WPS_, kNoFilter>(a, st);                     \
+        if (!a.cf) return launch_chain<K_, SIDE_, N2_, WPS_, kNoFilter>(a, st);                     \
         return a.mul ? launch_chain<K_, SIDE_, N2_, FWPS_, kFilterMul>(a, st) : launch_chain<K_, SIDE_, N2_, FWPS_, kFilterAdd>(a, st); \
     }
     DDF_CHAIN(64, 64, 64, 3, 3)

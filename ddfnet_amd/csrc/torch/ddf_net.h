@@ -146,7 +146,7 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
         if (i + 1 == p.blocks.size() || (down && b.stride != 1)) return 0;
         return ddf_hip_net_conv_chain_parts(n, ho, wo, b.width, down ? c : 0, b.conv3.t[0]->size(0), p.blocks[i + 1].width);
     };
-    // (whether that launch makes block i's dynamic filter, too)
+    // (whether that launch makes block i's spatial branch and dynamic filter, too)
     auto filtered = [n, &p](size_t i, int64_t ho, int64_t wo, int64_t c) {
         const NetBlock &b = p.blocks[i];
         return b.stride == 1 && ddf_hip_net_filter_chain_parts(n, ho, wo, b.width, b.down.t[0].defined() ? c : 0,
@@ -205,9 +205,9 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
             const bool fused = chained && filtered(i, ho, wo, c);
             nm = b.bn2.norm();
             if (fused)
-                covered(ddf_hip_net_branches(t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pooled, count,
-                                             b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid,
-                                             b.cgain_const, ptr_or_null(b.cgain), ptr_or_null(b.coffset), n, h, w, width, 1, st));
+                covered(ddf_hip_channel_branch_parts(pooled, count, 1.0 / (double)(h * w), b.w1->data_ptr(), ptr_or_null(b.b1),
+                                                     b.w2->data_ptr(), ptr_or_null(b.b2), cf, n, width, b.mid, 3, b.cgain_const,
+                                                     ptr_or_null(b.cgain), ptr_or_null(b.coffset), DDF_F16, st));
             else
                 covered(ddf_hip_net_ddf(t1, b.ws->data_ptr(), ptr_or_null(b.bs), sf, b.sgain, pooled, count,
                                         b.w1->data_ptr(), ptr_or_null(b.b1), b.w2->data_ptr(), ptr_or_null(b.b2), cf, b.mid,
@@ -223,8 +223,8 @@ inline py::object net_forward(const NetPlan &p, const at::Tensor &input) {
                 void *to = side ? other : cur;
                 const void *const res = side ? nullptr : cur, *const side_x = side ? cur : nullptr;
                 if (fused) {
-                    covered(ddf_hip_net_filter_chain(t1, cf, sf, &nm2, b.combine, b.conv3.t[0]->data_ptr(), &nm, res, side_x,
-                                                     ptr_or_null(b.down.t[0]), &down, side ? c : 0, to, next.conv1.t[0]->data_ptr(),
+                    covered(ddf_hip_net_filter_chain(t1, cf, b.ws->data_ptr(), ptr_or_null(b.bs), b.sgain, &nm2, b.combine,
+                                                     b.conv3.t[0]->data_ptr(), &nm, res, side_x, ptr_or_null(b.down.t[0]), &down, side ? c : 0, to, next.conv1.t[0]->data_ptr(),
                                                      &nm1, t2, pp, n, ho, wo, width, wide_c, next.width, st));
                     std::swap(t1, t2);
                 } else {

@@ -372,7 +372,7 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *           results with next_weight (next_O, O), both with ReLU, in one launch that leaves
  *           ddf_hip_net_conv_chain_parts partial sums (0: sizes that want the two calls).  residual may
  *           be output; next overlaps neither, and no input
- *   filter_chain  filter (stride 1) and conv_chain of its results in one launch (_parts 0: sizes that
+ *   filter_chain  the spatial branch, filter (stride 1) and conv_chain of its results in one launch (_parts 0: sizes
  *           want the two calls).  next may not be features: other workgroups still read a pixel's
  *           neighbours
  *   sum_parts  totals (N, C) of n_parts such partial sums per sample and channel
@@ -408,8 +408,8 @@ int ddf_hip_net_conv_chain(const void *features, const void *weight, const ddf_n
                            void *next, float *pool_parts, int64_t N, int64_t H, int64_t W, int64_t C, int64_t O,
                            int64_t next_O, void *stream);
 int64_t ddf_hip_net_filter_chain_parts(int64_t N, int64_t H, int64_t W, int64_t C, int64_t side_C, int64_t O, int64_t next_O);
-int ddf_hip_net_filter_chain(const void *features, const void *channel_filter, const void *spatial_filter,
-                             const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
+int ddf_hip_net_filter_chain(const void *features, const void *channel_filter, const void *spatial_weight,
+                             const void *spatial_bias, double spatial_gain, const ddf_net_norm_t *filter_norm, int combine, const void *weight, const ddf_net_norm_t *norm,
                              const void *residual, const void *side_features, const void *side_weight,
                              const ddf_net_norm_t *side_norm, int64_t side_C, void *output, const void *next_weight,
                              const ddf_net_norm_t *next_norm, void *next, float *pool_parts, int64_t N, int64_t H, int64_t W,

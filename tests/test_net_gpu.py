@@ -279,12 +279,11 @@ def test_conv_chain(n, h, w, c, side, o, next_o, bn):
     (3100, 2, 4, 128, 0, 64, 128, 0, 1), (1, 7, 4096, 64, 0, 64, 128, 1, 1),       # samples of a lane's pixels; the widest rows
 ])
 def test_filter_chain(n, h, w, c, side, o, next_o, combine, bn):
-    """The filter in front of the chain's launch: what the two calls leave, to the bit."""
+    """The spatial branch and the filter in front of the chain's launch: what the three calls leave, to the bit."""
     torch.manual_seed(c + o + next_o + w)
     x = torch.randn(n, h, w, c, device='cuda').half()
     cf = torch.randn(n, c, 9, device='cuda').half()
-    sf = torch.randn(n, h * w, 12, device='cuda').half()
-    sf[..., 9:] = float('nan')       # (padding)
+    tap_w, tap_b = (torch.randn(9, c, device='cuda') * c ** -0.5).half(), torch.randn(9, device='cuda').half() if bn else None
     wt, ws, wn = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((o, c), (o, side or 1), (next_o, o)))
     (norm_f, _, keep_f), (norm, _, keep), (norm_s, _, keep_s), (norm_n, _, keep_n) = (make_norm(k, bn, 1) for k in (c, o, o, next_o))
     xs = torch.randn(n, h, w, side, device='cuda').half() if side else None
@@ -293,7 +292,9 @@ def test_filter_chain(n, h, w, c, side, o, next_o, combine, bn):
     assert (count > 0) == (w <= 4096) and _lib.lib().ddf_hip_net_filter_chain_parts(n, h, w + 2, c, side, o, next_o) == 0
     if not count:
         return
-    filtered = torch.empty_like(x)
+    filtered, sf = torch.empty_like(x), torch.empty(n, h * w, 12, device='cuda', dtype=torch.float16)
+    sums, n_sums = torch.empty(n, 1, c, device='cuda'), ctypes.c_int(0)
+    call('ddf_hip_net_spatial', x, tap_w, tap_b, sf, sums, ctypes.byref(n_sums), n, h, w, c, 1, 0.7)
     call('ddf_hip_net_filter', x, cf, sf, norm_f, filtered, n, h, w, c, 1, combine)
 
     def outputs():
@@ -301,7 +302,7 @@ def test_filter_chain(n, h, w, c, side, o, next_o, combine, bn):
                 torch.empty(n, h, w, next_o, device='cuda', dtype=torch.float16),
                 torch.full((n, count + 1, next_o), float('nan'), device='cuda'))
     want, got = outputs(), outputs()
-    for (out, nxt, parts), filters in ((want, None), (got, (cf, sf, norm_f, combine))):
+    for (out, nxt, parts), filters in ((want, None), (got, (cf, tap_w, tap_b, 0.7, norm_f, combine))):
         call('ddf_hip_net_filter_chain' if filters else 'ddf_hip_net_conv_chain', x if filters else filtered, *(filters or ()), wt,
              norm, None if side else out, xs, ws if side else None, norm_s if side else None, side, out, wn, norm_n, nxt, parts,
              n, h, w, c, o, next_o)
