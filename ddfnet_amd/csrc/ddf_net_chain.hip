@@ -532,18 +532,18 @@ hipError_t launch_chain(const NetChain &a, hipStream_t st) {
 
 }  // namespace
 
-// Whether the two convolutions are one launch: three quarters of a workgroup per compute unit at least (us, two
-// launches / one: 8 x 56 x 56, 196 workgroups, 14.5 / 14.0 and 18.7 / 17.0 with the projection; 16 x 28 x 28, 98 of
-// them, 15.8 / 23.3; 32 x 28 x 28, 196, 26 / 23); where 256 channels follow, two workgroups at most, which
-// then run side by side (28 x 28 x 128 -> 512 -> 256: 32 images 30.1 / 28.9, 64 47.8 / 43.8, 96, 588 workgroups, 63.9 / 70.3).
+// Whether the two convolutions are one launch: with the spatial branch and the filter in front of it, as
+// networks have it, that pays from few tiles on.  us for a whole network, as separate launches / as one: 64 channels, 98
+// tiles (4 x 224 x 224) 375 / 371, 147 411 / 404, 49 337 / 342; 128 channels, 98 tiles (16 x 224 x 224) 505 / 523, 128 516 / 525,
+// 147 586 / 582.  Where 256 channels follow, two workgroups run side by side on a compute unit and a second
+// round of them may be half full, which the launches that are saved make up for: 128 x 28 x 28 x 128 -> 512 -> 256 with
+// what is in front of it 103 / 84 us, the network 1653 / 1622.
 bool net_chain_covers(int64_t M, int64_t K, int64_t side, int64_t N, int64_t N2) {
-    constexpr int kFew = 192, kSideBySide = 512;
     if (N % kChunk || N < kChunk || N > kMaxWide || M > INT32_MAX - 256) return false;
     const int64_t tiles = cdiv(M, kChainRows);
-    if (tiles < kFew) return false;
+    if (tiles < (K == 64 ? 96 : 144)) return false;
     if (side) return K == 64 && side == 64 && N2 == 64;
-    if (K == 64) return N2 == 64 || N2 == 128;
-    return K == 128 && (N2 == 128 || (N2 == 256 && tiles <= kSideBySide));
+    return (K == 64 && (N2 == 64 || N2 == 128)) || (K == 128 && (N2 == 128 || N2 == 256));
 }
 
 // (runs of four pixels; rows of 4096, far more than an image has, keep a tile's neighbours within 2 MB.  No

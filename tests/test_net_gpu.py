@@ -275,6 +275,7 @@ def test_conv_chain(n, h, w, c, side, o, next_o, bn):
     (8, 56, 56, 64, 0, 256, 64, 0, 1), (9, 55, 52, 64, 0, 256, 64, 1, 1),          # samples that end inside tiles
     (21, 56, 56, 64, 64, 256, 64, 0, 1), (70, 33, 28, 64, 0, 192, 128, 1, 0),      # a projection; no BatchNorm
     (84, 28, 28, 128, 0, 512, 128, 0, 1), (32, 28, 28, 128, 0, 128, 256, 1, 1),
+    (4, 56, 56, 64, 64, 64, 64, 0, 1),                                              # fewest tiles
     (1, 1, 24804, 64, 0, 64, 64, 0, 1), (2, 4100, 4, 64, 64, 64, 64, 0, 1),        # one row (no fused launch: None), rows of one run
     (3100, 2, 4, 128, 0, 64, 128, 0, 1), (1, 7, 4096, 64, 0, 64, 128, 1, 1),       # samples of a lane's pixels; the widest rows
 ])
