@@ -254,6 +254,12 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     }
     int buf = 0;
     auto nothing = [](int) __attribute__((always_inline)) {};
+    auto loads_to = [&](int to) __attribute__((always_inline)) {
+        return [&, to](int kk) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = kk * (RX + RW) / STEPS; i < (kk + 1) * (RX + RW) / STEPS; ++i) load_one(i, to);
+        };
+    };
     auto multiply_stage = [&](int k, auto meanwhile) __attribute__((always_inline)) {
         multiply(buf, meanwhile);
         buf = buf == ST - 1 ? 0 : buf + 1;
@@ -278,21 +284,27 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     // residual's RO, which are asked for a stage earlier than they were and in one go (a branch for
     // each and a wait between them took a memory latency per tile).  No load moves across arrive().
     if constexpr (PAIR) {
-        for (int k = 0; k < nk; ++k) {
+        int k = 0;
+        if constexpr (STEPS > 2) {
+            for (; k < nk - (ST - 1); ++k) {
+                arrive<(ST - 2) * (RX + RW)>();
+                if (k + ST - 1 == nk0) aim(a);
+                multiply_stage(k, loads_to(buf == 0 ? ST - 1 : buf - 1));
+            }
+        }
+        // (short stages, three workgroups a unit: 75 us where the loads between the steps take 78, 128 x 28 x 28 x
+        // 128 + 256 -> 512)
+        for (; k < nk; ++k) {
             if (k + 1 < nk) arrive<(ST - 2) * (RX + RW)>();
             else arrive<0>();
-            if (k + ST - 1 < nk) load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+            if (STEPS <= 2 && k + ST - 1 < nk) load_stage(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
             multiply_stage(k, nothing);
         }
     } else {
         int k = 0;
         for (; k < nk - 2; ++k) {
             arrive<(ST - 2) * (RX + RW)>();
-            const int to = buf == 0 ? ST - 1 : buf - 1;
-            multiply_stage(k, [&](int kk) __attribute__((always_inline)) {
-#pragma unroll
-                for (int i = kk * (RX + RW) / STEPS; i < (kk + 1) * (RX + RW) / STEPS; ++i) load_one(i, to);
-            });
+            multiply_stage(k, loads_to(buf == 0 ? ST - 1 : buf - 1));
         }
         if (nk > 1) {
             arrive<(ST - 2) * (RX + RW)>();
@@ -1045,7 +1057,7 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     const int64_t tiles = cdiv(a.M, BM) * tiles_n;
     if (tiles > (1 << 30)) return hipErrorInvalidConfiguration;
     const int lds = conv_lds_halves<BM, BN, KST, ST>() * (int)sizeof(_Float16);
-    constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) < 64 * 1024;
+    constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) <= 64 * 1024;
     if (first && !kPair) return hipErrorNotSupported;
     if (first)
         hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
@@ -1077,11 +1089,15 @@ bool conv_in_tiles(const NetConv &a) {
 // 42.2 / 43.4, 392 of 14 x 14 x 1024 -> 256 24.1 / 28.5).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
 // 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
 enum ConvTile { kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64, kTileSplit };
+// The same holds for pairs (batch 128, short / long: 7 x 7 x 512 + 1024 -> 2048, 784 tiles, 67.5 / 54, 32 x 28 x 28 x 128 + 256
+// -> 512, 784, 25.2 / 24; 64 images of it, 1568 tiles, 40.1 / 41.7, 128 76.4 / 79.9), but where three
+// workgroups per unit are one round and two a full one or more (a network of 96 images, 588 tiles, 1351 / 1357, of
+// 64 of 256 x 256, 512, 1085 / 1088).
 ConvTile conv_tile(const NetConv &a, bool pair) {
     auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
     constexpr int kMany = 1024, kFew = 320;
     if (!conv_in_tiles(a)) return kTileSplit;
-    if (a.N >= 128 && count(128, 128) >= (pair ? kFew : kMany)) return kTile128;
+    if (a.N >= 128 && (count(128, 128) >= kMany || (pair && count(128, 128) >= 512 && count(128, 128) <= 768))) return kTile128;
     if (a.N >= 128 && count(128, 128) >= kFew) return kTile128Long;
     if (count(128, 64) >= kMany) return kTile128x64;
     if (count(128, 64) >= 448) return kTile128x64Long;
