@@ -1018,9 +1018,15 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
         const int64_t nvec = vectors(cand);
         const int64_t tiles = cdiv(nvec, kWave) * N * head;
         int wv = 1;
-        // (nearly a wave per SIMD with whole channel walks: better than splitting them)
+        // (nearly a wave per SIMD with whole channel walks: better than splitting them.  With few waves the walk is all
+        // there is: four share it where that leaves one round each, eight where they are fewest.  us of a layer's
+        // inference, two rounds each at least / so: fp16 7 x 44 x 30 x 24 with two heads 20.1 / 14.4, 1 x 40 x 40 x 43 18.0 / 12.7, 8 x 40 x
+        // 23 x 32 19.7 / 14.1, fp32 54 x 88 x 12 x 8 under stride 2 14.8 / 13.9; eight from more waves on 61 x 140 x 8 x 7 15.2 /
+        // 16.2, sixteen 7 x 144 x 25 x 24 14.9 / 15.9; 200 sizes drawn at random 2.3 % on average.)
+        auto round_is_enough = [&](int wv) { return tiles * wv <= (wv <= 2 ? 512 : wv == 4 ? 128 : 0); };
         if (tiles < tune_int("DDF_TUNE_SPATIAL_WHOLE", 768))
-            while (wv < 16 && wv * 2 * cand <= 32 && tiles * wv < want && (C / U) / (wv * 2) >= 2 * NST)
+            while (wv < 16 && wv * 2 * cand <= 32 && tiles * wv < want &&
+                   (C / U) / (wv * 2) >= (round_is_enough(wv) ? NST : 2 * NST))
                 wv *= 2;
         // Vectors that do not divide the run, where half as wide ones do not either (or are single pixels): where they
         // fill the machine, with a quarter to spare where a workgroup is sixteen waves, whose sums meet in

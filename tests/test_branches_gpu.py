@@ -53,6 +53,7 @@ SPATIAL_CASES = [
     (2, 256, 28, 28, 2, 1), (2, 256, 14, 14, 1, 1), (2, 512, 14, 14, 2, 1), (2, 512, 7, 7, 1, 1),
     (1, 8, 5, 3, 1, 1), (1, 6, 5, 3, 2, 1), (2, 36, 13, 17, 2, 3), (1, 4, 64, 64, 1, 1),
     (5, 1024, 7, 9, 1, 1), (2, 20, 40, 24, 2, 2), (2, 7, 10, 12, 1, 1), (40, 32, 28, 28, 1, 1),
+    (7, 44, 30, 24, 1, 2), (1, 40, 40, 43, 1, 2), (2, 184, 17, 15, 1, 2), (3, 40, 38, 40, 2, 1),    # a round of channels per wave
 ]
 
 
