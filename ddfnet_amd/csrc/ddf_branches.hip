@@ -810,6 +810,44 @@ __global__ __launch_bounds__(kCollapseThreads) void k_collapse_parts(const float
 constexpr int kChannelThreads = 1024;  // sixteen waves: the rows of a block's taps are dealt out to them
 constexpr int kChannelWaves = kChannelThreads / kWave;
 
+// Products of R weight rows (lane sl of sixteen) with NS vectors in LDS, `pitch` apart, vectors of 16
+// bytes at any element address: sixteen single elements are 64 bytes of a row, 32 in fp16, and the address path
+// serves four such rows a load.  us, single elements / vectors: fp32 32 x 512 21.0 / 13.9, 64 x 512 22.2 / 16.2, 56 x 456 19.9 /
+// 15.6, fp16 56 x 456 19.2 / 16.0; up to 384 channels the same.
+template <typename T, int R, int NS>
+__device__ __forceinline__ void row_products(const T *const (&row)[R], int len, const float *x, int pitch, int sl, float (&p)[R][NS]) {
+    constexpr int V = 16 / (int)sizeof(T), kUnroll = R == 1 && NS == 1 ? 8 : 2;
+    struct Pack { T e[V]; };
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) p[u][s] = 0.f;
+#pragma unroll kUnroll
+    for (int c = sl * V; c + V <= len; c += 16 * V) {
+        Pack w[R];
+#pragma unroll
+        for (int u = 0; u < R; ++u) __builtin_memcpy(&w[u], row[u] + c, sizeof(Pack));
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            float xv[V];
+            __builtin_memcpy(xv, x + s * pitch + c, sizeof(xv));
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+#pragma unroll
+                for (int k = 0; k < V; ++k) p[u][s] = fmaf(ld(&w[u].e[k]), xv[k], p[u][s]);
+        }
+    }
+    const int c = len / V * V + sl;    // (what is left of a row: less than a vector)
+    if (c < len) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const float wv = ld(row[u] + c);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) p[u][s] = fmaf(wv, x[s * pitch + c], p[u][s]);
+        }
+    }
+}
+
 // grid (channel blocks of BLOCK channels, groups of NS samples).  LDS: the pooled
 // vectors (NS * C floats), the hidden vectors (NS * mid floats), the block's
 // un-normalised taps (NS * BLOCK * KK).  Every weight a lane loads serves the NS
@@ -874,21 +912,13 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     // hidden vectors: rows of w1
     for (int m0 = wave * 4; m0 < mid; m0 += kChannelWaves * 4) {
         const int m = min(m0 + seg, mid - 1);
-        const T *row = w1 + (int64_t)m * C;
-        float p[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) p[s] = 0.f;
-        int c = sl;
-#pragma unroll 8
-        for (; c < C; c += 16) {
-            const float wv = ld(row + c);
-#pragma unroll
-            for (int s = 0; s < NS; ++s) p[s] = fmaf(wv, v[s * C + c], p[s]);
-        }
+        const T *const row[1] = {w1 + (int64_t)m * C};
+        float p[1][NS];
+        row_products<T, 1, NS>(row, C, v, C, sl, p);
         const float bias = b1 ? ld(b1 + m) : 0.f;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const float tot = row_sum(p[s]);
+            const float tot = row_sum(p[0][s]);
             if (sl == 0 && m0 + seg < mid) {
                 const float hm = relu(tot + bias);
                 h[s * mid + m0 + seg] = hm;
@@ -909,23 +939,8 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         float p[RT][NS];
         const T *wrow[RT];
 #pragma unroll
-        for (int u = 0; u < RT; ++u) {
-#pragma unroll
-            for (int s = 0; s < NS; ++s) p[u][s] = 0.f;
-            wrow[u] = w2 + ((int64_t)cb * KK + min(r0 + 4 * u + seg, rows - 1)) * mid;
-        }
-#pragma unroll 2
-        for (int m = sl; m < mid; m += 16) {
-            float hm[NS];
-#pragma unroll
-            for (int s = 0; s < NS; ++s) hm[s] = h[s * mid + m];
-#pragma unroll
-            for (int u = 0; u < RT; ++u) {
-                const float wv = ld(wrow[u] + m);
-#pragma unroll
-                for (int s = 0; s < NS; ++s) p[u][s] = fmaf(wv, hm[s], p[u][s]);
-            }
-        }
+        for (int u = 0; u < RT; ++u) wrow[u] = w2 + ((int64_t)cb * KK + min(r0 + 4 * u + seg, rows - 1)) * mid;
+        row_products<T, RT, NS>(wrow, mid, h, mid, sl, p);
 #pragma unroll
         for (int u = 0; u < RT; ++u) {
             const int r = r0 + 4 * u + seg;
@@ -1295,8 +1310,9 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
             return hipGetLastError();
         }
     }
-    // (wide layers: fewer, larger blocks, as every block of a sample recomputes the hidden vector)
-    const int block = C >= 512 ? 128 : 64;
+    // (wide layers: fewer, larger blocks, as every block of a sample recomputes the hidden vector, unless smaller ones
+    // still have a compute unit each: fp32 32 x 512 13.9 us in blocks of 128, 11.2 of 64; 40 x 512 14 and 14.8)
+    const int block = C >= 512 && cdiv(C, 64) * N > 256 ? 128 : 64;
     // samples per workgroup: as many as keep every compute unit busy and fit the LDS
     auto lds_of = [&](int ns) { return ((size_t)C + (size_t)mid + (size_t)block * kk) * ns * sizeof(float); };
     int ns = 1;

@@ -98,7 +98,8 @@ def test_spatial_branch_unaligned_views(dtype, tol):
                                    # fp16 on the matrix cores: hidden layers of exactly one step, of a
                                    # step and a few values, of several steps; batches that end inside a tile
                                    (16, 160, 3), (4, 192, 3), (20, 320, 3), (2, 448, 5), (33, 1024, 3),
-                                   (17, 1280, 3)])
+                                   (17, 1280, 3),
+                                   (32, 512, 3), (40, 512, 3), (56, 456, 3), (70, 250, 3), (300, 130, 3), (9, 99, 5)])
 def test_channel_branch_matches_fp64(n, c, k, dtype, tol):
     torch.manual_seed(n + c)
     mid = int(c * 0.2)
