@@ -341,6 +341,12 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
     const VectorAt at = vector_of<VP, S>(g, v);
     const int p = at.p;                                        // first of the lane's result pixels
     const uint32_t xb = live ? (uint32_t)at.in * (uint32_t)sizeof(T) : kOutside;
+    // The row below, which the sums of head 0 need.  For the other heads its offsets lie outside: under a branch
+    // per channel the compiler asks for a step's lower rows before the upper ones.  us, branches / offsets:
+    // fp16 128 x 128 x 56 x 56 26.0 / 24.1, with two heads 35.8 / 35.2, 128 x 256 x 28 x 28 16.4 / 15.0, 8 x 64 x
+    // 200 x 304 16.8 / 15.9, fp32 32 x 128 x 56 x 56 13.3 / 12.9; single pixels keep the branch (128 x 512 x 14 x 14
+    // 16.6 / 17.4).
+    const uint32_t low = live && head == 0 ? xb + (uint32_t)g.W * (uint32_t)sizeof(T) : kOutside;
     constexpr bool kMasked = POOL && RAGGED && VP > 1;
     uint32_t mask[NWX];
     if constexpr (kMasked) words_from<T, NWX>(S * at.again, mask);
@@ -382,10 +388,8 @@ __global__ __launch_bounds__(WAVES * kWave) void k_spatial_stream(
                 for (int k = 0; k < 4; ++k) xw[ST][u][k] = q[k];
             }
             if constexpr (POOL && S == 2) {
-                if (head == 0)
-                    load_vec<kXB>(xr, vb == kOutside ? kOutside : vb + (uint32_t)g.W * (uint32_t)sizeof(T) +
-                                                                       cb + (uint32_t)u * plane_bytes,
-                                  xlow[ST][u]);
+                if (VP > 1 || head == 0)
+                    load_vec<kXB>(xr, have && low != kOutside ? low + cb + (uint32_t)u * plane_bytes : kOutside, xlow[ST][u]);
             }
         }
     };
