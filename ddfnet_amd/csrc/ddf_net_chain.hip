@@ -247,7 +247,8 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
     float *const scale2 = norms + (K2 ? 5 : 3) * N, *const shift2 = scale2 + N2, *const start2 = shift2 + N2;
 
     // (rows past the last pixel read zeros and are not stored: every one of these loads and stores is
-    // issued whatever the tile, the waits below count them)
+    // issued whatever the tile, the waits below count them.  A row is in the lane's offset throughout: the
+    // scalar offset, which moves inside a row, is left out of the descriptor's range check)
     const __amdgpu_buffer_rsrc_t rr = plane_rsrc(K2 ? nullptr : static_cast<const _Float16 *>(a.res) + m0 * N, K2 ? 0 : rows * N * 2);
     const __amdgpu_buffer_rsrc_t orr = plane_rsrc(static_cast<_Float16 *>(a.out) + m0 * N, rows * N * 2);
     const StageRows<kChunk, K> sw(tid, K);
@@ -294,11 +295,17 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
     // a lane's vectors on their way out: eight channels of every eighth pixel
     const int c8 = lane & 7, px0 = wave * 32 + (lane >> 3);
     rows_u4 rv[RV];
+    // (worked out where it is used: four kept in registers spill where four waves share a SIMD's)
+    auto vector_at = [&](int i) __attribute__((always_inline)) {
+        int step = 8 * N * 2;
+        asm volatile("" : "+s"(step));
+        return (px0 * N + c8 * 8) * 2 + i * step;
+    };
     auto residual = [&](int j) __attribute__((always_inline)) {
         if constexpr (K2 == 0) {
 #pragma unroll
             for (int i = 0; i < RV; ++i)
-                rv[i] = __builtin_amdgcn_raw_buffer_load_b128(rr, (px0 * N + c8 * 8) * 2, (i * 8 * N + j * kChunk) * 2, 0);
+                rv[i] = __builtin_amdgcn_raw_buffer_load_b128(rr, vector_at(i), j * (kChunk * 2), 0);
         }
     };
     residual(0);
@@ -416,8 +423,7 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
                 v[i] = __builtin_elementwise_maximum(v[i], half8_t{0, 0, 0, 0, 0, 0, 0, 0});
                 *reinterpret_cast<half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8) = v[i];
             }
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, v[i]), orr, (px0 * N + c8 * 8) * 2,
-                                                   (i * 8 * N + j * kChunk) * 2, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, v[i]), orr, vector_at(i), j * (kChunk * 2), 0);
         }
         // w2's rows are there; everybody is done with w's
         arrive<RV>();

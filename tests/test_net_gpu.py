@@ -311,6 +311,36 @@ def test_filter_chain(n, h, w, c, side, o, next_o, combine, bn):
         assert torch.equal(g.nan_to_num(nan=-7.), v.nan_to_num(nan=-7.))
 
 
+@pytest.mark.parametrize('n,h,w,c,side,o,next_o,filtered', [
+    (1, 1, 12289, 64, 0, 256, 64, 0), (5, 47, 53, 64, 64, 256, 64, 0),        # a last tile of one pixel, of 39
+    (3, 79, 52, 64, 0, 64, 128, 0), (1, 1, 18305, 128, 0, 512, 128, 0), (9, 47, 49, 128, 0, 128, 256, 0),     # 36, 1, 119
+    (9, 55, 52, 64, 0, 256, 64, 1), (1, 53, 236, 64, 64, 256, 64, 1),         # 12, 92
+    (1, 1, 4100 * 3, 64, 0, 64, 128, 0), (1, 3073, 4, 64, 0, 256, 128, 1),    # 12, 4
+    (1, 4577, 4, 128, 0, 512, 128, 1), (23, 33, 28, 128, 0, 512, 256, 1),     # 4, 4
+])
+def test_chains_store_nothing_behind_the_last_pixel(n, h, w, c, side, o, next_o, filtered):
+    """Tiles that end early: rows of another value behind both results stay, also where the residual is the output."""
+    torch.manual_seed(c + o + next_o + w)
+    m, behind = n * h * w, 128
+    assert m % 128
+    x = torch.randn(m, c, device='cuda').half()
+    wt, ws, wn = ((torch.randn(a, b, device='cuda') * b ** -0.5).half() for a, b in ((o, c), (o, side or 1), (next_o, o)))
+    (norm_f, _, keep_f), (norm, _, keep), (norm_s, _, keep_s), (norm_n, _, keep_n) = (make_norm(k, 1, 1) for k in (c, o, o, next_o))
+    front = (torch.randn(n, c, 9, device='cuda').half(), (torch.randn(9, c, device='cuda') * c ** -0.5).half(), None, 0.7, norm_f, 0)
+    xs = torch.randn(m, side, device='cuda').half() if side else None
+    name = 'filter' if filtered else 'conv'
+    count = getattr(_lib.lib(), 'ddf_hip_net_%s_chain_parts' % name)(n, h, w, c, side, o, next_o)
+    assert count > 0
+    parts = torch.full((n * count + 1, next_o), 7., device='cuda')
+    out, nxt = (torch.full((m + behind, k), 7., device='cuda', dtype=torch.float16) for k in (o, next_o))
+    if not side:
+        out[:m].normal_()
+    call('ddf_hip_net_%s_chain' % name, x, *(front if filtered else ()), wt, norm, None if side else out, xs,
+         ws if side else None, norm_s if side else None, side, out, wn, norm_n, nxt, parts, n, h, w, c, o, next_o)
+    assert (out[m:] == 7).all() and (nxt[m:] == 7).all() and (parts[-1] == 7).all()
+    assert torch.isfinite(out).all() and not (out[:m] == 7).all(1).any() and not (nxt[:m] == 7).all(1).any()
+
+
 @pytest.mark.parametrize('n,h,w,c,s,mid,n_parts', [
     (1, 56, 56, 64, 1, 12, 49), (70, 6, 10, 64, 2, 12, 3), (300, 4, 4, 64, 1, 12, 1),     # samples past one per compute unit
     (3, 9, 13, 128, 1, 25, 8), (2, 4, 6, 128, 2, 25, 9),
