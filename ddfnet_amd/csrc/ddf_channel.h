@@ -322,8 +322,9 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
     if (wave < kPoolWaves) {
         const int stride = kPoolWaves / share;    // samples at a time
         if (a.parts) {
-            // (a sample at a time behind a descriptor: beyond its partial sums there are zeros)
-            const uint32_t bytes = (uint32_t)(a.nparts * C) * 4u;
+            // (a sample at a time behind a descriptor: beyond its partial sums there are zeros.  The row is in the lane's
+            // offset: a scalar one is left out of the range check)
+            const uint32_t bytes = (uint32_t)(a.nparts * C) * 4u, row = (uint32_t)(share * C) * 4u;
             auto sample = [&](int s) __attribute__((always_inline)) {
                 return rows::plane_rsrc(a.parts + (int64_t)(n0 + min(s, ns - 1)) * a.nparts * C, s < ns ? bytes : 0u);
             };
@@ -331,14 +332,14 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
                 const __amdgpu_buffer_rsrc_t r[2] = {sample(s), sample(s + stride)};
                 for (int c4 = lane; c4 < c4s; c4 += kWave) {
                     float4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                    uint32_t at = (uint32_t)(g * C + c4 * 4) * 4u;
                     for (int q0 = g; q0 < a.nparts; q0 += kMmaRound * share) {
                         float4_t x[2][kMmaRound];
 #pragma unroll
-                        for (int i = 0; i < 2; ++i)
+                        for (int u = 0; u < kMmaRound; ++u, at += row)
 #pragma unroll
-                            for (int u = 0; u < kMmaRound; ++u)
-                                x[i][u] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                    r[i], c4 * 16, (q0 + u * share) * C * 4, 0));
+                            for (int i = 0; i < 2; ++i)
+                                x[i][u] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r[i], (int)at, 0, 0));
                         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                         for (int i = 0; i < 2; ++i)

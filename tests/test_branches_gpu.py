@@ -304,6 +304,21 @@ def test_channel_branch_parts_matches_fp64(n, c, k, tiles, dtype, tol):
     assert err < tol, err
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('n,c,mid,tiles', [(1, 256, 51, 1), (2, 256, 51, 9), (3, 160, 32, 13), (17, 320, 64, 11),
+                                           (5, 64, 12, 3), (300, 96, 19, 2)])
+def test_channel_branch_reads_no_partial_sums_but_its_own(n, c, mid, tiles, dtype):
+    """Partial sums are asked for eight at a time: NaN in front of and behind them stays out of every filter."""
+    torch.manual_seed(c + mid)
+    around = torch.full((n * tiles * c + 2 * 64 * c,), float('nan'), device='cuda')
+    parts = around[64 * c:-64 * c].view(n, tiles, c).normal_()
+    w1 = (torch.randn(mid, c, device='cuda') * c ** -0.5).to(dtype)
+    w2 = (torch.randn(c * 9, mid, device='cuda') * mid ** -0.5).to(dtype)
+    out = _lib.channel_branch_parts(parts, 0.25, w1, None, w2, None, 3, 0.7)
+    assert torch.equal(out, _lib.channel_branch_parts(parts.clone(), 0.25, w1, None, w2, None, 3, 0.7))
+    assert torch.isfinite(out).all()
+
+
 @pytest.mark.parametrize('dtype,tol', [(torch.float32, 2e-5), (torch.float16, 6e-3)])
 @pytest.mark.parametrize('n,c,mid,tiles', [(1, 64, 16, 1), (3, 64, 17, 8), (2, 65, 16, 9), (3, 128, 31, 8), (2, 129, 32, 3),
                                            (2, 257, 20, 2), (3, 300, 65, 8), (1, 511, 3, 9), (2, 1, 1, 1)])
