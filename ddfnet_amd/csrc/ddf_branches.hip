@@ -814,19 +814,18 @@ __global__ __launch_bounds__(kCollapseThreads) void k_collapse_parts(const float
 constexpr int kChannelThreads = 1024;  // sixteen waves: the rows of a block's taps are dealt out to them
 constexpr int kChannelWaves = kChannelThreads / kWave;
 
-// Products of R weight rows (lane sl of sixteen) with NS vectors in LDS, `pitch` apart, vectors of 16
-// bytes at any element address: sixteen single elements are 64 bytes of a row, 32 in fp16, and the address path
-// serves four such rows a load.  us, single elements / vectors: fp32 32 x 512 21.0 / 13.9, 64 x 512 22.2 / 16.2, 56 x 456 19.9 /
-// 15.6, fp16 56 x 456 19.2 / 16.0; up to 384 channels the same.
-template <typename T, int R, int NS>
+// Products of R weight rows (lane sl of sixteen) with NS vectors in LDS, `pitch` apart.  WIDE: as vectors of 16
+// bytes at any element address; sixteen single elements are 64 bytes of a row, 32 in fp16, and the address path
+// serves four such rows a load.
+template <typename T, int R, int NS, bool WIDE>
 __device__ __forceinline__ void row_products(const T *const (&row)[R], int len, const float *x, int pitch, int sl, float (&p)[R][NS]) {
-    constexpr int V = 16 / (int)sizeof(T), kUnroll = R == 1 && NS == 1 ? 8 : 2;
+    constexpr int V = WIDE ? 16 / (int)sizeof(T) : 1;
     struct Pack { T e[V]; };
 #pragma unroll
     for (int u = 0; u < R; ++u)
 #pragma unroll
         for (int s = 0; s < NS; ++s) p[u][s] = 0.f;
-#pragma unroll kUnroll
+#pragma unroll 2
     for (int c = sl * V; c + V <= len; c += 16 * V) {
         Pack w[R];
 #pragma unroll
@@ -841,13 +840,51 @@ __device__ __forceinline__ void row_products(const T *const (&row)[R], int len, 
                 for (int k = 0; k < V; ++k) p[u][s] = fmaf(ld(&w[u].e[k]), xv[k], p[u][s]);
         }
     }
-    const int c = len / V * V + sl;    // (what is left of a row: less than a vector)
-    if (c < len) {
+    if constexpr (WIDE) {    // (what is left of a row: less than a vector)
+        const int c = len / V * V + sl;
+        if (c < len) {
 #pragma unroll
-        for (int u = 0; u < R; ++u) {
-            const float wv = ld(row[u] + c);
+            for (int u = 0; u < R; ++u) {
+                const float wv = ld(row[u] + c);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) p[u][s] = fmaf(wv, x[s * pitch + c], p[u][s]);
+                for (int s = 0; s < NS; ++s) p[u][s] = fmaf(wv, x[s * pitch + c], p[u][s]);
+            }
+        }
+    }
+}
+// The same of one long row, eight elements in flight; with few samples the last of them, which may be fewer, too (a
+// loop over what is left takes a memory latency for each).
+template <typename T, int NS>
+__device__ __forceinline__ void row_product(const T *row, int len, const float *x, int pitch, int sl, float (&p)[NS]) {
+    constexpr int ROUND = 8, STEP = 16;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) p[s] = 0.f;
+    int c = sl;
+    if constexpr (NS < 4) {
+        // (zero on both sides past the end: neither may be an infinity's product)
+        auto round = [&](auto partial) __attribute__((always_inline)) {
+            constexpr bool PARTIAL = decltype(partial)::value;
+            T w[ROUND];
+#pragma unroll
+            for (int k = 0; k < ROUND; ++k) w[k] = row[PARTIAL ? min(c + k * STEP, len - 1) : c + k * STEP];
+#pragma unroll
+            for (int k = 0; k < ROUND; ++k) {
+                const bool in = !PARTIAL || c + k * STEP < len;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const float xv = x[s * pitch + (PARTIAL ? min(c + k * STEP, len - 1) : c + k * STEP)];
+                    p[s] = fmaf(in ? ld(&w[k]) : 0.f, in ? xv : 0.f, p[s]);
+                }
+            }
+        };
+        for (; c - sl + ROUND * STEP <= len; c += ROUND * STEP) round(std::false_type{});
+        if (c - sl < len) round(std::true_type{});
+    } else {
+#pragma unroll ROUND
+        for (; c < len; c += STEP) {
+            const float wv = ld(row + c);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) p[s] = fmaf(wv, x[s * pitch + c], p[s]);
         }
     }
 }
@@ -859,8 +896,8 @@ __device__ __forceinline__ void row_products(const T *const (&row)[R], int len, 
 // per sample they cost more L2 bandwidth than anything else here).  Every
 // workgroup of a sample recomputes the hidden vector, so the blocks are large:
 // smaller ones had all compute units read the same rows of w1 at once, which
-// the L2 serves one after the other.
-template <typename T, int KK, int BLOCK, int NS>
+// the L2 serves one after the other.  WIDE: rows of w2 as vectors (see the launcher).
+template <typename T, int KK, int BLOCK, int NS, bool WIDE>
 __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     const T *__restrict__ pooled, const T *__restrict__ w1, const T *__restrict__ b1,
     const T *__restrict__ w2, const T *__restrict__ b2, T *__restrict__ cf, int N, int C, int mid,
@@ -916,13 +953,12 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
     // hidden vectors: rows of w1
     for (int m0 = wave * 4; m0 < mid; m0 += kChannelWaves * 4) {
         const int m = min(m0 + seg, mid - 1);
-        const T *const row[1] = {w1 + (int64_t)m * C};
-        float p[1][NS];
-        row_products<T, 1, NS>(row, C, v, C, sl, p);
+        float p[NS];
+        row_product<T, NS>(w1 + (int64_t)m * C, C, v, C, sl, p);
         const float bias = b1 ? ld(b1 + m) : 0.f;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const float tot = row_sum(p[0][s]);
+            const float tot = row_sum(p[s]);
             if (sl == 0 && m0 + seg < mid) {
                 const float hm = relu(tot + bias);
                 h[s * mid + m0 + seg] = hm;
@@ -944,7 +980,7 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
         const T *wrow[RT];
 #pragma unroll
         for (int u = 0; u < RT; ++u) wrow[u] = w2 + ((int64_t)cb * KK + min(r0 + 4 * u + seg, rows - 1)) * mid;
-        row_products<T, RT, NS>(wrow, mid, h, mid, sl, p);
+        row_products<T, RT, NS, WIDE>(wrow, mid, h, mid, sl, p);
 #pragma unroll
         for (int u = 0; u < RT; ++u) {
             const int r = r0 + 4 * u + seg;
@@ -1315,7 +1351,7 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
         }
     }
     // (wide layers: fewer, larger blocks, as every block of a sample recomputes the hidden vector, unless smaller ones
-    // still have a compute unit each: fp32 32 x 512 13.9 us in blocks of 128, 11.2 of 64; 40 x 512 14 and 14.8)
+    // still have a compute unit each: fp32 32 x 512 12.8 us in blocks of 128, 10.2 of 64; 44 x 512 13.2 and 13.9)
     const int block = C >= 512 && cdiv(C, 64) * N > 256 ? 128 : 64;
     // samples per workgroup: as many as keep every compute unit busy and fit the LDS
     auto lds_of = [&](int ns) { return ((size_t)C + (size_t)mid + (size_t)block * kk) * ns * sizeof(float); };
@@ -1326,15 +1362,36 @@ hipError_t channel_branch(const T *pooled, const T *w1, const T *b1, const T *w2
     const size_t lds = lds_of(ns);
     if (N > 65535 * ns || mid < 1 || lds > 48 * 1024) return hipErrorNotSupported;
     const dim3 grid((unsigned)cdiv(C, block), (unsigned)cdiv(N, ns));
-#define DDF_CHANNEL_LAUNCH(KK_, BLOCK_, NS_)                                                     \
-    hipLaunchKernelGGL((k_channel_branch<T, KK_, BLOCK_, NS_>), grid, dim3(kChannelThreads), lds, \
+    // Rows of w2 as vectors: where they take fewer round trips to memory than single elements, two of either in flight and
+    // what is less than a vector behind them, or as many where a row is longer than 32 (not of two samples in fp16).  us, single elements /
+    // vectors: fp32 32 x 512 13.4 / 10.2, 64 x 512 20.6 / 14.3, 128 x 512 21.6 / 16.5, 250 x 200 11.5 / 10.4, 100 x 156 with 20 hidden values
+    // 8.9 / 7.7, with 16 7.0 / 7.7, with 39 10.6 / 9.2, 5 x 5 taps 64 x 256 16.6 / 13.1, fp16 56 x 456 18.0 / 14.3, 40 x 1000 35.4 / 29.2, 100 x 156
+    // with 24 9.3 / 8.6, with 32 8.0 / 8.6, two samples 307 x 164 with 41 12.3 / 13.3, with 56 13.1 / 12.0.
+    // More samples, or longer rows of fp16: the vectors of x take their time in LDS (fp16 500 x 200 17.9 / 29.9, 128 x 456 20.8 / 25.8, two
+    // samples 128 x 584 with 292 hidden values 50 / 59, fp32 391 x 346 42.6 / 47.6), which is had back where rows come from far: a block's are a
+    // megabyte, or less where the blocks do not divide the XCDs, each of which otherwise keeps its block's rows in its L2 (fp32 300 x 1024
+    // 125 / 150, but 132 x 998 with 499 hidden values 343 / 287, 253 x 896 80.3 / 73.1, 300 x 1028 201 / 167, fp16 5 x 5 taps 128 x 548 with 274
+    // 256 / 170).  (Rows of w1 as vectors as well: fp32 300 x 1024 182, fp16 40 x 1000 38.5.)
+    auto trips = [](int64_t n) { return n / 32 + (n % 32 == 0 ? 0 : n % 32 <= 16 ? 1 : 2); };
+    constexpr int V = 16 / (int)sizeof(T);
+    constexpr bool kHalf = sizeof(T) == 2;
+    const int64_t singles = trips(mid), wide = trips(mid / V) + (mid % V ? 1 : 0), blocks = cdiv(C, block);
+    const int64_t row_bytes = block * kk * mid * (int64_t)sizeof(T);
+    const bool far = block == 128 && (row_bytes >= 1 << 20 || (8 % blocks != 0 && (row_bytes >= 3 << 18 || blocks > 6)));
+    const bool fewer = wide < singles || (wide == singles && mid > 32 && !(kHalf && ns == 2));
+    const bool vectors = ns == 1 ? wide < singles || mid > 32 : ns == 2 ? fewer && (!kHalf || mid <= 128 || far) : !kHalf && far;
+#define DDF_CHANNEL_LAUNCH(KK_, BLOCK_, NS_, WIDE_)                                              \
+    hipLaunchKernelGGL((k_channel_branch<T, KK_, BLOCK_, NS_, WIDE_>), grid, dim3(kChannelThreads), lds, \
                        st, pooled, w1, b1, w2, b2, cf, (int)N, (int)C, (int)mid, (float)gain,    \
                        gain_vec, offset_vec, parts, nparts, (float)scale, save)
 #define DDF_CHANNEL_CASE(KK_, BLOCK_)                                                            \
     do {                                                                                         \
-        if (ns == 4) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 4);                                         \
-        else if (ns == 2) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 2);                                    \
-        else DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 1);                                                 \
+        if (ns == 4 && vectors) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 4, sizeof(T) == 4);              \
+        else if (ns == 4) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 4, false);                             \
+        else if (ns == 2 && vectors) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 2, true);                   \
+        else if (ns == 2) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 2, false);                             \
+        else if (vectors) DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 1, true);                              \
+        else DDF_CHANNEL_LAUNCH(KK_, BLOCK_, 1, false);                                          \
     } while (0)
     if (k == 3 && block == 64) DDF_CHANNEL_CASE(9, 64);
     else if (k == 3) DDF_CHANNEL_CASE(9, 128);

@@ -304,6 +304,32 @@ def test_channel_branch_parts_matches_fp64(n, c, k, tiles, dtype, tol):
     assert err < tol, err
 
 
+@pytest.mark.parametrize('dtype,tol', [(torch.float32, 2e-5), (torch.float16, 6e-3)])
+@pytest.mark.parametrize('n,c,mid,k', [
+    (100, 200, 39, 3), (100, 200, 40, 3), (101, 201, 47, 3),     # one sample a workgroup: rows of w2 as elements, as vectors
+    (250, 200, 39, 3), (251, 200, 41, 3), (137, 300, 130, 3),    # two samples
+    (500, 200, 40, 3), (503, 200, 41, 3),                        # four
+    (5, 70, 39, 5), (5, 70, 40, 5), (3, 90, 167, 5),
+])
+def test_channel_branch_rows_of_the_second_product(n, c, mid, k, dtype, tol):
+    """Hidden layers around the length from which rows come in as vectors: what is left of a row, rows at odd addresses;
+    an infinite weight at the end of a row reaches its own channel's taps only."""
+    torch.manual_seed(n + mid)
+    pooled = torch.randn(n, c, device='cuda').to(dtype)
+    w1 = (torch.randn(mid, c, device='cuda') * c ** -0.5).to(dtype)
+    b1 = torch.rand(mid, device='cuda').to(dtype) + 1     # (the last hidden value is not zero for every sample)
+    w2 = (torch.randn(c * k * k, mid, device='cuda') * mid ** -0.5).to(dtype)
+    b2 = torch.randn(c * k * k, device='cuda').to(dtype)
+    out = _lib.channel_branch(pooled, w1, b1, w2, b2, k, 0.7)
+    ref = channel_reference(*(t.cpu() for t in (pooled, w1, b1, w2, b2)), k, 0.7, None, None)
+    err = ((out.double().cpu() - ref).abs().max() / ref.abs().max()).item()
+    assert err < tol, err
+    w2[(c // 2) * k * k, mid - 1] = float('inf')
+    got = _lib.channel_branch(pooled, w1, b1, w2, b2, k, 0.7)
+    same = (got == out).flatten(2).all(-1)
+    assert same[:, :c // 2].all() and same[:, c // 2 + 1:].all() and not same[:, c // 2].all()
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
 @pytest.mark.parametrize('n,c,mid,tiles', [(1, 256, 51, 1), (2, 256, 51, 9), (3, 160, 32, 13), (17, 320, 64, 11),
                                            (5, 64, 12, 3), (300, 96, 19, 2)])
