@@ -1120,10 +1120,18 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
             tune_int("DDF_TUNE_SPATIAL_MMA", 1) != 0) {
             constexpr int kPixels = 4 * kWave;     // of a workgroup, four per lane
             const int64_t tiles8 = cdiv(vectors(8), kWave), tiles4 = cdiv(vectors(4), kWave), left = channel_parts_left(N, C, C / 5, esz);
-            const int64_t full = head * (C <= 64 ? N * tiles4 : N * npix / kPixels);
+            // Vectors that do not divide the plane: of eight where seven tenths of the lanes have one, of four where half
+            // have (three tenths from four channel groups on), all of them counted in pixels.  Small odd planes leave a
+            // workgroup with a few vectors whatever their number: us, both branches, k_spatial_stream / vectors of four / of eight,
+            // 1563 x 32 x 7 x 7 18.3 / 21.5 / 26.3, 700 x 256 x 7 x 7 22.9 / 27.7 / -, 819 x 32 x 11 x 11 13.6 / 14.3 / 16.8, 537 x 48 x 14 x 14
+            // - / 15.1 / 17.2, 148 x 80 x 26 x 26 18.7 / 15.8 / 17.7, but 635 x 160 x 9 x 9 27 / 21.6, 114 x 80 x 29 x 29 16.1 / - / 13.4.  (900 sizes:
+            // 1.9 % over the best of the three, 4.8 % without, a third of the worst 1.4 times as long as k_spatial_stream.)
+            auto lanes = [&](int vp, int64_t tiles, int tenths) { return divides(vp) || vectors(vp) * 10 >= tiles * kWave * tenths; };
+            const int64_t full = head * (C <= 64 && divides(4) ? N * tiles4 : N * npix / kPixels);
             const bool odd = (C / kSpatialMmaGroup) % 2 != 0 && C < 64;
-            const bool wide = fits(8) && full >= (odd ? 2048 : C <= 64 ? 768 : 256);
-            const bool narrow = fits(4) && full >= (C <= 80 ? 64 : C <= 256 ? 128 : 256) && !(odd && full >= 512);
+            const bool wide = fits(8) && lanes(8, tiles8, 7) && full >= (odd ? 2048 : C <= 64 ? 768 : 256);
+            const bool narrow = fits(4) && lanes(4, tiles4, C < 64 ? 5 : 3) && full >= (C <= 80 ? 64 : C <= 256 ? 128 : 256) &&
+                                !(odd && full >= 512);
             if (wide || narrow) {
                 mma = true;
                 vp = wide || (pool && fits(8) && tiles4 > left && tiles8 <= left) ? 8 : 4;

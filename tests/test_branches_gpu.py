@@ -231,7 +231,7 @@ RAGGED_CASES = [
     (54, 100, 41, 25, 1, 2, 'h', 4), (46, 200, 41, 15, 1, 2, 'h', 4), (65, 12, 75, 63, 1, 2, 'h', 8), (65, 100, 75, 22, 1, 2, 'h', 8),
     (80, 12, 38, 94, 2, 2, 'h', 2), (64, 200, 106, 6, 2, 2, 'h', 2), (59, 12, 118, 82, 2, 2, 'h', 4),
     (32, 64, 7, 6, 1, 2, 'h', 4), (40, 48, 51, 53, 1, 1, 'h', 4), (12, 64, 151, 149, 1, 2, 'h', 8), (40, 256, 45, 47, 1, 1, 'h', 8),
-    (65000, 16, 1, 9, 1, 1, 'h', 8),
+    (65000, 16, 1, 9, 1, 1, 'h', 8), (300, 64, 11, 11, 1, 1, 'h', 4), (500, 160, 9, 9, 1, 1, 'h', 4),     # a third of the lanes
 ]
 
 
