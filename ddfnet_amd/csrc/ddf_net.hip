@@ -1089,15 +1089,15 @@ bool conv_in_tiles(const NetConv &a) {
 // 42.2 / 43.4, 392 of 14 x 14 x 1024 -> 256 24.1 / 28.5).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
 // 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
 enum ConvTile { kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64, kTileSplit };
-// The same holds for pairs (batch 128, short / long: 7 x 7 x 512 + 1024 -> 2048, 784 tiles, 67.5 / 54, 32 x 28 x 28 x 128 + 256
-// -> 512, 784, 25.2 / 24; 64 images of it, 1568 tiles, 40.1 / 41.7, 128 76.4 / 79.9), but where three
-// workgroups per unit are one round and two a full one or more (a network of 96 images, 588 tiles, 1351 / 1357, of
-// 64 of 256 x 256, 512, 1085 / 1088).
+// The same holds for pairs, but from 513 to 768 tiles three workgroups per unit are one round and two a full one and a
+// part.  us, short / long stages: 28 x 28 x 128 + 256 -> 512 344 tiles 14.9 / 13.8, 516 20.1 / 21.9, 588 21.6 / 23.7, 760 24.2 / 25.8, 784 28.1 / 26.8,
+// 980 31.4 / 29.7; 14 x 14 x 256 + 512 -> 1024 592 30.9 / 34.5, 784 41.6 / 38.8; 7 x 7 x 512 + 1024 -> 2048 592 50.8 / 52.1, 784
+// 70.3 / 62.4; 512 tiles of 8 x 8 x 512 + 1024 -> 2048 42.7 / 35.1, of 16 x 16 x 256 + 512 -> 1024 25.4 / 22.6.
 ConvTile conv_tile(const NetConv &a, bool pair) {
     auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
     constexpr int kMany = 1024, kFew = 320;
     if (!conv_in_tiles(a)) return kTileSplit;
-    if (a.N >= 128 && (count(128, 128) >= kMany || (pair && count(128, 128) >= 512 && count(128, 128) <= 768))) return kTile128;
+    if (a.N >= 128 && (count(128, 128) >= kMany || (pair && count(128, 128) > 512 && count(128, 128) <= 768))) return kTile128;
     if (a.N >= 128 && count(128, 128) >= kFew) return kTile128Long;
     if (count(128, 64) >= kMany) return kTile128x64;
     if (count(128, 64) >= 448) return kTile128x64Long;

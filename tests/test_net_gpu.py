@@ -86,7 +86,11 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     (8, 28, 28, 256, 512, 1024, 2, 1),         # tiles of 64
     (16, 28, 28, 128, 256, 264, 1, 1),         # 128 x 64
     (42, 56, 56, 64, 64, 136, 1, 1),           # 128 x 128, many
-    (27, 56, 56, 128, 256, 512, 2, 1),         # 128 x 128, few
+    (27, 56, 56, 128, 256, 512, 2, 1),         # 128 x 128, 664 tiles: short stages
+    (7, 45, 44, 64, 64, 264, 1, 1),            # long ones, 327 tiles, rows and channels past the last: a stage of K each
+    (64, 16, 16, 64, 192, 2048, 2, 0),         # 512, one stage and three
+    (26, 56, 55, 192, 128, 520, 2, 1),         # 800, three and two
+    (21, 31, 33, 320, 256, 640, 1, 1),         # 840, five and four
     (42, 56, 56, 128, 64, 64, 1, 1),           # 64 channels, many
 ])
 def test_conv_pair(n, h, w, c, side, o, stride, relu):
