@@ -281,6 +281,7 @@ __device__ __forceinline__ void words_from(int again, uint32_t (&mask)[NW]) {
     for (int k = 0; k < NW; ++k) {
         if constexpr (sizeof(T) == 4) mask[k] = k >= again ? ~0u : 0u;
         else mask[k] = (2 * k >= again ? 0xffffu : 0u) | (2 * k + 1 >= again ? 0xffff0000u : 0u);
+        asm volatile("" : "+v"(mask[k]));    // (not as comparisons: pairs of scalar registers, of which there are none left)
     }
 }
 
