@@ -1091,7 +1091,11 @@ hipError_t spatial_stream(const T *x, const T *w, const T *bias, T *sf, int64_t 
         // 27.2, 26 x 48 x 65 x 145 41.9 / 39.4, stride 2 8 x 256 x 98 x 98 45.2 / 40.2, fp16 8 x 64 x 199 x 301 71.8 / 60.4,
         // 16 x 176 x 57 x 55 39.3 / 30.6; left alone 64 x 256 x 15 x 15 26.7 / 27.3, 32 x 256 x 7 x 7 17.1 / 18.1, two heads of
         // 48 x 432 x 15 x 19 48.0 / 49.8 and 1 x 324 x 165 x 238 52.4 / 56.0, stride 2 32 x 256 x 26 x 30 23.2 / 26.5.
-        if (!divides(cand) && ((cand > 2 && divides(cand / 2)) || nvec * 5 < cdiv(nvec, kWave) * kWave * 4 ||
+        // Under stride 2 the workgroups of head 0 add up the planes and take longest: not where several heads' of eight waves
+        // are a round and a part (branch alone, fp32, four heads: 5 x 412 x 74 x 82 23.7 / 40.2, 43 x 360 x 34 x 26 30.3 / 43.9, 4 x 312 x 92 x 98
+        // 25.6 / 33.8; a round of fp16 2 x 428 x 136 x 118 26.8 / 17.7, more 6 x 260 x 78 x 102 31.2 / 19.6; rows of a few pixels not measured).
+        const bool part_round = stride == 2 && head > 1 && Wo >= 8 && wv == 8 && tiles * wv > want && tiles * wv < 2800;
+        if (!divides(cand) && (part_round || (cand > 2 && divides(cand / 2)) || nvec * 5 < cdiv(nvec, kWave) * kWave * 4 ||
                                tiles * wv < (wv == 16 ? want + want / 4 : wv == 1 ? 1280 : want)))
             continue;
         vp = cand;
