@@ -556,11 +556,11 @@ __device__ __forceinline__ double lane_broadcast<double>(double v, int src_lane)
     return __hiloint2double(hi, lo);
 }
 
-// BWD = false: out = forward(x, cf, sf).  BWD = true: x is dO and out is dX.
 // Whether a lane's feature rows are taken one after another (see compute()).
 template <typename T, int K, int VX, int R>
 constexpr bool by_row() { return K == 5 && R == 1 && VX * sizeof(T) == 16; }
 
+// BWD = false: out = forward(x, cf, sf).  BWD = true: x is dO and out is dX.
 // WPE: waves per SIMD the register allocation must leave room for.
 // S = 2 (forward, 3 x 3, one row per lane): g describes the result plane, the
 // lane's feature vectors are 2 * VX elements wide (LaneStride2).
@@ -866,8 +866,8 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
         // 66 / 62; fp16 32 x 128 x 56 x 56 29.9 / 27.7, ragged rows, two waves all the same (15 registers spill at three),
         // 8 x 64 x 200 x 300 60.8 / 55.2, 8 x 96 x 92 x 130 22.7 / 22.9.  (The channel's taps moved to vector registers as
         // well, whose multiply-adds issue faster: 34.0 where this takes 31.1.)  Shorter vectors have the room anyway and
-        // are 1 % faster without it.
-        constexpr bool kByRow = by_row<T, K, VX, R>();
+        // are 1 % faster without it, and fp16 is where two waves per SIMD are all there are (launch_kdv).
+        constexpr bool kByRow = by_row<T, K, VX, R>() && (sizeof(T) == 4 || TAIL > 0 || WPE > 2);
         if constexpr (!kByRow) {
 #pragma unroll
             for (int rr = 0; rr < ROWS; ++rr)

@@ -435,6 +435,20 @@ def test_tensors_that_start_at_odd_addresses(shape, stride, dtype):
             assert rel_err(got.detach(), w) <= TOL[dtype]
 
 
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('d', [1, 2])
+@pytest.mark.parametrize('few,many,shape', [(9, 10, (128, 56, 56)), (10, 30, (16, 112, 80)), (300, 600, (32, 12, 8)), (1, 700, (24, 9, 16))],
+                         ids=_ids)
+def test_fp16_five_by_five_of_few_and_many_waves(few, many, shape, d, combine):
+    """Up to two waves per SIMD take another kernel than more of them: a sample's results are the same bits in either."""
+    x, cf, sf, go = random_case(many, *shape, 5, 1, torch.float16, seed=few)
+    dev = to_dev(x, cf, sf, go)
+    wide = run_ddf(*dev, 5, d, 1, combine, need=(True, False, False))
+    slim = run_ddf(*(t[:few].contiguous() for t in dev), 5, d, 1, combine, need=(True, False, False))
+    assert all(torch.equal(a, b[:few]) for a, b in zip(slim[:2], wide[:2]))
+    check_against_oracle(x[:1], cf[:1], sf[:1], go[:1], 5, d, 1, combine)
+
+
 def test_runs_on_the_current_stream():
     from ddfnet_amd import ddf
     x, cf, sf, _ = random_case(4, 16, 14, 14, 3, 1, torch.float32, seed=12)
