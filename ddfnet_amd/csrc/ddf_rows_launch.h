@@ -28,7 +28,8 @@ hipError_t launch_kdv(const Problem &p, const RowsGeom &g, bool backward, const 
     // fp16, 25 taps: rows one after another make room for a third wave per SIMD; where there are no more waves than two
     // each, all rows at once are faster (k_rows' kByRow).  us, one after another / at once, forward and dX, taps two apart: 1 x 32 x
     // 12 x 8 6.6 / 5.7; one apart: 1 x 296 x 52 x 48 7.0 / 6.7, 'add' 5 x 32 x 25 x 24 6.8 / 6.4; 240 sizes: up to 512 waves 4 % (two apart 14,
-    // 'add' 5 and 0.5), up to 2048 1 %, beyond one after another is 1 to 4 % faster (32 x 128 x 56 x 56 27.7 / 29.9).
+    // 'add' 5 and 0.5), up to 2048 1 %, beyond one after another is 1 to 4 % faster (32 x 128 x 56 x 56 27.7 / 29.9).  The forward
+    // pass of 'add' one apart over unpadded rows is faster one after another at any size (1 x 8 x 56 x 40 6.3 / 6.7).
     constexpr int kWpe = waves_per_simd<T, K, VX, R>(), kFewWpe = K == 5 && sizeof(T) == 2 ? 2 : kWpe;
     constexpr int kSimds = 1024;
     const bool few = kFewWpe != kWpe && g.nwork <= kFewWpe * kSimds;
@@ -39,7 +40,7 @@ hipError_t launch_kdv(const Problem &p, const RowsGeom &g, bool backward, const 
     do {                                                                                        \
         if (pad && few) DDF_ROWS_LAUNCH(MUL_, BWD_, true, kFewWpe);                             \
         else if (pad) DDF_ROWS_LAUNCH(MUL_, BWD_, true, kWpe);                                  \
-        else if (few) DDF_ROWS_LAUNCH(MUL_, BWD_, false, kFewWpe);                              \
+        else if (few) DDF_ROWS_LAUNCH(MUL_, BWD_, false, (MUL_ || BWD_ || D != 1 ? kFewWpe : kWpe)); \
         else DDF_ROWS_LAUNCH(MUL_, BWD_, false, kWpe);                                          \
     } while (0)
     if (p.mul) {
