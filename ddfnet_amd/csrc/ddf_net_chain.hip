@@ -15,7 +15,7 @@ using rows::plane_rsrc;
 // out (M, N) = relu(norm(x . w) + res), or relu(norm(x . w) + norm'(side . side_w));
 // next (M, N2) = relu(norm''(out . w2)), and next's sums over its pixels.
 //
-// The wide result is written once and not read back: a workgroup takes 32 * P pixels of all channels,
+// The wide result is written once and not read back: a workgroup takes kChainRows pixels of all channels,
 // goes over the wide channels by kChunk, and each chunk is the next block of the summed dimension of
 // the second product, whose sums stay in registers.  A wave has 32 pixels: their x in registers as the
 // operand of every chunk, a tile of LDS for the chunk's results, which are rounded, meet the residual
@@ -221,7 +221,8 @@ struct Norms {
         }
     }
 };
-// (passes of the wide channels: what a launch takes)
+// (passes of the wide channels: what a launch takes; a network's have 512 at most, past 1024 there are only other callers'.
+// The second pass asks behind its descriptors then, which return zeros without a trip to memory)
 constexpr int kMaxWide = 2048, kWidePasses = kMaxWide / (4 * kThreads);
 
 enum { kNoFilter, kFilterMul, kFilterAdd };
@@ -552,8 +553,9 @@ bool net_chain_covers(int64_t M, int64_t K, int64_t side, int64_t N, int64_t N2)
     return (K == 64 && (N2 == 64 || N2 == 128)) || (K == 128 && (N2 == 128 || N2 == 256));
 }
 
-// (runs of four pixels; rows of 4096, far more than an image has, keep a tile's neighbours within 2 MB.  No
-// size was found where the two launches are faster.)
+// (runs of four pixels; rows of 4096 pixels keep a tile's neighbours within 2.2 MB, far from where 32-bit offsets end.
+// No size was found where the two launches are faster.  The instances without a filter serve ddf_hip_net_conv_chain; a
+// network, whose rows are whole runs, takes one only for images wider than 16384.)
 bool net_chain_filters(int64_t W, int64_t K) { return W % kRun == 0 && W <= 4096 && (K == 64 || K == 128); }
 
 int net_chain_pool_slots(int64_t M, int npix) {

@@ -241,6 +241,7 @@ def test_conv_pool(n, h, w, c, o):
     (60, 28, 28, 128, 0, 512, 256, 1), (1, 199, 199, 128, 0, 128, 256, 1),
     (1100, 8, 8, 64, 0, 256, 64, 0), (70000, 1, 1, 128, 0, 128, 128, 0),   # folded BatchNorm; samples of a tile, of a pixel
     (700, 6, 6, 64, 64, 128, 64, 0),
+    (8, 56, 56, 64, 0, 1088, 64, 1), (29, 21, 23, 64, 64, 2048, 64, 1), (27, 28, 28, 128, 0, 2048, 256, 0),    # wide ones past 1024
 ])
 def test_conv_chain(n, h, w, c, side, o, next_o, bn):
     """The two convolutions of one launch: what the two calls leave, and the sums over the pixels."""
@@ -282,6 +283,7 @@ def test_conv_chain(n, h, w, c, side, o, next_o, bn):
     (4, 56, 56, 64, 64, 64, 64, 0, 1),                                              # fewest tiles
     (1, 1, 24804, 64, 0, 64, 64, 0, 1), (2, 4100, 4, 64, 64, 64, 64, 0, 1),        # one row (no fused launch: None), rows of one run
     (3100, 2, 4, 128, 0, 64, 128, 0, 1), (1, 7, 4096, 64, 0, 64, 128, 1, 1),       # samples of a lane's pixels; the widest rows
+    (5, 53, 52, 64, 64, 1088, 64, 0, 1), (27, 28, 28, 128, 0, 2048, 256, 1, 0),    # wide channels past 1024
 ])
 def test_filter_chain(n, h, w, c, side, o, next_o, combine, bn):
     """The spatial branch and the filter in front of the chain's launch: what the three calls leave, to the bit."""
@@ -457,6 +459,27 @@ def test_network_of_large_images(n, h, w):
         hw = [v >> (2 + max(k - 1, 0)) for v in (h, w)]
         left.append(lib.ddf_hip_net_conv_pool_parts(n, *hw, c, width) <= lib.ddf_hip_net_parts_left(n, width, int(.2 * width)))
     assert True in left and False in left
+    torch.manual_seed(n)
+    model = ddf_resnet.ddf_mul_resnet50(num_classes=10, zero_init_last_bn=False).cuda().half().eval()
+    x = torch.randn(n, 3, h, w, device='cuda').half()
+    with torch.no_grad():
+        out = ddfnet_amd.functional.extension().net_forward(
+            model._native_plan(ddfnet_amd.functional.extension()), x)
+        modules = lambda net, y: net.fc(net.global_pool(net.forward_features(y)).flatten(1))
+        by_modules = modules(model, x).float()
+        want = modules(model.float(), x.float())
+    off = lambda y: ((y.float() - want).norm() / want.norm()).item()
+    assert off(out) <= max(4e-3, 1.3 * off(by_modules))
+
+
+def test_network_of_images_wider_than_the_filter_takes():
+    """Rows of more than 4096 pixels behind the stem: a block's last convolution and the next one's first are one launch,
+    its branches and filter others."""
+    n, h, w = 1, 32, 16416
+    lib = _lib.lib()
+    for side, next_o in ((64, 64), (0, 64), (0, 128)):
+        assert lib.ddf_hip_net_conv_chain_parts(n, h // 4, w // 4, 64, side, 256, next_o) > 0
+        assert lib.ddf_hip_net_filter_chain_parts(n, h // 4, w // 4, 64, side, 256, next_o) == 0
     torch.manual_seed(n)
     model = ddf_resnet.ddf_mul_resnet50(num_classes=10, zero_init_last_bn=False).cuda().half().eval()
     x = torch.randn(n, 3, h, w, device='cuda').half()
