@@ -63,6 +63,8 @@ def close(got, want, tol):
     (1, 5, 7, 576, 200, 1, 1, 1, 1, 1),        # K split over the waves: 9 blocks, rows and channels past a tile
     (17, 1, 1, 64, 33, 1, 0, 1, 0, 1),         # one block of K
     (1, 13, 9, 1088, 31, 2, 1, 0, 0, 0),       # 17 blocks, under stride 2
+    (1, 16, 16, 192, 4096, 1, 1, 0, 0, 1), (1, 1, 257, 320, 4096, 1, 1, 0, 1, 1),    # 256 tiles of 64, three stages; 320, five
+    (20, 4, 8, 1024, 256, 1, 1, 0, 1, 1), (10, 8, 8, 2048, 1000, 1, 0, 1, 0, 0),     # 40, 160: a workgroup per unit at most
 ])
 def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     torch.manual_seed(c + o)
@@ -215,7 +217,7 @@ def test_network_matches_its_modules(build, n, size, classes):
     (5, 7, 7, 64, 64), (3, 5, 7, 512, 512),     # samples that end inside tiles of 64 rows, of 16
     (1, 14, 14, 1024, 256), (2, 14, 14, 1024, 256),
     (9, 28, 28, 64, 128), (33, 28, 28, 256, 64), (16, 28, 28, 128, 264), (42, 56, 56, 64, 136),
-    (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64),
+    (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64), (20, 4, 8, 1024, 256),
 ])
 def test_conv_pool(n, h, w, c, o):
     """The results of conv, and their sums over the pixels, slot by slot of the tiles."""
