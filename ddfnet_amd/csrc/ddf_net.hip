@@ -62,6 +62,12 @@ using rows::plane_rsrc;
 // 56 x 56 x 64 -> 256 with a residual 91.9 -> 85.0, 28 x 28 x 128 -> 512 54.4 -> 48.3, 14 x 14 x
 // 256 -> 1024 38.4 -> 34.2; pairs 95 -> 81 (28 x 28 x 128 + 256 -> 512), 80 -> 67 (7 x 7).
 //
+// What a launch of few tiles takes besides its products is its way to the first load and from the last product to the stores:
+// arguments at once, tiles and pixels by multiplications, the first stages in front of the norm's parameters, scale and
+// shift by a thread per channel.  First loads out / end, us inside the launch: 14 x 14 x 256 -> 1024 with a residual 1.00 / 2.90
+// -> 0.44 / 2.32, 56 x 56 x 256 -> 64 1.06 / 3.44 -> 0.48 / 2.73; networks of 1, 8, 32 and 128 images of 224 x 224 310.4 -> 299.3, 415
+// -> 402, 670 -> 662, 1634 -> 1614 us, 48 of 256 x 256 889 -> 876.
+//
 // With PAIR the tile is act(affine(x w) + affine'(x' w')) of two products, a bottleneck's last
 // convolution and its projection: x' w' goes first, its affine result stays in registers as
 // the fp16 values that a projection of its own would have stored.
@@ -72,21 +78,30 @@ constexpr int conv_lds_halves() {
     return ring > tile ? ring : tile;
 }
 
+// The tiles of a product, row by row; of a pair's first product, the pixels it samples.
+struct TileCut {
+    int tiles;
+    Divisor tiles_n, npix, Wo;
+};
+
 // ALONE: a stage's loads in front of its products instead of between them (see launch_conv).
 template <int BM, int BN, int KST, int ST, int WG, bool PAIR, bool POOL, bool RES, bool ALONE = false>
-__global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, int tiles_n, int tiles) {
+__global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, TileCut cut) {
     constexpr int CH = KST / 8, STAGE = (BM + BN) * KST;
     constexpr int RX = BM * CH / kThreads, RW = BN * CH / kThreads;
     constexpr int TM = BM / 64, TN = BN / 64;      // 32-wide tiles per wave: pixels, channels
     constexpr int PITCH = BN + 8;
     static_assert((ST == 2 || ST == 3) && (CH == 4 || CH == 8) && RX > 0 && RW > 0 && !(RES && PAIR));
     extern __shared__ __align__(16) _Float16 net_smem[];
-    __shared__ float affine[PAIR ? 4 : 1][PAIR ? BN : 1];    // scale, shift; of the first product, too
+    __shared__ __align__(16) float affine[PAIR ? 4 : 2][BN];    // scale, shift; of the first product, too
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int block = xcd_block(blockIdx.x, tiles);
-    if (block >= tiles) return;
-    const int tm = block / tiles_n, tn = block - tm * tiles_n;
+    at_once(a.x, a.w, a.M, a.N, a.K, cut.tiles, cut.tiles_n.by, cut.tiles_n.magic);
+    at_once(a.norm.weight, a.norm.bias, a.norm.mean, a.norm.var, a.norm.conv_bias, a.out, a.res, a.relu);
+    if constexpr (PAIR) at_once(first.x, first.w, first.K, first.stride, first.H, first.W, first.norm.var, first.norm.weight);
+    const int block = xcd_block(blockIdx.x, cut.tiles);
+    if (block >= cut.tiles) return;
+    const int tm = (int)cut.tiles_n.of(block), tn = block - tm * (int)cut.tiles_n.by;
     const int64_t m0 = (int64_t)tm * BM;
     const int n0 = tn * BN;
     const int rows = (int)min((int64_t)BM, a.M - m0);    // pixels of the tile
@@ -96,13 +111,13 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     auto aim = [&](const NetConv &c) __attribute__((always_inline)) {
         const _Float16 *x = static_cast<const _Float16 *>(c.x), *w = static_cast<const _Float16 *>(c.w) + (int64_t)n0 * c.K;
         if (c.stride > 1) {
-            const int64_t sample = m0 / c.npix;
+            const int64_t sample = m0 >> 32 == 0 ? (uint32_t)m0 / (uint32_t)c.npix : m0 / c.npix;
             const int at = (int)(m0 - sample * c.npix);
 #pragma unroll
             for (int i = 0; i < RX; ++i) {
                 const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
-                const unsigned pix = (unsigned)(at + min(r, rows - 1)), n = pix / (unsigned)c.npix, p = pix - n * c.npix;
-                const unsigned y = p / (unsigned)c.Wo, xx = p - y * c.Wo;
+                const unsigned pix = (unsigned)(at + min(r, rows - 1)), n = cut.npix.of(pix), p = pix - n * c.npix;
+                const unsigned y = cut.Wo.of(p), xx = p - y * c.Wo;
                 xp[i] = x + (((sample + n) * c.H + y * c.stride) * c.W + xx * c.stride) * c.K + ch * 8;
             }
         } else {
@@ -146,20 +161,6 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     // nn.Linear has it.  Elsewhere, and in a pair, the sum is rounded first, as a convolution's
     // result is.  (A bias in a pair's accumulators had the 128 x 128 tiles spill: 86 -> 117 us.)
     const bool bias_in_sum = !PAIR && !a.norm.var && a.norm.conv_bias;
-    if (bias_in_sum) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int o = n0 + channel(j, g);    // (rows are whole vectors of 8)
-                half4_t b = {0, 0, 0, 0};
-                if (o < a.N) __builtin_memcpy(&b, static_cast<const _Float16 *>(a.norm.conv_bias) + o, sizeof(b));
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)b[e];
-            }
-    }
     // `meanwhile`: what goes out behind the products of a step, the stage's loads spread over its steps.  The
     // next step's operands are asked for in front of a step's products: left to itself the compiler keeps one set of
     // registers for operands, and every step waits out LDS.  Batch 128, us before / now: 14 x 14 x 1024 -> 256 24.2 / 22.5,
@@ -202,7 +203,6 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     constexpr int RO = BM * CPR / kThreads, STEP = kThreads / CPR;
     const int cq = tid % CPR, r0 = tid / CPR, c = n0 + cq * 8;
     const bool cok = c < a.N;
-    Affine<PAIR ? 1 : 8> aff;
     half8_t rv[RES ? RO : 1];
     auto residual = [&]() __attribute__((always_inline)) {
         if constexpr (RES) {
@@ -223,17 +223,8 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     };
 
     const int nk0 = PAIR ? first.K / KST : 0, nk = nk0 + a.K / KST;
-    Affine<1> of[2];
-    if constexpr (PAIR) {
-        if (tid < BN) {
-            of[0].request(a.norm, min(n0 + tid, a.N - 1));
-            of[1].request(first.norm, min(n0 + tid, a.N - 1));
-        }
-        aim(first);
-    } else {
-        aff.request(a.norm, cok ? c : 0, !bias_in_sum);
-        aim(a);
-    }
+    // (the first stages go out before anything else is asked for)
+    aim(PAIR ? first : a);
     auto load_stage = [&](int k, int buf) __attribute__((always_inline)) {
         if (PAIR && k == nk0) aim(a);
 #pragma unroll
@@ -242,15 +233,37 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
         if (s < nk) load_stage(s, s);
+    // (scale and shift by a thread per channel: worked out by every thread for its own eight, they were half of the way out
+    // of a small launch)
+    Affine<1> of[PAIR ? 2 : 1];
+    if (tid < BN) {
+        of[0].request(a.norm, min(n0 + tid, a.N - 1), PAIR || !bias_in_sum);
+        if constexpr (PAIR) of[1].request(first.norm, min(n0 + tid, a.N - 1));
+    }
+    auto put_affine = [&](int which, const NetNorm &n) __attribute__((always_inline)) {
+        float sc[1], sh[1];
+        of[which].finish(n, sc, sh);
+        affine[2 * which][tid] = sc[0];
+        affine[2 * which + 1][tid] = sh[0];
+    };
+    if (bias_in_sum) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int o = n0 + channel(j, g);    // (rows are whole vectors of 8)
+                half4_t b = {0, 0, 0, 0};
+                if (o < a.N) __builtin_memcpy(&b, static_cast<const _Float16 *>(a.norm.conv_bias) + o, sizeof(b));
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)b[e];
+            }
+    }
     if constexpr (PAIR) {
         if (tid < BN) {
-            float sc[1], sh[1];
-            of[0].finish(a.norm, sc, sh);
-            affine[0][tid] = sc[0];
-            affine[1][tid] = sh[0];
-            of[1].finish(first.norm, sc, sh);
-            affine[2][tid] = sc[0];
-            affine[3][tid] = sh[0];
+            put_affine(0, a.norm);
+            put_affine(1, first.norm);
         }
     }
     int buf = 0;
@@ -321,6 +334,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             multiply_stage(k, nothing);
             arrive<RES ? RO : 0>();
         }
+        if (tid < BN) put_affine(0, a.norm);
         multiply_stage(nk - 1, nothing);
     }
     __syncthreads();
@@ -360,7 +374,16 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         results[i] = *reinterpret_cast<const half8_t *>(net_smem + (r0 + i * STEP) * PITCH + cq * 8);
     if constexpr (!PAIR) {
         float sc[8], sh[8];
-        aff.finish(a.norm, sc, sh);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float4_t s4 = *reinterpret_cast<const float4_t *>(&affine[0][cq * 8 + h * 4]);
+            const float4_t o4 = *reinterpret_cast<const float4_t *>(&affine[1][cq * 8 + h * 4]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sc[4 * h + e] = s4[e];
+                sh[4 * h + e] = o4[e];
+            }
+        }
 #pragma unroll
         for (int i = 0; i < RO; ++i) {
 #pragma unroll
@@ -382,8 +405,8 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
         // tile; the tile with a sample's last pixel clears the slots that sample does not use.
         float *red = reinterpret_cast<float *>(net_smem + BM * PITCH);    // [waves][BN]
         const int first = (int)m0, end = (int)min(m0 + BM, a.M);
-        const int n_last = (end - 1) / a.npix;
-        for (int n = first / a.npix; n <= n_last; ++n) {
+        const int n_last = (int)cut.npix.of(end - 1);
+        for (int n = (int)cut.npix.of(first); n <= n_last; ++n) {
             const int lo = n * a.npix - first, hi = lo + a.npix;
             float sum[8];
 #pragma unroll
@@ -439,12 +462,14 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
 // 9.7, 7.2; 196 x 1024 -> 256 6.7, 9.9, 5.7; 1 x 2048 -> 1000 7.1, 7.1, 5.2; without a last round of
 // loads that nothing used 16 x 16 takes 5.7, 4.2 and 4.3).
 template <bool POOL>
-__global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, int tiles_n) {
+__global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, Divisor tiles_n) {
     constexpr int WAVES = kThreads / kWave, D = 4, T = 16;
     __shared__ float red[WAVES][T][T + 1];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+    at_once(a.x, a.w, a.M, a.N, a.K, a.stride, tiles_n.by, tiles_n.magic);
+    at_once(a.norm.weight, a.norm.bias, a.norm.mean, a.norm.var, a.norm.conv_bias, a.out, a.res, a.relu);
+    const int tm = (int)tiles_n.of(blockIdx.x), tn = blockIdx.x - tm * (int)tiles_n.by;
     const int col = lane & 15, quad = lane >> 4;
     const int n0 = tn * T;
     int64_t m = (int64_t)tm * T + col;
@@ -1061,6 +1086,9 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     const int64_t tiles = cdiv(a.M, BM) * tiles_n;
     if (tiles > (1 << 30)) return hipErrorInvalidConfiguration;
     const int lds = conv_lds_halves<BM, BN, KST, ST>() * (int)sizeof(_Float16);
+    // (a strided product's pixels are counted from a sample's first: below npix + BM; a pooled one's from the first)
+    const NetConv &x = first ? *first : a;
+    const TileCut cut{(int)tiles, Divisor::make(tiles_n, tiles), Divisor::make(x.npix, a.pool ? a.M : x.npix + (int64_t)BM), Divisor::make(x.Wo, x.npix)};
     constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) <= 64 * 1024;
     if (first && !kPair) return hipErrorNotSupported;
     // A workgroup that has its unit to itself waits for its next stages: their loads go out in front of the products.  us, between / in
@@ -1073,14 +1101,14 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     do {                                                                                            \
         if (alone)                                                                                  \
             hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, POOL_, RES_, kSmall>), dim3(xcd_grid(tiles)), \
-                               dim3(kThreads), lds, st, a, a, tiles_n, (int)tiles);                 \
+                               dim3(kThreads), lds, st, a, a, cut);                 \
         else                                                                                        \
             hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, POOL_, RES_>), dim3(xcd_grid(tiles)), \
-                               dim3(kThreads), lds, st, a, a, tiles_n, (int)tiles);                 \
+                               dim3(kThreads), lds, st, a, a, cut);                 \
     } while (0)
     if (first)
         hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
-                           *first, tiles_n, (int)tiles);
+                           *first, cut);
     else if (a.pool) DDF_NET_CONV(true, false);
     else if (a.res) DDF_NET_CONV(false, true);
     else DDF_NET_CONV(false, false);
@@ -1149,9 +1177,9 @@ hipError_t net_conv(const NetConv &a, hipStream_t st) {
     const int64_t blocks = cdiv(a.M, 16) * tiles_n;
     if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
     if (a.pool)
-        hipLaunchKernelGGL((k_net_conv_split<true>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
+        hipLaunchKernelGGL((k_net_conv_split<true>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, Divisor::make(tiles_n, blocks));
     else
-        hipLaunchKernelGGL((k_net_conv_split<false>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, tiles_n);
+        hipLaunchKernelGGL((k_net_conv_split<false>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, Divisor::make(tiles_n, blocks));
     return hipGetLastError();
 }
 

@@ -22,34 +22,61 @@ __device__ __forceinline__ int xcd_block(int block, int blocks) {
 }
 inline unsigned xcd_grid(int64_t blocks) { return (unsigned)(cdiv(blocks, kXcd) * kXcd); }
 
+// A kernel's arguments, all in front of its first instruction: they are read from memory, and read where each is needed a
+// launch of a few microseconds waits for them two or three times (0.2 us each).
+template <typename A, typename B, typename C, typename D>
+__device__ __forceinline__ void at_once(A a, B b, C c, D d) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+}
+template <typename A, typename B, typename C, typename D, typename... More>
+__device__ __forceinline__ void at_once(A a, B b, C c, D d, More... more) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+    at_once(more...);
+}
+
+// Division by a number that the host knows: by a multiplication where that is exact (0: it is not).
+struct Divisor {
+    uint32_t by, magic;
+    // of numbers below `most`
+    static Divisor make(int64_t by, int64_t most) {
+        return {(uint32_t)by, by > 1 && by * most < (1ll << 32) ? (uint32_t)(((1ull << 32) + by - 1) / by) : 0u};
+    }
+    __device__ __forceinline__ uint32_t of(uint32_t n) const { return by == 1 ? n : magic ? __umulhi(n, magic) : n / by; }
+};
+
 // y = scale * x + shift of the convolution's bias and the BatchNorm behind it, for V
 // consecutive channels: requested as vectors early, worked out where they are needed.  (Read
-// channel by channel at the end of a kernel they cost more than small kernels do.)
+// channel by channel at the end of a kernel they cost more than small kernels do.)  A parameter that is not there is asked
+// for behind a descriptor that holds nothing: no branches, which the loads behind them wait for.
 template <int V>
 struct Affine {
     typedef _Float16 vec __attribute__((ext_vector_type(V)));
     vec w, b, m, v, cb;
     // bias: the convolution's is part of it.
     __device__ __forceinline__ void request(const NetNorm &n, int c, bool bias = true) {
-        auto get = [&](const void *p, _Float16 other) {
-            vec r;
-            if (p) __builtin_memcpy(&r, static_cast<const _Float16 *>(p) + c, sizeof(vec));
-            else
-#pragma unroll
-                for (int e = 0; e < V; ++e) r[e] = other;
-            return r;
+        auto get = [&](const void *p) __attribute__((always_inline)) {
+            const __amdgpu_buffer_rsrc_t r = rows::plane_rsrc(p, p ? 0x7fffffffu : 0u);
+            if constexpr (V == 1) {
+                return __builtin_bit_cast(vec, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, c * 2, 0, 0));
+            } else {
+                uint32_t q[V / 2];
+                rows::load_words<V / 2>(r, (uint32_t)c * 2, q);
+                return __builtin_bit_cast(vec, q);
+            }
         };
-        w = get(n.var ? n.weight : nullptr, (_Float16)1);
-        b = get(n.var ? n.bias : nullptr, (_Float16)0);
-        m = get(n.var ? n.mean : nullptr, (_Float16)0);
-        v = get(n.var, (_Float16)1);
-        cb = get(bias ? n.conv_bias : nullptr, (_Float16)0);
+        const bool bn = n.var;
+        w = get(bn ? n.weight : nullptr);
+        b = get(bn ? n.bias : nullptr);
+        m = get(bn ? n.mean : nullptr);
+        v = get(n.var);
+        cb = get(bias ? n.conv_bias : nullptr);
     }
     __device__ __forceinline__ void finish(const NetNorm &n, float (&scale)[V], float (&shift)[V]) const {
-        const float eps = n.var ? n.eps : 0.f;
+        const bool bn = n.var;
+        const float eps = bn ? n.eps : 1.f;
 #pragma unroll
         for (int e = 0; e < V; ++e) {
-            scale[e] = (float)w[e] * rsqrtf((float)v[e] + eps);
+            scale[e] = (bn && n.weight ? (float)w[e] : 1.f) * rsqrtf((float)v[e] + eps);
             shift[e] = (float)b[e] + ((float)cb[e] - (float)m[e]) * scale[e];
         }
     }

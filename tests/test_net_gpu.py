@@ -94,6 +94,7 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     (26, 56, 55, 192, 128, 520, 2, 1),         # 800, three and two
     (21, 31, 33, 320, 256, 640, 1, 1),         # 840, five and four
     (42, 56, 56, 128, 64, 64, 1, 1),           # 64 channels, many
+    (1, 520, 516, 64, 64, 64, 2, 1),           # 67080 pixels: too many for a division by multiplying
 ])
 def test_conv_pair(n, h, w, c, side, o, stride, relu):
     torch.manual_seed(c + o)
@@ -218,6 +219,7 @@ def test_network_matches_its_modules(build, n, size, classes):
     (1, 14, 14, 1024, 256), (2, 14, 14, 1024, 256),
     (9, 28, 28, 64, 128), (33, 28, 28, 256, 64), (16, 28, 28, 128, 264), (42, 56, 56, 64, 136),
     (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64), (20, 4, 8, 1024, 256),
+    (1, 260, 258, 64, 64),                      # 67080 pixels: too many for a division by multiplying
 ])
 def test_conv_pool(n, h, w, c, o):
     """The results of conv, and their sums over the pixels, slot by slot of the tiles."""
