@@ -1009,14 +1009,14 @@ __global__ __launch_bounds__(kChannelThreads) void k_channel_branch(
 template <typename T, bool SAVE>
 __global__ __launch_bounds__(kRowsThreads) void k_channel_branch_rows(ChannelRows<T> a) {
     extern __shared__ __align__(16) unsigned char rows_smem[];
-    channel_rows<T, SAVE>(a, blockIdx.x, blockIdx.y, rows_smem, Nothing(), Nothing(), ToFilter<T, kRowsKK>{a.cf, a.C});
+    channel_rows<T, SAVE>(a, blockIdx.x, blockIdx.y, rows_smem, Nothing(), Nothing(), Nothing(), ToFilter<T, kRowsKK>{a.cf, a.C});
 }
 
 template <int KK, bool SAVE>
 __global__ __launch_bounds__(kMmaThreads) void k_channel_branch_mma(ChannelMma a) {
     extern __shared__ __align__(16) unsigned char mma_smem[];
     const int n0 = blockIdx.y * kMmaSamples;
-    channel_mma<KK, SAVE>(a, blockIdx.x, n0, min(kMmaSamples, a.N - n0), mma_smem, Nothing(),
+    channel_mma<KK, SAVE>(a, blockIdx.x, n0, min(kMmaSamples, a.N - n0), mma_smem, Nothing(), Nothing(),
                           Nothing(), ToFilter<__half, KK>{a.cf, a.C});
 }
 

@@ -186,10 +186,11 @@ __device__ __forceinline__ void load_to_lds(uint32_t lds, const char *base, int 
 // This wave's are there.
 __device__ __forceinline__ void loads_to_lds_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// What a workgroup does beside the branch - while its first requests are on their way; once a
-// wave's hidden values are made - and where a channel's taps go.
+// What a workgroup does beside the branch - in front of its first requests, behind them in a wave that fetches weights
+// (true); while they are on their way; once a wave's hidden values are made - and where a channel's taps go.
 struct Nothing {
-    __device__ __forceinline__ void operator()() const {}
+    template <typename... A>
+    __device__ __forceinline__ void operator()(A...) const {}
 };
 template <typename T, int KK>
 struct ToFilter {    // (sample, channel, taps) to a tensor
@@ -205,13 +206,14 @@ struct ToFilter {    // (sample, channel, taps) to a tensor
 
 // Channels 16 * bx on of the ns (up to 16) samples from n0 on, kMmaThreads threads.  SAVE: a.save
 // is wanted (compiled in, as a branch around every store has the loads before it wait one by one).
-template <int KK, bool SAVE, typename Meanwhile, typename After, typename Sink>
+template <int KK, bool SAVE, typename Begin, typename Meanwhile, typename After, typename Sink>
 __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0, int ns, unsigned char *smem,
-                                            const Meanwhile &meanwhile, const After &after, const Sink &sink) {
+                                            const Begin &begin, const Meanwhile &meanwhile, const After &after, const Sink &sink) {
     constexpr int TPW = KK <= 9 ? 2 : 4, TAP_WAVES = (KK + TPW - 1) / TPW;      // taps per wave
     constexpr int NORM_WAVES = kMmaSamples * kMmaChannels / kWave;
     static_assert(TAP_WAVES <= kMmaWaves && NORM_WAVES <= kMmaWaves && KK % 8 == 1);
     constexpr int ZP = kMmaChannels * KK + 1;            // (odd: samples in different banks)
+    at_once(a.w1, a.w2, a.parts, a.b1, a.C, a.mid, a.nparts, a.lds.w1, a.lds.w2, a.lds.chunk, a.lds.pitch, a.lds.hidden);
     const int C = a.C, mid = a.mid;
     _Float16 *pv = reinterpret_cast<_Float16 *>(smem);   // [C / 32][16 samples][32]: pooled vectors
     float *z = reinterpret_cast<float *>(smem);          // [sample][channel][tap], in their place and w1's
@@ -241,10 +243,18 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
             // two rows per load
             constexpr int ROUND = 8 / LOADERS;
             const int hi = lane >> 5;
-            int c[ROUND];
+            int c[ROUND], q0 = w;
 #pragma unroll
             for (int i = 0; i < ROUND; ++i) c[i] = (lane & 31) ^ (2 * (w + i * LOADERS) + hi);
-            for (int q0 = w; 2 * q0 < rows; q0 += 8)
+            // (whole rounds of rows that fill the lanes: no masks, which cost as many instructions again)
+            if (chunks == 32)
+                for (; 2 * (q0 + 8 - LOADERS) + 1 < rows; q0 += 8)
+#pragma unroll
+                    for (int i = 0; i < ROUND; ++i) {
+                        const int q = q0 + i * LOADERS;
+                        load_to_lds(to + q * 1024, base + q * 1024, (hi * 32 + c[i]) * 16);
+                    }
+            for (; 2 * q0 < rows; q0 += 8)
 #pragma unroll
                 for (int i = 0; i < ROUND; ++i) {
                     const int q = q0 + i * LOADERS;
@@ -258,7 +268,15 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
                 int c[ROUND];
 #pragma unroll
                 for (int i = 0; i < ROUND; ++i) c[i] = (piece * kWave + lane) ^ (w + i * LOADERS);
-                for (int q0 = w; q0 < rows; q0 += 16)
+                int q0 = w;
+                if (piece * kWave + kWave <= chunks)
+                    for (; q0 + 16 - LOADERS < rows; q0 += 16)
+#pragma unroll
+                        for (int i = 0; i < ROUND; ++i) {
+                            const int r = q0 + i * LOADERS;
+                            load_to_lds(to + (r * pieces + piece) * 1024, base + r * (C * 2), c[i] * 16);
+                        }
+                for (; q0 < rows; q0 += 16)
 #pragma unroll
                     for (int i = 0; i < ROUND; ++i) {
                         const int r = q0 + i * LOADERS;
@@ -297,6 +315,7 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
         if (together) stage_w2(wave - kPoolWaves, kMmaWaves - kPoolWaves);
         request_bias(wave);
     }
+    begin(wave >= kPoolWaves);
 
     // ---- the pooled vectors: given, or scale * the sum of nparts partial sums per value ----
     // A wave takes a sample, a lane four channels; where there are fewer samples than waves,
@@ -373,12 +392,16 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
     if (share > 1) {
         __syncthreads();
         if (wave < kPoolWaves && g == 0 && wave / share < ns && lane < c4s) {
-            float4_t sum = ps[wave * kWave + lane];
-            for (int k = 1; k < share; ++k) sum += ps[(wave + k) * kWave + lane];
+            float4_t x[kPoolWaves], sum = ps[wave * kWave + lane];
+#pragma unroll
+            for (int k = 1; k < kPoolWaves; ++k) x[k] = ps[min(wave + k, kPoolWaves - 1) * kWave + lane];
+#pragma unroll
+            for (int k = 1; k < kPoolWaves; ++k)
+                if (k < share) sum += x[k];
             put_pooled(wave / share, lane, scaled(sum));
         }
     }
-    meanwhile();
+    meanwhile(wave >= kPoolWaves);
     if (wave >= kPoolWaves) loads_to_lds_done();
     __syncthreads();
 
@@ -394,7 +417,7 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
         for (int t = r0 / 16 + wave; t * 16 < rend; t += kMmaWaves) {
             if (t != wave) request_bias(t);
             const unsigned char *arow = w1s + (t * 16 + col - r0) * a.lds.pitch;
-            const _Float16 *brow = pv + col * kMmaStep + quad * 8;
+            const _Float16 *brow = pv + min(col, ns - 1) * kMmaStep + quad * 8;    // (columns past the last: not used; fewer rows, fewer conflicts)
             float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
             constexpr int U = 8;
 #pragma unroll 1
@@ -414,7 +437,9 @@ __device__ __forceinline__ void channel_mma(const ChannelMma &a, int bx, int n0,
             half4_t h;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float v = relu(acc[0][e] + acc[1][e] + (float)__builtin_bit_cast(_Float16, b1v[e]));
+                uint32_t bias = b1v[e];
+                asm volatile("" : "+v"(bias));    // (converted here, not where it is asked for, which would be a wait there)
+                const float v = relu(acc[0][e] + acc[1][e] + (float)__builtin_bit_cast(_Float16, (uint16_t)bias));
                 h[e] = t * 16 + quad * 4 + e < mid ? (_Float16)v : (_Float16)0;
             }
             *reinterpret_cast<half4_t *>(hv + ((t >> 1) * kMmaSamples + col) * kMmaStep + (t & 1) * 16 + quad * 4) = h;
@@ -577,12 +602,18 @@ struct ChannelRows {
     // LDS, bytes: pooled vector, hidden vector, taps, partial sums | w1 by `chunk` rows | the
     // first `early` of the block's rows of w2, the others where w1 was
     int block, chunk, early, w1_at, w2_at, total;
+    // waves that have a value of the pooled vector per lane, that share a value's partial sums, both; 256 / width, rounded up
+    int width, share, pool_waves, width_magic;
 };
 // The layout for blocks of `block` channels; false: rows too long.
 template <typename T>
 inline bool channel_rows_lds(ChannelRows<T> &a, int block) {
     const int64_t row1 = (int64_t)a.C * sizeof(T), row2 = (int64_t)a.mid * sizeof(T), rows = (int64_t)block * kRowsKK;
     a.block = block;
+    a.width = (a.C + kWave - 1) / kWave;
+    a.share = a.parts && a.nparts > kMmaRound && a.width <= kRowsPoolWaves / 2 ? kRowsPoolWaves / a.width : 1;
+    a.pool_waves = std::min(a.width * a.share, kRowsPoolWaves);
+    a.width_magic = (256 + a.width - 1) / a.width;
     a.w1_at = mma_round(((int64_t)a.C + a.mid + rows + kRowsPoolWaves * kWave) * 4);
     const int64_t left = kMmaLds - a.w1_at - 32;
     if (left < 8 * row1) return false;
@@ -654,10 +685,12 @@ __device__ __forceinline__ float row_sum(float v) {
 
 
 // Block bx of sample n's channels, kRowsThreads threads.
-template <typename T, bool SAVE, typename Meanwhile, typename After, typename Sink>
+template <typename T, bool SAVE, typename Begin, typename Meanwhile, typename After, typename Sink>
 __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, int64_t n, unsigned char *smem,
-                                             const Meanwhile &meanwhile, const After &after, const Sink &sink) {
+                                             const Begin &begin, const Meanwhile &meanwhile, const After &after, const Sink &sink) {
     constexpr int KK = kRowsKK, VE = 16 / sizeof(T);
+    at_once(a.w1, a.w2, a.parts, a.b1, a.C, a.mid, a.nparts, a.block, a.w1_at, a.w2_at, a.chunk, a.early);
+    at_once(a.gain_vec, a.offset_vec, a.b2, a.width, a.share, a.pool_waves, a.width_magic, a.scale);
     const int C = a.C, mid = a.mid;
     float *v = reinterpret_cast<float *>(smem);     // [C]
     float *h = v + C;                               // [mid]
@@ -683,22 +716,38 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
             if (at < count) *reinterpret_cast<T *>(smem + to + at * (int)sizeof(T)) = from[at];
         }
     };
-    T gain[KK] = {}, offset[KK] = {}, bias[KK] = {};
+    // a channel's KK contiguous values of a parameter, in 16 bytes at a time and the last one
+    typedef typename std::conditional<sizeof(T) == 2, _Float16, float>::type raw_t;
+    typedef raw_t vec_t __attribute__((ext_vector_type(VE)));
+    static_assert(KK % VE == 1);
+    struct Values {
+        vec_t v[KK / VE];
+        raw_t last;
+        __device__ __forceinline__ float at(int j) const { return (float)(j < KK - 1 ? v[j / VE][j % VE] : last); }
+    };
+    Values gain, offset, bias;
     // (a lane of the first waves takes a channel of the pooled vector; of many partial sums several
     // waves share a channel's; the others fetch the weights)
-    const int width = (C + kWave - 1) / kWave;      // waves side by side
-    const int share = a.parts && a.nparts > kMmaRound && width <= kRowsPoolWaves / 2 ? kRowsPoolWaves / width : 1;
-    const int pool_waves = min(width * share, kRowsPoolWaves);
+    const int width = a.width, share = a.share, pool_waves = a.pool_waves;
     if (wave >= pool_waves) {
         stage(a.w1, min(a.chunk, mid) * C, a.w1_at, wave - pool_waves, kRowsWaves - pool_waves);
         stage(a.w2 + (int64_t)cb * KK * mid, early * mid, a.w2_at, wave - pool_waves, kRowsWaves - pool_waves);
     }
 
+    begin(wave >= pool_waves);
+
     const int seg = lane >> 4, sl = lane & 15;
-    const float b1_first = a.b1 ? ld(a.b1 + min(wave * 4 + seg, mid - 1)) : 0.f;
+    // (behind a descriptor that holds nothing where there is no bias: a branch would be waited in)
+    float b1_first;
+    {
+        const __amdgpu_buffer_rsrc_t r = rows::plane_rsrc(a.b1, a.b1 ? (uint32_t)(mid * sizeof(T)) : 0u);
+        const int at = min(wave * 4 + seg, mid - 1) * (int)sizeof(T);
+        if constexpr (sizeof(T) == 2) b1_first = (float)__builtin_bit_cast(_Float16, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0));
+        else b1_first = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0));
+    }
 
     // The pooled vector: given, or scale * the sum of nparts partial sums per value.
-    const int g = wave / width;
+    const int g = (wave * a.width_magic) >> 8;      // (used where width is four at most: wave / width)
     if (wave < pool_waves) {
         auto put = [&](int c, float x) __attribute__((always_inline)) {
             v[c] = x;
@@ -730,9 +779,14 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
         }
         // gains, offsets and biases of the channel that the thread normalises
         if (tid < channels) {
+            // (no such parameter: anything that is there, C * KK values of it at least.  Under a branch each, and in
+            // single values, they took a trip to memory in front of the barrier.)
             const int64_t at = (int64_t)(cb + tid) * KK;
-            auto get = [&](const T *p, T (&to)[KK]) __attribute__((always_inline)) {
-                if (p) __builtin_memcpy(to, p + at, sizeof(to));
+            auto get = [&](const T *p, Values &to) __attribute__((always_inline)) {
+                const T *from = (p ? p : a.w2) + at;
+#pragma unroll
+                for (int k = 0; k < KK / VE; ++k) __builtin_memcpy(&to.v[k], from + k * VE, sizeof(vec_t));
+                __builtin_memcpy(&to.last, from + KK - 1, sizeof(raw_t));
             };
             get(a.gain_vec, gain);
             get(a.offset_vec, offset);
@@ -742,15 +796,19 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
     if (share > 1) {
         __syncthreads();
         if (wave < width && tid < C) {
-            float sum = sums[tid];
-            for (int k = 1; k < share; ++k) sum += sums[(k * width + wave) * kWave + lane];
+            float x[kRowsPoolWaves];
+#pragma unroll
+            for (int k = 0; k < kRowsPoolWaves; ++k) x[k] = sums[min(k * width + wave, kRowsPoolWaves - 1) * kWave + lane];
+            float sum = x[0];
+#pragma unroll
+            for (int k = 1; k < kRowsPoolWaves; ++k) sum += k < share ? x[k] : 0.f;
             v[tid] = sum * a.scale;
             if constexpr (SAVE) {
                 if (a.save.pooled && bx == 0) a.save.pooled[n * C + tid] = sum * a.scale;
             }
         }
     }
-    meanwhile();
+    meanwhile(wave >= pool_waves);
     if (wave >= pool_waves) loads_to_lds_done();
     __syncthreads();
 
@@ -851,9 +909,9 @@ __device__ __forceinline__ void channel_rows(const ChannelRows<T> &a, int bx, in
 #pragma unroll
     for (int j = 0; j < KK; ++j) {
         u[j] = f[tid * KK + j];
-        params.gain[j] = a.gain_vec ? ld(&gain[j]) : a.gain;
-        params.offset[j] = ld(&offset[j]);
-        params.bias[j] = ld(&bias[j]);
+        params.gain[j] = a.gain_vec ? gain.at(j) : a.gain;
+        params.offset[j] = a.offset_vec ? offset.at(j) : 0.f;
+        params.bias[j] = a.b2 ? bias.at(j) : 0.f;
     }
     const int64_t to = (n * C + cb + tid) * KK;
     if constexpr (SAVE) {

@@ -308,4 +308,28 @@ hipError_t tiled_backward(const Problem &p, const T *go, const T *x, const T *cf
                           const T *sf, T *dx, T *dcf, T *dsf, void *ws,
                           unsigned need, hipStream_t st, NormTail<T> *norm = nullptr);
 
+#ifdef __HIPCC__
+// A kernel's arguments, all in front of its first instruction: they are read from memory, and read where each is needed a
+// launch of a few microseconds waits for them two or three times (0.2 us each).
+template <typename A, typename B, typename C, typename D>
+__device__ __forceinline__ void at_once(A a, B b, C c, D d) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+}
+template <typename A, typename B, typename C, typename D, typename... More>
+__device__ __forceinline__ void at_once(A a, B b, C c, D d, More... more) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+    at_once(more...);
+}
+
+// Division by a number that the host knows: by a multiplication where that is exact (0: it is not).
+struct Divisor {
+    uint32_t by, magic;
+    // of numbers below `most`
+    static Divisor make(int64_t by, int64_t most) {
+        return {(uint32_t)by, by > 1 && by * most < (1ll << 32) ? (uint32_t)(((1ull << 32) + by - 1) / by) : 0u};
+    }
+    __device__ __forceinline__ uint32_t of(uint32_t n) const { return by == 1 ? n : magic ? __umulhi(n, magic) : n / by; }
+};
+#endif  // __HIPCC__
+
 }  // namespace ddf

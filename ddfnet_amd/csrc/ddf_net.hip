@@ -774,10 +774,10 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps tap
             const int by = block / blocks_x, bx = block - by * blocks_x;
             const ToFilter<__half, 9> sink{channels.a.cf, channels.a.C};
             if constexpr (CH == kChannelsRows) {
-                channel_rows<__half, false>(channels.a, bx, by, branch_smem, Nothing(), Nothing(), sink);
+                channel_rows<__half, false>(channels.a, bx, by, branch_smem, Nothing(), Nothing(), Nothing(), sink);
             } else {
                 const int n0 = by * kMmaSamples;
-                channel_mma<9, false>(channels.a, bx, n0, min(kMmaSamples, channels.a.N - n0), branch_smem, Nothing(), Nothing(), sink);
+                channel_mma<9, false>(channels.a, bx, n0, min(kMmaSamples, channels.a.N - n0), branch_smem, Nothing(), Nothing(), Nothing(), sink);
             }
             return;
         }
@@ -947,15 +947,23 @@ struct NetFew {
     int sf, tile, channels;                    // where in LDS (bytes): spatial taps, rows, the channel branch's
 };
 constexpr int kFewItems = 3;
+// One workgroup per compute unit, of up to this many pixels: with more of them the launch takes longer than the two it
+// replaces (ResNet-50, us, at most 256 or 512 / at most 128 / two launches: 1 image 342 / 340 / 385, 8 471 / 458 /
+// 468, 16 596 / 573 / 570).
+constexpr int kFewBlocks = 256, kFewPixels = 128;
 constexpr int kFewCf = 9 * kMmaChannels * 2;   // the channels' taps [tap][channel], at LDS 0
 
 template <int KS, int S, bool MUL, bool WIDE, int CH>
 __global__ __launch_bounds__(branch_threads(CH)) void k_net_filter_few(NetFew a, ChannelArgs<CH> channels) {
     constexpr int C = KS * 32, KK = 9, GROUPS = C / kMmaChannels, THREADS = branch_threads(CH), WAVES = THREADS / kWave;
     constexpr int ITEMS = kFewItems;           // 16-byte vectors of the rows per thread at most
+    constexpr int V = kMmaChannels * kFewPixels / THREADS, PER = kMmaChannels / V;    // channels of a thread, threads of a pixel
+    typedef _Float16 lane_t __attribute__((ext_vector_type(V)));
     extern __shared__ __align__(16) unsigned char few_smem[];
     _Float16 *cfs = reinterpret_cast<_Float16 *>(few_smem), *sfs = reinterpret_cast<_Float16 *>(few_smem + a.sf);
     rows_u4 *tile = reinterpret_cast<rows_u4 *>(few_smem + a.tile);
+    at_once(a.x, a.H, a.W, a.Ho, a.Wo, a.rows, a.per_row, a.per_row_magic, a.wo_magic, a.sf, a.tile, a.channels);
+    at_once(a.norm.weight, a.norm.bias, a.norm.mean, a.norm.var);
     const int g = blockIdx.x % GROUPS, chunk = blockIdx.x / GROUPS, n = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int y0 = chunk * a.rows, rows = min(a.rows, a.Ho - y0), pixels = rows * a.Wo;
@@ -969,21 +977,11 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_filter_few(NetFew a,
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(xn, sample_bytes);
     rows_u4 part[ITEMS];
     int to[ITEMS];
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        const int i = wave + k * WAVES, yy = (int)((uint32_t)i * a.per_row_magic >> 16), at = (i - yy * a.per_row) * kWave + lane;
-        const int y = S * y0 - 1 + yy, x = (at >> 1) - 1;
-        to[k] = i < waves_of && at < 2 * pitch ? yy * 2 * pitch + at : -1;
-        const bool in = to[k] >= 0 && y >= 0 && y < a.H && x >= 0 && x < a.W;
-        part[k] = __builtin_bit_cast(rows_u4, __builtin_amdgcn_raw_buffer_load_b128(
-            xr, in ? ((y * a.W + x) * C + g * kMmaChannels + (at & 1) * 8) * 2 : (int)kOutside, 0, 0));
-    }
     // (row of a result pixel of the workgroup: below 512, as Wo is)
     auto row_of = [&](int q) __attribute__((always_inline)) { return (int)(((uint32_t)q * a.wo_magic) >> 20); };
-    const int o = tid & 1, p = tid >> 1;
-    const int c = g * kMmaChannels + o * 8;
-    Affine<8> aff;
-    aff.request(a.norm, c);
+    const int o = tid % PER, p = tid / PER;
+    const int c = g * kMmaChannels + o * V;
+    Affine<V> aff;
     // Spatial taps by the last waves first, which have nothing to do when the hidden values are
     // made: the pixels of a wave's first tile are requested early, its taps are worked out then.
     TapWeights<KS> weights;
@@ -996,18 +994,38 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_filter_few(NetFew a,
     };
     const int t_first = WAVES - 1 - wave;
     constexpr bool kEarly = KS <= 8;           // (512 channels: no registers for that)
-    auto meanwhile = [&]() __attribute__((always_inline)) {
+    // (a wave that fetches weights asks for these behind them: it waits for all of it)
+    auto early = [&]() __attribute__((always_inline)) {
+        aff.request(a.norm, c);
         if (kEarly && t_first * 16 < pixels) {
             pixels_of(t_first);
             weights.request(a.tap_w, a.tap_bias, lane);
         }
+    };
+    auto begin = [&](bool loader) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            to[k] = -1;
+            if (wave + k * WAVES >= waves_of) continue;
+            const int i = wave + k * WAVES, yy = (int)((uint32_t)i * a.per_row_magic >> 16), at = (i - yy * a.per_row) * kWave + lane;
+            const int y = S * y0 - 1 + yy, x = (at >> 1) - 1;
+            to[k] = at < 2 * pitch ? yy * 2 * pitch + at : -1;
+            const bool in = to[k] >= 0 && y >= 0 && y < a.H && x >= 0 && x < a.W;
+            part[k] = __builtin_bit_cast(rows_u4, __builtin_amdgcn_raw_buffer_load_b128(
+                xr, in ? ((y * a.W + x) * C + g * kMmaChannels + (at & 1) * 8) * 2 : (int)kOutside, 0, 0));
+        }
+        if (loader) early();
+    };
+    auto meanwhile = [&](bool loader) __attribute__((always_inline)) {
+        if (!loader) early();
 #pragma unroll
         for (int k = 0; k < ITEMS; ++k)
             if (to[k] >= 0) tile[to[k]] = part[k];
     };
-    float sc[8], sh[8];
+    float sc[V], sh[V];
     auto after = [&]() __attribute__((always_inline)) {
         aff.finish(a.norm, sc, sh);
+        weights.hold();
         for (int t = t_first; t * 16 < pixels; t += WAVES) {
             if (!kEarly || t != t_first) pixels_of(t);
             if (!kEarly) weights.request(a.tap_w, a.tap_bias, lane);
@@ -1018,16 +1036,17 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_filter_few(NetFew a,
 #pragma unroll
         for (int t = 0; t < KK; ++t) cfs[t * kMmaChannels + (c & (kMmaChannels - 1))] = (_Float16)u[t];
     };
-    if constexpr (CH == kChannelsRows) channel_rows<__half, false>(channels.a, g, n, few_smem + a.channels, meanwhile, after, sink);
-    else channel_mma<KK, false>(channels.a, g, n, 1, few_smem + a.channels, meanwhile, after, sink);
+    if constexpr (CH == kChannelsRows) channel_rows<__half, false>(channels.a, g, n, few_smem + a.channels, begin, meanwhile, after, sink);
+    else channel_mma<KK, false>(channels.a, g, n, 1, few_smem + a.channels, begin, meanwhile, after, sink);
     __syncthreads();
     if (p >= pixels) return;
     const int y = row_of(p), x = p - y * a.Wo;
     uint32_t tap[6];
     __builtin_memcpy(tap, __builtin_assume_aligned(sfs + p * kTapPitch, 8), sizeof(tap));
-    float acc[8];
+    float acc[V];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    for (int e = 0; e < V; ++e) acc[e] = 0.f;
+    const lane_t *const xs = reinterpret_cast<const lane_t *>(tile) + o, *const cs = reinterpret_cast<const lane_t *>(cfs) + o;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1035,17 +1054,15 @@ __global__ __launch_bounds__(branch_threads(CH)) void k_net_filter_few(NetFew a,
             const int t = i * 3 + j;
             const half2_t sp = __builtin_bit_cast(half2_t, tap[t / 2]);
             const half2_t sv = {sp[t & 1], sp[t & 1]};
-            const rows_u4 xw = tile[((S * y + i) * pitch + S * x + j) * 2 + o];
-            const rows_u4 cw = *reinterpret_cast<const rows_u4 *>(cfs + t * kMmaChannels + o * 8);
+            const lane_t xw = xs[((S * y + i) * pitch + S * x + j) * PER], cw = cs[t * PER];
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                filter_pair<MUL, WIDE>(__builtin_bit_cast(half2_t, (uint32_t)cw[k]), sv,
-                                       __builtin_bit_cast(half2_t, (uint32_t)xw[k]), acc[2 * k], acc[2 * k + 1]);
+            for (int k = 0; k < V / 2; ++k)
+                filter_pair<MUL, WIDE>(half2_t{cw[2 * k], cw[2 * k + 1]}, sv, half2_t{xw[2 * k], xw[2 * k + 1]}, acc[2 * k], acc[2 * k + 1]);
         }
-    half8_t r;
+    lane_t r;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (_Float16)relu(fmaf((float)(_Float16)acc[e], sc[e], sh[e]));
-    *reinterpret_cast<half8_t *>(a.out + (((int64_t)n * a.Ho + y0 + y) * a.Wo + x) * C + c) = r;
+    for (int e = 0; e < V; ++e) r[e] = (_Float16)relu(fmaf((float)(_Float16)acc[e], sc[e], sh[e]));
+    *reinterpret_cast<lane_t *>(a.out + (((int64_t)n * a.Ho + y0 + y) * a.Wo + x) * C + c) = r;
 }
 
 // ---- mean (fp16) or sum (fp32) over the pixels ---------------------------------------------
@@ -1208,11 +1225,6 @@ hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *o
                        (const _Float16 *)img, (const _Float16 *)w, norm, (_Float16 *)out, (int)N, (int)H, (int)W, tx, ty);
     return hipGetLastError();
 }
-
-// One workgroup per compute unit, of up to this many pixels: a pixel is a thread's pair, and with
-// more of them the launch takes longer than the two it replaces (ResNet-50, us, at most 256 or 512 /
-// at most 128 / two launches: 1 image 342 / 340 / 385, 8 471 / 458 / 468, 16 596 / 573 / 570).
-constexpr int kFewBlocks = 256, kFewPixels = 128;
 
 // Waves of the spatial branch at most: the weights a wave loads first are paid for once per walk.
 constexpr int kMaxTapWaves = 8192;

@@ -22,28 +22,6 @@ __device__ __forceinline__ int xcd_block(int block, int blocks) {
 }
 inline unsigned xcd_grid(int64_t blocks) { return (unsigned)(cdiv(blocks, kXcd) * kXcd); }
 
-// A kernel's arguments, all in front of its first instruction: they are read from memory, and read where each is needed a
-// launch of a few microseconds waits for them two or three times (0.2 us each).
-template <typename A, typename B, typename C, typename D>
-__device__ __forceinline__ void at_once(A a, B b, C c, D d) {
-    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
-}
-template <typename A, typename B, typename C, typename D, typename... More>
-__device__ __forceinline__ void at_once(A a, B b, C c, D d, More... more) {
-    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
-    at_once(more...);
-}
-
-// Division by a number that the host knows: by a multiplication where that is exact (0: it is not).
-struct Divisor {
-    uint32_t by, magic;
-    // of numbers below `most`
-    static Divisor make(int64_t by, int64_t most) {
-        return {(uint32_t)by, by > 1 && by * most < (1ll << 32) ? (uint32_t)(((1ull << 32) + by - 1) / by) : 0u};
-    }
-    __device__ __forceinline__ uint32_t of(uint32_t n) const { return by == 1 ? n : magic ? __umulhi(n, magic) : n / by; }
-};
-
 // y = scale * x + shift of the convolution's bias and the BatchNorm behind it, for V
 // consecutive channels: requested as vectors early, worked out where they are needed.  (Read
 // channel by channel at the end of a kernel they cost more than small kernels do.)  A parameter that is not there is asked
@@ -104,7 +82,7 @@ template <int KS>
 struct TapWeights {
     static constexpr int KK = 9;
     half8_t w[KS];
-    uint16_t b[4];
+    uint32_t b[4];
     // (rows past the ninth, and a bias that is not there, lie outside their buffers: zeros)
     __device__ __forceinline__ void request(const _Float16 *weight, const _Float16 *bias, int lane) {
         const int col = lane & 15, quad = lane >> 4;
@@ -113,7 +91,12 @@ struct TapWeights {
         for (int ks = 0; ks < KS; ++ks)
             w[ks] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(wr, col * KS * 64 + quad * 16, ks * 64, 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) b[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(br, (quad * 4 + e) * 2, 0, 0);
+        for (int e = 0; e < 4; ++e) b[e] = __builtin_amdgcn_raw_buffer_load_b16(br, (quad * 4 + e) * 2, 0, 0);
+    }
+    // The bias is converted behind this: the compiler has it done, and waited for, where it is asked for.
+    __device__ __forceinline__ void hold() {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(b[e]));
     }
     // v: channels ks * 32 + quad * 8 .. + 7 of the lane's pixel; `at`: where its taps go
     __device__ __forceinline__ void taps(const half8_t (&v)[KS], float gain, bool there, _Float16 *sf, int64_t at, int lane) const {
@@ -125,7 +108,7 @@ struct TapWeights {
         float f[4], s = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            f[e] = acc[e] + (float)__builtin_bit_cast(_Float16, b[e]);
+            f[e] = acc[e] + (float)__builtin_bit_cast(_Float16, (uint16_t)b[e]);
             s += f[e];
         }
         const float mean = rows_total(s) / (float)KK;
