@@ -850,7 +850,7 @@ int net_chain_impl(const char *name, const void *features, const void *channel_f
     const ddf::NetChain a{features, weight, residual, side_features, side_weight, next_weight, output, next, pool_parts,
                           net_norm(norm), net_norm(side_norm), net_norm(next_norm), M, (int)C, (int)side_C, (int)O,
                           (int)next_O, (int)(H * W), channel_filter, spatial_weight, spatial_bias, (float)spatial_gain,
-                          net_norm(filter_norm), (int)W, combine == DDF_MUL, 0, 0};
+                          net_norm(filter_norm), (int)W, combine == DDF_MUL, 0, 0, {}, {}};
     return net_result(ddf::net_chain(a, (hipStream_t)stream), name);
 }
 }  // namespace

@@ -144,6 +144,32 @@ template <typename T>
 hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t H, int64_t W, int64_t mid,
                          int head, int stride, void *ws, hipStream_t st);
 
+#ifdef __HIPCC__
+// A kernel's arguments, all in front of its first instruction: they are read from memory, and read where each is needed a
+// launch of a few microseconds waits for them two or three times (0.2 us each).
+template <typename A, typename B, typename C, typename D>
+__device__ __forceinline__ void at_once(A a, B b, C c, D d) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+}
+template <typename A, typename B, typename C, typename D, typename... More>
+__device__ __forceinline__ void at_once(A a, B b, C c, D d, More... more) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+    at_once(more...);
+}
+#endif  // __HIPCC__
+
+// Division by a number that the host knows: by a multiplication where that is exact (0: it is not).
+struct Divisor {
+    uint32_t by, magic;
+    // of numbers below `most`
+    static Divisor make(int64_t by, int64_t most) {
+        return {(uint32_t)by, by > 1 && by * most < (1ll << 32) ? (uint32_t)(((1ull << 32) + by - 1) / by) : 0u};
+    }
+#ifdef __HIPCC__
+    __device__ __forceinline__ uint32_t of(uint32_t n) const { return by == 1 ? n : magic ? __umulhi(n, magic) : n / by; }
+#endif
+};
+
 // Channels-last fp16 kernels of the DDF-ResNets' inference (ddf_net.hip).
 // The per-channel affine map behind a convolution: its bias and the BatchNorm (eval mode)
 // that follows; null pointers: absent (var null: no BatchNorm).
@@ -185,7 +211,9 @@ struct NetChain {
     float tap_gain;
     NetNorm filter_norm;
     int W, mul;
-    int tiles, pool_slots;    // (net_chain's own)
+    // net_chain's own
+    int tiles, pool_slots;
+    Divisor row, rows;        // pixels of a row, rows of an image
 };
 bool net_chain_covers(int64_t M, int64_t K, int64_t side_K, int64_t N, int64_t N2);
 // whether the spatial branch and the filter are made in front of it by the same launch
@@ -307,29 +335,5 @@ template <typename T>
 hipError_t tiled_backward(const Problem &p, const T *go, const T *x, const T *cf,
                           const T *sf, T *dx, T *dcf, T *dsf, void *ws,
                           unsigned need, hipStream_t st, NormTail<T> *norm = nullptr);
-
-#ifdef __HIPCC__
-// A kernel's arguments, all in front of its first instruction: they are read from memory, and read where each is needed a
-// launch of a few microseconds waits for them two or three times (0.2 us each).
-template <typename A, typename B, typename C, typename D>
-__device__ __forceinline__ void at_once(A a, B b, C c, D d) {
-    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
-}
-template <typename A, typename B, typename C, typename D, typename... More>
-__device__ __forceinline__ void at_once(A a, B b, C c, D d, More... more) {
-    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
-    at_once(more...);
-}
-
-// Division by a number that the host knows: by a multiplication where that is exact (0: it is not).
-struct Divisor {
-    uint32_t by, magic;
-    // of numbers below `most`
-    static Divisor make(int64_t by, int64_t most) {
-        return {(uint32_t)by, by > 1 && by * most < (1ll << 32) ? (uint32_t)(((1ull << 32) + by - 1) / by) : 0u};
-    }
-    __device__ __forceinline__ uint32_t of(uint32_t n) const { return by == 1 ? n : magic ? __umulhi(n, magic) : n / by; }
-};
-#endif  // __HIPCC__
 
 }  // namespace ddf

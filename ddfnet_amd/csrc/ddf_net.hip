@@ -727,6 +727,7 @@ struct NetTaps {
     _Float16 *sf;
     int W, Wo, npix, plane, pixels, tiles;    // npix, plane: results, pixels of a sample; pixels: results of all
     float gain;
+    Divisor sample, row;    // by npix, by Wo
 };
 
 template <int KS, int S, int U>
@@ -742,7 +743,7 @@ __device__ __forceinline__ void net_taps(const NetTaps &a, int wave, int waves) 
             const int p = min((t0 + u) * 16 + col, a.pixels - 1);    // (past the last: not stored)
             int64_t at = p;
             if constexpr (S == 2) {
-                const int n = p / a.npix, q = p - n * a.npix, y = q / a.Wo, xx = q - y * a.Wo;
+                const int n = (int)a.sample.of(p), q = p - n * a.npix, y = (int)a.row.of(q), xx = q - y * a.Wo;
                 at = (int64_t)n * a.plane + 2 * y * a.W + 2 * xx;
             }
             const _Float16 *src = a.x + at * C + quad * 8;
@@ -768,6 +769,7 @@ template <int KS, int S, int U, int CH>
 __global__ __launch_bounds__(branch_threads(CH)) void k_net_branches(NetTaps taps, ChannelArgs<CH> channels, int blocks_x,
                                                                      int blocks) {
     extern __shared__ __align__(16) unsigned char branch_smem[];
+    at_once(taps.x, taps.w, taps.bias, taps.sf, taps.W, taps.Wo, taps.npix, taps.plane, taps.pixels, taps.tiles, blocks, blocks_x);
     const int block = blockIdx.x;
     if constexpr (CH != kNoChannels) {
         if (block < blocks) {
@@ -805,9 +807,11 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
                                                          const _Float16 *__restrict__ cf,
                                                          const _Float16 *__restrict__ sf, NetNorm norm,
                                                          _Float16 *__restrict__ out, int H, int W, int Ho, int Wo,
-                                                         int runs, int run, int units, int blocks, uint32_t x_bytes,
-                                                         uint32_t out_bytes, uint32_t tap_bytes) {
+                                                         Divisor runs, Divisor rows, int run, int units, int blocks,
+                                                         uint32_t x_bytes, uint32_t out_bytes, uint32_t tap_bytes) {
     constexpr int C = LP * 8, SLOTS = kWave / LP, KK = 9;
+    at_once(x, cf, sf, out, H, W, Wo, run, units, blocks, x_bytes, tap_bytes);
+    at_once(runs.by, runs.magic, rows.by, rows.magic);
     const int block = xcd_block(blockIdx.x, blocks);
     if (block >= blocks) return;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -815,8 +819,8 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
     const int unit = (block * (kThreads / kWave) + wave) * SLOTS + lane / LP;
     const bool live = unit < units;
     const int u = live ? unit : units - 1;
-    const int row = u / runs, r = u - row * runs;
-    const int n = row / Ho, y = row - n * Ho;
+    const int row = (int)runs.of(u), r = u - row * (int)runs.by;
+    const int n = (int)rows.of(row), y = row - n * Ho;
     const int x0 = r * run;
     const int x1 = live ? min(x0 + run, Wo) : x0;
     // (lanes of a wave may belong to different samples: one descriptor over all of them)
@@ -930,11 +934,13 @@ __global__ __launch_bounds__(kThreads) void k_net_filter(const _Float16 *__restr
 // taps of `rows` result rows and those rows' results of its channels: every workgroup of a sample
 // recomputes the hidden vector, every one of a row its spatial taps, and neither goes through
 // memory.  The rows it reads (and zeros around them) come into LDS as [pixel][16 channels] while
-// the channel branch waits for its weights, the spatial taps are computed meanwhile; then a
-// thread takes eight channels of a pixel.  Rounding is k_net_filter's.  us, two
-// launches / this: one image 56 x 56 x 64 10.3 / 7.7, 28 x 28 x 128 10.4 / 6.9, 14 x 14 x 256 10.6 /
-// 6.9, 7 x 7 x 512 11.9 / 9.6; most of it is the channel branch's chain and the instructions in front
-// of the first barrier (divisions by runtime values there cost 1 us).
+// the channel branch waits for its weights, the spatial taps are computed meanwhile; then every
+// thread takes four (of sixteen waves, two) channels of a pixel.  Rounding is k_net_filter's.  us, two
+// launches / this: one image 56 x 56 x 64 10.3 / 6.2, 28 x 28 x 128 10.4 / 5.9, 14 x 14 x 256 10.6 /
+// 6.1, 7 x 7 x 512 11.9 / 7.9; most of it is the channel branch's chain and the instructions in front
+// of the first barrier (divisions by runtime values there cost 1 us).  Weights go out in front of everything else; a
+// conversion that the compiler does where its operand is asked for was a trip to memory in front of a barrier, and eight
+// channels to half of the threads 0.4 us: 7.4, 7.0, 6.7 and 8.1 us a launch with those.
 struct NetFew {
     const _Float16 *x, *tap_w, *tap_bias;
     _Float16 *out;
@@ -1256,7 +1262,8 @@ hipError_t net_branches(const void *x, const void *w, const void *bias, void *sf
     const int64_t pixels = N * (H / stride) * (W / stride);
     const NetTaps taps{(const _Float16 *)x, (const _Float16 *)w, (const _Float16 *)bias, (_Float16 *)sf, (int)W,
                        (int)(W / stride), (int)((H / stride) * (W / stride)), (int)(H * W), (int)pixels,
-                       (int)cdiv(pixels, 16), (float)gain};
+                       (int)cdiv(pixels, 16), (float)gain,
+                       Divisor::make((H / stride) * (W / stride), pixels), Divisor::make(W / stride, (H / stride) * (W / stride))};
     ChannelArgs<kChannelsMma> mma{};
     ChannelArgs<kChannelsRows> rows{};
     int kind = kNoChannels, blocks_x = 1, blocks = 0, lds = 0;
@@ -1351,8 +1358,8 @@ hipError_t net_filter(const void *x, const void *cf, const void *sf, const NetNo
         bool done = false;
 #define DDF_NET_FILTER_LAUNCH(LP_, S_, MUL_, WIDE_)                                                         \
     hipLaunchKernelGGL((k_net_filter<LP_, S_, MUL_, WIDE_>), dim3(xcd_grid(blocks)), dim3(kThreads), 0, st, \
-                       xn, cn, sn, norm, on, (int)H, (int)W, (int)Ho, (int)Wo, (int)runs, run, (int)units,  \
-                       (int)blocks, (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2),        \
+                       xn, cn, sn, norm, on, (int)H, (int)W, (int)Ho, (int)Wo, Divisor::make(runs, units),  \
+                       Divisor::make(Ho, cnt * Ho), run, (int)units, (int)blocks, (uint32_t)(cnt * sample), (uint32_t)(cnt * Ho * Wo * C * 2),        \
                        (uint32_t)(cnt * Ho * Wo * kTapPitch * 2))
 #define DDF_NET_FILTER(LP_, S_)                                     \
     if (C == LP_ * 8 && stride == S_) {                             \

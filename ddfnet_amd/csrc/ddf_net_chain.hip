@@ -66,7 +66,7 @@ template <int K, bool MUL>
 __device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int wave, int lane, _Float16 *to, _Float16 *sf) {
     constexpr int KS = K / 32, LP = K / 8, SLOTS = kWave / LP, PER = 32 / SLOTS, RING = 5;
     static_assert(PER % kRun == 0);
-    const int cl = lane % LP, H = a.npix / a.W, W = a.W;
+    const int cl = lane % LP, H = (int)a.rows.by, W = a.W;
     // (all offsets from a pixel in front of the tile's neighbours: a tile's are 32-bit ones)
     const int64_t base = m0 - W - 1 > 0 ? m0 - W - 1 : 0;
     const __amdgpu_buffer_rsrc_t xr = plane_rsrc(static_cast<const _Float16 *>(a.x) + base * K,
@@ -93,8 +93,8 @@ __device__ __forceinline__ void filter_pixels(const NetChain &a, int64_t m0, int
     for (int run = 0; run < PER / kRun; ++run) {
         const int px = wave * 32 + lane / LP * PER + run * kRun;    // in the tile
         const bool live = m0 + px < a.M;
-        const unsigned pix = live ? (unsigned)m0 + px : (unsigned)m0, row = pix / (unsigned)W;
-        const int xx = (int)(pix - row * W), n = (int)(row / (unsigned)H), y = (int)(row - (unsigned)n * H);
+        const unsigned pix = live ? (unsigned)m0 + px : (unsigned)m0, row = a.row.of(pix);
+        const int xx = (int)(pix - row * W), n = (int)a.rows.of(row), y = (int)(row - (unsigned)n * H);
         uint32_t rowo[3];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
@@ -237,6 +237,9 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int l32 = lane & 31, hi = lane >> 5;
+    at_once(a.x, a.w, a.w2, a.res, a.out, a.M, a.N, a.npix, a.tiles, a.norm.weight, a.norm.bias, a.norm.mean);
+    at_once(a.norm.var, a.norm.conv_bias, a.norm2.weight, a.norm2.bias, a.norm2.mean, a.norm2.var, a.norm2.conv_bias, a.next);
+    if constexpr (FILTER) at_once(a.cf, a.tap_w, a.tap_bias, a.W, a.row.by, a.row.magic, a.rows.by, a.rows.magic);
     const int block = xcd_block(blockIdx.x, a.tiles);
     if (block >= a.tiles) return;
     const int64_t m0 = (int64_t)block * BM;
@@ -570,6 +573,10 @@ hipError_t net_chain(NetChain a, hipStream_t st) {
     if (a.cf && !net_chain_filters(a.W, a.K)) return hipErrorNotSupported;
     a.tiles = (int)cdiv(a.M, kChainRows);
     a.pool_slots = net_chain_pool_slots(a.M, a.npix);
+    if (a.cf) {
+        a.row = Divisor::make(a.W, a.M);
+        a.rows = Divisor::make(a.npix / a.W, a.M / a.W);
+    }
 #define DDF_CHAIN(K_, SIDE_, N2_, WPS_, FWPS_) \
     if (a.K == K_ && a.side_K == SIDE_ && a.N2 == N2_) {                                            \
         if (!a.cf) return launch_chain<K_, SIDE_, N2_, WPS_, kNoFilter>(a, st);                     \
