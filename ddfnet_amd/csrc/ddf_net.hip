@@ -78,12 +78,6 @@ constexpr int conv_lds_halves() {
     return ring > tile ? ring : tile;
 }
 
-// The tiles of a product, row by row; of a pair's first product, the pixels it samples.
-struct TileCut {
-    int tiles;
-    Divisor tiles_n, npix, Wo;
-};
-
 // ALONE: a stage's loads in front of its products instead of between them (see launch_conv).
 template <int BM, int BN, int KST, int ST, int WG, bool PAIR, bool POOL, bool RES, bool ALONE = false>
 __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, TileCut cut) {
@@ -448,109 +442,6 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
                     while (++slot < a.pool_slots) to[(int64_t)slot * a.N] = 0.f;
             }
             if (n < n_last) __syncthreads();
-        }
-    }
-}
-
-// Few pixels, where tiles of 64 leave most of the chip idle: a workgroup takes 16 pixels x 16
-// channels, its four waves a quarter of K each, operands straight from memory (every value is
-// used by one wave only); the waves' sums meet in LDS.  K goes by in blocks of 64 of which a lane
-// takes a quarter, 32 contiguous bytes in two loads (the order of the summed dimension is free
-// as long as both operands agree), four blocks of a wave in flight.  What the launch takes is what
-// one compute unit's operands take on their way in, so smaller tiles are faster than larger ones
-// and than more waves (us for 32 x 32, the same with sixteen waves, 16 x 16: 49 x 2048 -> 512 9.7,
-// 9.7, 7.2; 196 x 1024 -> 256 6.7, 9.9, 5.7; 1 x 2048 -> 1000 7.1, 7.1, 5.2; without a last round of
-// loads that nothing used 16 x 16 takes 5.7, 4.2 and 4.3).
-template <bool POOL>
-__global__ __launch_bounds__(kThreads) void k_net_conv_split(NetConv a, Divisor tiles_n) {
-    constexpr int WAVES = kThreads / kWave, D = 4, T = 16;
-    __shared__ float red[WAVES][T][T + 1];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    at_once(a.x, a.w, a.M, a.N, a.K, a.stride, tiles_n.by, tiles_n.magic);
-    at_once(a.norm.weight, a.norm.bias, a.norm.mean, a.norm.var, a.norm.conv_bias, a.out, a.res, a.relu);
-    const int tm = (int)tiles_n.of(blockIdx.x), tn = blockIdx.x - tm * (int)tiles_n.by;
-    const int col = lane & 15, quad = lane >> 4;
-    const int n0 = tn * T;
-    int64_t m = (int64_t)tm * T + col;
-    if (m >= a.M) m = a.M - 1;
-    if (a.stride > 1) {
-        const int64_t n = m / a.npix;
-        const int p = (int)(m - n * a.npix), y = p / a.Wo, xx = p - y * a.Wo;
-        m = (n * a.H + y * a.stride) * a.W + xx * a.stride;
-    }
-    const int blocks = a.K / 64, per = (blocks + WAVES - 1) / WAVES;
-    const int b0 = wave * per, b1 = min(b0 + per, blocks);
-    const _Float16 *xp = static_cast<const _Float16 *>(a.x) + m * a.K + quad * 16;
-    const _Float16 *wp = static_cast<const _Float16 *>(a.w) + (int64_t)min(n0 + col, a.N - 1) * a.K + quad * 16;
-    half8_t xv[D][2], wv[D][2];
-    auto request = [&](int set, int b) __attribute__((always_inline)) {
-        const int k = min(b, blocks - 1) * 64;    // (past the wave's range: not used)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            xv[set][u] = *reinterpret_cast<const half8_t *>(xp + k + u * 8);
-            wv[set][u] = *reinterpret_cast<const half8_t *>(wp + k + u * 8);
-        }
-    };
-#pragma unroll
-    for (int d = 0; d < D; ++d) request(d, b0 + d);
-    // (a thread finishes one channel of one pixel)
-    const int oc = n0 + (tid & (T - 1));
-    const int64_t om = (int64_t)tm * T + tid / T;
-    const bool ok = oc < a.N && om < a.M;
-    const _Float16 *res = static_cast<const _Float16 *>(a.res);
-    Affine<1> aff;
-    aff.request(a.norm, oc < a.N ? oc : 0);
-    const _Float16 rv = res ? res[ok ? om * a.N + oc : 0] : (_Float16)0;
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int d) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[d][u], xv[d][u], acc, 0, 0, 0);
-    };
-    // (the last round asks for nothing: its loads would be as many again as K = 1024 has)
-    int b = b0;
-    for (; b + D < b1; b += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            multiply(d);
-            request(d, b + d + D);
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-        if (b + d < b1) multiply(d);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][4 * quad + e][col] = acc[e];
-    __syncthreads();
-    float sc[1], sh[1];
-    aff.finish(a.norm, sc, sh);
-    if (!POOL && !ok) return;
-    float f = 0.f;
-#pragma unroll
-    for (int k = 0; k < WAVES; ++k) f += red[k][tid & (T - 1)][tid / T];
-    f = fmaf(a.norm.var ? (float)(_Float16)f : f, sc[0], sh[0]) + (float)rv;    // (see k_net_conv)
-    if (a.relu) f = relu(f);
-    if (!POOL || ok) static_cast<_Float16 *>(a.out)[om * a.N + oc] = (_Float16)f;
-    if constexpr (POOL) {
-        // (see k_net_conv: a channel's sums by one thread)
-        __shared__ float results[T][T + 1];
-        results[tid / T][tid & (T - 1)] = (float)(_Float16)f;
-        __syncthreads();
-        if (tid >= T || n0 + tid >= a.N) return;
-        const int first = tm * T, end = (int)min((int64_t)first + T, a.M), n_last = (end - 1) / a.npix;
-        float v[T];
-#pragma unroll
-        for (int r = 0; r < T; ++r) v[r] = results[r][tid];
-        for (int n = first / a.npix; n <= n_last; ++n) {
-            const int lo = n * a.npix - first, hi = lo + a.npix;
-            float sum = 0.f;
-#pragma unroll
-            for (int r = 0; r < T; ++r) sum += r >= lo && r < hi ? v[r] : 0.f;
-            float *to = a.pool + (int64_t)n * a.pool_slots * a.N + n0 + tid;
-            int slot = tm - (int)((int64_t)n * a.npix / T);
-            to[(int64_t)slot * a.N] = sum;
-            if (hi <= end - first)
-                while (++slot < a.pool_slots) to[(int64_t)slot * a.N] = 0.f;
         }
     }
 }
@@ -1139,39 +1030,43 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Rows of whole vectors, unless K is long and 16 x 16 results make a workgroup per compute unit
-// at most (us in tiles of 64 / split: 392 x 1024 -> 256, 400 workgroups, 6.1 / 6.1; 392 x 512 -> 256,
-// 400, 4.5 / 5.8; 784 x 1024 -> 256, 784, 6.4 / 9.4; split below that, 196 x 1024 -> 256, 208, takes
-// 4.2 and 98 x 2048 -> 512, 224, 6.1).
-bool conv_in_tiles(const NetConv &a) {
-    return a.N % 8 == 0 && !(a.K >= 512 && cdiv(a.M, 16) * cdiv(a.N, 16) <= 256);
-}
-
 // The largest tiles that leave somewhat more than a workgroup per compute unit.  Where a unit
 // goes through several, short stages leave room for one workgroup more; where it has one or
 // two, long stages cost fewer barriers (batch 128, us long / short stages: 3136 tiles of
 // 56 x 56 x 64 -> 256 76 / 65, 1568 of 28 x 28 x 512 -> 256 54 / 50, 784 of 14 x 14 x 1024 -> 512
 // 42.2 / 43.4, 392 of 14 x 14 x 1024 -> 256 24.1 / 28.5).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
 // 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
-enum ConvTile { kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64, kTileSplit };
+// In small tiles (ddf_net_small.hip), whose workgroups bring in a quarter of K per wave, what leaves most of the chip idle in tiles
+// of 64: 16 x 16 up to two workgroups per compute unit, 32 x 32 of a K that is worth four waves up to one.  us, tiles of 64 / 16 x 16 / 32 x 32:
+// 64 -> 64 of 1024 pixels, 256 tiles of 16, 2.95 / 2.88, 392 2.96 / 3.18 (a K of 64 is one wave's); 512 -> 128 784 pixels, 392, 4.28 / 3.58,
+// 1568 pixels, 784 and 196 of 32, 4.35 / 5.52 / 4.29; 256 -> 128 512 tiles 3.65 / 3.32, 784 and 196 3.69 / 4.96 / 3.95; 1024 -> 256 196
+// pixels 4.35 / 3.60, 400 5.70 / 4.27 / 5.05, 784 6.19 / 6.72 / 5.21, 1568, 392 of 32, 6.67 / 11.3 / 9.14; 2048 -> 512 49 6.09 / 4.26, 400
+// 10.2 / 10.1 / 7.1; 512 -> 2048 with a residual 49 pixels 4.21 / 3.14; pairs 256 + 512 -> 1024 49 7.06 / 3.68, 196 6.53 / 6.83 / 5.34, 512 +
+// 1024 -> 2048 49, 512 tiles, 8.95 / 5.86, 98 9.73 / 9.64 / 7.42; 2048 -> 1000 of 1, 49 and 128 rows 4.51 / 3.71, 6.53 / 5.23, 9.5 / 7.3 / 5.9.
+enum ConvTile { kSmall16, kSmall32, kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64 };
 // The same holds for pairs, but from 513 to 768 tiles three workgroups per unit are one round and two a full one and a
 // part.  us, short / long stages: 28 x 28 x 128 + 256 -> 512 344 tiles 14.9 / 13.8, 516 20.1 / 21.9, 588 21.6 / 23.7, 760 24.2 / 25.8, 784 28.1 / 26.8,
 // 980 31.4 / 29.7; 14 x 14 x 256 + 512 -> 1024 592 30.9 / 34.5, 784 41.6 / 38.8; 7 x 7 x 512 + 1024 -> 2048 592 50.8 / 52.1, 784
 // 70.3 / 62.4; 512 tiles of 8 x 8 x 512 + 1024 -> 2048 42.7 / 35.1, of 16 x 16 x 256 + 512 -> 1024 25.4 / 22.6.
-ConvTile conv_tile(const NetConv &a, bool pair) {
+ConvTile conv_tile(const NetConv &a, const NetConv *first) {
+    const bool pair = first;
+    const int64_t K = (int64_t)a.K + (pair ? first->K : 0);
     auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
     constexpr int kMany = 1024, kFew = 320;
-    if (!conv_in_tiles(a)) return kTileSplit;
+    if (a.N % 8 != 0 || count(16, 16) <= (K > 64 ? 512 : 256)) return kSmall16;
+    if (K > 256 && count(32, 32) <= 256) return kSmall32;
     if (a.N >= 128 && (count(128, 128) >= kMany || (pair && count(128, 128) > 512 && count(128, 128) <= 768))) return kTile128;
     if (a.N >= 128 && count(128, 128) >= kFew) return kTile128Long;
     if (count(128, 64) >= kMany) return kTile128x64;
     if (count(128, 64) >= 448) return kTile128x64Long;
     return kTile64;
 }
-int tile_rows(ConvTile t) { return t == kTileSplit ? 16 : t == kTile64 ? 64 : 128; }
+int tile_rows(ConvTile t) { return t == kSmall16 ? 16 : t == kSmall32 ? 32 : t == kTile64 ? 64 : 128; }
 
 hipError_t conv_tiles(ConvTile tile, const NetConv &a, const NetConv *first, hipStream_t st) {
     switch (tile) {
+        case kSmall16: return net_conv_small(16, a, first, st);
+        case kSmall32: return net_conv_small(32, a, first, st);
         case kTile128: return launch_conv<128, 128, 32, 3, 3>(a, first, st);
         case kTile128Long: return launch_conv<128, 128, 64, 2, 2>(a, first, st);
         case kTile128x64: return launch_conv<128, 64, 32, 3, 4>(a, first, st);
@@ -1187,36 +1082,20 @@ bool net_conv_supported(const NetConv &a) { return a.K % 64 == 0 && a.K > 0 && a
 // Slots of a sample in a convolution's sums over its pixels: one per tile of rows that a sample
 // can touch (samples start at multiples of the common divisor of their pixels and the tile).
 int net_conv_pool_slots(const NetConv &a) {
-    const int rows = tile_rows(conv_tile(a, false)), start = a.M > a.npix ? rows - std::gcd(rows, a.npix) : 0;
+    const int rows = tile_rows(conv_tile(a, nullptr)), start = a.M > a.npix ? rows - std::gcd(rows, a.npix) : 0;
     return (start + a.npix - 1) / rows + 1;
 }
 
 hipError_t net_conv(const NetConv &a, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_conv_supported(a) || (a.pool && a.M > INT32_MAX - 256)) return hipErrorNotSupported;
-    const ConvTile tile = conv_tile(a, false);
-    if (tile != kTileSplit) return conv_tiles(tile, a, nullptr, st);
-    const int tiles_n = (int)cdiv(a.N, 16);
-    const int64_t blocks = cdiv(a.M, 16) * tiles_n;
-    if (blocks > (1 << 30)) return hipErrorInvalidConfiguration;
-    if (a.pool)
-        hipLaunchKernelGGL((k_net_conv_split<true>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, Divisor::make(tiles_n, blocks));
-    else
-        hipLaunchKernelGGL((k_net_conv_split<false>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a, Divisor::make(tiles_n, blocks));
-    return hipGetLastError();
+    return conv_tiles(conv_tile(a, nullptr), a, nullptr, st);
 }
 
-// One launch where both products are made in tiles; else the projection's results wait in
-// `out`.
 hipError_t net_conv_pair(const NetConv &a, const NetConv &first, hipStream_t st) {
     if (a.M == 0) return hipSuccess;
     if (!net_conv_supported(a) || !net_conv_supported(first)) return hipErrorNotSupported;
-    if (conv_in_tiles(a) && conv_in_tiles(first)) return conv_tiles(conv_tile(a, true), a, &first, st);
-    hipError_t err = net_conv(first, st);
-    if (err != hipSuccess) return err;
-    NetConv last = a;
-    last.res = a.out;
-    return net_conv(last, st);
+    return conv_tiles(conv_tile(a, &first), a, &first, st);
 }
 
 hipError_t net_stem(const void *img, const void *w, const NetNorm &norm, void *out, int64_t N, int64_t H, int64_t W,

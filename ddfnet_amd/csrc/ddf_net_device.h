@@ -22,6 +22,12 @@ __device__ __forceinline__ int xcd_block(int block, int blocks) {
 }
 inline unsigned xcd_grid(int64_t blocks) { return (unsigned)(cdiv(blocks, kXcd) * kXcd); }
 
+// The tiles of a product, row by row; of a pair's first product, the pixels it samples.
+struct TileCut {
+    int tiles;
+    Divisor tiles_n, npix, Wo;
+};
+
 // y = scale * x + shift of the convolution's bias and the BatchNorm behind it, for V
 // consecutive channels: requested as vectors early, worked out where they are needed.  (Read
 // channel by channel at the end of a kernel they cost more than small kernels do.)  A parameter that is not there is asked
@@ -215,4 +221,7 @@ __device__ __forceinline__ void arrive() {
 }
 
 }  // namespace net
+
+// A convolution (two with `first`) in the tiles of ddf_net_small.hip: 16 x 16 or 32 x 32.
+hipError_t net_conv_small(int rows, const NetConv &a, const NetConv *first, hipStream_t st);
 }  // namespace ddf

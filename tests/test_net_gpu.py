@@ -65,6 +65,11 @@ def close(got, want, tol):
     (1, 13, 9, 1088, 31, 2, 1, 0, 0, 0),       # 17 blocks, under stride 2
     (1, 16, 16, 192, 4096, 1, 1, 0, 0, 1), (1, 1, 257, 320, 4096, 1, 1, 0, 1, 1),    # 256 tiles of 64, three stages; 320, five
     (20, 4, 8, 1024, 256, 1, 1, 0, 1, 1), (10, 8, 8, 2048, 1000, 1, 0, 1, 0, 0),     # 40, 160: a workgroup per unit at most
+    (1, 16, 32, 128, 256, 1, 1, 0, 1, 1), (1, 27, 19, 128, 256, 1, 1, 0, 1, 1),      # 512 tiles of 16 x 16; 528, and K short: of 64
+    (1, 16, 16, 64, 256, 1, 1, 1, 0, 0), (1, 16, 17, 64, 256, 1, 1, 1, 0, 0),        # 256 of a K of 64; 272
+    (1, 16, 16, 320, 1024, 1, 1, 0, 1, 1), (1, 1, 257, 320, 1024, 1, 1, 0, 1, 1),    # 256 tiles of 32 x 32, five blocks of K; 288: of 64
+    (3, 25, 26, 576, 264, 2, 1, 1, 1, 1), (10, 8, 8, 2048, 520, 1, 0, 1, 0, 0),      # 32 x 32 under stride 2, channels past a tile; no BatchNorm
+    (1, 64, 65, 64, 33, 1, 1, 0, 1, 1),        # 780 tiles of 16 x 16, channels no multiple of 8
 ])
 def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     torch.manual_seed(c + o)
@@ -84,7 +89,7 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
 @pytest.mark.parametrize('n,h,w,c,side,o,stride,relu', [
     (3, 5, 7, 64, 64, 64, 1, 1),               # a stage of K each, one tile
     (5, 9, 13, 64, 192, 136, 2, 0),            # rows and channels past a tile
-    (1, 14, 14, 512, 1024, 2048, 2, 1),        # few pixels, long rows: two launches
+    (1, 14, 14, 512, 1024, 2048, 2, 1),        # few pixels, long rows: 512 tiles of 16 x 16
     (8, 28, 28, 256, 512, 1024, 2, 1),         # tiles of 64
     (16, 28, 28, 128, 256, 264, 1, 1),         # 128 x 64
     (42, 56, 56, 64, 64, 136, 1, 1),           # 128 x 128, many
@@ -94,6 +99,8 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     (26, 56, 55, 192, 128, 520, 2, 1),         # 800, three and two
     (21, 31, 33, 320, 256, 640, 1, 1),         # 840, five and four
     (42, 56, 56, 128, 64, 64, 1, 1),           # 64 channels, many
+    (5, 9, 13, 192, 64, 133, 2, 0),            # channels no multiple of 8
+    (3, 25, 26, 128, 320, 264, 2, 1), (2, 17, 16, 64, 256, 520, 1, 0),    # tiles of 32 x 32, a wave with both products; channels past a tile
     (1, 520, 516, 64, 64, 64, 2, 1),           # 67080 pixels: too many for a division by multiplying
 ])
 def test_conv_pair(n, h, w, c, side, o, stride, relu):
@@ -110,6 +117,21 @@ def test_conv_pair(n, h, w, c, side, o, stride, relu):
     out = torch.empty(n, ho, wo, o, device='cuda', dtype=torch.float16)
     call('ddf_hip_net_conv_pair', x, wt, norm, c, xs, ws, norm_s, h, w, side, stride, out, n, o, relu)
     close(out, want, 3e-3)
+
+
+@pytest.mark.parametrize('n,c,side,o', [(40, 64, 192, 96), (600, 128, 320, 264)])
+def test_conv_pair_without_batchnorm(n, c, side, o):
+    """A bias joins the fp32 sum: each product is rounded once, and their sum once (2^-11 of it each)."""
+    torch.manual_seed(c + o)
+    x, xs = (torch.randn(n, 1, 1, k, device='cuda').half() for k in (c, side))
+    wt, ws = ((torch.randn(o, k, device='cuda') * k ** -0.5).half() for k in (c, side))
+    (norm, _, keep), (norm_s, _, keep_s) = (make_norm(o, 0, 1) for _ in range(2))
+    a = x.view(n, c).double() @ wt.double().t() + keep['conv_bias'].double()
+    b = xs.view(n, side).double() @ ws.double().t() + keep_s['conv_bias'].double()
+    out = torch.empty(n, o, device='cuda', dtype=torch.float16)
+    call('ddf_hip_net_conv_pair', x, wt, norm, c, xs, ws, norm_s, 1, 1, side, 1, out, n, o, 0)
+    bound = (a.abs() + b.abs() + (a + b).abs()) * 2.0 ** -11 + 1e-4    # (and the fp32 sums)
+    assert ((out.double() - a - b).abs() <= bound).all()
 
 
 @pytest.mark.parametrize('n,h,w', [(1, 32, 32), (2, 64, 96), (3, 40, 36), (70, 64, 64)])
@@ -219,6 +241,7 @@ def test_network_matches_its_modules(build, n, size, classes):
     (1, 14, 14, 1024, 256), (2, 14, 14, 1024, 256),
     (9, 28, 28, 64, 128), (33, 28, 28, 256, 64), (16, 28, 28, 128, 264), (42, 56, 56, 64, 136),
     (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64), (20, 4, 8, 1024, 256),
+    (5, 11, 11, 320, 264), (50, 3, 4, 576, 264), (3, 16, 16, 2048, 264), (7, 13, 9, 128, 65),    # 32 x 32, samples ending inside; 16 x 16
     (1, 260, 258, 64, 64),                      # 67080 pixels: too many for a division by multiplying
 ])
 def test_conv_pool(n, h, w, c, o):
