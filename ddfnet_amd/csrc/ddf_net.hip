@@ -38,7 +38,7 @@ using rows::plane_rsrc;
 
 // ---- 1x1 convolution ----------------------------------------------------------
 // out[m, o] = act(affine(sum_k x[row(m), k] w[o, k]) (+ res[m, o])), row(m) the sampled
-// pixel under a stride.  Tiles of BM pixels x BN channels; four waves, 2 x 2 over the tile,
+// pixel under a stride.  Tiles of BM pixels x BN channels; 2 x WN waves over the tile,
 // each in 32x32x16 steps.  W is the A operand, so a lane ends with runs of four channels of
 // one pixel; the tile goes through LDS once more and leaves as whole 16-byte vectors.
 // K comes in stages of KST that go from memory straight into a ring of ST LDS buffers, ST - 1
@@ -71,19 +71,19 @@ using rows::plane_rsrc;
 // With PAIR the tile is act(affine(x w) + affine'(x' w')) of two products, a bottleneck's last
 // convolution and its projection: x' w' goes first, its affine result stays in registers as
 // the fp16 values that a projection of its own would have stored.
-template <int BM, int BN, int KST, int ST>
+template <int BM, int BN, int KST, int ST, int WAVES>
 constexpr int conv_lds_halves() {
     // (behind the tile: the waves' sums over its pixels)
-    const int ring = (BM + BN) * KST * ST, tile = BM * (BN + 8) + kThreads / kWave * BN * 2;
+    const int ring = (BM + BN) * KST * ST, tile = BM * (BN + 8) + WAVES * BN * 2;
     return ring > tile ? ring : tile;
 }
 
 // ALONE: a stage's loads in front of its products instead of between them (see launch_conv).
-template <int BM, int BN, int KST, int ST, int WG, bool PAIR, bool POOL, bool RES, bool ALONE = false>
-__global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv first, TileCut cut) {
-    constexpr int CH = KST / 8, STAGE = (BM + BN) * KST;
-    constexpr int RX = BM * CH / kThreads, RW = BN * CH / kThreads;
-    constexpr int TM = BM / 64, TN = BN / 64;      // 32-wide tiles per wave: pixels, channels
+template <int BM, int BN, int KST, int ST, int WN, int WG, bool PAIR, bool POOL, bool RES, bool ALONE = false>
+__global__ __launch_bounds__(2 * WN * kWave, WG * WN / 2) void k_net_conv(NetConv a, NetConv first, TileCut cut) {
+    constexpr int WAVES = 2 * WN, T = WAVES * kWave, CH = KST / 8, STAGE = (BM + BN) * KST;
+    constexpr int RX = BM * CH / T, RW = BN * CH / T;
+    constexpr int TM = BM / 64, TN = BN / 32 / WN;      // 32-wide tiles per wave: pixels, channels
     constexpr int PITCH = BN + 8;
     static_assert((ST == 2 || ST == 3) && (CH == 4 || CH == 8) && RX > 0 && RW > 0 && !(RES && PAIR));
     extern __shared__ __align__(16) _Float16 net_smem[];
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             const int at = (int)(m0 - sample * c.npix);
 #pragma unroll
             for (int i = 0; i < RX; ++i) {
-                const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+                const int q = tid + i * T, r = q / CH, ch = (q % CH) ^ turn(r);
                 const unsigned pix = (unsigned)(at + min(r, rows - 1)), n = cut.npix.of(pix), p = pix - n * c.npix;
                 const unsigned y = cut.Wo.of(p), xx = p - y * c.Wo;
                 xp[i] = x + (((sample + n) * c.H + y * c.stride) * c.W + xx * c.stride) * c.K + ch * 8;
@@ -118,13 +118,13 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             x += m0 * c.K;
 #pragma unroll
             for (int i = 0; i < RX; ++i) {
-                const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+                const int q = tid + i * T, r = q / CH, ch = (q % CH) ^ turn(r);
                 xp[i] = x + ((int64_t)min(r, rows - 1) * c.K + ch * 8);
             }
         }
 #pragma unroll
         for (int i = 0; i < RW; ++i) {
-            const int q = tid + i * kThreads, r = q / CH, ch = (q % CH) ^ turn(r);
+            const int q = tid + i * T, r = q / CH, ch = (q % CH) ^ turn(r);
             wp[i] = w + ((int64_t)min(r, a.N - 1 - n0) * c.K + ch * 8);
         }
     };
@@ -133,14 +133,14 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     auto load_one = [&](int i, int buf) __attribute__((always_inline)) {
         const uint32_t at = ring + (uint32_t)(buf * STAGE) * 2 + (uint32_t)wave * (kWave * 16);
         const _Float16 *&p = i < RX ? xp[i < RX ? i : 0] : wp[i < RX ? 0 : i - RX];
-        load_to_lds(at + (i < RX ? i * kThreads * 16 : BM * KST * 2 + (i - RX) * kThreads * 16), p);
+        load_to_lds(at + (i < RX ? i * T * 16 : BM * KST * 2 + (i - RX) * T * 16), p);
         p += KST;
     };
     const int wm = wave & 1, wn = wave >> 1;
     const int l32 = lane & 31, hi = lane >> 5;
     // Lane column of a 32x32 step's D = pixel l32, rows (channels) 8 * g + 4 * hi + 0..3 in
     // registers 4g .. 4g+3.
-    auto channel = [&](int j, int g) { return wn * (BN / 2) + j * 32 + 8 * g + 4 * hi; };
+    auto channel = [&](int j, int g) { return wn * (BN / WN) + j * 32 + 8 * g + 4 * hi; };
     float16_t acc[TM][TN];
     auto clear = [&]() {
 #pragma unroll
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             const int ch = kk * 2 + hi;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                const int r = wn * (BN / 2) + j * 32 + l32;
+                const int r = wn * (BN / WN) + j * 32 + l32;
                 wv[kk & 1][j] = *reinterpret_cast<const half8_t *>(s + BM * KST + r * KST + (ch ^ turn(r)) * 8);
             }
 #pragma unroll
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
     // what the tile's results meet on their way out: this thread's eight channels, and the
     // residual of its pixels
     constexpr int CPR = BN / 8;                     // vectors per pixel
-    constexpr int RO = BM * CPR / kThreads, STEP = kThreads / CPR;
+    constexpr int RO = BM * CPR / T, STEP = T / CPR;
     const int cq = tid % CPR, r0 = tid / CPR, c = n0 + cq * 8;
     const bool cok = c < a.N;
     half8_t rv[RES ? RO : 1];
@@ -437,7 +437,9 @@ __global__ __launch_bounds__(kThreads, WG) void k_net_conv(NetConv a, NetConv fi
             if (tid < BN && n0 + tid < a.N) {
                 float *to = a.pool + (int64_t)n * a.pool_slots * a.N + n0 + tid;
                 int slot = tm - (int)((int64_t)n * a.npix / BM);
-                to[(int64_t)slot * a.N] = (red[tid] + red[BN + tid]) + (red[2 * BN + tid] + red[3 * BN + tid]);
+                float total = (red[tid] + red[BN + tid]) + (red[2 * BN + tid] + red[3 * BN + tid]);
+                if constexpr (WAVES == 8) total += (red[4 * BN + tid] + red[5 * BN + tid]) + (red[6 * BN + tid] + red[7 * BN + tid]);
+                to[(int64_t)slot * a.N] = total;
                 if (hi <= end - first)
                     while (++slot < a.pool_slots) to[(int64_t)slot * a.N] = 0.f;
             }
@@ -994,17 +996,15 @@ __global__ __launch_bounds__(kThreads) void k_net_pool(const _Float16 *__restric
     else out[(int64_t)n * C + cc] = s;
 }
 
-template <int BM, int BN, int KST, int ST, int WG>
+template <int BM, int BN, int KST, int ST, int WN, int WG>
 hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     const int tiles_n = (int)cdiv(a.N, BN);
     const int64_t tiles = cdiv(a.M, BM) * tiles_n;
     if (tiles > (1 << 30)) return hipErrorInvalidConfiguration;
-    const int lds = conv_lds_halves<BM, BN, KST, ST>() * (int)sizeof(_Float16);
+    const int lds = conv_lds_halves<BM, BN, KST, ST, 2 * WN>() * (int)sizeof(_Float16);
     // (a strided product's pixels are counted from a sample's first: below npix + BM; a pooled one's from the first)
     const NetConv &x = first ? *first : a;
     const TileCut cut{(int)tiles, Divisor::make(tiles_n, tiles), Divisor::make(x.npix, a.pool ? a.M : x.npix + (int64_t)BM), Divisor::make(x.Wo, x.npix)};
-    constexpr bool kPair = (BM + BN) * KST * ST * (int)sizeof(_Float16) <= 64 * 1024;
-    if (first && !kPair) return hipErrorNotSupported;
     // A workgroup that has its unit to itself waits for its next stages: their loads go out in front of the products.  us, between / in
     // front, 640 x 2048 -> 1000, 160 tiles, 11.7 / 11.0, 400 x 2048 -> 1000, 112, 10.8 / 10.0; networks of 14 to 27 images of 96 x 96
     // or 64 x 128 0.5 to 1 % less.  With more tiles other workgroups fill the waits, and in front is the slower order (a network of 56 images of
@@ -1014,14 +1014,14 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
 #define DDF_NET_CONV(POOL_, RES_)                                                                   \
     do {                                                                                            \
         if (alone)                                                                                  \
-            hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, POOL_, RES_, kSmall>), dim3(xcd_grid(tiles)), \
-                               dim3(kThreads), lds, st, a, a, cut);                 \
+            hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WN, WG, false, POOL_, RES_, kSmall>), dim3(xcd_grid(tiles)), \
+                               dim3(2 * WN * kWave), lds, st, a, a, cut);                 \
         else                                                                                        \
-            hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, false, POOL_, RES_>), dim3(xcd_grid(tiles)), \
-                               dim3(kThreads), lds, st, a, a, cut);                 \
+            hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WN, WG, false, POOL_, RES_>), dim3(xcd_grid(tiles)), \
+                               dim3(2 * WN * kWave), lds, st, a, a, cut);                 \
     } while (0)
     if (first)
-        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WG, kPair, false, false>), dim3(xcd_grid(tiles)), dim3(kThreads), lds, st, a,
+        hipLaunchKernelGGL((k_net_conv<BM, BN, KST, ST, WN, WG, true, false, false>), dim3(xcd_grid(tiles)), dim3(2 * WN * kWave), lds, st, a,
                            *first, cut);
     else if (a.pool) DDF_NET_CONV(true, false);
     else if (a.res) DDF_NET_CONV(false, true);
@@ -1030,12 +1030,21 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
     return hipGetLastError();
 }
 
-// The largest tiles that leave somewhat more than a workgroup per compute unit.  Where a unit
-// goes through several, short stages leave room for one workgroup more; where it has one or
-// two, long stages cost fewer barriers (batch 128, us long / short stages: 3136 tiles of
-// 56 x 56 x 64 -> 256 76 / 65, 1568 of 28 x 28 x 512 -> 256 54 / 50, 784 of 14 x 14 x 1024 -> 512
-// 42.2 / 43.4, 392 of 14 x 14 x 1024 -> 256 24.1 / 28.5).  128 x 64 from 448 tiles on: 588 of 14 x 14 x
-// 256 -> 1024 10.0 and 10.9 in tiles of 64, 320 of 7 x 7 x 512 -> 2048 8.9 and 8.3.
+// Tiles of 128 x 128, two workgroups of eight waves per compute unit, wherever they leave more than one workgroup per unit.  Four waves per SIMD
+// cover one another's LDS and barriers better than two or three (four waves per workgroup: 132 to 203 registers), whatever the stages.
+// us, four waves of three short stages / of two long ones / eight of two long ones: 25088 pixels 1024 -> 256 with sums over the pixels 24.1 / 21.9 / 21.7, 256 -> 1024
+// with a residual 27.9 / 27.8 / 27.1, 50176 512 -> 256 25.5 / 22.9 / 22.6, pairs 128 + 256 -> 512 of 12544, 25088 and 50176 pixels 14.5 / 13.8 / 13.4, 25.9 / 24.2 /
+// 22.7, 40.2 / 41.8 / 38.9, 256 + 512 -> 1024 of 25088 64.9 / 62.8 / 60.0.  From 2048 tiles on, where memory
+// counts more, three workgroups in short stages are ahead (pairs of 100352 pixels, 3136 tiles, 78 / - / 82; 1568 tiles of 100352 512 -> 256 with sums 50.8 / 52.9 /
+// 53.5, the one exception seen below that).
+// Up to one workgroup per unit the stages themselves are the time, and a third one in flight is what helps: us, tiles of 64 x 64 / 128 x 128 in two
+// stages / in three, 12544 pixels 1024 -> 256, 196 tiles, 16.9 / 16.1 / 13.2, 6272 2048 -> 512 28.4 / 28.8 / 22.1, pairs 256 + 512 -> 1024 of 3136 14.8 /
+// 13.2 / 11.9, 512 + 1024 -> 2048 of 1568 24.3 / 23.5 / 18.4, 148 tiles of K = 2048 21.7 / 27.5 / 20.9.  Fewer than that fill the chip better in
+// tiles of 64: 100 of K = 2048 16.0 / 26.0 / 19.5, of 1024 9.8 / 13.8 / 11.5; 160 of 512 8.1 / 8.9 / 8.3; 152 of 256 5.7 / 6.1 / 6.2.
+// Where the last round of two per unit would be nearly empty, 128 x 64, three workgroups per unit: us, 128 x 128 / 128 x 64, 294 tiles
+// of 18816 1024 -> 256 20.4 / 20.0, 304 of 2048 19.6 / 18.5, 304 of a pair 27.6 / 26.8; 588 of 75264 512 -> 128 22.0 / 20.5, 592 of 512 -> 2048 19.6 / 18.5, of
+// pairs 27.8 / 26.9 and 49.2 / 46.3; 344 tiles 20.2 / 20.1, 688 50.2 / 51.1.  Of fewer than 128 channels 128 x 64 in short stages from 1024 tiles on, in long
+// ones from 448.
 // In small tiles (ddf_net_small.hip), whose workgroups bring in a quarter of K per wave, what leaves most of the chip idle in tiles
 // of 64: 16 x 16 up to two workgroups per compute unit, 32 x 32 of a K that is worth four waves up to one.  us, tiles of 64 / 16 x 16 / 32 x 32:
 // 64 -> 64 of 1024 pixels, 256 tiles of 16, 2.95 / 2.88, 392 2.96 / 3.18 (a K of 64 is one wave's); 512 -> 128 784 pixels, 392, 4.28 / 3.58,
@@ -1043,21 +1052,22 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
 // pixels 4.35 / 3.60, 400 5.70 / 4.27 / 5.05, 784 6.19 / 6.72 / 5.21, 1568, 392 of 32, 6.67 / 11.3 / 9.14; 2048 -> 512 49 6.09 / 4.26, 400
 // 10.2 / 10.1 / 7.1; 512 -> 2048 with a residual 49 pixels 4.21 / 3.14; pairs 256 + 512 -> 1024 49 7.06 / 3.68, 196 6.53 / 6.83 / 5.34, 512 +
 // 1024 -> 2048 49, 512 tiles, 8.95 / 5.86, 98 9.73 / 9.64 / 7.42; 2048 -> 1000 of 1, 49 and 128 rows 4.51 / 3.71, 6.53 / 5.23, 9.5 / 7.3 / 5.9.
-enum ConvTile { kSmall16, kSmall32, kTile128, kTile128Long, kTile128x64, kTile128x64Long, kTile64 };
-// The same holds for pairs, but from 513 to 768 tiles three workgroups per unit are one round and two a full one and a
-// part.  us, short / long stages: 28 x 28 x 128 + 256 -> 512 344 tiles 14.9 / 13.8, 516 20.1 / 21.9, 588 21.6 / 23.7, 760 24.2 / 25.8, 784 28.1 / 26.8,
-// 980 31.4 / 29.7; 14 x 14 x 256 + 512 -> 1024 592 30.9 / 34.5, 784 41.6 / 38.8; 7 x 7 x 512 + 1024 -> 2048 592 50.8 / 52.1, 784
-// 70.3 / 62.4; 512 tiles of 8 x 8 x 512 + 1024 -> 2048 42.7 / 35.1, of 16 x 16 x 256 + 512 -> 1024 25.4 / 22.6.
+enum ConvTile { kSmall16, kSmall32, kTile128, kTile128Short, kTile128Deep, kTile128x64, kTile128x64Long, kTile64 };
 ConvTile conv_tile(const NetConv &a, const NetConv *first) {
     const bool pair = first;
     const int64_t K = (int64_t)a.K + (pair ? first->K : 0);
     auto count = [&](int bm, int bn) { return cdiv(a.M, bm) * cdiv(a.N, bn); };
-    constexpr int kMany = 1024, kFew = 320;
+    constexpr int kMany = 1024;
     if (a.N % 8 != 0 || count(16, 16) <= (K > 64 ? 512 : 256)) return kSmall16;
     if (K > 256 && count(32, 32) <= 256) return kSmall32;
-    if (a.N >= 128 && (count(128, 128) >= kMany || (pair && count(128, 128) > 512 && count(128, 128) <= 768))) return kTile128;
-    if (a.N >= 128 && count(128, 128) >= kFew) return kTile128Long;
-    if (count(128, 64) >= kMany) return kTile128x64;
+    if (a.N >= 128) {
+        const int64_t tiles = count(128, 128);
+        if (tiles <= 256 && tiles > (K >= 1024 ? 128 : 160)) return kTile128Deep;
+        if (tiles >= 2048) return kTile128Short;
+        if (tiles >= 320 && (tiles <= 512 || tiles > 608)) return kTile128;
+    } else if (count(128, 64) >= kMany) {
+        return kTile128x64;
+    }
     if (count(128, 64) >= 448) return kTile128x64Long;
     return kTile64;
 }
@@ -1067,11 +1077,12 @@ hipError_t conv_tiles(ConvTile tile, const NetConv &a, const NetConv *first, hip
     switch (tile) {
         case kSmall16: return net_conv_small(16, a, first, st);
         case kSmall32: return net_conv_small(32, a, first, st);
-        case kTile128: return launch_conv<128, 128, 32, 3, 3>(a, first, st);
-        case kTile128Long: return launch_conv<128, 128, 64, 2, 2>(a, first, st);
-        case kTile128x64: return launch_conv<128, 64, 32, 3, 4>(a, first, st);
-        case kTile128x64Long: return launch_conv<128, 64, 64, 2, 3>(a, first, st);
-        default: return launch_conv<64, 64, 64, 3, 3>(a, first, st);
+        case kTile128: return launch_conv<128, 128, 64, 2, 4, 2>(a, first, st);
+        case kTile128Short: return launch_conv<128, 128, 32, 3, 2, 3>(a, first, st);
+        case kTile128Deep: return launch_conv<128, 128, 64, 3, 4, 1>(a, first, st);
+        case kTile128x64: return launch_conv<128, 64, 32, 3, 2, 4>(a, first, st);
+        case kTile128x64Long: return launch_conv<128, 64, 64, 2, 2, 3>(a, first, st);
+        default: return launch_conv<64, 64, 64, 3, 2, 3>(a, first, st);
     }
 }
 

@@ -70,6 +70,9 @@ def close(got, want, tol):
     (1, 16, 16, 320, 1024, 1, 1, 0, 1, 1), (1, 1, 257, 320, 1024, 1, 1, 0, 1, 1),    # 256 tiles of 32 x 32, five blocks of K; 288: of 64
     (3, 25, 26, 576, 264, 2, 1, 1, 1, 1), (10, 8, 8, 2048, 520, 1, 0, 1, 0, 0),      # 32 x 32 under stride 2, channels past a tile; no BatchNorm
     (1, 64, 65, 64, 33, 1, 1, 0, 1, 1),        # 780 tiles of 16 x 16, channels no multiple of 8
+    # 128 x 128 in three stages, a workgroup per unit: one, two, three and seventeen stages of K, rows and channels past a tile; 592: 128 x 64
+    (1, 129, 163, 64, 128, 1, 1, 0, 1, 1), (1, 129, 163, 128, 128, 1, 0, 1, 0, 0), (1, 90, 120, 192, 136, 1, 1, 0, 1, 1),
+    (1, 65, 128, 1088, 256, 1, 1, 0, 0, 1), (1, 172, 220, 192, 256, 1, 1, 0, 1, 1),
 ])
 def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     torch.manual_seed(c + o)
@@ -93,8 +96,8 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     (8, 28, 28, 256, 512, 1024, 2, 1),         # tiles of 64
     (16, 28, 28, 128, 256, 264, 1, 1),         # 128 x 64
     (42, 56, 56, 64, 64, 136, 1, 1),           # 128 x 128, many
-    (27, 56, 56, 128, 256, 512, 2, 1),         # 128 x 128, 664 tiles: short stages
-    (7, 45, 44, 64, 64, 264, 1, 1),            # long ones, 327 tiles, rows and channels past the last: a stage of K each
+    (27, 56, 56, 128, 256, 512, 2, 1),         # 128 x 128, 664 tiles
+    (7, 45, 44, 64, 64, 264, 1, 1),            # 327 tiles, rows and channels past the last: a stage of K each
     (64, 16, 16, 64, 192, 2048, 2, 0),         # 512, one stage and three
     (26, 56, 55, 192, 128, 520, 2, 1),         # 800, three and two
     (21, 31, 33, 320, 256, 640, 1, 1),         # 840, five and four
@@ -102,6 +105,8 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     (5, 9, 13, 192, 64, 133, 2, 0),            # channels no multiple of 8
     (3, 25, 26, 128, 320, 264, 2, 1), (2, 17, 16, 64, 256, 520, 1, 0),    # tiles of 32 x 32, a wave with both products; channels past a tile
     (1, 520, 516, 64, 64, 64, 2, 1),           # 67080 pixels: too many for a division by multiplying
+    # 128 x 128 in three stages: one and one of K, two and three, fourteen and three; 596 tiles: 128 x 64
+    (7, 45, 44, 64, 64, 256, 1, 1), (28, 45, 44, 128, 192, 136, 2, 0), (5, 40, 42, 896, 192, 256, 1, 1), (16, 68, 70, 128, 64, 512, 2, 1),
 ])
 def test_conv_pair(n, h, w, c, side, o, stride, relu):
     torch.manual_seed(c + o)
@@ -243,6 +248,7 @@ def test_network_matches_its_modules(build, n, size, classes):
     (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64), (20, 4, 8, 1024, 256),
     (5, 11, 11, 320, 264), (50, 3, 4, 576, 264), (3, 16, 16, 2048, 264), (7, 13, 9, 128, 65),    # 32 x 32, samples ending inside; 16 x 16
     (1, 260, 258, 64, 64),                      # 67080 pixels: too many for a division by multiplying
+    (110, 14, 14, 192, 128), (45, 14, 14, 1024, 264), (7, 41, 43, 64, 136),    # 128 x 128 in three stages
 ])
 def test_conv_pool(n, h, w, c, o):
     """The results of conv, and their sums over the pixels, slot by slot of the tiles."""
