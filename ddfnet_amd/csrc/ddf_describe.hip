@@ -74,6 +74,13 @@ int describe_backward(const Problem &p, int dtype, unsigned need, char *buf, int
         add("%s", sums_name(fneed, rg.csplit, rg.nstrips, norm, p.kk));
         return n;
     }
+    RowsGeom gx; int vxf;
+    if ((need & DDF_NEED_DX) && fneed && dtype != DDF_F64 && tune_int("DDF_TUNE_ROWSF", 1) != 0 &&
+        rows_taprow_backward_plan(p, dtype, &rg, &gx, &vxf, &vx)) {
+        add("k_rows_taprow_backward<VXF=%d,VX=%d,%s>", vxf, vx, layout_name(rg));
+        add("%s", sums_name(fneed, rg.csplit, rg.nstrips, norm, p.kk));
+        return n;
+    }
     if (fuse) {
         add("%s", "k_backward_filters<DX>");
         add("%s", sums_name(fneed, wg.csplit, wg.nstrips, norm, p.kk));

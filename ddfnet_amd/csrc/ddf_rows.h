@@ -567,10 +567,8 @@ constexpr bool by_row() { return K == 5 && R == 1 && VX * sizeof(T) == 16; }
 // TAIL: rows that are no whole number of vectors (Ragged).
 template <typename T, int K, int D, bool MUL, bool BWD, int VX, int R, bool PAD, int NST, int WPE,
           int S = 1, int TAIL = 0>
-__global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const T *__restrict__ x,
-                                                         const T *__restrict__ cf,
-                                                         const T *__restrict__ sf,
-                                                         T *__restrict__ out) {
+__device__ __forceinline__ void rows_walk(const RowsGeom &g, int block, const T *__restrict__ x, const T *__restrict__ cf,
+                                          const T *__restrict__ sf, T *__restrict__ out) {
     using A = typename Acc<T>::type;
     constexpr int KK = K * K, RAD = K / 2, HX = RAD * D, HY = RAD * D;
     constexpr int ROWS = R + 2 * HY;
@@ -589,7 +587,7 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     Work wk;
-    if (!wk.init(g, blockIdx.x, wave) || wk.c_end <= wk.c_begin) return;
+    if (!wk.init(g, block, wave) || wk.c_end <= wk.c_begin) return;
     const int nch = wk.c_end - wk.c_begin;
     const int64_t plane = (int64_t)g.H * g.W;   // result plane
     const uint32_t plane_bytes = (uint32_t)plane * (uint32_t)sizeof(T);
@@ -997,6 +995,15 @@ __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const
         if constexpr (NST > 2) step(std::integral_constant<int, 2>{}, ci + 2);
         if constexpr (NST > 3) step(std::integral_constant<int, 3>{}, ci + 3);
     }
+}
+
+template <typename T, int K, int D, bool MUL, bool BWD, int VX, int R, bool PAD, int NST, int WPE,
+          int S = 1, int TAIL = 0>
+__global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const T *__restrict__ x,
+                                                         const T *__restrict__ cf,
+                                                         const T *__restrict__ sf,
+                                                         T *__restrict__ out) {
+    rows_walk<T, K, D, MUL, BWD, VX, R, PAD, NST, WPE, S, TAIL>(g, blockIdx.x, x, cf, sf, out);
 }
 
 #endif  // __HIPCC__

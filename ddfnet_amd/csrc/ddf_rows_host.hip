@@ -711,6 +711,21 @@ bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r)
     return true;
 }
 
+bool rows_taprow_backward_plan(const Problem &p, int dtype, RowsGeom *g, RowsGeom *gx, int *vxf, int *vx) {
+    int r, r_dx;
+    if (p.k != 5 || p.s != 1 || (p.d != 1 && p.d != 2) || (dtype != DDF_F16 && dtype != DDF_F32) ||
+        tune_int("DDF_TUNE_ROWS", 1) == 0 || !rows_taprow_plan(p, dtype, g, vxf, &r) ||
+        !rows_plan(p, dtype, gx, vx, &r_dx, true))
+        return false;
+    // (ragged rows: the same vectors; else those of the filter gradients may be half as long)
+    if (r != 1 || r_dx != 1 || (*vxf != *vx && (g->tail != 0 || *vxf * 2 != *vx)) || gx->tail != g->tail || gx->shift != g->shift ||
+        rows_shift_in_as_is(*gx) != rows_shift_in_as_is(*g))
+        return false;
+    gx->wpb = rows::kTaprowWaves;
+    gx->xcd_per = (unsigned)cdiv(cdiv(gx->nwork, gx->wpb), rows::kXcd);
+    return true;
+}
+
 bool rows_cover_backward(const Problem &p, int dtype) {
     RowsGeom g; int vx, r;
     return rows_plan(p, dtype, &g, &vx, &r, true) &&

@@ -110,6 +110,12 @@ hipError_t rows_ragged_taprow_launch(const Problem &p, const RowsGeom &g, int vx
                                      const T *x, const T *cf, const T *sf, T *dcf, T *dsf,
                                      typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf,
                                      unsigned need, int x_mod, hipStream_t st);
+// All gradients of 5 x 5 filters (rows_taprow_backward_plan), built in files of their own (ddf_rows_backward5.h).
+template <typename T>
+hipError_t rows_taprow_backward_launch(const Problem &p, const RowsGeom &g, const RowsGeom &gx, int vxf, int vx, const T *go,
+                                       const T *x, const T *cf, const T *sf, T *dx, T *dcf, T *dsf,
+                                       typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf, unsigned need,
+                                       hipStream_t st);
 
 // Forward (backward = false: x -> out) or feature gradient (backward = true:
 // dO -> dX) on the row-register kernels.  hipErrorNotSupported: not covered
@@ -286,7 +292,7 @@ hipError_t launch_taprow_v(const Problem &p, const RowsGeom &g, const T *go, con
 
 // Filter gradients on the row-register kernel, partial sums included; with
 // dx != nullptr the same launch also writes the feature gradient
-// (rows_filters_geometry(..., fused = true) must cover the problem).
+// (rows_taprow_backward_plan or rows_filters_geometry(..., fused = true) must cover the problem).
 // hipErrorNotSupported: not covered (nothing was launched).  `ws` must hold
 // rows_filters_workspace() bytes.
 template <typename T>
@@ -296,10 +302,11 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
     using A = typename Acc<T>::type;
     const int dtype = sizeof(T) == 2 ? DDF_F16 : sizeof(T) == 4 ? DDF_F32 : DDF_F64;
     const bool fused = dx != nullptr;
-    RowsGeom g;
-    int vx, r;
+    RowsGeom g, gx;
+    int vx, r, vxf;
     // (5 x 5: the tap rows go to the waves of a workgroup)
-    const bool taprow = !fused && rows_taprow_plan(p, dtype, &g, &vx, &r);
+    const bool taprow = fused ? x_mod == 0 && rows_taprow_backward_plan(p, dtype, &g, &gx, &vxf, &vx)
+                              : rows_taprow_plan(p, dtype, &g, &vx, &r);
     if (!taprow && !rows_filters_plan(p, dtype, fused, &g, &vx, &r)) return hipErrorNotSupported;
     // (ragged rows take any address of their elements)
     const bool ragged = g.tail > 0 || g.cw > 0;
@@ -319,7 +326,9 @@ hipError_t rows_filters_launch(const Problem &p, const T *go, const T *x, const 
     if ((need & DDF_NEED_DCF) && g.nstrips > 1) ws_cf = reinterpret_cast<A *>(wp);
     hipError_t err = hipErrorNotSupported;
     if constexpr (sizeof(T) != 8) {
-        if (ragged) {
+        if (taprow && fused) {
+            err = rows_taprow_backward_launch<T>(p, g, gx, vxf, vx, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, st);
+        } else if (ragged) {
             err = taprow ? rows_ragged_taprow_launch<T>(p, g, vx, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod, st)
                          : rows_ragged_filters_launch<T>(p, g, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, x_mod, st);
         } else if (p.s == 2) {

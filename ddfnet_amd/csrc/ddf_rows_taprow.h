@@ -36,9 +36,9 @@ constexpr int taprow_lds_bytes(int asz) {
 
 #ifdef __HIPCC__
 
-template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, int NST, int WPE, int TAIL = 0>
-__global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filters(
-    RowsGeom g, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,
+template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, int NST, int TAIL = 0>
+__device__ __forceinline__ void taprow_walk(
+    const RowsGeom &g, int block, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,
     const T *__restrict__ sf, T *__restrict__ dcf, T *__restrict__ dsf,
     typename Acc<T>::type *__restrict__ ws_sf, typename Acc<T>::type *__restrict__ ws_cf,
     unsigned need, int x_mod) {
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int item = Work::item_of(g, blockIdx.x, wave);
+    const int item = Work::item_of(g, block, wave);
     if (item < 0) return;
     const int trow = item % K;   // filter row of this wave
     Work wk;
@@ -316,6 +316,32 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
     }
 }
 
+template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, int NST, int WPE, int TAIL = 0>
+__global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filters(
+    RowsGeom g, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,
+    const T *__restrict__ sf, T *__restrict__ dcf, T *__restrict__ dsf,
+    typename Acc<T>::type *__restrict__ ws_sf, typename Acc<T>::type *__restrict__ ws_cf,
+    unsigned need, int x_mod) {
+    taprow_walk<T, K, D, MUL, VX, R, PAD, NST, TAIL>(g, blockIdx.x, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, x_mod);
+}
+
+// All gradients in one launch: workgroups of filter gradients in front of those of the feature gradient (k_rows' walk,
+// regrouped into as many waves).  The filter gradients are K waves per strip and sample, two and a fraction per SIMD: those with
+// three of them keep their vector ALU busy to the end, the others idle for the last third, and the feature gradient, bound by the vector ALU as
+// well, begins behind that.  Here its workgroups take the places that are left.  Kernel times of a whole step, us, two launches /
+// this: fp32 32 x 128 x 56 x 56 taps two apart 133.9 / 108.3 (the gradients 102 / 77), one apart 128.6 / 105.6, 8 x 256 x 28 x 28 39.0 / 29.2, 3 x 256 x 100
+// x 104 84.4 / 73.1, 5 x 33 x 200 x 190 81.7 / 73.0, 2 x 64 x 40 x 52 25.1 / 19.1; fp16 32 x 128 x 56 x 56 131.8 / 108.7, 'add' 107.8 / 91.0, 8 x 64 x 200
+// x 200 184.9 / 179.6, 21 x 104 x 57 x 61 114.8 / 106.0, 1 x 512 x 50 x 75 51.1 / 41.3.  No size was found where two are faster.
+template <typename T, int D, bool MUL, int VXF, int VX, bool PAD, int NST, int WPE, int TAIL>
+__global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_backward(
+    RowsGeom g, RowsGeom gx, int blocks, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,
+    const T *__restrict__ sf, T *__restrict__ dx, T *__restrict__ dcf, T *__restrict__ dsf,
+    typename Acc<T>::type *__restrict__ ws_sf, typename Acc<T>::type *__restrict__ ws_cf, unsigned need) {
+    const int block = blockIdx.x;
+    if (block < blocks) taprow_walk<T, 5, D, MUL, VXF, 1, PAD, NST, TAIL>(g, block, go, x, cf, sf, dcf, dsf, ws_sf, ws_cf, need, 0);
+    else rows_walk<T, 5, D, MUL, true, VX, 1, PAD, 2, WPE, 1, TAIL>(gx, block - blocks, go, cf, sf, dx);
+}
+
 #endif  // __HIPCC__
 
 }  // namespace rows
@@ -326,5 +352,8 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
 bool rows_taprow_geometry(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r);
 // What runs: that geometry or the one for ragged rows (see rows_plan).
 bool rows_taprow_plan(const Problem &p, int dtype, RowsGeom *g, int *vx, int *r);
+// Both of a 5 x 5 backward pass in one launch (k_rows_taprow_backward): the filter gradients' geometry and the
+// feature gradient's, whose waves come in workgroups of as many here.
+bool rows_taprow_backward_plan(const Problem &p, int dtype, RowsGeom *g, RowsGeom *gx, int *vxf, int *vx);
 
 }  // namespace ddf

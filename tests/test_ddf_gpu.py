@@ -449,6 +449,33 @@ def test_fp16_five_by_five_of_few_and_many_waves(few, many, shape, d, combine):
     check_against_oracle(x[:1], cf[:1], sf[:1], go[:1], 5, d, 1, combine)
 
 
+# rows of whole vectors (as long for both halves, half as long for the filter gradients), ragged, cut into segments or a run; a channel walk
+# whole and split, one strip and several; a workgroup of the feature gradient with fewer than four waves
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16], ids=str)
+@pytest.mark.parametrize('shape,d', [
+    ((1, 3, 9, 8), 1), ((5, 33, 20, 12), 1), ((3, 20, 14, 28), 1), ((2, 40, 24, 64), 2), ((32, 24, 56, 56), 1), ((32, 24, 56, 56), 2), ((64, 16, 56, 64), 1),
+    ((2, 19, 23, 27), 1), ((3, 40, 31, 30), 2), ((40, 16, 33, 45), 1), ((1, 72, 40, 229), 2), ((4, 24, 44, 39), 1), ((1, 9, 70, 264), 1), ((1, 16, 90, 68), 2),
+    ((8, 8, 200, 204), 1), ((8, 8, 200, 201), 2),
+], ids=_ids)
+def test_five_by_five_gradients_in_one_launch(shape, d, dtype, combine):
+    """All gradients at once are the bits that each half leaves alone.  (The channel filter's in fp16 'add' are fp32 sums of H * W products of
+    two fp16 values; the compiler adds two of them at a time where it likes: an error of 2^-24 of the sum of magnitudes per addition, and a
+    rounding to fp16.)"""
+    x, cf, sf, go = random_case(*shape, 5, 1, dtype, seed=shape[1])
+    dev = to_dev(x, cf, sf, go)
+    _, dx, dcf, dsf = run_ddf(*dev, 5, d, 1, combine)
+    assert torch.equal(dx, run_ddf(*dev, 5, d, 1, combine, need=(True, False, False))[1])
+    _, _, cf_alone, sf_alone = run_ddf(*dev, 5, d, 1, combine, need=(False, True, True))
+    assert torch.equal(dsf, sf_alone)
+    if dtype == torch.float16 and combine == 'add':
+        most = (x.float().abs().max() * go.float().abs().max()).item()
+        torch.testing.assert_close(dcf, cf_alone, rtol=2. ** -10, atol=most * shape[2] * shape[3] * 2. ** -24)
+    else:
+        assert torch.equal(dcf, cf_alone)
+    check_against_oracle(x[:1], cf[:1], sf[:1], go[:1], 5, d, 1, combine)
+
+
 def test_runs_on_the_current_stream():
     from ddfnet_amd import ddf
     x, cf, sf, _ = random_case(4, 16, 14, 14, 3, 1, torch.float32, seed=12)
