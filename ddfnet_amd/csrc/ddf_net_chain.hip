@@ -343,21 +343,56 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
         // w's rows are there (the residual may be on its way); everybody is done with w2's
         arrive<K2 ? 0 : RV>();
         sw2.load(lds0 + L::w2 * 2, wave, w2 + j * kChunk, N);
-        half4_t side[K2 ? TA : 1][4];
         float16_t sum[TA];
-        if constexpr (K2 > 0) {
-#pragma unroll
-            for (int t = 0; t < TA; ++t) clear(sum[t]);
-            product(chain_smem + L::wd, std::integral_constant<int, K2 ? K2 : 16>{}, dv, sum);
+        // sums rounded to fp16, to the wave's tile
+        auto put = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int t = 0; t < TA; ++t)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const float4_t sc = *reinterpret_cast<const float4_t *>(side_scale + j * kChunk + channel(t, q));
-                    const float4_t sh = *reinterpret_cast<const float4_t *>(side_shift + j * kChunk + channel(t, q));
+                    half4_t v;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) side[t][q][e] = (_Float16)fmaf((float)(_Float16)sum[t][4 * q + e], sc[e], sh[e]);
+                    for (int e = 0; e < 4; ++e) v[e] = (_Float16)sum[t][4 * q + e];
+                    *reinterpret_cast<half4_t *>(tile + l32 * kTilePitch + channel(t, q)) = v;
                 }
+            asm volatile("" ::: "memory");    // (a wave's LDS operations keep their order)
+        };
+        // scale and shift of a lane's eight channels of the chunk, and its vectors
+        auto get = [&](const float *scales, const float *shifts, float (&sc)[8], float (&sh)[8], half8_t (&v)[RV]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4_t s = *reinterpret_cast<const float4_t *>(scales + j * kChunk + c8 * 8 + h * 4);
+                const float4_t o = *reinterpret_cast<const float4_t *>(shifts + j * kChunk + c8 * 8 + h * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sc[4 * h + e] = s[e];
+                    sh[4 * h + e] = o[e];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RV; ++i)
+                v[i] = *reinterpret_cast<const half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8);
+        };
+        float sc[8], sh[8];
+        half8_t v[RV];
+        // A projection's results take the residual's place.  Worked out where the product leaves them, four channels of a pixel at a
+        // time, the scales and shifts of both products were 128 KB a chunk of the 290 that LDS was read for; here they are 32.
+        // us, 56 x 56 x 64 + 64 -> 256 -> 64 of 128, 64, 32 and 16 images with all that is in front: 117.4 / 115.0, 61.9 / 60.6, 39.2 / 38.4, 24.0 /
+        // 23.4.  (In k_net_conv's pairs, whose tiles are shared and take two barriers more: 128 x 128 in short stages 79.3 / 76.9, in long ones
+        // no difference, tiles of 64 14.2 / 15.2.)
+        if constexpr (K2 > 0) {
+#pragma unroll
+            for (int t = 0; t < TA; ++t) clear(sum[t]);
+            product(chain_smem + L::wd, std::integral_constant<int, K2 ? K2 : 16>{}, dv, sum);
+            put();
+            get(side_scale, side_shift, sc, sh, v);
+#pragma unroll
+            for (int i = 0; i < RV; ++i) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[i][e] = (_Float16)fmaf((float)v[i][e], sc[e], sh[e]);    // (rounded once, as in a pair)
+                rv[i] = __builtin_bit_cast(rows_u4, v[i]);
+            }
+            asm volatile("" ::: "memory");
         }
 #pragma unroll
         for (int t = 0; t < TA; ++t) clear(sum[t]);
@@ -372,61 +407,20 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
                 }
         }
         product(chain_smem + L::w, std::integral_constant<int, K>{}, xv, sum);
-        // to the tile: sums rounded to fp16, with a side product the results
-#pragma unroll
-        for (int t = 0; t < TA; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                half4_t v;
-                if constexpr (K2 > 0) {
-                    const float4_t sc = *reinterpret_cast<const float4_t *>(scale + j * kChunk + channel(t, q));
-                    const float4_t sh = *reinterpret_cast<const float4_t *>(shift + j * kChunk + channel(t, q));
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float f = fmaf((float)(_Float16)sum[t][4 * q + e], sc[e], sh[e]);
-                        f = fmaf((float)side[t][q][e], one, f);
-                        asm volatile("" : "+v"(f));
-                        v[e] = (_Float16)f;
-                    }
-                    v = __builtin_elementwise_maximum(v, half4_t{0, 0, 0, 0});
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (_Float16)sum[t][4 * q + e];
-                }
-                *reinterpret_cast<half4_t *>(tile + l32 * kTilePitch + channel(t, q)) = v;
-            }
-        asm volatile("" ::: "memory");    // (a wave's LDS operations keep their order)
-        float sc[8], sh[8];
-        if constexpr (K2 == 0) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const float4_t s = *reinterpret_cast<const float4_t *>(scale + j * kChunk + c8 * 8 + h * 4);
-                const float4_t o = *reinterpret_cast<const float4_t *>(shift + j * kChunk + c8 * 8 + h * 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    sc[4 * h + e] = s[e];
-                    sh[4 * h + e] = o[e];
-                }
-            }
-        }
-        half8_t v[RV];
-#pragma unroll
-        for (int i = 0; i < RV; ++i)
-            v[i] = *reinterpret_cast<const half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8);
+        put();
+        get(scale, shift, sc, sh, v);
 #pragma unroll
         for (int i = 0; i < RV; ++i) {
-            if constexpr (K2 == 0) {
-                const half8_t r = __builtin_bit_cast(half8_t, rv[i]);
+            const half8_t r = __builtin_bit_cast(half8_t, rv[i]);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    float f = fmaf((float)v[i][e], sc[e], sh[e]);
-                    f = fmaf((float)r[e], one, f);
-                    asm volatile("" : "+v"(f));    // (rounded to fp32 first in every instance)
-                    v[i][e] = (_Float16)f;
-                }
-                v[i] = __builtin_elementwise_maximum(v[i], half8_t{0, 0, 0, 0, 0, 0, 0, 0});
-                *reinterpret_cast<half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8) = v[i];
+            for (int e = 0; e < 8; ++e) {
+                float f = fmaf((float)v[i][e], sc[e], sh[e]);
+                f = fmaf((float)r[e], one, f);
+                asm volatile("" : "+v"(f));    // (rounded to fp32 first in every instance)
+                v[i][e] = (_Float16)f;
             }
+            v[i] = __builtin_elementwise_maximum(v[i], half8_t{0, 0, 0, 0, 0, 0, 0, 0});
+            *reinterpret_cast<half8_t *>(tile + (px0 - wave * 32 + i * 8) * kTilePitch + c8 * 8) = v[i];
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(rows_u4, v[i]), orr, vector_at(i), j * (kChunk * 2), 0);
         }
         // w2's rows are there; everybody is done with w's
