@@ -39,13 +39,27 @@ struct PackDims {
 };
 
 // ---- second convolution of the channel branch --------------------------------
-// A workgroup takes kFc2Channels channels (36 rows of W2) and 64 hidden values, a lane one
+// A workgroup takes CW channels (9 * CW rows of W2) and 64 hidden values, a lane one
 // hidden value; samples come in chunks of 64 through LDS.  dW2: every wave owns one channel's
-// rows and reads their dZ2 as LDS broadcasts; dh: every wave owns every fourth sample, with
-// the lane's column of the 36 rows of W2 in registers.  (Eight channels and chunks of 32
-// samples: 22.8 us at 64 x 128 where this takes 13.)
-constexpr int kFc2Channels = kWaves, kFc2Rows = kFc2Channels * KK, kFc2Samples = kThreads / kFc2Channels;
+// rows for a CW-th quarter of the samples and reads their dZ2 as LDS broadcasts; dh: every wave owns
+// every fourth sample, with the lane's column of the rows of W2 in registers.  LDS reads bound it (a
+// wave's 36 multiply-adds of a sample are nine reads of 16 bytes) and, behind them, the chain from the
+// first load over the normalisation to the last sum: everything is asked for before anything is waited for
+// (W2's rows, the gains and the hidden values under conditions, one after another, cost 2 us; W2's rows first, their
+// addresses would not fit the registers of four waves per SIMD behind the others).
+constexpr int kFc2Samples = 64, kFc2MaxChannels = kWaves, kUnits = 256;    // (compute units)
 constexpr int kFc2Pitch = 12;    // a channel's nine values, 16-byte rows
+
+// Channels per workgroup: few as long as the workgroups do not outnumber the compute units.  Every channel block
+// leaves a partial dh of all samples, so no more of them than fill the chip.  The launch with four channels
+// each and this, us (fp16, medians under the profiler): 64 x 128 x 28 x 28 18.2 / 8.8, 64 x 64 x 56 x 56 19.4 / 8.8, 64 x 256 x 14 x 14 17.6 / 8.5, 256 x 128 x
+// 14 x 14 55.4 / 19.6, 1 x 512 x 14 x 14 6.4 / 5.8, fp32 32 x 256 x 28 x 28 15.0 / 10.4; four of them with the loads asked for at once: 64 x 512 x 7 x 7
+// 18.9 / 13.6, 3 x 2048 x 7 x 7 31.8 / 23.9.  (8 x 64 x 200 x 300, whose time is the other half's: 13.0 / 13.7.)
+inline int fc2_channels(int64_t C, int64_t mid) {
+    int cw = 1;
+    while (cw < kFc2MaxChannels && cdiv(C, cw) * cdiv(mid, kWave) > kUnits) cw *= 2;
+    return cw;
+}
 
 template <typename T>
 struct Fc2Args {
@@ -57,114 +71,153 @@ struct Fc2Args {
     int mchunks;
 };
 
+template <int CW>
 struct Fc2Smem {
-    float dz[kFc2Samples][kFc2Channels][kFc2Pitch];
-    float dg[kFc2Samples][kFc2Rows];
-    float h[kFc2Samples][kWave];
+    static constexpr int rows = CW * KK, parts = kWaves / CW;
+    float dz[kFc2Samples][CW][kFc2Pitch];
+    float dg[kFc2Samples][rows];
+    union {
+        float h[kFc2Samples][kWave];
+        struct { float dw[kWaves][KK][kWave], col[parts][2 * rows]; } sums;    // at the end
+    };
 };
 
-template <typename T>
-__device__ __forceinline__ void fc2_block(const PackDims &d, const Fc2Args<T> &a, int block, Fc2Smem &sm) {
+template <typename T, int CW>
+__device__ __forceinline__ void fc2_block(const PackDims &d, const Fc2Args<T> &a, int block, Fc2Smem<CW> &sm) {
+    constexpr int ROWS = Fc2Smem<CW>::rows, PARTS = Fc2Smem<CW>::parts, PASSES = kFc2Samples / kWaves;
+    constexpr int HELD = CW < 4 ? PASSES : 4;    // (four channels' weights leave few registers)
+    static_assert(2 * ROWS * PARTS <= kThreads && CW * kFc2Samples <= kThreads);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int blk = block / a.mchunks, m0 = (block - blk * a.mchunks) * kWave;
-    const int cb = blk * kFc2Channels;
-    const int rows = min(kFc2Rows, (d.C - cb) * KK);
+    const int cb = blk * CW;
+    const int rows = min(ROWS, (d.C - cb) * KK);
     const int m = m0 + lane;
     const bool mok = m < d.mid;
     const int mc = mok ? m : d.mid - 1;
-    float w2[kFc2Rows];
-#pragma unroll
-    for (int r = 0; r < kFc2Rows; ++r) w2[r] = ld(a.w2 + ((int64_t)cb * KK + min(r, rows - 1)) * d.mid + mc);
     float acc[KK];
 #pragma unroll
     for (int t = 0; t < KK; ++t) acc[t] = 0.f;
     float col_sum = 0.f;
-    const int item_n = threadIdx.x / kFc2Channels, item_c = threadIdx.x % kFc2Channels;
+    const int item_n = threadIdx.x / CW, item_c = threadIdx.x % CW, wc = wave % CW, part = wave / CW;
+    const int col_part = threadIdx.x / (2 * ROWS), col_at = threadIdx.x % (2 * ROWS);
+    const bool col_mine = m0 == 0 && col_part < PARTS;
+    float w2[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) w2[r] = ld(a.w2 + ((int64_t)cb * KK + min(r, rows - 1)) * d.mid + mc);
     for (int n0 = 0; n0 < d.N; n0 += kFc2Samples) {
         const int cnt = min(kFc2Samples, d.N - n0);
-        if (n0 > 0) __syncthreads();
-        {
+        // (addresses clamped instead of loads under conditions, which would wait for one another)
+        const int n = min(n0 + item_n, d.N - 1), c = min(cb + item_c, d.C - 1);
+        const int64_t at = ((int64_t)n * d.C + c) * KK;
+        float z[KK], dc[KK], gain[KK], held[HELD];
+        auto hold = [&](int first) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < HELD; ++k) held[k] = a.hidden[(int64_t)(n0 + min(wave + (first + k) * kWaves, cnt - 1)) * d.mid + mc];
+        };
+#pragma unroll
+        for (int t = 0; t < KK; ++t) {
+            z[t] = a.taps[at + t];
+            dc[t] = ld(a.dcf + at + t);
+        }
+#pragma unroll
+        for (int t = 0; t < KK; ++t) gain[t] = a.gain;
+        if (a.gain_vec) {
+#pragma unroll
+            for (int t = 0; t < KK; ++t) gain[t] = ld(a.gain_vec + c * KK + t);
+        }
+        if (HELD == PASSES) hold(0);
+        if (n0 > 0) __syncthreads();    // (the chunk before has been read)
+        if (item_n < kFc2Samples) {
             // one filter per thread: dCF through the normalisation (see ddf_filter_norm.hip)
-            float dz[KK], dg[KK];
-#pragma unroll
-            for (int t = 0; t < KK; ++t) dz[t] = dg[t] = 0.f;
-            const int n = n0 + item_n, c = cb + item_c;
-            if (n < d.N && c < d.C) {
-                const int64_t at = ((int64_t)n * d.C + c) * KK;
-                float z[KK], g[KK], dc[KK], sum = 0.f;
-#pragma unroll
-                for (int t = 0; t < KK; ++t) {
-                    z[t] = a.taps[at + t];
-                    dc[t] = ld(a.dcf + at + t);
-                    g[t] = dc[t] * (a.gain_vec ? ld(a.gain_vec + c * KK + t) : a.gain);
-                    sum += z[t];
-                }
-                const float mean = sum / (float)KK;
-                float sq = 0.f, s1 = 0.f, s2 = 0.f;
-#pragma unroll
-                for (int t = 0; t < KK; ++t) {
-                    z[t] -= mean;
-                    sq += z[t] * z[t];
-                    s1 += g[t];
-                    s2 += g[t] * z[t];
-                }
-                const float sd = sqrtf(sq / (float)(KK - 1));
-                const float inv = 1.f / (sd + 1e-10f);
-                const float m1 = s1 / (float)KK, k2 = inv * inv * s2 / (sd * (float)(KK - 1));
-#pragma unroll
-                for (int t = 0; t < KK; ++t) {
-                    dz[t] = inv * (g[t] - m1) - z[t] * k2;
-                    dg[t] = dc[t] * z[t] * inv;
-                }
-            }
+            const bool there = n0 + item_n < d.N && cb + item_c < d.C;
+            float g[KK], sum = 0.f;
 #pragma unroll
             for (int t = 0; t < KK; ++t) {
-                sm.dz[item_n][item_c][t] = dz[t];
-                sm.dg[item_n][item_c * KK + t] = dg[t];
+                g[t] = dc[t] * gain[t];
+                sum += z[t];
+            }
+            const float mean = sum / (float)KK;
+            float sq = 0.f, s1 = 0.f, s2 = 0.f;
+#pragma unroll
+            for (int t = 0; t < KK; ++t) {
+                z[t] -= mean;
+                sq += z[t] * z[t];
+                s1 += g[t];
+                s2 += g[t] * z[t];
+            }
+            const float sd = sqrtf(sq / (float)(KK - 1));
+            const float inv = 1.f / (sd + 1e-10f);
+            const float m1 = s1 / (float)KK, k2 = inv * inv * s2 / (sd * (float)(KK - 1));
+#pragma unroll
+            for (int t = 0; t < KK; ++t) {
+                sm.dz[item_n][item_c][t] = there ? inv * (g[t] - m1) - z[t] * k2 : 0.f;
+                sm.dg[item_n][item_c * KK + t] = there ? dc[t] * z[t] * inv : 0.f;
             }
         }
-        for (int e = threadIdx.x; e < kFc2Samples * kWave; e += kThreads) {
-            const int i = e / kWave, mm = e % kWave;
-            sm.h[i][mm] = (i < cnt && m0 + mm < d.mid) ? a.hidden[(int64_t)(n0 + i) * d.mid + m0 + mm] : 0.f;
+        for (int first = 0; first < PASSES; first += HELD) {
+            if (HELD < PASSES && first * kWaves >= cnt) break;
+            if (HELD < PASSES) hold(first);
+#pragma unroll
+            for (int k = 0; k < HELD; ++k) sm.h[wave + (first + k) * kWaves][lane] = held[k];
         }
         __syncthreads();
 #pragma unroll 4
-        for (int i = 0; i < cnt; ++i) {
+        for (int i = part; i < cnt; i += PARTS) {
             const float hv = sm.h[i][lane];
 #pragma unroll
-            for (int t = 0; t < KK; ++t) acc[t] = fmaf(sm.dz[i][wave][t], hv, acc[t]);
+            for (int t = 0; t < KK; ++t) acc[t] = fmaf(sm.dz[i][wc][t], hv, acc[t]);
         }
 #pragma unroll 2
         for (int i = wave; i < cnt; i += kWaves) {
-            float p[kFc2Channels];
+            float p[CW];
 #pragma unroll
-            for (int c = 0; c < kFc2Channels; ++c) {
+            for (int c = 0; c < CW; ++c) {
                 p[c] = 0.f;
 #pragma unroll
                 for (int t = 0; t < KK; ++t) p[c] = fmaf(sm.dz[i][c][t], w2[c * KK + t], p[c]);
             }
-            if (mok) a.dh_part[((int64_t)blk * d.N + n0 + i) * d.mid + m] = (p[0] + p[1]) + (p[2] + p[3]);
+            float sum = p[0];
+            if constexpr (CW == 2) sum = p[0] + p[1];
+            if constexpr (CW == 4) sum = (p[0] + p[1]) + (p[2] + p[3]);
+            if (mok) a.dh_part[((int64_t)blk * d.N + n0 + i) * d.mid + m] = sum;
         }
-        if (m0 == 0 && threadIdx.x < 2 * kFc2Rows) {
-            const bool gain = threadIdx.x >= kFc2Rows;
-            const int col = gain ? threadIdx.x - kFc2Rows : threadIdx.x;
-            const float *src = gain ? &sm.dg[0][col] : &sm.dz[0][col / KK][col % KK];
-            const int pitch = gain ? kFc2Rows : kFc2Channels * kFc2Pitch;
+        if (col_mine) {
+            const bool gains = col_at >= ROWS;
+            const int col = gains ? col_at - ROWS : col_at;
+            const float *src = gains ? &sm.dg[0][col] : &sm.dz[0][col / KK][col % KK];
+            const int pitch = gains ? ROWS : CW * kFc2Pitch;
 #pragma unroll 8
-            for (int i = 0; i < cnt; ++i) col_sum += src[i * pitch];
+            for (int i = col_part; i < cnt; i += PARTS) col_sum += src[i * pitch];
         }
     }
-    if (mok && cb + wave < d.C) {
+    if constexpr (PARTS > 1) {
+        // (the sums of a channel's parts, in order)
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < KK; ++t) sm.sums.dw[wave][t][lane] = acc[t];
+        if (col_mine) sm.sums.col[col_part][col_at] = col_sum;
+        __syncthreads();
+        for (int r = wave; r < rows; r += kWaves) {
+            const int c = r / KK, t = r - c * KK;
+            float total = sm.sums.dw[c][t][lane];
+#pragma unroll
+            for (int k = 1; k < PARTS; ++k) total += sm.sums.dw[k * CW + c][t][lane];
+            if (mok) st(a.dw2 + ((int64_t)cb * KK + r) * d.mid + m, total);
+        }
+        if (col_mine && col_part == 0) {
+#pragma unroll
+            for (int k = 1; k < PARTS; ++k) col_sum += sm.sums.col[k][col_at];
+        }
+    } else if (mok && cb + wave < d.C) {
 #pragma unroll
         for (int t = 0; t < KK; ++t) st(a.dw2 + ((int64_t)(cb + wave) * KK + t) * d.mid + m, acc[t]);
     }
-    if (m0 == 0) {
-        const int r = threadIdx.x;
-        if (r < rows) {
-            if (a.db2) st(a.db2 + cb * KK + r, col_sum);
-        } else if (r >= kFc2Rows && r < kFc2Rows + rows) {
-            if (a.dgain) st(a.dgain + cb * KK + r - kFc2Rows, col_sum);
+    if (col_mine && col_part == 0) {
+        if (col_at < rows) {
+            if (a.db2) st(a.db2 + cb * KK + col_at, col_sum);
+        } else if (col_at >= ROWS && col_at < ROWS + rows) {
+            if (a.dgain) st(a.dgain + cb * KK + col_at - ROWS, col_sum);
         }
     }
 }
@@ -276,11 +329,11 @@ __device__ __forceinline__ void ws_item(const PackDims &d, const WsArgs<T> &a, i
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_pack_fc2(PackDims d, Fc2Args<T> f, WsArgs<T> w, int fc2_blocks) {
-    __shared__ __align__(16) Fc2Smem sm;
+template <typename T, int CW>
+__global__ __launch_bounds__(kThreads, 4) void k_pack_fc2(PackDims d, Fc2Args<T> f, WsArgs<T> w, int fc2_blocks) {
+    __shared__ __align__(16) Fc2Smem<CW> sm;
     if ((int)blockIdx.x < fc2_blocks) {
-        fc2_block<T>(d, f, blockIdx.x, sm);
+        fc2_block<T, CW>(d, f, blockIdx.x, sm);
         return;
     }
     const int item = ((int)blockIdx.x - fc2_blocks) * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -290,7 +343,9 @@ __global__ __launch_bounds__(kThreads) void k_pack_fc2(PackDims d, Fc2Args<T> f,
 }
 
 // ---- hidden layer's gradient, and the sums of the partial dWs ------------------
-constexpr int kSumGroups = 4, kSumCols = kThreads / kSumGroups;
+// (sixteen threads share an output's parts, eight of them on their way at a time; four threads, us: 8 x 64 x 200 x 300 fp16
+// 8.4 / 4.6, 64 x 64 x 56 x 56 6.6 / 4.8, 3 x 2048 x 7 x 7 7.9 / 5.0)
+constexpr int kSumGroups = 16, kSumCols = kThreads / kSumGroups, kSumAhead = 8;
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_pack_hidden(PackDims d, const float *__restrict__ dh_part,
@@ -307,8 +362,13 @@ __global__ __launch_bounds__(kThreads) void k_pack_hidden(PackDims d, const floa
     const int np = hid ? parts : ws_parts;
     float a = 0.f;
     if (i < count) {
-#pragma unroll 8
-        for (int q = grp; q < np; q += kSumGroups) a += src[q * count + i];
+        for (int q0 = grp; q0 < np; q0 += kSumGroups * kSumAhead) {
+            float v[kSumAhead];
+#pragma unroll
+            for (int k = 0; k < kSumAhead; ++k) v[k] = src[min(q0 + k * kSumGroups, np - 1) * count + i];
+#pragma unroll
+            for (int k = 0; k < kSumAhead; ++k) a += q0 + k * kSumGroups < np ? v[k] : 0.f;
+        }
     }
     red[grp][col] = a;
     __syncthreads();
@@ -513,7 +573,7 @@ size_t pack_backward_workspace(int64_t N, int64_t C, int64_t mid, int64_t H, int
     int splits, split_pix;
     const int64_t npix = (H / stride) * (W / stride);
     ws_split(N, C, npix, dtype == DDF_F16 ? 32 : 16, &splits, &split_pix);
-    return floats256(cdiv(C, kFc2Channels) * N * mid) + floats256(N * mid) + floats256(N * C) +
+    return floats256(cdiv(C, fc2_channels(C, mid)) * N * mid) + floats256(N * mid) + floats256(N * C) +
            floats256(N * splits * head * KK * (C + 1));
 }
 
@@ -525,7 +585,7 @@ hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t
     constexpr int STEP = 4 * Quad<T>::n;
     int splits, split_pix;
     ws_split(N, C, npix, STEP, &splits, &split_pix);
-    const int cblocks = (int)cdiv(C, kFc2Channels);
+    const int cw2 = fc2_channels(C, mid), cblocks = (int)cdiv(C, cw2);
     unsigned char *q = static_cast<unsigned char *>(ws);
     float *dh_part = reinterpret_cast<float *>(q); q += floats256((int64_t)cblocks * N * mid);
     float *dz1 = reinterpret_cast<float *>(q); q += floats256(N * mid);
@@ -537,8 +597,10 @@ hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t
     WsArgs<T> w{b.x, b.draw, ws_part, (int)cdiv(C, kRowTile), splits, split_pix, 0};
     w.nwork = (int)(N * splits * w.ctiles);
     const int fc2_blocks = cblocks * f.mchunks;
-    hipLaunchKernelGGL((k_pack_fc2<T>), dim3((unsigned)(fc2_blocks + cdiv(w.nwork, kWaves))), dim3(kThreads), 0, st,
-                       d, f, w, fc2_blocks);
+    const dim3 grid2((unsigned)(fc2_blocks + cdiv(w.nwork, kWaves)));
+    if (cw2 == 1) hipLaunchKernelGGL((k_pack_fc2<T, 1>), grid2, dim3(kThreads), 0, st, d, f, w, fc2_blocks);
+    else if (cw2 == 2) hipLaunchKernelGGL((k_pack_fc2<T, 2>), grid2, dim3(kThreads), 0, st, d, f, w, fc2_blocks);
+    else hipLaunchKernelGGL((k_pack_fc2<T, 4>), grid2, dim3(kThreads), 0, st, d, f, w, fc2_blocks);
     const int hid_blocks = (int)cdiv(N * mid, kSumCols);
     hipLaunchKernelGGL((k_pack_hidden<T>), dim3((unsigned)(hid_blocks + cdiv((int64_t)head * KK * (C + 1), kSumCols))),
                        dim3(kThreads), 0, st, d, dh_part, b.hidden, dz1, cblocks, hid_blocks, ws_part,

@@ -19,6 +19,9 @@ CASES = [
     (5, 32, 18, 10, 2, 1, 'mul'),      # stride 2
     (2, 48, 20, 28, 2, 2, 'mul'),
     (1, 64, 61, 50, 1, 1, 'mul'),      # several pixel ranges per sample
+    (70, 24, 3, 5, 1, 1, 'mul'),       # samples past a chunk of 64 where a workgroup has one channel,
+    (65, 300, 4, 2, 1, 1, 'add'),      # two,
+    (131, 344, 2, 3, 1, 1, 'mul'),     # and four
 ]
 
 
