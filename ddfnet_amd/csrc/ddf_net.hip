@@ -456,24 +456,28 @@ __global__ __launch_bounds__(2 * WN * kWave, WG * WN / 2) void k_net_conv(NetCon
 // and those (the fourth channel, zeros, and that column, cleared after the read lest an infinity
 // in it make a NaN, meet zero weights), so that a tile starts at an even column and comes in as
 // pairs of columns.  The weights stay in registers over the tiles a workgroup walks.
-// Convolution results never leave LDS (205 MB at batch 128).  The vector ALU was busy half of the
-// time: pixel by pixel with a division each, and ReLU and the image's edge value by value, 128
-// images of 224 x 224 took 90.8 us, now 72.9 (26 at the matrix cores' rate, 17 for the bytes).
+// Convolution results never leave LDS (205 MB at batch 128).  The vector ALU (46 % of the clocks) and the matrix cores (44 %) bound
+// it, with two waves per SIMD that wait for one another's barriers: a round's products go out between the instructions that
+// finish the round before, results outside the image are left out by the pooling's addresses instead of masked one by
+// one, and the pooling's lanes are laid over LDS without conflicts (8.5 -> 4.9 M clocks of them).  us, 128, 32, 8 and one image of
+// 224 x 224 75.0 / 66.7, 27.6 / 25.8, 14.3 / 13.2, 10.3 / 9.0, 64 of 192 x 192 34.3 / 31.0 (128 of 224 x 224: 26 at the matrix cores' rate, 17
+// for the bytes).  The first tile and the norm's parameters asked for in front of the weights: no faster.
 constexpr int kPoolTile = 8, kConvTile = 2 * kPoolTile + 1, kImgRows = 2 * (kConvTile - 1) + 7, kImgCols = kImgRows + 1;
 constexpr int kConvPitch = 64 + 8, kStemOut = 64;
-constexpr int kStemPixels = kConvTile * kConvTile, kStemTiles = (kStemPixels + 15) / 16;
+constexpr int kStemPixels = kConvTile * kConvTile, kStemTiles = (kStemPixels + 15) / 16,
+              kStemRounds = (kStemTiles + kThreads / kWave - 1) / (kThreads / kWave);
 
 __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__restrict__ img,
                                                           const _Float16 *__restrict__ w, NetNorm norm,
                                                           _Float16 *__restrict__ out, int N, int H, int W, int tiles_x,
                                                           int tiles_y) {
     __shared__ __align__(16) _Float16 tile[kImgRows * kImgCols * 4];
-    __shared__ __align__(16) _Float16 conv[kStemTiles * 16 * kConvPitch];
-    static_assert(kStemOut * 7 * 32 <= kStemTiles * 16 * kConvPitch, "the weights pass through the results' space");
+    __shared__ __align__(16) _Float16 conv[kStemPixels * kConvPitch];
+    static_assert(kStemOut * 7 * 32 <= kStemPixels * kConvPitch, "the weights pass through the results' space");
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int row = lane & 15, quad = lane >> 4;
-    const int Hc = H / 2, Wc = W / 2, Hp = Hc / 2, Wp = Wc / 2;
+    const int Hp = H / 4, Wp = W / 4;
     const uint32_t first_column = quad == 0 ? 0u : ~0u;   // (columns 2 * quad and 2 * quad + 1 of eight)
     // weights to LDS as [output][filter row][column * 4 + channel], then to registers
     {
@@ -534,10 +538,15 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
                 pix[k][ch] = __builtin_amdgcn_raw_buffer_load_b32(in, (int)off, (int)(ch * plane_b), 0);
         }
     };
+    // Pooled pixel of a row and eight channels of a lane, a wave a row.  A pixel's neighbour is 18 places of 16 bytes further on, so
+    // pixels x and x + 4 fill the sixteen places that an LDS read serves at once (lanes 0-3, 12-15, 20-27 and 4-11, 16-19,
+    // 28-31 of 32).
+    const int part = (lane >> 2) & 7;
+    const int pool_x = ((part ^ (part >> 1) ^ (part >> 2)) & 1) + (part >> 2) * 4 + (lane >> 5) * 2;
+    const int pool_c = (lane & 3) + ((part >> 1) & 1) * 4;
     if ((int)blockIdx.x < total) request(blockIdx.x);
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         const int n = t / per_image, r = t - n * per_image, ty = r / tiles_x, tx = r - ty * tiles_x;
-        const int cy0 = 2 * ty * kPoolTile - 1, cx0 = 2 * tx * kPoolTile - 1;   // first convolution result
 #pragma unroll
         for (int k = 0; k < RI; ++k) {
             const int i = tid + k * kThreads;
@@ -547,55 +556,82 @@ __global__ __launch_bounds__(kThreads, 2) void k_net_stem(const _Float16 *__rest
         }
         if (t + (int)gridDim.x < total) request(t + gridDim.x);
         __syncthreads();   // (also: the weights, or the last tile's results, have been read)
-        for (int pt = wave; pt < kStemTiles; pt += kThreads / kWave) {
-            const int px = pt * 16 + row, pc = min(px, kStemPixels - 1);
-            const int cy = pc / kConvTile, cx = pc - cy * kConvTile;
-            const _Float16 *src = tile + (2 * cy * kImgCols + 2 * cx + quad * 2) * 4;
-            float4_t acc[4];
+        // Sixteen results per wave and round.  A round's products go out between the instructions that finish the
+        // round before: 28 of 16 clocks in the matrix cores, beside some 120 in the vector ALU.
+        float4_t acc[2][4];
+        int pixel[2];
+        rows::static_for<0, kStemRounds + 1>([&](auto round) __attribute__((always_inline)) {
+            constexpr int I = decltype(round)::value;
+            if constexpr (I < kStemRounds) {
+                // (past the last: the last one again, the same bits to the same place)
+                const int pc = min((I * (kThreads / kWave) + wave) * 16 + row, kStemPixels - 1);
+                const int cy = pc / kConvTile, cx = pc - cy * kConvTile;
+                const _Float16 *src = tile + (2 * cy * kImgCols + 2 * cx + quad * 2) * 4;
+                pixel[I & 1] = pc;
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct) acc[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
+                for (int ct = 0; ct < 4; ++ct) acc[I & 1][ct] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ky = 0; ky < 7; ++ky) {
-                rows_u4 words = *reinterpret_cast<const rows_u4 *>(src + ky * kImgCols * 4);
-                words[0] &= first_column;
-                words[1] &= first_column;
-                const half8_t b = __builtin_bit_cast(half8_t, words);
+                for (int ky = 0; ky < 7; ++ky) {
+                    rows_u4 words = *reinterpret_cast<const rows_u4 *>(src + ky * kImgCols * 4);
+                    words[0] &= first_column;
+                    words[1] &= first_column;
+                    const half8_t b = __builtin_bit_cast(half8_t, words);
 #pragma unroll
-                for (int ct = 0; ct < 4; ++ct)
-                    acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[ct][ky], b, acc[ct], 0, 0, 0);
-            }
-            // (results outside the image: zero, which no maximum of ReLUs notices)
-            const int yy = cy0 + cy, xx = cx0 + cx;
-            const uint32_t in_image = (unsigned)yy < (unsigned)Hc && (unsigned)xx < (unsigned)Wc ? ~0u : 0u;
-#pragma unroll
-            for (int ct = 0; ct < 4; ++ct) {
-                half4_t v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float f = fmaf((float)(_Float16)acc[ct][e], sc[ct][e], sh[ct][e]);
-                    asm volatile("" : "+v"(f));
-                    v[e] = (_Float16)f;
+                    for (int ct = 0; ct < 4; ++ct)
+                        acc[I & 1][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[ct][ky], b, acc[I & 1][ct], 0, 0, 0);
                 }
-                v = __builtin_elementwise_maximum(v, half4_t{0, 0, 0, 0});
-                typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
-                *reinterpret_cast<pair_t *>(conv + px * kConvPitch + ct * 16 + quad * 4) = __builtin_bit_cast(pair_t, v) & in_image;
             }
-        }
+            if constexpr (I > 0) {
+                // (results outside the image are whatever the zeros there give: no maximum reads them)
+                constexpr int P = (I - 1) & 1;
+                _Float16 *const to = conv + pixel[P] * kConvPitch + quad * 4;
+#pragma unroll
+                for (int ct = 0; ct < 4; ++ct) {
+                    half4_t v;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+                        // (two sums rounded by one instruction)
+                        uint32_t sums = __builtin_bit_cast(uint32_t, half2_t{(_Float16)acc[P][ct][2 * h], (_Float16)acc[P][ct][2 * h + 1]});
+                        asm volatile("" : "+v"(sums));
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            float f = fmaf((float)__builtin_bit_cast(half2_t, sums)[e], sc[ct][2 * h + e], sh[ct][2 * h + e]);
+                            asm volatile("" : "+v"(f));
+                            v[2 * h + e] = (_Float16)f;
+                        }
+                    }
+                    *reinterpret_cast<half4_t *>(to + ct * 16) = __builtin_elementwise_maximum(v, half4_t{0, 0, 0, 0});
+                }
+            }
+            if constexpr (I > 0 && I < kStemRounds) {
+                __builtin_amdgcn_sched_group_barrier(0x100 /* LDS reads */, 7, 0);
+                rows::static_for<0, 28>([&](auto) __attribute__((always_inline)) {
+                    __builtin_amdgcn_sched_group_barrier(0x2 /* vector ALU */, 4, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x8 /* a product */, 1, 0);
+                });
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
         __syncthreads();
-        for (int i = tid; i < kPoolTile * kPoolTile * 8; i += kThreads) {
-            const int cq = i & 7, p = i >> 3, py = p / kPoolTile, pxx = p % kPoolTile;
-            const int oy = ty * kPoolTile + py, ox = tx * kPoolTile + pxx;
+#pragma unroll
+        for (int k = 0; k < kPoolTile * kWave / kThreads; ++k) {
+            const int py = wave + k * (kThreads / kWave);
+            const int oy = ty * kPoolTile + py, ox = tx * kPoolTile + pool_x;
+            // (the row above and the column left of the image: the next ones, which a maximum takes in any case.
+            // Those past its other edges belong to pixels that are not stored)
+            const int up = 2 * py + (oy == 0), left = 2 * pool_x + (ox == 0);
             half8_t m = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
             for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
                 for (int dx = 0; dx < 3; ++dx) {
                     const half8_t v = *reinterpret_cast<const half8_t *>(
-                        conv + ((2 * py + dy) * kConvTile + 2 * pxx + dx) * kConvPitch + cq * 8);
+                        conv + ((dy ? 2 * py + dy : up) * kConvTile + (dx ? 2 * pool_x + dx : left)) * kConvPitch + pool_c * 8);
                     m = __builtin_elementwise_maximum(m, v);
                 }
             if (oy < Hp && ox < Wp)
-                *reinterpret_cast<half8_t *>(out + (((int64_t)n * Hp + oy) * Wp + ox) * kStemOut + cq * 8) = m;
+                *reinterpret_cast<half8_t *>(out + (((int64_t)n * Hp + oy) * Wp + ox) * kStemOut + pool_c * 8) = m;
         }
         // (the next tile's image part does not touch `conv`, and its barrier comes before
         // the next results do)
