@@ -55,9 +55,11 @@ constexpr int kFc2Pitch = 12;    // a channel's nine values, 16-byte rows
 // each and this, us (fp16, medians under the profiler): 64 x 128 x 28 x 28 18.2 / 8.8, 64 x 64 x 56 x 56 19.4 / 8.8, 64 x 256 x 14 x 14 17.6 / 8.5, 256 x 128 x
 // 14 x 14 55.4 / 19.6, 1 x 512 x 14 x 14 6.4 / 5.8, fp32 32 x 256 x 28 x 28 15.0 / 10.4; four of them with the loads asked for at once: 64 x 512 x 7 x 7
 // 18.9 / 13.6, 3 x 2048 x 7 x 7 31.8 / 23.9.  (8 x 64 x 200 x 300, whose time is the other half's: 13.0 / 13.7.)
-inline int fc2_channels(int64_t C, int64_t mid) {
+// Batches whose parts would pass 64 MB, 25 us to write and read again at a copy's rate, take more channels: the workspace stays bounded.
+constexpr int64_t kFc2MostParts = 1 << 24;
+inline int fc2_channels(int64_t N, int64_t C, int64_t mid) {
     int cw = 1;
-    while (cw < kFc2MaxChannels && cdiv(C, cw) * cdiv(mid, kWave) > kUnits) cw *= 2;
+    while (cw < kFc2MaxChannels && (cdiv(C, cw) * cdiv(mid, kWave) > kUnits || cdiv(C, cw) * N * mid > kFc2MostParts)) cw *= 2;
     return cw;
 }
 
@@ -573,7 +575,7 @@ size_t pack_backward_workspace(int64_t N, int64_t C, int64_t mid, int64_t H, int
     int splits, split_pix;
     const int64_t npix = (H / stride) * (W / stride);
     ws_split(N, C, npix, dtype == DDF_F16 ? 32 : 16, &splits, &split_pix);
-    return floats256(cdiv(C, fc2_channels(C, mid)) * N * mid) + floats256(N * mid) + floats256(N * C) +
+    return floats256(cdiv(C, fc2_channels(N, C, mid)) * N * mid) + floats256(N * mid) + floats256(N * C) +
            floats256(N * splits * head * KK * (C + 1));
 }
 
@@ -585,7 +587,7 @@ hipError_t pack_backward(const PackBackward<T> &b, int64_t N, int64_t C, int64_t
     constexpr int STEP = 4 * Quad<T>::n;
     int splits, split_pix;
     ws_split(N, C, npix, STEP, &splits, &split_pix);
-    const int cw2 = fc2_channels(C, mid), cblocks = (int)cdiv(C, cw2);
+    const int cw2 = fc2_channels(N, C, mid), cblocks = (int)cdiv(C, cw2);
     unsigned char *q = static_cast<unsigned char *>(ws);
     float *dh_part = reinterpret_cast<float *>(q); q += floats256((int64_t)cblocks * N * mid);
     float *dz1 = reinterpret_cast<float *>(q); q += floats256(N * mid);
