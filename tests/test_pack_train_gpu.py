@@ -22,6 +22,7 @@ CASES = [
     (70, 24, 3, 5, 1, 1, 'mul'),       # samples past a chunk of 64 where a workgroup has one channel,
     (65, 300, 4, 2, 1, 1, 'add'),      # two,
     (131, 344, 2, 3, 1, 1, 'mul'),     # and four
+    (30000, 64, 1, 1, 1, 1, 'mul'),    # so many that two keep the partial sums within their bound
 ]
 
 
