@@ -31,34 +31,15 @@ hipError_t rows_taprow_backward_launch(const Problem &p, const RowsGeom &g, cons
                                        const T *x, const T *cf, const T *sf, T *dx, T *dcf, T *dsf,
                                        typename Acc<T>::type *ws_sf, typename Acc<T>::type *ws_cf, unsigned need,
                                        hipStream_t st) {
-    const int tail = g.tail == 0 ? 0 : g.shift ? 2 : 1;
-    const bool pad = tail > 0 || rows_shift_in_as_is(g);
+    const int tail = rows::taprow_backward_tail(g);
+    const bool pad = rows::taprow_backward_pad(g);
 #define DDF_BACKWARD_CASE(D_, VXF_, VX_, PAD_, TAIL_)                                              \
     if (p.d == D_ && vxf == VXF_ && vx == VX_ && pad == PAD_ && tail == TAIL_)                     \
-        return rows::launch_taprow_backward<T, D_, VXF_, VX_, PAD_, TAIL_>(p, g, gx, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, st)
-#define DDF_BACKWARD_EXACT(D_, VXF_, VX_)       \
-    DDF_BACKWARD_CASE(D_, VXF_, VX_, false, 0); \
-    DDF_BACKWARD_CASE(D_, VXF_, VX_, true, 0)
-    // (taps two apart reach two pixels into a lane's neighbours: no vectors of two)
-    DDF_BACKWARD_EXACT(1, 2, 4);
-    DDF_BACKWARD_EXACT(1, 4, 4);
-    DDF_BACKWARD_EXACT(2, 4, 4);
-    if constexpr (sizeof(T) == 4) {
-        DDF_BACKWARD_CASE(1, 4, 4, true, 1);
-        DDF_BACKWARD_CASE(2, 4, 4, true, 1);
-    } else {
-        DDF_BACKWARD_CASE(1, 4, 4, true, 2);
-        DDF_BACKWARD_CASE(2, 4, 4, true, 2);
-        DDF_BACKWARD_EXACT(1, 4, 8);
-        DDF_BACKWARD_EXACT(2, 4, 8);
-        DDF_BACKWARD_EXACT(1, 8, 8);
-        DDF_BACKWARD_EXACT(2, 8, 8);
-        DDF_BACKWARD_CASE(1, 8, 8, true, 1);
-        DDF_BACKWARD_CASE(2, 8, 8, true, 1);
-        DDF_BACKWARD_CASE(1, 8, 8, true, 2);
-        DDF_BACKWARD_CASE(2, 8, 8, true, 2);
+        return rows::launch_taprow_backward<T, D_, VXF_, VX_, PAD_, TAIL_>(p, g, gx, go, x, cf, sf, dx, dcf, dsf, ws_sf, ws_cf, need, st);
+    DDF_BACKWARD5_BOTH_TYPES(DDF_BACKWARD_CASE)
+    if constexpr (sizeof(T) == 2) {
+        DDF_BACKWARD5_F16(DDF_BACKWARD_CASE)
     }
-#undef DDF_BACKWARD_EXACT
 #undef DDF_BACKWARD_CASE
     return hipErrorNotSupported;
 }

@@ -717,9 +717,9 @@ bool rows_taprow_backward_plan(const Problem &p, int dtype, RowsGeom *g, RowsGeo
         tune_int("DDF_TUNE_ROWS", 1) == 0 || !rows_taprow_plan(p, dtype, g, vxf, &r) ||
         !rows_plan(p, dtype, gx, vx, &r_dx, true))
         return false;
-    // (ragged rows: the same vectors; else those of the filter gradients may be half as long)
-    if (r != 1 || r_dx != 1 || (*vxf != *vx && (g->tail != 0 || *vxf * 2 != *vx)) || gx->tail != g->tail || gx->shift != g->shift ||
-        rows_shift_in_as_is(*gx) != rows_shift_in_as_is(*g))
+    // (the two walks are built with one PAD and one TAIL: a plane that they would lay out differently takes two launches)
+    if (r != 1 || r_dx != 1 || gx->tail != g->tail || gx->shift != g->shift || rows_shift_in_as_is(*gx) != rows_shift_in_as_is(*g) ||
+        !rows::taprow_backward_built(dtype == DDF_F16 ? 2 : 4, p.d, *vxf, *vx, rows::taprow_backward_pad(*g), rows::taprow_backward_tail(*g)))
         return false;
     gx->wpb = rows::kTaprowWaves;
     gx->xcd_per = (unsigned)cdiv(cdiv(gx->nwork, gx->wpb), rows::kXcd);

@@ -34,6 +34,26 @@ constexpr int taprow_lds_bytes(int asz) {
     return kTaprowWaves * taprow_flush_channels<K>() * K * kRedPitch * asz;
 }
 
+// What k_rows_taprow_backward is built for, X(D, VXF, VX, PAD, TAIL): the one list that its plan and its launcher go by.
+// (Taps two apart reach two pixels into a lane's neighbours: no vectors of two.  TAIL 2: an odd tail of fp16.)
+#define DDF_BACKWARD5_EXACT(X, D, VXF, VX) X(D, VXF, VX, false, 0) X(D, VXF, VX, true, 0)
+#define DDF_BACKWARD5_BOTH_TYPES(X)                                                             \
+    DDF_BACKWARD5_EXACT(X, 1, 2, 4) DDF_BACKWARD5_EXACT(X, 1, 4, 4) DDF_BACKWARD5_EXACT(X, 2, 4, 4) \
+    X(1, 4, 4, true, 1) X(2, 4, 4, true, 1)
+#define DDF_BACKWARD5_F16(X)                                                                    \
+    X(1, 4, 4, true, 2) X(2, 4, 4, true, 2)                                                     \
+    DDF_BACKWARD5_EXACT(X, 1, 4, 8) DDF_BACKWARD5_EXACT(X, 2, 4, 8)                             \
+    DDF_BACKWARD5_EXACT(X, 1, 8, 8) DDF_BACKWARD5_EXACT(X, 2, 8, 8)                             \
+    X(1, 8, 8, true, 1) X(2, 8, 8, true, 1) X(1, 8, 8, true, 2) X(2, 8, 8, true, 2)
+
+inline int taprow_backward_tail(const RowsGeom &g) { return g.tail == 0 ? 0 : g.shift ? 2 : 1; }
+inline bool taprow_backward_pad(const RowsGeom &g) { return g.tail > 0 || rows_shift_in_as_is(g); }
+inline bool taprow_backward_built(int esz, int d, int vxf, int vx, bool pad, int tail) {
+#define DDF_BACKWARD5_IS(D_, VXF_, VX_, PAD_, TAIL_) || (d == D_ && vxf == VXF_ && vx == VX_ && pad == PAD_ && tail == TAIL_)
+    return (false DDF_BACKWARD5_BOTH_TYPES(DDF_BACKWARD5_IS)) || (esz == 2 && (false DDF_BACKWARD5_F16(DDF_BACKWARD5_IS)));
+#undef DDF_BACKWARD5_IS
+}
+
 #ifdef __HIPCC__
 
 template <typename T, int K, int D, bool MUL, int VX, int R, bool PAD, int NST, int TAIL = 0>
@@ -331,7 +351,11 @@ __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_filte
 // well, begins behind that.  Here its workgroups take the places that are left.  Kernel times of a whole step, us, two launches /
 // this: fp32 32 x 128 x 56 x 56 taps two apart 133.9 / 108.3 (the gradients 102 / 77), one apart 128.6 / 105.6, 8 x 256 x 28 x 28 39.0 / 29.2, 3 x 256 x 100
 // x 104 84.4 / 73.1, 5 x 33 x 200 x 190 81.7 / 73.0, 2 x 64 x 40 x 52 25.1 / 19.1; fp16 32 x 128 x 56 x 56 131.8 / 108.7, 'add' 107.8 / 91.0, 8 x 64 x 200
-// x 200 184.9 / 179.6, 21 x 104 x 57 x 61 114.8 / 106.0, 1 x 512 x 50 x 75 51.1 / 41.3.  No size was found where two are faster.
+// x 200 184.9 / 179.6, 21 x 104 x 57 x 61 114.8 / 106.0, 1 x 512 x 50 x 75 51.1 / 41.3.  The gradients and their sums alone, even tails of
+// fp16: 13 x 120 x 34 x 34 taps two apart 33.6 / 28.4, 6 x 76 x 9 x 66 20.8 / 13.9, 4 x 256 x 50 x 74 49.5 / 40.2, 16 x 64 x 90 x 90 65.6 / 55.4.  No size
+// was found where two are faster.  Two remain for one half on its own, for operands that are not aligned to dX's vectors, and where the halves'
+// layouts have no instance here in common (an eighth of fp16's sizes, a sixteenth of fp32's): filter gradients in vectors a quarter as long or half
+// as long as ragged ones, or one half as a run, in segments or with idle lanes between rows and the other not.
 template <typename T, int D, bool MUL, int VXF, int VX, bool PAD, int NST, int WPE, int TAIL>
 __global__ __launch_bounds__(kWave * kTaprowWaves, WPE) void k_rows_taprow_backward(
     RowsGeom g, RowsGeom gx, int blocks, const T *__restrict__ go, const T *__restrict__ x, const T *__restrict__ cf,

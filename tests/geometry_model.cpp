@@ -411,6 +411,43 @@ static void check_rows_run(long N, long C, long H, long W, int k, int d, int dty
     g_fails = 0;
 }
 
+// All gradients of 5 x 5 filters in one launch: the lanes of both walks, and the feature gradient's work items in
+// workgroups of as many waves as the filter gradients have.  (Ragged strips of whole rows: their work items.)
+static void check_rows_backward5(long N, long C, long H, long W, int d, int dtype) {
+    const Problem p = make_problem(N, C, H, W, 5, d, 1, 0);
+    RowsGeom g{}, gx{};
+    int vxf, vx;
+    if (!rows_taprow_backward_plan(p, dtype, &g, &gx, &vxf, &vx)) {
+        printf("kind rows-backward5 %ldx%ldx%ldx%ld d%d dt%d: unsupported\n", N, C, H, W, d, dtype);
+        return;
+    }
+    printf("kind rows-backward5 %ldx%ldx%ldx%ld d%d dt%d: vxf=%d vx=%d tail=%d halo=%d,%d csplit=%d,%d nwork=%d,%d\n", N, C, H, W, d,
+           dtype, vxf, vx, g.tail, g.halo, gx.halo, g.csplit, gx.csplit, g.nwork, gx.nwork);
+    CHECK(2 * d <= vxf && 2 * d <= vx, "taps reach beyond the neighbouring lane");
+    CHECK(g.wpb == rows::kTaprowWaves && gx.wpb == rows::kTaprowWaves, "waves per workgroup");
+    CHECK(rows::taprow_lds_bytes<5>(4) <= 64 * 1024, "LDS");
+    CHECK(((long)g.xcd_per + gx.xcd_per) * 8 < (1l << 30), "workgroups");
+    bool filters = false, features = false;
+#define WALK_CASE(VX_)                                                                             \
+    if (vxf == VX_) {                                                                              \
+        if (g.halo) for (int i = 0; i < 5; ++i) replay_rows_run<1, 0, VX_>(g, N, C, 2, 5, (i - 2) * d); \
+        else if (g.tail == 0) replay_rows<1, 0, VX_>(g, N, C, 2, 5, d);                            \
+        else check_work_items(g, N, C, 2, 5);                                                      \
+        filters = true;                                                                            \
+    }                                                                                              \
+    if (vx == VX_) {                                                                               \
+        if (gx.halo) d == 1 ? replay_rows_run<1, 2, VX_>(gx, N, C, 0, 0, 0) : replay_rows_run<1, 4, VX_>(gx, N, C, 0, 0, 0); \
+        else if (gx.tail == 0) d == 1 ? replay_rows<1, 2, VX_>(gx, N, C, 0) : replay_rows<1, 4, VX_>(gx, N, C, 0); \
+        else check_work_items(gx, N, C, 0, 0);                                                     \
+        features = true;                                                                           \
+    }
+    WALK_CASE(2) WALK_CASE(4) WALK_CASE(8)
+#undef WALK_CASE
+    CHECK(filters && features, "no replay for vectors of %d and %d", vxf, vx);
+    if (g_fails) printf("  -> %d violations\n", g_fails);
+    g_fails = 0;
+}
+
 // Stride 2 (3 x 3) on the row-register kernels: lanes are laid out over the result plane;
 // rows::LaneStride2 says where the lane's three feature vectors (2 * VX elements each) and
 // its VX result pixels are.
@@ -607,6 +644,7 @@ int main() {
             for (int dtype = 0; dtype < 3; ++dtype) {
                 check_rows(sh[0], sh[1], sh[2], sh[3], 5, d, dtype, false);
                 check_rows(sh[0], sh[1], sh[2], sh[3], 5, d, dtype, true, false, true);
+                check_rows_backward5(sh[0], sh[1], sh[2], sh[3], d, dtype);
                 check_rows(sh[0], sh[1], sh[2], sh[3], 3, d, dtype, true, false, true);
             }
     for (auto &sh : shapes)
@@ -639,6 +677,7 @@ int main() {
                     check_rows_run(8, 96, H, W, 3, d, dtype, 1);
                     check_rows_run(8, 96, H, W, 3, d, dtype, 1, true);
                     check_rows_run(8, 96, H, W, 5, d, dtype, 2);
+                    check_rows_backward5(8, 96, H, W, d, dtype);
                 }
     // seeded random shapes on top of the fixed list
     unsigned long long state = 0x9E3779B97F4A7C15ull;
@@ -657,6 +696,8 @@ int main() {
         check_rows(N, C, H, (W / 8 + 1) * 8, 5, next(1, 2), next(0, 1), false);
         check_rows(N, C, H, (W / 8 + 1) * 8 * next(1, 6), 3, next(1, 2), next(0, 1), next(0, 1) != 0);
         check_rows(N, C, H, (W / 4 + 1) * 4, 5, next(1, 2), next(0, 1), true, false, true);
+        check_rows_backward5(N, C, H, W + 3, 1 + i % 2, i / 2 % 2);
+        check_rows_backward5(N, C, H, (W / 4 + 1) * 4, 1 + i % 2, i / 2 % 2);
         check_rows_stride2(N, C, H + 1, (W / 4 + 1) * 4, next(0, 1), next(0, 1) != 0);
         check_rows_stride2(N, C, H + 1, (W / 16 + 1) * 16, next(0, 1), next(0, 1) != 0);
         check_rows_stride2(N, C, H + 1, (W / 16 + 1) * 16, next(0, 1), true, true);

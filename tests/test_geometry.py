@@ -9,6 +9,8 @@ kernel size and scale they take).  A launch
 geometry that would make a kernel read or write out of bounds - the kind of
 mistake that faults a GPU - shows up here as a VIOLATION line instead."""
 import os
+import random
+import re
 import shutil
 import subprocess
 
@@ -88,3 +90,30 @@ def test_filter_gradients_of_whole_lines_stay_rows(dtype, shape, run):
     for need in (_lib.NEED_DCF | _lib.NEED_DSF, _lib.NEED_DX | _lib.NEED_DCF | _lib.NEED_DSF):
         name = _lib.describe(shape, 3, 1, 1, 'mul', getattr(torch, dtype), need)
         assert ('run>' in name) == run, name
+
+
+@pytest.mark.skipif(shutil.which('nm') is None, reason='nm not available')
+def test_every_plan_of_all_five_by_five_gradients_has_its_kernel():
+    """What describe names as one launch is one: the library holds the kernel that the plan asks for."""
+    import torch
+    from ddfnet_amd import LIB_PATH, _lib
+    names = subprocess.run(['nm', '-C', LIB_PATH], capture_output=True, text=True, check=True).stdout
+    built = set(re.findall(r'k_rows_taprow_backward<(float|__half), (\d), (true|false), (\d), (\d), (true|false), \d+, \d+, (\d)>', names))
+    rng = random.Random(5)
+    shapes = [(13, 120, 34, 34, 2), (6, 76, 9, 66, 1), (3, 40, 31, 30, 2), (4, 256, 50, 74, 1), (2, 64, 100, 150, 1)]
+    shapes += [(rng.randint(1, 40), rng.randint(1, 200), rng.randint(3, 200), rng.randint(4, 260), rng.choice((1, 2))) for _ in range(1500)]
+    met = set()
+    for n, c, h, w, d in shapes:
+        for dtype, element in ((torch.float32, 'float'), (torch.float16, '__half')):
+            for combine in ('mul', 'add'):
+                plan = re.match(r'k_rows_taprow_backward<VXF=(\d),VX=(\d),(.*?)>', _lib.describe((n, c, h, w), 5, d, 1, combine, dtype, need=7))
+                if not plan:
+                    continue
+                vxf, vx, layout = plan.groups()
+                ragged = 'ragged' in layout    # (odd fp16 tails: the lane loads from one element further left)
+                tail = 0 if not ragged else 2 if dtype == torch.float16 and w % int(vx) % 2 else 1
+                pads = ('true', 'false') if layout == 'run' else ('false',) if layout == 'plain' else ('true',)
+                wanted = {(element, str(d), 'true' if combine == 'mul' else 'false', vxf, vx, pad, str(tail)) for pad in pads}
+                assert wanted & built, ((n, c, h, w), d, dtype, plan.group(0))
+                met |= wanted & built
+    assert len(met) > 40    # (the sweep meets most of them)
