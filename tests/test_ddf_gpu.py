@@ -461,19 +461,95 @@ def test_fp16_five_by_five_of_few_and_many_waves(few, many, shape, d, combine):
 def test_five_by_five_gradients_in_one_launch(shape, d, dtype, combine):
     """All gradients at once are the bits that each half leaves alone.  (The channel filter's in fp16 'add' are fp32 sums of H * W products of
     two fp16 values; the compiler adds two of them at a time where it likes: an error of 2^-24 of the sum of magnitudes per addition, and a
-    rounding to fp16.)"""
+    rounding to fp16.)  fp16 sizes whose halves are laid out differently take two launches."""
+    from ddfnet_amd import _lib
+    apart = dtype == torch.float16 and (shape, d) in (((1, 3, 9, 8), 1), ((1, 9, 70, 264), 1), ((8, 8, 200, 204), 1), ((8, 8, 200, 201), 2))
+    assert ('k_rows_taprow_backward<' in _lib.describe(shape, 5, d, 1, combine, dtype, need=7)) != apart
+    _gradients_at_once_and_apart(shape, d, dtype, combine)
+
+
+def _gradients_at_once_and_apart(shape, d, dtype, combine):
     x, cf, sf, go = random_case(*shape, 5, 1, dtype, seed=shape[1])
     dev = to_dev(x, cf, sf, go)
     _, dx, dcf, dsf = run_ddf(*dev, 5, d, 1, combine)
     assert torch.equal(dx, run_ddf(*dev, 5, d, 1, combine, need=(True, False, False))[1])
     _, _, cf_alone, sf_alone = run_ddf(*dev, 5, d, 1, combine, need=(False, True, True))
     assert torch.equal(dsf, sf_alone)
-    if dtype == torch.float16 and combine == 'add':
-        most = (x.float().abs().max() * go.float().abs().max()).item()
-        torch.testing.assert_close(dcf, cf_alone, rtol=2. ** -10, atol=most * shape[2] * shape[3] * 2. ** -24)
-    else:
-        assert torch.equal(dcf, cf_alone)
+    most = (x.float().abs().max() * go.float().abs().max()).item()
+
+    def same_channel_filters(got, want):
+        if dtype == torch.float16 and combine == 'add':
+            torch.testing.assert_close(got, want, rtol=2. ** -10, atol=most * shape[2] * shape[3] * 2. ** -24)
+        else:
+            assert torch.equal(got, want)
+
+    same_channel_filters(dcf, cf_alone)
+    # the feature gradient with one of the filters'
+    _, dx_cf, only_cf, _ = run_ddf(*dev, 5, d, 1, combine, need=(True, True, False))
+    _, dx_sf, _, only_sf = run_ddf(*dev, 5, d, 1, combine, need=(True, False, True))
+    assert torch.equal(dx, dx_cf) and torch.equal(dx, dx_sf) and torch.equal(dsf, only_sf)
+    same_channel_filters(only_cf, cf_alone)
     check_against_oracle(x[:1], cf[:1], sf[:1], go[:1], 5, d, 1, combine)
+
+
+def _backward_launches(shape, d, dtype, combine):
+    """How many launches the three gradients of a call are, by the nodes of a captured graph."""
+    import ctypes
+
+    from ddfnet_amd import _lib, ddf
+    dev = to_dev(*random_case(*shape, 5, 1, dtype, seed=1))
+    leaves = [t.requires_grad_(True) for t in dev[:3]]
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        out = ddf(*leaves, 5, d, 1, combine)
+        torch.autograd.grad(out, leaves, dev[3], retain_graph=True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=stream):
+            grads = torch.autograd.grad(out, leaves, dev[3], retain_graph=True)
+    nodes = ctypes.c_size_t()
+    assert _lib.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    del grads
+    return nodes.value
+
+
+# one size for every kernel of the one launch (vectors of the filter gradients and of the feature gradient, layout): (dtypes, d, shape, name)
+_F16, _F32, _BOTH = (torch.float16,), (torch.float32,), (torch.float16, torch.float32)
+_ONE_LAUNCH = [
+    (_BOTH, 1, (1, 1, 3, 4), '2,VX=4,padded'), (_BOTH, 1, (2, 3, 44, 4), '2,VX=4,plain'), (_BOTH, 1, (1, 2, 3, 68), '2,VX=4,segments'),
+    (_F16, 1, (2, 90, 9, 132), '2,VX=4,run'), (_F32, 1, (2, 117, 13, 72), '2,VX=4,run'),
+    (_F16, 1, (28, 1, 59, 60), '4,VX=4,padded'), (_F32, 1, (30, 1, 41, 80), '4,VX=4,padded'), (_BOTH, 2, (1, 1, 3, 4), '4,VX=4,padded'),
+    (_BOTH, 1, (42, 1, 110, 20), '4,VX=4,plain'), (_BOTH, 2, (1, 1, 33, 4), '4,VX=4,plain'),
+    (_F16, 1, (41, 1, 12, 196), '4,VX=4,segments'), (_F16, 2, (1, 2, 3, 148), '4,VX=4,segments'), (_F32, 2, (1, 2, 3, 136), '4,VX=4,segments'),
+    (_F16, 1, (1, 123, 58, 52), '4,VX=4,run'), (_F16, 2, (2, 52, 13, 252), '4,VX=4,run'), (_F32, 1, (5, 98, 8, 88), '4,VX=4,run'),
+    # two pixels past the last vector of four, and one or three
+    (_F16, 1, (1, 2, 5, 26), '4,VX=4,ragged'), (_BOTH, 2, (1, 1, 5, 26), '4,VX=4,ragged'), (_F16, 2, (3, 40, 31, 30), '4,VX=4,ragged'),
+    (_F16, 1, (6, 83, 16, 38), '4,VX=4,ragged run'), (_F16, 2, (3, 105, 5, 258), '4,VX=4,ragged run'),
+    (_F16, 1, (1, 2, 3, 130), '4,VX=4,ragged segments'), (_BOTH, 2, (1, 2, 3, 130), '4,VX=4,ragged segments'),
+    (_BOTH, 1, (1, 1, 10, 13), '4,VX=4,ragged'), (_F16, 2, (1, 1, 10, 13), '4,VX=4,ragged'),
+    (_F16, 1, (7, 70, 3, 261), '4,VX=4,ragged run'), (_BOTH, 2, (1, 97, 15, 259), '4,VX=4,ragged run'),
+    (_BOTH, 1, (1, 2, 3, 129), '4,VX=4,ragged segments'), (_F16, 2, (1, 1, 3, 137), '4,VX=4,ragged segments'),
+    # vectors of eight
+    (_F16, 1, (55, 2, 17, 104), '4,VX=8,padded'), (_F16, 1, (32, 2, 75, 40), '4,VX=8,plain'), (_F16, 1, (26, 1, 16, 240), '4,VX=8,segments'),
+    (_F16, 1, (5, 98, 8, 88), '4,VX=8,run'), (_F16, 2, (1, 2, 3, 8), '4,VX=8,padded'), (_F16, 2, (1, 2, 43, 8), '4,VX=8,plain'),
+    (_F16, 2, (1, 2, 3, 136), '4,VX=8,segments'), (_F16, 2, (5, 100, 3, 264), '4,VX=8,run'),
+    (_F16, 1, (27, 1, 64, 120), '8,VX=8,padded'), (_F16, 1, (43, 2, 109, 40), '8,VX=8,plain'), (_F16, 1, (5, 1, 164, 184), '8,VX=8,run'),
+    (_F16, 2, (62, 3, 26, 120), '8,VX=8,padded'), (_F16, 2, (60, 1, 197, 16), '8,VX=8,plain'), (_F16, 2, (5, 1, 116, 264), '8,VX=8,run'),
+    (_F16, 1, (41, 1, 138, 148), '8,VX=8,ragged'), (_F16, 1, (28, 1, 177, 243), '8,VX=8,ragged'), (_F16, 1, (41, 2, 126, 132), '8,VX=8,ragged run'),
+    (_F16, 2, (36, 1, 222, 110), '8,VX=8,ragged'), (_F16, 2, (48, 1, 104, 241), '8,VX=8,ragged'), (_F16, 2, (14, 2, 189, 252), '8,VX=8,ragged run'),
+]
+
+
+@pytest.mark.parametrize('combine', ['mul', 'add'])
+@pytest.mark.parametrize('dtype,d,shape,name', [(t,) + c[1:] for c in _ONE_LAUNCH for t in c[0]], ids=_ids)
+def test_five_by_five_gradients_in_every_kernel_of_the_one_launch(dtype, d, shape, name, combine):
+    """The launch that describe names is the one that runs, and its bits are those of each half alone."""
+    from ddfnet_amd import _lib
+    names = _lib.describe(shape, 5, d, 1, combine, dtype, need=7)
+    assert names.startswith('k_rows_taprow_backward<VXF=%s>' % name), names
+    assert _backward_launches(shape, d, dtype, combine) == names.count(' + ') + 1
+    _gradients_at_once_and_apart(shape, d, dtype, combine)
 
 
 def test_runs_on_the_current_stream():
