@@ -73,6 +73,8 @@ def close(got, want, tol):
     # 128 x 128 in three stages, a workgroup per unit: one, two, three and seventeen stages of K, rows and channels past a tile; 592: 128 x 64
     (1, 129, 163, 64, 128, 1, 1, 0, 1, 1), (1, 129, 163, 128, 128, 1, 0, 1, 0, 0), (1, 90, 120, 192, 136, 1, 1, 0, 1, 1),
     (1, 65, 128, 1088, 256, 1, 1, 0, 0, 1), (1, 172, 220, 192, 256, 1, 1, 0, 1, 1),
+    # 1536 tiles of 128 x 128: a short K in short stages, a long one by eight waves
+    (1, 256, 256, 704, 264, 1, 1, 0, 1, 1), (1, 241, 272, 832, 264, 1, 1, 0, 1, 1),
 ])
 def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
     torch.manual_seed(c + o)
@@ -249,6 +251,7 @@ def test_network_matches_its_modules(build, n, size, classes):
     (5, 11, 11, 320, 264), (50, 3, 4, 576, 264), (3, 16, 16, 2048, 264), (7, 13, 9, 128, 65),    # 32 x 32, samples ending inside; 16 x 16
     (1, 260, 258, 64, 64),                      # 67080 pixels: too many for a division by multiplying
     (110, 14, 14, 192, 128), (45, 14, 14, 1024, 264), (7, 41, 43, 64, 136),    # 128 x 128 in three stages
+    (99, 14, 14, 256, 520),                     # 760 of them in two
 ])
 def test_conv_pool(n, h, w, c, o):
     """The results of conv, and their sums over the pixels, slot by slot of the tiles."""
