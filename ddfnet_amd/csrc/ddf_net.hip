@@ -153,7 +153,9 @@ __global__ __launch_bounds__(2 * WN * kWave, WG * WN / 2) void k_net_conv(NetCon
     clear();
     // Without a BatchNorm (the classifier) a bias is part of the sum, which is rounded once, as
     // nn.Linear has it.  Elsewhere, and in a pair, the sum is rounded first, as a convolution's
-    // result is.  (A bias in a pair's accumulators had the 128 x 128 tiles spill: 86 -> 117 us.)
+    // result is.  (A bias in a pair's accumulators had the 128 x 128 tiles spill: 86 -> 117 us; the rounding left out where there is no BatchNorm
+    // takes 14 to 17 registers of a pair's and spills 33 of those in short stages.  A pair without one in the small tiles of ddf_net_small.hip, which have room,
+    // and as the two launches it once was, is rounded once less.)
     const bool bias_in_sum = !PAIR && !a.norm.var && a.norm.conv_bias;
     // `meanwhile`: what goes out behind the products of a step, the stage's loads spread over its steps.  The
     // next step's operands are asked for in front of a step's products: left to itself the compiler keeps one set of
@@ -1084,7 +1086,8 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
 // tiles of 64: 100 of K = 2048 16.0 / 26.0 / 19.5, of 1024 9.8 / 13.8 / 11.5; 160 of 512 8.1 / 8.9 / 8.3; 152 of 256 5.7 / 6.1 / 6.2.
 // Where the last round of two per unit would be nearly empty, 128 x 64, three workgroups per unit: us, 128 x 128 / 128 x 64, 294 tiles
 // of 18816 1024 -> 256 20.4 / 20.0, 304 of 2048 19.6 / 18.5, 304 of a pair 27.6 / 26.8; 588 of 75264 512 -> 128 22.0 / 20.5, 592 of 512 -> 2048 19.6 / 18.5, of
-// pairs 27.8 / 26.9 and 49.2 / 46.3; 344 tiles 20.2 / 20.1, 688 50.2 / 51.1.  Of fewer than 128 channels 128 x 64 in short stages from 1024 tiles on, in long
+// pairs 27.8 / 26.9 and 49.2 / 46.3; 344 tiles 20.2 / 20.1, 688 50.2 / 51.1 (operands in cache, 60 sizes of 520 to 608 tiles 1 to 12 % less; from memory 3 to 9 %
+// less for 256 channels, up to 14 more for 2048).  Of fewer than 128 channels 128 x 64 in short stages from 1024 tiles on, in long
 // ones from 448.
 // In small tiles (ddf_net_small.hip), whose workgroups bring in a quarter of K per wave, what leaves most of the chip idle in tiles
 // of 64: 16 x 16 up to two workgroups per compute unit, 32 x 32 of a K that is worth four waves up to one.  us, tiles of 64 / 16 x 16 / 32 x 32:

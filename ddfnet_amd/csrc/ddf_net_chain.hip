@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kThreads, WPS) void k_net_chain(NetChain a) {
 #pragma unroll
             for (int i = 0; i < RV; ++i) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[i][e] = (_Float16)fmaf((float)v[i][e], sc[e], sh[e]);    // (rounded once, as in a pair)
+                for (int e = 0; e < 8; ++e) v[i][e] = (_Float16)fmaf((float)v[i][e], sc[e], sh[e]);    // (rounded once, as in k_net_conv's pairs)
                 rv[i] = __builtin_bit_cast(rows_u4, v[i]);
             }
             asm volatile("" ::: "memory");

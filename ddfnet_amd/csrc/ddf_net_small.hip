@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_net_conv_small(NetConv a, NetCo
     sums_t side;
     if constexpr (PAIR) side = total(0);
     lane_t v;
-    // (under a BatchNorm the sum is rounded first, as a convolution's result is; without one a bias is part of it)
+    // (under a BatchNorm the sum is rounded first, as a convolution's result is; without one a bias is part of it, of a pair's sums too,
+    // which k_net_conv rounds first)
     auto under = [](const NetNorm &n, float x) { return n.var ? (float)(_Float16)x : x; };
 #pragma unroll
     for (int e = 0; e < V; ++e) {

@@ -358,7 +358,8 @@ int ddf_hip_pack_backward(const void *features, const void *grad_channel_filter,
  *           C a multiple of 64
  *   conv_pair out = act(norm(1x1 convolution of features (N, Ho, Wo, C)) + norm'(1x1 convolution of
  *           stride `stride` of side_features (N, H, W, side_C))): a bottleneck's last convolution
- *           and its projection; out overlaps neither input; C and side_C multiples of 64
+ *           and its projection; out overlaps neither input; C and side_C multiples of 64.  (A sum is rounded to
+ *           fp16 in front of its BatchNorm; without one, where pixels are many, in front of its bias)
  *   stem    max_pool(relu(norm(7x7 convolution, stride 2, padding 3, weight (64, 3, 7, 7))), 3x3,
  *           stride 2, padding 1) of a planar (N, 3, H, W) image; H and W multiples of 4
  *   spatial the spatial filter branch (3x3 taps, one head): spatial_filter (N, Ho*Wo, 12), nine

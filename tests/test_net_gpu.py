@@ -58,13 +58,14 @@ def close(got, want, tol):
     (5, 28, 30, 256, 512, 2, 1, 0, 0, 0),      # projection under stride 2
     (40, 56, 56, 256, 512, 2, 1, 0, 0, 0),
     (16, 28, 28, 128, 264, 1, 1, 0, 1, 1),     # tiles of 128 x 64, channels past the last
-    (42, 56, 56, 64, 136, 1, 1, 1, 0, 1),      # tiles of 128 x 128 in short stages
-    (3, 7, 7, 2112, 520, 1, 1, 0, 1, 1),       # tiles of 64, 33 stages of K
+    (42, 56, 56, 64, 136, 1, 1, 1, 0, 1),      # 2058 tiles of 128 x 128 in short stages
+    (3, 7, 7, 2112, 520, 1, 1, 0, 1, 1),       # 330 tiles of 16 x 16, 33 blocks of K
+    (10, 8, 8, 2112, 520, 1, 1, 0, 1, 1), (20, 8, 8, 2112, 1000, 1, 1, 0, 1, 1),    # tiles of 64, 33 stages of K: 90 of them; 320
     (1, 5, 7, 576, 200, 1, 1, 1, 1, 1),        # K split over the waves: 9 blocks, rows and channels past a tile
     (17, 1, 1, 64, 33, 1, 0, 1, 0, 1),         # one block of K
     (1, 13, 9, 1088, 31, 2, 1, 0, 0, 0),       # 17 blocks, under stride 2
     (1, 16, 16, 192, 4096, 1, 1, 0, 0, 1), (1, 1, 257, 320, 4096, 1, 1, 0, 1, 1),    # 256 tiles of 64, three stages; 320, five
-    (20, 4, 8, 1024, 256, 1, 1, 0, 1, 1), (10, 8, 8, 2048, 1000, 1, 0, 1, 0, 0),     # 40, 160: a workgroup per unit at most
+    (20, 4, 8, 1024, 256, 1, 1, 0, 1, 1), (10, 8, 8, 2048, 1000, 1, 0, 1, 0, 0),     # 160 of 32 x 32; 160 of 64, a workgroup per unit
     (1, 16, 32, 128, 256, 1, 1, 0, 1, 1), (1, 27, 19, 128, 256, 1, 1, 0, 1, 1),      # 512 tiles of 16 x 16; 528, and K short: of 64
     (1, 16, 16, 64, 256, 1, 1, 1, 0, 0), (1, 16, 17, 64, 256, 1, 1, 1, 0, 0),        # 256 of a K of 64; 272
     (1, 16, 16, 320, 1024, 1, 1, 0, 1, 1), (1, 1, 257, 320, 1024, 1, 1, 0, 1, 1),    # 256 tiles of 32 x 32, five blocks of K; 288: of 64
@@ -93,20 +94,20 @@ def test_conv(n, h, w, c, o, stride, bn, bias, res, relu):
 
 @pytest.mark.parametrize('n,h,w,c,side,o,stride,relu', [
     (3, 5, 7, 64, 64, 64, 1, 1),               # a stage of K each, one tile
-    (5, 9, 13, 64, 192, 136, 2, 0),            # rows and channels past a tile
+    (5, 9, 13, 64, 192, 136, 2, 0),            # tiles of 16 x 16, rows and channels past one
     (1, 14, 14, 512, 1024, 2048, 2, 1),        # few pixels, long rows: 512 tiles of 16 x 16
     (8, 28, 28, 256, 512, 1024, 2, 1),         # tiles of 64
     (16, 28, 28, 128, 256, 264, 1, 1),         # 128 x 64
-    (42, 56, 56, 64, 64, 136, 1, 1),           # 128 x 128, many
+    (42, 56, 56, 64, 64, 136, 1, 1),           # 128 x 128, 2058: short stages
     (27, 56, 56, 128, 256, 512, 2, 1),         # 128 x 128, 664 tiles
     (7, 45, 44, 64, 64, 264, 1, 1),            # 327 tiles, rows and channels past the last: a stage of K each
     (64, 16, 16, 64, 192, 2048, 2, 0),         # 512, one stage and three
     (26, 56, 55, 192, 128, 520, 2, 1),         # 800, three and two
     (21, 31, 33, 320, 256, 640, 1, 1),         # 840, five and four
-    (42, 56, 56, 128, 64, 64, 1, 1),           # 64 channels, many
+    (42, 56, 56, 128, 64, 64, 1, 1),           # 128 x 64, 1029: short stages
     (5, 9, 13, 192, 64, 133, 2, 0),            # channels no multiple of 8
-    (3, 25, 26, 128, 320, 264, 2, 1), (2, 17, 16, 64, 256, 520, 1, 0),    # tiles of 32 x 32, a wave with both products; channels past a tile
-    (1, 520, 516, 64, 64, 64, 2, 1),           # 67080 pixels: too many for a division by multiplying
+    (3, 25, 26, 128, 320, 264, 2, 1), (2, 17, 16, 64, 256, 520, 1, 0),    # tiles of 32 x 32, a wave with both products; of 64, channels past a tile
+    (1, 520, 516, 64, 64, 64, 2, 1),           # 128 x 64, 67080 pixels: too many for a division by multiplying
     # 128 x 128 in three stages: one and one of K, two and three, fourteen and three; 596 tiles: 128 x 64
     (7, 45, 44, 64, 64, 256, 1, 1), (28, 45, 44, 128, 192, 136, 2, 0), (5, 40, 42, 896, 192, 256, 1, 1), (16, 68, 70, 128, 64, 512, 2, 1),
 ])
@@ -126,18 +127,24 @@ def test_conv_pair(n, h, w, c, side, o, stride, relu):
     close(out, want, 3e-3)
 
 
-@pytest.mark.parametrize('n,c,side,o', [(40, 64, 192, 96), (600, 128, 320, 264)])
-def test_conv_pair_without_batchnorm(n, c, side, o):
-    """A bias joins the fp32 sum: each product is rounded once, and their sum once (2^-11 of it each)."""
+@pytest.mark.parametrize('n,c,side,o,once', [
+    (40, 64, 192, 96, 1), (600, 128, 320, 264, 1),                              # tiles of 16 x 16, of 32 x 32
+    (1200, 64, 256, 520, 0), (5000, 128, 64, 1000, 0), (3000, 512, 512, 1000, 0),      # of 64, of 128 x 128, in three stages
+    (9600, 64, 128, 1000, 0), (33000, 64, 64, 1000, 0), (132000, 64, 128, 64, 0),      # of 128 x 64, of 128 x 128 in short stages, of 128 x 64 in those
+])
+def test_conv_pair_without_batchnorm(n, c, side, o, once):
+    """In small tiles a bias joins the fp32 sum: each product is rounded once, and their sum once (2^-11 of it each).  Larger ones
+    round a product's sum in front of its bias as well."""
     torch.manual_seed(c + o)
     x, xs = (torch.randn(n, 1, 1, k, device='cuda').half() for k in (c, side))
     wt, ws = ((torch.randn(o, k, device='cuda') * k ** -0.5).half() for k in (c, side))
     (norm, _, keep), (norm_s, _, keep_s) = (make_norm(o, 0, 1) for _ in range(2))
-    a = x.view(n, c).double() @ wt.double().t() + keep['conv_bias'].double()
-    b = xs.view(n, side).double() @ ws.double().t() + keep_s['conv_bias'].double()
+    sum_a, sum_b = x.view(n, c).double() @ wt.double().t(), xs.view(n, side).double() @ ws.double().t()
+    a, b = sum_a + keep['conv_bias'].double(), sum_b + keep_s['conv_bias'].double()
     out = torch.empty(n, o, device='cuda', dtype=torch.float16)
     call('ddf_hip_net_conv_pair', x, wt, norm, c, xs, ws, norm_s, 1, 1, side, 1, out, n, o, 0)
-    bound = (a.abs() + b.abs() + (a + b).abs()) * 2.0 ** -11 + 1e-4    # (and the fp32 sums)
+    rounded = a.abs() + b.abs() if once else sum_a.abs() + sum_b.abs() + b.abs()
+    bound = (rounded + (a + b).abs()) * 2.0 ** -11 + 1e-4    # (and the fp32 sums)
     assert ((out.double() - a - b).abs() <= bound).all()
 
 
@@ -244,7 +251,7 @@ def test_network_matches_its_modules(build, n, size, classes):
 
 @pytest.mark.parametrize('n,h,w,c,o', [
     (1, 1, 1, 64, 64),                          # one pixel
-    (5, 7, 7, 64, 64), (3, 5, 7, 512, 512),     # samples that end inside tiles of 64 rows, of 16
+    (5, 7, 7, 64, 64), (3, 5, 7, 512, 512),     # samples that end inside tiles of 16 rows
     (1, 14, 14, 1024, 256), (2, 14, 14, 1024, 256),
     (9, 28, 28, 64, 128), (33, 28, 28, 256, 64), (16, 28, 28, 128, 264), (42, 56, 56, 64, 136),
     (200, 14, 14, 256, 520), (1, 56, 56, 256, 72), (42, 56, 56, 64, 64), (20, 4, 8, 1024, 256),
