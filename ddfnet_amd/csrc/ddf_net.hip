@@ -1073,13 +1073,14 @@ hipError_t launch_conv(const NetConv &a, const NetConv *first, hipStream_t st) {
 // us, four waves of three short stages / of two long ones / eight of two long ones: 25088 pixels 1024 -> 256 with sums over the pixels 24.1 / 21.9 / 21.7, 256 -> 1024
 // with a residual 27.9 / 27.8 / 27.1, 50176 512 -> 256 25.5 / 22.9 / 22.6, pairs 128 + 256 -> 512 of 12544, 25088 and 50176 pixels 14.5 / 13.8 / 13.4, 25.9 / 24.2 /
 // 22.7, 40.2 / 41.8 / 38.9, 256 + 512 -> 1024 of 25088 64.9 / 62.8 / 60.0.  With many tiles of short sums memory counts more, and three
-// workgroups of four waves in short stages are ahead: a product of less than 768 from 1024 tiles on, a pair of less than 1024 from 2048.  us, eight waves /
+// workgroups of four waves in short stages are ahead: a product of less than 768 from 1024 tiles on, with a residual from 2048, a pair of less than 1024 from 2048.  us, eight waves /
 // short stages, operands of the call before in cache | others': with sums over the pixels 100352 pixels, 1568 tiles, 64 -> 256 16.0 / 15.3 | 21.5 / 20.1, 256 -> 256
 // 31.2 / 26.8 | 37.2 / 32.6, 512 -> 256 45.4 / 41.9 | 54.2 / 50.4, 640 -> 256 52.9 / 52.1 | 66.3 / 62.4, 768 -> 256 61.1 / 61.1 | 73.9 / 70.2, 1024 -> 256 76.2 / 80.2 | 91.3 /
 // 91.1, 2048 -> 256 171.7 / 171.8 | 169.5 / 172.1; 25088 512 -> 1024 40.0 / 41.5 | 49.7 / 45.7, 768 -> 1024 55.1 / 60.2 | 66.8 / 64.7; with a residual
 // 50176 256 -> 512 28.9 / 27.6 | 36.5 / 34.1, 1024 -> 512 71.7 / 77.3 | 88.7 / 87.7; below 1024 tiles 760 of 256 20.6 / 18.8 and 1018 23.5 / 23.8 (not in cache); pairs
 // 128 + 256 -> 512 1300 tiles 32.0 / 32.9 | 36.4 / 37.3, 1960 43.4 / 44.6 | 51.1 / 50.6, 3136 68.9 / 69.8 | 82.0 / 79.4, 256 + 512 -> 1024 1300 48.4 / 52.7 | 54.9 / 55.7, 3136 110 /
-// 119 | 130 / 128, 512 + 1024 -> 2048 3136 191 / 221 | 214 / 228.  (A network's time is the same with either: its products of these sizes are in chains.)
+// 119 | 130 / 128, 512 + 1024 -> 2048 3136 191 / 221 | 214 / 228.  (In a network, whose other products of
+// these sizes are in chains, five of 25088 256 -> 1024 with a residual, 1568 tiles, by eight waves are 2 us less of 1534, of 104 images 3 of 1351.)
 // Up to one workgroup per unit the stages themselves are the time, and a third one in flight is what helps: us, tiles of 64 x 64 / 128 x 128 in two
 // stages / in three, 12544 pixels 1024 -> 256, 196 tiles, 16.9 / 16.1 / 13.2, 6272 2048 -> 512 28.4 / 28.8 / 22.1, pairs 256 + 512 -> 1024 of 3136 14.8 /
 // 13.2 / 11.9, 512 + 1024 -> 2048 of 1568 24.3 / 23.5 / 18.4, 148 tiles of K = 2048 21.7 / 27.5 / 20.9.  Fewer than that fill the chip better in
@@ -1107,7 +1108,7 @@ ConvTile conv_tile(const NetConv &a, const NetConv *first) {
     if (a.N >= 128) {
         const int64_t tiles = count(128, 128);
         if (tiles <= 256 && tiles > (K >= 1024 ? 128 : 160)) return kTile128Deep;
-        if (pair ? tiles >= 2048 && K < 1024 : tiles >= 1024 && K < 768) return kTile128Short;
+        if (tiles >= (pair || a.res ? 2048 : 1024) && K < (pair ? 1024 : 768)) return kTile128Short;
         if (tiles >= 320 && (tiles <= 512 || tiles > 608)) return kTile128;
     } else if (count(128, 64) >= kMany) {
         return kTile128x64;
