@@ -50,12 +50,13 @@ struct PackDims {
 constexpr int kFc2Samples = 64, kFc2MaxChannels = kWaves, kUnits = 256;    // (compute units)
 constexpr int kFc2Pitch = 12;    // a channel's nine values, 16-byte rows
 
-// Channels per workgroup: few as long as the workgroups do not outnumber the compute units.  Every channel block
-// leaves a partial dh of all samples, so no more of them than fill the chip.  The launch with four channels
+// Channels per workgroup: one or two as long as the workgroups do not outnumber the compute units, else four.  Every channel block
+// leaves a partial dh of all samples, so no more of them than fill the chip where there is a choice.  The launch with four channels
 // each and this, us (fp16, medians under the profiler): 64 x 128 x 28 x 28 18.2 / 8.8, 64 x 64 x 56 x 56 19.4 / 8.8, 64 x 256 x 14 x 14 17.6 / 8.5, 256 x 128 x
 // 14 x 14 55.4 / 19.6, 1 x 512 x 14 x 14 6.4 / 5.8, fp32 32 x 256 x 28 x 28 15.0 / 10.4; four of them with the loads asked for at once: 64 x 512 x 7 x 7
 // 18.9 / 13.6, 3 x 2048 x 7 x 7 31.8 / 23.9.  (8 x 64 x 200 x 300, whose time is the other half's: 13.0 / 13.7.)
-// Batches whose parts would pass 64 MB, 25 us to write and read again at a copy's rate, take more channels: the workspace stays bounded.
+// Batches whose parts would pass 64 MB, 25 us to write and read again at a copy's rate, take more channels: one or two of them never ask for more
+// workspace than that.  Four are the most (registers), and their parts grow with the batch: 256 x 2048 with 512 hidden values 256 MB.
 constexpr int64_t kFc2MostParts = 1 << 24;
 inline int fc2_channels(int64_t N, int64_t C, int64_t mid) {
     int cw = 1;

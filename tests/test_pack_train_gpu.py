@@ -12,8 +12,8 @@ CASES = [
     # n, c, h, w, stride, head, combine
     (2, 64, 14, 14, 1, 1, 'mul'),
     (1, 16, 1, 1, 1, 1, 'add'),        # a single pixel: one step, all of it remainder
-    (33, 20, 7, 7, 1, 1, 'mul'),       # samples past a chunk of 32, odd planes, mid = 4
-    (3, 136, 9, 11, 1, 2, 'mul'),      # channels past a block of 8 and a tile of 16, two heads
+    (33, 20, 7, 7, 1, 1, 'mul'),       # odd planes, mid = 4
+    (3, 136, 9, 11, 1, 2, 'mul'),      # channels past a tile of 16, two heads
     (2, 64, 12, 16, 1, 4, 'add'),
     (2, 340, 8, 6, 1, 1, 'mul'),       # mid = 68: past one chunk of 64 hidden values
     (5, 32, 18, 10, 2, 1, 'mul'),      # stride 2
