@@ -67,3 +67,28 @@ def test_native_training_step_has_no_second_derivative_and_follows_changes():
     pack.channel_branch[1].weight.requires_grad_(False)             # partly frozen: op by op
     pack(x).sum().backward()
     assert pack.channel_branch[1].weight.grad is None and pack.channel_branch[3].weight.grad is not None
+
+
+@pytest.mark.parametrize('n,levels', [(16, 4), (33, 6)])
+def test_sums_over_samples_are_added_in_pairs(n, levels):
+    """A sample's gradient of 2^24 and the others' of one, added up by sixteen threads: each level of pairs loses one at most (half of
+    2^24's last place), where one after another all of them would be lost."""
+    from ctypes import c_void_p
+    from ddfnet_amd import _lib
+    c, h, w, mid = 16, 4, 4, 3
+    lib = _lib.lib()
+
+    def zeros(*shape):
+        return torch.zeros(*shape, device='cuda')
+    x, dcf, draw, pooled, hidden, taps = zeros(n, c, h, w), zeros(n, c, 9), zeros(n, 9, h, w), zeros(n, c), zeros(n, mid), torch.randn(n, c * 9, device='cuda')
+    w1, w2, ws = zeros(mid, c), zeros(9 * c, mid), zeros(9, c)
+    draw[:, :, 1, 2] = 1.
+    draw[0, :, 1, 2] = 2. ** 24
+    grads = [zeros(9, c), zeros(9), zeros(mid, c), zeros(mid), zeros(9 * c, mid), zeros(9 * c), zeros(9 * c)]
+    size = lib.ddf_hip_pack_backward_workspace_bytes(n, c, h, w, mid, 1, 3, 1, _lib.DTYPE[torch.float32])
+    space = torch.empty(size, dtype=torch.uint8, device='cuda')
+    pointers = [c_void_p(t.data_ptr()) for t in (x, dcf, draw, pooled, hidden, taps, ws, w1, w2)]
+    _lib.check(lib.ddf_hip_pack_backward(*pointers, None, 1.0, None, *(c_void_p(g.data_ptr()) for g in grads), c_void_p(space.data_ptr()), size,
+                                         n, c, h, w, mid, 1, 3, 1, _lib.DTYPE[torch.float32],
+                                         c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert (grads[1].double() - (2 ** 24 + n - 1)).abs().max() <= levels
