@@ -997,6 +997,9 @@ __device__ __forceinline__ void rows_walk(const RowsGeom &g, int block, const T 
     }
 }
 
+// (As a function of its own the walk asks for the kernel's arguments in fewer, wider loads, and computes less in front of its first
+// vectors, than the same code in the kernel did: 220 forward calls and layers without gradients 2.1 % less on average, from 12 % less, 3.68 /
+// 3.24 us at fp16 1 x 360 x 16 x 12 under stride 2, to 3.4 % more, 13.42 / 13.88 at fp16 6 x 320 x 67 x 86.)
 template <typename T, int K, int D, bool MUL, bool BWD, int VX, int R, bool PAD, int NST, int WPE,
           int S = 1, int TAIL = 0>
 __global__ __launch_bounds__(kWave * kMaxWpb, WPE) void k_rows(RowsGeom g, const T *__restrict__ x,
